@@ -87,6 +87,9 @@ _SIGS = {
     "grag_relu2": [P, I64, I, P],
     "grag_decay_attn_scan": [P, I, I, I, I, P, P, P, P, P, P, I, I, I, I, I, I, P, I, I, P, P, I, I, F, P],
     "grag_decay_attn_chunk": [],
+    "grag_linear_scan_max_dim": [],
+    "grag_linear_scan_decay": [P, I, I, I, I, P, P, P, P, P, P, I, I, I, I, I, I, P, P, I, I, I, P, P, I, I, F, P],
+    "grag_linear_scan_ssm": [P, I, I, I, P, I, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P, P, I, I, P],
     "grag_mingru_chunk": [],
     "grag_gated_rmsnorm": [P, P, P, I, I, P, I, I, I, F, F, I, I, I, P],
     "grag_mingru_scan": [P, I, I, I, I, P, P, P, P, P, P, P, I, I, I, I, P, I, P],
@@ -190,7 +193,7 @@ def call(name: str, *args) -> None:
 
 
 # ---------------------------------------------------------------- device index guard (csrc/kernels/common.h)
-ERR_UNITS = ("norm", "elementwise", "attention", "gemm_tile", "gemm_stream", "seqmix", "gatedmix", "ssm", "moe", "delta")
+ERR_UNITS = ("norm", "elementwise", "attention", "gemm_tile", "gemm_stream", "seqmix", "gatedmix", "ssm", "moe", "delta", "linscan")
 ERR_CODES = {1 << 0: "embed_gather: token id >= vocab", 1 << 1: "qkv_rope_kvstore: KV slot id >= cache slots",
              1 << 2: "qkv_rope_kvstore: position >= RoPE table rows",
              1 << 3: "prefill attention: block-table entry >= KV blocks",

@@ -24,6 +24,49 @@ def _chunk_ws(kind: str, m: AttnMetadata, per_chunk: int, device) -> torch.Tenso
     return torch.empty(m.num_seqs * -(-m.max_q_len // chunk) * per_chunk, dtype=torch.float32, device=device)
 
 
+LINEAR_SCAN_MIN = 8  # tokens of the longest portion from which the matrix-core scan is taken
+LINEAR_SCAN_CHUNK = 64
+
+
+def _scan_taken(m: AttnMetadata, d: int, tiles: int, split: bool) -> bool:
+    """Whether a step runs the matrix-core scan.  A workgroup's chunk costs the same for 1 or 64 tokens; the one-pass
+    kernels pay per token (4 sequences x 8 tokens x 28 heads: 16 us against 52; one of 64 tokens: 16 against 263).  Only
+    where many short portions fill the chip several times does the chunk cost more, and only with operands in three parts
+    (64 x 8 tokens x 28 heads: 190 us against 109; 64 x 16: 190 against 177; 20 x 30: 72 against 173)."""
+    if m.max_q_len < LINEAR_SCAN_MIN or d > lib().grag_linear_scan_max_dim():
+        return False
+    return not split or m.max_q_len >= 3 * LINEAR_SCAN_MIN or m.num_seqs * tiles <= 512
+
+
+def _scan_part(max_q: int, tokens: int, nseq: int, tiles: int, split: bool) -> int:
+    """Tokens per part of the matrix-core scan (csrc/kernels/linscan.hip) for a step of ``nseq`` portions with ``tokens``
+    tokens, the longest ``max_q``, and ``tiles`` (head, 64 columns) tiles a portion.  In walks of a 64-token chunk: whole
+    portions cost the longest walk, or the chip's share of all; cut into parts, every round of workgroups walks a part
+    twice (the first walk, for the state alone, is about half) and reads the states of the parts before it.  ``split``:
+    operands in three parts (one workgroup a CU, 12 us a chunk), else two workgroups a CU and 5 us."""
+    slots, read = (256, 0.06) if split else (512, 0.28)
+    chunks, total = -(-max_q // LINEAR_SCAN_CHUNK), tokens / LINEAR_SCAN_CHUNK
+    whole = max(chunks, total * tiles / slots)
+    best, part, s = 0.85 * whole, chunks, 1
+    while s < chunks:
+        rounds = -(-int((total / s + nseq / 2) * tiles) // slots)
+        cost = max(1, rounds) * (1.5 * s + read * chunks / s) + 1
+        if cost < best:
+            best, part = cost, s
+        s *= 2
+    return part * LINEAR_SCAN_CHUNK
+
+
+def _scan_ws(m: AttnMetadata, rows: int, H: int, d: int, vd: int, split: bool, device):
+    """(part, ws, wa) of a matrix-core scan: the part length and its fp32 scratch (None where no portion is cut)."""
+    part = _scan_part(m.max_q_len, rows, m.num_seqs, H * -(-vd // 64), split)
+    if m.max_q_len <= part:
+        return part, None, None
+    n = m.num_seqs * -(-m.max_q_len // part)
+    return (part, torch.empty(n * H * d * vd, dtype=torch.float32, device=device),
+            torch.empty(n * H, dtype=torch.float32, device=device))
+
+
 def _dt(t: torch.Tensor) -> int:
     return 0 if t.dtype == torch.bfloat16 else 1
 
@@ -60,6 +103,14 @@ def decay_attention(proj: torch.Tensor, qoff: int, koff: int, voff: int, decay: 
             continue
         assert proj.stride(1) == 1 and state.dtype == torch.float32 and state.is_contiguous()
         x = proj[r0:r1]
+        split = act or rd > 0 or _dt(proj) != 0
+        if _scan_taken(m, d, H * -(-vd // 64), split):
+            part, ws, wa = _scan_ws(m, r1 - r0, H, d, vd, split, proj.device)
+            call("grag_linear_scan_decay", ptr(x), proj.stride(0), qoff, koff, voff, ptr(decay), ptr(state),
+                 ptr(m.state_slots), ptr(m.q_start), ptr(m.ctx_len), ptr(out[r0:r1]), m.num_seqs, H, d, vd,
+                 state.shape[0], _dt(proj), ptr(ws), ptr(wa), part, m.max_q_len, 1 if act else 0, ptr(pos), ptr(rope), rd,
+                 rope.shape[0] if rd else 0, float(k_scale))
+            continue
         ws = _chunk_ws("decay", m, H * d * vd, proj.device)
         call("grag_decay_attn_scan", ptr(x), proj.stride(0), qoff, koff, voff, ptr(decay), ptr(state),
              ptr(m.state_slots), ptr(m.q_start), ptr(m.ctx_len), ptr(out[r0:r1]), m.num_seqs, H, d, vd,
@@ -226,6 +277,12 @@ def ssm_scan(xbc: torch.Tensor, proj: torch.Tensor, dtoff: int, dt_bias: torch.T
             continue
         assert xbc.is_contiguous() and proj.stride(1) == 1 and state.dtype == torch.float32 and state.is_contiguous()
         assert xbc.dtype == proj.dtype and state.shape[1:] == (H, N, P)
+        if _scan_taken(m, N, H * -(-P // 64), _dt(xbc) != 0):
+            part, ws, wa = _scan_ws(m, r1 - r0, H, N, P, _dt(xbc) != 0, xbc.device)
+            call("grag_linear_scan_ssm", ptr(xbc[r0:r1]), C, H * P, H * P + G * N, ptr(proj[r0:r1]), proj.stride(0), dtoff,
+                 ptr(dt_bias), ptr(a_log), ptr(skip), ptr(state), ptr(m.state_slots), ptr(m.q_start), ptr(m.ctx_len),
+                 ptr(out[r0:r1]), m.num_seqs, H, G, N, P, state.shape[0], _dt(xbc), ptr(ws), ptr(wa), part, m.max_q_len)
+            continue
         chunk = lib().grag_ssm_chunk()
         ws = wa = None
         if m.max_q_len > chunk:

@@ -1,0 +1,129 @@
+"""The matrix-core scan of the decay linear attention and of the state-space mixer (csrc/kernels/linscan.hip) against the
+recurrences written out in 64 bits: sizes around its tiles (64 tokens, 64 columns, 32 rows), portions cut into parts,
+carried states, every form of its operands."""
+import pytest
+import torch
+
+from githubrepostorag_amd.ops import recurrent
+from githubrepostorag_amd.ops.attention import AttnMetadata
+
+pytestmark = pytest.mark.gpu
+# Both sides sum the same terms; B is the same recurrence over their absolute values.  fp32 sums of up to 64 + 128 terms
+# round by at most (64 + 128) / 2 ulp of 6e-8 of B in the worst order, and the weights 2^(L_t - L_s) carry a few ulp more.
+TOL = 1.2e-5
+
+
+def _meta(lens, past, dev):
+    q = [0]
+    for n in lens:
+        q.append(q[-1] + n)
+    t = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    return AttnMetadata(q_start=t(q), ctx_len=t([n + p for n, p in zip(lens, past)]), block_tables=None, slot_mapping=None,
+                        max_q_len=max(lens), num_seqs=len(lens), num_tokens=q[-1],
+                        state_slots=t([len(lens) - 1 - i for i in range(len(lens))])), q
+
+
+def _walk(a, k, v, q, S):
+    """S_t = a_t S + k_t v_t^T, o_t = S_t^T q_t over [n, H, ...] float64."""
+    out = []
+    for t in range(q.shape[0]):
+        S = a[t][:, None, None] * S + k[t][:, :, None] * v[t][:, None, :]
+        out.append((S * q[t][:, :, None]).sum(1))
+    return torch.stack(out), S
+
+
+def _check(got, want, bound, what):
+    worst = ((got.double().cpu() - want).abs() / (bound + 1e-30)).max().item()
+    assert worst < TOL, f"{what}: {worst:.2e} of the bound"
+
+
+CASES = [
+    # lens, past, H, d, vd, dtype, act, rope dims, part
+    ([64], [0], 2, 128, 128, torch.bfloat16, False, 0, 64),
+    ([65, 8, 130], [0, 7, 3], 3, 128, 64, torch.bfloat16, True, 0, 1 << 20),
+    ([200, 63, 1], [0, 5, 0], 2, 24, 40, torch.bfloat16, False, 0, 64),
+    ([300, 129], [0, 9], 2, 128, 128, torch.bfloat16, True, 0, 128),
+    ([257], [4], 3, 33, 65, torch.bfloat16, True, 22, 64),
+    ([190, 64], [0, 1], 2, 100, 70, torch.float32, False, 0, 64),
+    ([130], [0], 1, 17, 9, torch.float32, True, 6, 64),
+    ([9], [2], 2, 5, 3, torch.bfloat16, False, 0, 64),
+]
+
+
+@pytest.mark.parametrize("lens,past,H,d,vd,dtype,act,rd,part", CASES)
+def test_decay_scan(lens, past, H, d, vd, dtype, act, rd, part, monkeypatch):
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(sum(lens) + d)
+    m, qs = _meta(lens, past, dev)
+    T = qs[-1]
+    monkeypatch.setattr(recurrent, "_scan_part", lambda *a: part)
+    pad = 0 if d % 4 == 0 else 3  # odd sizes go with rows that are not aligned
+    proj = torch.randn(T, H * (2 * d + vd) + pad, generator=g).to(dtype)
+    decay = torch.tensor([1.0, 0.0, -0.97][:H] if d < 64 else [0.996, 0.05, 0.75][:H])
+    state = torch.randn(len(lens) + 1, H, d, vd, generator=g)
+    rope = torch.randn(512, rd, generator=g) if rd else None
+    pos = torch.cat([torch.arange(p, p + n) for n, p in zip(lens, past)]).to(torch.int32)
+    ks = 0.3
+    st = state.to(dev)
+    got = recurrent.decay_attention(proj.to(dev), 0, H * d, 2 * H * d, decay.to(dev), st, m, H, d, vd, act=act,
+                                    positions=pos.to(dev) if rd else None, rope=rope.to(dev) if rd else None, k_scale=ks)
+    x = proj.double()
+    f = torch.nn.functional.silu if act else (lambda t: t)
+    q, k = (f(x[:, o:o + H * d]).view(T, H, d) for o in (0, H * d))
+    v = f(x[:, 2 * H * d:2 * H * d + H * vd]).view(T, H, vd)
+
+    def rot(t):
+        if not rd:
+            return t
+        c, s = (rope.double()[pos.long()][:, None, o:o + rd // 2] for o in (0, rd // 2))
+        u, w = t[..., :rd // 2], t[..., rd // 2:rd]
+        return torch.cat([u * c - w * s, w * c + u * s, t[..., rd:]], -1)
+
+    q, k = rot(q), rot(k) * ks
+    for i, (a, b) in enumerate(zip(qs, qs[1:])):
+        slot = len(lens) - 1 - i
+        lam = decay.double().expand(b - a, H)
+        S0 = state[slot].double() if past[i] else torch.zeros(H, d, vd, dtype=torch.float64)
+        o, S = _walk(lam, k[a:b], v[a:b], q[a:b], S0)
+        bo, bS = _walk(lam.abs(), k[a:b].abs(), v[a:b].abs(), q[a:b].abs(), S0.abs())
+        _check(got[a:b].view(-1, H, vd), o, bo, "outputs")
+        _check(st[slot], S, bS, "state")
+    assert torch.equal(st[len(lens)].cpu(), state[len(lens)])
+
+
+SSM = [
+    # lens, past, H, G, N, P, dtype, part
+    ([64, 70], [0, 3], 4, 1, 128, 64, torch.bfloat16, 1 << 20),
+    ([300, 65, 8], [0, 0, 11], 6, 2, 128, 64, torch.bfloat16, 64),
+    ([193], [5], 6, 2, 12, 8, torch.bfloat16, 128),
+    ([129, 128], [0, 2], 3, 3, 50, 67, torch.float32, 64),
+]
+
+
+@pytest.mark.parametrize("lens,past,H,G,N,P,dtype,part", SSM)
+def test_state_space_scan(lens, past, H, G, N, P, dtype, part, monkeypatch):
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(sum(lens) + N)
+    m, qs = _meta(lens, past, dev)
+    T = qs[-1]
+    monkeypatch.setattr(recurrent, "_scan_part", lambda *a: part)
+    xbc = torch.randn(T, H * P + 2 * G * N, generator=g).to(dtype)
+    proj = (2 * torch.randn(T, H + 5, generator=g)).to(dtype)
+    dtb, alog, skip = torch.randn(H, generator=g), torch.linspace(-2.0, 3.0, H), torch.randn(H, generator=g)
+    state = torch.randn(len(lens) + 1, H, N, P, generator=g)
+    st = state.to(dev)
+    got = recurrent.ssm_scan(xbc.to(dev), proj.to(dev), 2, dtb.to(dev), alog.to(dev), skip.to(dev), st, m, H, G, N, P)
+    x = xbc.double()
+    v = x[:, :H * P].view(T, H, P)
+    Bm, Cm = (x[:, H * P + o * G * N:H * P + (o + 1) * G * N].view(T, G, N).repeat_interleave(H // G, 1) for o in (0, 1))
+    dt = torch.nn.functional.softplus(proj.double()[:, 2:2 + H] + dtb.double(), threshold=60.0)
+    a = torch.exp(-torch.exp(alog.double()) * dt)
+    k = Bm * dt[:, :, None]
+    for i, (s, e) in enumerate(zip(qs, qs[1:])):
+        slot = len(lens) - 1 - i
+        S0 = state[slot].double() if past[i] else torch.zeros(H, N, P, dtype=torch.float64)
+        o, S = _walk(a[s:e], k[s:e], v[s:e], Cm[s:e], S0)
+        bo, bS = _walk(a[s:e], k[s:e].abs(), v[s:e].abs(), Cm[s:e].abs(), S0.abs())
+        extra = skip.double()[:, None] * v[s:e]
+        _check(got[s:e].view(-1, H, P), o + extra, bo + extra.abs(), "outputs")
+        _check(st[slot], S, bS, "state")
