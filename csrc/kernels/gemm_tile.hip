@@ -34,7 +34,7 @@
 // (LDS image lane-linear, rule 21) — conflict-free for the b128 lane groups.
 // The MFMA is issued with the W fragment as operand A, so each lane ends with
 // 4 consecutive output columns of one row: 8-byte bf16 / 16-byte fp32 stores.
-#include "common.h"
+#include "tile256.h"
 
 using namespace grag;
 
@@ -290,71 +290,16 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tile_kernel(Args p) {
           glds16(srcB[q][i] + kt * 64, dst);
       }
     };
+    if constexpr (SCHED == 2) {
+      // the two-phase schedule (tile256.h): half the barriers per MFMA of the 4-phase schedules; an interval's fixed cost --
+      // barrier skew over 8 waves, setprio hand-off, wait -- is what kept those at 71-74 % MFMA busy
+      tile256_loop<false>(smem, rsA, rsB, offA, offB, nk, 128, acc00, acc01, acc11, acc10);
+      return;
+    }
     acc_zero<MF>(acc00);
     acc_zero<MF>(acc01);
     acc_zero<MF>(acc11);
     acc_zero<MF>(acc10);
-    if constexpr (SCHED == 2) {
-      // Two-phase schedule: 32 MFMAs per barrier interval instead of 16 (half the barriers per MFMA; the
-      // interval's fixed cost -- barrier skew over 8 waves, setprio hand-off, wait -- is what kept the 4-phase
-      // schedules at 71-74 % MFMA busy, profiles/pmc_tile_r5.txt).  Per K-tile t (buffer b = t & 1):
-      //   L1 reads A q0, B q0, B q1 (16 b128)  refill A q1 of tile t+1 (buffer b^1; read there in L2(t-1))
-      //   M1 acc00 = A0 B0, acc01 = A0 B1       (32 MFMAs)
-      //   L2 reads A q1 (8 b128)                refill A q0, B q0, B q1 of tile t+2 (buffer b; read in L1(t))
-      //   M2 acc10 = A1 B0, acc11 = A1 B1       (32 MFMAs; B q0 / q1 held from L1)
-      // Every load segment ends with a counted vmcnt(8) (its own 2 or 6 refills plus the other segment's are
-      // the 8 youngest), which retires the batch the NEXT load segment reads -- for the lagging half too,
-      // whose load segments coincide with the leading half's MFMA segments.  A refill is issued one segment
-      // after the barrier that closes the last read of its slot by either half.  Refills past the last
-      // K-tile re-load it (clamped index) into slots nobody reads again, so the counts never change.
-      const int klast = nk - 1;
-      issueA(0, 0, 0);
-      issueB(0, 0, 0);
-      issueB(1, 0, 0);
-      issueA(1, 0, 0);
-      issueA(0, min(1, klast), 1);
-      issueB(0, min(1, klast), 1);
-      issueB(1, min(1, klast), 1);
-      wait_vm<6>();  // tile 0 landed (tile 1's A0 / B0 / B1 are the 6 youngest)
-      bar();
-      if (lag) bar();
-      auto ktile2 = [&](int kt, auto odd_c) {
-        constexpr int buf = decltype(odd_c)::value ? 1 : 0;
-        // L1
-        readA(a, 0, buf);
-        readB(b0, 0, buf);
-        readB(b1, 1, buf);
-        issueA(1, min(kt + 1, klast), buf ^ 1);
-        wait_vm<8>();
-        wait_lgkm0();
-        bar();
-        // M1
-        mma_cluster<MF>(acc00, a, b0);
-        mma_cluster<MF>(acc01, a, b1);
-        bar();
-        // L2
-        readA(a, 1, buf);
-        issueA(0, min(kt + 2, klast), buf);
-        issueB(0, min(kt + 2, klast), buf);
-        issueB(1, min(kt + 2, klast), buf);
-        wait_vm<8>();
-        wait_lgkm0();
-        bar();
-        // M2
-        mma_cluster<MF>(acc10, a, b0);
-        mma_cluster<MF>(acc11, a, b1);
-        bar();
-      };
-      int kt = 0;
-      for (; kt < klast; kt += 2) {
-        ktile2(kt, std::integral_constant<bool, false>{});
-        ktile2(kt + 1, std::integral_constant<bool, true>{});
-      }
-      if (kt == klast) ktile2(kt, std::integral_constant<bool, false>{});
-      wait_vm<0>();  // the clamped re-loads land before the LDS is reused (next segment / stream-K flag)
-      if (!lag) bar();
-      return;
-    }
     if constexpr (SCHED == 1) {
       // Balanced schedule: 8 / 4 / 8 / 4 fragment reads per phase instead of 12 / 4 / 8 / 0.  P4 of
       // K-tile t reads the B quadrant that tile t+1 starts with (its own MFMAs use the other one), so

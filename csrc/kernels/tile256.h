@@ -1,0 +1,162 @@
+// The 256 x 256 bf16 tile product that the dense and the grouped GEMM share (gemm_tile.hip, moe_tile.hip): 8 waves (512
+// threads) as 2 (rows) x 4 (columns), K steps of 64, 16x16x32 matrix-core products, two LDS buffers refilled by LDS-DMA.
+// Wave (wr, wc) owns rows [128 wr, +128) x columns [64 wc, +64) as 2 x 2 quadrants of 64 x 32.  A buffer holds 4 slots of 16 KB
+// (A q0, A q1, B q0, B q1), each the 128 rows (both wave rows / all 4 wave columns) that one quadrant needs; rows are 128
+// bytes, their 16-byte chunks XOR-swizzled by (row >> 1) & 7 on the source address.
+#pragma once
+#include "common.h"
+
+namespace grag {
+
+typedef __attribute__((address_space(3))) void tile_lds_t;
+
+constexpr int kTileSlot = 128 * 128;        // bytes: 128 rows x 64 bf16
+constexpr int kTileBuf = 4 * kTileSlot;     // one K step: A q0, A q1, B q0, B q1
+constexpr int kTileThreads = 512;
+
+typedef f32x4_t TileAcc[4][2];   // a quadrant: [16 rows][16 columns]
+typedef bf16x8_t TileA[4][2];    // [16 rows][k step of 32]
+typedef bf16x8_t TileB[2][2];    // [16 columns][k step]
+
+__device__ __forceinline__ void tile_zero(TileAcc& c) {
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int n = 0; n < 2; ++n) c[m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+}
+// (the W fragment is operand A, so that a lane ends with 4 consecutive output columns of one row)
+__device__ __forceinline__ void tile_mma(TileAcc& acc, const TileA& a, const TileB& b) {
+  __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt)
+        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[nt][s], a[mt][s], acc[mt][nt], 0, 0, 0);
+  __builtin_amdgcn_s_setprio(0);
+}
+// raw barrier: never drains the LDS-DMA in flight (a __syncthreads() would emit vmcnt(0))
+__device__ __forceinline__ void tile_bar() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+template <int N> __device__ __forceinline__ void tile_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory"); }
+__device__ __forceinline__ void tile_wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// The LDS row (0..127) and 16-byte source chunk (0..7) of the thread's DMA piece i (0, 1) of a slot
+__device__ __forceinline__ int tile_piece_row(int i) {
+  return (2 * (threadIdx.x >> 6) + i) * 8 + ((threadIdx.x & 63) >> 3);
+}
+__device__ __forceinline__ int tile_piece_chunk(int i) { return (threadIdx.x & 7) ^ ((tile_piece_row(i) >> 1) & 7); }
+
+// Two-phase schedule: 32 MFMAs per barrier interval.  Per K step t (buffer b = t & 1):
+//   L1 reads A q0, B q0, B q1 (16 b128)  refill A q1 of step t+1 (buffer b^1; read there in L2(t-1))
+//   M1 acc00 = A0 B0, acc01 = A0 B1       (32 MFMAs)
+//   L2 reads A q1 (8 b128)                refill A q0, B q0, B q1 of step t+2 (buffer b; read in L1(t))
+//   M2 acc10 = A1 B0, acc11 = A1 B1       (32 MFMAs; B q0 / q1 held from L1)
+// Waves 4-7 (wr = 1) run one barrier interval behind waves 0-3: on every SIMD one wave loads while its partner multiplies.
+// Every load segment ends with a counted vmcnt(8) (its own 2 or 6 refills plus the other segment's are the 8 youngest), which
+// retires the batch the NEXT load segment reads -- for the lagging half too, whose load segments coincide with the leading
+// half's MFMA segments.  A refill is issued one segment after the barrier that closes the last read of its slot by either
+// half.  Refills past the last K step re-load it (clamped index) into slots nobody reads again, so the counts never change.
+// offA / offB [quadrant][piece]: byte offsets of the thread's DMA pieces at the first K step (tile_piece_row / _chunk say
+// which).  live: rows of this wave's 128 that exist; quadrants without any are not multiplied (PARTIAL only).
+template <bool PARTIAL>
+__device__ __forceinline__ void tile256_loop(char* smem, const __amdgpu_buffer_rsrc_t& rsA, const __amdgpu_buffer_rsrc_t& rsB,
+                                             const unsigned (&offA)[2][2], const unsigned (&offB)[2][2], int nk, int live,
+                                             TileAcc& acc00, TileAcc& acc01, TileAcc& acc11, TileAcc& acc10) {
+  const int L = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = w >> 2, wc = w & 3;
+  const bool lag = w >= 4;
+  const int cb = (L >> 4) ^ ((L >> 1) & 7);
+  const int off0 = (L & 15) * 128 + cb * 16, off1 = (L & 15) * 128 + (cb ^ 4) * 16;
+  auto readA = [&](TileA& a, int q, int buf) {
+    const char* base = smem + buf * kTileBuf + q * kTileSlot + wr * 64 * 128;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      a[mt][0] = *reinterpret_cast<const bf16x8_t*>(base + mt * 2048 + off0);
+      a[mt][1] = *reinterpret_cast<const bf16x8_t*>(base + mt * 2048 + off1);
+    }
+  };
+  auto readB = [&](TileB& b, int q, int buf) {
+    const char* base = smem + buf * kTileBuf + (2 + q) * kTileSlot + wc * 32 * 128;
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      b[nt][0] = *reinterpret_cast<const bf16x8_t*>(base + nt * 2048 + off0);
+      b[nt][1] = *reinterpret_cast<const bf16x8_t*>(base + nt * 2048 + off1);
+    }
+  };
+  auto issueA = [&](int q, int kt, int buf) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, (tile_lds_t*)(smem + buf * kTileBuf + q * kTileSlot + (2 * w + i) * 1024),
+                                               16, offA[q][i], kt * 128, 0, 0);
+  };
+  auto issueB = [&](int q, int kt, int buf) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, (tile_lds_t*)(smem + buf * kTileBuf + (2 + q) * kTileSlot + (2 * w + i) * 1024),
+                                               16, offB[q][i], kt * 128, 0, 0);
+  };
+  TileA a;
+  TileB b0, b1;
+  tile_zero(acc00);
+  tile_zero(acc01);
+  tile_zero(acc11);
+  tile_zero(acc10);
+  const int klast = nk - 1;
+  issueA(0, 0, 0);
+  issueB(0, 0, 0);
+  issueB(1, 0, 0);
+  issueA(1, 0, 0);
+  issueA(0, min(1, klast), 1);
+  issueB(0, min(1, klast), 1);
+  issueB(1, min(1, klast), 1);
+  tile_wait_vm<6>();  // step 0 landed (step 1's A0 / B0 / B1 are the 6 youngest)
+  tile_bar();
+  if (lag) tile_bar();
+  auto step = [&](int kt, auto odd_c) {
+    constexpr int buf = decltype(odd_c)::value ? 1 : 0;
+    // L1
+    readA(a, 0, buf);
+    readB(b0, 0, buf);
+    readB(b1, 1, buf);
+    issueA(1, min(kt + 1, klast), buf ^ 1);
+    tile_wait_vm<8>();
+    tile_wait_lds();
+    tile_bar();
+    // M1
+    if (!PARTIAL || live > 0) {
+      tile_mma(acc00, a, b0);
+      tile_mma(acc01, a, b1);
+    }
+    tile_bar();
+    // L2
+    readA(a, 1, buf);
+    issueA(0, min(kt + 2, klast), buf);
+    issueB(0, min(kt + 2, klast), buf);
+    issueB(1, min(kt + 2, klast), buf);
+    tile_wait_vm<8>();
+    tile_wait_lds();
+    tile_bar();
+    // M2
+    if (!PARTIAL || live > 64) {
+      tile_mma(acc10, a, b0);
+      tile_mma(acc11, a, b1);
+    }
+    tile_bar();
+  };
+  int kt = 0;
+  for (; kt < klast; kt += 2) {
+    step(kt, std::integral_constant<bool, false>{});
+    step(kt + 1, std::integral_constant<bool, true>{});
+  }
+  if (kt == klast) step(kt, std::integral_constant<bool, false>{});
+  tile_wait_vm<0>();  // the clamped re-loads land before the LDS is reused
+  if (!lag) tile_bar();
+}
+
+}  // namespace grag
