@@ -30,6 +30,9 @@ constexpr int RT_KC = 128;    // columns of h / the router matrix staged per ste
 constexpr int RT_LD = RT_KC + 4;  // LDS row stride (floats): 16-byte rows, banks spread over the rows
 constexpr int RT_MAXR = 256;  // logit rows (experts + the shared gate's row) at most
 constexpr int RT_MAXTOP = 16;
+// tokens from which the matrix-core router is taken: up to 128 a workgroup per token is as fast or faster (12 us against 19, 64
+// rows 30 against 43)
+constexpr int ROUTE_MFMA_MIN = 129;
 
 // One token's choice from its logits z [R] (in LDS, overwritten), by SW = 16, 32 or 64 neighbouring lanes (SW >= E, or 64):
 // lane l of them holds the rows l, l + SW, ...
@@ -283,6 +286,70 @@ moe_route_kernel(const T* __restrict__ h, int ld, const float* __restrict__ wr, 
     constexpr int SW = decltype(sw)::value;
     for (int i = threadIdx.x / SW; i < RT_TOK && t0 + i < T_; i += 256 / SW)
       route_select<SW>(lgs + i * (R + 1), E, R, top, ngroups, keep, t0 + i, ids, wts, sgate, rx);
+  };
+  if (E <= 16) select(Lanes<16>());
+  else if (E <= 32) select(Lanes<32>());
+  else select(Lanes<64>());
+}
+
+// The logits on the fp32 matrix cores: a workgroup of 16 waves forms those of 16 tokens, wave w the columns of W that its
+// 32-column steps w, w + 16, ... hold, and the waves' sums meet in LDS.  A step is one 16- or 32-byte load per lane and operand
+// (row lane % 16, columns 8 (lane / 16) .. + 7; the order of a sum is free, so product i takes the lanes' number i), all of a
+// wave's steps independent.  The kernels around it walk W serially: 128 columns between barriers, 16 tokens a workgroup
+// (64 us from 129 to 4096 tokens), or a wave per logit row that reads the router once per token (14 us up to 128).
+// R <= 16 NT.  17 logit rows, width 3584: 64 -> 19 us at 300 tokens, 69 -> 22 at 4096; 64 rows: 151 -> 43 and 173 -> 48.
+template <typename T, int NT>
+__global__ void __launch_bounds__(1024)
+moe_route_mfma_kernel(const T* __restrict__ h, int ld, const float* __restrict__ wr, int W, int E, int R, int top, int ngroups,
+                      int keep, int* __restrict__ ids, float* __restrict__ wts, float* __restrict__ sgate, int T_,
+                      RouteExtra rx) {
+  constexpr int ZL = 16 * NT + 1;
+  __shared__ __attribute__((aligned(16))) float part[16][NT][256];
+  __shared__ float z[RT_TOK * ZL];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, ql = lane & 15, quad = lane >> 4;
+  const int t0 = blockIdx.x * RT_TOK;
+  const T* hp = h + (size_t)min(t0 + ql, T_ - 1) * ld;
+  f32x4_t acc[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) acc[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+  for (int k0 = 32 * wid; k0 < W; k0 += 32 * 16) {
+    const bool ok = k0 + 8 * quad < W;  // (W is a multiple of 8)
+    const int k = ok ? k0 + 8 * quad : 0;
+    float a[8];
+    if constexpr (sizeof(T) == 2) {
+      unpack8(*reinterpret_cast<const bf16x8_t*>(hp + k), a);
+    } else {
+      *reinterpret_cast<f32x4_t*>(a) = *reinterpret_cast<const f32x4_t*>(hp + k);
+      *reinterpret_cast<f32x4_t*>(a + 4) = *reinterpret_cast<const f32x4_t*>(hp + k + 4);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a[i] = ok ? a[i] : 0.f;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const float* wp = wr + (size_t)min(16 * n + ql, R - 1) * W + k;
+      const f32x4_t w[2] = {*reinterpret_cast<const f32x4_t*>(wp), *reinterpret_cast<const f32x4_t*>(wp + 4)};
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], ok ? w[i >> 2][i & 3] : 0.f, acc[n], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4_t*>(&part[wid][n][lane * 4]) = acc[n];
+  __syncthreads();
+  // element x of a block: lane x / 4, number x % 4, i.e. token 4 (lane / 16) + x % 4, logit row lane % 16
+  for (int idx = threadIdx.x; idx < NT * 256; idx += 1024) {
+    const int n = idx >> 8, x = idx & 255;
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) s += part[w][n][x];
+    z[(4 * (x >> 6) + (x & 3)) * ZL + 16 * n + ((x >> 2) & 15)] = s;
+  }
+  __syncthreads();
+  auto select = [&](auto sw) {
+    constexpr int SW = decltype(sw)::value;
+    for (int i = threadIdx.x / SW; i < RT_TOK && t0 + i < T_; i += 1024 / SW)
+      route_select<SW>(z + i * ZL, E, R, top, ngroups, keep, t0 + i, ids, wts, sgate, rx);
   };
   if (E <= 16) select(Lanes<16>());
   else if (E <= 32) select(Lanes<32>());
@@ -1178,6 +1245,21 @@ GRAG_API hipError_t grag_moe_route(const void* h, int ld, const float* wr, int W
   const size_t bytes = ((size_t)(RT_TOK + R) * RT_LD + (size_t)RT_TOK * (R + 1)) * sizeof(float);
   const int vec = W % 8 == 0 && ld % 8 == 0 && (reinterpret_cast<uintptr_t>(h) & 15) == 0 &&
                   (reinterpret_cast<uintptr_t>(wr) & 15) == 0;
+  if (vec && R <= 64 && T_ >= ROUTE_MFMA_MIN) {
+    const dim3 g((T_ + RT_TOK - 1) / RT_TOK);
+#define ROUTE_MFMA(NT)                                                                                                 \
+  DT_DISPATCH(dt, hipLaunchKernelGGL((moe_route_mfma_kernel<T, NT>), g, dim3(1024), 0, st, (const T*)h, ld, wr, W, E, \
+                                     R, top, ngroups, keep, ids, wts, sgate, T_, rx);)
+    if (R <= 16) {
+      ROUTE_MFMA(1)
+    } else if (R <= 32) {
+      ROUTE_MFMA(2)
+    } else {
+      ROUTE_MFMA(4)
+    }
+#undef ROUTE_MFMA
+    return hipGetLastError();
+  }
   if (T_ <= 128) {  // decode rows, short portions
     DT_DISPATCH(dt, hipLaunchKernelGGL(moe_route_rows_kernel<T>, dim3(T_), dim3(256), 0, st, (const T*)h, ld, wr, W, E, R,
                                        top, ngroups, keep, ids, wts, sgate, vec, rx);)
