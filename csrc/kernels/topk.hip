@@ -14,7 +14,13 @@
 // At the end the four lanes of a query merge with two bitonic xor-shuffle
 // rounds (top-K of two sorted lists = elementwise max against the reversed
 // partner list, then a half-cleaner network), so each wave emits one list per
-// query.  The host merges the per-wave partial lists (tiny) with topk.
+// query.  In a flat scan the workgroup's waves merge theirs through LDS (three
+// rounds), and topk_lists_merge_kernel folds the workgroups' lists: a sorted
+// list per thread, then the same network across lanes and waves.  (The lists of
+// all waves through a library sort took 15 launches and 100 us behind a scan of
+// 330 us: 1M x 768, 16 queries, k = 10, 428 -> 323, 20K rows
+// 103 -> 38.)
+// Work items leave a list per wave for grag_topk_merge.
 //
 // Filters (N3c): up to 4 predicates over dictionary-encoded int32 columns
 // (op 1: col == val, op 2: (col & val) != 0 for multi-valued bitset columns)
@@ -24,6 +30,9 @@
 //   flat : blockIdx.x = row chunk, blockIdx.y = query tile (NQT*16 queries)
 //   work : blockIdx.x = work item {row range, NQT*16 query ids} (IVF probes:
 //          rows of one inverted list scanned for the queries that probe it)
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 
 using namespace grag;
@@ -59,6 +68,16 @@ struct TopkParams {
   int64_t* out_i;
 };
 
+// f(0) ... f(N - 1) with compile-time numbers: the lists are register arrays, and a loop that the unroller gives up on (their
+// networks are long) would index them in scratch memory
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(static_cast<F&&>(f));
+  }
+}
+
 template <int K>
 __device__ __forceinline__ void list_insert(float (&v)[K], uint32_t (&id)[K], float x, uint32_t xi) {
   if (x > v[K - 1]) {
@@ -76,15 +95,9 @@ __device__ __forceinline__ void list_insert(float (&v)[K], uint32_t (&id)[K], fl
   }
 }
 
+// the best K of a sorted list and of another in rising order (w)
 template <int K>
-__device__ __forceinline__ void list_merge_xor(float (&v)[K], uint32_t (&id)[K], int mask) {
-  float w[K];
-  uint32_t wi[K];
-#pragma unroll
-  for (int i = 0; i < K; ++i) {
-    w[i] = __shfl_xor(v[K - 1 - i], mask, 64);
-    wi[i] = (uint32_t)__shfl_xor((int)id[K - 1 - i], mask, 64);
-  }
+__device__ __forceinline__ void list_merge(float (&v)[K], uint32_t (&id)[K], const float (&w)[K], const uint32_t (&wi)[K]) {
 #pragma unroll
   for (int i = 0; i < K; ++i) {
     const bool take = w[i] > v[i];
@@ -107,6 +120,18 @@ __device__ __forceinline__ void list_merge_xor(float (&v)[K], uint32_t (&id)[K],
       }
     }
   }
+}
+
+template <int K>
+__device__ __forceinline__ void list_merge_xor(float (&v)[K], uint32_t (&id)[K], int mask) {
+  float w[K];
+  uint32_t wi[K];
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    w[i] = __shfl_xor(v[K - 1 - i], mask, 64);
+    wi[i] = (uint32_t)__shfl_xor((int)id[K - 1 - i], mask, 64);
+  }
+  list_merge<K>(v, id, w, wi);
 }
 
 __device__ __forceinline__ bool row_passes(const TopkParams& p, int64_t row) {
@@ -179,13 +204,13 @@ __global__ __launch_bounds__(64 * NWAVES) void score_topk_kernel(TopkParams p) {
 
   float ls[NQT][KMAX];
   uint32_t lid[NQT][KMAX];
-#pragma unroll
-  for (int qt = 0; qt < NQT; ++qt)
+  static_for<NQT>([&](auto qt) {
 #pragma unroll
     for (int i = 0; i < KMAX; ++i) {
       ls[qt][i] = -INFINITY;
       lid[qt][i] = 0xFFFFFFFFu;
     }
+  });
 
   const int nc = d / 32;
   for (int64_t t0 = r0 + wave * 16; t0 < r1; t0 += 16 * NWAVES) {
@@ -213,41 +238,126 @@ __global__ __launch_bounds__(64 * NWAVES) void score_topk_kernel(TopkParams p) {
         }
       }
     }
-#pragma unroll
+#pragma unroll(NQT * KMAX > 32 ? 1 : 4)
     for (int r = 0; r < 4; ++r) {
       const int64_t row = t0 + 4 * h4 + r;
       const bool ok = row < r1 && row_passes(p, row);
       const uint32_t off = (uint32_t)(row - r0);
-#pragma unroll
-      for (int qt = 0; qt < NQT; ++qt) {
+      static_for<NQT>([&](auto qt) {
         bool okq = ok;
         if (qsel[qt] >= 0 && okq) okq = p.qcols[qsel[qt]][row] == qv[qt];
-        list_insert<KMAX>(ls[qt], lid[qt], okq ? acc[qt][r] : -INFINITY, off);
-      }
+        const float x = r < 2 ? (r == 0 ? acc[qt][0] : acc[qt][1]) : (r == 2 ? acc[qt][2] : acc[qt][3]);
+        list_insert<KMAX>(ls[qt], lid[qt], okq ? x : -INFINITY, off);
+      });
     }
   }
 
-#pragma unroll
-  for (int qt = 0; qt < NQT; ++qt) {
+  static_for<NQT>([&](auto qt) {
     list_merge_xor<KMAX>(ls[qt], lid[qt], 16);
     list_merge_xor<KMAX>(ls[qt], lid[qt], 32);
+  });
+  int lists = NWAVES, mine = wave;  // lists per query of this workgroup, this wave's
+  if (!p.work_rows) {  // the waves' lists into wave 0's, over the query tile's LDS
+    float* lv = reinterpret_cast<float*>(qlds);
+    uint32_t* li_ = reinterpret_cast<uint32_t*>(lv + NWAVES / 2 * NQ * KMAX);
+#pragma unroll 1
+    for (int half = NWAVES / 2; half > 0; half >>= 1) {
+      __syncthreads();
+      if (wave >= half && wave < 2 * half && h4 == 0) {
+        static_for<NQT>([&](auto qt) {
+#pragma unroll
+          for (int i = 0; i < KMAX; ++i) {  // (element-major: 16 lanes in a row)
+            const int o = (((wave - half) * NQT + qt) * KMAX + KMAX - 1 - i) * 16 + li;
+            lv[o] = ls[qt][i];
+            li_[o] = lid[qt][i];
+          }
+        });
+      }
+      __syncthreads();
+      if (wave < half) {
+        static_for<NQT>([&](auto qt) {
+          float w[KMAX];
+          uint32_t wi[KMAX];
+#pragma unroll
+          for (int i = 0; i < KMAX; ++i) {
+            const int o = ((wave * NQT + qt) * KMAX + i) * 16 + li;
+            w[i] = lv[o];
+            wi[i] = li_[o];
+          }
+          list_merge<KMAX>(ls[qt], lid[qt], w, wi);
+        });
+      }
+    }
+    if (wave != 0) return;
+    lists = 1;
   }
   if (h4 != 0) return;
+  static_for<NQT>([&](auto qt) {
+    const int64_t slot = ((slot_base + qt * 16 + li) * lists + mine) * p.k;
 #pragma unroll
-  for (int qt = 0; qt < NQT; ++qt) {
-    const int64_t slot = ((slot_base + qt * 16 + li) * NWAVES + wave) * p.k;
-    for (int i = 0; i < p.k; ++i) {
+    for (int i = 0; i < KMAX; ++i) {
+      if (i >= p.k) continue;
       const bool valid = ls[qt][i] != -INFINITY && lid[qt][i] != 0xFFFFFFFFu;
       const int64_t row = r0 + (int64_t)lid[qt][i];
       p.out_s[slot + i] = ls[qt][i];
       p.out_i[slot + i] = valid ? (p.row_ids ? p.row_ids[row] : row) : -1;
     }
+  });
+}
+
+// The final lists of a flat scan: query q's sorted lists of k are rows (q / G * n + j) * G + q % G, j < n, of ps / pi.
+// grid (nq), 256 threads.
+template <int K>
+__global__ __launch_bounds__(256) void topk_lists_merge_kernel(const float* __restrict__ ps, const int64_t* __restrict__ pi,
+                                                               int n, int G, int k, float* __restrict__ out_s,
+                                                               int64_t* __restrict__ out_i) {
+  __shared__ float lv[4][K];
+  __shared__ uint32_t li[4][K];
+  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t base = (int64_t)(q / G) * n * G + q % G;
+  float v[K];
+  uint32_t id[K];
+#pragma unroll
+  for (int i = 0; i < K; ++i) v[i] = -INFINITY, id[i] = 0;
+  for (int j = tid; j < n; j += 256) {
+    const float* l = ps + (base + (int64_t)j * G) * k;
+    float w[K];
+    uint32_t wi[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      const int t = K - 1 - i;
+      w[i] = t < k ? l[t] : -INFINITY;
+      wi[i] = (uint32_t)(j * k + t);
+    }
+    if (w[K - 1] > v[K - 1]) list_merge<K>(v, id, w, wi);
+  }
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) list_merge_xor<K>(v, id, m);
+  if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) lv[wave][i] = v[i], li[wave][i] = id[i];
+  }
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll
+  for (int i = 0; i < K; ++i) v[i] = lv[lane & 3][i], id[i] = li[lane & 3][i];
+  list_merge_xor<K>(v, id, 1);
+  list_merge_xor<K>(v, id, 2);
+  if (lane != 0) return;
+#pragma unroll
+  for (int i = 0; i < K; ++i) {
+    if (i >= k) break;
+    const bool any = v[i] != -INFINITY;
+    const uint32_t j = id[i] / (uint32_t)k;
+    out_s[(int64_t)q * k + i] = v[i];
+    out_i[(int64_t)q * k + i] = any ? pi[(base + (int64_t)j * G) * k + id[i] % (uint32_t)k] : -1;
   }
 }
 
 template <int NQT, int KMAX>
 int launch_topk(const TopkParams& prm, dim3 grid, hipStream_t stream) {
-  const size_t lds = (size_t)NQT * 16 * prm.d * 2;
+  const size_t merge = (size_t)NWAVES / 2 * NQT * 16 * KMAX * 8;  // the waves' lists, where the query tile was
+  const size_t lds = std::max((size_t)NQT * 16 * prm.d * 2, prm.work_rows ? (size_t)0 : merge);
   static bool attr_set = false;
   if (!attr_set) {
     hipFuncSetAttribute((const void*)score_topk_kernel<NQT, KMAX>,
@@ -291,7 +401,17 @@ void fill_filters(TopkParams& prm, const int32_t* const* fcols, const int32_t* f
 
 GRAG_API int grag_topk_num_waves() { return NWAVES; }
 
-// Flat scan.  Output slots: [nqtiles][nchunks][nqt*16][NWAVES][k].
+// The final top-k of a flat scan's lists (out_s / out_i of grag_score_topk_flat): [nq][k], -1 where fewer rows passed.
+GRAG_API int grag_topk_lists_merge(const float* ps, const int64_t* pi, int n, int G, int nq, int k, float* out_s,
+                                   int64_t* out_i, hipStream_t stream) {
+  if (nq <= 0) return 0;
+  if (n < 1 || G < 1 || k < 1 || k > 32 || (int64_t)n * k >= (1LL << 32)) return (int)hipErrorInvalidValue;
+  if (k <= 16) topk_lists_merge_kernel<16><<<nq, 256, 0, stream>>>(ps, pi, n, G, k, out_s, out_i);
+  else topk_lists_merge_kernel<32><<<nq, 256, 0, stream>>>(ps, pi, n, G, k, out_s, out_i);
+  return (int)hipGetLastError();
+}
+
+// Flat scan.  Output slots: [nqtiles][nchunks][nqt*16][k].
 GRAG_API int grag_score_topk_flat(const void* X, int64_t row_begin, int64_t row_end,
                                   int64_t rows_per_wg, int d, const void* Q, int nq, int k,
                                   int nqt, int kmax, const int32_t* const* fcols,

@@ -11,6 +11,10 @@ from ._lib import call, lib, ptr
 OP_EQ, OP_BITAND = 1, 2
 MAX_FILTERS = 4
 MAX_K = 32
+# 64 queries a workgroup read the rows once for all of them but leave two waves a SIMD for the lists' upkeep: from ~half a
+# million rows the reads win (1M x 768: 64 queries 639 -> 532 us, 128 1220 -> 870), below they do not (100K: 122 against 221)
+NQT4_MIN_ROWS = 1 << 19
+NQT4_MAX_D = 1152  # widest rows of which a workgroup's LDS holds 64 queries
 
 
 @dataclass
@@ -99,12 +103,12 @@ def _kmax(k):
     raise ValueError("k > 32")
 
 
-def _nqt_for(nq, d, kmax):
+def _nqt_for(nq, d, kmax, rows):
     if kmax == 32:
         return 1 if nq <= 16 else 2
     if nq <= 16:
         return 1
-    if nq <= 32 or d > 512:
+    if nq <= 32 or d > NQT4_MAX_D or rows < NQT4_MIN_ROWS:
         return 2
     return 4
 
@@ -129,31 +133,25 @@ def score_topk(X: torch.Tensor, Q: torch.Tensor, k: int, preds=None, bitmap=None
         return (torch.full((nq, k), float("-inf"), device=X.device),
                 torch.full((nq, k), -1, dtype=torch.long, device=X.device))
     kmax = _kmax(k)
-    nqt = _nqt_for(nq, d, kmax)
-    nqtiles = (nq + nqt * 16 - 1) // (nqt * 16)
     rows = N - row_begin
+    nqt = _nqt_for(nq, d, kmax, rows)
+    nqtiles = (nq + nqt * 16 - 1) // (nqt * 16)
     target = max(1, 1024 // nqtiles)
     rows_per_wg = max(128, -(-rows // target))
     rows_per_wg = -(-rows_per_wg // 16) * 16
     nchunks = -(-rows // rows_per_wg)
-    nw = num_waves()
-    slots = nqtiles * nchunks * nqt * 16 * nw
-    out_s = torch.empty(slots * k, dtype=torch.float32, device=X.device)
-    out_i = torch.empty(slots * k, dtype=torch.int64, device=X.device)
+    slots = nqtiles * nchunks * nqt * 16  # a list per workgroup and query
+    part_s = torch.empty(slots * k, dtype=torch.float32, device=X.device)
+    part_i = torch.empty(slots * k, dtype=torch.int64, device=X.device)
     cols, vals, ops, nf = _filter_args(preds)
     qc, nqc, qsel, qval = _qpred_args(qpred)
     Q = Q.contiguous()
     call("grag_score_topk_flat", ptr(X), row_begin, N, rows_per_wg, d, ptr(Q), nq, k, nqt, kmax,
-         cols, vals, ops, nf, ptr(bitmap), ptr(row_ids), qc, nqc, ptr(qsel), ptr(qval), ptr(out_s), ptr(out_i))
-    s = out_s.view(nqtiles, nchunks, nqt * 16, nw * k).permute(0, 2, 1, 3).reshape(nqtiles * nqt * 16, -1)[:nq]
-    i = out_i.view(nqtiles, nchunks, nqt * 16, nw * k).permute(0, 2, 1, 3).reshape(nqtiles * nqt * 16, -1)[:nq]
-    kk = min(k, s.shape[1])
-    bs, sel = s.topk(kk, dim=1)
-    bi = i.gather(1, sel)
-    if kk < k:
-        bs = torch.cat([bs, torch.full((nq, k - kk), float("-inf"), device=X.device)], 1)
-        bi = torch.cat([bi, torch.full((nq, k - kk), -1, dtype=torch.long, device=X.device)], 1)
-    return bs, bi
+         cols, vals, ops, nf, ptr(bitmap), ptr(row_ids), qc, nqc, ptr(qsel), ptr(qval), ptr(part_s), ptr(part_i))
+    out_s = torch.empty(nq, k, dtype=torch.float32, device=X.device)
+    out_i = torch.empty(nq, k, dtype=torch.int64, device=X.device)
+    call("grag_topk_lists_merge", ptr(part_s), ptr(part_i), nchunks, nqt * 16, nq, k, ptr(out_s), ptr(out_i))
+    return out_s, out_i
 
 
 def score_topk_work(X, Q, k, work_rows: torch.Tensor, work_q: torch.Tensor, nqt: int, preds=None,
