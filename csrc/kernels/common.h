@@ -84,6 +84,30 @@ __device__ __forceinline__ bf16x8_t pack8(const float* f) {
   return v;
 }
 
+// GELU with the normal distribution, x * Phi(x): Phi(-a) = exp2(P(a)) for a >= 0, P the degree-10 minimax fit (Lawson
+// iteration, relative weight 1 up to a = 2 and falling to 1e-4 at 6) of log2 of that tail on [0, 5.5]; its leading
+// coefficient is negative and P falls on, so larger a end in 0.  The upper half is 1 - Phi(-a).  Against 64 bits over
+// [-8, 8]: at most 3.8e-7 in absolute value, where 0.5 x (1 + erff(x / sqrt 2)) has 4.5e-7, and in [-5, -3] 1.1e-5 of
+// the value, where that form's 1 + erf cancels to 4.8e-2.  One hardware exponential and ten fmas without a branch:
+// erff takes both of its branches in nearly every wave.  Encoder's 24000 x 3072 x 768 product with bias and GELU in the
+// epilogue (73.7 M values): 212 us with erff, 182 with this, 142 without an activation; 4000 rows 38.8 -> 30.7 (26.7).
+// inf -> inf, -inf -> NaN (-inf * 0), NaN -> NaN as in that form.
+__device__ __forceinline__ float gelu_erf(float x) {
+  const float a = fabsf(x);
+  float p = fmaf(-3.7635938809899017e-08f, a, 1.035111267810862e-06f);
+  p = fmaf(p, a, -1.237917513208231e-05f);
+  p = fmaf(p, a, 8.218956645578146e-05f);
+  p = fmaf(p, a, -0.00029183205333538353f);
+  p = fmaf(p, a, 1.169378992926795e-05f);
+  p = fmaf(p, a, 0.006946496199816465f);
+  p = fmaf(p, a, -0.05244869366288185f);
+  p = fmaf(p, a, -0.4592163562774658f);
+  p = fmaf(p, a, -1.1511049270629883f);
+  p = fmaf(p, a, -1.f);
+  const float q = __builtin_amdgcn_exp2f(p);
+  return x * (x < 0.f ? q : 1.f - q);
+}
+
 // ---- wave / block reductions (wave64) ----
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

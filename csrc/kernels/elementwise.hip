@@ -14,9 +14,6 @@ namespace {
 constexpr int kThreads = 256;
 
 __device__ __forceinline__ float silu(float x) { return x / (1.f + __expf(-x)); }
-__device__ __forceinline__ float gelu_erf(float x) {
-  return 0.5f * x * (1.f + erff(x * 0.70710678118654752f));
-}
 // GPT-2 "gelu_new": 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3))),
 // tanh(u) = 1 - 2 / (1 + exp(2u)) (saturates correctly at +-inf)
 __device__ __forceinline__ float gelu_tanh(float x) {

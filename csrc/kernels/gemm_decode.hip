@@ -63,14 +63,13 @@ __device__ __forceinline__ void static_for(F&& f) {
 enum { ACT_NONE = 0, ACT_GELU = 1, ACT_GELU_TANH = 3 };
 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.f + __expf(-x)); }
-__device__ __forceinline__ float gelu_erf_f(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 __device__ __forceinline__ float gelu_tanh_f(float x) {
   const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
   return 0.5f * x * (2.f - 2.f * __builtin_amdgcn_rcpf(1.f + __expf(2.f * u)));
 }
 template <int ACT>
 __device__ __forceinline__ float act_f(float x) {
-  if constexpr (ACT == ACT_GELU) return gelu_erf_f(x);
+  if constexpr (ACT == ACT_GELU) return gelu_erf(x);
   else if constexpr (ACT == ACT_GELU_TANH) return gelu_tanh_f(x);
   else return x;
 }
