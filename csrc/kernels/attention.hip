@@ -154,7 +154,7 @@ __device__ __forceinline__ void glds16_s(const void* sbase, uint32_t voff, void*
 }
 
 template <int D, int NW, bool PAGED>
-__global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(AttnParams p) {
+__global__ __launch_bounds__(64 * NW, D <= 64 && NW == 4 ? 4 : 1) void attn_fwd_kernel(AttnParams p) {
   constexpr int CPR = D / 8;      // 16-B chunks per K/V row
   constexpr int RB = 2 * D;       // bytes per K/V row
   constexpr int NC = D / 32;      // k-chunks of the QK^T product
@@ -206,30 +206,60 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(AttnParams p) {
 #pragma unroll
   for (int n = 0; n < ND; ++n) o[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
+  // one 16-B chunk of K and of V of a tile
+  auto load_kv = [&](int kt0, int c, bf16x8_t& kk, bf16x8_t& vv) {
+    const int j = kt0 + c / CPR, ch = c % CPR;
+    kk = vv = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+    if (j < kv_hi) {
+      size_t off;
+      if constexpr (PAGED) {
+        int blk = p.block_tables[(size_t)seq * p.bt_stride + j / p.BS];
+        if (!index_ok(blk, p.nblocks, ERR_BLOCK_PREFILL)) blk = 0;
+        off = (((size_t)blk * p.Hkv + kvh) * p.BS + (j % p.BS)) * D + ch * 8;
+      } else {
+        off = (size_t)(q0 + j) * p.kv_stride + (size_t)kvh * D + ch * 8;
+      }
+      kk = *reinterpret_cast<const bf16x8_t*>(p.k + off);
+      vv = *reinterpret_cast<const bf16x8_t*>(p.v + off);
+    }
+  };
+  auto put_kv = [&](int c, bf16x8_t kk, bf16x8_t vv) {  // -> swizzled LDS image
+    const int r = c / CPR, ch = c % CPR;
+    *reinterpret_cast<bf16x8_t*>(k_lds + r * RB + ((ch ^ kswz<D>(r)) << 4)) = kk;
+    *reinterpret_cast<bf16x8_t*>(v_lds + r * RB + ((ch ^ vswz<D>(r)) << 4)) = vv;
+  };
+  // with few chunks a thread (1 or 2), a tile waits in registers while the tile before it is computed, so its way from
+  // memory is off the path; at 4 and more the registers would cost waves (or spill, D = 128).  With the exponential
+  // below as the bare instruction (exp2f's denormal guard was a fifth of a tile's vector instructions, and what it
+  // guards, p < 2^-126, is nothing beside the row's largest p = 1) and the output kept out of the accumulation
+  // registers (launch bounds), the vector issue that bounds this kernel falls from 360 to 250 instructions a tile:
+  // 128 sequences of 60-320 rows, 12 heads, D = 64 86 -> 61 us, D = 32 57 -> 43; 64 of 500-512 160 -> 129, 127 -> 113
+  constexpr int NV = KT * CPR / (64 * NW);
+  constexpr bool kAhead = NV <= 2;
+  bf16x8_t ka[kAhead ? NV : 1], va[kAhead ? NV : 1];
+  if constexpr (kAhead) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) load_kv(kv_lo, threadIdx.x + i * 64 * NW, ka[i], va[i]);
+  }
   for (int kt0 = kv_lo; kt0 < kv_hi; kt0 += KT) {
     __syncthreads();  // previous tile fully consumed
-    // cooperative K/V tile load: global (16 B/lane) -> swizzled LDS image
-    for (int c = threadIdx.x; c < KT * CPR; c += 64 * NW) {
-      const int r = c / CPR, ch = c % CPR;
-      const int j = kt0 + r;
-      bf16x8_t kk = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-      bf16x8_t vv = kk;
-      if (j < kv_hi) {
-        size_t off;
-        if constexpr (PAGED) {
-          int blk = p.block_tables[(size_t)seq * p.bt_stride + j / p.BS];
-          if (!index_ok(blk, p.nblocks, ERR_BLOCK_PREFILL)) blk = 0;
-          off = (((size_t)blk * p.Hkv + kvh) * p.BS + (j % p.BS)) * D + ch * 8;
-        } else {
-          off = (size_t)(q0 + j) * p.kv_stride + (size_t)kvh * D + ch * 8;
-        }
-        kk = *reinterpret_cast<const bf16x8_t*>(p.k + off);
-        vv = *reinterpret_cast<const bf16x8_t*>(p.v + off);
+    if constexpr (kAhead) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) put_kv(threadIdx.x + i * 64 * NW, ka[i], va[i]);
+    } else {
+      for (int c = threadIdx.x; c < KT * CPR; c += 64 * NW) {
+        bf16x8_t kk, vv;
+        load_kv(kt0, c, kk, vv);
+        put_kv(c, kk, vv);
       }
-      *reinterpret_cast<bf16x8_t*>(k_lds + r * RB + ((ch ^ kswz<D>(r)) << 4)) = kk;
-      *reinterpret_cast<bf16x8_t*>(v_lds + r * RB + ((ch ^ vswz<D>(r)) << 4)) = vv;
     }
     __syncthreads();
+    if constexpr (kAhead) {
+      if (kt0 + KT < kv_hi) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) load_kv(kt0 + KT, threadIdx.x + i * 64 * NW, ka[i], va[i]);
+      }
+    }
 
     // S^T = K Q^T for 4 key sub-tiles of 16
     f32x4_t s[4];
@@ -269,7 +299,7 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(AttnParams p) {
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
     const float m_new = fmaxf(m, tmax);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = exp2f(m - m_use);
+    const float alpha = __builtin_amdgcn_exp2f(m - m_use);
     m = m_new;
     lsum *= alpha;
 #pragma unroll
@@ -279,7 +309,7 @@ __global__ __launch_bounds__(64 * NW) void attn_fwd_kernel(AttnParams p) {
     for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        pr[t][r] = exp2f(s[t][r] - m_use);
+        pr[t][r] = __builtin_amdgcn_exp2f(s[t][r] - m_use);
         lsum += pr[t][r];
       }
 

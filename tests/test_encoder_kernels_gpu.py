@@ -29,3 +29,20 @@ def test_layernorm_rows(H, T, bias, res):
         assert torch.equal(r1, s)
         ref = torch.nn.functional.layer_norm(s.double(), (H,), ga.double(), be.double(), 1e-12)
         assert ((y - ref).abs() <= ref.abs() * 2 ** -8 + 2e-5).all()
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("lens", [[1, 63, 64, 65], [17, 128, 129, 2, 200], [15, 16, 3]])
+def test_varlen_attention_edges(D, causal, lens):
+    from githubrepostorag_amd.ops.attention import varlen_attention, varlen_attention_ref
+
+    H = 3
+    st = torch.tensor([0] + lens).cumsum(0).int().to(dev)
+    sl = torch.tensor(lens).int().to(dev)
+    q = torch.randn(int(st[-1]), 3 * H * D, generator=torch.Generator(device=dev).manual_seed(D), device=dev).to(bf)
+    q[:, : H * D] *= 3  # some rows' softmax close to one key
+    y = varlen_attention(q, st, sl, max(lens), H, D, D ** -0.5, causal).float().cpu()
+    r = varlen_attention_ref(q.float().cpu(), st.cpu(), H, D, D ** -0.5, causal)
+    # weights and result rounded to bf16 of 8 bits (2^-8 of a value at most, each, relative to the largest value a row can hold)
+    assert (y - r).abs().max() <= 2 * 2 ** -8 * q[:, 2 * H * D:].float().abs().max().item() + 1e-5
