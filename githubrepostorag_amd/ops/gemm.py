@@ -197,10 +197,24 @@ OWN_SLACK = float(os.environ.get("GRAG_OWN_SLACK", "1.06"))  # beyond the 3-5 % 
 PREFILL_MIN_M = 257  # above one 256-row tile: the prefill regime (decode batches use plan())
 
 
+def unmeasured_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
+    """(ksplit, sk) of the owned kernel for a plain GEMM whose (N, K) the sweep's table does not have; None: the library.
+
+    Owned, whole tiles, where the contraction is short (K <= 1024) and the tiles are more than one round of the chip:
+    launches back to back over 8 shapes of N 384-3072, K 384-768 at 277-24000 rows, library / owned there is 1.19 in the
+    median of 13 points (0.90-1.48: 2304 x 768 at 7300 rows 64 -> 43 us, at 24000 106 -> 95, at 8192 38 -> 42); with fewer tiles the
+    library's smaller ones win (0.3-1.0).  No stream-K there: a part's slab out and in costs more than the K steps it
+    saves (3072 x 768 at 24000 rows: 149 us, whole tiles 124).  Deeper contractions are level in the median (0.94-1.05)
+    and stay."""
+    if (N, K, 0) in _prefill_table() or K > 1024 or max(M, N) * K >= 1 << 30:
+        return None
+    return (1, 0) if -(-M // 256) * -(-N // 256) > _num_cus() else None
+
+
 def schedule(M: int, N: int, K: int, silu: bool = False) -> tuple[int, int]:
     """(ksplit, sk) the owned kernel runs a shape with when the caller does not pin one."""
     if M >= PREFILL_MIN_M:
-        p = prefill_plan(M, N, K, silu)
+        p = prefill_plan(M, N, K, silu) or (None if silu else unmeasured_plan(M, N, K))
         if p is not None:
             return p
     return plan(M, N, K)

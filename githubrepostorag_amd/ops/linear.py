@@ -18,7 +18,8 @@ A/B in scripts/bench_gemm.py:
 * larger M (prefill, encoder batches): the owned tile kernel wherever the
   dense M sweep of scripts/sweep_prefill_gemm.py measured it faster
   (``gemm.prefill_plan``; e.g. Qwen2-7B down_proj at the bench's ~7.1K-row
-  prefill steps: 771 vs 1131 us), else hipBLASLt through
+  prefill steps: 771 vs 1131 us) and, for shapes outside that sweep, wherever
+  ``gemm.unmeasured_plan`` places it, else hipBLASLt through
   ``torch.nn.functional.linear`` — the library is used only for plain
   (epilogue-free / bias-only) GEMMs; everything fused around them
   (bias+RoPE+KV store, SiLU*mul, bias+GELU, bias+residual+LayerNorm,
@@ -32,6 +33,7 @@ import os
 from pathlib import Path
 
 import torch
+from torch.autograd import forward_ad as fwAD
 
 from . import gemm as _tile
 from ._lib import call, lib, ptr
@@ -310,10 +312,18 @@ def kernel_for(M: int, N: int, K: int, tile_ok: bool = True, dev: torch.device |
         return "skinny"
     if K % 16 == 0 and N % 4 == 0 and use_stream(M, N, K) and stream_ready:
         return "stream"
+    if tile_ok and _tile.unmeasured_plan(M, N, K) is not None and (dev is None or _tile.capture_ok(dev, M, N, K)):
+        return "tile_prefill"
     return "library"
 
 
 OWNED_KINDS = ("decode", "tile", "tile_prefill", "skinny", "stream")
+
+
+def _differentiated(*ts) -> bool:
+    """A gradient is recorded through one of the tensors, or a forward-mode level is open: the library's product has
+    derivatives, the owned kernel has none."""
+    return fwAD._current_level >= 0 or (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts))
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> torch.Tensor:
@@ -336,7 +346,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> t
             return _tile.gemm(x, w, b)
         if kind == "tile_prefill":
             p = _tile.prefill_plan(M, N, K)
-            return _tile.gemm(x, w, b, ksplit=p[0], sk=p[1])
+            if p is not None:
+                return _tile.gemm(x, w, b, ksplit=p[0], sk=p[1])
+            if not _differentiated(x, w, b) and (b is None or (b.dtype == x.dtype and b.is_contiguous() and b.numel() == N)):
+                p = _tile.unmeasured_plan(M, N, K)
+                return _tile.gemm(x, w, b, ksplit=p[0], sk=p[1])
+            return torch.nn.functional.linear(x, w, b)
         if kind == "splitk":
             return gemm_splitk(x, w, b, splitk_parts(M, N, K))
         if kind == "skinny":
