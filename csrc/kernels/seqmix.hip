@@ -24,15 +24,21 @@ template <> __device__ __forceinline__ void stf<float>(float* p, float v) { *p =
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + __expf(-x)); }
 __device__ __forceinline__ float sigmoid_acc(float x) { return 1.f / (1.f + expf(-x)); }
 __device__ __forceinline__ float silu_acc(float x) { return x / (1.f + expf(-x)); }
-// tanh in fp32 to a few ulp: (1 - e^-2|x|) / (1 + e^-2|x|), a short odd series below 0.02 where that form cancels
+// tanh in fp32 to a few ulp: (1 - e^-2|x|) / (1 + e^-2|x|), a short odd series below 0.02 where that form cancels.
+// The exponential is the bare instruction with its argument's rounding put back; the quotient (divisor in [1, 2]) is a
+// reciprocal with one correction step instead of the scaled IEEE division.
 __device__ __forceinline__ float tanh_acc(float x) {
   const float a = fabsf(x);
-  if (a < 0.02f) {
-    const float x2 = x * x;
-    return x * (1.f + x2 * (-0.33333334f + x2 * 0.13333334f));
-  }
-  const float t = expf(-2.f * a);
-  return copysignf((1.f - t) / (1.f + t), x);
+  const float x2 = x * x;
+  const float small = x * (1.f + x2 * (-0.33333334f + x2 * 0.13333334f));
+  const float h = -2.885390043258667f * a;                             // -2 / ln 2, its first 24 bits
+  const float l = fmaf(-2.885390043258667f, a, -h) - 3.8519259e-8f * a;  // the product's rounding and the rest of it
+  float t = __builtin_amdgcn_exp2f(h);
+  t = fmaf(t, a < 40.f ? 0.6931472f * l : 0.f, t);
+  const float n = 1.f - t, d = 1.f + t, rc = __builtin_amdgcn_rcpf(d);
+  float q = n * rc;
+  q = fmaf(fmaf(-d, q, n), rc, q);
+  return a < 0.02f ? small : copysignf(q, x);
 }
 
 // ------------------------------------------------------------------------------------------------ embedding
@@ -74,29 +80,69 @@ __global__ void dyt_residual_kernel(const T* __restrict__ y, float a1, const flo
   }
 }
 
-// H % 4 == 0: four consecutive elements per thread (16-byte loads of the stream and of the norm vectors)
 template <typename T>
-__global__ void dyt_residual_vec_kernel(const T* __restrict__ y, float a1, const float* __restrict__ w1,
-                                        const float* __restrict__ b1, float* __restrict__ resid,
-                                        const float* __restrict__ add_rows, const float* __restrict__ add_vec,
-                                        float a2, const float* __restrict__ w2, const float* __restrict__ b2,
-                                        T* __restrict__ out, int H) {
-  const size_t base = (size_t)blockIdx.x * H;
+__device__ __forceinline__ f32x4_t ld4(const T* p) {
+  if constexpr (sizeof(T) == 2) {
+    const bf16x4_t v = *reinterpret_cast<const bf16x4_t*>(p);
+    return f32x4_t{bits2f(v[0]), bits2f(v[1]), bits2f(v[2]), bits2f(v[3])};
+  } else {
+    return *reinterpret_cast<const f32x4_t*>(p);
+  }
+}
+template <typename T>
+__device__ __forceinline__ void st4(T* p, const f32x4_t& v) {
+  if constexpr (sizeof(T) == 2)
+    *reinterpret_cast<bf16x4_t*>(p) = bf16x4_t{f2bits(v[0]), f2bits(v[1]), f2bits(v[2]), f2bits(v[3])};
+  else
+    *reinterpret_cast<f32x4_t*>(p) = v;
+}
+
+// The same, H a multiple of 4 and every pointer aligned: four consecutive elements per thread and row, R rows of the
+// stream a thread, so that the norm vectors (four fp32 numbers an element beside its twelve bytes of stream) are read
+// once for them.  grid (ceil(T / R), ceil(H / 1024)): row blockIdx.x + k gridDim.x.  Bound by its 12 bytes an element of
+// stream at many rows (the accurate tanh twice an element was as long as they): with four 2-byte accesses a thread and the
+// scaled division 8192 x 3584 83 us, now 60; 1187 x 3584 14.0 -> 10.7, 64 x 3584 3.5 -> 3.0.
+template <typename T, int R>
+__global__ void __launch_bounds__(256)
+dyt_residual_vec_kernel(const T* __restrict__ y, float a1, const float* __restrict__ w1, const float* __restrict__ b1,
+                        float* __restrict__ resid, const float* __restrict__ add_rows, const float* __restrict__ add_vec,
+                        float a2, const float* __restrict__ w2, const float* __restrict__ b2, T* __restrict__ out, int T_,
+                        int H) {
   const int i = blockIdx.y * 1024 + threadIdx.x * 4;
   if (i >= H) return;
-  f32x4_t x = *reinterpret_cast<const f32x4_t*>(resid + base + i);
-  if (y != nullptr) {
-    const f32x4_t w = *reinterpret_cast<const f32x4_t*>(w1 + i), b = *reinterpret_cast<const f32x4_t*>(b1 + i);
+  const f32x4_t zero = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  f32x4_t x[R], yv[R], rv[R];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] += tanh_acc(a1 * ldf(y + base + i + e)) * w[e] + b[e];
+  for (int k = 0; k < R; ++k) {
+    const int t = blockIdx.x + k * gridDim.x;
+    const size_t at = (size_t)(R == 1 ? t : min(t, T_ - 1)) * H + i;
+    x[k] = *reinterpret_cast<const f32x4_t*>(resid + at);
+    yv[k] = y != nullptr ? ld4(y + at) : zero;
+    rv[k] = add_rows != nullptr ? *reinterpret_cast<const f32x4_t*>(add_rows + at) : zero;
   }
-  if (add_rows != nullptr) x += *reinterpret_cast<const f32x4_t*>(add_rows + base + i);
-  if (add_vec != nullptr) x += *reinterpret_cast<const f32x4_t*>(add_vec + i);
-  if (y != nullptr || add_rows != nullptr || add_vec != nullptr) *reinterpret_cast<f32x4_t*>(resid + base + i) = x;
-  if (out != nullptr) {
-    const f32x4_t w = *reinterpret_cast<const f32x4_t*>(w2 + i), b = *reinterpret_cast<const f32x4_t*>(b2 + i);
+  const f32x4_t w1v = y != nullptr ? *reinterpret_cast<const f32x4_t*>(w1 + i) : zero;
+  const f32x4_t b1v = y != nullptr ? *reinterpret_cast<const f32x4_t*>(b1 + i) : zero;
+  const f32x4_t av = add_vec != nullptr ? *reinterpret_cast<const f32x4_t*>(add_vec + i) : zero;
+  const f32x4_t w2v = out != nullptr ? *reinterpret_cast<const f32x4_t*>(w2 + i) : zero;
+  const f32x4_t b2v = out != nullptr ? *reinterpret_cast<const f32x4_t*>(b2 + i) : zero;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) stf(out + base + i + e, tanh_acc(a2 * x[e]) * w[e] + b[e]);
+  for (int k = 0; k < R; ++k) {
+    const int t = blockIdx.x + k * gridDim.x;
+    if (R > 1 && t >= T_) break;
+    const size_t at = (size_t)t * H + i;
+    if (y != nullptr) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[k][e] += tanh_acc(a1 * yv[k][e]) * w1v[e] + b1v[e];
+    }
+    if (add_rows != nullptr) x[k] += rv[k];
+    if (add_vec != nullptr) x[k] += av;
+    if (y != nullptr || add_rows != nullptr || add_vec != nullptr) *reinterpret_cast<f32x4_t*>(resid + at) = x[k];
+    if (out != nullptr) {
+      f32x4_t o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = tanh_acc(a2 * x[k][e]) * w2v[e] + b2v[e];
+      st4(out + at, o);
+    }
   }
 }
 
@@ -1470,9 +1516,19 @@ GRAG_API hipError_t grag_dyt_residual(const void* y, float a1, const float* w1, 
                                       const float* b2, void* out, int T_, int H, int dt, hipStream_t st) {
   if (T_ <= 0) return hipSuccess;
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (H % 4 == 0 && al16(resid) && al16(w1) && al16(b1) && al16(w2) && al16(b2) && al16(add_rows) && al16(add_vec)) {
-    DT_DISPATCH(dt, hipLaunchKernelGGL(dyt_residual_vec_kernel<T>, dim3(T_, (H + 1023) / 1024), dim3(256), 0, st,
-                                       (const T*)y, a1, w1, b1, resid, add_rows, add_vec, a2, w2, b2, (T*)out, H);)
+  if (H % 4 == 0 && al16(y) && al16(out) && al16(resid) && al16(w1) && al16(b1) && al16(w2) && al16(b2) && al16(add_rows) &&
+      al16(add_vec)) {
+#define DYT_VEC(R)                                                                                                        \
+  hipLaunchKernelGGL((dyt_residual_vec_kernel<T, R>), dim3((T_ + R - 1) / R, (H + 1023) / 1024), dim3(256), 0, st,        \
+                     (const T*)y, a1, w1, b1, resid, add_rows, add_vec, a2, w2, b2, (T*)out, T_, H)
+    DT_DISPATCH(dt, {
+      if ((long)((T_ + 3) / 4) * ((H + 1023) / 1024) >= DYT_ROWS_MIN) {
+        DYT_VEC(4);
+      } else {
+        DYT_VEC(1);
+      }
+    })
+#undef DYT_VEC
     return hipGetLastError();
   }
   DT_DISPATCH(dt, hipLaunchKernelGGL(dyt_residual_kernel<T>, dim3(T_, (H + 1023) / 1024), dim3(256), 0, st, (const T*)y, a1, w1, b1,
@@ -1520,6 +1576,9 @@ hipError_t sink_prefill_launch(const void* q, const void* k, const void* v, void
                                const int* q_start, const int* ctx_len, const float* sinks, int nseq, int max_q_len, int H, int G,
                                int d, float scale, float out_scale, int nblocks, const float* hscale, const void* hgate,
                                int gate_ld, int chunk, int window, float softcap, int keep, hipStream_t st);
+// From this many workgroups at four rows a thread they are taken; fewer leave the chip short of loads in flight (1187 x 1536:
+// 6.4 us with one row, 8.7 with four)
+constexpr long DYT_ROWS_MIN = 2048;
 }  // namespace grag
 
 static int sa_key_tile(int d, int vd, size_t* bytes) {
