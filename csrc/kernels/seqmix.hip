@@ -226,16 +226,18 @@ __global__ void rope_vnorm_store_kernel(const T* __restrict__ proj, int ld, int 
   }
 }
 
-// The same in 16-byte accesses (bf16; d, vd and rd multiples of 16, d <= 256, halves rotated, values without RMS division):
+// The same in 16-byte accesses (bf16; d, vd and rd multiples of 16, d <= 256, halves rotated; vnorm: values divided by RMS):
 // a lane owns 16 elements of a head -- 8 of the first rotated half and the 8 they are paired with, or 16 consecutive ones
 // past the rotated part -- and LG lanes a head, so a head's sum of squares stays inside LG lanes.
 // grid (ceil(T (H + 2 G) LG / 256)), 256 threads: (token, head) pairs in a row, q heads, then k heads, then v heads.
+// Bound by bandwidth at many tokens: 8192 tokens of 28 + 4 + 4 heads of 128 with value norms 108 us in 2-byte accesses, a
+// wave a head, 26 here; 1187 of 12 + 2 + 2 9.3 -> 4.1; 64 of 36 3.6 -> 3.1.
 template <int LG>
 __global__ void __launch_bounds__(256)
 rope_store_vec_kernel(const bf16* __restrict__ proj, int ld, int qoff, int koff, int voff, const int* __restrict__ positions,
                       const float* __restrict__ table, int table_rows, const int* __restrict__ slot_mapping,
                       bf16* __restrict__ q_out, bf16* __restrict__ k_cache, bf16* __restrict__ v_cache, int T_, int H, int G,
-                      int d, int vd, int rd, int BS, long nslots, float eps, const float* __restrict__ bias,
+                      int d, int vd, int rd, int BS, long nslots, float eps, bool vnorm, const float* __restrict__ bias,
                       const float* __restrict__ qw, const float* __restrict__ kw) {
   const int nh = H + 2 * G;
   const long pair = ((long)blockIdx.x * 256 + threadIdx.x) / LG;
@@ -284,6 +286,13 @@ rope_store_vec_kernel(const bf16* __restrict__ proj, int ld, int qoff, int koff,
     for (int e = 0; e < 8; ++e) {
       a[e] *= r * nw[i0 + e];
       b[e] *= r * nw[i1 + e];
+    }
+  } else if (isv && vnorm) {
+    const float r = 1.f / sqrtf(ss / (float)n + eps);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      a[e] *= r;
+      b[e] *= r;
     }
   }
   if (rot) {
@@ -1544,7 +1553,7 @@ GRAG_API hipError_t grag_rope_vnorm_store(const void* proj, int ld, int qoff, in
   if (T_ <= 0) return hipSuccess;
   if (H + 2 * G > 4 * 65535) return hipErrorInvalidValue;
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  if (dt == 0 && flags == 2 && d % 16 == 0 && vd % 16 == 0 && rd % 16 == 0 && d <= 256 && vd <= 256 && ld % 8 == 0 &&
+  if (dt == 0 && !(flags & 1) && d % 16 == 0 && vd % 16 == 0 && rd % 16 == 0 && d <= 256 && vd <= 256 && ld % 8 == 0 &&
       qoff % 8 == 0 && koff % 8 == 0 && voff % 8 == 0 && al16(proj) && al16(q_out) && al16(k_cache) && al16(v_cache) &&
       al16(table) && al16(bias)) {
     const int units = (d > vd ? d : vd) / 16;
@@ -1554,7 +1563,7 @@ GRAG_API hipError_t grag_rope_vnorm_store(const void* proj, int ld, int qoff, in
 #define ROPE_VEC(L)                                                                                                       \
   hipLaunchKernelGGL(rope_store_vec_kernel<L>, vgrid, dim3(256), 0, st, (const bf16*)proj, ld, qoff, koff, voff,          \
                      positions, table, table_rows, slot_mapping, (bf16*)q_out, (bf16*)k_cache, (bf16*)v_cache, T_, H, G,  \
-                     d, vd, rd, BS, nslots, eps, bias, qw, kw)
+                     d, vd, rd, BS, nslots, eps, !(flags & 2), bias, qw, kw)
     if (LG == 1) ROPE_VEC(1);
     else if (LG == 2) ROPE_VEC(2);
     else if (LG == 4) ROPE_VEC(4);

@@ -50,3 +50,26 @@ def test_dyt_residual_special():
     v = r.cpu()[0]
     assert v[2].isnan() and v[[0, 1, 3, 5, 6]].tolist() == [1.0, -1.0, 0.0, -1.0, 1.0]
     assert abs(v[4].item() - 1e-30) < 1e-36 and abs(v[7].item() - 0.0199973340) < 1e-8
+
+
+@pytest.mark.parametrize("d,vd,rd,H,G", [(16, 32, 16, 3, 1), (128, 128, 128, 4, 2), (64, 128, 32, 2, 1), (128, 64, 0, 2, 2), (256, 256, 64, 1, 1)])
+@pytest.mark.parametrize("T", [1, 37])
+def test_rope_store_value_norm(d, vd, rd, H, G, T):
+    from githubrepostorag_amd.ops.elementwise import rope_table, rope_vnorm_store
+
+    g = torch.Generator().manual_seed(d + vd + T)
+    ld = (H + G) * d + G * vd + 8
+    p, pos = rnd(g, T, ld).to(bf), torch.randint(0, 90, (T,), generator=g).int()
+    p[0, (H + G) * d:] = 0  # a value of zero: eps alone under the root
+    tab = rope_table(90, rd, 1e4) if rd else None
+    slots = torch.randperm(T + 16, generator=g)[:T].int()
+    slots[T // 2] = -1
+    outs = []
+    for dv in ("cpu", dev):
+        kc, vc = torch.zeros(4, G, 16, d, dtype=bf, device=dv), torch.zeros(4, G, 16, vd, dtype=bf, device=dv)
+        q = rope_vnorm_store(p.to(dv), 0, H * d, (H + G) * d, pos.to(dv), None if tab is None else tab.to(dv), slots.to(dv), kc, vc,
+                             H, G, d, vd, rd, 1e-6)
+        outs.append([t.float().cpu() for t in (q, kc, vc)])
+    for a, b in zip(*outs):
+        # both round once from fp32: half a unit each way, plus a rotation's cancellation in fp32
+        assert ((a - b).abs() <= a.abs() * 2 ** -7 + 1e-5).all()
