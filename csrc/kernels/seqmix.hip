@@ -1370,6 +1370,52 @@ gated_rmsnorm_vec_kernel(const float* __restrict__ x, const float* __restrict__ 
     *reinterpret_cast<f32x4_t*>(dst) = v;
 }
 
+// and for wider groups (the same alignment, 256 < N <= 8192): a workgroup a group, its values and gates kept in registers
+// between the sum and the product, V accesses of four columns a thread.  grid (T, groups).  Bound by its 8 bytes an element;
+// the general form reads rows and gates twice in scalar accesses and gates twice: 8192 x 3584 65 -> 47 us, 4096 x 8 groups
+// of 896 77 -> 48 (one wave a group, 14 accesses), 64 x 3584 6.9 -> 4.3.
+template <typename T, int V>
+__global__ void __launch_bounds__(256)
+gated_rmsnorm_row_kernel(const float* __restrict__ x, const float* __restrict__ w, const T* __restrict__ proj, int ld, int goff,
+                         T* __restrict__ out, int out_ld, int N, float eps, float out_scale, int silu_gate) {
+  __shared__ float red[4];
+  const int t = blockIdx.x, c0 = blockIdx.y * N;
+  const float* xr = x + (size_t)t * N * gridDim.y + c0;
+  const T* gr = proj + (size_t)t * ld + goff + c0;
+  const bool first = silu_gate & 2;
+  f32x4_t v[V], gt[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int i = (threadIdx.x + k * blockDim.x) * 4;
+    v[k] = gt[k] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (i < N) {
+      v[k] = *reinterpret_cast<const f32x4_t*>(xr + i);
+      gt[k] = ld4(gr + i);
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < V; ++k)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      gt[k][e] = (silu_gate & 1) ? silu_acc(gt[k][e]) : sigmoid_acc(gt[k][e]);
+      const float u = first ? v[k][e] * gt[k][e] : v[k][e];
+      ss = fmaf(u, u, ss);
+    }
+  ss = block_sum(ss, red);
+  const float r = out_scale / sqrtf(ss / (float)N + eps);
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int i = (threadIdx.x + k * blockDim.x) * 4;
+    if (i >= N) break;
+    const f32x4_t wv = w ? *reinterpret_cast<const f32x4_t*>(w + c0 + i) : f32x4_t{1.f, 1.f, 1.f, 1.f};
+    f32x4_t o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = v[k][e] * r * wv[e] * gt[k][e];
+    st4(out + (size_t)t * out_ld + c0 + i, o);
+  }
+}
+
 // ------------------------------------------------------------------------------------------------ minGRU
 // z = sigmoid(pz + bz), u = px + bx, c = u >= 0 ? u + 1/2 : sigmoid(u); S_t = (1 - z) S_(t-1) + z c;
 // out = S_t * silu(pg).  grid (ceil(W / 256), nseq): one thread per channel walks the launch's tokens in order.
@@ -1520,6 +1566,9 @@ GRAG_API hipError_t grag_embed_f32(const int* ids, const void* table, float* out
   return hipGetLastError();
 }
 
+// From this many workgroups at four rows a thread they are taken; fewer leave the chip short of loads in flight (1187 x 1536:
+// 6.4 us with one row, 8.7 with four)
+constexpr long DYT_ROWS_MIN = 2048;
 GRAG_API hipError_t grag_dyt_residual(const void* y, float a1, const float* w1, const float* b1, float* resid,
                                       const float* add_rows, const float* add_vec, float a2, const float* w2,
                                       const float* b2, void* out, int T_, int H, int dt, hipStream_t st) {
@@ -1585,9 +1634,6 @@ hipError_t sink_prefill_launch(const void* q, const void* k, const void* v, void
                                const int* q_start, const int* ctx_len, const float* sinks, int nseq, int max_q_len, int H, int G,
                                int d, float scale, float out_scale, int nblocks, const float* hscale, const void* hgate,
                                int gate_ld, int chunk, int window, float softcap, int keep, hipStream_t st);
-// From this many workgroups at four rows a thread they are taken; fewer leave the chip short of loads in flight (1187 x 1536:
-// 6.4 us with one row, 8.7 with four)
-constexpr long DYT_ROWS_MIN = 2048;
 }  // namespace grag
 
 static int sa_key_tile(int d, int vd, size_t* bytes) {
@@ -1813,9 +1859,29 @@ GRAG_API hipError_t grag_gated_rmsnorm(const float* x, const float* w, const voi
   if (groups < 1 || groups > 65535 || N % groups) return hipErrorInvalidValue;
   const int n = N / groups;
   const uintptr_t am = dt == 0 ? 7 : 15;
-  if (groups > 1 && n <= 256 && n % 4 == 0 && ld % 4 == 0 && goff % 4 == 0 && out_ld % 4 == 0 &&
-      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0 &&
-      ((reinterpret_cast<uintptr_t>(proj) | reinterpret_cast<uintptr_t>(out)) & am) == 0) {
+  const bool vec = n % 4 == 0 && ld % 4 == 0 && goff % 4 == 0 && out_ld % 4 == 0 &&
+                   ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0 &&
+                   ((reinterpret_cast<uintptr_t>(proj) | reinterpret_cast<uintptr_t>(out)) & am) == 0;
+  if (vec && n > 256 && n <= 8192) {
+    const int threads = n <= 512 ? 128 : 256, per = (n + 4 * threads - 1) / (4 * threads);
+#define GATED_ROW(V)                                                                                                   \
+  hipLaunchKernelGGL((gated_rmsnorm_row_kernel<T, V>), dim3(T_, groups), dim3(threads), 0, st, x, w, (const T*)proj, ld, goff, \
+                     (T*)out, out_ld, n, eps, out_scale, silu_gate)
+    DT_DISPATCH(dt, {
+      if (per <= 1) {
+        GATED_ROW(1);
+      } else if (per <= 2) {
+        GATED_ROW(2);
+      } else if (per <= 4) {
+        GATED_ROW(4);
+      } else {
+        GATED_ROW(8);
+      }
+    })
+#undef GATED_ROW
+    return hipGetLastError();
+  }
+  if (groups > 1 && vec && n <= 256) {
 #define GATED_VEC(LG)                                                                                                  \
   hipLaunchKernelGGL((gated_rmsnorm_vec_kernel<T, LG>), dim3((unsigned)(((size_t)T_ * groups * LG + 255) / 256)), dim3(256), \
                      0, st, x, w, (const T*)proj, ld, goff, (T*)out, out_ld, T_, n, groups, eps, out_scale, silu_gate)
