@@ -661,6 +661,148 @@ moe_gemm_mfma_kernel(const bf16* __restrict__ a, int lda, const bf16* __restrict
   }
 }
 
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(static_cast<F&&>(f));
+  }
+}
+
+// Few rows an expert (bf16, K a multiple of 64): the weights' bytes are the work, so they go from memory straight to the
+// registers as operands of v_mfma_f32_16x16x32_bf16, without LDS or a barrier on their way.  A workgroup takes 64 rows of an
+// expert's matrix (32 of the gate and the 32 of the up half that belong to them) against a tile of 16 MT sorted rows; its four
+// waves share K, wave w the 64-column blocks w, w + 4, ... (whole 128-byte lines; the four walk neighbouring ones), each with
+// the operands of two blocks in flight; the rows of `a` come through the caches the same way.  The waves' partial sums meet in
+// LDS once, at the end, in wave order.  Operand lane: row lane % 16, k = 8 (lane / 16) .. + 7; the weights are operand
+// A, so that a lane ends with four consecutive columns of one row.  Bound by the weights' stream: gate | up and down of 16
+// experts (1.3 GB), 4 rows each 240 us (5.4 TB/s), 1 row of 4 experts 66 us; the staged 32 x 64 tiles below 294 and 160 (their
+// K step of 32 waits for each load).  Widths of 1536 / 1792, 16 rows each: 97 -> 66.  Loads through a buffer resource instead
+// of pointers: 259 where these take 242; non-temporal ones 307 (each half of a line fetched by itself).
+template <int GATED, int MT>
+__global__ void __launch_bounds__(256, 2)
+moe_gemm_stream_kernel(const bf16* __restrict__ a, int lda, const bf16* __restrict__ w, const int* __restrict__ offs,
+                       const int* __restrict__ order, int E, int top, int N, int K, bf16* __restrict__ out, int ldo, MoeEpi ep) {
+  constexpr int TM = 16 * MT, COLS = GATED == 1 ? 32 : 64, D = 2;
+  __shared__ f32x4_t part[4][4 * MT][64];
+  __shared__ int rows[TM];
+  int e = 0, tile = blockIdx.y, r0 = -1, rend = 0;
+  for (; e < E; ++e) {
+    const int b = offs[e], n = offs[e + 1] - b, nt = (n + TM - 1) / TM;
+    if (tile < nt) {
+      r0 = b + tile * TM;
+      rend = b + n;
+      break;
+    }
+    tile -= nt;
+  }
+  if (r0 < 0) return;
+  const int n0 = blockIdx.x * COLS;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ql = lane & 15, quad = lane >> 4;
+  if (threadIdx.x < TM) {
+    const int o = order[min(r0 + (int)threadIdx.x, rend - 1)];
+    rows[threadIdx.x] = o;
+  }
+  __syncthreads();
+  const size_t wn = (size_t)(GATED == 1 ? 2 * N : N) * K;
+  const char* we = reinterpret_cast<const char*>(w + (size_t)e * wn);
+  unsigned wo[4], ao[MT];  // byte offsets of the lane's rows
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int n = GATED == 1 ? (c >> 1) * N + min(n0 + 16 * (c & 1) + ql, N - 1) : min(n0 + 16 * c + ql, N - 1);
+    wo[c] = ((unsigned)n * (unsigned)K + 8u * quad) * 2u;
+  }
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int src = GATED == 0 ? min(r0 + 16 * m + ql, rend - 1) : rows[16 * m + ql] / top;
+    ao[m] = ((unsigned)src * (unsigned)lda + 8u * quad) * 2u;
+  }
+  f32x4_t acc[4][MT];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[c][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int nb = ((K >> 6) - wid + 3) >> 2;  // the wave's blocks of 64
+  bf16x8_t wf[D][4][2], af[D][MT][2];
+  // (both halves of a row's line one after the other: apart, the second would find the line gone)
+  auto load = [&](int b, auto slot) __attribute__((always_inline)) {
+    constexpr int i = decltype(slot)::value;
+    const size_t kb = (size_t)(wid + 4 * min(b, nb - 1)) * 128;  // past the end: the last block again, never used
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) wf[i][c][h] = *reinterpret_cast<const bf16x8_t*>(we + kb + wo[c] + 64 * h);
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        af[i][m][h] = *reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const char*>(a) + kb + ao[m] + 64 * h);
+  };
+  auto mul = [&](auto slot) __attribute__((always_inline)) {
+    constexpr int i = decltype(slot)::value;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          acc[c][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i][c][h], af[i][m][h], acc[c][m], 0, 0, 0);
+  };
+  if (nb > 0) {
+    static_for<D>([&](auto i) __attribute__((always_inline)) { load(decltype(i)::value, i); });
+    int b = 0;
+    for (; b + D <= nb; b += D)
+      static_for<D>([&](auto i) __attribute__((always_inline)) {
+        mul(i);
+        if (MT == 4) __builtin_amdgcn_sched_barrier(0);  // (hoisted over the products, a third block's registers spill)
+        load(b + D + decltype(i)::value, i);
+        if (MT == 4) __builtin_amdgcn_sched_barrier(0);
+      });
+    static_for<D>([&](auto i) __attribute__((always_inline)) {
+      if (b + decltype(i)::value < nb) mul(i);
+    });
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) part[wid][c * MT + m][lane] = acc[c][m];
+  __syncthreads();
+  // tile (c, m) of the workgroup: columns 16 c + 4 (lane / 16) .. + 3, row 16 m + lane % 16
+  auto total = [&](int t) {
+    f32x4_t v = part[0][t][lane];
+#pragma unroll
+    for (int k = 1; k < 4; ++k) v += part[k][t][lane];
+    return v;
+  };
+  const bool wide = ((uintptr_t)out & 7) == 0 && (ldo & 3) == 0 && (N & 3) == 0;
+#pragma unroll
+  for (int j = 0; j < (GATED == 1 ? (2 * MT + 3) / 4 : MT); ++j) {
+    const int t = wid + 4 * j;
+    if (GATED == 1 && t >= 2 * MT) break;
+    f32x4_t v = total(t);
+    if (GATED == 1) {
+      const f32x4_t u = total(t + 2 * MT);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = glu_unit(v[i], u[i], ep);
+    }
+    if (GATED == 3) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = relu2_unit(v[i]);
+    }
+    const int c = t / MT, lr = 16 * (t % MT) + ql, n = n0 + 16 * c + 4 * quad;
+    if (r0 + lr >= rend) continue;
+    bf16* dst = out + (size_t)(GATED == 0 ? rows[lr] : r0 + lr) * ldo + n;
+    if (wide) {
+      if (n < N) *reinterpret_cast<bf16x4_t*>(dst) = bf16x4_t{f2bits(v[0]), f2bits(v[1]), f2bits(v[2]), f2bits(v[3])};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (n + i < N) dst[i] = (bf16)v[i];
+    }
+  }
+}
+
 // Large tiles for prompt-sized row counts (bf16): 128 rows x 128 columns per workgroup, 4 waves of 64 x 64 (wave w: rows
 // 64 (w / 2), columns 64 (w % 2)), v_mfma_f32_16x16x32_bf16 (operand lane: row / column lane % 16, k = 8 (lane / 16)
 // .. + 7), K steps of 64 (one 128-byte line per row) staged through LDS with the next step's global loads in flight
@@ -1333,8 +1475,34 @@ GRAG_API hipError_t grag_moe_gemm(const void* a, int lda, const void* w, const i
 #undef MOE_TILE
     return hipGetLastError();
   }
-  if (dt == 0 && K % 8 == 0 && lda % 8 == 0 && al16(a) && al16(w) && rows >= 48 * E) {
-    // prompt-sized row counts (half a large tile per expert on average, or more): the 128 x 128 tiles
+  // The weights' stream or the 128 x 128 tiles, by rows an expert and tiles for the chip (us, both products, 16 experts; widths
+  // 3584 / 3776 with 480 and 448 tiles, and 1536 / 1792 with 224 and 192): 1 row 167 against 213, 36 against 70; 8 rows 246 / 242,
+  // 63 / 74; 12 rows 251 / 241, 64 / 75; 24 rows 273 / 250, 70 / 79; 48 rows 341 / 262, 89 / 85.  Between them the tiles of
+  // 16, 32 and 64 rows: the smallest that holds nearly every expert's rows (a second tile reads the weights again: 16 rows
+  // an expert 312 us in tiles of 16, 257 of 32, 274 of 64; 28 rows 309 of 32, 300 of 64).
+  const bool tiles128 = rows >= 48 * E || (rows >= 12 * E && (long)E * ((N + 127) / 128) >= 384);
+  if (dt == 0 && gated != 2 && !tiles128 && K % 64 == 0 && lda % 8 == 0 && al16(a) && al16(w) && a_bytes < (1L << 31) &&
+      w_bytes < (1L << 31)) {
+    const int mt = rows <= 6 * E ? 1 : rows <= 26 * E ? 2 : 4;
+    const dim3 sgrid((N + (gated == 1 ? 31 : 63)) / (gated == 1 ? 32 : 64), (rows + 16 * mt - 1) / (16 * mt) + E);
+#define MOE_STREAM(G, M)                                                                                                  \
+  hipLaunchKernelGGL((moe_gemm_stream_kernel<G, M>), sgrid, dim3(256), 0, st, (const bf16*)a, lda, (const bf16*)w, offs, order, \
+                     E, top, N, K, (bf16*)out, ldo, ep)
+#define MOE_STREAM_M(G)                  \
+  {                                      \
+    if (mt == 1) MOE_STREAM(G, 1);       \
+    else if (mt == 2) MOE_STREAM(G, 2);  \
+    else MOE_STREAM(G, 4);               \
+  }
+    if (gated == 1) MOE_STREAM_M(1)
+    else if (gated == 3) MOE_STREAM_M(3)
+    else MOE_STREAM_M(0)
+#undef MOE_STREAM_M
+#undef MOE_STREAM
+    return hipGetLastError();
+  }
+  if (dt == 0 && K % 8 == 0 && lda % 8 == 0 && al16(a) && al16(w) && (gated == 2 ? rows >= 48 * E : tiles128)) {
+    // prompt-sized row counts, and decode batches over experts wide enough to fill the chip
     const int btiles = (rows + 127) / 128 + E;
     const dim3 bgrid((N + 127) / 128, btiles);
     MOE_LAUNCH(moe_gemm_big_kernel, bgrid, (const bf16*)a, (const bf16*)w, (bf16*)out)

@@ -1,0 +1,41 @@
+"""The experts' grouped GEMM at decode's row counts (csrc/kernels/moe.hip moe_gemm_stream_kernel, and the 128-row tiles that
+take over where the experts fill the chip) against a plain fp32 product per pair: row counts around the tiles of 16, 32 and 64
+rows, none among them, contractions shorter than the waves' blocks, columns past the last whole tile."""
+import pytest
+import torch
+
+from githubrepostorag_amd.ops.moe import moe_experts
+
+pytestmark = pytest.mark.gpu
+
+FEW = [0, 1, 16, 17, 3, 0, 2, 5, 1, 2]           # at most 6 a mean expert
+SOME = [0, 1, 32, 33, 31, 16, 40, 24]            # at most 26
+MANY = [0, 64, 65, 20, 63, 33, 1]                # at most 48
+EVEN = [13] * 16                                 # with 24 column tiles an expert: the 128-row tiles
+
+
+@pytest.mark.parametrize("counts,W,F", [(c, W, F) for c in (FEW, SOME, MANY) for W, F in ((64, 128), (192, 64), (328, 392), (640, 1088))]
+                         + [(EVEN, 64, 3072), ([1], 256, 512), ([0, 1, 0, 0], 448, 192)])
+@pytest.mark.parametrize("unit,limit", [("glu", None), ("glu", 2.0), ("relu2", None)])
+def test_moe_stream(counts, W, F, unit, limit):
+    g = torch.Generator().manual_seed(W + F + len(counts))
+    E, top = len(counts), 1 if sum(counts) % 2 else 2
+    flat = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)] + [torch.tensor([-1, E])])
+    flat = flat[torch.randperm(len(flat), generator=g)]
+    flat = flat[: len(flat) // top * top]
+    T = len(flat) // top
+    ids = flat.view(T, top).to(torch.int32)
+    h = torch.randn(T, W, generator=g).bfloat16()
+    wgu = (torch.randn(E, F if unit == "relu2" else 2 * F, W, generator=g) * W ** -0.5).bfloat16()
+    wd = (torch.randn(E, W, F, generator=g) * F ** -0.5).bfloat16()
+    kw = dict(unit=unit) if unit == "relu2" else dict(limit=limit, alpha=1.3 if limit else 1.0, shift=0.5 if limit else 0.0)
+    wide = torch.zeros(T, W + 8, dtype=torch.bfloat16, device="cuda")
+    wide[:, :W] = h.cuda()
+    got = moe_experts(wide[:, :W], ids.cuda(), wgu.cuda(), wd.cuda(), **kw).float().cpu()
+    want = moe_experts(h, ids, wgu, wd, **kw).float()
+    ok = (ids >= 0) & (ids < E)
+    # both round the unit's output and the result to bf16 (2^-8 apart at most where fp32 sums of another order fall on
+    # different sides); the second product averages the first rounding over F terms
+    err = (got - want)[ok].abs().max() / want[ok].abs().max()
+    assert err < 2 ** -7, err
+    assert (got - want)[ok].norm() / want[ok].norm() < 5e-3
