@@ -15,47 +15,15 @@
 // rows in step 221, half a tile apart 225, 16 waves 223; 128 rows by 4 waves of 32 rows 200, but 49 against 43 on a
 // prompt of 1187 tokens, 12 / 2 heads.  Measured, old -> new: window 345 -> 208 us, all keys 811 -> 479, blocks of 1024
 // 214 -> 141, 1 x 8192 tokens of all keys 1466 -> 714; 12 / 2 heads, 1 x 1187 tokens 75 -> 43.
-#include "common.h"
+#include "sink.h"
 
 GRAG_ERR_UNIT(sink_prefill)
 
 namespace grag {
 
 constexpr int SP_KT = 64;         // keys per tile
-constexpr int SP_BS = 16;         // keys per cache block
 constexpr int SP_MAXB = 2048;     // cache blocks a workgroup can walk (32 K keys): its part of the block table, in LDS
 constexpr int SP_ROWS = 128;      // rows of a workgroup: 8 waves of 16
-constexpr float SP_RESCALE = 8.f;
-
-struct SinkArgs {
-  const bf16 *q, *k, *v;
-  bf16* out;
-  const int *bt, *q_start, *ctx_len;
-  const float *sinks, *hscale;
-  const bf16* hgate;
-  int out_ld, bt_stride, H, G, R, nblocks, tiles, gate_ld, chunk, window, keep;
-  float scale, out_scale, softcap;
-};
-
-typedef __attribute__((address_space(3))) void sp_lds_t;
-typedef __attribute__((address_space(3))) bf16x4_t sp_lds4_t;
-
-// swizzles of the 16-byte chunks of a tile's rows: K is read as row fragments, V by the transposed read (8 rows x 4 units of 8
-// bytes at a time); both spread a read over all banks
-template <int D> __device__ __forceinline__ int sp_kswz(int row) { return D == 128 ? row & 15 : (row >> 1) & 7; }
-template <int D> __device__ __forceinline__ int sp_vswz(int row) { return D == 128 ? (row & 7) << 1 : ((row >> 1) & 3) << 1; }
-
-// 16 bytes a lane from `off` bytes behind a wave-uniform base of `bytes` bytes into 1 KB of LDS, lane after lane
-__device__ __forceinline__ void sp_dma(const bf16* base, int bytes, int off, char* dst) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000), (sp_lds_t*)dst, 16,
-                                           off, 0, 0, 0);
-}
-
-// first key of the block / window of the query at `pos` (never falls as pos grows)
-__device__ __forceinline__ int sp_first(const SinkArgs& p, int pos) {
-  const int lo = p.chunk > 0 ? pos - pos % p.chunk : 0;
-  return p.window > 0 ? max(lo, pos - p.window + 1) : lo;
-}
 
 template <int D, bool CAP>
 __global__ void __launch_bounds__(512, 4) sink_prefill_kernel(const SinkArgs p) {

@@ -195,7 +195,7 @@ def call(name: str, *args) -> None:
 
 # ---------------------------------------------------------------- device index guard (csrc/kernels/common.h)
 ERR_UNITS = ("norm", "elementwise", "attention", "gemm_tile", "gemm_stream", "seqmix", "gatedmix", "ssm", "moe", "delta", "linscan",
-             "sink_prefill")
+             "sink_prefill", "sink_decode")
 ERR_CODES = {1 << 0: "embed_gather: token id >= vocab", 1 << 1: "qkv_rope_kvstore: KV slot id >= cache slots",
              1 << 2: "qkv_rope_kvstore: position >= RoPE table rows",
              1 << 3: "prefill attention: block-table entry >= KV blocks",
