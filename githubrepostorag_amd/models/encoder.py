@@ -16,6 +16,9 @@ the fp32 vector and the bf16 copy the index stores.
 """
 from __future__ import annotations
 
+import itertools
+
+import numpy as np
 import torch
 
 from ..ops.attention import varlen_attention
@@ -119,16 +122,22 @@ class BertEncoder:
         cfg = self.cfg
         dev = self.device
         lens = [max(1, min(len(x), cfg.max_position)) for x in batch]
-        flat = []
-        for x, n in zip(batch, lens):
-            flat.extend(x[:n] if x else [0])
-        starts = [0]
-        for n in lens:
-            starts.append(starts[-1] + n)
-        ids = torch.tensor(flat, dtype=torch.int32, device=dev)
-        pos_ids = torch.cat([torch.arange(n, dtype=torch.int32) for n in lens]).to(dev)
-        seq_start = torch.tensor(starts, dtype=torch.int32, device=dev)
-        seq_len = torch.tensor(lens, dtype=torch.int32, device=dev)
+        T, n = sum(lens), len(lens)
+        parts = [(x if len(x) == k else x[:k]) if x else [0] for x, k in zip(batch, lens)]
+        # ids | positions | starts | lengths in one buffer and one copy to the device; the ids through one iterator (24000
+        # tokens in 128 parts: 1.9 -> 0.7 ms of a slow core, 0.35 ms of a batch of 6.6 with the GPU idle)
+        host = np.empty(2 * T + 2 * n + 1, dtype=np.int32)
+        try:
+            host[:T] = np.fromiter(itertools.chain.from_iterable(parts), dtype=np.int32, count=T)
+        except (TypeError, ValueError, OverflowError):  # what numpy does not read as whole numbers: torch decides
+            host[:T] = torch.tensor([t for x in parts for t in x], dtype=torch.int32).numpy()
+        starts, length = host[2 * T: 2 * T + n + 1], host[2 * T + n + 1:]
+        length[:] = lens
+        starts[0] = 0
+        np.cumsum(length, out=starts[1:])
+        host[T: 2 * T] = np.arange(T, dtype=np.int32) - np.repeat(starts[:-1], length)
+        buf = torch.from_numpy(host).to(dev)
+        ids, pos_ids, seq_start, seq_len = buf[:T], buf[T: 2 * T], buf[2 * T: 2 * T + n + 1], buf[2 * T + n + 1:]
         return self.forward(ids, pos_ids, seq_start, seq_len, max(lens), want_bf16)
 
     def forward(self, ids, pos_ids, seq_start, seq_len, max_len: int, want_bf16: bool = True):
