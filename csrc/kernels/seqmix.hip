@@ -1244,6 +1244,84 @@ decay_attn_scan_kernel(const T* __restrict__ proj, int ld, int qoff, int koff, i
   }
 }
 
+// One token per sequence (decode; vd a multiple of 4, aligned state, d and vd at most 256): the state is read and written once
+// and nothing else is of size, so a thread owns four columns of rows rg, rg + RG, ... (RG = 256 / (vd / 4) row groups) in 16-byte
+// accesses that are all under way before q, k and v are made.  The same recurrence; o's sum is over a thread's rows, then the
+// groups in order.  grid (H, nseq).  64 sequences x 28 heads of 128 x 128 (235 MB): 65 us a column a thread, 46 here.
+template <typename T, int RPT>
+__global__ void __launch_bounds__(256)
+decay_step_kernel(const T* __restrict__ proj, int ld, int qoff, int koff, int voff, const float* __restrict__ decay,
+                  float* __restrict__ state, const int* __restrict__ slots, const int* __restrict__ q_start,
+                  const int* __restrict__ ctx_len, float* __restrict__ out, int H, int d, int vd, int nslots, int act,
+                  const int* __restrict__ positions, const float* __restrict__ rope_tab, int rd, int tab_rows, float kscale) {
+  __shared__ float qs[256], ks[256];
+  __shared__ __attribute__((aligned(16))) float part[256 * 4];
+  const int h = blockIdx.x, seq = blockIdx.y, tok = q_start[seq];
+  if (q_start[seq + 1] <= tok) return;
+  const bool fresh = ctx_len[seq] == 1;
+  const int slot = slots[seq];
+  const bool slot_ok = index_ok(slot, nslots, ERR_SAMPLER_SLOT);
+  float* Sg = state + ((size_t)(slot_ok ? slot : 0) * H + h) * d * vd;
+  const int nc = vd >> 2, RG = 256 / nc, rg = threadIdx.x / nc, c = (threadIdx.x - rg * nc) * 4;
+  const bool on = rg < RG;
+  f32x4_t S[RPT];
+#pragma unroll
+  for (int u = 0; u < RPT; ++u) {
+    const int r = rg + RG * u;
+    S[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (!fresh && slot_ok && on && r < d) S[u] = *reinterpret_cast<const f32x4_t*>(Sg + (size_t)r * vd + c);
+  }
+  const T* row = proj + (size_t)tok * ld;
+  for (int i2 = threadIdx.x; i2 < 2 * d; i2 += 256) {
+    const int which = i2 >= d, i = which ? i2 - d : i2;
+    const T* x = row + (which ? koff : qoff) + h * d;
+    float val = ldf(x + i);
+    if (act) val = silu_acc(val);
+    if (i < rd) {
+      const int half = rd >> 1, fi = i < half ? i : i - half;
+      float other = ldf(x + (i < half ? i + half : i - half));
+      if (act) other = silu_acc(other);
+      int p = positions[tok];
+      if (!index_ok(p, tab_rows, ERR_ROPE_POS)) p = 0;
+      const float cs = rope_tab[(size_t)p * rd + fi], sn = rope_tab[(size_t)p * rd + half + fi];
+      val = i < half ? val * cs - other * sn : val * cs + other * sn;
+    }
+    if (which) ks[i] = val * kscale;
+    else qs[i] = val;
+  }
+  f32x4_t v = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if (on) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = ldf(row + voff + h * vd + c + e);
+      if (act) v[e] = silu_acc(v[e]);
+    }
+  }
+  const float lam = decay[h];
+  __syncthreads();
+  f32x4_t o = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < RPT; ++u) {
+    const int r = rg + RG * u;
+    if (on && r < d) {
+      const float k = ks[r], q = qs[r];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        S[u][e] = fmaf(lam, S[u][e], k * v[e]);
+        o[e] = fmaf(S[u][e], q, o[e]);
+      }
+      if (slot_ok) *reinterpret_cast<f32x4_t*>(Sg + (size_t)r * vd + c) = S[u];
+    }
+  }
+  if (on) *reinterpret_cast<f32x4_t*>(part + rg * vd + c) = o;
+  __syncthreads();
+  for (int j = threadIdx.x; j < vd; j += 256) {
+    float sum = 0.f;
+    for (int k = 0; k < RG; ++k) sum += part[k * vd + j];
+    out[(size_t)tok * (H * vd) + h * vd + j] = sum;
+  }
+}
+
 // ws[seq, c] (chunk c's own contribution) -> the state at the start of chunk c; the slot's state <- the state after
 // the last chunk.  grid (H, nseq, ceil(d * vd / 256)): one thread per state element.
 __global__ void decay_chunk_prefix_kernel(const float* __restrict__ decay, float* __restrict__ state,
@@ -1868,6 +1946,24 @@ GRAG_API hipError_t grag_decay_attn_scan(const void* proj, int ld, int qoff, int
   if (nseq <= 0) return hipSuccess;
   if (d > 256 || vd > 256) return hipErrorInvalidValue;
   if (rd < 0 || rd > d || (rd & 1) || (rd > 0 && (positions == nullptr || rope_tab == nullptr))) return hipErrorInvalidValue;
+  if (max_q_len == 1 && vd >= 4 && vd % 4 == 0 && (reinterpret_cast<uintptr_t>(state) & 15) == 0) {
+    const int RG = 256 / (vd / 4), per = (d + RG - 1) / RG;
+#define DECAY_STEP(R)                                                                                                 \
+  hipLaunchKernelGGL((decay_step_kernel<T, R>), dim3(H, nseq), dim3(256), 0, st, (const T*)proj, ld, qoff, koff, voff, \
+                     decay, state, slots, q_start, ctx_len, out, H, d, vd, nslots, act, positions, rope_tab, rd,      \
+                     tab_rows, kscale)
+    if (per <= 16) {
+      DT_DISPATCH(dt, {
+        if (per <= 4) {
+          DECAY_STEP(4);
+        } else {
+          DECAY_STEP(16);
+        }
+      })
+      return hipGetLastError();
+    }
+#undef DECAY_STEP
+  }
   if (ws == nullptr || max_q_len <= DECAY_CHUNK) {
     DT_DISPATCH(dt, return (launch_decay_scan<T, 0>((const T*)proj, ld, qoff, koff, voff, decay, state, slots, q_start,
                                                     ctx_len, out, nseq, H, d, vd, nslots, nullptr, 0, act, positions, rope_tab,
