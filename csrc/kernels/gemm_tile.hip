@@ -7,6 +7,9 @@
 //   EPI_STORE   bf16 out = act(acc + bias)                (act: none / gelu-erf / gelu-tanh)
 //   EPI_SILU    bf16 out[M, N/2] = silu(g + bg) * (u + bu) (gate/up rows interleaved in 32-row
 //               blocks by ops/gemm.py: rows [64j, 64j+32) = gate j*32.., [64j+32, 64j+64) = up)
+//   EPI_GLU     bf16 out[M, N/2] = glu(gate, up) of a W whose first N/2 rows are the gate and whose others the up
+//               half (a tile takes 128 of each): g sigmoid(alpha g) (u + shift), g and u clamped (8192 rows, 2 x 18944 x 3584:
+//               library product and unit 1706 us, here 1581)
 //   EPI_PARTIAL fp32 split-K slab ws[split][M][N] (reduced + epilogued by splitk_reduce_kernel)
 //
 // Geometry (cdna_hip_programming.md §5 "The 256² 8-phase template", re-derived
@@ -47,13 +50,25 @@ constexpr int kSlot = 128 * 128;  // 128 rows x 64 bf16
 constexpr int kBuf = 4 * kSlot;   // one K-tile: A q0, A q1, B q0, B q1
 constexpr int kThreads = 512;
 
-enum { EPI_STORE = 0, EPI_SILU = 1, EPI_PARTIAL = 2 };
+enum { EPI_STORE = 0, EPI_SILU = 1, EPI_PARTIAL = 2, EPI_GLU = 3 };
 enum { ACT_NONE = 0, ACT_GELU = 1, ACT_SILU = 2, ACT_GELU_TANH = 3 };
 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.f + __expf(-x)); }
 __device__ __forceinline__ float gelu_tanh_f(float x) {
   const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
   return 0.5f * x * (2.f - 2.f * __builtin_amdgcn_rcpf(1.f + __expf(2.f * u)));
+}
+// g sigmoid(alpha g) (u + shift) with g = min(g, limit), u = clamp(u, +-limit).  The exponential is the bare instruction, the
+// quotient a reciprocal with one correction step; where the exponential passes 2^126 the sigmoid is 0.
+__device__ __forceinline__ float glu_f(float g, float u, float limit, float alpha, float shift) {
+  g = fminf(g, limit);
+  u = fminf(fmaxf(u, -limit), limit);
+  const float e = -1.4426950408889634f * (alpha * g);
+  const float d = 1.f + __builtin_amdgcn_exp2f(fminf(e, 126.f));
+  const float rc = __builtin_amdgcn_rcpf(d);
+  float q = g * rc;
+  q = fmaf(fmaf(-d, q, g), rc, q);
+  return (e > 126.f ? g * 0.f : q) * (u + shift);
 }
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return (uint32_t)(uint16_t)f2bits(lo) | ((uint32_t)(uint16_t)f2bits(hi) << 16);
@@ -94,6 +109,7 @@ struct Args {
   float* slab;     // split-K partial planes, or 2 x 256 KB stream-K slots per SK workgroup
   unsigned* cnt;   // stream-K arrival tickets, one per SK tile (zero at rest)
   int a_bytes, w_bytes;  // buffer-resource extents of A / W (SCHED 1; both < 2 GB)
+  float limit, alpha, shift;  // EPI_GLU
 };
 
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
@@ -259,6 +275,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tile_kernel(Args p) {
         gm = gm < p.M ? gm : p.M - 1;
         int gn = n0 + (rs >> 5) * 64 + q * 32 + (rs & 31);
         gn = gn < p.N ? gn : p.N - 1;
+        if constexpr (EPI == EPI_GLU)  // column quadrant 0 is 32 gate rows, 1 the 32 up rows that belong to them
+          gn = q * (p.N / 2) + min(n0 / 2 + (rs >> 5) * 32 + (rs & 31), p.N / 2 - 1);
         if constexpr (SCHED >= 1) {
           offA[q][i] = (unsigned)(gm * p.lda + koff) * 2u;
           offB[q][i] = (unsigned)(gn * p.ldw + koff) * 2u;
@@ -479,7 +497,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tile_kernel(Args p) {
   };
   auto epilogue = [&](int m0, int n0, int split) {
     const int mrow = m0 + wr * 128;
-    if constexpr (EPI == EPI_SILU) {
+    if constexpr (EPI == EPI_SILU || EPI == EPI_GLU) {
       bf16* C = (bf16*)p.C;
       const int nb = n0 + wc * 64;  // this wave's 64-column gate/up block: output cols [nb / 2, +32)
       const int obase = nb / 2;
@@ -489,11 +507,14 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tile_kernel(Args p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int n = nb + ccol(i) + r;
-          bg[i][r] = (p.bias && n < p.N) ? (float)p.bias[n] : 0.f;
-          bu[i][r] = (p.bias && n + 32 < p.N) ? (float)p.bias[n + 32] : 0.f;
+          bg[i][r] = (EPI == EPI_SILU && p.bias && n < p.N) ? (float)p.bias[n] : 0.f;
+          bu[i][r] = (EPI == EPI_SILU && p.bias && n + 32 < p.N) ? (float)p.bias[n + 32] : 0.f;
         }
       // the wave's 32 output columns of this 64-column gate/up block are whole: 16-byte stores
       const bool wide = wide_ok && 2 * (obase + 32) <= p.N;
+      auto unit = [&](float g, float u, float bgv, float buv) {
+        return EPI == EPI_GLU ? glu_f(g, u, p.limit, p.alpha, p.shift) : silu_f(g + bgv) * (u + buv);
+      };
       auto emit = [&](const Acc& g, const Acc& u, int qm) {
 #pragma unroll
         for (int rs = 0; rs < kRows; ++rs) {
@@ -506,8 +527,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tile_kernel(Args p) {
               const f32x4_t gv = chunk_get<MF>(g, rs * kCpr + i), uv = chunk_get<MF>(u, rs * kCpr + i);
 #pragma unroll
               for (int h = 0; h < 2; ++h)
-                d[i][h] = pack_bf16x2(silu_f(gv[2 * h] + bg[i][2 * h]) * (uv[2 * h] + bu[i][2 * h]),
-                                      silu_f(gv[2 * h + 1] + bg[i][2 * h + 1]) * (uv[2 * h + 1] + bu[i][2 * h + 1]));
+                d[i][h] = pack_bf16x2(unit(gv[2 * h], uv[2 * h], bg[i][2 * h], bu[i][2 * h]),
+                                      unit(gv[2 * h + 1], uv[2 * h + 1], bg[i][2 * h + 1], bu[i][2 * h + 1]));
             }
             store_row(C + (size_t)m * p.ldc + obase, d);
             continue;
@@ -519,7 +540,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tile_kernel(Args p) {
             const f32x4_t gv = chunk_get<MF>(g, rs * kCpr + i), uv = chunk_get<MF>(u, rs * kCpr + i);
             bf16x4_t o;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o[r] = f2bits(silu_f(gv[r] + bg[i][r]) * (uv[r] + bu[i][r]));
+            for (int r = 0; r < 4; ++r) o[r] = f2bits(unit(gv[r], uv[r], bg[i][r], bu[i][r]));
             *reinterpret_cast<bf16x4_t*>(C + (size_t)m * p.ldc + oc) = o;
           }
         }
@@ -820,9 +841,9 @@ int device_cus() {
 }
 }  // namespace
 
-GRAG_API int grag_gemm_tile(const void* A, const void* W, const void* bias, void* C, int lda, int ldw, int ldc,
-                            int M, int N, int K, int epi, int act, int ksplit, int sk_grid, void* ws, void* cnt,
-                            hipStream_t stream) {
+static int gemm_tile_run(const void* A, const void* W, const void* bias, void* C, int lda, int ldw, int ldc, int M, int N,
+                         int K, int epi, int act, int ksplit, int sk_grid, void* ws, void* cnt, float limit, float alpha,
+                         float shift, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
   if (K % 64 != 0 || K < 128 || lda % 8 != 0 || ldw % 8 != 0 || ldc % 8 != 0 || N % 8 != 0)
     return (int)hipErrorInvalidValue;
@@ -830,9 +851,10 @@ GRAG_API int grag_gemm_tile(const void* A, const void* W, const void* bias, void
   // epi 2 (EPI_PARTIAL, ksplit > 1 only): leave the fp32 planes in ws for a consumer that reduces
   // them itself (grag_splitk_add_rmsnorm)
   const bool keep = epi == EPI_PARTIAL;
-  if (epi != EPI_STORE && epi != EPI_SILU && !keep) return (int)hipErrorInvalidValue;
+  if (epi != EPI_STORE && epi != EPI_SILU && epi != EPI_GLU && !keep) return (int)hipErrorInvalidValue;
   if (act != ACT_NONE && act != ACT_GELU && act != ACT_GELU_TANH) return (int)hipErrorInvalidValue;
-  if ((epi == EPI_SILU || keep) && act != ACT_NONE) return (int)hipErrorInvalidValue;
+  if (epi == EPI_GLU && (ksplit > 1 || bias != nullptr || N % 16 != 0)) return (int)hipErrorInvalidValue;
+  if ((epi == EPI_SILU || epi == EPI_GLU || keep) && act != ACT_NONE) return (int)hipErrorInvalidValue;
   if (keep && (ksplit <= 1 || bias != nullptr)) return (int)hipErrorInvalidValue;
   const int kt = K / 64;
   if (ksplit < 1) ksplit = 1;
@@ -849,6 +871,7 @@ GRAG_API int grag_gemm_tile(const void* A, const void* W, const void* bias, void
   a.cnt = (unsigned*)cnt;
   a.lda = lda; a.ldw = ldw; a.ldc = ldc;
   a.M = M; a.N = N; a.K = K;
+  a.limit = limit; a.alpha = alpha; a.shift = shift;
   {  // SCHED 1's 32-bit offsets: operands of 2 GB or more take schedule 0 (64-bit pointers)
     const long ab = (long)M * lda * 2, wb = (long)N * ldw * 2;
     a.a_bytes = ab < (1L << 31) ? (int)ab : 0;
@@ -891,9 +914,27 @@ GRAG_API int grag_gemm_tile(const void* A, const void* W, const void* bias, void
     return (int)hipGetLastError();
   }
   if (epi == EPI_SILU) return launch<EPI_SILU, ACT_NONE>(a, stream);
+  if (epi == EPI_GLU) return launch<EPI_GLU, ACT_NONE>(a, stream);
   if (act == ACT_GELU) return launch<EPI_STORE, ACT_GELU>(a, stream);
   if (act == ACT_GELU_TANH) return launch<EPI_STORE, ACT_GELU_TANH>(a, stream);
   return launch<EPI_STORE, ACT_NONE>(a, stream);
+}
+
+GRAG_API int grag_gemm_tile(const void* A, const void* W, const void* bias, void* C, int lda, int ldw, int ldc,
+                            int M, int N, int K, int epi, int act, int ksplit, int sk_grid, void* ws, void* cnt,
+                            hipStream_t stream) {
+  if (epi == EPI_GLU) return (int)hipErrorInvalidValue;
+  return gemm_tile_run(A, W, bias, C, lda, ldw, ldc, M, N, K, epi, act, ksplit, sk_grid, ws, cnt, 0.f, 0.f, 0.f, stream);
+}
+
+// C [M, F] = g sigmoid(alpha g) (u + shift), g = min(x wg^T, limit), u = clamp(x wu^T, +-limit), W [2F, K] = wg | wu, F % 8 == 0;
+// whole tiles.
+GRAG_API int grag_gemm_tile_glu(const void* A, const void* W, void* C, int lda, int ldw, int ldc, int M, int F, int K,
+                                float limit, float alpha, float shift, hipStream_t stream) {
+  if (M <= 0 || F <= 0) return 0;
+  if (F > (1 << 30)) return (int)hipErrorInvalidValue;
+  return gemm_tile_run(A, W, nullptr, C, lda, ldw, ldc, M, 2 * F, K, EPI_GLU, ACT_NONE, 1, 0, nullptr, nullptr, limit, alpha,
+                       shift, stream);
 }
 
 GRAG_ERR_UNIT(gemm_tile)

@@ -31,8 +31,8 @@ import math
 import torch
 
 from ..ops.attention import AttnMetadata, sink_attention
-from ..ops.elementwise import clamped_glu, rope_table, rope_vnorm_store
-from ..ops.linear import linear
+from ..ops.elementwise import rope_table, rope_vnorm_store
+from ..ops.linear import glu_linear, linear
 from ..ops.moe import moe_experts, moe_route
 from ..ops.norm import embed_gather_f32, residual_layernorm
 from ..ops.recurrent import causal_conv, gated_delta
@@ -263,7 +263,7 @@ class KapanexModel:
                                     scale=f.scale)
         add = {"e": moe_experts(h, ids, L.wgu, L.wd), "ecoef": wts}
         if L.wsgu is not None:
-            add.update(b=linear(clamped_glu(linear(h, L.wsgu), None, 1.0, 0.0), L.wsd), bcoef=sgate)
+            add.update(b=linear(glu_linear(h, L.wsgu, None, 1.0, 0.0), L.wsd), bcoef=sgate)
         return add
 
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor, meta: AttnMetadata, kv_caches,

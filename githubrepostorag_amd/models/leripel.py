@@ -32,8 +32,8 @@ import math
 import torch
 
 from ..ops.attention import AttnMetadata, sink_attention
-from ..ops.elementwise import clamped_glu, rope_table, rope_vnorm_store
-from ..ops.linear import linear
+from ..ops.elementwise import rope_table, rope_vnorm_store
+from ..ops.linear import glu_linear, linear
 from ..ops.moe import moe_experts, moe_route
 from ..ops.norm import embed_gather_f32, residual_rmsnorm
 from ..ops.recurrent import causal_conv, decay_attention, gated_rmsnorm, ssm_scan
@@ -303,7 +303,7 @@ class LeripelModel:
         e = moe_experts(h, ids, L.wgu, L.wd)
         b = None
         if L.wsgu is not None:
-            b = linear(clamped_glu(linear(h, L.wsgu), None, 1.0, 0.0), L.wsd)
+            b = linear(glu_linear(h, L.wsgu, None, 1.0, 0.0), L.wsd)
         return b, sgate, e, wts
 
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor, meta: AttnMetadata, kv_caches,

@@ -33,8 +33,8 @@ import math
 import torch
 
 from ..ops.attention import AttnMetadata, sigmoid_window_attention, sink_attention
-from ..ops.elementwise import clamped_glu, latent_store, qk_norm_store, rope_table
-from ..ops.linear import linear
+from ..ops.elementwise import latent_store, qk_norm_store, rope_table
+from ..ops.linear import glu_linear, linear
 from ..ops.norm import embed_gather_f32, hyper_mix, rmsnorm_rows
 from ..ops.recurrent import decay_attention, gated_rmsnorm
 from ..parallel.comm import Group
@@ -328,7 +328,7 @@ class NamudraModel:
             y, hc = self._mixer(L, h, positions, meta, kv_caches[ri], state[ri]), L.hc1
             if L.wgu is not None:
                 h, _ = hyper_mix(xs, y, hc[0], hc[1], L.hc2[2], L.norm2, eps, dt)
-                y, hc = linear(clamped_glu(linear(h, L.wgu), None, 1.0, 0.0), L.wd), L.hc2
+                y, hc = linear(glu_linear(h, L.wgu, None, 1.0, 0.0), L.wd), L.hc2
         if taps is not None and self.runs:
             taps.append(hyper_mix(xs, y, hc[0], hc[1], self.ones, None, eps, dt, want_sum=True)[1])
             y = hc = None

@@ -30,8 +30,8 @@ import math
 import torch
 
 from ..ops.attention import AttnMetadata, sink_attention
-from ..ops.elementwise import clamped_glu, rope_table, rope_vnorm_store
-from ..ops.linear import linear
+from ..ops.elementwise import rope_table, rope_vnorm_store
+from ..ops.linear import glu_linear, linear
 from ..ops.norm import dyt_residual, embed_gather_f32
 from ..ops.recurrent import decay_attention, gated_rmsnorm, mingru_scan
 from ..parallel.comm import Group
@@ -297,7 +297,7 @@ class ZofesunModel:
             y, post = self._mixer(L, h, positions, meta, kv_caches[ri], state[ri]), L.norm1b
             if L.wgu is not None:
                 h = dyt_residual(x, y, post, pre=L.norm2, out_dtype=dt)
-                y, post = linear(clamped_glu(linear(h, L.wgu), L.spec.mlp.limit, GLU_SIGMOID_SLOPE), L.wd), L.norm2b
+                y, post = linear(glu_linear(h, L.wgu, L.spec.mlp.limit, GLU_SIGMOID_SLOPE), L.wd), L.norm2b
         if taps is not None and self.runs:
             dyt_residual(x, y, post, out_dtype=dt)
             y = post = None

@@ -18,6 +18,7 @@ from __future__ import annotations
 import bisect
 import contextlib
 import json
+import math
 import os
 import threading
 from pathlib import Path
@@ -391,6 +392,16 @@ def gemm_silu(x: torch.Tensor, w_gu: torch.Tensor, b_gu: torch.Tensor | None = N
     if out is None:
         out = torch.empty(M, N2 // 2, dtype=x.dtype, device=x.device)
     return _launch(x, w_gu, b_gu, out, EPI_SILU, ACT_NONE, ksplit, sk)
+
+
+def gemm_glu(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: float, shift: float) -> torch.Tensor:
+    """h [M, F] = g sigmoid(alpha g) (u + shift), g = min(x wg^T, limit), u = clamp(x wu^T, +-limit), w [2F, K] = wg | wu."""
+    M, K = x.shape
+    F = w.shape[0] // 2
+    out = torch.empty(M, F, dtype=x.dtype, device=x.device)
+    call("grag_gemm_tile_glu", ptr(x), ptr(w), ptr(out), x.stride(0), w.stride(0), F, M, F, K,
+         float(math.inf if limit is None else limit), float(alpha), float(shift))
+    return out
 
 
 # ---------------------------------------------------------------- decode regime (csrc/kernels/gemm_decode.hip)

@@ -1,0 +1,70 @@
+"""The gated unit in the tile GEMM's epilogue (csrc/kernels/gemm_tile.hip EPI_GLU) against 64-bit values: widths that end inside a
+wave's and a tile's columns, ragged rows, odd numbers of K steps, clamps and none; and the rule that takes it."""
+import pytest
+import torch
+
+from githubrepostorag_amd.ops import gemm as G
+from githubrepostorag_amd.ops import linear as L
+
+bf = torch.bfloat16
+
+
+def unit64(x, w, limit, alpha, shift):
+    z = x.double() @ w.double().t()
+    F = w.shape[0] // 2
+    g, u = z[:, :F], z[:, F:]
+    if limit is not None:
+        g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+    return g * torch.sigmoid(alpha * g) * (u + shift)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,F,K", [(1, 8, 128), (257, 120, 192), (300, 128, 128), (511, 136, 320), (600, 1000, 704), (256, 160, 64 * 7)])
+@pytest.mark.parametrize("limit,alpha,shift", [(None, 1.0, 0.0), (2.0, 1.702, 1.0)])
+@pytest.mark.parametrize("strided", [False, True])
+def test_gemm_glu(M, F, K, limit, alpha, shift, strided):
+    g = torch.Generator(device="cuda").manual_seed(M + F)
+    x = (torch.randn(M, K + 8, generator=g, device="cuda") * 2).to(bf)
+    x = x[:, 8:] if strided else x[:, :K].contiguous()
+    w = (torch.randn(2 * F, K, generator=g, device="cuda") * K ** -0.5).to(bf)
+    y, r = G.gemm_glu(x, w, limit, alpha, shift).double(), unit64(x, w, limit, alpha, shift)
+    # bf16 rounding of the result (2^-8 of it) and the fp32 sums: K 2^-24 of terms whose unit grows by at most a few
+    assert ((y - r).abs() <= r.abs() * 2 ** -8 + 40 * K * 2 ** -24).all()
+
+
+@pytest.mark.gpu
+def test_gemm_glu_special():
+    """Sums at the ends of fp32: the unit is 0 or the product there, not a number that is none."""
+    x = torch.zeros(3, 128, device="cuda", dtype=bf)
+    x[:, 0] = torch.tensor([1.0, -1.0, 1e-30], device="cuda").to(bf)
+    w = torch.zeros(16, 128, device="cuda", dtype=bf)
+    w[:8, 0], w[8:, 0] = 3e38, 1.0
+    y = G.gemm_glu(x, w, None, 1.0, 0.0).float().cpu()
+    assert (y[0] > 2.9e38).all() and (y[1] == 0).all() and (y[2].abs() < 1e-20).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,F,K,fused", [(1187, 8960, 128, True), (277, 8960, 128, False), (300, 136, 96, False), (40, 64, 128, False)])
+def test_glu_linear(M, F, K, fused, monkeypatch):
+    from githubrepostorag_amd.ops.elementwise import clamped_glu
+
+    seen = []
+    orig = G.gemm_glu
+    monkeypatch.setattr(G, "gemm_glu", lambda *a: seen.append(1) or orig(*a))
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, generator=g, device="cuda").to(bf)
+    w = (torch.randn(2 * F, K, generator=g, device="cuda") * K ** -0.5).to(bf)
+    y = L.glu_linear(x, w, 7.0)
+    assert bool(seen) == fused
+    r = unit64(x, w, 7.0, 1.702, 1.0)
+    # the two launches round gate and up as well: two more roundings of 2^-8, times what the unit makes of them
+    assert ((y.double() - r).abs() <= r.abs() * 2 ** -8 + (1e-3 if fused else 0.15)).all()
+    z = clamped_glu(L.linear(x, w), 7.0)
+    assert (z.double() - y.double()).norm() / z.double().norm() < 6e-3
+
+
+def test_glu_linear_cpu():
+    from githubrepostorag_amd.ops.elementwise import clamped_glu
+
+    x, w = torch.randn(5, 32), torch.randn(24, 32)
+    assert torch.equal(L.glu_linear(x, w, None, 1.0, 0.0), clamped_glu(L.linear(x, w), None, 1.0, 0.0))
