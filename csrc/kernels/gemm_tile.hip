@@ -58,18 +58,6 @@ __device__ __forceinline__ float gelu_tanh_f(float x) {
   const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
   return 0.5f * x * (2.f - 2.f * __builtin_amdgcn_rcpf(1.f + __expf(2.f * u)));
 }
-// g sigmoid(alpha g) (u + shift) with g = min(g, limit), u = clamp(u, +-limit).  The exponential is the bare instruction, the
-// quotient a reciprocal with one correction step; where the exponential passes 2^126 the sigmoid is 0.
-__device__ __forceinline__ float glu_f(float g, float u, float limit, float alpha, float shift) {
-  g = fminf(g, limit);
-  u = fminf(fmaxf(u, -limit), limit);
-  const float e = -1.4426950408889634f * (alpha * g);
-  const float d = 1.f + __builtin_amdgcn_exp2f(fminf(e, 126.f));
-  const float rc = __builtin_amdgcn_rcpf(d);
-  float q = g * rc;
-  q = fmaf(fmaf(-d, q, g), rc, q);
-  return (e > 126.f ? g * 0.f : q) * (u + shift);
-}
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return (uint32_t)(uint16_t)f2bits(lo) | ((uint32_t)(uint16_t)f2bits(hi) << 16);
 }

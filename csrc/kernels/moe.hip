@@ -463,9 +463,7 @@ struct MoeEpi {
   int gate_ld;
 };
 __device__ __forceinline__ float glu_unit(float g, float u, const MoeEpi& ep) {
-  g = fminf(g, ep.limit);
-  u = fminf(fmaxf(u, -ep.limit), ep.limit);
-  return g / (1.f + expf(-ep.alpha * g)) * (u + ep.shift);
+  return glu_f(g, u, ep.limit, ep.alpha, ep.shift);
 }
 __device__ __forceinline__ float relu2_unit(float v) {
   v = fmaxf(v, 0.f);
