@@ -102,12 +102,12 @@ __device__ __forceinline__ void st4(T* p, const f32x4_t& v) {
 // once for them.  grid (ceil(T / R), ceil(H / 1024)): row blockIdx.x + k gridDim.x.  Bound by its 12 bytes an element of
 // stream at many rows (the accurate tanh twice an element was as long as they): with four 2-byte accesses a thread and the
 // scaled division 8192 x 3584 83 us, now 60; 1187 x 3584 14.0 -> 10.7, 64 x 3584 3.5 -> 3.0.
-template <typename T, int R>
+template <typename T, int R, bool SPLIT>
 __global__ void __launch_bounds__(256)
-dyt_residual_vec_kernel(const T* __restrict__ y, float a1, const float* __restrict__ w1, const float* __restrict__ b1,
+dyt_residual_vec_kernel(const T* __restrict__ y, const float* __restrict__ planes, int S, size_t plane, float a1, const float* __restrict__ w1, const float* __restrict__ b1,
                         float* __restrict__ resid, const float* __restrict__ add_rows, const float* __restrict__ add_vec,
                         float a2, const float* __restrict__ w2, const float* __restrict__ b2, T* __restrict__ out, int T_,
-                        int H) {
+                        int H) {  // SPLIT: y is the sum of S fp32 planes, of a projection whose split-K reduction was left to here
   const int i = blockIdx.y * 1024 + threadIdx.x * 4;
   if (i >= H) return;
   const f32x4_t zero = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -117,11 +117,13 @@ dyt_residual_vec_kernel(const T* __restrict__ y, float a1, const float* __restri
     const int t = blockIdx.x + k * gridDim.x;
     const size_t at = (size_t)(R == 1 ? t : min(t, T_ - 1)) * H + i;
     x[k] = *reinterpret_cast<const f32x4_t*>(resid + at);
-    yv[k] = y != nullptr ? ld4(y + at) : zero;
+    if constexpr (SPLIT) yv[k] = plane_sum4(planes + at, plane, S);
+    else yv[k] = y != nullptr ? ld4(y + at) : zero;
     rv[k] = add_rows != nullptr ? *reinterpret_cast<const f32x4_t*>(add_rows + at) : zero;
   }
-  const f32x4_t w1v = y != nullptr ? *reinterpret_cast<const f32x4_t*>(w1 + i) : zero;
-  const f32x4_t b1v = y != nullptr ? *reinterpret_cast<const f32x4_t*>(b1 + i) : zero;
+  const bool has_y = SPLIT || y != nullptr;
+  const f32x4_t w1v = has_y ? *reinterpret_cast<const f32x4_t*>(w1 + i) : zero;
+  const f32x4_t b1v = has_y ? *reinterpret_cast<const f32x4_t*>(b1 + i) : zero;
   const f32x4_t av = add_vec != nullptr ? *reinterpret_cast<const f32x4_t*>(add_vec + i) : zero;
   const f32x4_t w2v = out != nullptr ? *reinterpret_cast<const f32x4_t*>(w2 + i) : zero;
   const f32x4_t b2v = out != nullptr ? *reinterpret_cast<const f32x4_t*>(b2 + i) : zero;
@@ -130,13 +132,13 @@ dyt_residual_vec_kernel(const T* __restrict__ y, float a1, const float* __restri
     const int t = blockIdx.x + k * gridDim.x;
     if (R > 1 && t >= T_) break;
     const size_t at = (size_t)t * H + i;
-    if (y != nullptr) {
+    if (has_y) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) x[k][e] += tanh_acc(a1 * yv[k][e]) * w1v[e] + b1v[e];
     }
     if (add_rows != nullptr) x[k] += rv[k];
     if (add_vec != nullptr) x[k] += av;
-    if (y != nullptr || add_rows != nullptr || add_vec != nullptr) *reinterpret_cast<f32x4_t*>(resid + at) = x[k];
+    if (has_y || add_rows != nullptr || add_vec != nullptr) *reinterpret_cast<f32x4_t*>(resid + at) = x[k];
     if (out != nullptr) {
       f32x4_t o;
 #pragma unroll
@@ -1674,8 +1676,8 @@ GRAG_API hipError_t grag_dyt_residual(const void* y, float a1, const float* w1, 
   if (H % 4 == 0 && al16(y) && al16(out) && al16(resid) && al16(w1) && al16(b1) && al16(w2) && al16(b2) && al16(add_rows) &&
       al16(add_vec)) {
 #define DYT_VEC(R)                                                                                                        \
-  hipLaunchKernelGGL((dyt_residual_vec_kernel<T, R>), dim3((T_ + R - 1) / R, (H + 1023) / 1024), dim3(256), 0, st,        \
-                     (const T*)y, a1, w1, b1, resid, add_rows, add_vec, a2, w2, b2, (T*)out, T_, H)
+  hipLaunchKernelGGL((dyt_residual_vec_kernel<T, R, false>), dim3((T_ + R - 1) / R, (H + 1023) / 1024), dim3(256), 0, st, \
+                     (const T*)y, nullptr, 0, (size_t)0, a1, w1, b1, resid, add_rows, add_vec, a2, w2, b2, (T*)out, T_, H)
     DT_DISPATCH(dt, {
       if ((long)((T_ + 3) / 4) * ((H + 1023) / 1024) >= DYT_ROWS_MIN) {
         DYT_VEC(4);
@@ -1688,6 +1690,20 @@ GRAG_API hipError_t grag_dyt_residual(const void* y, float a1, const float* w1, 
   }
   DT_DISPATCH(dt, hipLaunchKernelGGL(dyt_residual_kernel<T>, dim3(T_, (H + 1023) / 1024), dim3(256), 0, st, (const T*)y, a1, w1, b1,
                                      resid, add_rows, add_vec, a2, w2, b2, (T*)out, H);)
+  return hipGetLastError();
+}
+
+// The same with y = the sum of S fp32 planes [S][T][H] (bf16 activations, H a multiple of 4, aligned pointers).
+GRAG_API hipError_t grag_dyt_residual_splitk(const float* planes, int S, float a1, const float* w1, const float* b1, float* resid,
+                                             const float* add_rows, const float* add_vec, float a2, const float* w2,
+                                             const float* b2, void* out, int T_, int H, hipStream_t st) {
+  if (T_ <= 0) return hipSuccess;
+  auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  if (planes == nullptr || S < 1 || H % 4 != 0 || !al16(planes) || !al16(out) || !al16(resid) || !al16(w1) || !al16(b1) || !al16(w2) ||
+      !al16(b2) || !al16(add_rows) || !al16(add_vec))
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL((dyt_residual_vec_kernel<bf16, 1, true>), dim3(T_, (H + 1023) / 1024), dim3(256), 0, st, (const bf16*)nullptr,
+                     planes, S, (size_t)T_ * H, a1, w1, b1, resid, add_rows, add_vec, a2, w2, b2, (bf16*)out, T_, H);
   return hipGetLastError();
 }
 

@@ -31,7 +31,7 @@ import torch
 
 from ..ops.attention import AttnMetadata, sink_attention
 from ..ops.elementwise import rope_table, rope_vnorm_store
-from ..ops.linear import glu_linear, linear
+from ..ops.linear import glu_linear, linear, linear_deferred
 from ..ops.norm import dyt_residual, embed_gather_f32
 from ..ops.recurrent import decay_attention, gated_rmsnorm, mingru_scan
 from ..parallel.comm import Group
@@ -263,7 +263,7 @@ class ZofesunModel:
         p = linear(h, L.wp)
         if m.kind == "mingru":
             zo, xo, go = L.off
-            return linear(mingru_scan(p, zo, xo, go, L.bz, L.bx, state, meta, m.width), L.wo)
+            return linear_deferred(mingru_scan(p, zo, xo, go, L.bz, L.bx, state, meta, m.width), L.wo)
         l, r = m.left, m.right
         lq, lk, lv, rq, rk, rv, rg = L.off
         kc, vc = kv
@@ -274,7 +274,7 @@ class ZofesunModel:
         sink_attention(q, kc, vc, meta, l.scale, L.sinks, out=both[:, :nl], out_scale=m.left_scale)
         o = decay_attention(p, rq, rk, rv, L.decay, state, meta, r.heads, r.dim, r.vdim)
         gated_rmsnorm(o, L.rnorm, p, rg, self.cfg.norm_eps, both[:, nl:], out_scale=m.right_scale)
-        return linear(both, L.wo)
+        return linear_deferred(both, L.wo)
 
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor, meta: AttnMetadata, kv_caches,
                 state=None, taps: list | None = None) -> torch.Tensor:
@@ -297,7 +297,7 @@ class ZofesunModel:
             y, post = self._mixer(L, h, positions, meta, kv_caches[ri], state[ri]), L.norm1b
             if L.wgu is not None:
                 h = dyt_residual(x, y, post, pre=L.norm2, out_dtype=dt)
-                y, post = linear(glu_linear(h, L.wgu, L.spec.mlp.limit, GLU_SIGMOID_SLOPE), L.wd), L.norm2b
+                y, post = linear_deferred(glu_linear(h, L.wgu, L.spec.mlp.limit, GLU_SIGMOID_SLOPE), L.wd), L.norm2b
         if taps is not None and self.runs:
             dyt_residual(x, y, post, out_dtype=dt)
             y = post = None

@@ -150,7 +150,8 @@ def dyt_residual(resid: torch.Tensor, y: torch.Tensor | None = None, post=None, 
     """One pass over the fp32 residual stream ``resid`` [T, H] (updated in place):
     resid += dyt_post(y) (+ add_rows [T, H] fp32) (+ add_vec [H] fp32), then returns dyt_pre(resid) in
     ``out_dtype`` (None without ``pre``).  ``post`` / ``pre`` are (alpha, w fp32 [H], b fp32 [H]) triples:
-    the norm that closes one sublayer and the norm that opens the next, fused at the sublayer boundary."""
+    the norm that closes one sublayer and the norm that opens the next, fused at the sublayer boundary.  ``y`` may be
+    a projection whose split-K reduction was deferred (ops/linear.py linear_deferred): its planes are summed here."""
     assert resid.dtype == torch.float32 and resid.is_contiguous()
     T, H = resid.shape
     if not _on_gpu(resid):
@@ -162,6 +163,13 @@ def dyt_residual(resid: torch.Tensor, y: torch.Tensor | None = None, post=None, 
             resid += add_vec
         return None if pre is None else dyt_ref(resid, *pre).to(out_dtype)
     out = torch.empty(T, H, dtype=out_dtype, device=resid.device) if pre is not None else None
+    if isinstance(y, SplitKPartial):
+        if out_dtype == torch.bfloat16 and y.shape == resid.shape:
+            a2, w2, b2 = pre if pre is not None else (0.0, None, None)
+            call("grag_dyt_residual_splitk", ptr(y.planes), y.S, float(post[0]), ptr(post[1]), ptr(post[2]), ptr(resid),
+                 ptr(add_rows), ptr(add_vec), float(a2), ptr(w2), ptr(b2), ptr(out), T, H)
+            return out
+        y = y.materialize()
     if y is not None:
         assert y.dtype == out_dtype and y.is_contiguous() and y.shape == resid.shape
     a1, w1, b1 = post if y is not None else (0.0, None, None)

@@ -91,3 +91,22 @@ def test_rope_store_value_norm(d, vd, rd, H, G, T):
     for a, b in zip(*outs):
         # both round once from fp32: half a unit each way, plus a rotation's cancellation in fp32
         assert ((a - b).abs() <= a.abs() * 2 ** -7 + 1e-5).all()
+
+
+@pytest.mark.parametrize("T,H,S", [(1, 8, 1), (3, 1032, 7), (300, 64, 9), (2, 3584, 17)])
+def test_dyt_residual_splitk(T, H, S):
+    """The planes of a deferred split-K product in place of its sum."""
+    from githubrepostorag_amd.ops.gemm import SplitKPartial
+    from githubrepostorag_amd.ops.norm import dyt_residual
+
+    g = torch.Generator().manual_seed(T + H)
+    planes, r = rnd(g, S, T, H).to(dev), rnd(g, T, H)
+    po, pr, av = (0.7, rnd(g, H), rnd(g, H)), (0.9, rnd(g, H), rnd(g, H)), rnd(g, H)
+    on = lambda t: (t[0], t[1].to(dev), t[2].to(dev))
+    r1 = r.clone().to(dev)
+    h = dyt_residual(r1, SplitKPartial(planes, S, T, H, bf), on(po), None, av.to(dev), on(pr))
+    x = r.double() + torch.tanh(po[0] * planes.double().sum(0).cpu()) * po[1].double() + po[2].double() + av.double()
+    # a handful of fp32 roundings of terms of a few units, S of them in the sum
+    assert (r1.cpu().double() - x).abs().max() <= 4e-6 + S * 1e-6
+    o = torch.tanh(pr[0] * x) * pr[1].double() + pr[2].double()
+    assert ((h.cpu().double() - o).abs() <= o.abs() * 2 ** -8 + 4e-5 + S * 4e-6).all()
