@@ -23,23 +23,22 @@ namespace grag {
 
 constexpr int SP_KT = 64;         // keys per tile
 constexpr int SP_MAXB = 2048;     // cache blocks a workgroup can walk (32 K keys): its part of the block table, in LDS
-constexpr int SP_ROWS = 128;      // rows of a workgroup: 8 waves of 16
 
-template <int D, bool CAP>
-__global__ void __launch_bounds__(512, 4) sink_prefill_kernel(const SinkArgs p) {
+template <int D, bool CAP, int NW>
+__global__ void __launch_bounds__(64 * NW, 4) sink_prefill_kernel(const SinkArgs p) {
   constexpr int RB = 2 * D, CPR = D / 8, NC = D / 32, ND = D / 16, TILE = SP_KT * RB;
-  constexpr int PPW = TILE / 1024 / 8, RPP = 1024 / RB;
+  constexpr int ROWS = 16 * NW, PPW = TILE / 1024 / NW, RPP = 1024 / RB;
   static_assert(PPW >= 1 && SP_BS % (PPW * RPP) == 0, "a wave's DMA rows sit in one cache block");
   __shared__ __attribute__((aligned(16))) char smem[2 * 2 * TILE];
   __shared__ int bt_lds[SP_MAXB];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h4 = lane >> 4, li = lane & 15;
   const int seq = blockIdx.x / p.tiles, kvh = blockIdx.y;
-  const int row_base = (p.tiles - 1 - (int)(blockIdx.x % p.tiles)) * SP_ROWS;  // (the longest walks first)
+  const int row_base = (p.tiles - 1 - (int)(blockIdx.x % p.tiles)) * ROWS;  // (the longest walks first)
   const int q0 = p.q_start[seq], qlen = p.q_start[seq + 1] - q0, ctx = p.ctx_len[seq], pos0 = ctx - qlen;
   const int R = p.R, nrows = qlen * R;
   if (row_base >= nrows) return;
-  const int last_row = min(row_base + SP_ROWS, nrows) - 1;
+  const int last_row = min(row_base + ROWS, nrows) - 1;
   const int kv_hi = min(ctx, pos0 + last_row / R + 1);
   // tiles: nkeep of kept keys, then those from the first key that any row sees.  Table entry i of the walk is cache block i, or
   // i + skip behind the kept ones.
@@ -49,7 +48,7 @@ __global__ void __launch_bounds__(512, 4) sink_prefill_kernel(const SinkArgs p) 
   const int kb = nkeep * (SP_KT / SP_BS), skip = kfirst / SP_BS - kb;
   const int nb = min((kv_hi + SP_BS - 1) / SP_BS - skip, SP_MAXB);
   const int* bt = p.bt + (size_t)seq * p.bt_stride;
-  for (int i = threadIdx.x; i < nb; i += 512) {
+  for (int i = threadIdx.x; i < nb; i += 64 * NW) {
     int b = bt[i < kb ? i : i + skip];
     if (!index_ok(b, p.nblocks, ERR_BLOCK_PREFILL)) b = 0;  // reported; block 0 read instead of faulting
     bt_lds[i] = b;
@@ -212,7 +211,7 @@ bool sink_prefill_takes(int d, int vd, int v_ld, int BS, int max_q_len, int R, i
   if ((d != 64 && d != 128) || vd != d || v_ld != d || BS != SP_BS || max_q_len < 16 || out_ld % 4) return false;
   if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15 || (uintptr_t)out & 7) return false;
   // the most keys a workgroup walks: the kept ones and its rows' windows (or their blocks, two where the rows straddle), or all
-  const long rows = SP_ROWS / R + 2;
+  const long rows = 128 / R + 2;
   long keys = (long)bt_stride * BS;
   if (window > 0) keys = keys < window + rows + keep + 3 * SP_KT ? keys : window + rows + keep + 3 * SP_KT;
   if (chunk > 0) keys = keys < chunk + rows + keep + 3 * SP_KT ? keys : chunk + rows + keep + 3 * SP_KT;
@@ -229,17 +228,25 @@ hipError_t sink_prefill_launch(const void* q, const void* k, const void* v, void
   a.out_ld = out_ld, a.bt_stride = bt_stride, a.H = H, a.G = G, a.R = H / G, a.nblocks = nblocks;
   a.gate_ld = gate_ld, a.chunk = chunk, a.window = window, a.keep = keep;
   a.scale = scale, a.out_scale = out_scale, a.softcap = softcap;
-  const long tiles = ((long)max_q_len * a.R + SP_ROWS - 1) / SP_ROWS;
+  // 128 rows a workgroup, or 64 where those are few for the chip: a walk's time is the chain of its tiles, shorter with one wave a
+  // SIMD than with two.  us of 128 / 64 rows, all keys: 12 / 2 heads, 300 tokens 15 / 13, 1187 (112 workgroups) 43 / 37, 2048
+  // (192) 67 / 55; 28 / 4 heads, 1500 (332) 63 / 53; past the line 12 x 300 (360) 22 / 24, 28 / 4 heads, 2048 (448) 76 / 90.
+  long tiles = ((long)max_q_len * a.R + 127) / 128;
+  const bool few = tiles * nseq * G <= 340;
+  if (few) tiles = ((long)max_q_len * a.R + 63) / 64;
   if (tiles * nseq > 0x7fffffffL || G > 65535) return hipErrorInvalidValue;
   a.tiles = (int)tiles;
   const dim3 grid((unsigned)(tiles * nseq), G);
-  if (d == 64) {
-    if (softcap > 0.f) hipLaunchKernelGGL((sink_prefill_kernel<64, true>), grid, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((sink_prefill_kernel<64, false>), grid, dim3(512), 0, st, a);
-  } else {
-    if (softcap > 0.f) hipLaunchKernelGGL((sink_prefill_kernel<128, true>), grid, dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((sink_prefill_kernel<128, false>), grid, dim3(512), 0, st, a);
+#define SINK_PREFILL(DD, CAP)                                                                                        \
+  {                                                                                                                  \
+    if (few) hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 4>), grid, dim3(256), 0, st, a);                       \
+    else hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 8>), grid, dim3(512), 0, st, a);                           \
   }
+  if (d == 64 && softcap > 0.f) SINK_PREFILL(64, true)
+  else if (d == 64) SINK_PREFILL(64, false)
+  else if (softcap > 0.f) SINK_PREFILL(128, true)
+  else SINK_PREFILL(128, false)
+#undef SINK_PREFILL
   return hipGetLastError();
 }
 
