@@ -56,7 +56,7 @@ template <> __device__ __forceinline__ void st4s<bf16>(bf16* p, f32x4_t v) {
 
 // ------------------------------------------------------------------------------------------------ causal convolution
 constexpr int CONV_MAX_TAPS = 16;
-constexpr int CONV_TT = 16;  // tokens per workgroup
+constexpr int CONV_TT = 8;  // tokens per workgroup
 
 // out [T][C] = SiLU(b[c] + sum_j w[c][j] in[t - (taps - 1) + j][c]), in = proj columns coff .. coff + C; inputs before
 // the portion come from cstate [slots][taps - 1][C] (oldest first), zeros for a sequence that starts at position 0.
@@ -117,14 +117,20 @@ causal_conv_kernel(const T* __restrict__ proj, int ld, int coff, int C, int taps
 
 // The same for up to MT taps and rows in groups of four channels (C, ld, coff multiples of 4, aligned pointers): a thread
 // owns four channels of a token tile, all of whose inputs are in flight before the first sum.  The weights stand at the
-// end of MT places (zeros before them), so every register index is known when the kernel is compiled.
+// end of MT places (zeros before them), so every register index is known when the kernel is compiled.  The pool's update is
+// the first tile's, without a second kernel (mode bit 2 means nothing here).
 // grid (ceil(C / 1024), ceil(max_q_len / CONV_TT), nseq); the mode bits as above.
+// Bound by its 4 bytes an element and, at few tokens, by a thread's first loads: sixteen 4-byte loads of weights 64 bytes apart
+// touched more lines than the tile's inputs.  us before and now, with 4 taps, bf16: 3 x 1365 tokens x 3840 channels 36 and 20,
+// x 12288 74 and 47; 1 x 8192 x 7168 81 and 54; 64 x 1 x 7168 7.6 and 4.2.  (Tokens a tile, with this form's weights: 16 29 /
+// 57 / 63 us, 8 23 / 51 / 54, with the second kernel's 5.)
 template <typename T, int MT>
 __global__ void __launch_bounds__(256)
 causal_conv_vec_kernel(const T* __restrict__ proj, int ld, int coff, int C, int taps, const float* __restrict__ w,
                        const float* __restrict__ b, T* __restrict__ cstate, const int* __restrict__ slots,
                        const int* __restrict__ q_start, const int* __restrict__ ctx_len, T* __restrict__ out, int nslots,
                        int mode) {
+  static_assert(MT - 1 < CONV_TT, "only the first tile reads the pool");
   const int seq = blockIdx.z, c = (blockIdx.x * 256 + threadIdx.x) * 4;
   const int qa = q_start[seq], qlen = q_start[seq + 1] - qa;
   const int t0 = blockIdx.y * CONV_TT;
@@ -149,10 +155,19 @@ causal_conv_vec_kernel(const T* __restrict__ proj, int ld, int coff, int C, int 
     }
   }
   float wt[MT][4];
+  if (MT == 4 && taps == MT && (reinterpret_cast<uintptr_t>(w) & 15) == 0) {  // a channel's weights in one access
 #pragma unroll
-  for (int j = 0; j < MT; ++j)
+    for (int v = 0; v < 4; ++v) {
+      const f32x4_t x = *reinterpret_cast<const f32x4_t*>(w + (size_t)(c + v) * 4);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) wt[j][v] = j >= lead ? w[(size_t)(c + v) * taps + j - lead] : 0.f;
+      for (int j = 0; j < 4; ++j) wt[j][v] = x[j];
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) wt[j][v] = j >= lead ? w[(size_t)(c + v) * taps + j - lead] : 0.f;
+  }
   const f32x4_t bias = b ? *reinterpret_cast<const f32x4_t*>(b + c) : f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int tt = 0; tt < CONV_TT; ++tt) {
@@ -175,17 +190,19 @@ causal_conv_vec_kernel(const T* __restrict__ proj, int ld, int coff, int C, int 
       win[MT - 2] = cur[tt];
     }
   }
-  if ((mode & 4) && taps > 1 && index_ok(slot, nslots, ERR_SAMPLER_SLOT)) {  // (t0 is 0: one tile holds the portion)
+  // the first tile's threads, the only ones that read the pool (taps - 1 < CONV_TT), leave the portion's last inputs there
+  if (t0 == 0 && taps > 1 && index_ok(slot, nslots, ERR_SAMPLER_SLOT)) {
     T* dst = cstate + (size_t)slot * (taps - 1) * C + c;
 #pragma unroll
     for (int j = 0; j < MT - 1; ++j) {
       if (j < lead) continue;
-      st4s(dst + (size_t)(j - lead) * C, win[j]);
+      const f32x4_t v = qlen <= CONV_TT ? win[j] : ld4s(in + (size_t)(qlen - (MT - 1) + j) * ld);
+      st4s(dst + (size_t)(j - lead) * C, v);
     }
   }
 }
 
-// the pool after the step: the last taps - 1 inputs of every sequence (runs after the kernel above, on the same stream).
+// the pool after the step: the last taps - 1 inputs of every sequence (runs after causal_conv_kernel, on the same stream).
 // grid (ceil(C / 256), nseq): a thread reads all it needs of its channel before it writes.
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -801,7 +818,7 @@ GRAG_API hipError_t grag_causal_conv(const void* proj, int ld, int coff, int C, 
     else
       hipLaunchKernelGGL(causal_conv_kernel<T>, grid, dim3(256), 0, st, (const T*)proj, ld, coff, C, taps, w, b,
                        (T*)cstate, slots, q_start, ctx_len, (T*)out, nslots, mode);
-    if (taps > 1 && !one_tile)
+    if (taps > 1 && !one_tile && !vec)
       hipLaunchKernelGGL(conv_state_kernel<T>, dim3((C + 255) / 256, nseq), dim3(256), 0, st, (const T*)proj, ld, coff, C,
                          taps, (T*)cstate, slots, q_start, ctx_len, nslots);
   })
