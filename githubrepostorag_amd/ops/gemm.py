@@ -205,11 +205,21 @@ def unmeasured_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
     launches back to back over 8 shapes of N 384-3072, K 384-768 at 277-24000 rows, library / owned there is 1.19 in the
     median of 13 points (0.90-1.48: 2304 x 768 at 7300 rows 64 -> 43 us, at 24000 106 -> 95, at 8192 38 -> 42); with fewer tiles the
     library's smaller ones win (0.3-1.0).  No stream-K there: a part's slab out and in costs more than the K steps it
-    saves (3072 x 768 at 24000 rows: 149 us, whole tiles 124).  Deeper contractions are level in the median (0.94-1.05)
-    and stay."""
-    if (N, K, 0) in _prefill_table() or K > 1024 or max(M, N) * K >= 1 << 30:
+    saves (3072 x 768 at 24000 rows: 149 us, whole tiles 124).
+
+    Deeper contractions are level in the median (0.94-1.05) and stay, but for one round and a thin rest of tiles at K >= 2048:
+    every tile of the rest cut into four equal K parts is a quarter of a round where others pay one -- 1.05 in the median
+    of 11 points (0.99-1.10; 768 x 3072 at 24000 rows 114 -> 105, 3584 x 7168 at 5000 223 -> 203), rows that pad a tenth of
+    the tiles or more left out (37888 x 3584 at 277 rows 0.87)."""
+    if (N, K, 0) in _prefill_table() or M < PREFILL_MIN_M or max(M, N) * K >= 1 << 30:
         return None
-    return (1, 0) if -(-M // 256) * -(-N // 256) > _num_cus() else None
+    tiles, ncu = -(-M // 256) * -(-N // 256), _num_cus()
+    if K <= 1024:
+        return (1, 0) if tiles > ncu else None
+    tail = tiles - ncu
+    if K >= 2048 and 0 < tail <= ncu // 4 and M * N >= 0.9 * 65536 * tiles and sk_ok(M, N, K, 1, -4 * tail):
+        return 1, -4 * tail
+    return None
 
 
 def schedule(M: int, N: int, K: int, silu: bool = False) -> tuple[int, int]:

@@ -19,10 +19,16 @@ def test_rule():
     assert G.unmeasured_plan(8192, 2304, 1088) is None         # deep K
     assert G.unmeasured_plan(1 << 21, 2304, 1024) is None      # operands past the kernel's 32-bit byte offsets
     assert G.schedule(24000, 3072, 768) == (1, 0)
+    # one round and a rest of at most a quarter: four K parts a tile
+    assert G.unmeasured_plan(24000, 768, 3072) == G.schedule(24000, 768, 3072) == (1, -104)
+    assert G.unmeasured_plan(21504, 768, 3072) is None          # 252 tiles
+    assert G.unmeasured_plan(27648, 768, 3072) is None          # 324: a rest of 68
+    assert G.unmeasured_plan(277, 38144, 4096) is None          # rows that are mostly padding
+    assert G.unmeasured_plan(24000, 768, 1984) is None
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(65537, 72, 128), (300, 32904, 192), (8191, 2120, 768), (3001, 5624, 960)])
+@pytest.mark.parametrize("M,N,K", [(65537, 72, 128), (300, 32904, 192), (8191, 2120, 768), (3001, 5624, 960), (22000, 768, 2304), (5100, 3584, 2304)])
 @pytest.mark.parametrize("bias,strided", [(False, False), (True, True)])
 def test_linear_unmeasured(M, N, K, bias, strided):
     g = torch.Generator(device="cuda").manual_seed(M)
