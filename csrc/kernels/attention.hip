@@ -165,7 +165,14 @@ __global__ __launch_bounds__(64 * NW, D <= 64 && NW == 4 ? 4 : 1) void attn_fwd_
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int h4 = lane >> 4, li = lane & 15;
-  const int seq = blockIdx.x / p.tiles_per_seq, tile = blockIdx.x % p.tiles_per_seq;
+  // Neighbouring workgroups go to the eight XCDs in turn: of every eight sequences each XCD gets one, with all its row tiles,
+  // which read the same K / V; which one turns with the head, so that long sequences meet every XCD (the sequences behind the
+  // last eight stay dealt tile by tile).  128 sequences of 60-320 rows, 12 heads, D = 64 61 -> 56 us (65 without the turn),
+  // D = 32 43 -> 39; 64 of 500-512 129 -> 112, 113 -> 71.
+  const int grouped = gridDim.x / p.tiles_per_seq / 8 * 8 * p.tiles_per_seq, bj = blockIdx.x >> 3;
+  const bool in_group = (int)blockIdx.x < grouped;
+  const int seq = in_group ? bj / p.tiles_per_seq * 8 + ((blockIdx.x + blockIdx.y) & 7) : blockIdx.x / p.tiles_per_seq;
+  const int tile = in_group ? bj % p.tiles_per_seq : blockIdx.x % p.tiles_per_seq;
   const int kvh = blockIdx.y, split = blockIdx.z;
   const int q0 = p.q_start[seq], qlen = p.q_start[seq + 1] - q0;
   const int ctx = p.ctx_len[seq];

@@ -33,7 +33,7 @@ def test_layernorm_rows(H, T, bias, res):
 
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("causal", [False, True])
-@pytest.mark.parametrize("lens", [[1, 63, 64, 65], [17, 128, 129, 2, 200], [15, 16, 3]])
+@pytest.mark.parametrize("lens", [[1, 63, 64, 65], [17, 128, 129, 2, 200], [15, 16, 3], [5, 70, 64, 1, 130, 20, 3, 65, 33] * 2])
 def test_varlen_attention_edges(D, causal, lens):
     from githubrepostorag_amd.ops.attention import varlen_attention, varlen_attention_ref
 
