@@ -6,10 +6,10 @@ ingest/src/app/services/vector_write_service.py:117).
 Varlen packing: sequences are concatenated token-major (no pad tokens are
 ever computed — the reference pads each sentence-transformers batch of 32 to
 its longest member).  Per layer:
-  qkv = h W_qkv^T + b                      (hipBLASLt, bias epilogue)
+  qkv = h W_qkv^T + b                      (linear(): tile kernel or hipBLASLt)
   a   = bidirectional MFMA attention       [grag_varlen_attention]
   h   = LN(a W_o^T + b_o + h)              [grag_layernorm: bias+residual+LN]
-  f   = GELU(h W_1^T + b_1)                [grag_bias_act]
+  f   = GELU(h W_1^T + b_1)                [tile kernel's epilogue, else grag_bias_act]
   h   = LN(f W_2^T + b_2 + h)              [grag_layernorm]
 then masked-mean or CLS pooling + L2 normalisation [grag_pool_l2norm] writing
 the fp32 vector and the bf16 copy the index stores.
