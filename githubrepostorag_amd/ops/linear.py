@@ -327,6 +327,20 @@ def _differentiated(*ts) -> bool:
     return fwAD._current_level >= 0 or (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts))
 
 
+def _plain_product(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> bool:
+    """Whether the owned kernel may stand in for the library's product of x [M, K] and w: it checks no operand against
+    another, and it knows no derivative, trace, dispatch mode or autocast.  What fails here goes to the library, which
+    handles or refuses it."""
+    at = x.get_device()
+    if w.dim() != 2 or w.size(1) != x.size(1) or w.get_device() != at or w.dtype != x.dtype or w.is_meta:
+        return False
+    if b is not None and not (b.dim() == 1 and b.size(0) == w.size(0) and b.get_device() == at and b.dtype == x.dtype
+                              and not b.is_meta and b.is_contiguous() and b.data_ptr() % 16 == 0):
+        return False
+    return not (_differentiated(x, w, b) or torch.is_autocast_enabled() or torch._C._get_tracing_state() is not None
+                or torch._C._len_torch_dispatch_stack() or at >= 0 and at != torch.cuda.current_device())
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> torch.Tensor:
     """y = x @ w.T (+ b); w is [out, in] (K-contiguous, TN GEMM)."""
     if not x.is_cuda:
@@ -349,7 +363,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> t
             p = _tile.prefill_plan(M, N, K)
             if p is not None:
                 return _tile.gemm(x, w, b, ksplit=p[0], sk=p[1])
-            if not _differentiated(x, w, b) and (b is None or (b.dtype == x.dtype and b.is_contiguous() and b.numel() == N)):
+            if _plain_product(x, w, b):
                 p = _tile.unmeasured_plan(M, N, K)
                 return _tile.gemm(x, w, b, ksplit=p[0], sk=p[1])
             return torch.nn.functional.linear(x, w, b)
@@ -374,7 +388,7 @@ def glu_linear(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: flo
     last round that is nearly empty, rows that are mostly padding, or few tiles).  Error against 64 bits 0.59 of the two
     launches', which round gate and up to bf16 between them."""
     if (x.is_cuda and x.dim() == 2 and x.shape[0] >= _tile.PREFILL_MIN_M and w.shape[0] % 16 == 0 and _tile.supported(x, w)
-            and not _differentiated(x, w)):
+            and _plain_product(x, w)):
         M, N = x.shape[0], w.shape[0]
         tiles, ncu = -(-M // 256) * -(-N // 256), _tile._num_cus()
         if M * N >= GLU_FILL * 65536 * ncu * -(-tiles // ncu):

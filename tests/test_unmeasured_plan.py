@@ -2,6 +2,7 @@
 that kernel against 64-bit products over the layouts it accepts there."""
 import pytest
 import torch
+from torch.utils.flop_counter import FlopCounterMode
 
 from githubrepostorag_amd.ops import gemm as G
 from githubrepostorag_amd.ops import linear as L
@@ -51,3 +52,38 @@ def test_linear_unmeasured_gradient():
     w = torch.randn(2304, 768, device="cuda").to(bf)
     L.linear(x, w).sum().backward()
     assert x.grad is not None and torch.isfinite(x.grad).all()
+
+
+def test_what_the_library_keeps():
+    """Operands that do not fit each other, and calls under a trace, a dispatch mode or autocast, are the library's."""
+    x, w, b = torch.randn(4, 128).to(bf), torch.randn(8, 128).to(bf), torch.randn(16).to(bf)
+    assert L._plain_product(x, w) and L._plain_product(x, w, b[:8])
+    for bad in ((x, w[:, :64]), (x, torch.randn(8, 192).to(bf)), (x, w.to("meta")), (x, w.float()), (x, w, b), (x, w, b[1:9]),
+                (x, w, b[::2]), (x, w, b[:8].float()), (x, w, b[:8].to("meta")), (x, w, b[:1]), (x, w, b[:8].view(1, 8))):
+        assert not L._plain_product(*bad)
+    seen = []
+
+    def f(t):
+        seen.append(L._plain_product(t, w))
+        return t + 1
+    torch.jit.trace(f, (x,), check_trace=False)
+    torch.set_autocast_enabled("cuda", True)
+    try:
+        f(x)
+    finally:
+        torch.set_autocast_enabled("cuda", False)
+    with FlopCounterMode(display=False):
+        f(x)
+    f(x.clone().requires_grad_())
+    assert seen == [False] * 4
+
+
+@pytest.mark.gpu
+def test_linear_refuses_what_does_not_fit():
+    assert G.prefill_plan(7400, 2304, 768) is None  # (the rule is asked, not the table)
+    x = torch.randn(7400, 768, device="cuda").to(bf)
+    for w in (torch.randn(2304, 704, device="cuda").to(bf), torch.randn(2304, 832, device="cuda").to(bf), torch.randn(2304, 768).to(bf)):
+        with pytest.raises(RuntimeError):
+            L.linear(x, w)
+        with pytest.raises(RuntimeError):
+            L.glu_linear(x, w, 7.0)
