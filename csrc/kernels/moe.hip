@@ -356,40 +356,52 @@ moe_route_mfma_kernel(const T* __restrict__ h, int ld, const float* __restrict__
   else select(Lanes<64>());
 }
 
-// A few tokens (decode rows): one workgroup per token, one wave per logit row (rows w, w + 4, ...), the lanes split the
-// row's columns (8 consecutive ones per lane and step when `vec`), so the row's loads are all in flight at once and
-// the sum is a wave reduction: the latency of a step no longer scales with the model width.
+// A few tokens (decode rows): one workgroup per token, one wave per logit row (rows w, w + 16, ...), the lanes split the
+// row's columns (8 consecutive ones per lane and step when `vec`) and the sum is a wave reduction.  Bound by round trips to
+// memory: the loads of UN steps (2048 columns) are all issued before their first product.  us with four waves that waited
+// for each step and now, 64 tokens: 17 rows of 3584 12.0 and 9.5, behind an expert layer whose weights push the rows out of
+// the caches 24 and 13; 65 rows 30.0 and 21.4; 17 of 1536 9.2 and 8.0 (with UN = 8 9.5); 8 of 8192 10.5 and 8.8.
 template <typename T>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(1024)
 moe_route_rows_kernel(const T* __restrict__ h, int ld, const float* __restrict__ wr, int W, int E, int R, int top,
                       int ngroups, int keep, int* __restrict__ ids, float* __restrict__ wts,
                       float* __restrict__ sgate, int vec, RouteExtra rx) {
   __shared__ float z[RT_MAXR + 1];
+  constexpr int UN = 4;  // steps whose loads are under way together
   const int t = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const T* hr = h + (size_t)t * ld;
-  for (int r = wid; r < R; r += 4) {
+  for (int r = wid; r < R; r += 16) {
     const float* w = wr + (size_t)r * W;
     float a = 0.f;
     if (vec) {
-      for (int k = lane * 8; k < W; k += 512) {
-        float hv[8];
-        if (sizeof(T) == 2) {
-          const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(hr + k);
+      for (int k0 = lane * 8; k0 < W; k0 += 512 * UN) {
+        f32x4_t w0[UN], w1[UN];
+        bf16x8_t hb[UN];
+        f32x4_t hf[UN][2];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) hv[i] = bits2f(v[i]);
-        } else {
+        for (int u = 0; u < UN; ++u) {
+          const int k = k0 + 512 * u < W ? k0 + 512 * u : k0;  // (past the row: read, not added)
+          if constexpr (sizeof(T) == 2) {
+            hb[u] = *reinterpret_cast<const bf16x8_t*>(hr + k);
+          } else {
+            hf[u][0] = *reinterpret_cast<const f32x4_t*>(hr + k);
+            hf[u][1] = *reinterpret_cast<const f32x4_t*>(hr + k + 4);
+          }
+          w0[u] = *reinterpret_cast<const f32x4_t*>(w + k);
+          w1[u] = *reinterpret_cast<const f32x4_t*>(w + k + 4);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // (the loads stay together; a branch below would pull them apart)
 #pragma unroll
-          for (int i = 0; i < 8; i += 4) {
-            const f32x4_t v = *reinterpret_cast<const f32x4_t*>(hr + k + i);
+        for (int u = 0; u < UN; ++u) {
+          const bool in = k0 + 512 * u < W;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) hv[i + j] = v[j];
+          for (int i = 0; i < 8; ++i) {
+            float hv;
+            if constexpr (sizeof(T) == 2) hv = bits2f(hb[u][i]);
+            else hv = hf[u][i >> 2][i & 3];
+            a = fmaf(in ? hv : 0.f, in ? (i < 4 ? w0[u][i & 3] : w1[u][i & 3]) : 0.f, a);
           }
         }
-        const f32x4_t w0 = *reinterpret_cast<const f32x4_t*>(w + k), w1 = *reinterpret_cast<const f32x4_t*>(w + k + 4);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) a = fmaf(hv[i], w0[i], a);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) a = fmaf(hv[4 + i], w1[i], a);
       }
     } else {
       for (int k = lane; k < W; k += 64) a = fmaf(ldm(hr + k), w[k], a);
@@ -1401,7 +1413,7 @@ GRAG_API hipError_t grag_moe_route(const void* h, int ld, const float* wr, int W
     return hipGetLastError();
   }
   if (T_ <= 128) {  // decode rows, short portions
-    DT_DISPATCH(dt, hipLaunchKernelGGL(moe_route_rows_kernel<T>, dim3(T_), dim3(256), 0, st, (const T*)h, ld, wr, W, E, R,
+    DT_DISPATCH(dt, hipLaunchKernelGGL(moe_route_rows_kernel<T>, dim3(T_), dim3(1024), 0, st, (const T*)h, ld, wr, W, E, R,
                                        top, ngroups, keep, ids, wts, sgate, vec, rx);)
     return hipGetLastError();
   }

@@ -39,9 +39,13 @@ def test_moe_tile(unit, limit, W, F):
 @pytest.mark.parametrize("T,W,E,extra,groups,score,dtype", [
     (129, 1536, 16, 1, 4, "softmax", torch.bfloat16), (143, 40, 16, 0, 1, "sigmoid", torch.bfloat16),
     (200, 520, 30, 2, 5, "softmax", torch.float32), (161, 8, 64, 0, 8, "sigmoid", torch.bfloat16),
-    (130, 3592, 63, 1, 1, "softmax", torch.float32)])
-def test_router_on_matrix_cores(T, W, E, extra, groups, score, dtype):
-    """Step-sized token counts against the plain fp32 router: widths that end inside a wave's step, rows past a tile."""
+    (130, 3592, 63, 1, 1, "softmax", torch.float32),
+    (128, 2056, 16, 1, 4, "softmax", torch.bfloat16), (1, 8, 3, 0, 1, "sigmoid", torch.bfloat16),
+    (64, 2048, 64, 1, 8, "softmax", torch.float32), (65, 6152, 17, 0, 1, "softmax", torch.bfloat16),
+    (127, 5128, 200, 1, 8, "sigmoid", torch.float32), (64, 2060, 16, 1, 4, "softmax", torch.bfloat16)])
+def test_router(T, W, E, extra, groups, score, dtype):
+    """Token counts of steps (matrix cores) and of decode rows (a wave a row) against the plain fp32 router: widths that end
+    inside a wave's step, one that is no multiple of 8, rows past a tile or a round of waves."""
     from githubrepostorag_amd.ops.moe import moe_route
 
     g = torch.Generator().manual_seed(T + W)
@@ -49,9 +53,10 @@ def test_router_on_matrix_cores(T, W, E, extra, groups, score, dtype):
     wr = torch.randn(E + (extra == 1), W, generator=g) * 2 * W ** -0.5
     identity = extra if extra == 2 else 0
     kw = dict(score=score, identity=identity, corr=torch.randn(E, generator=g) * 0.01 if groups == 1 else None)
-    ids, wts, third = moe_route(h.cuda(), wr.cuda(), E, 4, groups, max(1, groups // 2), **{
+    top = min(E, 4)
+    ids, wts, third = moe_route(h.cuda(), wr.cuda(), E, top, groups, max(1, groups // 2), **{
         k: v.cuda() if torch.is_tensor(v) else v for k, v in kw.items()})
-    want_ids, want_wts, want_third = moe_route(h, wr, E, 4, groups, max(1, groups // 2), **kw)
+    want_ids, want_wts, want_third = moe_route(h, wr, E, top, groups, max(1, groups // 2), **kw)
     # logits differ by the order of W fp32 terms: sqrt(W) 2^-24 of their size 2, through a softmax of slope <= 1
     tol = 2e-6 + 2 * W ** 0.5 * 2 ** -24
     same = ids.cpu() == want_ids
