@@ -63,6 +63,7 @@ __global__ void __launch_bounds__(64 * NW, 4) sink_prefill_kernel(const SinkArgs
   const int head = kvh * R + (valid ? row - pq * R : 0), tok = q0 + pq;
   const int lim = valid ? min(kv_hi, pos0 + pq + 1) : 0, low = sp_first(p, pos0 + pq);
   const float sc = p.scale * (p.hscale ? p.hscale[head] : 1.f);
+  const bool pre = p.hscale || !(p.scale > 0.f);  // scores scaled before the mask and the maximum, else in the exponent's fma
   float m = p.sinks[head] * LOG2E, lsum = h4 == 0 ? 1.f : 0.f;  // the maximum starts at the sink, whose weight is 1 of the sum
   bf16x8_t qf[NC];
   const bf16* qp = p.q + ((size_t)tok * p.H + head) * D + 8 * h4;
@@ -116,7 +117,7 @@ __global__ void __launch_bounds__(64 * NW, 4) sink_prefill_kernel(const SinkArgs
       for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
         for (int r = 0; r < 4; ++r) s[tt][r] = c2 * tanhf(s[tt][r] * sc * ic);
-    } else if (p.hscale) {  // (a temperature may be of either sign: scaled before the maximum)
+    } else if (pre) {  // (a factor of 0 or less: it turns the order, and makes no 0 of a masked score)
       asm volatile("");
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) s[tt] *= sc * LOG2E;
@@ -132,7 +133,7 @@ __global__ void __launch_bounds__(64 * NW, 4) sink_prefill_kernel(const SinkArgs
           s[tt][r] = key < lim && (key >= low || key < p.keep) ? s[tt][r] : -INFINITY;
         }
     }
-    const float f = CAP || p.hscale ? 1.f : p.scale * LOG2E;
+    const float f = CAP || pre ? 1.f : p.scale * LOG2E;
     float tmax = -INFINITY;
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt)

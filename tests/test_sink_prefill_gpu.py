@@ -61,3 +61,25 @@ def test_sink_prefill(D, H, G, lens, past, form):
     # the result's own rounding to bf16 is 2^-9; the weights reach the sums with 16 bits
     err = (got - want).abs()
     assert (err <= 2 ** -8 * want.abs() + 2e-4).all(), err.max()
+
+
+@pytest.mark.parametrize("scale", [-0.11, 0.0])
+@pytest.mark.parametrize("form", ["causal", "window", "block_kept", "capped"])
+def test_scale_of_any_sign(form, scale):
+    """The scale is the caller's number: a negative one turns the order of the scores, with 0 every key weighs the same."""
+    g = torch.Generator().manual_seed(len(form))
+    D, H, G, n, past, BS = 64, 6, 2, 130, 70, 16
+    nb = -(-(n + past) // BS)
+    q = torch.randn(n, H, D, generator=g).bfloat16()
+    kc, vc = (torch.randn(nb, G, BS, D, generator=g).bfloat16() for _ in range(2))
+    sinks = torch.randn(H, generator=g)
+
+    def run(dev):
+        i32 = dict(dtype=torch.int32, device=dev)
+        m = AttnMetadata(q_start=torch.tensor([0, n], **i32), ctx_len=torch.tensor([n + past], **i32),
+                         block_tables=torch.arange(nb, **i32).view(1, nb), slot_mapping=None, max_q_len=n, num_seqs=1, num_tokens=n)
+        out = torch.empty(n, H * D, dtype=torch.bfloat16 if dev == "cuda" else torch.float32, device=dev)
+        return sink_attention(q.to(dev), kc.to(dev), vc.to(dev), m, scale, sinks.to(dev), out, **FORMS[form]).float().cpu()
+
+    got, want = run("cuda"), run("cpu")
+    assert ((got - want).abs() <= 2 ** -8 * want.abs() + 2e-4).all()  # (as above)
