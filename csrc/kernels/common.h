@@ -108,17 +108,17 @@ __device__ __forceinline__ float gelu_erf(float x) {
   return x * (x < 0.f ? q : 1.f - q);
 }
 
-// g sigmoid(alpha g) (u + shift) with g = min(g, limit), u = clamp(u, +-limit).  The exponential is the bare instruction, the
-// quotient a reciprocal with one correction step; where the exponential passes 2^126 the sigmoid is 0.
+// g sigmoid(alpha g) (u + shift) with g = min(g, limit), u = clamp(u, +-limit), for results that are rounded to bf16.  The
+// exponential is the bare instruction, the sigmoid a reciprocal with one correction step (of the reciprocal, not of the product
+// with g: an infinite g stays infinite); where the exponential passes 2^126 the sigmoid is 0.
 __device__ __forceinline__ float glu_f(float g, float u, float limit, float alpha, float shift) {
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
   const float e = -1.4426950408889634f * (alpha * g);
   const float d = 1.f + __builtin_amdgcn_exp2f(fminf(e, 126.f));
   const float rc = __builtin_amdgcn_rcpf(d);
-  float q = g * rc;
-  q = fmaf(fmaf(-d, q, g), rc, q);
-  return (e > 126.f ? g * 0.f : q) * (u + shift);
+  const float q = fmaf(fmaf(-d, rc, 1.f), rc, rc);
+  return g * (e > 126.f ? 0.f : q) * (u + shift);
 }
 
 // ---- wave / block reductions (wave64) ----

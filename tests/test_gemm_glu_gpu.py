@@ -68,3 +68,17 @@ def test_glu_linear_cpu():
 
     x, w = torch.randn(5, 32), torch.randn(24, 32)
     assert torch.equal(L.glu_linear(x, w, None, 1.0, 0.0), clamped_glu(L.linear(x, w), None, 1.0, 0.0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("alpha,shift", [(1.0, 0.0), (1.702, 1.0)])
+def test_gemm_glu_infinite(alpha, shift):
+    """A gate whose sum leaves fp32 upwards is infinite, as in the two launches; downwards there is no number (-inf * 0)."""
+    x = torch.zeros(3, 128, device="cuda", dtype=bf)
+    x[0, :2], x[1, :2], x[2, 0] = 1.0, -1.0, 0.5
+    w = torch.zeros(16, 128, device="cuda", dtype=bf)
+    w[:8, :2], w[8:, 2:] = 3e38, 1.0
+    x[:, 2] = 2.0
+    y = G.gemm_glu(x, w, None, alpha, shift).float().cpu()
+    assert (y[0] == float("inf")).all() and y[1].isnan().all() and (y[2] > 2.9e38).all()
+    assert (G.gemm_glu(x, w, 7.0, alpha, shift).float().cpu()[0] - 7.0 * (2.0 + shift)).abs().max() < 0.1

@@ -39,3 +39,16 @@ def test_moe_stream(counts, W, F, unit, limit):
     err = (got - want)[ok].abs().max() / want[ok].abs().max()
     assert err < 2 ** -7, err
     assert (got - want)[ok].norm() / want[ok].norm() < 5e-3
+
+
+@pytest.mark.parametrize("rows", [1, 20, 60, 300])  # the stream, its larger tile, the 128-row and the 256-row tiles
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_infinite_gate(rows, dtype):
+    """A gate whose sum leaves fp32 upwards gives an infinite unit."""
+    W = F = 128
+    h = torch.ones(rows, W, dtype=dtype, device="cuda")
+    wgu = torch.full((1, 2 * F, W), 2.0 ** -7, dtype=dtype, device="cuda")
+    wgu[0, 5] = 3e38
+    wd = torch.ones(1, W, F, dtype=dtype, device="cuda")
+    y = moe_experts(h, torch.zeros(rows, 1, dtype=torch.int32, device="cuda"), wgu, wd)
+    assert (y == float("inf")).all()
