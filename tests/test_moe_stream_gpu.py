@@ -52,3 +52,18 @@ def test_infinite_gate(rows, dtype):
     wd = torch.ones(1, W, F, dtype=dtype, device="cuda")
     y = moe_experts(h, torch.zeros(rows, 1, dtype=torch.int32, device="cuda"), wgu, wd)
     assert (y == float("inf")).all()
+
+
+def test_unit_in_fp32():
+    """fp32 experts: gates down to -80 (each a product of one term, and the second matrix the identity, so that only the unit
+    rounds: the exponential, sum, quotient and product by an ulp or half of 1.2e-7 each)."""
+    n = W = F = 256
+    g = torch.cat([torch.linspace(-80, -20, n // 2), torch.linspace(-20, 20, n // 2)])
+    h = torch.zeros(n, W)
+    h[:, 0], h[:, 1] = g, 1.0
+    wgu = torch.zeros(1, 2 * F, W)
+    wgu[0, :F, 0], wgu[0, F:, 1] = 1.0, torch.linspace(0.5, 3.0, F)
+    y = moe_experts(h.cuda(), torch.zeros(n, 1, dtype=torch.int32, device="cuda"), wgu.cuda(), torch.eye(F)[None].cuda())
+    want = (g.double() * torch.sigmoid(g.double()))[:, None] * wgu[0, F:, 1].double()
+    err = (y[:, 0].double().cpu() - want).abs() / want.abs()
+    assert err.max() < 5e-7, err.max()
