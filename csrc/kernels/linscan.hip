@@ -11,14 +11,17 @@
 // What bounds it: one thread per state column, three vector instructions per state element and token (the kernels of
 // seqmix.hip and ssm.hip, which still take decode rows and heads of more than 128 rows), waited on LDS broadcasts at 3 % of
 // the fp32 vector rate.  Here a chunk is bound by vector instructions (the splits, SiLU) and the latency of its dependent
-// steps.  Measured, old -> new: decay with SiLU, 28 heads of 128 x 128, 7 portions of 8192 tokens 2150 -> 690 us, 1 x 1187
-// 635 -> 128 us; without SiLU 2060 -> 249 and 602 -> 60; state space, 56 heads of 128 x 64, 3 x 1365 tokens 1450 -> 124 us.
+// steps.  Measured, old -> new: decay with SiLU, 28 heads of 128 x 128, 7 portions of 8192 tokens 2150 -> 677 us, 1 x 1187
+// 635 -> 130 us; without SiLU 2060 -> 214 and 602 -> 59; state space, 56 heads of 128 x 64, 3 x 1365 tokens 1450 -> 120 us.
 //
 // Precision: nothing is rounded to 16 bits that was not before.  An operand is the sum of bf16 parts of 8 bits of mantissa
 // each, and a product of operands is the matrix-core products of their parts (exact, fp32 sums).  What is fp32 (S, the
 // weighted triangle, the weighted v) has three parts; q, k and v have one (AP = 1) where they are bf16 numbers as they come,
 // and three (AP = 3) after SiLU or rotary, or where the activations are fp32.  Of three by three parts the three products
 // below 2^-24 of the result are left out: they lie under the rounding of an fp32 product.
+// An infinity has no such parts, and a product of matrices sums 0 times it into tokens that do not see it.  So a part is walked
+// token by token, with the recurrence as it stands above, from the first chunk on whose numbers are not all finite and small
+// (SCAN_BIG, SCAN_BIG_S: nothing in the products can overflow below them).
 //
 // A workgroup of 8 waves walks the chunks of one (sequence, head, 64 columns of v).  Wave w has 16 queries (block w % 4)
 // against 32 of the columns (half w / 4) for the outputs, and 16 columns (block w % 4) times half of the rows (w / 4) of S,
@@ -42,6 +45,9 @@ constexpr int LC = 64;     // tokens per chunk
 constexpr int LVT = 64;    // columns of v per workgroup
 constexpr int LTHREADS = 512;
 constexpr int LD_MAX = 128;  // rows of S at most
+// bounds of what the matrix products take: sums of squares of a thread's elements of q, k, v as they are stored (|x| < 2^20) and
+// of S (|S| < 2^60); |c_s| < 2^20 and a decay of at most 1.25 are asked too
+constexpr float SCAN_BIG = 0x1p40f, SCAN_BIG_S = 0x1p120f;
 
 struct ScanArgs {
   const void* x;  // q, k, v columns of rows of ld elements
@@ -118,9 +124,10 @@ __device__ __forceinline__ f32x4_t widen(f32x4_t v) { return v; }
 __device__ __forceinline__ float elt(const bf16* p) { return (float)*p; }
 __device__ __forceinline__ float elt(const float* p) { return *p; }
 __device__ __forceinline__ float softplus_x(float x) { return x > 20.f ? x : log1pf(expf(x)); }
+__device__ __forceinline__ float silu_acc(float x) { return x / (1.f + expf(-x)); }
 __device__ __forceinline__ float pow2(float x) { return __builtin_amdgcn_exp2f(x); }
 // x / (1 + e^-x) to the last bits: e^-x as 2^(hi + lo), with the part of -x log2 e that its fp32 product lost put back; the
-// reciprocal with one Newton step.  Below -87 the factor stays at e^-87 (times x: under 1e-36).
+// reciprocal with one Newton step.  Below -87 the factor stays at e^-87 (times |x| < 2^20: under 2e-32).
 __device__ __forceinline__ float silu_x(float x) {
   constexpr float L2E = 1.4426950408889634f, L2E_LO = 1.9259629911266175e-8f;
   const float m = fmaxf(x, -87.f), hi = -m * L2E, lo = fmaf(-m, L2E_LO, fmaf(-m, L2E, -hi));
@@ -143,6 +150,23 @@ __device__ __forceinline__ void wave_scan2(float& s, float& r) {
   scan_step<0x118, 0xf>(s, r);
   scan_step<0x142, 0xa>(s, r);
   scan_step<0x143, 0xc>(s, r);
+}
+
+// s + the squares of four stored elements
+__device__ __forceinline__ float squares(bf16x4_t v, float s) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  typedef short s2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int i = 0; i < 4; i += 2) {
+    const bf16x2_t p = __builtin_bit_cast(bf16x2_t, s2_t{v[i], v[i + 1]});
+    s = __builtin_amdgcn_fdot2_f32_bf16(p, p, s, false);
+  }
+  return s;
+}
+__device__ __forceinline__ float squares(f32x4_t v, float s) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s = fmaf(v[i], v[i], s);
+  return s;
 }
 
 template <typename T> struct V4;
@@ -224,7 +248,8 @@ linear_scan_kernel(const ScanArgs a) {
   __shared__ __attribute__((aligned(16))) bf16 Vs[AP * VN];                      // [part][16 tokens][32 columns]
   __shared__ __attribute__((aligned(16))) bf16 So[OUT ? 4 * ND * 3 * 512 : 8];  // [16 columns][32 dims][part]
   __shared__ __attribute__((aligned(16))) float sc[2][6][LC];  // L (two floats) | c_s | sign_t | 2^(L_t) | 2^(L_end - L_s) c_s
-  __shared__ float ends[2][2];                                 // 2^(L_end) | L_end
+  __shared__ float ends[2][3];                                 // 2^(L_end) | L_end | not 0: too large for the products
+  __shared__ __attribute__((aligned(16))) int odd[LTHREADS / 64];  // a wave's numbers are too large for the products
   const int ntile = (a.vd + LVT - 1) / LVT;
   int id = xcd_remap(blockIdx.x, gridDim.x);
   const int tile = id % ntile;
@@ -250,7 +275,7 @@ linear_scan_kernel(const ScanArgs a) {
   float* wsg = a.ws + ((size_t)seq * a.maxparts * a.H + h) * dv + col;  // part p's is p * H * dv further
   const size_t pstep = (size_t)a.H * dv;
   f32x4_t S[ND];
-  auto each = [&](auto&& f) {  // f(register block, element, row of S) of the rows that exist
+  auto each = [&](auto&& f) __attribute__((always_inline)) {  // f(register block, element, row of S) of the rows that exist
 #pragma unroll
     for (int b = 0; b < ND; ++b)
 #pragma unroll
@@ -299,13 +324,13 @@ linear_scan_kernel(const ScanArgs a) {
   const int vn = min(LVT, a.vd - tile * LVT);
   const int nch = (qlen + LC - 1) / LC;
 
-  // the chunk's rows, fetched while the chunk before is computed: per thread 8 dims of rows krow, krow + 512 / (4 ND), ... of k
+  // the chunk's rows, fetched while the chunk before is computed (q's behind its outputs): per thread 8 dims of rows krow, krow + 512 / (4 ND), ... of k
   // and 8 columns of a row of v; per wave its 16 rows of q as operands
   constexpr int KT = 4 * ND, KR = LTHREADS / KT, KL = LC / KR > 0 ? LC / KR : 1;  // threads a row, rows a pass, passes
   const int krow = tid / KT, kc = 8 * (tid % KT), vrow = tid >> 3, vc = 8 * (tid & 7);
   TI4 kr[KL][2], vr[2], qr[OUT ? ND : 1][2];
   float dtr = 0.f;
-  auto fetch = [&](int c) {
+  auto fetch = [&](int c) __attribute__((always_inline)) {
     const int end = min(qlen - c * LC, LC) - 1;
     const size_t t0 = (size_t)(qa + c * LC) * a.ld;
 #pragma unroll
@@ -314,6 +339,10 @@ linear_scan_kernel(const ScanArgs a) {
       for (int e = 0; e < 2; ++e) kr[x][e] = raw4<FULL>(xk + t0 + min(krow + x * KR, end) * a.ld, kc + 4 * e, a.d);
 #pragma unroll
     for (int e = 0; e < 2; ++e) vr[e] = raw4<FULL>(xv + t0 + min(vrow, end) * a.ld, vc + 4 * e, vn);
+  };
+  auto fetch_q = [&](int c) __attribute__((always_inline)) {
+    const int end = min(qlen - c * LC, LC) - 1;
+    const size_t t0 = (size_t)(qa + c * LC) * a.ld;
     if (OUT) {
 #pragma unroll
       for (int k = 0; k < ND; ++k)
@@ -322,11 +351,11 @@ linear_scan_kernel(const ScanArgs a) {
           qr[k][b] = raw4<FULL>(xq + t0 + min(16 * tb + ql, end) * a.ld, 32 * k + 16 * b + 4 * quad, a.d);
     }
   };
-  auto fetch_dt = [&](int c) {
+  auto fetch_dt = [&](int c) __attribute__((always_inline)) {
     if (SSM)
       dtr = c * LC + lane < qlen ? elt(reinterpret_cast<const TI*>(a.proj) + (size_t)(qa + c * LC + lane) * a.pld + a.dtoff + h) : 0.f;
   };
-  auto position = [&](int t) {
+  auto position = [&](int t) __attribute__((always_inline)) {
     if (AP == 1 || !a.rd) return 0;
     const int p = a.positions[t];
     return index_ok(p, a.tab_rows, ERR_ROPE_POS) ? p : 0;
@@ -336,7 +365,7 @@ linear_scan_kernel(const ScanArgs a) {
   const float lam = SSM ? 1.f : a.decay[h], bias = SSM ? a.dt_bias[h] : 0.f;
   const float rate = SSM ? -expf(a.a_log[h]) * 1.4426950408889634f : fmaxf(log2f(fabsf(lam)), -4000.f);  // (lam^n = 0 for 0)
   const bool neg = lam < 0.f;
-  auto scalars = [&](int c) {  // by one wave: lane = token of chunk c
+  auto scalars = [&](int c) __attribute__((always_inline)) {  // by one wave: lane = token of chunk c
     const int buf = c & 1, n = min(qlen - c * LC, LC);
     const float sign = neg && (lane & 1) ? -1.f : 1.f, esign = neg && (n & 1) ? -1.f : 1.f;  // of lam^lane, lam^n
     float cs = 0.f, hi, lo = 0.f, ehi, elo;
@@ -358,21 +387,38 @@ linear_scan_kernel(const ScanArgs a) {
     sc[buf][3][lane] = sign;
     sc[buf][4][lane] = pow2(hi) * (neg ? -sign : 1.f);
     sc[buf][5][lane] = pow2((ehi - hi) + (elo - lo)) * cs * (neg ? -sign * esign : 1.f);
+    const bool big = SSM ? __any(!(cs < 0x1p20f)) || !(rate > -0x1p60f) : !(fabsf(lam) <= 1.25f) || !(fabsf(a.kscale) < 0x1p20f);
     if (lane == 0) {
       ends[buf][0] = pow2(ehi) * esign;
       ends[buf][1] = ehi;
+      ends[buf][2] = big ? 1.f : 0.f;
     }
   };
+  const f32x4_t zero = f32x4_t{0.f, 0.f, 0.f, 0.f};
   if (w == 4) {
     fetch_dt(0);
     scalars(0);
     if (nch > 1) fetch_dt(1);
   }
   fetch(0);
-  const f32x4_t zero = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int c = 0; c < nch; ++c) {
+  fetch_q(0);
+  int c = 0;
+  for (; c < nch; ++c) {
     const int buf = c & 1, t0 = qa + c * LC, n = qlen - c * LC;
     // ---- k, v and S into LDS
+    float big = 0.f, big_s = 0.f;
+#pragma unroll
+    for (int b = 0; b < ND; ++b) big_s = squares(S[b], big_s);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+#pragma unroll
+      for (int x = 0; x < KL; ++x) big = squares(kr[x][e], big);
+      big = squares(vr[e], big);
+#pragma unroll
+      for (int k = 0; k < (OUT ? ND : 0); ++k) big = squares(qr[k][e], big);
+    }
+    const bool fits = __all(fmaf(big_s, SCAN_BIG / SCAN_BIG_S, big) < SCAN_BIG);  // (false for NaN)
+    if (lane == 0) odd[w] = !fits;
 #pragma unroll
     for (int x = 0; x < KL; ++x) {
       const int r = krow + x * KR;
@@ -422,6 +468,11 @@ linear_scan_kernel(const ScanArgs a) {
       }
     }
     __syncthreads();
+    typedef int i32x4_t __attribute__((ext_vector_type(4)));
+    const i32x4_t any = *reinterpret_cast<const i32x4_t*>(odd) | *reinterpret_cast<const i32x4_t*>(odd + 4);
+    const bool by_token = __builtin_amdgcn_readfirstlane(any[0] | any[1] | any[2] | any[3]) ||
+                          __builtin_amdgcn_readfirstlane(__float_as_int(ends[buf][2]));
+    if (by_token) break;
     if (c + 1 < nch) {
       fetch(c + 1);
       if (w == 4) {
@@ -495,6 +546,10 @@ linear_scan_kernel(const ScanArgs a) {
         }
       }
     }
+    // the next q not before the operands made of this one are done with: registers that spilled otherwise, and a spill's way back
+    // waits for the fetches before it (state space, 3 x 1365 tokens: 128 -> 117 us; 7 portions of 8192 without SiLU 281 -> 216)
+    __builtin_amdgcn_sched_barrier(0);
+    if (c + 1 < nch) fetch_q(c + 1);
     // ---- S at the chunk's end: 16 columns (block tb), rows of half vh
     const float end = ends[buf][0];
 #pragma unroll
@@ -525,6 +580,67 @@ linear_scan_kernel(const ScanArgs a) {
     }
     if (MODE == 1) lsum += ends[buf][1];
     if (c + 1 < nch) __syncthreads();
+  }
+  if (c < nch) {
+    // Token by token from chunk c on: q, k and v in LDS as they enter the recurrence, the sums of o over a wave's rows behind
+    // them.  (Empty asm around the thread's number and the arguments: what is made of them is not carried through the loop above.)
+    int me = threadIdx.x;
+    const ScanArgs* ap = (const ScanArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+v"(me), "+s"(ap));
+    const int mq = me & 15, mquad = (me & 63) >> 4, mcol = 16 * ((me >> 6) & 3) + mq;
+    float* qs = reinterpret_cast<float*>(Ks);
+    float *ks = qs + LD_MAX, *vs = ks + LD_MAX, *os = vs + LVT;
+    double l2 = 0.;
+    for (int t = qa + c * LC, stop = qa + qlen; t < stop; ++t) {
+      const TI* row = reinterpret_cast<const TI*>(ap->x) + (size_t)t * ap->ld;
+      float step = lam, cs = ap->kscale;
+      if (SSM) {
+        cs = softplus_x(elt(reinterpret_cast<const TI*>(ap->proj) + (size_t)t * ap->pld + ap->dtoff + h) + bias);
+        step = expf(-expf(ap->a_log[h]) * cs);
+      }
+      if (MODE == 1) l2 += SSM ? rate * cs : rate;
+      __syncthreads();
+      for (int i2 = me; i2 < 2 * ap->d + vn; i2 += LTHREADS) {
+        const bool isv = i2 >= 2 * ap->d, isk = !isv && i2 >= ap->d;
+        const int i = isv ? i2 - 2 * ap->d : isk ? i2 - ap->d : i2;
+        const TI* x = row + (isv ? ap->voff + h * ap->vd + tile * LVT : (isk ? ap->koff : ap->qoff) + (h / ap->R) * ap->d);
+        float val = elt(x + i);
+        if (ap->act) val = silu_acc(val);
+        if (!isv && i < ap->rd) {
+          const int half = ap->rd >> 1, fi = i < half ? i : i - half;
+          float other = elt(x + (i < half ? i + half : i - half));
+          if (ap->act) other = silu_acc(other);
+          const float* tab = ap->rope + (size_t)position(t) * ap->rd + fi;
+          val = i < half ? val * tab[0] - other * tab[half] : val * tab[0] + other * tab[half];
+        }
+        if (isk) val *= cs;
+        qs[isv ? 2 * LD_MAX + i : isk ? LD_MAX + i : i] = val;
+      }
+      __syncthreads();
+      const float v = vs[mcol];
+      float o = 0.f;
+#pragma unroll
+      for (int b = 0; b < ND; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = 16 * ((me >> 8) * ND + b) + 4 * mquad + i;
+          if (!FULL && !(mcol < vn && r < ap->d)) continue;
+          S[b][i] = fmaf(step, S[b][i], ks[r] * v);
+          o = fmaf(S[b][i], qs[r], o);
+        }
+      if (OUT) {
+        o += __shfl_xor(o, 16, 64);
+        o += __shfl_xor(o, 32, 64);
+        if (mquad == 0) os[(me >> 6) * 16 + mq] = o;
+        __syncthreads();
+        if (me < vn) {
+          float sum = os[me] + os[64 + me];
+          if (SSM) sum += ap->skip[h] * elt(row + ap->voff + h * ap->vd + tile * LVT + me);
+          ap->out[(size_t)t * ((size_t)ap->H * ap->vd) + h * ap->vd + tile * LVT + me] = sum;
+        }
+      }
+    }
+    lsum += (float)l2;
   }
   if (MODE == 1) {
     each([&](int b, int i, int r) { wsg[part * pstep + (size_t)r * a.vd] = S[b][i]; });

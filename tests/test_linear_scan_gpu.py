@@ -127,3 +127,88 @@ def test_state_space_scan(lens, past, H, G, N, P, dtype, part, monkeypatch):
         extra = skip.double()[:, None] * v[s:e]
         _check(got[s:e].view(-1, H, P), o + extra, bo + extra.abs(), "outputs")
         _check(st[slot], S, bS, "state")
+
+
+def _walk32(a, k, v, q, S):
+    """_walk in the kernels' own 32 bits."""
+    out = []
+    for t in range(q.shape[0]):
+        S = a[t][:, None, None] * S + k[t][:, :, None] * v[t][:, None, :]
+        out.append((S * q[t][:, :, None]).sum(1))
+    return torch.stack(out), S
+
+
+def _same(got, want, what):
+    """Infinite, no number and finite in the same places, and the finite numbers close to each other."""
+    assert torch.equal(got.isnan(), want.isnan()), f"{what}: NaN"
+    assert torch.equal(got.isinf(), want.isinf()) and torch.equal(got[got.isinf()], want[want.isinf()]), f"{what}: inf"
+    f = want.isfinite()
+    # (positive terms alone: no sum cancels, so TOL holds relative to the result, and the reference is a 32-bit one)
+    assert ((got[f] - want[f]).abs() <= 2 * TOL * want[f].abs() + 1e-30).all(), what
+
+
+@pytest.mark.parametrize("part", [64, 1 << 20])
+@pytest.mark.parametrize("d,vd,dtype,act", [(128, 64, torch.bfloat16, False), (128, 128, torch.bfloat16, True), (24, 40, torch.bfloat16, False),
+                                            (64, 64, torch.bfloat16, True), (20, 70, torch.float32, True)])
+def test_numbers_past_the_products(d, vd, dtype, act, part, monkeypatch):
+    """Infinities, NaN and numbers at the end of the range in v, k, q and the carried state: a token sees those of the tokens
+    before it and of itself, in their own columns, and no other."""
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(d + vd)
+    H, lens, past = 7, [200, 140], [0, 3]
+    m, qs = _meta(lens, past, dev)
+    T = qs[-1]
+    monkeypatch.setattr(recurrent, "_scan_part", lambda *a: part)
+    q, k, v = (torch.rand(T, H, n, generator=g) + 0.1 for n in (d, d, vd))
+    state = torch.rand(3, H, d, vd, generator=g)
+    inf = float("inf")
+    v[70, 0, 5] = inf
+    v[qs[1] + 10, 1, 3], v[qs[1] + 40, 1, 3], v[qs[1] + 90, 1, 2] = inf, -inf, float("nan")
+    k[130, 2, 7] = inf
+    q[100, 3, 2] = inf
+    state[0, 4, 2, 6], state[0, 4, 1, 1] = inf, 3.4e38  # (the second sequence's slot)
+    q[:, 4] *= 2.0 ** -9
+    v[150, 5, 0], q[:, 5] = 3.38e38, q[:, 5] * 2.0 ** -9
+    v[33, 6, 1], k[34, 6, 2] = (-inf, -3e38) if act else (inf, 1e30)
+    proj = torch.cat([t.reshape(T, -1) for t in (q, k, v)], 1).to(dtype)
+    decay = torch.tensor([0.996, 0.75, 0.5, 1.0, 0.9, 0.95, 0.8])
+    st = state.to(dev)
+    got = recurrent.decay_attention(proj.to(dev), 0, H * d, 2 * H * d, decay.to(dev), st, m, H, d, vd, act=act, k_scale=0.5)
+    got = got.float().cpu().view(T, H, vd)
+    x = proj.float()
+    f = (lambda t: t / (1 + torch.exp(-t))) if act else (lambda t: t)
+    q, k = (f(x[:, o:o + H * d]).view(T, H, d) for o in (0, H * d))
+    v = f(x[:, 2 * H * d:]).view(T, H, vd)
+    for i, (a, b) in enumerate(zip(qs, qs[1:])):
+        S0 = state[1 - i] if past[i] else torch.zeros(H, d, vd)
+        o, S = _walk32(decay.expand(b - a, H), k[a:b] * 0.5, v[a:b], q[a:b], S0)
+        for h in range(H):
+            _same(got[a:b, h], o[:, h], f"outputs of sequence {i}, head {h}")
+            _same(st[1 - i, h].cpu(), S[h], f"state of sequence {i}, head {h}")
+
+
+@pytest.mark.parametrize("part", [64, 1 << 20])
+@pytest.mark.parametrize("N,P,dtype", [(128, 64, torch.bfloat16), (32, 128, torch.bfloat16), (12, 8, torch.float32)])
+def test_state_space_past_the_products(N, P, dtype, part, monkeypatch):
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(N + P)
+    H, n = 4, 150
+    m, _ = _meta([n], [5], dev)
+    monkeypatch.setattr(recurrent, "_scan_part", lambda *a: part)
+    x, B, C = torch.rand(n, H, P, generator=g) + 0.1, torch.rand(n, N, generator=g) + 0.1, torch.rand(n, N, generator=g) + 0.1
+    dt = torch.rand(n, H, generator=g)
+    x[70, 0, 5], x[100, 1, 2], dt[80, 2] = float("inf"), float("nan"), float("inf")
+    xbc, proj = torch.cat([x.reshape(n, -1), B, C], 1).to(dtype), dt.to(dtype)
+    dtb, alog, skip = torch.zeros(H), torch.linspace(-2.0, 0.0, H), torch.rand(H, generator=g)
+    state = torch.rand(1, H, N, P, generator=g)
+    st = state.to(dev)
+    got = recurrent.ssm_scan(xbc.to(dev), proj.to(dev), 0, dtb.to(dev), alog.to(dev), skip.to(dev), st, m, H, 1, N, P)
+    got = got.float().cpu().view(n, H, P)
+    f = xbc.float()
+    v, B, C = f[:, :H * P].view(n, H, P), f[:, H * P:H * P + N], f[:, H * P + N:]
+    dt = torch.nn.functional.softplus(proj.float() + dtb)
+    o, S = _walk32(torch.exp(-torch.exp(alog) * dt), B[:, None] * dt[:, :, None], v, C[:, None].expand(n, H, N), state[0])
+    o = o + skip[:, None] * v
+    for h in range(H):
+        _same(got[:, h], o[:, h], f"outputs of head {h}")
+        _same(st[0, h].cpu(), S[h], f"state of head {h}")
