@@ -9,6 +9,8 @@ state after its last token there.  Tokens are consumed in order, so a prompt may
 """
 from __future__ import annotations
 
+import math
+
 import torch
 
 from ._lib import call, lib, ptr
@@ -28,33 +30,56 @@ LINEAR_SCAN_MIN = 8  # tokens of the longest portion from which the matrix-core 
 LINEAR_SCAN_CHUNK = 64
 
 
-def _scan_taken(m: AttnMetadata, d: int, tiles: int, split: bool) -> bool:
-    """Whether a step runs the matrix-core scan.  A workgroup's chunk costs the same for 1 or 64 tokens; the one-pass
-    kernels pay per token (4 sequences x 8 tokens x 28 heads: 16 us against 52; one of 64 tokens: 16 against 263).  Only
-    where many short portions fill the chip several times does the chunk cost more, and only with operands in three parts
-    (64 x 8 tokens x 28 heads: 190 us against 109; 64 x 16: 190 against 177; 20 x 30: 72 against 173)."""
-    if m.max_q_len < LINEAR_SCAN_MIN or d > lib().grag_linear_scan_max_dim():
-        return False
-    return not split or m.max_q_len >= 3 * LINEAR_SCAN_MIN or m.num_seqs * tiles <= 512
-
-
-def _scan_part(max_q: int, tokens: int, nseq: int, tiles: int, split: bool) -> int:
-    """Tokens per part of the matrix-core scan (csrc/kernels/linscan.hip) for a step of ``nseq`` portions with ``tokens``
-    tokens, the longest ``max_q``, and ``tiles`` (head, 64 columns) tiles a portion.  In walks of a 64-token chunk: whole
-    portions cost the longest walk, or the chip's share of all; cut into parts, every round of workgroups walks a part
-    twice (the first walk, for the state alone, is about half) and reads the states of the parts before it.  ``split``:
-    operands in three parts (one workgroup a CU, 12 us a chunk), else two workgroups a CU and 5 us."""
+def _scan_walks(max_q: int, tokens: int, nseq: int, tiles: float, split: bool) -> tuple[float, int]:
+    """(walks, chunks a part) of the matrix-core scan (csrc/kernels/linscan.hip) for a step of ``nseq`` portions with
+    ``tokens`` tokens, the longest ``max_q``, and ``tiles`` (head, 64 columns) tiles a portion: its length in walks of a
+    64-token chunk and the cut of a portion that makes it shortest.  Whole portions cost the longest walk, or the chip's
+    share of all; cut into parts, every round of workgroups walks a part twice (the first walk, for the state alone, is
+    about half) and reads the states of the parts before it.  ``split``: operands in three parts (one workgroup a CU,
+    12 us a chunk), else two workgroups a CU and 5 us."""
     slots, read = (256, 0.06) if split else (512, 0.28)
     chunks, total = -(-max_q // LINEAR_SCAN_CHUNK), tokens / LINEAR_SCAN_CHUNK
-    whole = max(chunks, total * tiles / slots)
-    best, part, s = 0.85 * whole, chunks, 1
+    best, part, s = 0.85 * max(chunks, total * tiles / slots), chunks, 1
     while s < chunks:
         rounds = -(-int((total / s + nseq / 2) * tiles) // slots)
         cost = max(1, rounds) * (1.5 * s + read * chunks / s) + 1
         if cost < best:
             best, part = cost, s
         s *= 2
-    return part * LINEAR_SCAN_CHUNK
+    return best, part
+
+
+def _scan_taken(m: AttnMetadata, tokens: int, H: int, d: int, vd: int, split: bool, exact: bool) -> bool:
+    """Whether a step runs the matrix-core scan: where its estimated time is below that of the one-pass kernels.  ``exact``: a
+    size that it is compiled for (_scan_exact); all others go as heads of 128 rows with a test per element, so small
+    or odd heads pay for rows that are not there once they fill the chip.
+
+    us, from 520 points of 26 sizes of d 8-128, vd 8-256, both types, 4-56 heads, 32-8192 tokens.  Scan: 9.5 + the walks
+    (of portions of a chunk: as many as their rounds) of 2.9 + 0.021 d where exact with one part an operand, 0.4 + 0.10 d
+    with three, 5.9 + 0.039 d and 14.6 + 0.084 d otherwise; a round of workgroups that share a CU costs 1.6 walks, of
+    those that do not 1.1.  One-pass kernels: 9.5 + a chain of 0.14 + 0.0345 d a token and 3.5e-7 a token and number of
+    the state, twice that where portions are cut at 64.  The choice is within 1 % of the faster side in the geometric
+    mean, also over 144 points of other sizes; a rule on the portions' length alone was 13 % off (scan against one pass: fp32, 28 heads of 16 x 16, 64 x 64
+    tokens 153 / 54; fp32 state space, 56 heads of 8 x 16, 7 portions of 8192 728 / 158)."""
+    if m.max_q_len < LINEAR_SCAN_MIN or d > lib().grag_linear_scan_max_dim():
+        return False
+    base, span = ((0.4, 0.10) if split else (2.9, 0.021)) if exact else ((14.6, 0.084) if split else (5.9, 0.039))
+    slots, crowd = (256, 1.1) if split else (512, 1.6)
+    load, cut = H * -(-vd // 64) * crowd, m.max_q_len > LINEAR_SCAN_CHUNK
+    walks = _scan_walks(m.max_q_len, tokens, m.num_seqs, load, split)[0] if cut else max(1.0, m.num_seqs * load / slots)
+    chain, work = min(m.max_q_len, 64) * (0.14 + 0.0345 * d), 3.5e-7 * tokens * H * d * vd
+    return (base + span * d) * walks < (2 if cut else 1) * math.hypot(chain, work)
+
+
+def _scan_exact(x: torch.Tensor, offs: tuple, d: int, vd: int, rd: int = 0) -> bool:
+    """Rows that the scan's kernels for 32, 64 and 128 state rows take as they are (grag_linear_scan_decay: full)."""
+    return (x.dtype == torch.bfloat16 and d in (32, 64, 128) and vd % 64 == 0 and rd % 8 == 0 and x.data_ptr() % 8 == 0
+            and x.stride(0) % 4 == 0 and all(o % 4 == 0 for o in offs))
+
+
+def _scan_part(max_q: int, tokens: int, nseq: int, tiles: int, split: bool) -> int:
+    """Tokens per part of the matrix-core scan."""
+    return _scan_walks(max_q, tokens, nseq, tiles, split)[1] * LINEAR_SCAN_CHUNK
 
 
 def _scan_ws(m: AttnMetadata, rows: int, H: int, d: int, vd: int, split: bool, device):
@@ -104,7 +129,7 @@ def decay_attention(proj: torch.Tensor, qoff: int, koff: int, voff: int, decay: 
         assert proj.stride(1) == 1 and state.dtype == torch.float32 and state.is_contiguous()
         x = proj[r0:r1]
         split = act or rd > 0 or _dt(proj) != 0
-        if _scan_taken(m, d, H * -(-vd // 64), split):
+        if _scan_taken(m, r1 - r0, H, d, vd, split, _scan_exact(x, (qoff, koff, voff), d, vd, rd)):
             part, ws, wa = _scan_ws(m, r1 - r0, H, d, vd, split, proj.device)
             call("grag_linear_scan_decay", ptr(x), proj.stride(0), qoff, koff, voff, ptr(decay), ptr(state),
                  ptr(m.state_slots), ptr(m.q_start), ptr(m.ctx_len), ptr(out[r0:r1]), m.num_seqs, H, d, vd,
@@ -277,7 +302,7 @@ def ssm_scan(xbc: torch.Tensor, proj: torch.Tensor, dtoff: int, dt_bias: torch.T
             continue
         assert xbc.is_contiguous() and proj.stride(1) == 1 and state.dtype == torch.float32 and state.is_contiguous()
         assert xbc.dtype == proj.dtype and state.shape[1:] == (H, N, P)
-        if _scan_taken(m, N, H * -(-P // 64), _dt(xbc) != 0):
+        if _scan_taken(m, r1 - r0, H, N, P, _dt(xbc) != 0, _scan_exact(xbc, (H * P, H * P + G * N), N, P)):
             part, ws, wa = _scan_ws(m, r1 - r0, H, N, P, _dt(xbc) != 0, xbc.device)
             call("grag_linear_scan_ssm", ptr(xbc[r0:r1]), C, H * P, H * P + G * N, ptr(proj[r0:r1]), proj.stride(0), dtoff,
                  ptr(dt_bias), ptr(a_log), ptr(skip), ptr(state), ptr(m.state_slots), ptr(m.q_start), ptr(m.ctx_len),
