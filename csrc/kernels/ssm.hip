@@ -56,7 +56,9 @@ template <> __device__ __forceinline__ void st4s<bf16>(bf16* p, f32x4_t v) {
 
 // ------------------------------------------------------------------------------------------------ causal convolution
 constexpr int CONV_MAX_TAPS = 16;
-constexpr int CONV_TT = 8;  // tokens per workgroup
+// tokens per workgroup: general form (every tile reads the taps - 1 inputs before it again: 3 x 1365 tokens x 3840 channels, 16
+// taps 148 us, in tiles of 8 224), and in groups of four channels
+constexpr int CONV_TT = 16, CONV_VTT = 8;
 
 // out [T][C] = SiLU(b[c] + sum_j w[c][j] in[t - (taps - 1) + j][c]), in = proj columns coff .. coff + C; inputs before
 // the portion come from cstate [slots][taps - 1][C] (oldest first), zeros for a sequence that starts at position 0.
@@ -119,7 +121,7 @@ causal_conv_kernel(const T* __restrict__ proj, int ld, int coff, int C, int taps
 // owns four channels of a token tile, all of whose inputs are in flight before the first sum.  The weights stand at the
 // end of MT places (zeros before them), so every register index is known when the kernel is compiled.  The pool's update is
 // the first tile's, without a second kernel (mode bit 2 means nothing here).
-// grid (ceil(C / 1024), ceil(max_q_len / CONV_TT), nseq); the mode bits as above.
+// grid (ceil(C / 1024), ceil(max_q_len / CONV_VTT), nseq); the mode bits as above.
 // Bound by its 4 bytes an element and, at few tokens, by a thread's first loads: sixteen 4-byte loads of weights 64 bytes apart
 // touched more lines than the tile's inputs.  us before and now, with 4 taps, bf16: 3 x 1365 tokens x 3840 channels 36 and 20,
 // x 12288 74 and 47; 1 x 8192 x 7168 81 and 54; 64 x 1 x 7168 7.6 and 4.2.  (Tokens a tile, with this form's weights: 16 29 /
@@ -130,20 +132,20 @@ causal_conv_vec_kernel(const T* __restrict__ proj, int ld, int coff, int C, int 
                        const float* __restrict__ b, T* __restrict__ cstate, const int* __restrict__ slots,
                        const int* __restrict__ q_start, const int* __restrict__ ctx_len, T* __restrict__ out, int nslots,
                        int mode) {
-  static_assert(MT - 1 < CONV_TT, "only the first tile reads the pool");
+  static_assert(MT - 1 < CONV_VTT, "only the first tile reads the pool");
   const int seq = blockIdx.z, c = (blockIdx.x * 256 + threadIdx.x) * 4;
   const int qa = q_start[seq], qlen = q_start[seq + 1] - qa;
-  const int t0 = blockIdx.y * CONV_TT;
+  const int t0 = blockIdx.y * CONV_VTT;
   if (t0 >= qlen || c >= C) return;
   const bool fresh = ctx_len[seq] - qlen == 0;
   const int slot = slots[seq];
   const bool slot_ok = fresh || index_ok(slot, nslots, ERR_SAMPLER_SLOT);
   const T* st = cstate + (size_t)(slot_ok && !fresh ? slot : 0) * (taps - 1) * C + c;
   const T* in = proj + (size_t)qa * ld + coff + c;
-  const int nt = min(CONV_TT, qlen - t0), lead = MT - taps;
-  f32x4_t cur[CONV_TT], win[MT - 1];  // the tile's inputs; the MT - 1 inputs before the one at hand, oldest first
+  const int nt = min(CONV_VTT, qlen - t0), lead = MT - taps;
+  f32x4_t cur[CONV_VTT], win[MT - 1];  // the tile's inputs; the MT - 1 inputs before the one at hand, oldest first
 #pragma unroll
-  for (int tt = 0; tt < CONV_TT; ++tt)
+  for (int tt = 0; tt < CONV_VTT; ++tt)
     cur[tt] = tt < nt ? ld4s(in + (size_t)(t0 + tt) * ld) : f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int j = 0; j < MT - 1; ++j) {
@@ -170,7 +172,7 @@ causal_conv_vec_kernel(const T* __restrict__ proj, int ld, int coff, int C, int 
   }
   const f32x4_t bias = b ? *reinterpret_cast<const f32x4_t*>(b + c) : f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int tt = 0; tt < CONV_TT; ++tt) {
+  for (int tt = 0; tt < CONV_VTT; ++tt) {
     if (tt < nt) {
       f32x4_t acc = bias;
 #pragma unroll
@@ -190,13 +192,13 @@ causal_conv_vec_kernel(const T* __restrict__ proj, int ld, int coff, int C, int 
       win[MT - 2] = cur[tt];
     }
   }
-  // the first tile's threads, the only ones that read the pool (taps - 1 < CONV_TT), leave the portion's last inputs there
+  // the first tile's threads, the only ones that read the pool (taps - 1 < CONV_VTT), leave the portion's last inputs there
   if (t0 == 0 && taps > 1 && index_ok(slot, nslots, ERR_SAMPLER_SLOT)) {
     T* dst = cstate + (size_t)slot * (taps - 1) * C + c;
 #pragma unroll
     for (int j = 0; j < MT - 1; ++j) {
       if (j < lead) continue;
-      const f32x4_t v = qlen <= CONV_TT ? win[j] : ld4s(in + (size_t)(qlen - (MT - 1) + j) * ld);
+      const f32x4_t v = qlen <= CONV_VTT ? win[j] : ld4s(in + (size_t)(qlen - (MT - 1) + j) * ld);
       st4s(dst + (size_t)(j - lead) * C, v);
     }
   }
@@ -804,16 +806,18 @@ GRAG_API hipError_t grag_causal_conv(const void* proj, int ld, int coff, int C, 
   if (nseq <= 0 || max_q_len <= 0) return hipSuccess;
   if (taps < 1 || taps > CONV_MAX_TAPS || C <= 0 || nseq > 65535) return hipErrorInvalidValue;
   const dim3 grid((C + 255) / 256, (max_q_len + CONV_TT - 1) / CONV_TT, nseq);
+  const int vtiles = (max_q_len + CONV_VTT - 1) / CONV_VTT;
   if (grid.y > 65535) return hipErrorInvalidValue;
   const bool one_tile = grid.y == 1;  // every portion in one token tile: the convolution's threads update the pool
   mode = (mode & 3) | (one_tile ? 4 : 0);
   const uintptr_t amask = dt == 0 ? 7 : 15;
-  const bool vec = C % 4 == 0 && ld % 4 == 0 && coff % 4 == 0 && taps <= 4 && (reinterpret_cast<uintptr_t>(b) & 15) == 0 &&
+  const bool vec = vtiles <= 65535 && C % 4 == 0 && ld % 4 == 0 && coff % 4 == 0 && taps <= 4 &&
+                   (reinterpret_cast<uintptr_t>(b) & 15) == 0 &&
                    ((reinterpret_cast<uintptr_t>(proj) | reinterpret_cast<uintptr_t>(cstate) |
                      reinterpret_cast<uintptr_t>(out)) & amask) == 0;
   DT_DISPATCH(dt, {
     if (vec)
-      hipLaunchKernelGGL((causal_conv_vec_kernel<T, 4>), dim3((C / 4 + 255) / 256, grid.y, nseq), dim3(256), 0, st,
+      hipLaunchKernelGGL((causal_conv_vec_kernel<T, 4>), dim3((C / 4 + 255) / 256, vtiles, nseq), dim3(256), 0, st,
                          (const T*)proj, ld, coff, C, taps, w, b, (T*)cstate, slots, q_start, ctx_len, (T*)out, nslots, mode);
     else
       hipLaunchKernelGGL(causal_conv_kernel<T>, grid, dim3(256), 0, st, (const T*)proj, ld, coff, C, taps, w, b,

@@ -37,3 +37,20 @@ def test_causal_conv(lens, past, C, taps, dtype, shift):
     assert torch.equal(s0, s1)
     # bf16: each rounds its result once (2^-8 of it); the sum of taps fp32 terms and the exponential
     assert ((o0 - o1).abs() <= o0.abs() * (2 ** -7 if dtype == torch.bfloat16 else 2e-6) + 4e-6).all()
+
+
+@pytest.mark.parametrize("n", [65535 * 8, 65535 * 8 + 1])
+def test_longest_portions(n):
+    """Portions up to and past the most token tiles of the four-channel form."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    C, taps = 8, 4
+    x = torch.randn(n, C, generator=g, device="cuda")
+    w = torch.randn(C, taps, generator=g, device="cuda")
+    pool = torch.randn(1, taps - 1, C, generator=g, device="cuda")
+    before = torch.cat([pool[0], x])
+    i32 = dict(dtype=torch.int32, device="cuda")
+    m = AttnMetadata(q_start=torch.tensor([0, n], **i32), ctx_len=torch.tensor([n + 9], **i32), block_tables=None, slot_mapping=None,
+                     max_q_len=n, num_seqs=1, num_tokens=n, state_slots=torch.zeros(1, **i32))
+    y = causal_conv(x, 0, w, None, pool, m)
+    want = torch.nn.functional.silu(sum(before[j:j + n] * w[:, j] for j in range(taps)))
+    assert ((y - want).abs() <= 2e-6 * want.abs() + 4e-6).all() and torch.equal(pool[0], x[-(taps - 1):])
