@@ -34,6 +34,7 @@ from pathlib import Path
 
 import torch
 from torch.autograd import forward_ad as fwAD
+from torch.overrides import has_torch_function
 
 from . import gemm as _tile
 from ._lib import call, lib, ptr
@@ -329,8 +330,10 @@ def _differentiated(*ts) -> bool:
 
 def _plain_product(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> bool:
     """Whether the owned kernel may stand in for the library's product of x [M, K] and w: it checks no operand against
-    another, and it knows no derivative, trace, dispatch mode or autocast.  What fails here goes to the library, which
-    handles or refuses it."""
+    another, and it knows no derivative, trace, dispatch or function mode, tensor subclass or autocast.  What fails here goes
+    to the library, which handles or refuses it."""
+    if has_torch_function((x, w, b)) or torch._C._len_torch_function_stack():
+        return False
     at = x.get_device()
     if w.dim() != 2 or w.size(1) != x.size(1) or w.get_device() != at or w.dtype != x.dtype or w.is_meta:
         return False

@@ -2,6 +2,7 @@
 that kernel against 64-bit products over the layouts it accepts there."""
 import pytest
 import torch
+from torch.overrides import TorchFunctionMode
 from torch.utils.flop_counter import FlopCounterMode
 
 from githubrepostorag_amd.ops import gemm as G
@@ -87,3 +88,44 @@ def test_linear_refuses_what_does_not_fit():
             L.linear(x, w)
         with pytest.raises(RuntimeError):
             L.glu_linear(x, w, 7.0)
+
+
+class Counted(torch.Tensor):
+    """A subclass that sees the functions called on it."""
+    seen: list = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.seen.append(func)
+        with torch._C.DisableTorchFunctionSubclass():
+            return func(*args, **(kwargs or {}))
+
+
+class Seen(TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen.append(func)
+        return func(*args, **(kwargs or {}))
+
+
+def test_what_overrides_functions_sees_the_product():
+    x, w = torch.randn(4, 128).to(bf), torch.randn(8, 128).to(bf)
+    assert L._plain_product(x, torch.nn.Parameter(w, requires_grad=False))
+    assert not L._plain_product(x.as_subclass(Counted), w) and not L._plain_product(x, w.as_subclass(Counted))
+    with Seen():
+        assert not L._plain_product(x, w)
+
+
+@pytest.mark.gpu
+def test_function_mode_sees_an_unmeasured_product():
+    x, w = torch.randn(7400, 768, device="cuda").to(bf), torch.randn(2304, 768, device="cuda").to(bf)
+    assert L.kernel_for(7400, 2304, 768) == "tile_prefill"
+    with Seen() as mode:
+        L.linear(x, w)
+    assert torch.nn.functional.linear in mode.seen
+    Counted.seen.clear()
+    L.linear(x.as_subclass(Counted), w)
+    assert torch.nn.functional.linear in Counted.seen
