@@ -218,7 +218,8 @@ def unmeasured_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
         return (1, 0) if tiles > ncu else None
     tail = tiles - ncu
     if K >= 2048 and 0 < tail <= ncu // 4 and M * N >= 0.9 * 65536 * tiles and sk_ok(M, N, K, 1, -4 * tail):
-        return 1, -4 * tail
+        sk = -4 * tail
+        return (1, sk) if WS.stream_ok(_ws_floats(M, N, 1, sk)) else None
     return None
 
 
@@ -250,6 +251,9 @@ def set_sched(sched: int) -> int:
 
 def _ws_floats(M: int, N: int, ksplit: int, sk: int) -> int:
     return ksplit * M * N if ksplit > 1 else (2 * abs(sk) * 65536 if sk else 0)
+
+
+TICKET_STREAMS = 32  # torch's streams of a device and priority
 
 
 class _Workspace:
@@ -331,6 +335,31 @@ class _Workspace:
         """The owner dict this thread's launches are routed to (None: thread-local scratch)."""
         return getattr(self._tls, "owner", None)
 
+    def stream_ok(self, floats: int) -> bool:
+        """Whether for_stream can serve a launch now: a graph keeps what it points at only where an owner does."""
+        if not (torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing()):
+            return True
+        dev = torch.device("cuda", torch.cuda.current_device())
+        return self.owner() is not None and self.ready(dev, floats) and self.has_counters(dev)
+
+    def for_stream(self, dev: torch.device, floats: int) -> tuple[torch.Tensor, torch.Tensor]:
+        """(slab, tickets) of a stream-K launch that callers without an owner make, on whatever streams they use: the slab is the
+        allocator's (ordered by the current stream), the tickets the current stream's own, of the TICKET_STREAMS used last by
+        this thread.  An owner runs on one stream at a time and has its own."""
+        if self.owner() is not None:
+            return self.get(dev, floats), self.counters(dev)
+        tab = getattr(self._tls, "tickets", None)
+        if tab is None:
+            tab = self._tls.tickets = {}
+        key = (dev.index, torch.cuda.current_stream(dev).cuda_stream)
+        c = tab.pop(key, None)
+        if c is None:
+            if len(tab) >= TICKET_STREAMS:
+                tab.pop(next(iter(tab)))
+            c = torch.zeros(1 << 14, dtype=torch.int32, device=dev)
+        tab[key] = c
+        return torch.empty(floats, dtype=torch.float32, device=dev), c
+
     def scratch(self, name: str, dev: torch.device, make):
         """A persistent per-owner scratch tensor (ticket arrays, small merge buffers) under ``name``: the
         owner's (an engine's, an embedder's) while one is set, else this thread's.  Every kernel that keeps
@@ -360,8 +389,11 @@ def _launch(x, w, b, out, epi, act, ksplit, sk):
     M, K = x.shape
     N = w.shape[0]
     fl = _ws_floats(M, N, ksplit, sk)
-    ws = WS.get(x.device, fl) if fl else None
-    cnt = WS.counters(x.device) if sk else None
+    if sk and epi == EPI_STORE and unmeasured_plan(M, N, K) == (ksplit, sk):  # (these callers may use several streams)
+        ws, cnt = WS.for_stream(x.device, fl)
+    else:
+        ws = WS.get(x.device, fl) if fl else None
+        cnt = WS.counters(x.device) if sk else None
     call("grag_gemm_tile", ptr(x), ptr(w), ptr(b), ptr(out), x.stride(0), w.stride(0), out.stride(0),
          M, N, K, epi, act, ksplit, sk, ptr(ws), ptr(cnt))
     return out

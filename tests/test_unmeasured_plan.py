@@ -129,3 +129,37 @@ def test_function_mode_sees_an_unmeasured_product():
     Counted.seen.clear()
     L.linear(x.as_subclass(Counted), w)
     assert torch.nn.functional.linear in Counted.seen
+
+
+def test_streams_of_one_thread_share_no_tickets(monkeypatch):
+    """A stream-K launch of an unmeasured shape from a thread without an owner (an encoder on several streams): each stream its own
+    tickets, each launch its own slab; an owner's launches keep the owner's; none in a capture that nothing owns."""
+    from types import SimpleNamespace
+
+    calls, at, capturing = [], [1], []
+    M, N, K = 24000, 768, 3072
+    x, w, out = (torch.empty(1, n, dtype=bf).expand(r, n) for r, n in ((M, K), (N, K), (M, N)))
+    monkeypatch.setattr(G, "call", lambda name, *a: calls.append(a[-2:]))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: SimpleNamespace(cuda_stream=at[0]))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: bool(capturing))
+    real, kept = torch.empty, []
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: kept.append(real(*a, **k)) or kept[-1])
+
+    def launch(stream):
+        at[0] = stream
+        G._launch(x, w, None, out, G.EPI_STORE, G.ACT_NONE, *G.unmeasured_plan(M, N, K))
+        return calls[-1]
+
+    (s1, t1), (s2, t2), (s3, t3) = launch(1), launch(2), launch(1)
+    assert t1 == t3 != t2 and len({s1, s2, s3}) == 3
+    for i in range(100):
+        launch(10 + i)
+    assert len(G.WS._tls.tickets) == G.TICKET_STREAMS
+    owner = {}
+    with G.WS.owned_by(owner):
+        assert launch(1) == launch(2) and calls[-1][1] == owner["cnts"][None].data_ptr()
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    capturing.append(1)
+    assert G.unmeasured_plan(M, N, K) is None and G.schedule(M, N, K) == (1, 0)
+    G.WS._tls.tickets.clear()
