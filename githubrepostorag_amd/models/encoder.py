@@ -16,7 +16,7 @@ the fp32 vector and the bf16 copy the index stores.
 """
 from __future__ import annotations
 
-import itertools
+from array import array
 
 import numpy as np
 import torch
@@ -124,12 +124,15 @@ class BertEncoder:
         lens = [max(1, min(len(x), cfg.max_position)) for x in batch]
         T, n = sum(lens), len(lens)
         parts = [(x if len(x) == k else x[:k]) if x else [0] for x, k in zip(batch, lens)]
-        # ids | positions | starts | lengths in one buffer and one copy to the device; the ids through one iterator (24000
-        # tokens in 128 parts: 1.9 -> 0.7 ms of a slow core, 0.35 ms of a batch of 6.6 with the GPU idle)
+        # ids | positions | starts | lengths in one buffer and one copy to the device (24000 tokens in 128 parts: 1.9 -> 0.5 ms of a
+        # slow core, 0.35 ms of a batch of 6.6 with the GPU idle); whole numbers only, as a string has no index
         host = np.empty(2 * T + 2 * n + 1, dtype=np.int32)
         try:
-            host[:T] = np.fromiter(itertools.chain.from_iterable(parts), dtype=np.int32, count=T)
-        except (TypeError, ValueError, OverflowError):  # what numpy does not read as whole numbers: torch decides
+            ids = array("i")
+            for x in parts:
+                ids.fromlist(x) if type(x) is list else ids.extend(x)
+            host[:T] = ids
+        except (TypeError, ValueError, OverflowError):  # what is no whole number of 32 bits: torch decides
             host[:T] = torch.tensor([t for x in parts for t in x], dtype=torch.int32).numpy()
         starts, length = host[2 * T: 2 * T + n + 1], host[2 * T + n + 1:]
         length[:] = lens

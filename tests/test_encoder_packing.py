@@ -1,4 +1,5 @@
 """BertEncoder.encode_ids packs ragged batches as the explicit tensors would: empty, over-long and tuple entries."""
+import numpy as np
 import pytest
 import torch
 
@@ -6,7 +7,7 @@ from githubrepostorag_amd.models.configs import EncoderConfig
 from githubrepostorag_amd.models.encoder import BertEncoder
 
 
-@pytest.mark.parametrize("batch", [[[3]], [[1, 2, 3], [], [7] * 40, (4, 5)], [[5, 6.0, True]]])
+@pytest.mark.parametrize("batch", [[[3]], [[1, 2, 3], [], [7] * 40, (4, 5)], [[5, 6.0, True]], [[np.int64(4), 2], (1, torch.tensor(8))]])
 def test_packing(batch):
     cfg = EncoderConfig("t", vocab_size=50, hidden_size=32, num_layers=1, num_heads=2, intermediate_size=64, max_position=16)
     enc = BertEncoder(cfg, device="cpu", dtype=torch.float32)
@@ -25,6 +26,6 @@ def test_packing(batch):
 def test_not_whole_numbers_refused():
     cfg = EncoderConfig("t", vocab_size=50, hidden_size=32, num_layers=1, num_heads=2, intermediate_size=64, max_position=16)
     enc = BertEncoder(cfg, device="cpu", dtype=torch.float32)
-    for bad in ([["a"]], [[None]], [[1 << 40]]):
+    for bad in ([["a"]], [[None]], [[1 << 40]], [["12"]], [["1", 2]], [("3", 4, 5)], [[b"12", 3]], [[np.float32(2.5)]]):
         with pytest.raises((TypeError, ValueError, RuntimeError, OverflowError)):
             enc.encode_ids(bad)
