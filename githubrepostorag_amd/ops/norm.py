@@ -164,8 +164,10 @@ def dyt_residual(resid: torch.Tensor, y: torch.Tensor | None = None, post=None, 
         return None if pre is None else dyt_ref(resid, *pre).to(out_dtype)
     out = torch.empty(T, H, dtype=out_dtype, device=resid.device) if pre is not None else None
     if isinstance(y, SplitKPartial):
-        if out_dtype == torch.bfloat16 and y.shape == resid.shape:
-            a2, w2, b2 = pre if pre is not None else (0.0, None, None)
+        a2, w2, b2 = pre if pre is not None else (0.0, None, None)
+        # (the kernel that sums planes has 16-byte accesses only)
+        wide = all(t is None or t.data_ptr() % 16 == 0 for t in (resid, post[1], post[2], add_rows, add_vec, w2, b2))
+        if out_dtype == torch.bfloat16 and y.shape == resid.shape and H % 4 == 0 and wide:
             call("grag_dyt_residual_splitk", ptr(y.planes), y.S, float(post[0]), ptr(post[1]), ptr(post[2]), ptr(resid),
                  ptr(add_rows), ptr(add_vec), float(a2), ptr(w2), ptr(b2), ptr(out), T, H)
             return out
