@@ -162,9 +162,11 @@ __global__ void __launch_bounds__(64 * NW, D == 64 ? 4 : 2) sink_decode_kernel(c
           pl[4 * tt + r] = f2bits(x - bits2f(b));
           lsum += x;
         }
-      // K and V of this tile have landed (loads do in issue order): behind them only the next tile's K is under way
+      // K and V of this tile have landed (loads do in issue order): behind them at least the 2 NC loads of the next tile's K are
+      // under way, which no load passes (the asm clobbers memory); more of them, a spill's say, would only wait for longer.  And
+      // the reads of the tile before have returned from the buffer that is filled now.
       if constexpr (decltype(more)::value) {
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NC) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * NC) : "memory");
         load_v(t + NW, std::integral_constant<int, 1 - S>{});
       } else {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

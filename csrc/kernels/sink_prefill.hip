@@ -182,9 +182,9 @@ __global__ void __launch_bounds__(64 * NW, 4) sink_prefill_kernel(const SinkArgs
   };
   issue(0, 0);
   for (int t = 0; t < ntiles; ++t) {
-    // the wave's own pieces of tile t landed; the barrier: everyone's, and everyone is done with tile t - 1, whose buffer the
-    // next issue fills
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // the wave's own pieces of tile t landed, its reads of tile t - 1 returned; the barrier: everyone's, and the buffer of tile
+    // t - 1 is free for the next issue
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (t + 1 < ntiles) issue(t + 1, (t + 1) & 1);
