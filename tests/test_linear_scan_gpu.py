@@ -53,6 +53,14 @@ CASES = [
     ([190, 64], [0, 1], 2, 100, 70, torch.float32, False, 0, 64),
     ([130], [0], 1, 17, 9, torch.float32, True, 6, 64),
     ([9], [2], 2, 5, 3, torch.bfloat16, False, 0, 64),
+    # the sizes of 32, 64 and 128 rows that are compiled for themselves
+    ([130, 64], [0, 5], 3, 32, 64, torch.bfloat16, False, 0, 64),
+    ([257, 33], [3, 0], 2, 32, 128, torch.bfloat16, True, 16, 128),
+    ([100, 129], [0, 7], 2, 64, 128, torch.bfloat16, False, 0, 1 << 20),
+    ([300], [9], 3, 64, 64, torch.bfloat16, True, 64, 64),
+    ([191, 20], [0, 30], 2, 64, 64, torch.bfloat16, True, 0, 1 << 20),
+    ([140, 65], [11, 0], 2, 128, 64, torch.bfloat16, True, 64, 64),
+    ([200], [0], 2, 128, 128, torch.bfloat16, False, 40, 128),
 ]
 
 
@@ -103,6 +111,9 @@ SSM = [
     ([300, 65, 8], [0, 0, 11], 6, 2, 128, 64, torch.bfloat16, 64),
     ([193], [5], 6, 2, 12, 8, torch.bfloat16, 128),
     ([129, 128], [0, 2], 3, 3, 50, 67, torch.float32, 64),
+    ([130, 64], [0, 4], 4, 2, 32, 64, torch.bfloat16, 64),
+    ([257], [3], 2, 1, 64, 64, torch.bfloat16, 128),
+    ([66, 190], [0, 1], 2, 1, 64, 128, torch.bfloat16, 1 << 20),
 ]
 
 
@@ -218,3 +229,28 @@ def test_state_space_past_the_products(N, P, dtype, part, monkeypatch):
     for h in range(H):
         _same(got[:, h], o[:, h], f"outputs of head {h}")
         _same(st[0, h].cpu(), S[h], f"state of head {h}")
+
+
+@pytest.mark.parametrize("d,vd,dtype", [(1, 70, torch.float32), (128, 64, torch.float32), (32, 64, torch.bfloat16), (128, 128, torch.bfloat16)])
+def test_all_parts_of_an_operand(d, vd, dtype):
+    """Outputs of one term each, so that nothing averages an operand's error away: k q v with a decay of 0, and S q of the carried
+    state alone.  fp32 operands, or SiLU of bf16.  Three roundings of 2^-24 and products left out below 2^-24 of each of the
+    two products; SiLU adds 2 ulp an operand.  An operand without its third part is off by 2^-17."""
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(d + vd)
+    n, H, act = 130, 2, dtype == torch.bfloat16
+    m, _ = _meta([n], [6], dev)
+    q, k, v = torch.zeros(n, H, d), torch.zeros(n, H, d), 1 + torch.rand(n, H, vd, generator=g)
+    q[..., 0], k[..., 0] = 1 + torch.rand(n, H, generator=g), 1 + torch.rand(n, H, generator=g)
+    k[:, 1] = 0
+    state = torch.zeros(1, H, d, vd)
+    state[:, 1, 0] = 1 + torch.rand(vd, generator=g)
+    proj = torch.cat([t.reshape(n, -1) for t in (q, k, v)], 1).to(dtype)
+    st = state.to(dev)
+    got = recurrent.decay_attention(proj.to(dev), 0, H * d, 2 * H * d, torch.tensor([0.0, 1.0], device=dev), st, m, H, d, vd, act=act)
+    got = got.double().cpu().view(n, H, vd)
+    x = proj.double()
+    x = torch.nn.functional.silu(x) if act else x
+    q, k, v = x[:, :H * d].view(n, H, d)[..., 0], x[:, H * d:2 * H * d].view(n, H, d)[..., 0], x[:, 2 * H * d:].view(n, H, vd)
+    want = torch.stack([(q * k)[:, 0, None] * v[:, 0], q[:, 1, None] * state[0, 1, 0].double()], 1)
+    assert ((got - want).abs() / want).max() < (9 + (6 if act else 0)) * 2.0 ** -24

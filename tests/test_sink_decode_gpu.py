@@ -39,16 +39,27 @@ def step(lens, H, G, D, nsplit, split_len, seed=0, BS=16):
 @pytest.mark.parametrize("opts", [{}, dict(window=100), dict(window=1500), dict(chunk=1100), dict(softcap=5.0),
                                   dict(window=40, softcap=3.0, scales=True), dict(scales=True, gate=True), dict(sinks=False)])
 def test_sink_decode(H, G, D, splits, opts):
-    q, kc, vc, m, g = step(LENS, H, G, D, *splits)
+    check(LENS, H, G, D, splits, opts)
+
+
+@pytest.mark.parametrize("H,G,D", [(28, 4, 128), (12, 4, 64)])
+@pytest.mark.parametrize("n,splits", [(64, (4, 512)), (129, (1, 0))])  # from 512 parts on: two waves, eight and more tiles each
+@pytest.mark.parametrize("opts", [{}, dict(window=700), dict(chunk=1100, softcap=5.0), dict(scales=True, gate=True)])
+def test_many_parts(H, G, D, n, splits, opts):
+    check([(i * 397 + 61) % 2048 + 1 for i in range(n)], H, G, D, splits, opts)
+
+
+def check(lens, H, G, D, splits, opts):
+    q, kc, vc, m, g = step(lens, H, G, D, *splits)
     opts = dict(opts)
     sinks = torch.randn(H, generator=g, device=dev) * 2 if opts.pop("sinks", True) else None
     if opts.pop("scales", False):
         opts["head_scale"] = torch.randn(H, generator=g, device=dev)
-    gate = torch.randn(len(LENS), H, generator=g, device=dev).bfloat16() if opts.pop("gate", False) else None
-    y = sink_attention(q, kc, vc, m, D ** -0.5, sinks, out_scale=1.5, head_gate=gate, **opts).float().view(len(LENS), H, D)
+    gate = torch.randn(len(lens), H, generator=g, device=dev).bfloat16() if opts.pop("gate", False) else None
+    y = sink_attention(q, kc, vc, m, D ** -0.5, sinks, out_scale=1.5, head_gate=gate, **opts).float().view(len(lens), H, D)
     kf, vf = kc.float().nan_to_num(0, 0, 0), vc.float().nan_to_num(0, 0, 0)
     s = sinks if sinks is not None else torch.full((H,), float("-inf"), device=dev)
-    r = sink_attention_ref(q.float(), kf, vf, m, D ** -0.5, s, **opts).float().view(len(LENS), H, D) * 1.5
+    r = sink_attention_ref(q.float(), kf, vf, m, D ** -0.5, s, **opts).float().view(len(lens), H, D) * 1.5
     if gate is not None:
         r = r * torch.sigmoid(gate.float())[:, :, None]
     # bf16 rounding of the result (2^-8 of it), and 16-bit weights of a sum that is at most the largest value

@@ -17,7 +17,8 @@ FORMS = {
 @pytest.mark.parametrize("form", sorted(FORMS))
 @pytest.mark.parametrize("D,H,G,lens,past", [
     (128, 28, 4, [37, 16, 300], [0, 61, 0]), (128, 4, 4, [257], [5]), (64, 12, 2, [129, 1, 64], [200, 0, 63]),
-    (64, 6, 1, [43], [400]), (128, 14, 2, [1], [0]), (64, 16, 8, [130] * 19 + [3], [0, 70] * 10)])  # the last: 128-row workgroups
+    (64, 6, 1, [43], [400]), (128, 14, 2, [1], [0]), (64, 16, 8, [130] * 19 + [3], [0, 70] * 10),
+    (128, 12, 4, [140] * 29 + [17], [0, 75, 3] * 10)])  # the last two: 128-row workgroups
 def test_sink_prefill(D, H, G, lens, past, form):
     g = torch.Generator().manual_seed(D + sum(lens) + len(form))
     BS = 16
