@@ -1500,6 +1500,9 @@ GRAG_API hipError_t grag_moe_gemm(const void* a, int lda, const void* w, const i
   // 63 / 74; 12 rows 251 / 241, 64 / 75; 24 rows 273 / 250, 70 / 79; 48 rows 341 / 262, 89 / 85.  Between them the tiles of
   // 16, 32 and 64 rows: the smallest that holds nearly every expert's rows (a second tile reads the weights again: 16 rows
   // an expert 312 us in tiles of 16, 257 of 32, 274 of 64; 28 rows 309 of 32, 300 of 64).
+  // The line of 384 tiles is a rough one: over 16 sizes of 128-512 tiles, 8-128 experts, 2-47 rows it takes the better side within
+  // 5 % but for 320-352 tiles of 32-47 rows (153 where 129 could be) and, of few K steps or one branch, 384-448 tiles of 12-26 (120 for
+  // 101, 82 for 69); neither side is anywhere behind the 32 x 64 tiles that took these row counts before (120, 111).
   const bool tiles128 = rows >= 48 * E || (rows >= 12 * E && (long)E * ((N + 127) / 128) >= 384);
   if (dt == 0 && gated != 2 && !tiles128 && K % 64 == 0 && lda % 8 == 0 && al16(a) && al16(w) && a_bytes < (1L << 31) &&
       w_bytes < (1L << 31)) {

@@ -554,7 +554,9 @@ GRAG_API int grag_splitk_add_rmsnorm(const void* ws, int S, void* residual, cons
   const size_t plane = (size_t)T * H;
   const float* wp = (const float*)ws;
   bf16* rp = (bf16*)residual;
-  // (1536 wide, 9 planes: 3.5 us in the general form, 3.9 here)
+  // The general form has a row of up to 2048 in flight as well, and past 8 planes (walked as 12 and 16) with fewer registers: us
+  // there / here at 512-2048 wide, 1-256 rows: 2-8 planes 2.4-5.1 / 1.9-5.0, 9-16 planes 2.6-7.4 / 2.9-7.7 (up to 16 rows of 16
+  // planes 4.6 / 3.7); wider it is never ahead (2304: 2 planes 3.1-3.8 / 2.2-2.8, 16 planes 8.7-13.2 / 3.7-8.2)
   if (T <= kWideRows && H <= 8192 && (H > 2048 || S <= 8)) {
     const int units = H / 4, V = units > 1024 ? 2 : 1, threads = ((units + V - 1) / V + 63) / 64 * 64;
     if (V == 1) splitk_rmsnorm_wide_kernel<1><<<T, threads, 0, stream>>>(wp, S, plane, rp, (const bf16*)w, (bf16*)out, H, eps);
