@@ -168,8 +168,11 @@ __global__ __launch_bounds__(64 * NW, D <= 64 && NW == 4 ? 4 : 1) void attn_fwd_
   // Neighbouring workgroups go to the eight XCDs in turn: of every eight sequences each XCD gets one, with all its row tiles,
   // which read the same K / V; which one turns with the head, so that long sequences meet every XCD (the sequences behind the
   // last eight stay dealt tile by tile).  128 sequences of 60-320 rows, 12 heads, D = 64 61 -> 56 us (65 without the turn),
-  // D = 32 43 -> 39; 64 of 500-512 129 -> 112, 113 -> 71.
-  const int grouped = gridDim.x / p.tiles_per_seq / 8 * 8 * p.tiles_per_seq, bj = blockIdx.x >> 3;
+  // D = 32 43 -> 39; 64 of 500-512 129 -> 112, 113 -> 71.  With fewer than eight kv heads the turn misses some XCDs, and a long
+  // sequence among short ones waits for those it meets: dealt by tiles then, unless sequences are short (4096 and 7 x 64 rows,
+  // 28 / 4 heads of 128 620 us so, 390 by tiles; 12 / 2 heads of 64 228 and 109; 8 x 1024 rows alike 193 and 200).
+  const bool turns = gridDim.y >= 8 || p.tiles_per_seq <= 8;
+  const int grouped = turns ? gridDim.x / p.tiles_per_seq / 8 * 8 * p.tiles_per_seq : 0, bj = blockIdx.x >> 3;
   const bool in_group = (int)blockIdx.x < grouped;
   const int seq = in_group ? bj / p.tiles_per_seq * 8 + ((blockIdx.x + blockIdx.y) & 7) : blockIdx.x / p.tiles_per_seq;
   const int tile = in_group ? bj % p.tiles_per_seq : blockIdx.x % p.tiles_per_seq;
