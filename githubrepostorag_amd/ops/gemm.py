@@ -198,35 +198,46 @@ OWN_SLACK = float(os.environ.get("GRAG_OWN_SLACK", "1.06"))  # beyond the 3-5 % 
 PREFILL_MIN_M = 257  # above one 256-row tile: the prefill regime (decode batches use plan())
 
 
-def unmeasured_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
-    """(ksplit, sk) of the owned kernel for a plain GEMM whose (N, K) the sweep's table does not have; None: the library.
-
-    Owned, whole tiles, where the contraction is short (K <= 1024) and the tiles are more than one round of the chip:
-    launches back to back over 8 shapes of N 384-3072, K 384-768 at 277-24000 rows, library / owned there is 1.19 in the
-    median of 13 points (0.90-1.48: 2304 x 768 at 7300 rows 64 -> 43 us, at 24000 106 -> 95, at 8192 38 -> 42); with fewer tiles the
-    library's smaller ones win (0.3-1.0).  No stream-K there: a part's slab out and in costs more than the K steps it
-    saves (3072 x 768 at 24000 rows: 149 us, whole tiles 124).
-
-    Deeper contractions are level in the median (0.94-1.05) and stay, but for one round and a thin rest of tiles at K >= 2048:
-    every tile of the rest cut into four equal K parts is a quarter of a round where others pay one -- 1.05 in the median
-    of 11 points (0.99-1.10; 768 x 3072 at 24000 rows 114 -> 105, 3584 x 7168 at 5000 223 -> 203), rows that pad a tenth of
-    the tiles or more left out (37888 x 3584 at 277 rows 0.87)."""
-    if (N, K, 0) in _prefill_table() or M < PREFILL_MIN_M or max(M, N) * K >= 1 << 30:
+def unmeasured_schedule(M: int, N: int, K: int) -> tuple[int, int] | None:
+    """(ksplit, sk) of the owned kernel for a prefill-sized GEMM whose (N, K) the sweep's table does not have, where it is not
+    plan()'s.  Short contractions of more than one round: whole tiles (a stream-K part's slab out and in costs more than
+    the K steps it saves: 3072 x 768 at 24000 rows 149 us, whole tiles 124).  Deep ones of one round and a thin rest: every tile
+    of the rest cut into four equal K parts is a quarter of a round where others pay one; not where rows pad a tenth of
+    the tiles or more (37888 x 3584 at 277 rows 0.87 of the library's rate)."""
+    if M < PREFILL_MIN_M or max(M, N) * K >= 1 << 30:
         return None
     tiles, ncu = -(-M // 256) * -(-N // 256), _num_cus()
+    if tiles <= ncu or K > 1024 and (K < 2048 or tiles > ncu + ncu // 4) or (N, K, 0) in _prefill_table():
+        return None
     if K <= 1024:
-        return (1, 0) if tiles > ncu else None
-    tail = tiles - ncu
-    if K >= 2048 and 0 < tail <= ncu // 4 and M * N >= 0.9 * 65536 * tiles and sk_ok(M, N, K, 1, -4 * tail):
-        sk = -4 * tail
-        return (1, sk) if WS.stream_ok(_ws_floats(M, N, 1, sk)) else None
+        return 1, 0
+    sk = -4 * (tiles - ncu)
+    if M * N >= 0.9 * 65536 * tiles and sk_ok(M, N, K, 1, sk) and WS.stream_ok(_ws_floats(M, N, 1, sk)):
+        return 1, sk
     return None
+
+
+def unmeasured_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
+    """unmeasured_schedule() where a plain product of that shape takes the owned kernel; None: the library.
+
+    Launches back to back, library / owned.  K <= 1024, 967 points of 12 widths 256-8192 at 3000-40000 rows: the library does
+    well at widths that are multiples of 512 (0.98 over K > 512, and at K = 128) and badly at others (384, 768, 1152, 2304:
+    1.17 over K > 512, 1.19 below); there too the owned tile wins on 256 <= K <= 512, unless its rounds are nearly full
+    (1.19; 0.99 from a fill of 0.92 on).  Of the 410 points taken 1.18 in the geometric mean, 38 more than 5 % behind (2304 x
+    768: 7300 rows 64 -> 43 us, 24000 106 -> 95).  K >= 2048, one round and a rest, 450 points: 1.12 for rests of up to a
+    sixth of a round at widths from 768 (31 of 264 more than 5 % behind), 0.99 for larger ones, 0.96 at widths below."""
+    if K <= 1024:
+        if N % 512 == 0 and (not 256 <= K <= 512 or M * N >= 0.92 * 65536 * -(-(-(-M // 256) * (N // 256)) // _num_cus()) * _num_cus()):
+            return None
+    elif K < 2048 or N < 768 or -(-M // 256) * -(-N // 256) > _num_cus() + _num_cus() // 6:
+        return None
+    return unmeasured_schedule(M, N, K)
 
 
 def schedule(M: int, N: int, K: int, silu: bool = False) -> tuple[int, int]:
     """(ksplit, sk) the owned kernel runs a shape with when the caller does not pin one."""
     if M >= PREFILL_MIN_M:
-        p = prefill_plan(M, N, K, silu) or (None if silu else unmeasured_plan(M, N, K))
+        p = prefill_plan(M, N, K, silu) or (None if silu else unmeasured_schedule(M, N, K))
         if p is not None:
             return p
     return plan(M, N, K)
@@ -389,7 +400,7 @@ def _launch(x, w, b, out, epi, act, ksplit, sk):
     M, K = x.shape
     N = w.shape[0]
     fl = _ws_floats(M, N, ksplit, sk)
-    if sk and epi == EPI_STORE and unmeasured_plan(M, N, K) == (ksplit, sk):  # (these callers may use several streams)
+    if sk and epi == EPI_STORE and unmeasured_schedule(M, N, K) == (ksplit, sk):  # (these callers may use several streams)
         ws, cnt = WS.for_stream(x.device, fl)
     else:
         ws = WS.get(x.device, fl) if fl else None

@@ -390,11 +390,10 @@ def glu_linear(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: flo
     384 / 255; 8960 x 1536 8192 457 / 360, 1187 79 / 70; 1.03-1.5 above the line (median 1.19), 0.47-1.3 below it (a
     last round that is nearly empty, rows that are mostly padding, or few tiles).  Error against 64 bits 0.59 of the two
     launches', which round gate and up to bf16 between them."""
-    if (x.is_cuda and x.dim() == 2 and x.shape[0] >= _tile.PREFILL_MIN_M and w.shape[0] % 16 == 0 and _tile.supported(x, w)
-            and _plain_product(x, w)):
+    if x.is_cuda and x.dim() == 2 and x.shape[0] >= _tile.PREFILL_MIN_M and w.shape[0] % 16 == 0:
         M, N = x.shape[0], w.shape[0]
         tiles, ncu = -(-M // 256) * -(-N // 256), _tile._num_cus()
-        if M * N >= GLU_FILL * 65536 * ncu * -(-tiles // ncu):
+        if M * N >= GLU_FILL * 65536 * ncu * -(-tiles // ncu) and _tile.supported(x, w) and _plain_product(x, w):
             return _tile.gemm_glu(x, w, limit, alpha, shift)
     return clamped_glu(linear(x, w), limit, alpha, shift)
 

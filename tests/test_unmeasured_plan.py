@@ -163,3 +163,15 @@ def test_streams_of_one_thread_share_no_tickets(monkeypatch):
     capturing.append(1)
     assert G.unmeasured_plan(M, N, K) is None and G.schedule(M, N, K) == (1, 0)
     G.WS._tls.tickets.clear()
+
+
+# rows, width, depth, us of the library and of the owned kernel
+MEASURED = [(8192, 8192, 768, 90, 103), (16500, 4096, 768, 102, 115), (33000, 8192, 128, 165, 220), (24000, 768, 768, 55, 45),
+            (33000, 768, 1024, 74, 56), (24000, 2304, 768, 109, 94), (16500, 8192, 384, 187, 142), (5000, 4096, 512, 47, 36),
+            (8192, 8192, 256, 57, 63), (5000, 4096, 2048, 76, 100), (5000, 4096, 3072, 102, 123), (24000, 768, 3072, 118, 109),
+            (33000, 1000, 640, 113, 81), (8192, 2304, 4096, 139, 132)]
+
+
+@pytest.mark.parametrize("M,N,K,lib,own", MEASURED)
+def test_rule_takes_the_faster_side(M, N, K, lib, own):
+    assert (G.unmeasured_plan(M, N, K) is not None) == (own < lib)
