@@ -358,16 +358,15 @@ moe_route_mfma_kernel(const T* __restrict__ h, int ld, const float* __restrict__
 
 // A few tokens (decode rows): one workgroup per token, one wave per logit row (rows w, w + 16, ...), the lanes split the
 // row's columns (8 consecutive ones per lane and step when `vec`) and the sum is a wave reduction.  Bound by round trips to
-// memory: the loads of UN steps (2048 columns) are all issued before their first product.  us with four waves that waited
-// for each step and now, 64 tokens: 17 rows of 3584 12.0 and 9.5, behind an expert layer whose weights push the rows out of
+// memory: the loads of UN steps of 512 columns (4, or 1 where that is the width) are all issued before their first product.  us
+// with four waves that waited for each step and now, 64 tokens: 201 rows of 512 27 and at most 14 (30 with UN = 4), 17 rows of 3584 12.0 and 9.5, behind an expert layer whose weights push the rows out of
 // the caches 24 and 13; 65 rows 30.0 and 21.4; 17 of 1536 9.2 and 8.0 (with UN = 8 9.5); 8 of 8192 10.5 and 8.8.
-template <typename T>
+template <typename T, int UN>
 __global__ void __launch_bounds__(1024)
 moe_route_rows_kernel(const T* __restrict__ h, int ld, const float* __restrict__ wr, int W, int E, int R, int top,
                       int ngroups, int keep, int* __restrict__ ids, float* __restrict__ wts,
                       float* __restrict__ sgate, int vec, RouteExtra rx) {
   __shared__ float z[RT_MAXR + 1];
-  constexpr int UN = 4;  // steps whose loads are under way together
   const int t = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const T* hr = h + (size_t)t * ld;
   for (int r = wid; r < R; r += 16) {
@@ -1423,8 +1422,15 @@ GRAG_API hipError_t grag_moe_route(const void* h, int ld, const float* wr, int W
     return hipGetLastError();
   }
   if (T_ <= 128) {  // decode rows, short portions
-    DT_DISPATCH(dt, hipLaunchKernelGGL(moe_route_rows_kernel<T>, dim3(T_), dim3(1024), 0, st, (const T*)h, ld, wr, W, E, R,
-                                       top, ngroups, keep, ids, wts, sgate, vec, rx);)
+#define ROUTE_ROWS(UN)                                                                                                      \
+  DT_DISPATCH(dt, hipLaunchKernelGGL((moe_route_rows_kernel<T, UN>), dim3(T_), dim3(1024), 0, st, (const T*)h, ld, wr, W, E, R, \
+                                     top, ngroups, keep, ids, wts, sgate, vec, rx);)
+    if (W <= 512) {
+      ROUTE_ROWS(1)
+    } else {
+      ROUTE_ROWS(4)
+    }
+#undef ROUTE_ROWS
     return hipGetLastError();
   }
   DT_DISPATCH(dt, {
