@@ -705,17 +705,28 @@ moe_gemm_stream_kernel(const bf16* __restrict__ a, int lda, const bf16* __restri
   constexpr int TM = 16 * MT, COLS = GATED == 1 ? 32 : 64, D = 2;
   __shared__ f32x4_t part[4][4 * MT][64];
   __shared__ int rows[TM];
-  int e = 0, tile = blockIdx.y, r0 = -1, rend = 0;
-  for (; e < E; ++e) {
-    const int b = offs[e], n = offs[e + 1] - b, nt = (n + TM - 1) / TM;
-    if (tile < nt) {
-      r0 = b + tile * TM;
-      rend = b + n;
+  // the expert of the row tile: 64 of them at a time, one a lane (a walk over 128 experts, each behind its load, was 20 us)
+  int e = -1, r0 = 0, rend = 0;
+  for (int e0 = 0, tile = blockIdx.y; e0 < E; e0 += 64) {
+    const int at = min(e0 + (int)(threadIdx.x & 63), E - 1);
+    const int b = offs[at], n = e0 + (int)(threadIdx.x & 63) < E ? offs[at + 1] - b : 0, nt = (n + TM - 1) / TM;
+    int upto = nt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(upto, d, 64);
+      if ((int)(threadIdx.x & 63) >= d) upto += v;
+    }
+    const unsigned long long behind = __ballot(upto > tile);
+    if (behind) {
+      const int l = __builtin_ctzll(behind);
+      e = e0 + l;
+      r0 = __builtin_amdgcn_readlane(b, l) + (tile - __builtin_amdgcn_readlane(upto - nt, l)) * TM;
+      rend = __builtin_amdgcn_readlane(b + n, l);
       break;
     }
-    tile -= nt;
+    tile -= __builtin_amdgcn_readlane(upto, 63);
   }
-  if (r0 < 0) return;
+  if (e < 0) return;
   const int n0 = blockIdx.x * COLS;
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ql = lane & 15, quad = lane >> 4;

@@ -67,3 +67,17 @@ def test_unit_in_fp32():
     want = (g.double() * torch.sigmoid(g.double()))[:, None] * wgu[0, F:, 1].double()
     err = (y[:, 0].double().cpu() - want).abs() / want.abs()
     assert err.max() < 5e-7, err.max()
+
+
+@pytest.mark.parametrize("E", [63, 64, 65, 130])
+def test_many_experts(E):
+    """Row tiles of experts past the first 64, and of the last."""
+    g = torch.Generator().manual_seed(E)
+    W, F, T = 64, 64, 40
+    ids = torch.randint(0, E, (T, 2), generator=g, dtype=torch.int32)
+    ids[:20, 0] = E - 1
+    h = torch.randn(T, W, generator=g).bfloat16()
+    wgu, wd = ((torch.randn(E, n, 64, generator=g) / 8).bfloat16() for n in (2 * F, W))
+    got = moe_experts(h.cuda(), ids.cuda(), wgu.cuda(), wd.cuda()).float().cpu()
+    want = moe_experts(h, ids, wgu, wd).float()
+    assert (got - want).abs().max() / want.abs().max() < 2 ** -7 and (got - want).norm() / want.norm() < 5e-3  # (as above)
