@@ -1499,9 +1499,13 @@ GRAG_API hipError_t grag_moe_gemm(const void* a, int lda, const void* w, const i
   // K in whole steps, and operands within 32-bit byte offsets (a gathered has at most rows / top rows, every row of h one pair)
   const long a_rows = moe_gathers(gated) ? (rows + top - 1) / top : rows;
   const long a_bytes = a_rows * lda * 2, w_bytes = (long)(gated == 1 ? 2 * N : N) * K * 2;
-  if (dt == 0 && gated != 2 && K % 64 == 0 && K >= 128 && lda % 8 == 0 && al16(a) && al16(w) && rows >= MOE_TILE_MIN * E &&
-      E <= RT_MAXR && a_bytes < (1L << 31) && w_bytes < (1L << 31)) {
-    const long blocks = ((long)rows / 256 + E) * ((N + (gated == 1 ? 127 : 255)) / (gated == 1 ? 128 : 256));
+  const int tcols = (N + (gated == 1 ? 127 : 255)) / (gated == 1 ? 128 : 256);
+  // (one branch, up to 64 tiles: the 128 x 128 tiles are four times as many workgroups, 60 tiles 66 us where these take 77, 24 24 / 25;
+  // from 96 on 52 / 42; with gate and up a tile has 128 columns, and 16 tiles take 19 for 21)
+  const bool many = gated == 1 || (long)((rows / E + 255) / 256) * E * tcols > 64;
+  if (dt == 0 && gated != 2 && many && K % 64 == 0 && K >= 128 && lda % 8 == 0 && al16(a) && al16(w) &&
+      rows >= MOE_TILE_MIN * E && E <= RT_MAXR && a_bytes < (1L << 31) && w_bytes < (1L << 31)) {
+    const long blocks = ((long)rows / 256 + E) * tcols;
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
 #define MOE_TILE(G)                                                                                                       \
   hipLaunchKernelGGL(moe_gemm_tile_kernel<G>, dim3((unsigned)blocks), dim3(kTileThreads), 0, st, (const bf16*)a, lda,     \
