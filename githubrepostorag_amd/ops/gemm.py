@@ -226,6 +226,8 @@ def unmeasured_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
     (1.19; 0.99 from a fill of 0.92 on).  Of the 410 points taken 1.18 in the geometric mean, 38 more than 5 % behind (2304 x
     768: 7300 rows 64 -> 43 us, 24000 106 -> 95).  K >= 2048, one round and a rest, 450 points: 1.12 for rests of up to a
     sixth of a round at widths from 768 (31 of 264 more than 5 % behind), 0.99 for larger ones, 0.96 at widths below."""
+    if (M + 255 >> 8) * (N + 255 >> 8) <= _num_cus():
+        return None
     if K <= 1024:
         if N % 512 == 0 and (not 256 <= K <= 512 or M * N >= 0.92 * 65536 * -(-(-(-M // 256) * (N // 256)) // _num_cus()) * _num_cus()):
             return None
