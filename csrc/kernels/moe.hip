@@ -477,14 +477,15 @@ __device__ __forceinline__ float glu_unit(float g, float u, const MoeEpi& ep) {
   return glu_f(g, u, ep.limit, ep.alpha, ep.shift);
 }
 // The same where the result may stay fp32: the exponent's rounding is put back and the quotient is IEEE's.  Largest error of the
-// value for gates of -80 to 20: glu_f 3.5e-6, with expf 2.7e-6, here 2.0e-7.
+// value for gates of -80 to 20: glu_f 3.5e-6, with expf 2.7e-6, here 2.0e-7.  Where the exponential is infinite the unit is 0.
 __device__ __forceinline__ float glu_unit_full(float g, float u, const MoeEpi& ep) {
   constexpr float L2E = 1.4426950408889634f, L2E_LO = 1.9259629911266175e-8f;  // log2 e in two parts
   g = fminf(g, ep.limit);
   u = fminf(fmaxf(u, -ep.limit), ep.limit);
   const float z = -ep.alpha * g, hi = z * L2E, lo = fmaf(z, L2E_LO, fmaf(z, L2E, -hi));
   const float t = __builtin_amdgcn_exp2f(hi);
-  return g / (1.f + fmaf(t, fabsf(hi) < 127.f ? 0.6931471805599453f * lo : 0.f, t)) * (u + ep.shift);
+  const float e = fabsf(hi) < 127.f ? fmaf(t, 0.6931471805599453f * lo, t) : t;  // (past that range t is 0 or infinite: as it is)
+  return g / (1.f + e) * (u + ep.shift);
 }
 __device__ __forceinline__ float relu2_unit(float v) {
   v = fmaxf(v, 0.f);

@@ -1,6 +1,8 @@
 """The experts' grouped GEMM at decode's row counts (csrc/kernels/moe.hip moe_gemm_stream_kernel, and the 128-row tiles that
 take over where the experts fill the chip) against a plain fp32 product per pair: row counts around the tiles of 16, 32 and 64
 rows, none among them, contractions shorter than the waves' blocks, columns past the last whole tile."""
+import math
+
 import pytest
 import torch
 
@@ -67,6 +69,20 @@ def test_unit_in_fp32():
     want = (g.double() * torch.sigmoid(g.double()))[:, None] * wgu[0, F:, 1].double()
     err = (y[:, 0].double().cpu() - want).abs() / want.abs()
     assert err.max() < 5e-7, err.max()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_unit_of_large_negative_gates(dtype):
+    """Where e^-g leaves fp32 (g < -88.7) the unit is 0, as the quotient by infinity is; just above, a number below 1e-35."""
+    g = torch.tensor([-86.0, -88.0, -88.5, -89.0, -90.0, -100.0, -128.0, -1e4, -1e30, 1.0])
+    n, W, F = len(g), 128, 128
+    h = torch.zeros(n, W, dtype=dtype)
+    h[:, 0], h[:, 1] = g, 1.0
+    wgu = torch.zeros(1, 2 * F, W, dtype=dtype)
+    wgu[0, :F, 0], wgu[0, F:, 1] = 1.0, 2.0
+    y = moe_experts(h.cuda(), torch.zeros(n, 1, dtype=torch.int32, device="cuda"), wgu.cuda(), torch.eye(F, dtype=dtype)[None].cuda())
+    y = y[:, :F].float().cpu()
+    assert (y[:-1].abs() < 1e-35).all() and ((y[-1] - 2 / (1 + math.exp(-1))).abs() < 2 ** -7).all()
 
 
 @pytest.mark.parametrize("E", [63, 64, 65, 130])
