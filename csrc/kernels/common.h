@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #define GRAG_API extern "C" __attribute__((visibility("default")))
 
 typedef short bf16x8_t __attribute__((ext_vector_type(8)));
@@ -23,6 +25,16 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16;
 
 namespace grag {
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): register arrays that its number indexes stay in registers,
+// also in loops that the unroller would give up on (they would lie in scratch memory)
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<N, I + 1>(static_cast<F&&>(f));
+  }
+}
 
 __device__ __forceinline__ float bf2f(bf16 v) { return (float)v; }
 __device__ __forceinline__ bf16 f2bf(float v) { return (bf16)v; }

@@ -38,7 +38,6 @@
 //     SiLU(gate)*up for the gate/up weight stored interleaved in 32-row blocks
 //     (ops/gemm.py interleave_gate_up): a wave's two n-tiles are then the 16
 //     gate rows and the 16 matching up rows, so the product forms in registers.
-#include <type_traits>
 
 #include "common.h"
 
@@ -51,15 +50,6 @@ namespace {
 
 enum { EPI_STORE = 0, EPI_SILU = 1, EPI_PARTIAL = 2 };
 
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): a compile-time loop (register arrays
-// indexed by its constant stay in registers)
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<N, I + 1>(static_cast<F&&>(f));
-  }
-}
 enum { ACT_NONE = 0, ACT_GELU = 1, ACT_GELU_TANH = 3 };
 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.f + __expf(-x)); }

@@ -681,14 +681,6 @@ moe_gemm_mfma_kernel(const bf16* __restrict__ a, int lda, const bf16* __restrict
   }
 }
 
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<N, I + 1>(static_cast<F&&>(f));
-  }
-}
-
 // Few rows an expert (bf16, K a multiple of 64): the weights' bytes are the work, so they go from memory straight to the
 // registers as operands of v_mfma_f32_16x16x32_bf16, without LDS or a barrier on their way.  A workgroup takes 64 rows of an
 // expert's matrix (32 of the gate and the 32 of the up half that belong to them) against a tile of 16 MT sorted rows; its four

@@ -1,4 +1,4 @@
-// The 256 x 256 bf16 tile product that the dense and the grouped GEMM share (gemm_tile.hip, moe_tile.hip): 8 waves (512
+// The 256 x 256 bf16 tile product that the dense and the grouped GEMM share (gemm_tile.hip, moe.hip): 8 waves (512
 // threads) as 2 (rows) x 4 (columns), K steps of 64, 16x16x32 matrix-core products, two LDS buffers refilled by LDS-DMA.
 // Wave (wr, wc) owns rows [128 wr, +128) x columns [64 wc, +64) as 2 x 2 quadrants of 64 x 32.  A buffer holds 4 slots of 16 KB
 // (A q0, A q1, B q0, B q1), each the 128 rows (both wave rows / all 4 wave columns) that one quadrant needs; rows are 128

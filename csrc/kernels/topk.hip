@@ -31,7 +31,6 @@
 //   work : blockIdx.x = work item {row range, NQT*16 query ids} (IVF probes:
 //          rows of one inverted list scanned for the queries that probe it)
 #include <algorithm>
-#include <type_traits>
 
 #include "common.h"
 
@@ -67,16 +66,6 @@ struct TopkParams {
   float* out_s;
   int64_t* out_i;
 };
-
-// f(0) ... f(N - 1) with compile-time numbers: the lists are register arrays, and a loop that the unroller gives up on (their
-// networks are long) would index them in scratch memory
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<N, I + 1>(static_cast<F&&>(f));
-  }
-}
 
 template <int K>
 __device__ __forceinline__ void list_insert(float (&v)[K], uint32_t (&id)[K], float x, uint32_t xi) {
