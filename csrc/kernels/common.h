@@ -120,14 +120,19 @@ __device__ __forceinline__ float gelu_erf(float x) {
   return x * (x < 0.f ? q : 1.f - q);
 }
 
-// g sigmoid(alpha g) (u + shift) with g = min(g, limit), u = clamp(u, +-limit), for results that are rounded to bf16.  The
-// exponential is the bare instruction, the sigmoid a reciprocal with one correction step (of the reciprocal, not of the product
-// with g: an infinite g stays infinite); where the exponential passes 2^126 the sigmoid is 0.
+// g sigmoid(alpha g) (u + shift) with g = min(g, limit), u = clamp(u, +-limit).  The exponential is the bare instruction, with what
+// its argument's products lost put back (largest error of the sigmoid for gates of -80 to 20, alpha 1 / 1.702: 2.4e-7 / 2.4e-7; with
+// expf 1.8e-7 / 3.9e-6; without that part 3.8e-6 / 7.6e-6).  The sigmoid is a reciprocal with one correction step (of the
+// reciprocal, not of the product with g: an infinite g stays infinite); where the exponential passes 2^126 it is 0.  The clamp of u
+// is one instruction, which pays for that part: 4096 tokens x 4 of 16 experts, width 3584, 1242 us without and with.
 __device__ __forceinline__ float glu_f(float g, float u, float limit, float alpha, float shift) {
+  constexpr float L2E = 1.4426950408889634f, L2E_LO = 1.9259629911266175e-8f;  // log2 e in two parts
   g = fminf(g, limit);
-  u = fminf(fmaxf(u, -limit), limit);
-  const float e = -1.4426950408889634f * (alpha * g);
-  const float d = 1.f + __builtin_amdgcn_exp2f(fminf(e, 126.f));
+  u = __builtin_amdgcn_fmed3f(u, -limit, limit);
+  const float c = -L2E * alpha, cl = fmaf(-L2E_LO, alpha, fmaf(-L2E, alpha, -c)), e = g * c;
+  const float lo = fminf(fmaf(g, cl, fmaf(g, c, -e)), 1.f);  // (no number for an infinite g: 1 then, beside t = 0)
+  const float t = __builtin_amdgcn_exp2f(e);
+  const float d = 1.f + fmaf(0.6931471805599453f * t, lo, t);
   const float rc = __builtin_amdgcn_rcpf(d);
   const float q = fmaf(fmaf(-d, rc, 1.f), rc, rc);
   return g * (e > 126.f ? 0.f : q) * (u + shift);

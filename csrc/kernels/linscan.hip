@@ -324,8 +324,8 @@ linear_scan_kernel(const ScanArgs a) {
   const int vn = min(LVT, a.vd - tile * LVT);
   const int nch = (qlen + LC - 1) / LC;
 
-  // the chunk's rows, fetched while the chunk before is computed (q's behind its outputs): per thread 8 dims of rows krow, krow + 512 / (4 ND), ... of k
-  // and 8 columns of a row of v; per wave its 16 rows of q as operands
+  // the chunk's rows, fetched while the chunk before is computed (q's behind its outputs): per thread 8 dims of rows krow,
+  // krow + 512 / (4 ND), ... of k and 8 columns of a row of v; per wave its 16 rows of q as operands
   constexpr int KT = 4 * ND, KR = LTHREADS / KT, KL = LC / KR > 0 ? LC / KR : 1;  // threads a row, rows a pass, passes
   const int krow = tid / KT, kc = 8 * (tid % KT), vrow = tid >> 3, vc = 8 * (tid & 7);
   TI4 kr[KL][2], vr[2], qr[OUT ? ND : 1][2];

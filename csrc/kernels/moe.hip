@@ -359,8 +359,9 @@ moe_route_mfma_kernel(const T* __restrict__ h, int ld, const float* __restrict__
 // A few tokens (decode rows): one workgroup per token, one wave per logit row (rows w, w + 16, ...), the lanes split the
 // row's columns (8 consecutive ones per lane and step when `vec`) and the sum is a wave reduction.  Bound by round trips to
 // memory: the loads of UN steps of 512 columns (4, or 1 where that is the width) are all issued before their first product.  us
-// with four waves that waited for each step and now, 64 tokens: 201 rows of 512 27 and at most 14 (30 with UN = 4), 17 rows of 3584 12.0 and 9.5, behind an expert layer whose weights push the rows out of
-// the caches 24 and 13; 65 rows 30.0 and 21.4; 17 of 1536 9.2 and 8.0 (with UN = 8 9.5); 8 of 8192 10.5 and 8.8.
+// with four waves that waited for each step and now, 64 tokens: 201 rows of 512 27 and at most 14 (30 with UN = 4), 17 rows of
+// 3584 12.0 and 9.5, behind an expert layer whose weights push the rows out of the caches 24 and 13; 65 rows 30.0 and 21.4;
+// 17 of 1536 9.2 and 8.0 (with UN = 8 9.5); 8 of 8192 10.5 and 8.8.
 template <typename T, int UN>
 __global__ void __launch_bounds__(1024)
 moe_route_rows_kernel(const T* __restrict__ h, int ld, const float* __restrict__ wr, int W, int E, int R, int top,
@@ -476,8 +477,8 @@ struct MoeEpi {
 __device__ __forceinline__ float glu_unit(float g, float u, const MoeEpi& ep) {
   return glu_f(g, u, ep.limit, ep.alpha, ep.shift);
 }
-// The same where the result may stay fp32: the exponent's rounding is put back and the quotient is IEEE's.  Largest error of the
-// value for gates of -80 to 20: glu_f 3.5e-6, with expf 2.7e-6, here 2.0e-7.  Where the exponential is infinite the unit is 0.
+// The same where the result may stay fp32: with the IEEE quotient.  Largest error of the value for gates of -80 to 20: with expf
+// 2.7e-6, here 2.0e-7.  Where the exponential is infinite the unit is 0.
 __device__ __forceinline__ float glu_unit_full(float g, float u, const MoeEpi& ep) {
   constexpr float L2E = 1.4426950408889634f, L2E_LO = 1.9259629911266175e-8f;  // log2 e in two parts
   g = fminf(g, ep.limit);
