@@ -145,7 +145,13 @@ GRAG_API int grag_ar_alloc(long bytes, void** ptr) {
   if (e != hipSuccess) return (int)e;
   return (int)hipMemset(*ptr, 0, (size_t)bytes);
 }
+// For the last moments of a process only: ordinary memory over a freed uncached region has read stale afterwards.
 GRAG_API int grag_ar_free(void* ptr) { return (int)hipFree(ptr); }
+// Zero a region that a new communicator takes over.
+GRAG_API int grag_ar_clear(void* ptr, long bytes) {
+  hipError_t e = hipMemset(ptr, 0, (size_t)bytes);
+  return e != hipSuccess ? (int)e : (int)hipDeviceSynchronize();
+}
 
 GRAG_API int grag_ar_get_handle(void* ptr, void* handle_out /* 64 bytes */) {
   hipIpcMemHandle_t h;

@@ -22,6 +22,7 @@ from __future__ import annotations
 import ctypes
 import logging
 import os
+import threading
 
 import torch
 
@@ -32,7 +33,7 @@ log = logging.getLogger(__name__)
 P, I, L = ctypes.c_void_p, ctypes.c_int, ctypes.c_long
 _SIGS = {
     "grag_ar_data_offset": ([], L), "grag_ar_region_bytes": ([L], L), "grag_ar_alloc": ([L, P], I),
-    "grag_ar_free": ([P], I), "grag_ar_get_handle": ([P, P], I), "grag_ar_handle_size": ([], I),
+    "grag_ar_clear": ([P, L], I), "grag_ar_free": ([P], I), "grag_ar_get_handle": ([P, P], I), "grag_ar_handle_size": ([], I),
     "grag_ar_open_handle": ([P, P], I), "grag_ar_close_handle": ([P], I),
     "grag_ar_oneshot": ([P, I, I, P, P, L, L, P, P, I, L, P], I),
     "grag_ar_oneshot_op": ([P, I, I, I, P, P, L, L, P, P, I, L, P], I),
@@ -48,10 +49,32 @@ def _fn(name):
     return f
 
 
+# A region is uncached device memory that kernels have read: it is never given back to the driver.  Ordinary tensors that
+# were allocated over freed uncached memory have read as zeros from kernels while a copy to the host gave the right values
+# (stale cache lines).  Regions of communicators that no other process has mapped are kept here by size and used again;
+# exported ones are only kept, since a peer may still hold its mapping: one of a few MiB per tensor-parallel group.
+_KEPT: dict[tuple[int, int], list[int]] = {}
+_KEY: dict[int, tuple[int, int]] = {}  # of every region: device, bytes
+_KEPT_LOCK = threading.Lock()
+
+
 def _alloc(nbytes: int) -> int:
+    key = (torch.cuda.current_device(), nbytes)
+    with _KEPT_LOCK:
+        base = _KEPT[key].pop() if _KEPT.get(key) else None
+    if base is not None:
+        check(_fn("grag_ar_clear")(base, nbytes), "grag_ar_clear")  # the flags' epochs start at 0 again
+        return base
     p = ctypes.c_void_p()
     check(_fn("grag_ar_alloc")(nbytes, ctypes.byref(p)), "grag_ar_alloc")
+    _KEY[p.value] = key
     return p.value
+
+
+def _keep(regions) -> None:
+    with _KEPT_LOCK:
+        for base in regions:
+            _KEPT.setdefault(_KEY[base], []).append(base)
 
 
 TIMEOUT_S = float(os.environ.get("GRAG_AR_TIMEOUT_S", "5"))  # a peer slower than this fails the exchange
@@ -60,8 +83,9 @@ TICKS_PER_S = 100_000_000  # s_memrealtime: 100 MHz
 
 class IpcAllReduce:
     def __init__(self, regions: list[int], rank: int, device, slot_bytes: int, owned: list[int],
-                 opened: list[int], grid: int = 64, timeout_s: float | None = None):
+                 opened: list[int], grid: int = 64, timeout_s: float | None = None, exported: bool = False):
         self.regions = regions
+        self._exported = exported
         self.W = len(regions)
         self.rank = rank
         self.device = torch.device(device)
@@ -104,7 +128,7 @@ class IpcAllReduce:
             regions.append(p.value)
             opened.append(p.value)
         dist.barrier(group=pg)
-        return cls(regions, rank, device, slot_bytes, [base], opened, grid)
+        return cls(regions, rank, device, slot_bytes, [base], opened, grid, exported=True)
 
     @classmethod
     def simulated(cls, world: int, device, slot_bytes: int = 1 << 20, grid: int = 64) -> list["IpcAllReduce"]:
@@ -113,14 +137,15 @@ class IpcAllReduce:
         region_bytes = int(_fn("grag_ar_region_bytes")(slot_bytes))
         regions = [_alloc(region_bytes) for _ in range(world)]
         comms = [cls(regions, r, device, slot_bytes, [], [], grid) for r in range(world)]
-        comms[0]._owned = list(regions)  # one owner frees them all
+        comms[0]._owned = list(regions)  # one owner gives them all back
         return comms
 
     def close(self) -> None:
+        """The caller has waited for the communicator's launches.  Regions are kept, never freed."""
         for p in self._opened:
             _fn("grag_ar_close_handle")(p)
-        for p in self._owned:
-            _fn("grag_ar_free")(p)
+        if not self._exported:
+            _keep(self._owned)
         self._opened, self._owned = [], []
 
     # ------------------------------------------------------------------ op
