@@ -703,6 +703,125 @@ auto slab_store = [&](const Acc& acc, int q) {
   }
 }
 
+// Whole tiles, one workgroup per CU that works off a chain of them (tile256_chain).  A workgroup for each tile (gemm_tile_kernel)
+// pays 8 - 10 us a round beside the products: a start, the first loads' way, and a write-out that all CUs begin together.
+// Measured, a workgroup a tile -> chains: 24000 x 2304 x 768 97 -> 85 us, 24000 x 3072 x 768 with GELU 145 -> 135, 24000 x 768 x 768
+// 44 -> 40; gate / up with SwiGLU 8192 x 37888 x 3584 1528 -> 1490, 2405 x 17920 x 1536 113 -> 107; 8192 x 14336 x 3584 597 -> 571, one
+// round of 8192 x 3584 x 18944 758 -> 761.  Bands of 4 or 6 row tiles in place of 8: within 1 %.  Bitwise the same results.
+constexpr int kChainBias = 14336;  // columns whose bias fits the LDS behind the two buffers (28 of 32 KB)
+
+template <int EPI, int ACT, bool BIAS>
+__global__ __launch_bounds__(kThreads, 2) void gemm_chain_kernel(Args p) {
+  constexpr bool GATED = EPI == EPI_SILU || EPI == EPI_GLU;
+  __shared__ __attribute__((aligned(16))) char smem[2 * kBuf + (BIAS ? kChainBias * 2 : 0)];
+  const int tid = threadIdx.x, L = tid & 63, g = L >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = w >> 2, wc = w & 3;
+  bf16* bias = reinterpret_cast<bf16*>(smem + 2 * kBuf);
+  if (BIAS) {
+    for (int i = tid * 8; i < p.N; i += kThreads * 8) *reinterpret_cast<bf16x8_t*>(bias + i) = *reinterpret_cast<const bf16x8_t*>(p.bias + i);
+    __syncthreads();
+  }
+  // an XCD (blockIdx % 8) has a contiguous range of the tiles, its workgroups every 32nd of that (as many as it has)
+  const int tiles = p.tiles_m * p.tiles_n, x = blockIdx.x & 7;
+  const int per = tiles >> 3, rest = tiles & 7, first = x * per + min(x, rest), last = first + per + (x < rest);
+  const int step = (gridDim.x - x + 7) >> 3, mine = first + (blockIdx.x >> 3);
+  if (mine >= last) return;
+  int em = 0, en = 0, m0 = 0, n0 = 0;  // the tile that is stored, the one whose loads were issued last
+  auto next = [&](int i, TileOff& o) __attribute__((always_inline)) {
+    const int t = mine + i * step;
+    if (t >= last) {
+      o = TileOff(kTileNone);
+      return false;
+    }
+    // bands of 8 row tiles x every column tile, rows first
+    constexpr int GM = 8;
+    const int band = GM * p.tiles_n, first_m = t / band * GM, gsz = min(p.tiles_m - first_m, GM);
+    m0 = __builtin_amdgcn_readfirstlane((first_m + t % band % gsz) * 256);
+    n0 = __builtin_amdgcn_readfirstlane(t % band / gsz * 256);
+    if (i == 0) em = m0, en = n0;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int rs = tile_piece_row(r), koff = tile_piece_chunk(r) * 8;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int gm = min(m0 + (rs >> 6) * 128 + q * 64 + (rs & 63), p.M - 1);
+        int gn = min(n0 + (rs >> 5) * 64 + q * 32 + (rs & 31), p.N - 1);
+        if constexpr (EPI == EPI_GLU)
+          gn = q * (p.N / 2) + min(n0 / 2 + (rs >> 5) * 32 + (rs & 31), p.N / 2 - 1);
+        o[2 * q + r] = (unsigned)(gm * p.lda + koff) * 2u;
+        o[4 + 2 * q + r] = (unsigned)(gn * p.ldw + koff) * 2u;
+      }
+    }
+    return true;
+  };
+  const int width = GATED ? p.N / 2 : p.N;
+  auto emit = [&](int q, const TileAcc& l, const TileAcc& r) __attribute__((always_inline)) {
+    const int rows = min(256, p.M - em);
+    // rows and columns that are not there: past the end of the tile's rows
+    const __amdgpu_buffer_rsrc_t rsC = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)((bf16*)p.C + (size_t)em * p.ldc), 0, ((rows - 1) * p.ldc + width) * 2, 0x00020000);
+    const int c0 = GATED ? en / 2 + wc * 32 : en + wc * 64, wcol = (g & 1) * 16 + (g >> 1) * 8;
+    float bv[2][2][4];
+    if constexpr (BIAS) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+          const int col = en + wc * 64 + h * 32 + nt * 16 + 4 * g;
+          const bf16x4_t v = col < p.N ? *reinterpret_cast<const bf16x4_t*>(bias + col) : bf16x4_t{0, 0, 0, 0};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) bv[h][nt][e] = bits2f(v[e]);
+        }
+    }
+    auto put = [&](int mt, int col, const float (&v)[2][4]) __attribute__((always_inline)) {
+      uint32_t d[2][2];
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) d[nt][h] = pack_bf16x2(v[nt][2 * h], v[nt][2 * h + 1]);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const auto s = __builtin_amdgcn_permlane16_swap(d[0][h], d[1][h], false, false);
+        d[0][h] = s[0];
+        d[1][h] = s[1];
+      }
+      const int row = wr * 128 + q * 64 + 16 * mt + (L & 15);
+      const unsigned off = row < rows && col + wcol < width ? (unsigned)(row * p.ldc + col + wcol) * 2u : kTileNone;
+      __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{d[0][0], d[0][1], d[1][0], d[1][1]}, rsC, off, 0, 0);
+    };
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      float v[2][4];
+      if constexpr (GATED) {
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if constexpr (EPI == EPI_GLU) v[nt][e] = glu_f(l[mt][nt][e], r[mt][nt][e], p.limit, p.alpha, p.shift);
+            else if constexpr (BIAS) v[nt][e] = silu_f(l[mt][nt][e] + bv[0][nt][e]) * (r[mt][nt][e] + bv[1][nt][e]);
+            else v[nt][e] = silu_f(l[mt][nt][e]) * r[mt][nt][e];
+          }
+        put(mt, c0, v);
+      } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const TileAcc& acc = h ? r : l;
+#pragma unroll
+          for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[nt][e] = act_f<ACT>(BIAS ? acc[mt][nt][e] + bv[h][nt][e] : acc[mt][nt][e]);
+          put(mt, c0 + 32 * h, v);
+        }
+      }
+    }
+    if (q == 1) em = m0, en = n0;
+  };
+  const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, p.a_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, p.w_bytes, 0x00020000);
+  tile256_chain<GATED ? 4 : 8>(smem, rsA, rsB, p.K >> 6, next, emit);
+}
+
 // Split-K combine: out = epilogue(sum_s ws[s]) — 8 output columns per thread.
 // EPI_STORE: out[M, N] = act(sum + bias); EPI_SILU: out[M, N/2] from the interleaved gate/up layout.
 template <int EPI, int ACT>
@@ -754,6 +873,20 @@ int g_mfma = 16;  // grag_gemm_tile_mfma()
 int g_sched = 2;  // grag_gemm_tile_sched(): 2 the two-phase schedule, 32 MFMAs per barrier interval (default:
                   // +0.9-4.1 % over 1 at 7104 rows, bitwise equal, profiles/ab_tile_sched_r6.json); 1 the balanced
                   // 8/4/8/4-read phase schedule (+5-10 % over 0, profiles/ab_tile_sched_r5.json); 0 the 12/4/8/0 one
+
+// Operands under 2 GB (32-bit offsets), a bias that fits and wide accesses to it and to C, a tile of C under 2 GB.  Whole tiles
+// that fail this take gemm_tile_kernel.
+bool chain_ok(const Args& a) {
+  return a.a_bytes > 0 && a.w_bytes > 0 && (a.bias == nullptr || (a.N <= kChainBias && !((uintptr_t)a.bias & 15))) &&
+         !((uintptr_t)a.C & 15) && a.ldc < (1 << 20);
+}
+template <int EPI, int ACT>
+int launch_chain(const Args& a, int ncu, hipStream_t stream) {
+  const int nwg = min(a.tiles_m * a.tiles_n, ncu);
+  if (a.bias != nullptr) gemm_chain_kernel<EPI, ACT, true><<<nwg, kThreads, 0, stream>>>(a);
+  else gemm_chain_kernel<EPI, ACT, false><<<nwg, kThreads, 0, stream>>>(a);
+  return (int)hipGetLastError();
+}
 
 template <int EPI, int ACT>
 int launch(const Args& a, hipStream_t stream) {
@@ -900,6 +1033,13 @@ static int gemm_tile_run(const void* A, const void* W, const void* bias, void* C
     else RED(EPI_STORE, ACT_NONE);
 #undef RED
     return (int)hipGetLastError();
+  }
+  if (g_mfma == 16 && g_sched == 2 && a.sk_grid == 0 && chain_ok(a)) {
+    if (epi == EPI_SILU) return launch_chain<EPI_SILU, ACT_NONE>(a, ncu, stream);
+    if (epi == EPI_GLU) return launch_chain<EPI_GLU, ACT_NONE>(a, ncu, stream);
+    if (act == ACT_GELU) return launch_chain<EPI_STORE, ACT_GELU>(a, ncu, stream);
+    if (act == ACT_GELU_TANH) return launch_chain<EPI_STORE, ACT_GELU_TANH>(a, ncu, stream);
+    return launch_chain<EPI_STORE, ACT_NONE>(a, ncu, stream);
   }
   if (epi == EPI_SILU) return launch<EPI_SILU, ACT_NONE>(a, stream);
   if (epi == EPI_GLU) return launch<EPI_GLU, ACT_NONE>(a, stream);

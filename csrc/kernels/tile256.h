@@ -51,6 +51,11 @@ __device__ __forceinline__ int tile_piece_row(int i) {
 }
 __device__ __forceinline__ int tile_piece_chunk(int i) { return (threadIdx.x & 7) ^ ((tile_piece_row(i) >> 1) & 7); }
 
+// 16 bytes a lane from rs + off + soff to dst + 16 * lane (no template: the host's pass knows the builtin in none)
+__device__ __forceinline__ void tile_dma(const __amdgpu_buffer_rsrc_t& rs, char* dst, unsigned off, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (tile_lds_t*)dst, 16, off, soff, 0, 0);
+}
+
 // Two-phase schedule: 32 MFMAs per barrier interval.  Per K step t (buffer b = t & 1):
 //   L1 reads A q0, B q0, B q1 (16 b128)  refill A q1 of step t+1 (buffer b^1; read there in L2(t-1))
 //   M1 acc00 = A0 B0, acc01 = A0 B1       (32 MFMAs)
@@ -156,6 +161,138 @@ __device__ __forceinline__ void tile256_loop(char* smem, const __amdgpu_buffer_r
   }
   if (kt == klast) step(kt, std::integral_constant<bool, false>{});
   tile_wait_vm<0>();  // the clamped re-loads land before the LDS is reused
+  if (!lag) tile_bar();
+}
+
+// The same schedule over a chain of tiles that one workgroup works off: the refills of a tile's last two steps are the next
+// tile's first ones, so the loop never drains, and a tile's results are stored while the other half of the waves multiplies and
+// the next tile's steps are in flight: its first row quadrants behind the loads of its last step's L2, the others behind those
+// of the next tile's first L1.  Loads wait for older stores in the memory counter (it counts in order); the waits of the first step
+// behind a tile leave out the 2 * ST2 stores in between, so the stores have a K step's time.
+//   next(i, off): byte offsets of the workgroup's i-th tile at its first K step (kTileNone in all: there is none); whether it is
+//   emit(q, l, r): stores row quadrant q (columns of acc(q)0, acc(q)1) of the tile in exactly ST2 vector-memory instructions
+typedef unsigned TileOff __attribute__((ext_vector_type(8)));  // A [quadrant][piece], B the same (a vector: kept in registers)
+constexpr unsigned kTileNone = 0x80000000u;      // past the end of any operand (< 2 GB): loads zeros without a trip to memory
+
+template <int ST2, typename Next, typename Emit>
+__device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_rsrc_t& rsA, const __amdgpu_buffer_rsrc_t& rsB,
+                                              int nk, Next&& next, Emit&& emit) {
+  const int L = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = w >> 2, wc = w & 3;
+  const bool lag = w >= 4;
+  const int cb = (L >> 4) ^ ((L >> 1) & 7);
+  const int off0 = (L & 15) * 128 + cb * 16, off1 = (L & 15) * 128 + (cb ^ 4) * 16;
+  auto readA = [&](TileA& a, int q, int buf) __attribute__((always_inline)) {
+    const char* base = smem + buf * kTileBuf + q * kTileSlot + wr * 64 * 128;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      a[mt][0] = *reinterpret_cast<const bf16x8_t*>(base + mt * 2048 + off0);
+      a[mt][1] = *reinterpret_cast<const bf16x8_t*>(base + mt * 2048 + off1);
+    }
+  };
+  auto readB = [&](TileB& b, int q, int buf) __attribute__((always_inline)) {
+    const char* base = smem + buf * kTileBuf + (2 + q) * kTileSlot + wc * 32 * 128;
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      b[nt][0] = *reinterpret_cast<const bf16x8_t*>(base + nt * 2048 + off0);
+      b[nt][1] = *reinterpret_cast<const bf16x8_t*>(base + nt * 2048 + off1);
+    }
+  };
+  auto issueA = [&](const TileOff& o, int q, int kt, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) tile_dma(rsA, smem + buf * kTileBuf + q * kTileSlot + (2 * w + i) * 1024, o[2 * q + i], kt * 128);
+  };
+  auto issueB = [&](const TileOff& o, int q, int kt, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      tile_dma(rsB, smem + buf * kTileBuf + (2 + q) * kTileSlot + (2 * w + i) * 1024, o[4 + 2 * q + i], kt * 128);
+  };
+  TileA a;
+  TileB b0, b1;
+  TileAcc acc00, acc01, acc11, acc10;
+  TileOff cur;
+  next(0, cur);
+  issueA(cur, 0, 0, 0);
+  issueB(cur, 0, 0, 0);
+  issueB(cur, 1, 0, 0);
+  issueA(cur, 1, 0, 0);
+  issueA(cur, 0, 1, 1);
+  issueB(cur, 0, 1, 1);
+  issueB(cur, 1, 1, 1);
+  tile_wait_vm<6>();  // step 0 landed
+  tile_bar();
+  if (lag) tile_bar();
+  tile_zero(acc00);
+  tile_zero(acc01);
+  int buf = 0;
+  bool more = true, behind = false;  // behind: a tile's stores lie between the loads
+  auto step = [&](int i, int kt, auto first_c, auto last_c) __attribute__((always_inline)) {
+    constexpr bool FIRST = decltype(first_c)::value, LAST = decltype(last_c)::value;
+    // L1
+    if (FIRST && behind) {  // (its results before the fragments: both would not fit the registers)
+      issueA(cur, 1, 1, buf ^ 1);
+      emit(1, acc10, acc11);
+    }
+    if (FIRST) {
+      tile_zero(acc10);
+      tile_zero(acc11);
+    }
+    readA(a, 0, buf);
+    readB(b0, 0, buf);
+    readB(b1, 1, buf);
+    if (FIRST && behind) {
+      tile_wait_vm<8 + 2 * ST2>();
+    } else {
+      issueA(cur, 1, LAST ? 0 : kt + 1, buf ^ 1);
+      tile_wait_vm<8>();
+    }
+    tile_wait_lds();
+    tile_bar();
+    // M1
+    tile_mma(acc00, a, b0);
+    tile_mma(acc01, a, b1);
+    tile_bar();
+    // L2
+    if (!LAST && kt + 2 == nk) more = next(i + 1, cur);
+    const int k2 = LAST ? 1 : kt + 2 < nk ? kt + 2 : 0;
+    auto refill = [&]() __attribute__((always_inline)) {
+      issueA(cur, 0, k2, buf);
+      issueB(cur, 0, k2, buf);
+      issueB(cur, 1, k2, buf);
+    };
+    if (LAST) {
+      refill();
+      tile_wait_vm<8>();
+      emit(0, acc00, acc01);
+      tile_zero(acc00);
+      tile_zero(acc01);
+      readA(a, 1, buf);
+    } else {
+      readA(a, 1, buf);
+      refill();
+      if (FIRST && behind) tile_wait_vm<8 + 2 * ST2>();
+      else tile_wait_vm<8>();
+    }
+    tile_wait_lds();
+    tile_bar();
+    // M2
+    tile_mma(acc10, a, b0);
+    tile_mma(acc11, a, b1);
+    tile_bar();
+    buf ^= 1;
+  };
+  const std::integral_constant<bool, true> yes{};
+  const std::integral_constant<bool, false> no{};
+  for (int i = 0;; ++i) {
+    step(i, 0, yes, no);
+    for (int kt = 1; kt + 1 < nk; ++kt) step(i, kt, no, no);
+    step(i, nk - 1, no, yes);
+    if (!more) break;
+    behind = true;
+  }
+  emit(1, acc10, acc11);
+  tile_wait_vm<0>();  // the loads of the tile that is not there
   if (!lag) tile_bar();
 }
 

@@ -1,0 +1,63 @@
+"""Whole tiles as chains (csrc/kernels/gemm_tile.hip gemm_chain_kernel): the results of one workgroup a tile, bit for bit, and
+the fp64 product within the rounding of the bf16 result."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from githubrepostorag_amd.ops import gemm as G
+
+pytestmark = pytest.mark.gpu
+
+# one row, ragged tiles in both directions, two K steps (the fewest), an odd count, fewer tiles than CUs and more than one and
+# two rounds of 256 with a ragged last one, 8 tiles more than a round
+SIZES = [(1, 64, 128), (130, 200, 128), (257, 448, 192), (300, 768, 320), (256 * 33, 2048, 128), (2500, 7040, 256), (9000, 4672, 192)]
+
+
+def _both(f):
+    """f's result from chains and from a workgroup a tile (another phase schedule of the same sums)."""
+    chain = f()
+    prev = G.set_sched(1)
+    try:
+        return chain, f()
+    finally:
+        G.set_sched(prev)
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+@pytest.mark.parametrize("bias", [False, True])
+def test_chain(dev, M, N, K, bias):
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    r = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    x, w = r(M, K).bfloat16(), (r(N, K) * K ** -0.5).bfloat16()
+    b = r(N).bfloat16() if bias else None
+    ref = x.double() @ w.double().T + (b.double() if bias else 0)
+    # half an ulp of bf16 (2^-9) of the value, the fp32 sums' rounding (K terms of order 1) and the activation's on top
+    tol = dict(rtol=2 ** -8, atol=2 ** -8 * 0.05)
+    for act, fn in ((G.ACT_NONE, lambda t: t), (G.ACT_GELU, F.gelu), (G.ACT_GELU_TANH, lambda t: F.gelu(t, approximate="tanh"))):
+        got, old = _both(lambda: G.gemm(x, w, b, act=act, ksplit=1, sk=0))
+        assert torch.equal(got, old)
+        torch.testing.assert_close(got.double(), fn(ref), **tol)
+    if N % 64 == 0:
+        got, old = _both(lambda: G.gemm_silu(x, w, b, ksplit=1, sk=0))
+        assert torch.equal(got, old)
+        gate, up = G.deinterleave_gate_up(ref.T.contiguous())
+        torch.testing.assert_close(got.double(), (F.silu(gate) * up).T, **tol)
+    if N % 16 == 0 and not bias:
+        got, old = _both(lambda: G.gemm_glu(x, w, 7.0, 1.702, 1.0))
+        assert torch.equal(got, old)
+        gate, up = ref.chunk(2, 1)
+        gate = gate.clamp(max=7.0)
+        torch.testing.assert_close(got.double(), gate * torch.sigmoid(1.702 * gate) * (up.clamp(-7, 7) + 1), **tol)
+
+
+def test_chain_writes_its_rows_only(dev):
+    """A result with a wider row stride: the columns between the rows stay, in ragged last tiles too."""
+    g = torch.Generator(device=dev).manual_seed(5)
+    M, N, K = 1300, 328, 256
+    x, w = (torch.randn(n, K, generator=g, device=dev).bfloat16() for n in (M, N))
+    big = torch.full((M + 2, N + 24), 7.0, dtype=torch.bfloat16, device=dev)
+    out = big[1:M + 1, 8:N + 8]
+    G.gemm(x, w, out=out, ksplit=1, sk=0)
+    assert torch.equal(out, G.gemm(x, w, ksplit=1, sk=0))
+    out.fill_(7.0)
+    assert bool((big == 7.0).all())
