@@ -11,8 +11,9 @@
 // What bounds it: one thread per state column, three vector instructions per state element and token (the kernels of
 // seqmix.hip and ssm.hip, which still take decode rows and heads of more than 128 rows), waited on LDS broadcasts at 3 % of
 // the fp32 vector rate.  Here a chunk is bound by vector instructions (the splits, SiLU) and the latency of its dependent
-// steps.  Measured, old -> new: decay with SiLU, 28 heads of 128 x 128, 7 portions of 8192 tokens 2150 -> 677 us, 1 x 1187
-// 635 -> 130 us; without SiLU 2060 -> 214 and 602 -> 59; state space, 56 heads of 128 x 64, 3 x 1365 tokens 1450 -> 120 us.
+// steps.  Measured, those kernels -> this one with workgroups in order of sequence -> longest first (scan_item): decay with
+// SiLU, 28 heads of 128 x 128, 7 portions of 8192 tokens 2150 -> 748 -> 410 us, 1 x 1187 635 -> 110; without SiLU 2060 -> 214 -> 153
+// and 602 -> 50; state space, 56 heads of 128 x 64, 3 portions of 4096 tokens 1450 -> 165 -> 115 us.
 //
 // Precision: nothing is rounded to 16 bits that was not before.  An operand is the sum of bf16 parts of 8 bits of mantissa
 // each, and a product of operands is the matrix-core products of their parts (exact, fp32 sums).  What is fp32 (S, the
@@ -55,7 +56,7 @@ struct ScanArgs {
   float* state;
   const int *slots, *q_start, *ctx_len;
   float* out;
-  int H, d, vd, nslots;
+  int nseq, H, d, vd, nslots;
   float *ws, *wa;
   int part, maxparts, full;
   // decay
@@ -233,8 +234,43 @@ __device__ __forceinline__ void parts4(const ScanArgs& a, bf16x4_t (&p)[3], TV r
 }
 
 // ------------------------------------------------------------------------------------------------ the scan
-// grid nseq * maxparts * H * ceil(vd / 64): the column tiles of a head beside each other, heads next (they share k / q rows
-// in the state-space form), on one XCD.  ND = ceil(d / 32).  AP = 1 takes 76 KB of LDS and 128 registers: two workgroups
+// The sequence and part of work item `item` (false: there is none).  Longest first: the full parts, then the rests by length,
+// so that the last workgroups to start are short ones.  Up to 64 sequences (a lane each); more are taken as they come.
+__device__ __forceinline__ bool scan_item(const ScanArgs& a, int item, int& seq, int& part) {
+  if (a.nseq > 64) {
+    seq = item / a.maxparts, part = item % a.maxparts;
+    return seq < a.nseq;
+  }
+  const int lane = threadIdx.x & 63;
+  const int len = lane < a.nseq ? a.q_start[lane + 1] - a.q_start[lane] : 0;
+  const int full = len / a.part, rest = len - full * a.part;
+  int upto = full;  // full parts of the lanes up to this one
+#pragma unroll
+  for (int o = 1; o < 64; o *= 2) {
+    const int v = __shfl_up(upto, o, 64);
+    if (lane >= o) upto += v;
+  }
+  const int nfull = __builtin_amdgcn_readlane(upto, 63);
+  if (item < nfull) {
+    seq = __ffsll((unsigned long long)__ballot(upto > item)) - 1;
+    part = __builtin_amdgcn_readlane(upto, seq) - 1 - item;  // (a sequence's last parts first: they fold the most states)
+    return true;
+  }
+  int before = 0;
+  for (int k = 0; k < a.nseq; ++k) {
+    const int r = __builtin_amdgcn_readlane(rest, k);
+    before += r > rest || (r == rest && k < lane);
+  }
+  const unsigned long long at = __ballot(rest > 0 && before == item - nfull);
+  if (!at) return false;
+  seq = __ffsll(at) - 1;
+  part = __builtin_amdgcn_readlane(full, seq);
+  return true;
+}
+
+// grid 8 * ceil(items * H / 8) * ceil(vd / 64): the column tiles of a head beside each other on one XCD (they read the same rows of q
+// and k), the next head on the next XCD, the items' heads in the order of scan_item.  With a contiguous range of sequences an XCD the
+// XCDs that had the long ones walked on while others were done: 7 portions of 8192 tokens, a CU was busy 48 % of the time.  ND = ceil(d / 32).  AP = 1 takes 76 KB of LDS and 128 registers: two workgroups
 // share a CU, one's products over the other's staging.  FULL: d = 32 ND, vd is a multiple of 64 and rows are aligned for
 // 4-element accesses (rd / 2 a multiple of 4), so that nothing is tested per element: of the ~4000 instructions a chunk took
 // with the tests, half were theirs.  Rows behind a portion's end are copies of its last row with weight c_s = 0.
@@ -251,12 +287,9 @@ linear_scan_kernel(const ScanArgs a) {
   __shared__ float ends[2][3];                                 // 2^(L_end) | L_end | not 0: too large for the products
   __shared__ __attribute__((aligned(16))) int odd[LTHREADS / 64];  // a wave's numbers are too large for the products
   const int ntile = (a.vd + LVT - 1) / LVT;
-  int id = xcd_remap(blockIdx.x, gridDim.x);
-  const int tile = id % ntile;
-  id /= ntile;
-  const int h = id % a.H;
-  id /= a.H;
-  const int part = id % a.maxparts, seq = id / a.maxparts;
+  const int tile = (blockIdx.x >> 3) % ntile, unit = (blockIdx.x >> 3) / ntile * 8 + (blockIdx.x & 7), h = unit % a.H;
+  int seq, part;
+  if (!scan_item(a, unit / a.H, seq, part)) return;
   const int q0 = a.q_start[seq], qall = a.q_start[seq + 1] - q0;
   if (part * a.part >= qall) return;
   const int nparts = (qall + a.part - 1) / a.part;
@@ -652,7 +685,7 @@ linear_scan_kernel(const ScanArgs a) {
 
 template <typename TI, int AP, bool SSM, bool FULL, int ND>
 static hipError_t launch_scan(const ScanArgs& a, int nseq, hipStream_t st) {
-  const long blocks = (long)nseq * a.maxparts * a.H * ((a.vd + LVT - 1) / LVT);
+  const long blocks = ((long)nseq * a.maxparts * a.H + 7) / 8 * 8 * ((a.vd + LVT - 1) / LVT);
   if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
   if (a.maxparts > 1)
     hipLaunchKernelGGL((linear_scan_kernel<TI, AP, SSM, FULL, ND, 1>), dim3((unsigned)blocks), dim3(LTHREADS), 0, st, a);
@@ -691,7 +724,7 @@ GRAG_API hipError_t grag_linear_scan_decay(const void* proj, int ld, int qoff, i
   ScanArgs a{};
   a.x = proj, a.ld = ld, a.qoff = qoff, a.koff = koff, a.voff = voff, a.R = 1;
   a.state = state, a.slots = slots, a.q_start = q_start, a.ctx_len = ctx_len, a.out = out;
-  a.H = H, a.d = d, a.vd = vd, a.nslots = nslots, a.ws = ws, a.wa = wa;
+  a.nseq = nseq, a.H = H, a.d = d, a.vd = vd, a.nslots = nslots, a.ws = ws, a.wa = wa;
   a.part = part, a.maxparts = (max_q_len + part - 1) / part;
   a.decay = decay, a.kscale = kscale, a.act = act, a.positions = positions, a.rope = rope_tab, a.rd = rd, a.tab_rows = tab_rows;
   a.full = !((ld | qoff | koff | voff) & 3) && !(vd & 63) && !(rd & 7) && !((uintptr_t)proj & 7) &&
@@ -711,7 +744,7 @@ GRAG_API hipError_t grag_linear_scan_ssm(const void* xbc, int C, int boff, int c
   ScanArgs a{};
   a.x = xbc, a.ld = C, a.qoff = coff, a.koff = boff, a.voff = 0, a.R = H / G;
   a.state = state, a.slots = slots, a.q_start = q_start, a.ctx_len = ctx_len, a.out = out;
-  a.H = H, a.d = N, a.vd = P, a.nslots = nslots, a.ws = ws, a.wa = wa;
+  a.nseq = nseq, a.H = H, a.d = N, a.vd = P, a.nslots = nslots, a.ws = ws, a.wa = wa;
   a.part = part, a.maxparts = (max_q_len + part - 1) / part;
   a.proj = proj, a.pld = ld, a.dtoff = dtoff, a.dt_bias = dt_bias, a.a_log = A_log, a.skip = Dv;
   a.full = !((C | boff | coff) & 3) && !(P & 63) && !((uintptr_t)xbc & 7) && !((uintptr_t)out & 15);

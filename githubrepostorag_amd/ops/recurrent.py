@@ -33,19 +33,32 @@ LINEAR_SCAN_CHUNK = 64
 def _scan_walks(max_q: int, tokens: int, nseq: int, tiles: float, split: bool) -> tuple[float, int]:
     """(walks, chunks a part) of the matrix-core scan (csrc/kernels/linscan.hip) for a step of ``nseq`` portions with
     ``tokens`` tokens, the longest ``max_q``, and ``tiles`` (head, 64 columns) tiles a portion: its length in walks of a
-    64-token chunk and the cut of a portion that makes it shortest.  Whole portions cost the longest walk, or the chip's
-    share of all; cut into parts, every round of workgroups walks a part twice (the first walk, for the state alone, is
-    about half) and reads the states of the parts before it.  ``split``: operands in three parts (one workgroup a CU,
-    12 us a chunk), else two workgroups a CU and 5 us."""
-    slots, read = (256, 0.06) if split else (512, 0.28)
-    chunks, total = -(-max_q // LINEAR_SCAN_CHUNK), tokens / LINEAR_SCAN_CHUNK
-    best, part, s = 0.85 * max(chunks, total * tiles / slots), chunks, 1
+    64-token chunk and the cut of a portion that makes it shortest.  Workgroups start longest first, so several portions
+    take the longest walk or the chip's share of all and about a third of a walk for its uneven end; a single portion whole
+    rounds of equal parts.  Where portions are cut, all parts but the last are walked for the state alone before (0.42 of a
+    walk), and a part reads the states of those before it.  ``split``: operands in three parts (one workgroup a CU, 12 us a
+    chunk), else two workgroups a CU and 5.7 us.
+
+    us, cut at 2 / 4 / 8 / 16 chunks / not at all: 28 heads of 128 x 128 with SiLU 3 portions of 4096 tokens 291 / 270 / 260
+    / 269 / 340 (taken 8), 7 of 8192 567 / 498 / 465 / 443 / 410 - 448 (none); state space, 56 heads of 128 x 64, 3 of 4096
+    141 / 116 / 110 / 149 / 171 (8); 24 of 128 x 64, one of 8192 177 / 122 / 115 / 146 / 517 (8)."""
+    slots, read, crowd = (256, 0.026, 1.0) if split else (512, 0.11, 1.2)  # (whole portions often have a CU of their own)
+    chunks, total = -(-max_q // LINEAR_SCAN_CHUNK), tokens / LINEAR_SCAN_CHUNK + (nseq - 1) / 2
+    share = tiles / slots  # of a round, a workgroup for each tile
+
+    def walk(s, work):  # of parts of s chunks that are ``work`` chunks together
+        if nseq == 1:
+            return -(-int(-(-work // s) * tiles) // slots) * s
+        return max(s, work * share + 0.35 * s)
+
+    best, part, s = max(chunks, total * share + 0.35 * total / nseq), chunks, 1
     while s < chunks:
-        rounds = -(-int((total / s + nseq / 2) * tiles) // slots)
-        cost = max(1, rounds) * (1.5 * s + read * chunks / s) + 1
+        ahead = total - nseq * s / 2 if nseq > 1 else (-(-chunks // s) - 1) * s
+        cost = walk(s, chunks if nseq == 1 else total) + 0.42 * walk(s, max(ahead, s)) + 1
+        cost = crowd * (cost + read * chunks / s * max(1.0, total / s * share))
         if cost < best:
             best, part = cost, s
-        s *= 2
+        s += max(1, s // 2) if s & (s - 1) == 0 else s // 3  # 1, 2, 3, 4, 6, 8, 12, 16, ..
     return best, part
 
 
