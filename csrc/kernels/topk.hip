@@ -15,8 +15,8 @@
 // rounds (top-K of two sorted lists = elementwise max against the reversed
 // partner list, then a half-cleaner network), so each wave emits one list per
 // query.  In a flat scan the workgroup's waves merge theirs through LDS (three
-// rounds), and topk_lists_merge_kernel folds the workgroups' lists: a sorted
-// list per thread, then the same network across lanes and waves.  (The lists of
+// rounds), and topk_lists_merge_kernel picks the best of the workgroups' lists.
+// (The lists of
 // all waves through a library sort took 15 launches and 100 us behind a scan of
 // 330 us: 1M x 768, 16 queries, k = 10, 428 -> 323, 20K rows
 // 103 -> 38.)
@@ -123,17 +123,42 @@ __device__ __forceinline__ void list_merge_xor(float (&v)[K], uint32_t (&id)[K],
   list_merge<K>(v, id, w, wi);
 }
 
-__device__ __forceinline__ bool row_passes(const TopkParams& p, int64_t row) {
-  if (p.bitmap && !((p.bitmap[row >> 5] >> (row & 31)) & 1u)) return false;
+// What the filters ask of rows row .. row + 3 (rows from r1 on: the last one's): a bit per row of the bitmap, a column's value per
+// filter and row
+typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
+struct RowKeys {
+  uint32_t alive;
+  i32x4_t col[4];
+};
+__device__ __forceinline__ RowKeys row_keys(const TopkParams& p, int64_t row, int64_t r1) {
+  RowKeys k;
+  k.alive = 15;
+  if (p.bitmap) {
+    k.alive = 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t at = min(row + r, r1 - 1);
+      k.alive |= ((p.bitmap[at >> 5] >> (at & 31)) & 1u) << r;
+    }
+  }
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+    if (f < p.nfilt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) k.col[f][r] = p.fcol[f][min(row + r, r1 - 1)];
+  return k;
+}
+__device__ __forceinline__ bool row_passes(const TopkParams& p, const RowKeys& k, int r) {
+  bool ok = (k.alive >> r) & 1u;
 #pragma unroll
   for (int f = 0; f < 4; ++f) {
     if (f < p.nfilt) {
-      const int32_t c = p.fcol[f][row];
-      if (p.fop[f] == 1 && c != p.fval[f]) return false;
-      if (p.fop[f] == 2 && (c & p.fval[f]) == 0) return false;
+      const int32_t c = r < 2 ? (r == 0 ? k.col[f][0] : k.col[f][1]) : (r == 2 ? k.col[f][2] : k.col[f][3]);
+      if (p.fop[f] == 1 && c != p.fval[f]) ok = false;
+      if (p.fop[f] == 2 && (c & p.fval[f]) == 0) ok = false;
     }
   }
-  return true;
+  return ok;
 }
 
 template <int NQT, int KMAX>
@@ -201,21 +226,28 @@ __global__ __launch_bounds__(64 * NWAVES) void score_topk_kernel(TopkParams p) {
     }
   });
 
+  // A tile's 32-dim steps in batches of U, two batches of registers: one in flight while the other is multiplied, the next tile's
+  // first one too, so that 8 waves a CU keep the stream up.  The filters' columns of a tile's rows are loaded ahead of its batches.
+  constexpr int U = NQT == 1 ? 6 : NQT == 2 ? 4 : 3, STEP = 16 * NWAVES;
   const int nc = d / 32;
-  for (int64_t t0 = r0 + wave * 16; t0 < r1; t0 += 16 * NWAVES) {
-    int64_t lrow = t0 + li;
-    if (lrow >= r1) lrow = r1 - 1;
-    const bf16* xp = p.X + lrow * d + 8 * h4;
+  bf16x8_t a0[U], a1[U];
+  auto load = [&](bf16x8_t (&a)[U], int64_t t0, int c) __attribute__((always_inline)) {
+    const bf16* xp = p.X + min(t0 + li, r1 - 1) * d + 8 * h4 + 32 * c;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (c + u < nc) a[u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(xp + 32 * u));
+  };
+  const int64_t first = r0 + wave * 16;
+  if (first < r1) load(a0, first, 0);
+#pragma unroll 1
+  for (int64_t t0 = first; t0 < r1; t0 += STEP) {
+    const RowKeys keys = row_keys(p, t0 + 4 * h4, r1);
     f32x4_t acc[NQT];
 #pragma unroll
     for (int qt = 0; qt < NQT; ++qt) acc[qt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    for (int c = 0; c < nc; c += 4) {
-      bf16x8_t a[4];
+    auto mul = [&](const bf16x8_t (&a)[U], int c) __attribute__((always_inline)) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (c + u < nc) a[u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(xp + 32 * (c + u)));
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < U; ++u) {
         if (c + u < nc) {
 #pragma unroll
           for (int qt = 0; qt < NQT; ++qt) {
@@ -226,11 +258,19 @@ __global__ __launch_bounds__(64 * NWAVES) void score_topk_kernel(TopkParams p) {
           }
         }
       }
+    };
+#pragma unroll 1
+    for (int c = 0; c < nc; c += 2 * U) {
+      if (c + U < nc) load(a1, t0, c + U);
+      mul(a0, c);
+      if (c + 2 * U < nc) load(a0, t0, c + 2 * U);
+      else if (t0 + STEP < r1) load(a0, t0 + STEP, 0);
+      mul(a1, c + U);
     }
 #pragma unroll(NQT * KMAX > 32 ? 1 : 4)
     for (int r = 0; r < 4; ++r) {
       const int64_t row = t0 + 4 * h4 + r;
-      const bool ok = row < r1 && row_passes(p, row);
+      const bool ok = row < r1 && row_passes(p, keys, r);
       const uint32_t off = (uint32_t)(row - r0);
       static_for<NQT>([&](auto qt) {
         bool okq = ok;
@@ -294,52 +334,109 @@ __global__ __launch_bounds__(64 * NWAVES) void score_topk_kernel(TopkParams p) {
   });
 }
 
-// The final lists of a flat scan: query q's sorted lists of k are rows (q / G * n + j) * G + q % G, j < n, of ps / pi.
-// grid (nq), 256 threads.
-template <int K>
+// (value, number) in falling order of value, ties by rising number
+__device__ __forceinline__ bool ahead(float v, uint32_t i, float w, uint32_t j) { return v > w || (v == w && i < j); }
+// the largest of a wave's numbers, by moves between neighbouring lanes (lane 63 ends with it)
+template <int CTRL, int ROWS> __device__ __forceinline__ float max_step(float v) {
+  const float low = -INFINITY;
+  return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(low), __float_as_int(v), CTRL, ROWS, 0xf, false)));
+}
+__device__ __forceinline__ float wave_top(float v) {
+  v = max_step<0x111, 0xf>(v);  // 1, 2, 4, 8 lanes down within 16, then lane 15 of rows 0, 2 and lane 31 into those behind
+  v = max_step<0x112, 0xf>(v);
+  v = max_step<0x114, 0xf>(v);
+  v = max_step<0x118, 0xf>(v);
+  v = max_step<0x142, 0xa>(v);
+  v = max_step<0x143, 0xc>(v);
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+constexpr int kMergeLists = 1024;  // lists of a query at most
+
+// The final lists of a flat scan: query q's sorted lists of k are rows (q / G * n + j) * G + q % G, j < n <= kMergeLists, of ps /
+// pi.  grid (nq), 256 threads.  Only the k lists with the best heads can hold one of the best k, and of those only what is not
+// behind the last of these heads: every wave takes the best k of its quarter of the heads one by one, wave 0 the best k of these;
+// their elements, loaded at once with their ids, are ranked by counting.  Three ways to memory, where folding list into list took
+// one for each of a thread's lists and then 64 merges of sorted lists in registers: 1M rows, 16 queries, k = 10 26 us -> 12,
+// 64 queries, k = 30 48 -> 28 (with 256 lists in place of 1024).
 __global__ __launch_bounds__(256) void topk_lists_merge_kernel(const float* __restrict__ ps, const int64_t* __restrict__ pi,
                                                                int n, int G, int k, float* __restrict__ out_s,
                                                                int64_t* __restrict__ out_i) {
-  __shared__ float lv[4][K];
-  __shared__ uint32_t li[4][K];
+  __shared__ float hv[4 * 32], cv[32 * 32];
+  __shared__ uint32_t hj[4 * 32], best[32], cnum[32 * 32];
+  __shared__ int64_t cid[32 * 32];
+  __shared__ float last_v;
+  __shared__ uint32_t last_j;
+  __shared__ int count;
   const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t base = (int64_t)(q / G) * n * G + q % G;
-  float v[K];
-  uint32_t id[K];
+  const uint32_t none = 0xFFFFFFFFu;
+  float h[kMergeLists / 256];
 #pragma unroll
-  for (int i = 0; i < K; ++i) v[i] = -INFINITY, id[i] = 0;
-  for (int j = tid; j < n; j += 256) {
-    const float* l = ps + (base + (int64_t)j * G) * k;
-    float w[K];
-    uint32_t wi[K];
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-      const int t = K - 1 - i;
-      w[i] = t < k ? l[t] : -INFINITY;
-      wi[i] = (uint32_t)(j * k + t);
-    }
-    if (w[K - 1] > v[K - 1]) list_merge<K>(v, id, w, wi);
+  for (int u = 0; u < kMergeLists / 256; ++u) {
+    const int j = u * 256 + tid;
+    h[u] = j < n ? ps[(base + (int64_t)j * G) * k] : -INFINITY;
   }
+  if (tid == 0) count = 0;
+  for (int r = 0; r < k; ++r) {
+    float v = -INFINITY;
+    uint32_t j = none;
 #pragma unroll
-  for (int m = 1; m < 64; m <<= 1) list_merge_xor<K>(v, id, m);
-  if (lane == 0) {
+    for (int u = 0; u < kMergeLists / 256; ++u)
+      if (h[u] > v) v = h[u], j = u * 256 + tid;
+    const float top = wave_top(v);
+    uint32_t first = none;  // of the lanes that have it the lowest list
+    for (unsigned long long at = __ballot(v == top && j != none); at; at &= at - 1)
+      first = min(first, (uint32_t)__builtin_amdgcn_readlane((int)j, __ffsll(at) - 1));
 #pragma unroll
-    for (int i = 0; i < K; ++i) lv[wave][i] = v[i], li[wave][i] = id[i];
+    for (int u = 0; u < kMergeLists / 256; ++u)
+      if (first == (uint32_t)(u * 256 + tid)) h[u] = -INFINITY;
+    if (lane == 0) hv[wave * 32 + r] = top, hj[wave * 32 + r] = first;
   }
   __syncthreads();
-  if (wave != 0) return;
-#pragma unroll
-  for (int i = 0; i < K; ++i) v[i] = lv[lane & 3][i], id[i] = li[lane & 3][i];
-  list_merge_xor<K>(v, id, 1);
-  list_merge_xor<K>(v, id, 2);
-  if (lane != 0) return;
-#pragma unroll
-  for (int i = 0; i < K; ++i) {
-    if (i >= k) break;
-    const bool any = v[i] != -INFINITY;
-    const uint32_t j = id[i] / (uint32_t)k;
-    out_s[(int64_t)q * k + i] = v[i];
-    out_i[(int64_t)q * k + i] = any ? pi[(base + (int64_t)j * G) * k + id[i] % (uint32_t)k] : -1;
+  // of 4 k heads the best k: as many as are ahead of one
+  if (tid < 128) {
+    const int r = tid & 31;
+    const bool on = r < k && hj[tid] != none;
+    int rank = 0;
+    if (on)
+      for (int w = 0; w < 4; ++w)
+        for (int i = 0; i < k; ++i) rank += ahead(hv[w * 32 + i], hj[w * 32 + i], hv[tid], hj[tid]) && hj[w * 32 + i] != none;
+    if (on && rank < k) best[rank] = hj[tid];
+    if (on && rank == k - 1) last_v = hv[tid], last_j = hj[tid];
+    const int got = __popcll(__ballot(on));
+    if (lane == 0) atomicAdd(&count, got);
+  }
+  __syncthreads();
+  const int lists = min(count, k), full = count >= k;  // (heads that are there: no list without one has anything)
+  __syncthreads();
+  if (tid == 0) count = 0;
+  __syncthreads();
+  for (int e = tid; e < lists * k; e += 256) {
+    const uint32_t j = best[e / k];
+    const int t = e % k;
+    const int64_t at = (base + (int64_t)j * G) * k + t;
+    const float v = ps[at];
+    const int64_t id = pi[at];
+    // (of lists with equal values the heads decide: behind the last head's list nothing that equals it is among the best)
+    if (v != -INFINITY && (!full || v > last_v || (v == last_v && j <= last_j))) {
+      const int c = atomicAdd(&count, 1);
+      cv[c] = v, cnum[c] = j * (uint32_t)k + t, cid[c] = id;
+    }
+  }
+  __syncthreads();
+  const int c = count;
+  for (int e = tid; e < c; e += 256) {
+    int rank = 0;
+    for (int i = 0; i < c; ++i) rank += ahead(cv[i], cnum[i], cv[e], cnum[e]);
+    if (rank < k) {
+      out_s[(int64_t)q * k + rank] = cv[e];
+      out_i[(int64_t)q * k + rank] = cid[e];
+    }
+  }
+  for (int r = c + tid; r < k; r += 256) {
+    out_s[(int64_t)q * k + r] = -INFINITY;
+    out_i[(int64_t)q * k + r] = -1;
   }
 }
 
@@ -394,9 +491,8 @@ GRAG_API int grag_topk_num_waves() { return NWAVES; }
 GRAG_API int grag_topk_lists_merge(const float* ps, const int64_t* pi, int n, int G, int nq, int k, float* out_s,
                                    int64_t* out_i, hipStream_t stream) {
   if (nq <= 0) return 0;
-  if (n < 1 || G < 1 || k < 1 || k > 32 || (int64_t)n * k >= (1LL << 32)) return (int)hipErrorInvalidValue;
-  if (k <= 16) topk_lists_merge_kernel<16><<<nq, 256, 0, stream>>>(ps, pi, n, G, k, out_s, out_i);
-  else topk_lists_merge_kernel<32><<<nq, 256, 0, stream>>>(ps, pi, n, G, k, out_s, out_i);
+  if (n < 1 || n > kMergeLists || G < 1 || k < 1 || k > 32) return (int)hipErrorInvalidValue;
+  topk_lists_merge_kernel<<<nq, 256, 0, stream>>>(ps, pi, n, G, k, out_s, out_i);
   return (int)hipGetLastError();
 }
 

@@ -7,6 +7,7 @@ from dataclasses import dataclass
 import torch
 
 from ._lib import call, lib, ptr
+from .linear import num_cus
 
 OP_EQ, OP_BITAND = 1, 2
 MAX_FILTERS = 4
@@ -14,6 +15,7 @@ MAX_K = 32
 # 64 queries a workgroup read the rows once for all of them but leave two waves a SIMD for the lists' upkeep: from ~half a
 # million rows the reads win (1M x 768: 64 queries 639 -> 532 us, 128 1220 -> 870), below they do not (100K: 122 against 221)
 NQT4_MIN_ROWS = 1 << 19
+_MAX_LISTS = 1024  # lists of a query that the merge takes
 NQT4_MAX_D = 1152  # widest rows of which a workgroup's LDS holds 64 queries
 
 
@@ -136,7 +138,10 @@ def score_topk(X: torch.Tensor, Q: torch.Tensor, k: int, preds=None, bitmap=None
     rows = N - row_begin
     nqt = _nqt_for(nq, d, kmax, rows)
     nqtiles = (nq + nqt * 16 - 1) // (nqt * 16)
-    target = max(1, 1024 // nqtiles)
+    # a workgroup per CU in all: the kernel keeps its stream up with 8 waves a CU, and every workgroup more is a list more to build and
+    # to merge (1M rows 1024 / 512 / 256 workgroups: 16 queries 334 / 304 / 298 us, 64 with k = 30 and a filter 831 / 741 / 665; 85K
+    # rows, 21 queries 104 / 79 / 61)
+    target = max(1, min(_MAX_LISTS, num_cus()) // nqtiles)
     rows_per_wg = max(128, -(-rows // target))
     rows_per_wg = -(-rows_per_wg // 16) * 16
     nchunks = -(-rows // rows_per_wg)
