@@ -28,7 +28,7 @@ import torch
 from ._lib import call, ptr
 
 ACT_NONE, ACT_GELU, ACT_SILU, ACT_GELU_TANH = 0, 1, 2, 3
-EPI_STORE, EPI_SILU, EPI_PARTIAL = 0, 1, 2
+EPI_STORE, EPI_SILU, EPI_PARTIAL, EPI_GLU = 0, 1, 2, 3
 _ON = os.environ.get("GRAG_TILE_GEMM", "1") != "0"
 
 
@@ -245,6 +245,76 @@ def schedule(M: int, N: int, K: int, silu: bool = False) -> tuple[int, int]:
     return plan(M, N, K)
 
 
+# ---------------------------------------------------------------- small tiles (csrc/kernels/gemm_pair.hip)
+PAIR_TILES = ((128, 192), (128, 128), (64, 128), (64, 64))  # by its number of a shape
+
+
+def _pair_tiles(shape: int, M: int, N: int) -> int:
+    bm, bn = PAIR_TILES[shape]
+    return -(-M // bm) * -(-N // bn)
+
+
+def pair_plan(M: int, N: int, K: int, fused: bool = False) -> int | None:
+    """The small-tile kernel's shape for a product that gives the 256 x 256 tile too few tiles, or None.  ``fused``: with an
+    activation or a gated unit in the epilogue (no library call does that in one launch), else plain.
+
+    One product after another of different weights, in a graph, us.  Plain, K <= 1024: 64 x 64 tiles up to two a CU beat the
+    library (768 x 768 at 300 / 1136 / 1752 rows 7.1 / 7.9 / 9.4 -> 6.1 / 6.4 / 7.7; 2304 x 768 600 9.4 -> 7.8, 1136, 648 tiles,
+    10.0 / 10.5) and the decode kernel's K parts (64 / 256 rows 10.5 / 19.6 -> 6.1 / 6.3); up to 32 rows the skinny kernel stays
+    (20 rows 4.5 / 6.0).  Fused, K <= 2048: 64 x 64 up to 704 tiles, then 64 x 128 and 128 x 128 up to 512 each, against the
+    256 x 256 tile (GELU 3072 x 768 at 300 / 1136 / 1752 / 2500 rows 24 / 31 / 42 / 45 -> 6.9 / 12.3 / 17.5 / 19.9, from 4200 on 29
+    / 33; SwiGLU 4096 x 1024 260 27 -> 10, 17920 x 1536 300 35 -> 29, 400 36 / 49; 22016 x 4096 260 80 / 104)."""
+    if not _ON or M < 1 or max(M, N) * K >= 1 << 30 or K > (2048 if fused else 1024):
+        return None
+    ncu = _num_cus()
+    if not fused:
+        return 3 if M >= 33 and _pair_tiles(3, M, N) <= 2 * ncu else None
+    if _pair_tiles(3, M, N) <= 2.75 * ncu:
+        return 3
+    return next((s for s in (2, 1) if _pair_tiles(s, M, N) <= 2 * ncu), None)
+
+
+def pair_fills(M: int, N: int, K: int) -> bool:
+    """Whether short contractions whose 256 x 256 tiles would leave their last round of CUs nearly empty go in 128 x 192 ones:
+    24000 x 768 x 768 (282 tiles) 40 -> 34.5 us, 8000 x 2304 x 768 (288) 38 -> 34; fuller ones not (12000 x 2304 x 768, 0.82 of
+    the rounds, 42 / 52)."""
+    tiles, ncu = -(-M // 256) * -(-N // 256), _num_cus()
+    return K <= 1024 and tiles > ncu and M * N < 0.62 * 65536 * ncu * -(-tiles // ncu)
+
+
+def pair_takes(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None, out: torch.Tensor | None = None) -> bool:
+    """Operands of ``supported`` that the small-tile kernel takes too: byte offsets of 31 bits, aligned bias and result."""
+    return (x.stride(0) * x.shape[0] < 1 << 30 and w.stride(0) * w.shape[0] < 1 << 30
+            and (b is None or (b.dtype == torch.bfloat16 and b.is_contiguous() and b.data_ptr() % 8 == 0))
+            and (out is None or (out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 8 == 0
+                                 and out.data_ptr() % 16 == 0)))
+
+
+def gemm_pair(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, shape: int, epi: int = EPI_STORE, act: int = ACT_NONE,
+              out: torch.Tensor | None = None, glu: tuple = (0.0, 0.0, 0.0)) -> torch.Tensor:
+    """The small-tile kernel: act(x @ w.T + b), the SwiGLU product (EPI_SILU) or the gated unit (EPI_GLU) of (limit, alpha,
+    shift), in tiles of PAIR_TILES[shape]."""
+    M, K = x.shape
+    N = w.shape[0]
+    if out is None:
+        out = torch.empty(M, N if epi == EPI_STORE else N // 2, dtype=x.dtype, device=x.device)
+    call("grag_gemm_pair", ptr(x), ptr(w), ptr(b), ptr(out), x.stride(0), w.stride(0), out.stride(0), M, N, K, epi, act, shape,
+         *map(float, glu))
+    return out
+
+
+def wide_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
+    """(1, 0) where a plain product of K >= 1152 outside the measured table goes to the owned kernel in whole tiles: where they
+    fill 0.65 of their rounds of CUs.  228 points of 19 widths and depths (1536 - 28672 x 1536 - 13824) at 400 - 8192 rows, one
+    product after another of different weights: library over owned 1.08 in the geometric mean above the line (102 points,
+    0.95 - 1.61: 18944 x 3584 at 2405 rows 360 / 232 us, 4000 500 / 385), 0.98 at 0.6 - 0.65 in one round, 0.84 and less
+    below a half."""
+    tiles, ncu = -(-M // 256) * -(-N // 256), _num_cus()
+    if M < PREFILL_MIN_M or K < 1152 or K % 64 or max(M, N) * K >= 1 << 30 or (N, K, 0) in _prefill_table():
+        return None
+    return (1, 0) if M * N >= 0.65 * 65536 * ncu * -(-tiles // ncu) else None
+
+
 def set_mfma(mf: int) -> int:
     """Select the tile kernel's MFMA shape for later launches (16: v_mfma_f32_16x16x32_bf16, the default;
     32: v_mfma_f32_32x32x16_bf16; csrc/kernels/gemm_tile.hip ``Shape``).  Returns the previous shape."""
@@ -424,7 +494,14 @@ def gemm(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None, act: i
         return y.to(x.dtype)
     M, K = x.shape
     N = w.shape[0]
-    ksplit, sk = schedule(M, N, K) if ksplit is None else (ksplit, sk or 0)
+    if ksplit is None:
+        shape = pair_plan(M, N, K, act != ACT_NONE)
+        if shape is not None and pair_takes(x, w, b, out):
+            return gemm_pair(x, w, b, shape, EPI_STORE, act, out)
+        ksplit, sk = schedule(M, N, K)
+        if (ksplit, sk) == (1, 0) and pair_fills(M, N, K) and pair_takes(x, w, b, out):
+            return gemm_pair(x, w, b, 0, EPI_STORE, act, out)
+    sk = sk or 0
     if out is None:
         out = torch.empty(M, N, dtype=x.dtype, device=x.device)
     return _launch(x, w, b, out, EPI_STORE, act, ksplit, sk)
@@ -443,7 +520,12 @@ def gemm_silu(x: torch.Tensor, w_gu: torch.Tensor, b_gu: torch.Tensor | None = N
         return (torch.nn.functional.silu(g) * u).to(x.dtype)
     if N2 % 64:
         raise ValueError("gemm_silu: 2I must be a multiple of 64")
-    ksplit, sk = schedule(M, N2, K, True) if ksplit is None else (ksplit, sk or 0)
+    if ksplit is None:
+        shape = pair_plan(M, N2, K, True)
+        if shape is not None and pair_takes(x, w_gu, b_gu, out):
+            return gemm_pair(x, w_gu, b_gu, shape, EPI_SILU, ACT_NONE, out)
+        ksplit, sk = schedule(M, N2, K, True)
+    sk = sk or 0
     if out is None:
         out = torch.empty(M, N2 // 2, dtype=x.dtype, device=x.device)
     return _launch(x, w_gu, b_gu, out, EPI_SILU, ACT_NONE, ksplit, sk)
@@ -453,9 +535,13 @@ def gemm_glu(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: float
     """h [M, F] = g sigmoid(alpha g) (u + shift), g = min(x wg^T, limit), u = clamp(x wu^T, +-limit), w [2F, K] = wg | wu."""
     M, K = x.shape
     F = w.shape[0] // 2
+    lim = math.inf if limit is None else limit
+    shape = pair_plan(M, 2 * F, K, True)
+    if shape is not None and pair_takes(x, w):
+        return gemm_pair(x, w, None, shape, EPI_GLU, glu=(lim, alpha, shift))
     out = torch.empty(M, F, dtype=x.dtype, device=x.device)
     call("grag_gemm_tile_glu", ptr(x), ptr(w), ptr(out), x.stride(0), w.stride(0), F, M, F, K,
-         float(math.inf if limit is None else limit), float(alpha), float(shift))
+         float(lim), float(alpha), float(shift))
     return out
 
 
@@ -837,8 +923,10 @@ def dec_capture_ok(dev: torch.device, M: int, N: int, K: int, silu: bool = False
     return fl == 0 or not torch.cuda.is_current_stream_capturing() or WS.ready(dev, fl)
 
 
-def capture_ok(dev: torch.device, M: int, N: int, K: int, silu: bool = False) -> bool:
+def capture_ok(dev: torch.device, M: int, N: int, K: int, silu: bool = False, act: int = ACT_NONE) -> bool:
     """False only inside a hipGraph capture whose split-K slab was not sized by an eager step."""
+    if pair_plan(M, N, K, silu or act != ACT_NONE) is not None:  # (no slab)
+        return True
     ks, sk = schedule(M, N, K, silu)
     fl = _ws_floats(M, N, ks, sk)
     return fl == 0 or not torch.cuda.is_current_stream_capturing() or (WS.ready(dev, fl) and (

@@ -285,13 +285,15 @@ def gemm_splitk(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None,
 
 
 def kernel_for(M: int, N: int, K: int, tile_ok: bool = True, dev: torch.device | None = None) -> str:
-    """The kernel linear() runs a bf16 [M, K] x [N, K]^T projection on: "decode" / "tile" / "tile_prefill"
+    """The kernel linear() runs a bf16 [M, K] x [N, K]^T projection on: "pair" / "decode" / "tile" / "tile_prefill"
     (owned MFMA kernels of ops/gemm.py), "skinny" / "stream" (owned weight-streaming kernels here),
     "splitk" (K-sliced library bmm) or "library" (hipBLASLt).  ``tile_ok``: the operands meet
     ops/gemm.supported (alignment, K % 64).  ``dev``: check that a hipGraph capture in progress can use
     the split-K / stream-K workspaces (None: plan as in steady state, workspaces ready)."""
     capturing = dev is not None and torch.cuda.is_current_stream_capturing()
     if tile_ok:
+        if _tile.pair_plan(M, N, K) is not None:
+            return "pair"
         if (TILE_MIN_M <= M or _tile.dec_small(M, N, K)) and _tile.dec_plan(M, N, K) is not None and (
                 dev is None or _tile.dec_capture_ok(dev, M, N, K)):
             return "decode"
@@ -314,12 +316,13 @@ def kernel_for(M: int, N: int, K: int, tile_ok: bool = True, dev: torch.device |
         return "skinny"
     if K % 16 == 0 and N % 4 == 0 and use_stream(M, N, K) and stream_ready:
         return "stream"
-    if tile_ok and _tile.unmeasured_plan(M, N, K) is not None and (dev is None or _tile.capture_ok(dev, M, N, K)):
+    if tile_ok and (_tile.wide_plan(M, N, K) is not None or _tile.unmeasured_plan(M, N, K) is not None and (
+            dev is None or _tile.capture_ok(dev, M, N, K))):
         return "tile_prefill"
     return "library"
 
 
-OWNED_KINDS = ("decode", "tile", "tile_prefill", "skinny", "stream")
+OWNED_KINDS = ("pair", "decode", "tile", "tile_prefill", "skinny", "stream")
 
 
 def _differentiated(*ts) -> bool:
@@ -358,6 +361,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> t
         M, K = x.shape
         N = w.shape[0]
         kind = kernel_for(M, N, K, _tile.supported(x, w), x.device)
+        if kind == "pair":
+            if _plain_product(x, w, b) and _tile.pair_takes(x, w, b):
+                return _tile.gemm_pair(x, w, b, _tile.pair_plan(M, N, K))
+            return torch.nn.functional.linear(x, w, b)
         if kind == "decode":
             return _tile.gemm_decode(x, w, b)
         if kind == "tile":
@@ -367,7 +374,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> t
             if p is not None:
                 return _tile.gemm(x, w, b, ksplit=p[0], sk=p[1])
             if _plain_product(x, w, b):
-                p = _tile.unmeasured_plan(M, N, K)
+                p = _tile.wide_plan(M, N, K) or _tile.unmeasured_plan(M, N, K)
+                if p == (1, 0) and _tile.pair_fills(M, N, K) and _tile.pair_takes(x, w, b):
+                    return _tile.gemm_pair(x, w, b, 0)
                 return _tile.gemm(x, w, b, ksplit=p[0], sk=p[1])
             return torch.nn.functional.linear(x, w, b)
         if kind == "splitk":
@@ -384,7 +393,8 @@ GLU_FILL = 0.55
 
 def glu_linear(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: float = 1.702, shift: float = 1.0) -> torch.Tensor:
     """clamped_glu(linear(x, w), limit, alpha, shift) for w [2F, K] (gate | up rows): at prefill sizes one launch, the unit in
-    the tile kernel's epilogue on the fp32 sums, where the product's useful tiles fill at least GLU_FILL of its rounds.
+    the kernel's epilogue on the fp32 sums, where the 256 x 256 tiles that are useful fill at least GLU_FILL of their rounds, or
+    where the small tiles take it (2048 x 1024 at 300 rows 12.0 -> 7.4 us, 12288 x 2048 34 -> 31).
 
     Back to back, library + unit / one launch, with 7 widths at 277-8192 rows: 18944 x 3584 8192 rows 1706 / 1581 us, 1187
     384 / 255; 8960 x 1536 8192 457 / 360, 1187 79 / 70; 1.03-1.5 above the line (median 1.19), 0.47-1.3 below it (a
@@ -393,7 +403,7 @@ def glu_linear(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: flo
     if x.is_cuda and x.dim() == 2 and x.shape[0] >= _tile.PREFILL_MIN_M and w.shape[0] % 16 == 0:
         M, N = x.shape[0], w.shape[0]
         tiles, ncu = -(-M // 256) * -(-N // 256), _tile._num_cus()
-        if M * N >= GLU_FILL * 65536 * ncu * -(-tiles // ncu) and _tile.supported(x, w) and _plain_product(x, w):
+        if (M * N >= GLU_FILL * 65536 * ncu * -(-tiles // ncu) or _tile.pair_plan(M, N, x.shape[1], True) is not None) and _tile.supported(x, w) and _plain_product(x, w):
             return _tile.gemm_glu(x, w, limit, alpha, shift)
     return clamped_glu(linear(x, w), limit, alpha, shift)
 

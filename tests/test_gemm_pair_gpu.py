@@ -1,0 +1,103 @@
+"""The small-tile GEMM (csrc/kernels/gemm_pair.hip): every tile shape and epilogue against the 256 x 256 tile's results, bit
+for bit, and the fp64 product within the rounding of the bf16 result; layouts; the products that linear() gives to it."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from githubrepostorag_amd.ops import gemm as G
+from githubrepostorag_amd.ops import linear as L
+
+# one row and column tile part, edges of 64 and 128 rows and of 64, 128 and 192 columns, one, two, three and many K steps
+SIZES = [(1, 8, 128), (64, 64, 128), (65, 72, 192), (127, 192, 256), (129, 200, 320), (300, 1000, 768), (257, 448, 64)]
+
+
+def _mk(dev, M, N, K):
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    r = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    return r(M, K).bfloat16(), (r(N, K) * K ** -0.5).bfloat16(), r(N).bfloat16()
+
+
+# half an ulp of bf16 (2^-9) of the value; fp32 sums of K terms of order 1 / sqrt(K) and the activation's rounding on top
+TOL = dict(rtol=2 ** -8, atol=2 ** -8 * 0.05)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", range(4))
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_epilogues(dev, M, N, K, shape):
+    x, w, b = _mk(dev, M, N, K)
+    for bias in (None, b):
+        ref = x.double() @ w.double().T + (0 if bias is None else bias.double())
+        for act, fn in ((G.ACT_NONE, lambda t: t), (G.ACT_GELU, F.gelu), (G.ACT_GELU_TANH, lambda t: F.gelu(t, approximate="tanh"))):
+            got = G.gemm_pair(x, w, bias, shape, act=act)
+            torch.testing.assert_close(got.double(), fn(ref), **TOL)
+            if K >= 128:
+                assert torch.equal(got, G.gemm(x, w, bias, act=act, ksplit=1, sk=0))
+        if N % 64 == 0:
+            got = G.gemm_pair(x, w, bias, shape, G.EPI_SILU)
+            gate, up = G.deinterleave_gate_up(ref.T.contiguous())
+            torch.testing.assert_close(got.double(), (F.silu(gate) * up).T, **TOL)
+            if K >= 128:
+                assert torch.equal(got, G.gemm_silu(x, w, bias, ksplit=1, sk=0))
+    if N % 16 == 0:
+        got = G.gemm_pair(x, w, None, shape, G.EPI_GLU, glu=(7.0, 1.702, 1.0))
+        gate, up = (x.double() @ w.double().T).chunk(2, 1)
+        gate = gate.clamp(max=7.0)
+        torch.testing.assert_close(got.double(), gate * torch.sigmoid(1.702 * gate) * (up.clamp(-7, 7) + 1), **TOL)
+
+
+@pytest.mark.gpu
+def test_layouts(dev):
+    """A column slice of a wider input, one row for all (stride 0), a result between other columns and rows."""
+    x, w, b = _mk(dev, 200, 328, 256)
+    wide = torch.randn(200, 512, device=dev).bfloat16()
+    want = G.gemm_pair(wide[:, 128:384].contiguous(), w, b, 3)
+    for shape in range(4):
+        assert torch.equal(G.gemm_pair(wide[:, 128:384], w, b, shape), want)
+        assert torch.equal(G.gemm_pair(x[:1].expand(200, 256), w, b, shape), G.gemm_pair(x[:1], w, b, shape).expand(200, 328))
+        big = torch.full((202, 352), 7.0, dtype=torch.bfloat16, device=dev)
+        G.gemm_pair(wide[:, 128:384], w, b, shape, out=big[1:201, 8:336])
+        assert torch.equal(big[1:201, 8:336], want)
+        big[1:201, 8:336] = 7.0
+        assert bool((big == 7.0).all())
+
+
+def test_rule(monkeypatch):
+    monkeypatch.setattr(G, "_NCU", [256])
+    assert [G.pair_plan(M, 768, 768) for M in (20, 33, 300, 2688, 2752)] == [None, 3, 3, 3, None]  # 504, 516 tiles
+    assert [G.pair_plan(M, 3072, 768, True) for M in (1, 300, 1136, 1752, 4200)] == [3, 3, 2, 1, None]
+    assert G.pair_plan(300, 3072, 1088) is None and G.pair_plan(300, 22016, 4096, True) is None  # deep
+    assert G.pair_fills(24000, 768, 768) and not G.pair_fills(12000, 2304, 768) and not G.pair_fills(21504, 768, 768)
+    # rows, width, depth, library and owned us
+    for M, N, K, lib, own in [(2405, 18944, 3584, 360, 232), (4000, 18944, 3584, 500, 385), (1641, 18944, 3584, 195, 212),
+                              (1187, 8192, 1536, 32, 34), (1641, 8192, 1536, 41, 38), (2405, 8192, 1536, 60, 68)]:
+        assert (G.wide_plan(M, N, K) is not None) == (own < lib), (M, N, K)
+    assert G.wide_plan(4000, 3584, 3584) is None  # a measured shape keeps its rows
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(40, 768, 768), (300, 2304, 768), (700, 18944, 1536), (8000, 2304, 768)])
+def test_linear(dev, M, N, K):
+    """Plain products that linear() runs here, with a gradient on the library's."""
+    x, w, b = _mk(dev, M, N, K)
+    ref = x.double() @ w.double().T + b.double()
+    torch.testing.assert_close(L.linear(x, w, b).double(), ref, **TOL)
+    w.requires_grad_(True)
+    y = L.linear(x, w, b)
+    y.sum().backward()
+    assert w.grad is not None and w.grad.shape == w.shape
+
+
+@pytest.mark.gpu
+def test_captured_without_an_eager_step(dev):
+    """A product that has no slab can be captured before any eager one."""
+    x, w, b = _mk(dev, 100, 3072, 768)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    assert G.capture_ok(x.device, 100, 3072, 768, act=G.ACT_GELU)
+    with G.WS.owned_by({}), torch.cuda.graph(g):
+        y = G.gemm(x, w, b, act=G.ACT_GELU)
+    for _ in range(3):
+        x.normal_()
+        g.replay()
+        assert torch.equal(y, G.gemm(x, w, b, act=G.ACT_GELU))
