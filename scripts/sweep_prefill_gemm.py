@@ -10,8 +10,8 @@ stream-K), check each owned arm against the library output, and record the
 fastest arm per M.  Writes githubrepostorag_amd/tuning/gemm_prefill_gfx950.json,
 which ops/linear.py (plain projections) and ops/gemm.py (fused SwiGLU) read.
 
-Both arms run interleaved in one process on the same random operands
-(cdna guide §5.4 rules 24/25); medians of CUDA-event timings.
+Every arm is captured in a graph, one launch for each of a set of weight copies that
+no cache holds; medians of the graph's replays.
 
 usage: python scripts/sweep_prefill_gemm.py [--models qwen2-7b,bge-large] [--mmin 384 --mmax 16384 --mstep 256]
 """
@@ -62,16 +62,25 @@ for _m, _tp in (("qwen2-72b", 8), ("qwen2-7b", 2), ("qwen2-7b", 4)):
     SHAPES[f"{_m}-tp{_tp}"] = _tp_shapes(_m, _tp)
 
 
-def med_us(fn, reps):
+def graph_us(fn, n, reps, owner):
+    """Median time of fn() captured n times in a graph: no launch from Python in it.  fn takes another copy of the weight each
+    time, together more than the caches hold."""
+    with G.WS.owned_by(owner):
+        fn()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            for _ in range(n):
+                fn()
     ts = []
-    for _ in range(reps):
+    for _ in range(reps + 1):
         s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         s.record()
-        fn()
+        g.replay()
         e.record()
         e.synchronize()
-        ts.append(s.elapsed_time(e) * 1e3)
-    return statistics.median(ts)
+        ts.append(s.elapsed_time(e) * 1e3 / n)
+    return statistics.median(ts[1:])
 
 
 def own_arms(M, N, K):
@@ -167,20 +176,17 @@ def main():
             if args.labels and label not in args.labels.split(","):
                 continue
             key = f"{N},{K},{int(silu)}"
-            ws = [((torch.rand(N, K, device=dev) * 2 - 1) * 0.05).to(torch.bfloat16) for _ in range(2)]
+            copies = max(3, min(24, int(600e6 / (2 * N * K))))
+            ws = [((torch.rand(N, K, device=dev) * 2 - 1) * 0.05).to(torch.bfloat16) for _ in range(copies)]
             xfull = (torch.rand(args.mmax, K, device=dev) * 2 - 1).to(torch.bfloat16)
             rows, trow = [], []
             for M in range(args.mmin, args.mmax + 1, args.mstep):
                 x = xfull[:M]
                 arms = own_arms(M, N, K)
-                for ks, sk in arms:
-                    G.WS.reserve(dev, G._ws_floats(M, N, ks, sk))
-                    if sk:
-                        G.WS.counters(dev)
                 it = {"i": 0}
 
                 def lib():
-                    w = ws[it["i"] & 1]
+                    w = ws[it["i"] % copies]
                     it["i"] += 1
                     y = torch.nn.functional.linear(x, w)
                     if silu:
@@ -190,7 +196,7 @@ def main():
 
                 def own(ks, sk):
                     def f():
-                        w = ws[it["i"] & 1]
+                        w = ws[it["i"] % copies]
                         it["i"] += 1
                         return G.gemm_silu(x, w, ksplit=ks, sk=sk) if silu else G.gemm(x, w, ksplit=ks, sk=sk)
                     return f
@@ -205,14 +211,11 @@ def main():
                     y = own(*a)().float()
                     ok[a] = ((y - ref).abs().max().item() / scale) < 2e-2
                 fns = {"lib": lib, **{a: own(*a) for a in arms if ok[a]}}
-                for f in fns.values():  # warm
-                    f()
-                torch.cuda.synchronize()
-                t = {k: [] for k in fns}
-                for _ in range(args.reps):  # interleaved rounds
-                    for k, f in fns.items():
-                        t[k].append(med_us(f, 1))
-                med = {k: statistics.median(v) for k, v in t.items()}
+                owner = {}
+                with G.WS.owned_by(owner):  # slab and tickets of every arm before any capture
+                    G.WS.reserve(dev, max(1, *(G._ws_floats(M, N, *a) for a in arms)))
+                    G.WS.counters(dev)
+                med = {k: graph_us(f, copies, args.reps, owner) for k, f in fns.items()}
                 best = min(med, key=med.get)
                 choice = ["lib", 1, 0] if best == "lib" else ["own", best[0], best[1]]
                 rows.append(table_row(M, med))
