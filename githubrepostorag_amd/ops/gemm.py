@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import bisect
 import contextlib
+import functools
 import json
 import math
 import os
@@ -254,6 +255,7 @@ def _pair_tiles(shape: int, M: int, N: int) -> int:
     return -(-M // bm) * -(-N // bn)
 
 
+@functools.lru_cache(4096)
 def pair_plan(M: int, N: int, K: int, fused: bool = False) -> int | None:
     """The small-tile kernel's shape for a product that gives the 256 x 256 tile too few tiles, or None.  ``fused``: with an
     activation or a gated unit in the epilogue (no library call does that in one launch), else plain.
@@ -274,6 +276,7 @@ def pair_plan(M: int, N: int, K: int, fused: bool = False) -> int | None:
     return next((s for s in (2, 1) if _pair_tiles(s, M, N) <= 2 * ncu), None)
 
 
+@functools.lru_cache(4096)
 def pair_fills(M: int, N: int, K: int) -> bool:
     """Whether short contractions whose 256 x 256 tiles would leave their last round of CUs nearly empty go in 128 x 192 ones:
     24000 x 768 x 768 (282 tiles) 40 -> 34.5 us, 8000 x 2304 x 768 (288) 38 -> 34; fuller ones not (12000 x 2304 x 768, 0.82 of
@@ -283,8 +286,8 @@ def pair_fills(M: int, N: int, K: int) -> bool:
 
 
 def pair_takes(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None, out: torch.Tensor | None = None) -> bool:
-    """Operands of ``supported`` that the small-tile kernel takes too: byte offsets of 31 bits, aligned bias and result."""
-    return (x.stride(0) * x.shape[0] < 1 << 30 and w.stride(0) * w.shape[0] < 1 << 30
+    """Whether the small-tile kernel takes operands of its types: byte offsets of 31 bits, aligned operands and result."""
+    return ((x.data_ptr() | w.data_ptr()) % 16 == 0 and x.stride(0) * x.shape[0] < 1 << 30 and w.stride(0) * w.shape[0] < 1 << 30
             and (b is None or (b.dtype == torch.bfloat16 and b.is_contiguous() and b.data_ptr() % 8 == 0))
             and (out is None or (out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 8 == 0
                                  and out.data_ptr() % 16 == 0)))
@@ -303,6 +306,7 @@ def gemm_pair(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, shape: i
     return out
 
 
+@functools.lru_cache(4096)
 def wide_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
     """(1, 0) where a plain product of K >= 1152 outside the measured table goes to the owned kernel in whole tiles: where they
     fill 0.65 of their rounds of CUs.  228 points of 19 widths and depths (1536 - 28672 x 1536 - 13824) at 400 - 8192 rows, one

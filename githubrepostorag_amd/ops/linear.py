@@ -37,8 +37,8 @@ from torch.autograd import forward_ad as fwAD
 from torch.overrides import has_torch_function
 
 from . import gemm as _tile
-from ._lib import call, lib, ptr
-from .elementwise import clamped_glu
+from ._lib import call, check, lib, ptr
+from .elementwise import bias_act, clamped_glu
 
 TUNING_DIR = Path(__file__).resolve().parents[1] / "tuning"
 _TUNED = {"done": False, "table": None}
@@ -386,6 +386,51 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> t
         if kind == "stream":
             return gemm_stream(x, w, b)
     return torch.nn.functional.linear(x, w, b)
+
+
+def bound_product(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, act: int = 0):
+    """linear(x, w, b) (or its product with an activation, ops/gemm.py) for a run of weights of w's shape, its kernel chosen once:
+    f(x, w, b, out, stream) -> result, in ``out`` [M, N] where an owned kernel writes it.  What has no such form, and a weight or
+    bias that is not laid out like w and b, goes the ordinary way.  A call from Python costs 4 us in place of 15 - 20."""
+    M, K = x.shape
+    N = w.shape[0]
+
+    def ordinary(x, w, b):
+        if not act:
+            return linear(x, w, b)
+        if _tile.supported(x, w) and _tile.capture_ok(x.device, M, N, K, act=act):
+            return _tile.gemm(x, w, b, act=act)
+        return bias_act(linear(x, w), b, act, inplace=True)
+
+    name, tail = None, ()
+    if x.is_cuda and _tile.supported(x, w) and _plain_product(x, w, b):
+        shape = _tile.pair_plan(M, N, K, act != 0)
+        kind = "tile_prefill" if act else kernel_for(M, N, K, True, x.device)
+        if shape is None and kind == "tile_prefill":
+            plan = _tile.schedule(M, N, K) if act else _tile.prefill_plan(M, N, K) or _tile.wide_plan(M, N, K) or _tile.unmeasured_plan(
+                M, N, K)
+            if plan == (1, 0):
+                measured = not act and _tile.prefill_plan(M, N, K) is not None
+                shape = 0 if not measured and _tile.pair_fills(M, N, K) else None
+                if shape is None:
+                    name, tail = "grag_gemm_tile", (_tile.EPI_STORE, act, 1, 0, None, None)
+        if shape is not None and (act or kind == "pair" or kind == "tile_prefill"):
+            name, tail = "grag_gemm_pair", (_tile.EPI_STORE, act, shape, 0.0, 0.0, 0.0)
+        elif name is None and kind == "library":
+            return lambda x, w, b, out, stream: torch.nn.functional.linear(x, w, b)
+    if name is None or not _tile.pair_takes(x, w, b):
+        return lambda x, w, b, out, stream: ordinary(x, w, b)
+    fn, wshape, dev = getattr(lib(), name), w.shape, w.device
+
+    def run(x, w, b, out, stream):
+        wp, bp = w.data_ptr(), 0 if b is None else b.data_ptr()
+        if (wp | bp) & 15 or w.shape != wshape or not w.is_contiguous() or w.dtype != torch.bfloat16 or w.device != dev or (
+                b is not None and (b.dtype != torch.bfloat16 or not b.is_contiguous())):
+            return ordinary(x, w, b)
+        check(fn(x.data_ptr(), wp, bp or None, out.data_ptr(), x.stride(0), K, N, M, N, K, *tail, stream), name)
+        return out
+
+    return run
 
 
 GLU_FILL = 0.55

@@ -9,6 +9,7 @@ state after its last token there.  Tokens are consumed in order, so a prompt may
 """
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -30,6 +31,7 @@ LINEAR_SCAN_MIN = 8  # tokens of the longest portion from which the matrix-core 
 LINEAR_SCAN_CHUNK = 64
 
 
+@functools.lru_cache(256)  # (a step's layers ask the same)
 def _scan_walks(max_q: int, tokens: int, nseq: int, tiles: float, split: bool) -> tuple[float, int]:
     """(walks, chunks a part) of the matrix-core scan (csrc/kernels/linscan.hip) for a step of ``nseq`` portions with
     ``tokens`` tokens, the longest ``max_q``, and ``tiles`` (head, 64 columns) tiles a portion: its length in walks of a
