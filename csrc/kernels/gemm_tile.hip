@@ -819,7 +819,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_chain_kernel(Args p) {
   };
   const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, p.a_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, p.w_bytes, 0x00020000);
-  tile256_chain<GATED ? 4 : 8>(smem, rsA, rsB, p.K >> 6, next, emit);
+  tile256_chain<GATED ? 4 : 8, false>(smem, rsA, rsB, p.K >> 6, next, emit, [](int) {}, [] { return 128; });
 }
 
 // Split-K combine: out = epilogue(sum_s ws[s]) — 8 output columns per thread.

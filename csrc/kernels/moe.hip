@@ -1051,6 +1051,136 @@ moe_gemm_tile_kernel(const bf16* __restrict__ a, int lda, int a_bytes, const bf1
   }
 }
 
+// 4 bytes a lane from rs + off to dst + 4 * lane (no template: the host's pass knows the builtin in none)
+__device__ __forceinline__ void moe_dma4(const __amdgpu_buffer_rsrc_t& rs, int* dst, unsigned off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (tile_lds_t*)dst, 4, off, 0, 0, 0);
+}
+
+// The same as chains of tiles, one workgroup a CU (tile256_chain): the next tile's source rows come to LDS while one is
+// multiplied, its first K steps behind this one's last, and the stores go out while the other waves multiply.  A workgroup a tile
+// waited for its expert's bounds, its rows, its first loads and, all CUs at once, for its stores: 4096 tokens x 4 of 16 experts,
+// width 3584, unit width 3776, routing and both products 1221 -> 1099 us (1.26 PFLOP/s in the products; the matrix cores and the
+// power they draw bound it).  K of at least 5 steps, all experts' weights and the result under 2 GB, 16-byte stores; other
+// products keep the workgroup a tile.
+template <int GATED>
+__global__ void __launch_bounds__(kTileThreads, 2)
+moe_gemm_chain_kernel(const bf16* __restrict__ a, int lda, int a_bytes, const bf16* __restrict__ w, int w_bytes,
+                      const int* __restrict__ offs, const int* __restrict__ order, int nrows, int E, int top, int N, int K,
+                      bf16* __restrict__ out, int ldo, int o_bytes, MoeEpi ep) {
+  constexpr int COLS = GATED == 1 ? 128 : 256;
+  // (one array: the compiler waits for every load in flight where a read of one array could meet a DMA into another)
+  __shared__ __attribute__((aligned(16))) char smem[2 * kTileBuf + 2 * 1024 + (RT_MAXR + 1) * 4];
+  int* srow = reinterpret_cast<int*>(smem + 2 * kTileBuf);  // [2][256] the entries of `order` of a tile's rows
+  int* so = srow + 512;
+  const int tid = threadIdx.x, L = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wid >> 2, wc = wid & 3;
+  for (int e = tid; e <= E; e += kTileThreads) so[e] = offs[e];
+  __syncthreads();
+  const int ncol = (N + COLS - 1) / COLS;
+  int nt = 0;
+  for (int e = 0; e < E; ++e) nt += (so[e + 1] - so[e] + 255) >> 8;
+  const int tiles = __builtin_amdgcn_readfirstlane(nt) * ncol;
+  // an XCD (blockIdx % 8) has a contiguous range of the tiles, its workgroups every step-th of that
+  const int x = blockIdx.x & 7, per = tiles >> 3, rest = tiles & 7, first = x * per + min(x, rest), last = first + per + (x < rest);
+  const int step = (gridDim.x - x + 7) >> 3, mine = first + (blockIdx.x >> 3);
+  if (mine >= last) return;
+  // tile t's expert, first row, rows and first column; from tile to tile t only rises
+  struct At { int e, base, r0, rows, n0; };
+  auto find = [&](int t, At p) __attribute__((always_inline)) {
+    int r, cnt;
+    for (;;) {
+      r = __builtin_amdgcn_readfirstlane(so[p.e]);
+      cnt = __builtin_amdgcn_readfirstlane(so[p.e + 1]) - r;
+      const int n = ((cnt + 255) >> 8) * ncol;
+      if (t < p.base + n) break;
+      p.base += n;
+      ++p.e;
+    }
+    const int in = t - p.base, m = (cnt + 255) >> 8;
+    p.r0 = r + in % m * 256;
+    p.rows = min(256, cnt - in % m * 256);
+    p.n0 = in / m * COLS;
+    return p;
+  };
+  const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc((void*)a, 0, a_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, w_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsC = __builtin_amdgcn_make_buffer_rsrc((void*)out, 0, o_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsO = __builtin_amdgcn_make_buffer_rsrc((void*)order, 0, nrows * 4, 0x00020000);
+  auto rows_to_lds = [&](int i, const At& p) __attribute__((always_inline)) {  // by waves 0 - 3, 64 rows each
+    if (wid < 4) moe_dma4(rsO, srow + (i & 1) * 256 + 64 * wid, (unsigned)(p.r0 + min(64 * wid + L, p.rows - 1)) * 4u);
+  };
+  At at = find(mine, At{0, 0, 0, 0, 0}), em = at, nx = at;  // of the loads issued last, of the results, of the rows brought last
+  rows_to_lds(0, at);
+  tile_wait_vm<0>();
+  __syncthreads();
+  auto ahead = [&](int i) __attribute__((always_inline)) {
+    if (mine + i * step >= last) return;
+    nx = find(mine + i * step, nx);
+    rows_to_lds(i, nx);
+  };
+  auto next = [&](int i, TileOff& o) __attribute__((always_inline)) {
+    if (mine + i * step >= last) {
+      o = TileOff(kTileNone);
+      return false;
+    }
+    at = nx;
+    const unsigned wbase = (unsigned)at.e * (unsigned)(GATED == 1 ? 2 * N : N);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int rs = tile_piece_row(r), c = tile_piece_chunk(r) * 8;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int lr = (rs >> 6) * 128 + q * 64 + (rs & 63);
+        const int src = GATED == 0 ? at.r0 + min(lr, at.rows - 1) : srow[(i & 1) * 256 + lr] / top;
+        const int gn = GATED == 1 ? q * N + min(at.n0 + (rs >> 5) * 32 + (rs & 31), N - 1)
+                                  : min(at.n0 + (rs >> 5) * 64 + q * 32 + (rs & 31), N - 1);
+        o[2 * q + r] = ((unsigned)src * (unsigned)lda + c) * 2u;
+        o[4 + 2 * q + r] = ((wbase + gn) * (unsigned)K + c) * 2u;
+      }
+    }
+    return true;
+  };
+  int ei = 0;  // the tile that is stored
+  auto emit = [&](int qm, const TileAcc& l, const TileAcc& r) __attribute__((always_inline)) {
+    const int wcol = ((L >> 4) & 1) * 16 + (L >> 5) * 8;
+    auto put = [&](int rs, int nb, auto&& val) __attribute__((always_inline)) {
+      uint32_t d[2][2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          d[i][h] = (uint32_t)(uint16_t)f2bits(val(rs, i, 2 * h)) | ((uint32_t)(uint16_t)f2bits(val(rs, i, 2 * h + 1)) << 16);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const auto s = __builtin_amdgcn_permlane16_swap(d[0][h], d[1][h], false, false);
+        d[0][h] = s[0];
+        d[1][h] = s[1];
+      }
+      const int lr = 128 * wr + 64 * qm + 16 * rs + (L & 15);
+      const unsigned row = (unsigned)(GATED == 0 ? srow[(ei & 1) * 256 + lr] : em.r0 + lr);
+      const unsigned off = lr < em.rows && nb + wcol < N ? (row * (unsigned)ldo + nb + wcol) * 2u : kTileNone;
+      typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
+      __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{d[0][0], d[0][1], d[1][0], d[1][1]}, rsC, off, 0, 0);
+    };
+#pragma unroll
+    for (int rs = 0; rs < 4; ++rs) {
+      if constexpr (GATED == 1) {
+        put(rs, em.n0 + wc * 32, [&](int s, int i, int c) { return glu_unit(l[s][i][c], r[s][i][c], ep); });
+      } else {
+#pragma unroll
+        for (int qn = 0; qn < 2; ++qn)
+          put(rs, em.n0 + wc * 64 + qn * 32, [&](int s, int i, int c) {
+            const float v = qn ? r[s][i][c] : l[s][i][c];
+            return GATED == 3 ? relu2_unit(v) : v;
+          });
+      }
+    }
+    if (qm == 1) em = at, ++ei;
+  };
+  tile256_chain<GATED == 1 ? 4 : 8, true>(smem, rsA, rsB, K >> 6, next, emit, ahead,
+                                          [&] { return __builtin_amdgcn_readfirstlane(at.rows - 128 * wr); });
+}
+
 // ------------------------------------------------------------------------------------------------ residual boundary
 // x [T][H] fp32, in place: x <- keep x + mult * sigmoid(gate + gbias) * (a + bcoef_t b + sum_k ecoef_(t,k) e_(t,k)), every
 // addend optional, the gate too (gate [T][gate_ld] logits in the activation type, gbias [H] fp32)
@@ -1466,6 +1596,19 @@ GRAG_API hipError_t grag_moe_table_route(const int* tok, const int* table, int n
   return hipGetLastError();
 }
 
+// compute units of the current device (cached per device; a host query, legal during graph capture)
+static int moe_cus() {
+  static int cus[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cus[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cus[dev] = n;
+  }
+  return cus[dev];
+}
+
 // rows = T * top sorted rows.  gated 1: a = h [T][lda], w = [E][2N][K], out [rows][N]; gated 0: a = [rows][lda] sorted,
 // w = [E][N][K], out [rows][ldo] in (token, choice) order; gated 3: as 1 with one branch, w = [E][N][K]; gated 2: one matrix per head (E heads, top = tokens, rows =
 // tokens * E): a = [tokens * E][lda], w = [E][N][K], out [tokens * E][ldo], offs / order unused.
@@ -1501,6 +1644,19 @@ GRAG_API hipError_t grag_moe_gemm(const void* a, int lda, const void* w, const i
       rows >= MOE_TILE_MIN * E && E <= RT_MAXR && a_bytes < (1L << 31) && w_bytes < (1L << 31)) {
     const long blocks = ((long)rows / 256 + E) * tcols;
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+    const long o_bytes = (long)rows * ldo * 2;
+    if (K >= 320 && w_bytes * E < (1L << 31) && o_bytes < (1L << 31) && N % 8 == 0 && ldo % 8 == 0 && al16(out) && rows < (1 << 28)) {
+      const int cus = moe_cus();
+#define MOE_CHAIN(G)                                                                                                     \
+  hipLaunchKernelGGL(moe_gemm_chain_kernel<G>, dim3((unsigned)(blocks < cus ? blocks : cus)), dim3(kTileThreads), 0, st, \
+                     (const bf16*)a, lda, (int)a_bytes, (const bf16*)w, (int)(w_bytes * E), offs, order, rows, E, top, N, K,     \
+                     (bf16*)out, ldo, (int)o_bytes, ep)
+      if (gated == 1) MOE_CHAIN(1);
+      else if (gated == 3) MOE_CHAIN(3);
+      else MOE_CHAIN(0);
+#undef MOE_CHAIN
+      return hipGetLastError();
+    }
 #define MOE_TILE(G)                                                                                                       \
   hipLaunchKernelGGL(moe_gemm_tile_kernel<G>, dim3((unsigned)blocks), dim3(kTileThreads), 0, st, (const bf16*)a, lda,     \
                      (int)a_bytes, (const bf16*)w, offs, order, E, top, N, K, (bf16*)out, ldo, ep)

@@ -171,12 +171,15 @@ __device__ __forceinline__ void tile256_loop(char* smem, const __amdgpu_buffer_r
 // behind a tile leave out the 2 * ST2 stores in between, so the stores have a K step's time.
 //   next(i, off): byte offsets of the workgroup's i-th tile at its first K step (kTileNone in all: there is none); whether it is
 //   emit(q, l, r): stores row quadrant q (columns of acc(q)0, acc(q)1) of the tile in exactly ST2 vector-memory instructions
+//   ahead(i): (nk >= 5) called in the second step of tile i - 1; what its vector-memory instructions bring to LDS is there for
+//   next(i)
+//   live(): rows of this wave's 128 that the tile of the last next has; quadrants without any are not multiplied (PARTIAL only)
 typedef unsigned TileOff __attribute__((ext_vector_type(8)));  // A [quadrant][piece], B the same (a vector: kept in registers)
 constexpr unsigned kTileNone = 0x80000000u;      // past the end of any operand (< 2 GB): loads zeros without a trip to memory
 
-template <int ST2, typename Next, typename Emit>
+template <int ST2, bool PARTIAL, typename Next, typename Emit, typename Ahead, typename Live>
 __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_rsrc_t& rsA, const __amdgpu_buffer_rsrc_t& rsB,
-                                              int nk, Next&& next, Emit&& emit) {
+                                              int nk, Next&& next, Emit&& emit, Ahead&& ahead, Live&& live) {
   const int L = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = w >> 2, wc = w & 3;
@@ -225,7 +228,7 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
   if (lag) tile_bar();
   tile_zero(acc00);
   tile_zero(acc01);
-  int buf = 0;
+  int buf = 0, rows = 128;
   bool more = true, behind = false;  // behind: a tile's stores lie between the loads
   auto step = [&](int i, int kt, auto first_c, auto last_c) __attribute__((always_inline)) {
     constexpr bool FIRST = decltype(first_c)::value, LAST = decltype(last_c)::value;
@@ -250,8 +253,10 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
     tile_wait_lds();
     tile_bar();
     // M1
-    tile_mma(acc00, a, b0);
-    tile_mma(acc01, a, b1);
+    if (!PARTIAL || rows > 0) {
+      tile_mma(acc00, a, b0);
+      tile_mma(acc01, a, b1);
+    }
     tile_bar();
     // L2
     if (!LAST && kt + 2 == nk) more = next(i + 1, cur);
@@ -277,15 +282,19 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
     tile_wait_lds();
     tile_bar();
     // M2
-    tile_mma(acc10, a, b0);
-    tile_mma(acc11, a, b1);
+    if (!PARTIAL || rows > 64) {
+      tile_mma(acc10, a, b0);
+      tile_mma(acc11, a, b1);
+    }
     tile_bar();
     buf ^= 1;
   };
   const std::integral_constant<bool, true> yes{};
   const std::integral_constant<bool, false> no{};
   for (int i = 0;; ++i) {
+    if (PARTIAL) rows = live();
     step(i, 0, yes, no);
+    ahead(i + 1);
     for (int kt = 1; kt + 1 < nk; ++kt) step(i, kt, no, no);
     step(i, nk - 1, no, yes);
     if (!more) break;
