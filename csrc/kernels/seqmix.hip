@@ -1744,8 +1744,8 @@ namespace grag {  // sink_prefill.hip
 bool sink_prefill_takes(int d, int vd, int v_ld, int BS, int max_q_len, int R, int bt_stride, int chunk, int window, int keep,
                         const void* q, const void* k, const void* v, const void* out, int out_ld);
 hipError_t sink_prefill_launch(const void* q, const void* k, const void* v, void* out, int out_ld, const int* bt, int bt_stride,
-                               const int* q_start, const int* ctx_len, const float* sinks, int nseq, int max_q_len, int H, int G,
-                               int d, float scale, float out_scale, int nblocks, const float* hscale, const void* hgate,
+                               const int* q_start, const int* ctx_len, const float* sinks, int nseq, int max_q_len, int rows, int H,
+                               int G, int d, float scale, float out_scale, int nblocks, const float* hscale, const void* hgate,
                                int gate_ld, int chunk, int window, float softcap, int keep, hipStream_t st);
 // sink_decode.hip
 bool sink_decode_takes(int d, int vd, int v_ld, int BS, int keep, const void* q, const void* k, const void* v, const void* out,
@@ -1770,10 +1770,10 @@ static int sa_key_tile(int d, int vd, size_t* bytes) {
 
 GRAG_API hipError_t grag_sink_attn_prefill(const void* q, const void* k_cache, const void* v_cache, void* out,
                                            int out_ld, const int* block_tables, int bt_stride, const int* q_start,
-                                           const int* ctx_len, const float* sinks, int nseq, int max_q_len, int H,
-                                           int G, int d, int vd, int BS, float scale, float out_scale, int nblocks,
-                                           int dt, int v_ld, const float* hscale, const void* hgate, int gate_ld,
-                                           int chunk, int window, float softcap, int keep, hipStream_t st) {
+                                           const int* ctx_len, const float* sinks, int nseq, int max_q_len, int rows,
+                                           int H, int G, int d, int vd, int BS, float scale, float out_scale, int nblocks,
+                                           int dt, int v_ld, const float* hscale, const void* hgate, int gate_ld, int chunk,
+                                           int window, float softcap, int keep, hipStream_t st) {
   const AttnExtra ex{hscale, hgate, gate_ld, chunk, window, softcap, chunk > 0 || window > 0 ? keep : 0};
   // v_ld: elements from one cached value row to the next (vd, or more when the value rows are the head of wider rows)
   if (nseq <= 0 || max_q_len <= 0) return hipSuccess;
@@ -1781,7 +1781,7 @@ GRAG_API hipError_t grag_sink_attn_prefill(const void* q, const void* k_cache, c
   if (dt == 0 && sink_prefill_takes(d, vd, v_ld, BS, max_q_len, H / G, bt_stride, chunk, window, ex.keep, q, k_cache, v_cache, out,
                                     out_ld))
     return sink_prefill_launch(q, k_cache, v_cache, out, out_ld, block_tables, bt_stride, q_start, ctx_len, sinks, nseq, max_q_len,
-                               H, G, d, scale, out_scale, nblocks, hscale, hgate, gate_ld, chunk, window, softcap, ex.keep, st);
+                               rows, H, G, d, scale, out_scale, nblocks, hscale, hgate, gate_ld, chunk, window, softcap, ex.keep, st);
   if (dt == 0 && v_ld % 8 == 0 && (reinterpret_cast<uintptr_t>(v_cache) & 15) == 0 && max_q_len >= 16 && d % 16 == 0 && vd % 16 == 0 && d <= 256 && vd <= 256 && out_ld % 4 == 0 &&
       (reinterpret_cast<uintptr_t>(out) & 7) == 0 && (reinterpret_cast<uintptr_t>(q) & 7) == 0) {
     const size_t mb = ((size_t)64 * (d + 8) + (size_t)16 * (vd * 4 + 8)) * sizeof(short);

@@ -13,7 +13,7 @@ struct SinkArgs {
   const int *bt, *q_start, *ctx_len;
   const float *sinks, *hscale;
   const bf16* hgate;
-  int out_ld, bt_stride, H, G, R, nblocks, tiles, gate_ld, chunk, window, keep;
+  int out_ld, bt_stride, H, G, R, nblocks, nseq, tiles, gate_ld, chunk, window, keep;
   float scale, out_scale, softcap;
 };
 
@@ -29,6 +29,15 @@ template <int D> __device__ __forceinline__ int sp_vswz(int row) { return D == 1
 __device__ __forceinline__ void sp_dma(const bf16* base, int bytes, int off, char* dst) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000), (sp_lds_t*)dst, 16,
                                            off, 0, 0, 0);
+}
+
+// The same from a wave-uniform base, with no bound, in a form whose wait the compiler leaves to the caller: it puts one for
+// everything in flight before each transposed read behind the builtin.
+__device__ __forceinline__ void sp_dma_s(const bf16* base, unsigned off, char* dst) {
+  const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(sp_lds_t*)dst);
+  unsigned keep;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+               : "=&s"(keep) : "v"(off), "s"(base), "s"(lds) : "memory");
 }
 
 // first key of the block / window of the query at `pos` (never falls as pos grows)

@@ -3,18 +3,19 @@
 // (grag_sink_attn_prefill says what each does).  Head size D = 64 or 128 for keys and values alike, 16-key cache blocks; other
 // sizes take the kernel of seqmix.hip.
 //
-// Rows are (position, query head) pairs of one kv head, R heads to a position: a workgroup is 8 waves of 16 rows, 128 rows on one
-// stream of K / V tiles (the other kernel reads every tile for 64 rows of one head).  Tiles of 64 keys arrive by LDS-DMA, the
-// next one in flight while one is computed.  Per tile
+// Rows are (position, query head) pairs of one kv head, R heads to a position: a workgroup is 4 waves of 32 rows, 128 rows on one
+// stream of K / V tiles (the other kernel reads every tile for 64 rows of one head), or of 16 rows where those are too few for the
+// chip.  Tiles of 64 keys arrive by LDS-DMA, K a tile further ahead than V, a piece at a time between the products.  Per tile
 //   S^T = K Q^T          bf16 products, exact in fp32,
 //   P = 2^(s - m)        fp32; m moves only when a row's scores pass it by 2^8 (its factor is exact then),
-//   O^T += V^T P^T       P as bf16 hi + lo, two products: 16 bits of the weights reach the accumulator.
-// What bounds it: matrix cores 36 % and vector instructions 46 % of all cycles at window 1024, 2 portions of 8192 tokens, 28 / 4
-// heads of 128 (the split is 1.5 times the products of a kernel with 16-bit weights).  Two workgroups share a CU, so that one's
-// softmax can meet the other's products.  Tried at that size, us: 128 rows x 2 208; one workgroup of 256 rows, 8 waves of 32
-// rows in step 221, half a tile apart 225, 16 waves 223; 128 rows by 4 waves of 32 rows 200, but 49 against 43 on a
-// prompt of 1187 tokens, 12 / 2 heads.  Measured, old -> new: window 345 -> 208 us, all keys 811 -> 479, blocks of 1024
-// 214 -> 141, 1 x 8192 tokens of all keys 1466 -> 714; 12 / 2 heads, 1 x 1187 tokens 75 -> 43.
+//   O^T += V^T P^T       P as bf16 hi + lo, two products: 16 bits of the weights reach the accumulator; the weights of the next
+//                        keys are formed between the products of these.
+// What bounds it: the split is 1.5 times the products of a kernel with 16-bit weights, and the chip's power, not its cycles.  At
+// window 1024, 2 portions of 8192 tokens, 28 / 4 heads of 128, waves of 16 rows, whose every tile waited for the DMA of the next
+// (the compiler's wait before the transposed reads), took 445 k cycles at 2.09 GHz; this takes 356 k at 1.95: matrix cores 45 %,
+// vector instructions 46 %, LDS 15 % of them.  The order of the walks, longest first over all portions and heads, is worth 5 to 9 %
+// (busy CUs 83 -> 93 % of the time).  Measured, us, before -> after: window 219 -> 200, capped 265 -> 239, blocks of 1024
+// 131 -> 121, all keys 7 x 8192 tokens 163 -> 148, 1 x 8192 710 -> 641, 3 x 2405 56 -> 50; 12 / 2 heads 1 x 1187 38 -> 35.
 #include "sink.h"
 
 GRAG_ERR_UNIT(sink_prefill)
@@ -24,17 +25,40 @@ namespace grag {
 constexpr int SP_KT = 64;         // keys per tile
 constexpr int SP_MAXB = 2048;     // cache blocks a workgroup can walk (32 K keys): its part of the block table, in LDS
 
-template <int D, bool CAP, int NW>
-__global__ void __launch_bounds__(64 * NW, 4) sink_prefill_kernel(const SinkArgs p) {
-  constexpr int RB = 2 * D, CPR = D / 8, NC = D / 32, ND = D / 16, TILE = SP_KT * RB;
-  constexpr int ROWS = 16 * NW, PPW = TILE / 1024 / NW, RPP = 1024 / RB;
-  static_assert(PPW >= 1 && SP_BS % (PPW * RPP) == 0, "a wave's DMA rows sit in one cache block");
-  __shared__ __attribute__((aligned(16))) char smem[2 * 2 * TILE];
-  __shared__ int bt_lds[SP_MAXB];
+// the larger of a lane's value and that of the lane 32 on, without LDS
+__device__ __forceinline__ float sp_max32(float v) {
+  const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(w[0]), __uint_as_float(w[1]));
+}
+
+// the swizzle of V's chunks: a transposed read takes 4 rows x 2 neighbouring units of 32 bytes at a time with 32-row waves
+template <int D, int MR> __device__ __forceinline__ int sp_pswz(int row) {
+  if constexpr (MR == 16) return sp_vswz<D>(row);
+  else return D == 128 ? (row & 3) << 2 : (row & 2) << 1;
+}
+
+// MR: rows a wave, the matrix instruction's width (16 x 16 x 32 or 32 x 32 x 16)
+template <int D, bool CAP, int MR>
+__global__ void __launch_bounds__(256, MR == 32 ? 2 : 4) sink_prefill_kernel(const SinkArgs p) {
+  constexpr int NW = 4, KD = 512 / MR, AR = MR * MR / 64;  // waves; a product's depth, its results a lane
+  constexpr int RB = 2 * D, CPR = D / 8, NC = D / KD, ND = D / MR, NT = SP_KT / MR, TILE = SP_KT * RB;
+  constexpr int ROWS = MR * NW, PPW = TILE / 1024 / NW, RPP = 1024 / RB;
+  typedef float acc_t __attribute__((ext_vector_type(AR)));
+  auto mma = [](bf16x8_t a, bf16x8_t b, acc_t c) {
+    if constexpr (MR == 16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+  };
+  static_assert(PPW * RPP == SP_BS, "a wave's DMA rows sit in one cache block");
+  // (one array: beside a second one the compiler waits for the DMA in flight before every tile's reads)
+  __shared__ __attribute__((aligned(16))) char smem[2 * 2 * TILE + 4 * SP_MAXB];
+  int* bt_lds = reinterpret_cast<int*>(smem + 2 * 2 * TILE);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int h4 = lane >> 4, li = lane & 15;
-  const int seq = blockIdx.x / p.tiles, kvh = blockIdx.y;
-  const int row_base = (p.tiles - 1 - (int)(blockIdx.x % p.tiles)) * ROWS;  // (the longest walks first)
+  const int hh = lane / MR, li = lane % MR;  // this lane's row is li; its keys (and head numbers) are 8 i + 4 hh + 0..3
+  // the walks of all portions and kv heads, longest first; turned by one from tile to tile, so that no XCD (the workgroups' number
+  // modulo 8) is left with the portions that have no such tile
+  const int streams = p.nseq * p.G, rank = blockIdx.x / streams, stream = (int)(blockIdx.x + rank) % streams;
+  const int seq = stream / p.G, kvh = stream % p.G;
+  const int row_base = (p.tiles - 1 - rank) * ROWS;
   const int q0 = p.q_start[seq], qlen = p.q_start[seq + 1] - q0, ctx = p.ctx_len[seq], pos0 = ctx - qlen;
   const int R = p.R, nrows = qlen * R;
   if (row_base >= nrows) return;
@@ -57,90 +81,116 @@ __global__ void __launch_bounds__(64 * NW, 4) sink_prefill_kernel(const SinkArgs
 
   // this lane's row
   const float LOG2E = 1.4426950408889634f;
-  const int row = row_base + wave * 16 + li;
+  const int row = row_base + wave * MR + li;
   const bool valid = row < nrows;
   const int pq = valid ? row / R : 0;
   const int head = kvh * R + (valid ? row - pq * R : 0), tok = q0 + pq;
   const int lim = valid ? min(kv_hi, pos0 + pq + 1) : 0, low = sp_first(p, pos0 + pq);
   const float sc = p.scale * (p.hscale ? p.hscale[head] : 1.f);
   const bool pre = p.hscale || !(p.scale > 0.f);  // scores scaled before the mask and the maximum, else in the exponent's fma
-  float m = p.sinks[head] * LOG2E, lsum = h4 == 0 ? 1.f : 0.f;  // the maximum starts at the sink, whose weight is 1 of the sum
+  float m = p.sinks[head] * LOG2E, lsum = hh == 0 ? 1.f : 0.f;  // the maximum starts at the sink, whose weight is 1 of the sum
   bf16x8_t qf[NC];
-  const bf16* qp = p.q + ((size_t)tok * p.H + head) * D + 8 * h4;
+  const bf16* qp = p.q + ((size_t)tok * p.H + head) * D + 8 * hh;
 #pragma unroll
   for (int c = 0; c < NC; ++c)
-    qf[c] = valid ? *reinterpret_cast<const bf16x8_t*>(qp + 32 * c) : bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+    qf[c] = valid ? *reinterpret_cast<const bf16x8_t*>(qp + KD * c) : bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
   // (a compiler-visible wait: the q loads retired, so that the loop needs no vmcnt of its own that would drain the DMA)
   __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();  // the table is there
   // of the wave's rows, the smallest and largest limit and first key
-  const int w0 = row_base + wave * 16, w1 = min(w0 + 16, nrows) - 1;
+  const int w0 = row_base + wave * MR, w1 = min(w0 + MR, nrows) - 1;
   const int p0 = pos0 + min(w0, nrows - 1) / R, p1 = pos0 + max(w1, 0) / R;
-  const int lim_min = w0 + 16 <= nrows ? min(kv_hi, p0 + 1) : 0, lim_max = w0 < nrows ? min(kv_hi, p1 + 1) : 0;
+  const int lim_min = w0 + MR <= nrows ? min(kv_hi, p0 + 1) : 0, lim_max = w0 < nrows ? min(kv_hi, p1 + 1) : 0;
   const int low_min = sp_first(p, p0), low_max = sp_first(p, p1);
 
-  const int lrow = lane / CPR, lch = lane % CPR;
-  const int wrow = wave * PPW * RPP, last_slot = (kv_hi - 1) % SP_BS;
-  auto issue = [&](int t, int stage) {
-    char* kdst = smem + stage * 2 * TILE;
-    const int blk = __builtin_amdgcn_readfirstlane(bt_lds[min(t * (SP_KT / SP_BS) + wrow / SP_BS, nb - 1)]);
-    const size_t base = ((size_t)blk * p.G + kvh) * SP_BS * D;
-    const int kt0 = start(t);
-#pragma unroll
-    for (int i = 0; i < PPW; ++i) {
-      const int piece = wave * PPW + i, kr = piece * RPP + lrow;
-      // keys past the last one re-read it (their weights are 0, and 0 times whatever lies there must be 0)
-      const int slot = kt0 + kr < kv_hi ? kr % SP_BS : last_slot;
-      sp_dma(p.k + base, SP_BS * RB, slot * RB + ((lch ^ sp_kswz<D>(kr)) << 4), kdst + piece * 1024);
-      sp_dma(p.v + base, SP_BS * RB, slot * RB + ((lch ^ sp_vswz<D>(kr)) << 4), kdst + TILE + piece * 1024);
-    }
+  // This wave's keys of a tile are one cache block: a wave-uniform base, a lane's offset behind it.  Keys past the last one re-read
+  // it (their weights are 0, and 0 times whatever lies there must be 0); tiles past the last one re-read that one, unused.
+  const int lrow = lane / CPR, lch = lane % CPR, last_slot = (kv_hi - 1) % SP_BS;
+  auto table = [&](int t) { return bt_lds[min(min(t, ntiles - 1) * (SP_KT / SP_BS) + wave, nb - 1)]; };
+  auto slots = [&](int t) {
+    const int left = kv_hi - 1 - start(min(t, ntiles - 1)) - wave * SP_BS;
+    return left < 0 ? last_slot : left;
   };
-  f32x4_t o[ND];
+  auto base = [&](int blk) { return ((size_t)blk * p.G + kvh) * SP_BS * D; };
+  auto dma_k = [&](int i, size_t at, int most, int t) {
+    const int r = i * RPP + lrow;
+    sp_dma_s(p.k + at, min(r, most) * RB + ((lch ^ sp_kswz<D>(r)) << 4), smem + (t & 1) * 2 * TILE + (wave * PPW + i) * 1024);
+  };
+  auto dma_v = [&](int i, size_t at, int most, int t) {
+    const int r = i * RPP + lrow;
+    sp_dma_s(p.v + at, min(r, most) * RB + ((lch ^ sp_pswz<D, MR>(r)) << 4), smem + (t & 1) * 2 * TILE + TILE + (wave * PPW + i) * 1024);
+  };
+  acc_t o[ND];
 #pragma unroll
-  for (int n = 0; n < ND; ++n) o[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  bf16x8_t ph[2], pl[2];  // the weights of 32 keys: a lane's row, keys 4 h4 + 0..3 and 16 + 4 h4 + 0..3
+  for (int n = 0; n < ND; ++n) o[n] = acc_t{};
+  constexpr int NP = SP_KT / KD;
+  acc_t s[NT];
+  bf16x8_t ph[2], pl[2], vf[2][ND];  // of KD keys: the weights of a lane's row, keys 4 hh + 0..3 and KD / 2 + 4 hh + 0..3; the values
 
+  const float f = CAP || pre ? 1.f : p.scale * LOG2E;
   auto scores = [&](int kt0, const char* k_lds) {
-    f32x4_t s[4];
+    bf16x8_t kf[NT][NC];
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-      const int kr = 16 * tt + li;
-      s[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
       for (int c = 0; c < NC; ++c)
-        s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            *reinterpret_cast<const bf16x8_t*>(k_lds + kr * RB + (((4 * c + h4) ^ sp_kswz<D>(kr)) << 4)), qf[c], s[tt], 0, 0, 0);
+        kf[tt][c] = *reinterpret_cast<const bf16x8_t*>(k_lds + (MR * tt + li) * RB + ((((KD / 8) * c + hh) ^ sp_kswz<D>(MR * tt + li)) << 4));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) {
+      s[tt] = acc_t{};
+#pragma unroll
+      for (int c = 0; c < NC; ++c) s[tt] = mma(kf[tt][c], qf[c], s[tt]);
     }
     if constexpr (CAP) {  // cap in the natural domain, then to log2
-      const float ic = 1.f / p.softcap, c2 = p.softcap * LOG2E;
+      // Below 1/4 by tanh's power series to x^9, whose next term is 1/10 of fp32's rounding there; a tile with a larger score by
+      // tanhf.
+      const float ic = 1.f / p.softcap, c2 = p.softcap * LOG2E, k = sc * ic;
+      float most = 0.f;
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt)
+      for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s[tt][r] = c2 * tanhf(s[tt][r] * sc * ic);
+        for (int r = 0; r < AR; ++r) most = fmaxf(most, fabsf(s[tt][r]));
+      if (__any(most * fabsf(k) >= 0.25f)) {
+        asm volatile("");
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+          for (int r = 0; r < AR; ++r) s[tt][r] = c2 * tanhf(s[tt][r] * k);
+      } else {
+#pragma unroll
+        for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+          for (int r = 0; r < AR; ++r) {
+            const float x = s[tt][r] * k, z = x * x, cx = c2 * x;
+            s[tt][r] = fmaf(cx, z * fmaf(fmaf(fmaf(62.f / 2835.f, z, -17.f / 315.f), z, 2.f / 15.f), z, -1.f / 3.f), cx);
+          }
+      }
     } else if (pre) {  // (a factor of 0 or less: it turns the order, and makes no 0 of a masked score)
       asm volatile("");
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt) s[tt] *= sc * LOG2E;
+      for (int tt = 0; tt < NT; ++tt) s[tt] *= sc * LOG2E;
     }
     // a real branch (the empty asm): as selects, the masks would cost every tile what only the edges need
     if (kt0 + SP_KT > lim_min || (kt0 < low_max && kt0 + SP_KT > p.keep)) {
       asm volatile("");
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt)
+      for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = kt0 + 16 * tt + 4 * h4 + r;
+        for (int r = 0; r < AR; ++r) {
+          const int key = kt0 + MR * tt + 8 * (r >> 2) + 4 * hh + (r & 3);
           s[tt][r] = key < lim && (key >= low || key < p.keep) ? s[tt][r] : -INFINITY;
         }
     }
-    const float f = CAP || pre ? 1.f : p.scale * LOG2E;
+  };
+  auto maximum = [&]() {
     float tmax = -INFINITY;
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt)
+    for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, s[tt][r]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+      for (int r = 0; r < AR; ++r) tmax = fmaxf(tmax, s[tt][r]);
+    if constexpr (MR == 16) tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+    tmax = sp_max32(tmax);
     const float cand = fmaxf(m, tmax * f);
     if (__any(cand > m + SP_RESCALE)) {  // every row takes its exact maximum, so o and lsum see one factor
       const float alpha = __builtin_amdgcn_exp2f(m - cand);
@@ -149,61 +199,109 @@ __global__ void __launch_bounds__(64 * NW, 4) sink_prefill_kernel(const SinkArgs
 #pragma unroll
       for (int n = 0; n < ND; ++n) o[n] *= alpha;
     }
+  };
+  auto weights = [&](int u) {
     float sum = 0.f;
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float x = __builtin_amdgcn_exp2f(fmaf(s[tt][r], f, -m));
-        const short hi = f2bits(x);
-        ph[tt >> 1][4 * (tt & 1) + r] = hi;
-        pl[tt >> 1][4 * (tt & 1) + r] = f2bits(x - bits2f(hi));
-        sum += x;
-      }
+    for (int i = 0; i < 8; ++i) {
+      const int e = 8 * u + i;
+      const float x = __builtin_amdgcn_exp2f(fmaf(s[e / AR][e % AR], f, -m));
+      const short hi = f2bits(x);
+      ph[u & 1][i] = hi;
+      pl[u & 1][i] = f2bits(x - bits2f(hi));
+      sum += x;
+    }
     lsum += sum;
   };
-  auto values = [&](const char* v_lds) {
-    const int tq = li >> 2, tp = li & 3;
+  auto load_v = [&](const char* v_lds, int u) {
+    const int tq = (lane & 15) >> 2, tp = lane & 3;
+    const int r0 = KD * u + 4 * hh + tq, r1 = r0 + KD / 2;
 #pragma unroll
-    for (int cc = 0; cc < 2; ++cc) {
-      const int r0 = 32 * cc + 4 * h4 + tq, r1 = r0 + 16;
-#pragma unroll
-      for (int n = 0; n < ND; ++n) {
-        const int unit = 4 * n + tp;
-        const bf16x4_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (sp_lds4_t*)(v_lds + r0 * RB + ((unit ^ (sp_vswz<D>(r0) << 1)) << 3)));
-        const bf16x4_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (sp_lds4_t*)(v_lds + r1 * RB + ((unit ^ (sp_vswz<D>(r1) << 1)) << 3)));
-        const bf16x8_t a = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
-        o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pl[cc], o[n], 0, 0, 0);
-        o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, ph[cc], o[n], 0, 0, 0);
-      }
+    for (int n = 0; n < ND; ++n) {
+      const int unit = (MR / 4) * n + (li >> 4) * 4 + tp;
+      const bf16x4_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (sp_lds4_t*)(v_lds + r0 * RB + ((unit ^ (sp_pswz<D, MR>(r0) << 1)) << 3)));
+      const bf16x4_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (sp_lds4_t*)(v_lds + r1 * RB + ((unit ^ (sp_pswz<D, MR>(r1) << 1)) << 3)));
+      vf[u & 1][n] = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
     }
   };
-  issue(0, 0);
+  // K of tile t + 1 and V of tile t are there after tile t's barrier, by which everyone has read K of tile t and V of tile t - 1:
+  // their buffers take K of tile t + 2 and V of tile t + 1, a piece at a time between the products (all at once, the waves of a
+  // CU wait for each other's)
+  size_t vat;
+  {
+    const int b0 = __builtin_amdgcn_readfirstlane(table(0)), b1 = __builtin_amdgcn_readfirstlane(table(1));
+#pragma unroll
+    for (int i = 0; i < PPW; ++i) dma_k(i, base(b0), slots(0), 0);
+#pragma unroll
+    for (int i = 0; i < PPW; ++i) dma_v(i, base(b0), slots(0), 0);
+    vat = base(b1);
+#pragma unroll
+    for (int i = 0; i < PPW; ++i) dma_k(i, vat, slots(1), 1);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PPW) : "memory");  // K of tile 0
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  }
   for (int t = 0; t < ntiles; ++t) {
-    // the wave's own pieces of tile t landed, its reads of tile t - 1 returned; the barrier: everyone's, and the buffer of tile
-    // t - 1 is free for the next issue
+    const int kt0 = start(t);
+    const char* k_lds = smem + (t & 1) * 2 * TILE;
+    const bool sees = kt0 < lim_max && (kt0 + SP_KT > low_min || kt0 < p.keep);  // a row of the wave, a key of the tile
+    const int nblk = table(t + 2);
+    if (sees) scores(kt0, k_lds);
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (t + 1 < ntiles) issue(t + 1, (t + 1) & 1);
-    const int kt0 = start(t);
-    if (kt0 >= lim_max || (kt0 + SP_KT <= low_min && kt0 >= p.keep)) continue;  // none of the wave's rows sees a key of it
-    const char* k_lds = smem + (t & 1) * 2 * TILE;
-    scores(kt0, k_lds);
-    values(k_lds + TILE);
+    const size_t kat = base(__builtin_amdgcn_readfirstlane(nblk));
+    const int kmost = slots(t + 2), vmost = slots(t + 1);
+    if (!sees) {
+#pragma unroll
+      for (int i = 0; i < PPW; ++i) dma_v(i, vat, vmost, t + 1), dma_k(i, kat, kmost, t);
+      vat = kat;
+      continue;
+    }
+    const char* v_lds = k_lds + TILE;
+    load_v(v_lds, 0);
+    maximum();
+    weights(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      if (u + 1 < NP) load_v(v_lds, u + 1);
+#pragma unroll
+      for (int n = 0; n < ND; ++n) {
+        o[n] = mma(vf[u & 1][n], pl[u & 1], o[n]);
+        o[n] = mma(vf[u & 1][n], ph[u & 1], o[n]);
+      }
+#pragma unroll
+      for (int i = u * PPW / NP; i < (u + 1) * PPW / NP; ++i) dma_v(i, vat, vmost, t + 1), dma_k(i, kat, kmost, t);
+      if (u + 1 < NP) {
+        weights(u + 1);
+#pragma unroll
+        for (int i = 0; i < 2 * ND; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, MR == 32 ? 5 : 2, 0);
+          if (MR == 32 || i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    vat = kat;
   }
-  lsum += __shfl_xor(lsum, 16, 64);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if constexpr (MR == 16) lsum += __shfl_xor(lsum, 16, 64);
   lsum += __shfl_xor(lsum, 32, 64);
   if (!valid) return;
   float r = p.out_scale / lsum;
   if (p.hgate) r /= 1.f + expf(-(float)p.hgate[(size_t)tok * p.gate_ld + head]);
-  bf16* op = p.out + (size_t)tok * p.out_ld + head * D + 4 * h4;
+  bf16* op = p.out + (size_t)tok * p.out_ld + head * D + 4 * hh;
 #pragma unroll
   for (int n = 0; n < ND; ++n)
-    *reinterpret_cast<bf16x4_t*>(op + 16 * n) =
-        bf16x4_t{f2bits(o[n][0] * r), f2bits(o[n][1] * r), f2bits(o[n][2] * r), f2bits(o[n][3] * r)};
+#pragma unroll
+    for (int i = 0; i < AR / 4; ++i)
+      *reinterpret_cast<bf16x4_t*>(op + MR * n + 8 * i) = bf16x4_t{f2bits(o[n][4 * i] * r), f2bits(o[n][4 * i + 1] * r),
+                                                                   f2bits(o[n][4 * i + 2] * r), f2bits(o[n][4 * i + 3] * r)};
 }
 
 // Whether the kernel takes a call; grag_sink_attn_prefill (seqmix.hip) asks before it launches.
@@ -220,8 +318,8 @@ bool sink_prefill_takes(int d, int vd, int v_ld, int BS, int max_q_len, int R, i
 }
 
 hipError_t sink_prefill_launch(const void* q, const void* k, const void* v, void* out, int out_ld, const int* bt, int bt_stride,
-                               const int* q_start, const int* ctx_len, const float* sinks, int nseq, int max_q_len, int H, int G,
-                               int d, float scale, float out_scale, int nblocks, const float* hscale, const void* hgate,
+                               const int* q_start, const int* ctx_len, const float* sinks, int nseq, int max_q_len, int rows, int H,
+                               int G, int d, float scale, float out_scale, int nblocks, const float* hscale, const void* hgate,
                                int gate_ld, int chunk, int window, float softcap, int keep, hipStream_t st) {
   SinkArgs a{};
   a.q = (const bf16*)q, a.k = (const bf16*)k, a.v = (const bf16*)v, a.out = (bf16*)out;
@@ -229,19 +327,21 @@ hipError_t sink_prefill_launch(const void* q, const void* k, const void* v, void
   a.out_ld = out_ld, a.bt_stride = bt_stride, a.H = H, a.G = G, a.R = H / G, a.nblocks = nblocks;
   a.gate_ld = gate_ld, a.chunk = chunk, a.window = window, a.keep = keep;
   a.scale = scale, a.out_scale = out_scale, a.softcap = softcap;
-  // 128 rows a workgroup, or 64 where those are few for the chip: a walk's time is the chain of its tiles, shorter with one wave a
-  // SIMD than with two.  us of 128 / 64 rows, all keys: 12 / 2 heads, 300 tokens 15 / 13, 1187 (112 workgroups) 43 / 37, 2048
-  // (192) 67 / 55; 28 / 4 heads, 1500 (332) 63 / 53; past the line 12 x 300 (360) 22 / 24, 28 / 4 heads, 2048 (448) 76 / 90.
+  // 128 rows a workgroup, or 64 in waves of 16 where those of all `rows` queries are few for the chip: a walk's time is the chain of
+  // its tiles, shorter with 16 rows a wave.  us of 128 / 64 rows, all keys, tokens by portions (128-row workgroups): 12 / 2 heads,
+  // 600 x 1 (57) 24.4 / 19.3, 1187 x 1 (112) 45.7 / 35.1, 2048 x 4 (192) 38.7 / 30.8, 3600 x 12 (338) 31.4 / 25.0, 8192 x 4 (768)
+  // 110 / 136; 28 / 4 heads, 1500 x 1 (329) 56.2 / 46.9, 2048 x 1 (448) 65.3 / 72.0, 2048 x 4 (448) 42.3 / 36.5, 3000 x 8 (657)
+  // 35.1 / 45.6; window 1024, 12 / 2 heads, 4000 x 2 (375) 54.0 / 64.1.
   long tiles = ((long)max_q_len * a.R + 127) / 128;
-  const bool few = tiles * nseq * G <= 340;
+  const bool few = ((long)rows * a.R + 127) / 128 * G <= 340;
   if (few) tiles = ((long)max_q_len * a.R + 63) / 64;
-  if (tiles * nseq > 0x7fffffffL || G > 65535) return hipErrorInvalidValue;
-  a.tiles = (int)tiles;
-  const dim3 grid((unsigned)(tiles * nseq), G);
+  if (tiles * nseq * G > 0x7fffffffL - (tiles > 0 ? tiles : 0)) return hipErrorInvalidValue;
+  a.tiles = (int)tiles, a.nseq = nseq;
+  const dim3 grid((unsigned)(tiles * nseq * G));
 #define SINK_PREFILL(DD, CAP)                                                                                        \
   {                                                                                                                  \
-    if (few) hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 4>), grid, dim3(256), 0, st, a);                       \
-    else hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 8>), grid, dim3(512), 0, st, a);                           \
+    if (few) hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 16>), grid, dim3(256), 0, st, a);                      \
+    else hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 32>), grid, dim3(256), 0, st, a);                          \
   }
   if (d == 64 && softcap > 0.f) SINK_PREFILL(64, true)
   else if (d == 64) SINK_PREFILL(64, false)

@@ -541,7 +541,7 @@ def sink_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
     else:
         call("grag_sink_attn_prefill", ptr(q), ptr(k_cache), ptr(v_cache), ptr(out), out.stride(0),
              ptr(meta.block_tables), meta.block_tables.stride(0), ptr(meta.q_start), ptr(meta.ctx_len), ptr(sinks),
-             meta.num_seqs, meta.max_q_len, H, G, d, vd, BS, float(scale), float(out_scale), k_cache.shape[0], dt, v_ld,
+             meta.num_seqs, meta.max_q_len, T, H, G, d, vd, BS, float(scale), float(out_scale), k_cache.shape[0], dt, v_ld,
              *extra)
     return out
 
