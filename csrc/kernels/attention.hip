@@ -382,7 +382,8 @@ __global__ __launch_bounds__(64 * NW, D <= 64 && NW == 4 ? 4 : 1) void attn_fwd_
 // The 4-wave kernel above stages 64 GQA rows per 32 KiB K/V tile through
 // registers, so every tile costs a full global->LDS round trip per 64 rows
 // and the load latency sits in front of the MFMAs.  Here a workgroup is 8
-// waves x RPW row groups of 16 = 256 rows (36 positions x 7 heads at GQA 7):
+// waves x RPW row groups of 16 = 256 rows (36 positions x 7 heads at GQA 7; fewer rows or waves where
+// those leave the chip idle, launch_prefill):
 //   * K and V tiles arrive by global_load_lds_dwordx4 (1 KiB per wave
 //     instruction, lane-linear LDS destination, XOR swizzle applied to the
 //     per-lane SOURCE chunk — rule 21), tile t+1 issued right after the
@@ -426,10 +427,13 @@ __global__ __launch_bounds__(64 * NW) void attn_prefill_kernel(AttnParams p) {
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int h4 = lane >> 4, li = lane & 15;
-  const int tiles = p.tiles_per_seq;
-  const int seq = blockIdx.x / tiles;
-  const int tile = tiles - 1 - (int)(blockIdx.x % tiles);
-  const int kvh = blockIdx.y;
+  // the tiles of all sequences and kv heads, longest walks first; turned by one from tile to tile, so that no XCD (the workgroups'
+  // number modulo 8) is left with the sequences that have no such tile: 7 sequences of 8192 tokens, 28 / 4 heads, 153 -> 140 us
+  // (sequence by sequence, the last one's long walks ran alone)
+  const int tiles = p.tiles_per_seq, streams = gridDim.x / tiles * gridDim.y;
+  const unsigned id = blockIdx.x + gridDim.x * blockIdx.y, rank = id / streams, stream = (id + rank) % streams;
+  const int seq = stream / gridDim.y, kvh = stream % gridDim.y;
+  const int tile = tiles - 1 - (int)rank;
   const int q0 = p.q_start[seq], qlen = p.q_start[seq + 1] - q0;
   const int ctx = p.ctx_len[seq];
   const int G = p.G;
@@ -1658,18 +1662,32 @@ int launch_decode_prefix(const AttnParams& prm, int n_items, int rg, hipStream_t
   return (int)hipGetLastError();
 }
 
-template <int D>
-int launch_prefill(const AttnParams& prm, int nseq, int nw, hipStream_t stream) {
-  dim3 grid(nseq * prm.tiles_per_seq, prm.Hkv, 1);
-  if (nw == 6)
-    attn_prefill_kernel<D, 2, 3><<<grid, 512, 0, stream>>>(prm);
-  else
-    attn_prefill_kernel<D, 2, 2><<<grid, 512, 0, stream>>>(prm);
+template <int D, int RPW, int NS, int NW>
+int launch_prefill_rows(const AttnParams& prm_in, int nseq, int max_q_len, hipStream_t stream) {
+  constexpr int ROWS = 16 * RPW * NW;
+  AttnParams prm = prm_in;
+  prm.tiles_per_seq = (max_q_len * prm.G + ROWS - 1) / ROWS;
+  attn_prefill_kernel<D, RPW, NS, NW><<<dim3(nseq * prm.tiles_per_seq, prm.Hkv), 64 * NW, 0, stream>>>(prm);
   return (int)hipGetLastError();
 }
 
+// Rows a workgroup by the 256-row workgroups that all rows make: a walk's time is the chain of its tiles, shorter with 16 rows a wave
+// than with 32, and few walks leave the chip idle, many are paid by the reads a row.  us of 256 rows (8 waves of 32) / 128 (8 of
+// 16) / 64 (4 of 16), tokens by sequences: 12 / 2 heads, 300 x 1 (16 workgroups) 18.3 / 12.8 / 13.7, 1187 x 1 (56) 43.3 / 29.9 /
+// 28.8, 3600 x 12 (170) 29.5 / 22.5 / 22.1, 8192 x 4 (384) 96.8 / 117 / 121; 28 / 4 heads, 600 x 1 (68) 27.6 / 18.8 / 17.6,
+// 1500 x 1 (168) 54.8 / 39.5 / 38.1, 2048 x 1 (224) 70.2 / 52.5 / 57.8, 2048 x 4 (224) 38.6 / 31.8 / 30.4, 3000 x 1 (332) 99.4 /
+// 106 / 106, 3000 x 8 (332) 37.4 / 41.4 / 39.7, 8192 x 7 (896) 129 / 159 / 162.
 template <int D>
-int dispatch_nw(const AttnParams& prm, int nseq, int nw, bool paged, hipStream_t stream) {
+int launch_prefill(const AttnParams& prm, int nseq, int max_q_len, int nw, hipStream_t stream) {
+  if (nw == 6) return launch_prefill_rows<D, 2, 3, 8>(prm, nseq, max_q_len, stream);
+  const long wgs = ((long)prm.total_q * prm.G + 255) / 256 * prm.Hkv;
+  if (wgs <= 200) return launch_prefill_rows<D, 1, 2, 4>(prm, nseq, max_q_len, stream);
+  if (wgs <= 280) return launch_prefill_rows<D, 1, 2, 8>(prm, nseq, max_q_len, stream);
+  return launch_prefill_rows<D, 2, 2, 8>(prm, nseq, max_q_len, stream);
+}
+
+template <int D>
+int dispatch_nw(const AttnParams& prm, int nseq, int max_q_len, int nw, bool paged, hipStream_t stream) {
   // nw == 1 / 3 with q_len == 1: LDS-DMA pipelined decode kernel with 64- / 32-key
   // tiles (32-key tiles halve the LDS ring so more single-wave workgroups share a
   // CU); nw == 2: the generic kernel with one wave per workgroup (A/B reference)
@@ -1681,7 +1699,7 @@ int dispatch_nw(const AttnParams& prm, int nseq, int nw, bool paged, hipStream_t
   if (nw == 5 || nw == 6) {  // LDS-DMA prefill: 8 waves, 2-stage (5) / staggered 3-stage (6) ring
     if constexpr (D == 128 || D == 64) {
       if (paged && prm.num_splits == 1 && prm.BS == 16 && prm.bt_stride <= kPrefillMaxBlocks)
-        return launch_prefill<D>(prm, nseq, nw, stream);
+        return launch_prefill<D>(prm, nseq, max_q_len, nw, stream);
     }
     return (int)hipErrorInvalidValue;
   }
@@ -1743,9 +1761,9 @@ GRAG_API int grag_paged_attention(const void* q, int q_stride, const void* k_cac
   prm.causal = causal;
   prm.nblocks = nblocks;
   switch (D) {
-    case 128: return dispatch_nw<128>(prm, nseq, nw, true, stream);
-    case 64: return dispatch_nw<64>(prm, nseq, nw, true, stream);
-    case 32: return dispatch_nw<32>(prm, nseq, nw, true, stream);
+    case 128: return dispatch_nw<128>(prm, nseq, max_q_len, nw, true, stream);
+    case 64: return dispatch_nw<64>(prm, nseq, max_q_len, nw, true, stream);
+    case 32: return dispatch_nw<32>(prm, nseq, max_q_len, nw, true, stream);
     default: return (int)hipErrorInvalidValue;
   }
 }
@@ -1954,9 +1972,9 @@ GRAG_API int grag_varlen_attention(const void* q, const void* k, const void* v, 
   prm.scale_log2 = scale * 1.4426950408889634f;
   prm.causal = causal;
   switch (D) {
-    case 128: return dispatch_nw<128>(prm, nseq, 4, false, stream);
-    case 64: return dispatch_nw<64>(prm, nseq, 4, false, stream);
-    case 32: return dispatch_nw<32>(prm, nseq, 4, false, stream);
+    case 128: return dispatch_nw<128>(prm, nseq, max_len, 4, false, stream);
+    case 64: return dispatch_nw<64>(prm, nseq, max_len, 4, false, stream);
+    case 32: return dispatch_nw<32>(prm, nseq, max_len, 4, false, stream);
     default: return (int)hipErrorInvalidValue;
   }
 }

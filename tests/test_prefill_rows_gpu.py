@@ -1,0 +1,34 @@
+"""Paged prefill attention by rows a workgroup (csrc/kernels/attention.hip launch_prefill: 64, 128 or 256 by all rows) against
+fp32 attention: portions that end beside a workgroup's and a wave's rows, cached tokens before some, one of one token."""
+import pytest
+import torch
+
+from githubrepostorag_amd.ops.attention import AttnMetadata, paged_attention, paged_attention_ref
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,H,G,lens,past,wgs", [
+    (128, 28, 4, [37, 1, 300, 64], [0, 61, 0, 5], (1, 200)), (64, 12, 2, [129, 16, 640], [200, 0, 63], (1, 200)),
+    (128, 28, 4, [1000, 33, 1, 910], [0, 31, 64, 1], (201, 280)), (64, 32, 8, [511, 257, 1, 900], [0, 7, 900, 0], (201, 280)),
+    (128, 28, 4, [1500, 17, 1201], [5, 0, 63], (281, 400)), (64, 32, 8, [1025, 700, 640, 1], [0, 1, 0, 300], (281, 400))])
+def test_rows(dev, D, H, G, lens, past, wgs):
+    g = torch.Generator(device=dev).manual_seed(D + sum(lens))
+    BS, ctx, T = 16, [n + p for n, p in zip(lens, past)], sum(lens)
+    assert wgs[0] <= -(-T * (H // G) // 256) * G <= wgs[1]
+    width, nb = -(-max(ctx) // BS), sum(-(-c // BS) for c in ctx)
+    perm, bt, at = torch.randperm(nb, generator=torch.Generator().manual_seed(1)), torch.zeros(len(ctx), width, dtype=torch.int32), 0
+    for i, c in enumerate(ctx):
+        n = -(-c // BS)
+        bt[i, :n], at = perm[at:at + n].int(), at + n
+    r = lambda *s: torch.randn(*s, generator=g, device=dev).bfloat16()  # noqa: E731
+    q, kc, vc = r(T, H, D), r(nb, G, BS, D), r(nb, G, BS, D)
+    i32 = lambda v: torch.as_tensor(v, dtype=torch.int32, device=dev)  # noqa: E731
+    m = AttnMetadata(q_start=i32(torch.tensor([0] + lens).cumsum(0)), ctx_len=i32(ctx), block_tables=bt.to(dev), slot_mapping=None,
+                     max_q_len=max(lens), num_seqs=len(ctx), num_tokens=T)
+    got = paged_attention(q, kc, vc, m, D ** -0.5).view(T, H, D).float()
+    want = paged_attention_ref(q.float(), kc, vc, m, D ** -0.5)
+    size = paged_attention_ref(q.float(), kc, vc.abs(), m, D ** -0.5)
+    # the weights and the result are rounded to bf16's 8 bits: at most 2^-8 of each (2^-9 of the next power of two); 1.05 for fp32's
+    # sums and exponents
+    assert ((got - want).abs() <= 1.05 * 2 ** -8 * (want.abs() + size)).all(), ((got - want).abs() / size).max()
