@@ -138,19 +138,32 @@ __device__ __forceinline__ void glds16(const void* src, void* lds_dst) {
 
 // The same LDS-DMA with the address as a wave-uniform 64-bit base in SGPRs plus a 32-bit per-lane byte
 // offset (global_load_lds saddr form): no 64-bit VALU address arithmetic per load.
+template <bool NT = false>
 __device__ __forceinline__ void glds16_s(const void* sbase, uint32_t voff, void* lds_dst) {
   const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds_dst;
   const uint32_t lu = __builtin_amdgcn_readfirstlane(lds);
   uint32_t keep;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %3\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(keep)
-      : "v"(voff), "s"(sbase), "s"(lu)
-      : "memory");
+  if constexpr (NT) {
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2 nt\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(keep)
+        : "v"(voff), "s"(sbase), "s"(lu)
+        : "memory");
+  } else {
+    asm volatile(
+        "s_mov_b32 %0, m0\n\t"
+        "s_mov_b32 m0, %3\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2\n\t"
+        "s_mov_b32 m0, %0"
+        : "=&s"(keep)
+        : "v"(voff), "s"(sbase), "s"(lu)
+        : "memory");
+  }
 }
 
 template <int D, int NW, bool PAGED>
@@ -745,37 +758,212 @@ __device__ __forceinline__ void merge_prefix(const AttnParams& p, int tok, int h
   m = M;
 }
 
+// One wave's walk over TK-key tiles of a decode sequence: its ring of NS K and NS V buffers in LDS, filled by LDS-DMA.  A K buffer
+// is filled again as soon as its tile's keys are in registers, a V buffer as soon as the values are, so 2 NS - 1 of the 2 NS
+// buffers are in flight while the wave computes (tile by tile, 2 NS - 2).  Addresses are formed once per 16 keys, which lie in one
+// cache block: a wave-uniform base and an offset a lane that only the context's end changes (with a division a piece and lane the
+// addresses took longer than the products).  The block ids of a window of 64 blocks live one per lane; readlane hands them to the
+// scalar unit.
+template <int D, int TK, int NS, bool NT>
+struct DecodeWalk {
+  static constexpr int RB = 2 * D, CPR = D / 8, NC = D / 32, ND = D / 16, TILE = TK * RB, NI = TILE / 1024;
+  static constexpr int RPI = 1024 / RB, PG = 16 / RPI, NG = TK / 16, NT16 = TK / 16, NCC = TK / 32;
+  static_assert((2 * NS - 1) * NI <= 63, "vmcnt range");
+  const AttnParams& p;
+  const int32_t* bt;
+  char* ring;
+  int kvh, last, nblk, lane, win, bvec, shift;
+  size_t at[NG];  // of the tile whose keys were issued last: its groups' first element, its last valid row
+  int lim[NG];
+  float m = -INFINITY, lsum = 0.f;
+  f32x4_t o[ND];
+
+  // `last`: the last key that may be read
+  __device__ __forceinline__ DecodeWalk(const AttnParams& p_, int seq, int kvh_, int ctx, int last_, int first, char* ring_)
+      : p(p_), bt(p_.block_tables + (size_t)seq * p_.bt_stride), ring(ring_), kvh(kvh_), last(last_), lane(threadIdx.x & 63) {
+    nblk = (ctx + p.BS - 1) / p.BS;
+    shift = (p.BS & (p.BS - 1)) == 0 ? __builtin_ctz(p.BS) : -1;
+    win = block_of(first) >> 6;
+    load_window();
+#pragma unroll
+    for (int n = 0; n < ND; ++n) o[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  __device__ __forceinline__ int block_of(int key) const {
+    if (shift >= 0) return key >> shift;
+    asm volatile("");
+    return key / p.BS;
+  }
+  __device__ __forceinline__ void load_window() {
+    bvec = bt[min((win << 6) + lane, nblk - 1)];
+    if (!index_ok(bvec, p.nblocks, ERR_BLOCK_DECODE)) bvec = 0;
+  }
+  __device__ __forceinline__ void issue_k(int kt0, int stage) {
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const int key = min(kt0 + 16 * g, last & ~15), b = block_of(key);  // (groups past the end re-read the last one)
+      if ((b >> 6) != win) {
+        win = b >> 6;
+        load_window();
+      }
+      at[g] = (((size_t)__builtin_amdgcn_readlane(bvec, b & 63) * p.Hkv + kvh) * p.BS + (key - b * p.BS)) * D;
+      lim[g] = last - key;
+#pragma unroll
+      for (int i = 0; i < PG; ++i) {
+        const int r = i * RPI + lane / CPR;
+        glds16_s<NT>(p.k + at[g], (uint32_t)(min(r, lim[g]) * RB + (((lane % CPR) ^ kswz<D>(r)) << 4)),
+                     ring + stage * 2 * TILE + (g * PG + i) * 1024);
+      }
+    }
+  }
+  __device__ __forceinline__ void issue_v(int stage) {
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int i = 0; i < PG; ++i) {
+        const int r = i * RPI + lane / CPR;
+        glds16_s<NT>(p.v + at[g], (uint32_t)(min(r, lim[g]) * RB + (((lane % CPR) ^ vswz<D>(r)) << 4)),
+                     ring + stage * 2 * TILE + TILE + (g * PG + i) * 1024);
+      }
+  }
+  template <int H>
+  __device__ __forceinline__ void wait() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(H * NI) : "memory");
+  }
+  // all but the `left` buffers issued last have landed
+  __device__ __forceinline__ void wait_left(int left) {
+    if (left >= 2 * NS - 1) return wait<2 * NS - 1>();
+    if constexpr (NS > 3)
+      if (left == 6) return wait<6>();
+    if constexpr (NS > 3)
+      if (left == 5) return wait<5>();
+    if constexpr (NS > 2)
+      if (left == 4) return wait<4>();
+    if constexpr (NS > 2)
+      if (left == 3) return wait<3>();
+    if (left == 2) return wait<2>();
+    if (left == 1) return wait<1>();
+    wait<0>();
+  }
+  // the first tiles' loads: tile t starts at key first + t * step
+  __device__ __forceinline__ void start(int first, int step, int n) {
+#pragma unroll
+    for (int t = 0; t < NS; ++t)
+      if (t < n) issue_k(first + t * step, t), issue_v(t);
+  }
+  // tiles 0 .. n - 1, keys below kv_hi; qf: the rows' fragments
+  __device__ __forceinline__ void run(int first, int step, int n, int kv_hi, const bf16x8_t (&qf)[NC]) {
+    const int h4 = lane >> 4, li = lane & 15, tq = li >> 2, tp = li & 3;
+    int stage = 0;
+    for (int t = 0; t < n; ++t) {
+      const int kt0 = first + t * step;
+      const char* k_lds = ring + stage * 2 * TILE;
+      const char* v_lds = k_lds + TILE;
+      wait_left(2 * (n - t) - 1);
+      bf16x8_t kf[NT16][NC];
+#pragma unroll
+      for (int tt = 0; tt < NT16; ++tt)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const int row = 16 * tt + li;
+          kf[tt][c] = *reinterpret_cast<const bf16x8_t*>(k_lds + row * RB + (((4 * c + h4) ^ kswz<D>(row)) << 4));
+        }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the keys are in registers
+      if (t + NS < n) issue_k(kt0 + NS * step, stage);
+      f32x4_t s[NT16];
+#pragma unroll
+      for (int tt = 0; tt < NT16; ++tt) {
+        s[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < NC; ++c) s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[tt][c], qf[c], s[tt], 0, 0, 0);
+      }
+      // raw-score max, scale folded into the exponent's FMA; deferred rescale as in the prefill kernel:
+      // O (held in accumulator registers) is touched only on tiles where some row's max moved by more
+      // than kRescaleLog2
+      float tmax = -INFINITY;
+      if (kt0 + TK > kv_hi) {  // the context's last tile only; a real branch (see attn_prefill_kernel)
+        asm volatile("");
+#pragma unroll
+        for (int tt = 0; tt < NT16; ++tt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int key = kt0 + 16 * tt + 4 * h4 + r;
+            s[tt][r] = key >= kv_hi ? -INFINITY : s[tt][r];
+          }
+      }
+#pragma unroll
+      for (int tt = 0; tt < NT16; ++tt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, s[tt][r]);
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+      const float m_cand = fmaxf(m, tmax * p.scale_log2);
+      if (__any(m_cand > m + kRescaleLog2)) {
+        const float m_use = m_cand == -INFINITY ? 0.f : m_cand;
+        const float alpha = exp2f(m - m_use);
+        m = m_cand;
+        lsum *= alpha;
+#pragma unroll
+        for (int n2 = 0; n2 < ND; ++n2) o[n2] *= alpha;
+      }
+      const float nm = m == -INFINITY ? 0.f : -m;
+      float pr[NT16][4];
+#pragma unroll
+      for (int tt = 0; tt < NT16; ++tt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          pr[tt][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[tt][r], p.scale_log2, nm));
+          lsum += pr[tt][r];
+        }
+      wait_left(min(2 * (n - t) - 2, 2 * NS - 1));
+      bf16x8_t vf[NCC][ND];
+#pragma unroll
+      for (int cc = 0; cc < NCC; ++cc) {
+        const int r0 = 32 * cc + 4 * h4 + tq;
+        const int r1 = r0 + 16;
+#pragma unroll
+        for (int n2 = 0; n2 < ND; ++n2) {
+          const int unit = 4 * n2 + tp;
+          const int b0 = r0 * RB + ((unit ^ (vswz<D>(r0) << 1)) << 3);
+          const int b1 = r1 * RB + ((unit ^ (vswz<D>(r1) << 1)) << 3);
+          const bf16x4_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4_t*)(v_lds + b0));
+          const bf16x4_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4_t*)(v_lds + b1));
+          vf[cc][n2] = bf16x8_t{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the values are in registers
+      if (t + NS < n) issue_v(stage);
+#pragma unroll
+      for (int cc = 0; cc < NCC; ++cc) {
+        bf16x8_t bp;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          bp[r] = f2bits(pr[2 * cc][r]);
+          bp[4 + r] = f2bits(pr[2 * cc + 1][r]);
+        }
+#pragma unroll
+        for (int n2 = 0; n2 < ND; ++n2) o[n2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[cc][n2], bp, o[n2], 0, 0, 0);
+      }
+      stage = stage + 1 == NS ? 0 : stage + 1;
+    }
+    lsum += __shfl_xor(lsum, 16, 64);
+    lsum += __shfl_xor(lsum, 32, 64);
+  }
+};
+
 // ---------------------------------------------------------------------------
 // Decode (q_len == 1) specialisation: one wave per (sequence, kv head, split).
-// The GQA group's G <= 16 query heads are the 16 MFMA columns.  K/V tiles are
-// fetched by LDS-DMA (global_load_lds_dwordx4: 1 KiB per wave instruction,
-// destination lane-linear, so the XOR swizzle of the K and V images is applied
-// to the per-lane SOURCE address — cdna guide §5.4 rule 21) into a 2-stage
-// ring; the block-table entry of every 4..16-key group is wave-uniform and
-// comes through the scalar cache, so no vector load sits between two tiles.
-// Tile t+1 is issued before tile t is computed and retired with a counted
-// vmcnt, keeping 32 KiB per wave in flight under the MFMA/softmax work.
-//
-// NS > 2 stages (round 4): NS - 1 tiles stay in flight while one is computed.
-// The ring is what bounds the bytes in flight per CU: with 32-key tiles a
-// 2-stage ring (32 KiB per wave, 5 waves per CU) keeps 5 x 16 KiB = 80 KiB
-// in flight, a 4-stage ring (64 KiB per wave, 2 waves per CU) 2 x 48 KiB =
-// 96 KiB, and 512 resident waves divide the (sequence x kv-head) grid of
-// power-of-two batches into whole rounds (2 048 / 4 096 waves at 512 / 1024
-// live sequences) where 1 280 resident waves leave a 0.2-0.6 partial round.
+// The GQA group's G <= 16 query heads are the 16 MFMA columns; the wave walks its part of the keys (DecodeWalk).  What bounds it:
+// a wave's chain of tiles, each a round trip to memory, over the bytes that its ring keeps in flight: with 32-key tiles and 2 stages
+// 24 KiB a wave, 5 waves a CU; 3 stages 40 KiB, 3 waves; 4 stages 56 KiB, 2 waves.  Buffers filled again one by one instead of
+// tile by tile, and no division a lane in the addresses: 64 sequences of 70000 keys, 28 / 4 heads of 128, combine included
+// 42.8 -> 34.1 us (143 MB), 128 of 130000 104 -> 59 (its ring now by the number of waves), 16 of 16000 22.8 -> 15.6, 24 of 300
+// each 20.4 -> 14.7.
 template <int D, int TK, int NS = 2, bool NT = false>
 __global__ __launch_bounds__(64) void paged_decode_kernel(AttnParams p) {
   static_assert(TK == 32 || TK == 64, "keys per tile");
   static_assert(NS >= 2 && NS <= 4, "ring stages");
-  constexpr int NT16 = TK / 16, NCC = TK / 32;
-  constexpr int RB = 2 * D;
-  constexpr int CPR = D / 8;
-  constexpr int NC = D / 32;
-  constexpr int ND = D / 16;
+  constexpr int RB = 2 * D, NC = D / 32, ND = D / 16;
   constexpr int TILE = TK * RB;      // bytes per K (or V) tile
-  constexpr int NI = TILE / 1024;    // LDS-DMA instructions per tile per tensor
-  constexpr int RPI = 1024 / RB;     // rows per instruction
-  static_assert((NS - 1) * 2 * NI <= 63, "vmcnt range");
   __shared__ __attribute__((aligned(16))) char smem[NS * 2 * TILE];
 
   const int lane = threadIdx.x;
@@ -803,147 +991,19 @@ __global__ __launch_bounds__(64) void paged_decode_kernel(AttnParams p) {
 #pragma unroll
     for (int c = 0; c < NC; ++c) qf[c] = *reinterpret_cast<const bf16x8_t*>(qp + 32 * c);
   }
-  const int32_t* bt = p.block_tables + (size_t)seq * p.bt_stride;
-  const int lrow = lane / CPR, lch = lane % CPR;
-  // Block ids of a 64-block window live one per lane; readlane with a
-  // wave-uniform index hands them to the scalar unit, so no vector load ever
-  // sits between two LDS-DMA issues (a vector load there costs a vmcnt(0)
-  // drain of the whole pipeline).
-  // A 64-key tile never straddles a window (64 blocks x BS keys, BS % 16 == 0),
-  // so the window is refreshed at most once per tile, outside the unrolled
-  // issue loop (once per split for split_len <= 64*BS).
-  const int nblk_seq = (ctx + p.BS - 1) / p.BS;
-  int win = (kv_lo / p.BS) >> 6;
-  int bvec = bt[min((win << 6) + lane, nblk_seq - 1)];
-  if (!index_ok(bvec, p.nblocks, ERR_BLOCK_DECODE)) bvec = 0;
+  DecodeWalk<D, TK, NS, NT> walk(p, seq, kvh, ctx, ctx - 1, kv_lo, smem);
   // Retire the Q and block-id loads with a wait hipcc understands, so its
   // scoreboard is empty when the asm-issued LDS-DMA pipeline starts (else it
   // re-waits vmcnt(0) for them inside every iteration).
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
 #pragma unroll
   for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(qf[c]));
-  asm volatile("" : "+v"(bvec));
-
-  auto issue = [&](int kt0, int stage) {
-    char* kdst = smem + stage * 2 * TILE;
-    char* vdst = kdst + TILE;
-    const int w = (kt0 / p.BS) >> 6;
-    if (w != win) {
-      win = w;
-      bvec = bt[min((w << 6) + lane, nblk_seq - 1)];
-      if (!index_ok(bvec, p.nblocks, ERR_BLOCK_DECODE)) bvec = 0;
-    }
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int key0 = min(kt0 + i * RPI, ctx - 1);        // wave-uniform
-      const int blk = __builtin_amdgcn_readlane(bvec, (key0 / p.BS) & 63);
-      const int row = i * RPI + lrow;
-      const int key = min(kt0 + row, ctx - 1);
-      const size_t off = (((size_t)blk * p.Hkv + kvh) * p.BS + (key % p.BS)) * D;
-      const bf16* ks = p.k + off + ((lch ^ kswz<D>(row)) << 3);
-      const bf16* vs = p.v + off + ((lch ^ vswz<D>(row)) << 3);
-      glds16<NT>(ks, kdst + i * 1024);
-      glds16<NT>(vs, vdst + i * 1024);
-    }
-  };
-
-  float m = -INFINITY, lsum = 0.f;
-  f32x4_t o[ND];
-#pragma unroll
-  for (int n = 0; n < ND; ++n) o[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  asm volatile("" : "+v"(walk.bvec));
   const int ntiles = (kv_hi - kv_lo + TK - 1) / TK;
-#pragma unroll
-  for (int t = 0; t < NS - 1; ++t)
-    if (t < ntiles) issue(kv_lo + t * TK, t);
-  for (int t = 0; t < ntiles; ++t) {
-    const int stage = t % NS;
-    const int kt0 = kv_lo + t * TK;
-    if (t + NS - 1 < ntiles) issue(kt0 + (NS - 1) * TK, (t + NS - 1) % NS);
-    // retire tile t: the tiles issued after it may stay in flight (counted, in issue order)
-    const int after = min(NS - 1, ntiles - 1 - t);
-    if (after >= 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * 2 * NI) : "memory");
-    else if (after == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * 2 * NI) : "memory");
-    else if (after == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NI) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const char* k_lds = smem + stage * 2 * TILE;
-    const char* v_lds = k_lds + TILE;
-    f32x4_t s[NT16];
-#pragma unroll
-    for (int tt = 0; tt < NT16; ++tt) {
-      s[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      const int row = 16 * tt + li;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const bf16x8_t a =
-            *reinterpret_cast<const bf16x8_t*>(k_lds + row * RB + (((4 * c + h4) ^ kswz<D>(row)) << 4));
-        s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[c], s[tt], 0, 0, 0);
-      }
-    }
-    // raw-score max, scale folded into the exponent's FMA; deferred rescale as in the prefill kernel:
-    // O (held in accumulator registers) is touched only on tiles where some row's max moved by more
-    // than kRescaleLog2
-    float tmax = -INFINITY;
-    if (kt0 + TK > kv_hi) {  // the context's last tile only; a real branch (see attn_prefill_kernel)
-      asm volatile("");
-#pragma unroll
-      for (int tt = 0; tt < NT16; ++tt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = kt0 + 16 * tt + 4 * h4 + r;
-          s[tt][r] = key >= kv_hi ? -INFINITY : s[tt][r];
-        }
-    }
-#pragma unroll
-    for (int tt = 0; tt < NT16; ++tt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, s[tt][r]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float m_cand = fmaxf(m, tmax * p.scale_log2);
-    if (__any(m_cand > m + kRescaleLog2)) {
-      const float m_use = m_cand == -INFINITY ? 0.f : m_cand;
-      const float alpha = exp2f(m - m_use);
-      m = m_cand;
-      lsum *= alpha;
-#pragma unroll
-      for (int n = 0; n < ND; ++n) o[n] *= alpha;
-    }
-    const float nm = m == -INFINITY ? 0.f : -m;
-    float pr[NT16][4];
-#pragma unroll
-    for (int tt = 0; tt < NT16; ++tt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        pr[tt][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[tt][r], p.scale_log2, nm));
-        lsum += pr[tt][r];
-      }
-    const int tq = li >> 2, tp = li & 3;
-#pragma unroll
-    for (int cc = 0; cc < NCC; ++cc) {
-      bf16x8_t bp;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        bp[r] = f2bits(pr[2 * cc][r]);
-        bp[4 + r] = f2bits(pr[2 * cc + 1][r]);
-      }
-      const int r0 = 32 * cc + 4 * h4 + tq;
-      const int r1 = r0 + 16;
-#pragma unroll
-      for (int n = 0; n < ND; ++n) {
-        const int unit = 4 * n + tp;
-        const int b0 = r0 * RB + ((unit ^ (vswz<D>(r0) << 1)) << 3);
-        const int b1 = r1 * RB + ((unit ^ (vswz<D>(r1) << 1)) << 3);
-        const bf16x4_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4_t*)(v_lds + b0));
-        const bf16x4_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4_t*)(v_lds + b1));
-        const bf16x8_t a = bf16x8_t{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-        o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bp, o[n], 0, 0, 0);
-      }
-    }
-    // every LDS read of this stage has been consumed before the next issue
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  }
-  lsum += __shfl_xor(lsum, 16, 64);
-  lsum += __shfl_xor(lsum, 32, 64);
+  walk.start(kv_lo, TK, ntiles);
+  walk.run(kv_lo, TK, ntiles, kv_hi, qf);
+  float m = walk.m, lsum = walk.lsum;
+  auto& o = walk.o;
   if (!row_valid) return;
   const int head = kvh * G + li;
   if (p.num_splits > 1) {
@@ -1252,15 +1312,10 @@ __device__ __forceinline__ f32x4_t rq_load4(const AttnParams& p, int t, int col)
 template <int D, int NW, bool FR>
 __global__ __launch_bounds__(64 * NW) void paged_decode_mw_kernel(AttnParams p, unsigned* counters) {
   constexpr int TK = 32, NS = 2;
-  constexpr int NT16 = TK / 16, NCC = TK / 32;
   constexpr int RB = 2 * D;
-  constexpr int CPR = D / 8;
   constexpr int NC = D / 32;
   constexpr int ND = D / 16;
   constexpr int TILE = TK * RB;      // bytes per K (or V) tile
-  constexpr int NI = TILE / 1024;    // LDS-DMA instructions per tile per tensor
-  constexpr int RPI = 1024 / RB;     // rows per instruction
-  static_assert((NS - 1) * 2 * NI <= 63, "vmcnt range");
   static_assert((NW * 16 * D + NW * 32 + 1) * 4 <= NW * NS * 2 * TILE, "merge scratch fits in the rings");
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
@@ -1288,46 +1343,16 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_mw_kernel(AttnParams p, 
 #pragma unroll
     for (int c = 0; c < NC; ++c) qf[c] = *reinterpret_cast<const bf16x8_t*>(qp + 32 * c);
   }
-  const int32_t* bt = p.block_tables + (size_t)seq * p.bt_stride;
-  const int lrow = lane / CPR, lch = lane % CPR;
-  const int nblk_seq = (ctx + p.BS - 1) / p.BS;
-  int win = ((kv_lo + w * TK) / p.BS) >> 6;
-  int bvec = bt[min((win << 6) + lane, nblk_seq - 1)];
-  if (!index_ok(bvec, p.nblocks, ERR_BLOCK_DECODE)) bvec = 0;
+  const int ntot = (kv_end - kv_lo + TK - 1) / TK;
+  const int nmine = w < ntot ? (ntot - w + NW - 1) / NW : 0;  // this wave's tiles: w, w + NW, ...
+  const int first = kv_lo + w * TK;
+  // (a wave without tiles, or the one key of a first token, reads nothing)
+  DecodeWalk<D, TK, NS, false> walk(p, seq, kvh, ctx, max(kv_end - 1, 0), min(first, ctx - 1), smem + w * NS * 2 * TILE);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): Q and block ids retired before the counted DMA pipeline
 #pragma unroll
   for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(qf[c]));
-  asm volatile("" : "+v"(bvec));
-
-  char* ring = smem + w * NS * 2 * TILE;
-  auto issue = [&](int kt0, int stage) {
-    char* kdst = ring + stage * 2 * TILE;
-    char* vdst = kdst + TILE;
-    const int wn = (kt0 / p.BS) >> 6;
-    if (wn != win) {
-      win = wn;
-      bvec = bt[min((wn << 6) + lane, nblk_seq - 1)];
-      if (!index_ok(bvec, p.nblocks, ERR_BLOCK_DECODE)) bvec = 0;
-    }
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int key0 = min(kt0 + i * RPI, kv_end - 1);
-      const int blk = __builtin_amdgcn_readlane(bvec, (key0 / p.BS) & 63);
-      const int row = i * RPI + lrow;
-      const int key = min(kt0 + row, kv_end - 1);
-      const size_t off = (((size_t)blk * p.Hkv + kvh) * p.BS + (key % p.BS)) * D;
-      glds16(p.k + off + ((lch ^ kswz<D>(row)) << 3), kdst + i * 1024);
-      glds16(p.v + off + ((lch ^ vswz<D>(row)) << 3), vdst + i * 1024);
-    }
-  };
-
-  float m = -INFINITY, lsum = 0.f;
-  f32x4_t o[ND];
-#pragma unroll
-  for (int n = 0; n < ND; ++n) o[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int ntot = (kv_end - kv_lo + TK - 1) / TK;
-  const int nmine = w < ntot ? (ntot - w + NW - 1) / NW : 0;  // this wave's tiles: w, w + NW, ...
-  if (nmine > 0) issue(kv_lo + w * TK, 0);
+  asm volatile("" : "+v"(walk.bvec));
+  walk.start(first, NW * TK, nmine);
   // FR staging past the rings (mw_rope_lds): q [16][D] bf16, the new K [D] bf16 and V [D] fp32
   bf16* q_st = reinterpret_cast<bf16*>(smem + NW * NS * 2 * TILE);
   bf16* k_st = q_st + 16 * D;
@@ -1377,90 +1402,9 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_mw_kernel(AttnParams p, 
 #pragma unroll
     for (int c = 0; c < NC; ++c) qf[c] = *reinterpret_cast<const bf16x8_t*>(qr + 32 * c);
   }
-  for (int t = 0; t < nmine; ++t) {
-    const int stage = t & 1;
-    const int kt0 = kv_lo + (w + t * NW) * TK;
-    if (t + 1 < nmine) {
-      issue(kt0 + NW * TK, stage ^ 1);
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NI) : "memory");  // tile t landed, t + 1 in flight
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    const char* k_lds = ring + stage * 2 * TILE;
-    const char* v_lds = k_lds + TILE;
-    f32x4_t sc[NT16];
-#pragma unroll
-    for (int tt = 0; tt < NT16; ++tt) {
-      sc[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      const int row = 16 * tt + li;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const bf16x8_t a =
-            *reinterpret_cast<const bf16x8_t*>(k_lds + row * RB + (((4 * c + h4) ^ kswz<D>(row)) << 4));
-        sc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[c], sc[tt], 0, 0, 0);
-      }
-    }
-    float tmax = -INFINITY;
-    if (kt0 + TK > kv_end) {  // the context's last tile only; a real branch (see attn_prefill_kernel)
-      asm volatile("");
-#pragma unroll
-      for (int tt = 0; tt < NT16; ++tt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int key = kt0 + 16 * tt + 4 * h4 + r;
-          sc[tt][r] = key >= kv_end ? -INFINITY : sc[tt][r];
-        }
-    }
-#pragma unroll
-    for (int tt = 0; tt < NT16; ++tt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, sc[tt][r]);
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float m_cand = fmaxf(m, tmax * p.scale_log2);
-    if (__any(m_cand > m + kRescaleLog2)) {
-      const float m_use = m_cand == -INFINITY ? 0.f : m_cand;
-      const float alpha = exp2f(m - m_use);
-      m = m_cand;
-      lsum *= alpha;
-#pragma unroll
-      for (int n = 0; n < ND; ++n) o[n] *= alpha;
-    }
-    const float nm = m == -INFINITY ? 0.f : -m;
-    float pr[NT16][4];
-#pragma unroll
-    for (int tt = 0; tt < NT16; ++tt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        pr[tt][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[tt][r], p.scale_log2, nm));
-        lsum += pr[tt][r];
-      }
-    const int tq = li >> 2, tp = li & 3;
-#pragma unroll
-    for (int cc = 0; cc < NCC; ++cc) {
-      bf16x8_t bp;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        bp[r] = f2bits(pr[2 * cc][r]);
-        bp[4 + r] = f2bits(pr[2 * cc + 1][r]);
-      }
-      const int r0 = 32 * cc + 4 * h4 + tq;
-      const int r1 = r0 + 16;
-#pragma unroll
-      for (int n = 0; n < ND; ++n) {
-        const int unit = 4 * n + tp;
-        const int b0 = r0 * RB + ((unit ^ (vswz<D>(r0) << 1)) << 3);
-        const int b1 = r1 * RB + ((unit ^ (vswz<D>(r1) << 1)) << 3);
-        const bf16x4_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4_t*)(v_lds + b0));
-        const bf16x4_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4_t*)(v_lds + b1));
-        const bf16x8_t a = bf16x8_t{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-        o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bp, o[n], 0, 0, 0);
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this stage's LDS reads done before its refill
-  }
-  lsum += __shfl_xor(lsum, 16, 64);
-  lsum += __shfl_xor(lsum, 32, 64);
+  walk.run(first, NW * TK, nmine, kv_end, qf);
+  float m = walk.m, lsum = walk.lsum;
+  auto& o = walk.o;
 
   if constexpr (FR) {
     if (newkey && w == 0) {  // (wave-uniform) the new token's key: one more online-softmax key, from the staging

@@ -10,7 +10,7 @@ Layer dataflow per step (T tokens, kernels in brackets):
     qkv = x W_qkv^T                                   [grag_gemm_tile at decode M, else library]
     q, K/V-cache <- bias + NeoX RoPE + paged store    [grag_qkv_rope_kvstore]
     a = paged flash attention (GQA-packed, MFMA)      [grag_paged_attention]
-      (1-16 decode rows: the two lines above in one launch, [grag_paged_decode_mw_rope])
+      (few decode rows: the two lines above in one launch, [grag_paged_decode_mw_rope])
     h = a W_o^T        (+ TP all-reduce, RCCL)
     residual += h ; x = RMSNorm(residual)            [grag_rmsnorm]
     m = SiLU(x W_g^T) * (x W_u^T)                     [grag_gemm_tile EPI_SILU: one GEMM, the
@@ -269,7 +269,7 @@ class Qwen2Model:
                 x = rmsnorm(h, L.in_norm, eps, residual=residual)
             if qkv is None:
                 qkv = self._proj(x, L, "qkv_w", defer=True)  # a K-split's reduce folds into the RoPE pass
-            # 1-16 decode rows: RoPE + K/V store inside the attention launch (ops/attention.py ROPE_FUSE)
+            # few decode rows: RoPE + K/V store inside the attention launch (ops/attention.py ROPE_FUSE)
             a = paged_decode_mw_rope(qkv, L.qkv_b, positions, self.cos_sin, kc, vc, meta, self.scale, self.hq,
                                      self.hkv, self.head_dim) if isinstance(qkv, SplitKPartial) else None
             if a is None:

@@ -19,17 +19,15 @@ _DEC_STAGES = int(os.environ.get("GRAG_DECODE_STAGES", "2"))
 DECODE_NW = {64: 1, 32: {2: 3, 3: 8, 4: 7}[_DEC_STAGES]}[int(os.environ.get("GRAG_DECODE_TK", "32"))]
 DECODE_RING_NW = {2: 3, 3: 8, 4: 7}  # stages -> nw code (microbench / A/B)
 _DEC_AUTO = "GRAG_DECODE_STAGES" not in os.environ and os.environ.get("GRAG_DECODE_TK", "32") == "32"
-# non-temporal K/V LDS-DMA loads (nt: the cache is read once per decode step; MI355X_MICROARCH 'nt-weights'):
-# codes 11 / 12 are 3 / 8 with nt.  profiles/mb_decode_nt_r4.json: B512 ctx1100 206.4 -> 186.8 us (5.59 -> 6.18
-# TB/s), B1024 413.7 -> 382.5, B256 113.3 -> 97.7, B176 ctx3000 (3 stages) 208.0 -> 197.0, B16 ctx6000 50.2 ->
-# 48.0; grids under ~1.5K waves gain nothing (B64 ctx1152 x 5 parts: 35.8 vs 36.7, B1: equal) -> default there
+# non-temporal K/V LDS-DMA loads (nt: the cache is read once per decode step): codes 11 / 12 are 3 / 8 with nt.
+# us of 3 / 11, combine included, 28 / 4 heads: B192 ctx3000 236 / 207, B128 ctx1500 82.1 / 71.8, B64 of 70000 keys in all
+# 40.3 / 33.7, B16 of 16000 17.3 / 15.6, B5 ctx3000 20.5 / 19.9, B24 ctx300 14.9 / 14.7: at every size
 DECODE_NT = {3: 11, 8: 12}
-# round 6 (profiles/attn_sweep_r6.json, one box): nt pays from ~700 waves too -- B176 ctx1500 one part 94.6 ->
-# 89.3 us, B256 134.8 -> 117.9 -- so the threshold moved down from 1536 waves
-DECODE_NT_MIN_WAVES = int(os.environ.get("GRAG_DECODE_NT_MIN_WAVES", "512"))
-# multi-part plans over >= this many (sequence x kv head) rows take the 3-stage ring: B192 ctx3000 (2 parts of
-# 2048 keys) 222.7 -> 191.7 us, B128 ctx1500 (2 x 1024) 73.5 -> 67.8 (0: off)
-DECODE_NS3_ROWS = int(os.environ.get("GRAG_DECODE_NS3_ROWS", "512"))
+DECODE_NT_MIN_WAVES = int(os.environ.get("GRAG_DECODE_NT_MIN_WAVES", "0"))
+# multi-part plans of more waves than the chip holds at once with 2-stage rings (5 a CU) take the 3-stage ring (3 a CU, as many
+# bytes in flight): us of 11 / 12, 28 / 4 heads: B192 ctx3000 (1536 waves) 207 / 194, B176 ctx1500 (1408) 104 / 97.5, but B128
+# ctx1500 (1024) 71.8 / 82.8 and B128 of 130000 keys in all (1024) 56.3 / 75.0 (0: off)
+DECODE_NS3_WAVES = int(os.environ.get("GRAG_DECODE_NS3_WAVES", "1280"))
 _DEC_NT = os.environ.get("GRAG_DECODE_NT", "auto")
 
 
@@ -39,6 +37,7 @@ _DEC_NT = os.environ.get("GRAG_DECODE_NT", "auto")
 DECODE_MW = {22: 2, 24: 4}
 DECODE_MW_CODE = int(os.environ.get("GRAG_DECODE_MW_CODE", "24"))
 DECODE_MW_ROWS = int(os.environ.get("GRAG_DECODE_MW", "16"))
+DECODE_MW_PARTS = 200  # or sequences x kv heads x parts at most this many (decode_mw_takes)
 MW_SPLITS = int(os.environ.get("GRAG_DECODE_MW_SPLITS", "20"))  # target parts per sequence at B = 1
 
 
@@ -62,6 +61,16 @@ def decode_mw_plan(B: int, Hkv: int, max_ctx: int, max_model_len: int, force: bo
     return max(1, min(ns, -(-max_model_len // split_len))), split_len
 
 
+def decode_mw_takes(meta, Hkv: int) -> bool:
+    """Whether a decode step without a kernel of its own choice takes the small-batch kernel: few rows, or so few parts in all
+    that the launches it saves (the combine, the RoPE pass) count for more than its 4 waves' LDS.  us without / with, RoPE pass not
+    counted, sequences x keys (parts): 28 / 4 heads 8 x 1000 (128) 15.3 / 14.6, 24 x 300 (192) 14.7 / 13.3, 5 x 3000 (240) 19.9 /
+    22.5; 12 / 2 heads 16 x 300 (64) 14.4 / 11.7, 12 x 2000 (192) 17.7 / 16.1."""
+    rows = meta.num_seqs * Hkv
+    few = meta.cascade is None and rows * meta.num_splits <= DECODE_MW_PARTS
+    return DECODE_MW_ROWS > 0 and (rows <= DECODE_MW_ROWS or few)
+
+
 def decode_counters(dev: torch.device) -> torch.Tensor:
     """The small-batch decode kernel's per-(sequence, kv head) tickets (zeroed once; every last arriver resets
     its word, so hipGraph replays need no memset).  Owned by the caller's workspace owner (ops/gemm.py
@@ -74,19 +83,12 @@ def decode_counters(dev: torch.device) -> torch.Tensor:
 
 
 def decode_variant(nsplit: int, split_len: int, waves: int | None = None) -> int:
-    """Decode kernel per split plan (profiles/mb_decode_ring_r4.json, 32-key tiles): long-context decode
-    (split-KV parts covering > 2048 keys: ingest's 3-6K-token prompts) keeps two tiles in flight per wave
-    in a 3-stage ring (B176 ctx3000: 238.8 -> 207.8 us, B16 ctx6000: 53.5 -> 50.1 us); the serving
-    batches (one part of ~1.1K keys, or 256-key parts) stay on the 2-stage ring, whose 5 waves per CU win
-    there (B512 ctx1100: 207.8 vs 222.8 us, B64 ctx1152: 35.6 vs 40.7 us).  ``waves``: the launch's
-    (sequence x kv-head x split) count; grids of >= DECODE_NT_MIN_WAVES load K/V non-temporally."""
-    # round 5 (profiles/attn_sweep_r5_mw.json, same box): the 3-stage ring lost at B16 4K (45.2 vs 32.1 us at
-    # 256-key parts) and tied elsewhere (B16 11.6K 78.0 vs 76.4, B176 1.5K 98.8 vs 96.5): 2 stages unless
-    # GRAG_DECODE_STAGES asks (the round-4 auto rule is kept behind GRAG_DECODE_RING_AUTO=1)
+    """Decode kernel per split plan, 32-key tiles.  ``waves``: the launch's (sequence x kv-head x split) count; more than
+    DECODE_NS3_WAVES of several parts take the 3-stage ring, at least DECODE_NT_MIN_WAVES load K/V non-temporally
+    (GRAG_DECODE_RING_AUTO=1: the 3-stage ring for parts that cover more than 2048 keys)."""
     auto3 = _DEC_AUTO and os.environ.get("GRAG_DECODE_RING_AUTO") == "1"
     nw = DECODE_RING_NW[3] if auto3 and nsplit > 1 and nsplit * split_len > 2048 else DECODE_NW
-    if (_DEC_AUTO and DECODE_NS3_ROWS and nsplit > 1 and waves is not None
-            and waves // nsplit >= DECODE_NS3_ROWS):
+    if _DEC_AUTO and DECODE_NS3_WAVES and nsplit > 1 and waves is not None and waves > DECODE_NS3_WAVES:
         nw = DECODE_RING_NW[3]
     nt = _DEC_NT == "1" or (_DEC_NT == "auto" and waves is not None and waves >= DECODE_NT_MIN_WAVES)
     return DECODE_NT.get(nw, nw) if nt else nw
@@ -308,7 +310,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         nw = meta.extra.get("decode_nw")
         if nw is None:
             nw = decode_variant(nsplit, meta.split_len, meta.num_seqs * Hkv * nsplit)
-            if DECODE_MW_ROWS and meta.num_seqs * Hkv <= DECODE_MW_ROWS:
+            if decode_mw_takes(meta, Hkv):
                 nw = DECODE_MW_CODE
         if nw in DECODE_MW and D in (64, 128) and Hq // Hkv <= 16 and BS % 16 == 0 \
                 and (nsplit == 1 or meta.split_len % 32 == 0) and meta.num_seqs * Hkv <= (1 << 16):
@@ -362,7 +364,7 @@ def paged_decode_mw_rope(qkv, bias, positions, cos_sin, k_cache, v_cache, meta: 
     BS = k_cache.shape[2]
     nsplit = meta.num_splits
     nw = meta.extra.get("decode_nw")
-    if nw is None and DECODE_MW_ROWS and meta.num_seqs * Hkv <= DECODE_MW_ROWS:
+    if nw is None and decode_mw_takes(meta, Hkv):
         nw = DECODE_MW_CODE
     if not (nw in DECODE_MW and D in (64, 128) and Hq // Hkv <= 16 and BS % 16 == 0 and qkv.N == (Hq + 2 * Hkv) * D
             and (nsplit == 1 or meta.split_len % 32 == 0) and meta.num_seqs * Hkv <= (1 << 16)
