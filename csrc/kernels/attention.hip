@@ -23,6 +23,7 @@
 // Both products use v_mfma_f32_16x16x32_bf16.  Online softmax runs in the
 // log2 domain (exp2).
 #include "common.h"
+#include "decode_loads.h"
 
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
@@ -82,89 +83,7 @@ struct AttnParams {
 // 2048 + 512-key split plan 233 -> 292 us
 int g_decode_xcd = 0;
 
-// Chunk (16 B) swizzle for the K image read as row fragments by ds_read_b128.
-template <int D>
-__device__ __forceinline__ int kswz(int row) {
-  if constexpr (D == 128) return row & 15;
-  else if constexpr (D == 64) return (row >> 1) & 7;
-  else return (row >> 2) & 3;
-}
-// Chunk (16 B) swizzle for the V image read with ds_read_b64_tr_b16: a 32-lane
-// half reads 8 consecutive rows x 4 8-byte units; these XORs spread them over
-// all 64 banks (derivation in docs/kernels.md).
-template <int D>
-__device__ __forceinline__ int vswz(int row) {
-  if constexpr (D == 128) return (row & 7) << 1;
-  else if constexpr (D == 64) return ((row >> 1) & 3) << 1;
-  else return ((row >> 2) & 1) << 1;
-}
-
 typedef __attribute__((address_space(3))) bf16x4_t lds_bf16x4_t;
-
-// One LDS-DMA wave instruction (global_load_lds_dwordx4): 16 B per lane from
-// each lane's `src` into the 1 KiB LDS block at wave-uniform `lds_dst`
-// (lane-linear).  Issued from inline asm so hipcc's waitcnt pass does not see
-// an LDS write it cannot disambiguate between ring stages (it would put a
-// vmcnt(0) in front of every ds_read); completion is tracked only by the
-// caller's explicit counted `s_waitcnt vmcnt(N)` (cdna guide §5.7 recipe:
-// M0 saved, set, used and restored inside one statement).
-template <bool NT = false>
-__device__ __forceinline__ void glds16(const void* src, void* lds_dst) {
-  const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds_dst;
-  const uint32_t lu = __builtin_amdgcn_readfirstlane(lds);
-  uint32_t keep;
-  if constexpr (NT) {  // non-temporal: once-read streams (decode K/V, MI355X_MICROARCH 'nt-weights')
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %2\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, off nt\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(keep)
-        : "v"(src), "s"(lu)
-        : "memory");
-  } else {
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %2\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, off\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(keep)
-        : "v"(src), "s"(lu)
-        : "memory");
-  }
-}
-
-// The same LDS-DMA with the address as a wave-uniform 64-bit base in SGPRs plus a 32-bit per-lane byte
-// offset (global_load_lds saddr form): no 64-bit VALU address arithmetic per load.
-template <bool NT = false>
-__device__ __forceinline__ void glds16_s(const void* sbase, uint32_t voff, void* lds_dst) {
-  const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds_dst;
-  const uint32_t lu = __builtin_amdgcn_readfirstlane(lds);
-  uint32_t keep;
-  if constexpr (NT) {
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %3\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, %2 nt\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(keep)
-        : "v"(voff), "s"(sbase), "s"(lu)
-        : "memory");
-  } else {
-    asm volatile(
-        "s_mov_b32 %0, m0\n\t"
-        "s_mov_b32 m0, %3\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, %2\n\t"
-        "s_mov_b32 m0, %0"
-        : "=&s"(keep)
-        : "v"(voff), "s"(sbase), "s"(lu)
-        : "memory");
-  }
-}
 
 template <int D, int NW, bool PAGED>
 __global__ __launch_bounds__(64 * NW, D <= 64 && NW == 4 ? 4 : 1) void attn_fwd_kernel(AttnParams p) {
@@ -758,97 +677,20 @@ __device__ __forceinline__ void merge_prefix(const AttnParams& p, int tok, int h
   m = M;
 }
 
-// One wave's walk over TK-key tiles of a decode sequence: its ring of NS K and NS V buffers in LDS, filled by LDS-DMA.  A K buffer
-// is filled again as soon as its tile's keys are in registers, a V buffer as soon as the values are, so 2 NS - 1 of the 2 NS
-// buffers are in flight while the wave computes (tile by tile, 2 NS - 2).  Addresses are formed once per 16 keys, which lie in one
-// cache block: a wave-uniform base and an offset a lane that only the context's end changes (with a division a piece and lane the
-// addresses took longer than the products).  The block ids of a window of 64 blocks live one per lane; readlane hands them to the
-// scalar unit.
+// One wave's softmax over the tiles of a decode sequence that DecodeLoads brings
 template <int D, int TK, int NS, bool NT>
-struct DecodeWalk {
-  static constexpr int RB = 2 * D, CPR = D / 8, NC = D / 32, ND = D / 16, TILE = TK * RB, NI = TILE / 1024;
-  static constexpr int RPI = 1024 / RB, PG = 16 / RPI, NG = TK / 16, NT16 = TK / 16, NCC = TK / 32;
-  static_assert((2 * NS - 1) * NI <= 63, "vmcnt range");
+struct DecodeWalk : DecodeLoads<D, TK, NS, NT> {
+  using L = DecodeLoads<D, TK, NS, NT>;
+  using L::lane, L::ring, L::issue_k, L::issue_v, L::wait_left;
+  static constexpr int RB = 2 * D, NC = D / 32, ND = D / 16, TILE = TK * RB, NT16 = TK / 16, NCC = TK / 32;
   const AttnParams& p;
-  const int32_t* bt;
-  char* ring;
-  int kvh, last, nblk, lane, win, bvec, shift;
-  size_t at[NG];  // of the tile whose keys were issued last: its groups' first element, its last valid row
-  int lim[NG];
   float m = -INFINITY, lsum = 0.f;
   f32x4_t o[ND];
 
-  // `last`: the last key that may be read
-  __device__ __forceinline__ DecodeWalk(const AttnParams& p_, int seq, int kvh_, int ctx, int last_, int first, char* ring_)
-      : p(p_), bt(p_.block_tables + (size_t)seq * p_.bt_stride), ring(ring_), kvh(kvh_), last(last_), lane(threadIdx.x & 63) {
-    nblk = (ctx + p.BS - 1) / p.BS;
-    shift = (p.BS & (p.BS - 1)) == 0 ? __builtin_ctz(p.BS) : -1;
-    win = block_of(first) >> 6;
-    load_window();
+  __device__ __forceinline__ DecodeWalk(const AttnParams& p_, int seq, int kvh, int ctx, int last, int first, char* ring_)
+      : L(p_.k, p_.v, p_.block_tables + (size_t)seq * p_.bt_stride, p_.BS, p_.Hkv, p_.nblocks, kvh, ctx, last, first, ring_), p(p_) {
 #pragma unroll
     for (int n = 0; n < ND; ++n) o[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  }
-  __device__ __forceinline__ int block_of(int key) const {
-    if (shift >= 0) return key >> shift;
-    asm volatile("");
-    return key / p.BS;
-  }
-  __device__ __forceinline__ void load_window() {
-    bvec = bt[min((win << 6) + lane, nblk - 1)];
-    if (!index_ok(bvec, p.nblocks, ERR_BLOCK_DECODE)) bvec = 0;
-  }
-  __device__ __forceinline__ void issue_k(int kt0, int stage) {
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      const int key = min(kt0 + 16 * g, last & ~15), b = block_of(key);  // (groups past the end re-read the last one)
-      if ((b >> 6) != win) {
-        win = b >> 6;
-        load_window();
-      }
-      at[g] = (((size_t)__builtin_amdgcn_readlane(bvec, b & 63) * p.Hkv + kvh) * p.BS + (key - b * p.BS)) * D;
-      lim[g] = last - key;
-#pragma unroll
-      for (int i = 0; i < PG; ++i) {
-        const int r = i * RPI + lane / CPR;
-        glds16_s<NT>(p.k + at[g], (uint32_t)(min(r, lim[g]) * RB + (((lane % CPR) ^ kswz<D>(r)) << 4)),
-                     ring + stage * 2 * TILE + (g * PG + i) * 1024);
-      }
-    }
-  }
-  __device__ __forceinline__ void issue_v(int stage) {
-#pragma unroll
-    for (int g = 0; g < NG; ++g)
-#pragma unroll
-      for (int i = 0; i < PG; ++i) {
-        const int r = i * RPI + lane / CPR;
-        glds16_s<NT>(p.v + at[g], (uint32_t)(min(r, lim[g]) * RB + (((lane % CPR) ^ vswz<D>(r)) << 4)),
-                     ring + stage * 2 * TILE + TILE + (g * PG + i) * 1024);
-      }
-  }
-  template <int H>
-  __device__ __forceinline__ void wait() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(H * NI) : "memory");
-  }
-  // all but the `left` buffers issued last have landed
-  __device__ __forceinline__ void wait_left(int left) {
-    if (left >= 2 * NS - 1) return wait<2 * NS - 1>();
-    if constexpr (NS > 3)
-      if (left == 6) return wait<6>();
-    if constexpr (NS > 3)
-      if (left == 5) return wait<5>();
-    if constexpr (NS > 2)
-      if (left == 4) return wait<4>();
-    if constexpr (NS > 2)
-      if (left == 3) return wait<3>();
-    if (left == 2) return wait<2>();
-    if (left == 1) return wait<1>();
-    wait<0>();
-  }
-  // the first tiles' loads: tile t starts at key first + t * step
-  __device__ __forceinline__ void start(int first, int step, int n) {
-#pragma unroll
-    for (int t = 0; t < NS; ++t)
-      if (t < n) issue_k(first + t * step, t), issue_v(t);
   }
   // tiles 0 .. n - 1, keys below kv_hi; qf: the rows' fragments
   __device__ __forceinline__ void run(int first, int step, int n, int kv_hi, const bf16x8_t (&qf)[NC]) {

@@ -3,13 +3,13 @@
 // D = 64 or 128 for keys and values alike, 16-key cache blocks; other calls take the kernel of seqmix.hip.
 //
 // A workgroup is a part of a sequence's keys for one kv head (and up to 16 of its query heads); wave w walks its tiles of 32 keys
-// w, w + NW, ... by itself, without a barrier.  K goes from memory to the registers as the operand of S^T = K Q^T, one tile
-// ahead; V by LDS-DMA into the wave's own two buffers and out of them by transposed reads.  Weights are fp32, bf16 hi + lo in
-// the second product.  The waves' sums meet in LDS once, at the end.
-// Bound by the bytes in flight: 64 sequences of 70000 keys in all, 28 / 4 heads of 128, parts of 512 keys, 42 us with the
-// combination (143 MB; 5 us of it the second launch), 82 in the staged 64-key tiles of four waves in step; 12 / 2 heads 45 ->
-// 25; 16 / 4 heads of 64 33 -> 21; 128 sequences of 130000 128 -> 67; one of 4000 28 -> 13.  With the compiler's LDS-DMA builtin
-// it drained every load before the transposed reads: 54.
+// w, w + NW, ... by itself, without a barrier, its loads ahead in a ring of its own (decode_loads.h).  Weights are fp32, bf16 hi +
+// lo in the second product.  The waves' sums meet in LDS once, at the end.
+// Bound by the bytes in flight and the chain of a wave's tiles.  us with the combination (5 of them the second launch), before, with
+// K from memory to the registers (64 bytes a row and instruction, which non-temporal loads tore: 42.9) -> now: 64 sequences of
+// 70000 keys in all, 28 / 4 heads of 128, parts of 512 keys (143 MB) 42.4 -> 36.1, 128 of 130000 70.3 -> 60.9, window 1024 of these
+// 25.3 -> 21.8 and 46.4 -> 40.3; 12 / 2 heads 128 of 130000 42.0 -> 36.6.
+#include "decode_loads.h"
 #include "sink.h"
 
 GRAG_ERR_UNIT(sink_decode)
@@ -24,29 +24,11 @@ struct SinkDecodeArgs {
   float *part_o, *part_ml;
 };
 
-// One LDS-DMA instruction: 16 bytes a lane from `src` into the 1 KB of LDS at the wave-uniform `dst`, lane after lane.  As asm
-// the compiler does not count it, so that it neither drains the vector memory counter before the transposed reads of the other
-// buffer nor reckons with it in its waits for the K registers; the waits below do.
-__device__ __forceinline__ void sd_dma(const void* src, char* dst) {
-  const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)dst);
-  uint32_t keep;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, off\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(keep)
-      : "v"(src), "s"(lds)
-      : "memory");
-}
-
 template <int D, int NW, bool CAP>
-__global__ void __launch_bounds__(64 * NW, D == 64 ? 4 : 2) sink_decode_kernel(const SinkDecodeArgs pa) {
+__global__ void __launch_bounds__(64 * NW) sink_decode_kernel(const SinkDecodeArgs pa) {
   const SinkArgs& p = pa.a;
-  constexpr int RB = 2 * D, CPR = D / 8, NC = D / 32, ND = D / 16, VT = SD_KT * RB;  // VT: bytes of a V tile
-  constexpr int NI = VT / 1024, RPI = 1024 / RB;                                     // DMA pieces of a tile, rows of a piece
-  __shared__ __attribute__((aligned(16))) char smem[NW * 2 * VT];
+  constexpr int RB = 2 * D, NC = D / 32, ND = D / 16, NS = 2, TILE = SD_KT * RB, RING = NS * 2 * TILE;
+  __shared__ __attribute__((aligned(16))) char smem[NW * RING];
   __shared__ float wm[NW][16], wl[NW][16];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h4 = lane >> 4, li = lane & 15;
@@ -74,47 +56,32 @@ __global__ void __launch_bounds__(64 * NW, D == 64 ? 4 : 2) sink_decode_kernel(c
 #pragma unroll
     for (int c = 0; c < NC; ++c)
       qf[c] = valid ? *reinterpret_cast<const bf16x8_t*>(qp + 32 * c) : bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-    const int* bt = p.bt + (size_t)seq * p.bt_stride;
-    const int last = (hi - 1) / SP_BS, last_slot = (hi - 1) % SP_BS;
-    int base = 0, bvec = 0;  // 64 entries of the block table, one a lane: 1024 keys
-    auto block = [&](int i) __attribute__((always_inline)) { return __builtin_amdgcn_readlane(bvec, min(i, last) - base); };
-    const int vrow = lane / CPR, vch = lane % CPR;
-    char* vbuf = smem + wave * 2 * VT;
-    bf16x8_t kf[2][2][NC];
-    auto at = [&](int kt0, int tt) __attribute__((always_inline)) {
-      return ((size_t)block((kt0 + 16 * tt) / SP_BS) * p.G + g) * SP_BS * D;
-    };
-    // K of tile t into register set `st`, V into buffer `st`.  Keys past the last one re-read it (their weights are 0, and 0
-    // times whatever lies there must be 0).
-    auto load_k = [&](int t, auto st) __attribute__((always_inline)) {
-      constexpr int S = decltype(st)::value;
-      const int kt0 = lo + t * SD_KT;
+    const int first = lo + wave * SD_KT, step = NW * SD_KT, n = (ntiles - wave + NW - 1) / NW;
+    DecodeLoads<D, SD_KT, NS, true> ld(p.k, p.v, p.bt + (size_t)seq * p.bt_stride, SP_BS, p.G, p.nblocks, g, hi, hi - 1, first,
+                                       smem + wave * RING);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): q and the table, so that the compiler waits for none of them in the loop
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
-        const bf16* kp = p.k + at(kt0, tt) + (kt0 + 16 * tt + li < hi ? li : last_slot) * D + 8 * h4;
+    for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(qf[c]));
+    asm volatile("" : "+v"(ld.bvec));
+    ld.start(first, step, n);
+    for (int t = 0; t < n; ++t) {
+      const int kt0 = first + t * step, stage = t & 1;
+      const char *k_lds = ld.ring + stage * 2 * TILE, *v_lds = k_lds + TILE;
+      ld.wait_left(2 * (n - t) - 1);
+      bf16x8_t kf[2][NC];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) kf[S][tt][c] = *reinterpret_cast<const bf16x8_t*>(kp + 32 * c);
-      }
-    };
-    auto load_v = [&](int t, auto st) __attribute__((always_inline)) {
-      constexpr int S = decltype(st)::value;
-      const int kt0 = lo + t * SD_KT;
-      const size_t a[2] = {at(kt0, 0), at(kt0, 1)};
+      for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int r = i * RPI + vrow, slot = kt0 + r < hi ? r % SP_BS : last_slot;
-        sd_dma(p.v + a[i * RPI / SP_BS] + slot * D + ((vch ^ sp_vswz<D>(r)) << 3), vbuf + S * VT + i * 1024);
-      }
-    };
-    auto tile = [&](int t, auto st, auto more) __attribute__((always_inline)) {
-      constexpr int S = decltype(st)::value;
-      const int kt0 = lo + t * SD_KT;
+        for (int c = 0; c < NC; ++c)
+          kf[tt][c] = *reinterpret_cast<const bf16x8_t*>(k_lds + (16 * tt + li) * RB + (((4 * c + h4) ^ kswz<D>(16 * tt + li)) << 4));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the keys are in registers
+      if (t + NS < n) ld.issue_k(kt0 + NS * step, stage);
       f32x4_t s[2];
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt) {
         s[tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int c = 0; c < NC; ++c) s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[S][tt][c], qf[c], s[tt], 0, 0, 0);
+        for (int c = 0; c < NC; ++c) s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[tt][c], qf[c], s[tt], 0, 0, 0);
       }
       if constexpr (CAP) {  // cap in the natural domain, then to log2
         const float ic = 1.f / p.softcap, c2 = p.softcap * LOG2E;
@@ -148,7 +115,7 @@ __global__ void __launch_bounds__(64 * NW, D == 64 ? 4 : 2) sink_decode_kernel(c
         m = cand;
         lsum *= alpha;
 #pragma unroll
-        for (int n = 0; n < ND; ++n) o[n] *= alpha;
+        for (int n2 = 0; n2 < ND; ++n2) o[n2] *= alpha;
       }
       const float mm = m == -INFINITY ? 0.f : m;
       bf16x8_t ph, pl;
@@ -162,61 +129,26 @@ __global__ void __launch_bounds__(64 * NW, D == 64 ? 4 : 2) sink_decode_kernel(c
           pl[4 * tt + r] = f2bits(x - bits2f(b));
           lsum += x;
         }
-      // K and V of this tile have landed (loads do in issue order): behind them at least the 2 NC loads of the next tile's K are
-      // under way, which no load passes (the asm clobbers memory); more of them, a spill's say, would only wait for longer.  And
-      // the reads of the tile before have returned from the buffer that is filled now.
-      if constexpr (decltype(more)::value) {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * NC) : "memory");
-        load_v(t + NW, std::integral_constant<int, 1 - S>{});
-      } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      }
-      const char* v_lds = vbuf + S * VT;
+      ld.wait_left(2 * (n - t) - 2);
       const int r0 = 4 * h4 + (li >> 2), r1 = r0 + 16, tp = li & 3;
+      bf16x8_t vf[ND];
 #pragma unroll
-      for (int n = 0; n < ND; ++n) {
-        const int unit = 4 * n + tp;
-        const bf16x4_t a0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (sp_lds4_t*)(v_lds + r0 * RB + ((unit ^ (sp_vswz<D>(r0) << 1)) << 3)));
-        const bf16x4_t a1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (sp_lds4_t*)(v_lds + r1 * RB + ((unit ^ (sp_vswz<D>(r1) << 1)) << 3)));
-        const bf16x8_t a = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
-        o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pl, o[n], 0, 0, 0);
-        o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, ph, o[n], 0, 0, 0);
+      for (int n2 = 0; n2 < ND; ++n2) {
+        const int unit = 4 * n2 + tp;
+        const bf16x4_t a0 =
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((sp_lds4_t*)(v_lds + r0 * RB + ((unit ^ (vswz<D>(r0) << 1)) << 3)));
+        const bf16x4_t a1 =
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((sp_lds4_t*)(v_lds + r1 * RB + ((unit ^ (vswz<D>(r1) << 1)) << 3)));
+        vf[n2] = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
       }
-    };
-    using S0 = std::integral_constant<int, 0>;
-    using S1 = std::integral_constant<int, 1>;
-    const std::true_type more{};
-    const std::false_type end{};
-    for (int w0 = 0; w0 < ntiles; w0 += 32) {  // the tiles of 64 entries
-      const int stop = min(ntiles, w0 + 32);
-      int t = w0 + wave;
-      if (t >= stop) break;
-      base = (lo + w0 * SD_KT) / SP_BS;
-      bvec = bt[min(base + lane, last)];
-      if (!index_ok(bvec, p.nblocks, ERR_BLOCK_DECODE)) bvec = 0;  // reported; block 0 read instead of faulting
-      __builtin_amdgcn_s_waitcnt(0x0F70);                          // vmcnt(0): q and the table
-      load_k(t, S0{});
-      load_v(t, S0{});
-      while (true) {  // one tile ahead: K before this tile's scores, V after them
-        if (t + NW >= stop) {
-          tile(t, S0{}, end);
-          break;
-        }
-        load_k(t + NW, S1{});
-        tile(t, S0{}, more);
-        t += NW;
-        if (t + NW >= stop) {
-          tile(t, S1{}, end);
-          break;
-        }
-        load_k(t + NW, S0{});
-        tile(t, S1{}, more);
-        t += NW;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the values are in registers
+      if (t + NS < n) ld.issue_v(stage);
+#pragma unroll
+      for (int n2 = 0; n2 < ND; ++n2) {
+        o[n2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[n2], pl, o[n2], 0, 0, 0);
+        o[n2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[n2], ph, o[n2], 0, 0, 0);
       }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
   lsum += __shfl_xor(lsum, 16, 64);
   lsum += __shfl_xor(lsum, 32, 64);
@@ -224,8 +156,8 @@ __global__ void __launch_bounds__(64 * NW, D == 64 ? 4 : 2) sink_decode_kernel(c
     wm[wave][li] = m;
     wl[wave][li] = lsum;
   }
-  // the wave's sums in its own V buffers, [head][D]; a row's 16-byte chunks turned by the row
-  float* ow = reinterpret_cast<float*>(smem + wave * 2 * VT);
+  // the wave's sums in its own buffers, [head][D]; a row's 16-byte chunks turned by the row
+  float* ow = reinterpret_cast<float*>(smem + wave * RING);
 #pragma unroll
   for (int n = 0; n < ND; ++n) *reinterpret_cast<f32x4_t*>(ow + li * D + (((4 * n + h4) ^ (li & 7)) << 2)) = o[n];
   __syncthreads();
@@ -240,7 +172,7 @@ __global__ void __launch_bounds__(64 * NW, D == 64 ? 4 : 2) sink_decode_kernel(c
     for (int w = 0; w < NW; ++w) {
       const float f = wm[w][h] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(wm[w][h] - M);
       L = fmaf(wl[w][h], f, L);
-      const f32x4_t x = *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(smem + w * 2 * VT) + h * D +
+      const f32x4_t x = *reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(smem + w * RING) + h * D +
                                                           ((c ^ (h & 7)) << 2));
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = fmaf(x[e], f, v[e]);
@@ -282,14 +214,17 @@ hipError_t sink_decode_launch(const void* q, const void* k, const void* v, void*
   a.scale = scale, a.out_scale = out_scale, a.softcap = softcap;
   pa.nsplit = nsplit, pa.split_len = split_len, pa.part_o = part_o, pa.part_ml = part_ml;
   const dim3 grid(nsplit, G * ((a.R + 15) / 16), nseq);
-  // four waves where the parts are few, two where they fill the chip anyway (and a smaller unit fills it more evenly): 448 parts
-  // of 256 keys 15.5 us with four, 15.8 with two; 1024 of 512 44.5 / 42.2; 16 of 256 13.2 / 14.1
-  const bool few = (long)nsplit * G * ((a.R + 15) / 16) * nseq < 512;
+  // Waves a part: many parts fill the chip by themselves, few are each a chain of tiles to be shared.  us of 1 / 2 / 4 waves, parts
+  // of keys: 1024 of 512 36.1 / 40.1 / 43.8, 1024 of 256 25.1 / 28.1 / 32.6, 816 of 256 24.8 / 26.2 / 27.8, 512 of 256 18.4 / 15.4 /
+  // 17.6, 384 of 256 18.8 / 15.8 / 18.2, 192 of 256 17.1 / 12.3 / 11.1, 36 of 128 13.6 / 11.1 / 10.2; 512 of 1024 46.6 / 40.3 /
+  // 42.1, 256 of 1024 43.6 / 26.1 / 21.8.
+  const long parts = (long)nsplit * G * ((a.R + 15) / 16) * nseq;
 #define SINK_DECODE_W(DD, CAP, NW) hipLaunchKernelGGL((sink_decode_kernel<DD, NW, CAP>), grid, dim3(64 * NW), 0, st, pa)
-#define SINK_DECODE(DD, CAP)              \
-  {                                       \
-    if (few) SINK_DECODE_W(DD, CAP, 4);   \
-    else SINK_DECODE_W(DD, CAP, 2);       \
+#define SINK_DECODE(DD, CAP)                          \
+  {                                                   \
+    if (parts >= 768) SINK_DECODE_W(DD, CAP, 1);      \
+    else if (parts >= 384) SINK_DECODE_W(DD, CAP, 2); \
+    else SINK_DECODE_W(DD, CAP, 4);                   \
   }
   if (d == 64 && softcap > 0.f) SINK_DECODE(64, true)
   else if (d == 64) SINK_DECODE(64, false)
