@@ -624,6 +624,11 @@ def dec_plan(M: int, N: int, K: int, silu: bool = False) -> tuple | None:
         tiles = N // (16 * nwv * ntw)
         if tiles >= ncu:
             return None
+        # too wide for two K-ranges and too narrow for the chip: the units dealt evenly to all CUs, 2-3 a workgroup (K 3584, us of
+        # one workgroup a tile / of these: N 18944 (148 tiles) 1 row 39.2 / 33.2, 32 36.6 / 34.8, 64 40.8 / 39.0, 128 51.8 / 48.6;
+        # N 23552 (184) 38.1 / 35.8, 39.1 / 36.7, 44.6 / 42.5, 55.2 / 52.2; N 28672 (224) 41.3 / 42.8, 44.1 / 44.4, 47.6 / 47.5)
+        if 2 * tiles > ncu and 5 * tiles <= 4 * ncu:
+            return mt, nwv, ntw, 1, ncu
         return mt, nwv, ntw, dec_ksplit(K, max(1, ncu // tiles))
     if M <= 192:
         if deep:

@@ -1,0 +1,25 @@
+"""Decode products whose column tiles are more than half the CUs and too few for all (ops/gemm.py dec_plan: their units dealt
+evenly to every CU) against fp64: the narrowest and the widest such product of the chip, 1 to 128 rows, one 64-deep round of K and
+several."""
+import pytest
+import torch
+
+from githubrepostorag_amd.ops.gemm import _num_cus, dec_plan, gemm_decode
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("K", [256, 1280])
+@pytest.mark.parametrize("M", [1, 17, 64, 128])
+@pytest.mark.parametrize("wide", [False, True])
+def test_dealt(dev, wide, M, K):
+    ncu = _num_cus()
+    N = 128 * (4 * ncu // 5 if wide else ncu // 2 + 1)
+    assert dec_plan(M, N, K)[3:] == (1, ncu)
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    x = torch.randn(M, K, generator=g, device=dev).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).bfloat16()
+    b = torch.randn(N, generator=g, device=dev).bfloat16()
+    want = x.double() @ w.double().T + b.double()
+    # the result's rounding to bf16's 8 bits, and fp32 sums of K products of about 1 / sqrt(K) each
+    assert ((gemm_decode(x, w, b).double() - want).abs() <= 2 ** -8 * want.abs() + 1e-5).all()
