@@ -1121,11 +1121,14 @@ __global__ __launch_bounds__(64) void paged_decode_prefix_kernel(AttnParams p) {
 //   * NW waves share one (sequence, kv head, split) and take its 32-key tiles round robin, each wave with
 //     its own 2-stage LDS-DMA ring (the single-wave kernel's body), so a split keeps NW tiles in flight and
 //     the split count -- the number of partials to merge -- drops NW-fold for the same parallelism;
-//   * the waves' (m, l, O) merge in LDS (the rings' space, after a barrier);
+//   * the waves' (m, l, O) merge in LDS (the rings' space, after a barrier), four dims a thread;
 //   * the splits of one (sequence, kv head) merge IN this launch: each workgroup writes its partial, takes
 //     an agent-scope ticket (release fence first, as gemm_stream.hip's split tiles), and the last arriver
 //     (acquire) reads the others' partials and writes the output; it resets its counter, so the launch
-//     replays inside hipGraphs without a memset.  No second kernel, no partial round trip for the others.
+//     replays inside hipGraphs without a memset.  No second kernel, no partial round trip for the others.  Its threads take
+//     four dims of a row each, and all splits' partials in one round trip for every eight: a value at a time, with the
+//     weights formed in between, the two merges were 6.1 of one sequence's 14.6 us (1100 keys, 9 parts); a decode step
+//     of one 530 -> 517 us, of three 3000-key ones at 12 / 2 heads 605 -> 547.
 //
 // FR (the RoPE pass folded in, ops/attention.py paged_decode_mw_rope): the workgroup forms its G q heads from
 // the qkv projection's split-K planes (sum in plane order, bias, NeoX RoPE: the values qkv_rope_kernel<true>
@@ -1149,6 +1152,18 @@ __device__ __forceinline__ f32x4_t rq_load4(const AttnParams& p, int t, int col)
     for (int r = 0; r < 4; ++r) x[r] = bits2f(f2bits(x[r] + bits2f(b[r])));
   }
   return x;
+}
+
+// four values of token `tok`'s output row, in one store where the caller's rows are aligned for it
+__device__ __forceinline__ void store_row4(const AttnParams& p, int tok, size_t at, f32x4_t v) {
+  bf16* op = p.out + (size_t)tok * p.out_stride + at;
+  const bf16x4_t b = bf16x4_t{f2bits(v[0]), f2bits(v[1]), f2bits(v[2]), f2bits(v[3])};
+  if (((uintptr_t)op & 7) == 0) {
+    *reinterpret_cast<bf16x4_t*>(op) = b;
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) op[r] = __builtin_bit_cast(bf16, (short)b[r]);
+  }
 }
 
 template <int D, int NW, bool FR>
@@ -1281,39 +1296,42 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_mw_kernel(AttnParams p, 
 
   // ---- the waves' states merge in LDS (the rings are free once every wave passed the barrier)
   __syncthreads();
-  float* so = reinterpret_cast<float*>(smem);  // [NW][16 rows][D]: lane (li, h4) holds O[row li][16 n + 4 h4 + r]
+  // [NW][16 rows][D], a row's 16-byte chunks turned by the row (lanes of a wave write the same chunk of 16 rows)
+  float* so = reinterpret_cast<float*>(smem);
   float* sml = so + NW * 16 * D;               // [NW][16][2]: (m, l)
   unsigned* flag = reinterpret_cast<unsigned*>(sml + NW * 32);
 #pragma unroll
   for (int n = 0; n < ND; ++n)
-    *reinterpret_cast<f32x4_t*>(so + (w * 16 + li) * D + 16 * n + 4 * h4) = o[n];
+    *reinterpret_cast<f32x4_t*>(so + (w * 16 + li) * D + (((4 * n + h4) ^ (li & 7)) << 2)) = o[n];
   if (h4 == 0) {
     sml[(w * 16 + li) * 2] = m;
     sml[(w * 16 + li) * 2 + 1] = lsum;
   }
   __syncthreads();
   const bool single = nvalid <= 1;
-  for (int idx = threadIdx.x; idx < G * D; idx += 64 * NW) {
-    const int row = idx / D, d = idx % D;
+  const size_t parts = (size_t)p.total_q * p.Hq;  // rows of a split's partials
+  for (int idx = threadIdx.x; idx < G * (D / 4); idx += 64 * NW) {  // four dims of a row a thread
+    const int row = idx / (D / 4), c = idx % (D / 4);
     float M = -INFINITY;
 #pragma unroll
     for (int wv = 0; wv < NW; ++wv) M = fmaxf(M, sml[(wv * 16 + row) * 2]);
-    float L = 0.f, acc = 0.f;
+    float L = 0.f;
+    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
     if (M != -INFINITY) {
 #pragma unroll
       for (int wv = 0; wv < NW; ++wv) {
         const float wt = exp2f(sml[(wv * 16 + row) * 2] - M);
         L += sml[(wv * 16 + row) * 2 + 1] * wt;
-        acc += so[(wv * 16 + row) * D + d] * wt;
+        acc += *reinterpret_cast<const f32x4_t*>(so + (wv * 16 + row) * D + ((c ^ (row & 7)) << 2)) * wt;
       }
     }
-    const int head = kvh * G + row;
+    const size_t head = kvh * G + row;
     if (single) {
-      p.out[(size_t)tok * p.out_stride + (size_t)head * D + d] = f2bf(L > 0.f ? acc / L : 0.f);
+      store_row4(p, tok, head * D + 4 * c, acc * (L > 0.f ? 1.f / L : 0.f));
     } else {
-      const size_t base = ((size_t)split * p.total_q + tok) * p.Hq + head;
-      p.part_o[base * D + d] = acc;
-      if (d == 0) {
+      const size_t base = split * parts + (size_t)tok * p.Hq + head;
+      *reinterpret_cast<f32x4_t*>(p.part_o + base * D + 4 * c) = acc;
+      if (c == 0) {
         p.part_ml[base * 2] = M;
         p.part_ml[base * 2 + 1] = L;
       }
@@ -1340,47 +1358,37 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_mw_kernel(AttnParams p, 
   }
   __syncthreads();
   if (flag[0] == 0u) return;
-  // last arriver: every split's (m, l) of the G rows staged in LDS in one parallel pass, the per-split
-  // weights formed once per row, then ONE pass over the partial O vectors (independent loads per thread)
-  float* wm = reinterpret_cast<float*>(smem);  // [nvalid][16]: m, then the split's weight
-  float* wl = wm + nvalid * 16;                // [nvalid][16]: l
-  float* rowL = wl + nvalid * 16;              // [16]
-  for (int e = threadIdx.x; e < nvalid * 16; e += 64 * NW) {
-    const int sp = e >> 4, row = e & 15;
-    float mv = -INFINITY, lv = 0.f;
-    if (row < G) {
-      const size_t base = (((size_t)sp * p.total_q + tok) * p.Hq + kvh * G + row) * 2;
-      mv = p.part_ml[base];
-      lv = p.part_ml[base + 1];
+  // last arriver: four dims of a row a thread, the partials and (m, l) of kAt splits in one round trip
+  constexpr int kAt = 8;
+  for (int idx = threadIdx.x; idx < G * (D / 4); idx += 64 * NW) {
+    const int row = idx / (D / 4), c = idx % (D / 4);
+    const size_t base = (size_t)tok * p.Hq + kvh * G + row;
+    float M = -INFINITY, L = 0.f;
+    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < nvalid; s0 += kAt) {
+      f32x4_t x[kAt];
+      float2 ml[kAt];
+#pragma unroll
+      for (int i = 0; i < kAt; ++i) {
+        const size_t r = min(s0 + i, nvalid - 1) * parts + base;
+        x[i] = *reinterpret_cast<const f32x4_t*>(p.part_o + r * D + 4 * c);
+        ml[i] = *reinterpret_cast<const float2*>(p.part_ml + r * 2);
+      }
+      float top = M;
+#pragma unroll
+      for (int i = 0; i < kAt; ++i) top = fmaxf(top, ml[i].x);  // (the last split's again past the end: no other maximum)
+      const float mu = top == -INFINITY ? 0.f : top, keep = exp2f(M - mu);
+      M = top;
+      L *= keep;
+      acc *= keep;
+#pragma unroll
+      for (int i = 0; i < kAt; ++i) {
+        const float wt = s0 + i < nvalid ? exp2f(ml[i].x - mu) : 0.f;
+        L = fmaf(ml[i].y, wt, L);
+        acc += x[i] * wt;
+      }
     }
-    wm[e] = mv;
-    wl[e] = lv;
-  }
-  __syncthreads();
-  if (threadIdx.x < 16) {
-    const int row = threadIdx.x;
-    float M = -INFINITY;
-    for (int sp = 0; sp < nvalid; ++sp) M = fmaxf(M, wm[sp * 16 + row]);
-    const float Mu = M == -INFINITY ? 0.f : M;
-    float L = 0.f;
-    for (int sp = 0; sp < nvalid; ++sp) {
-      const float wt = exp2f(wm[sp * 16 + row] - Mu);
-      wm[sp * 16 + row] = wt;
-      L += wl[sp * 16 + row] * wt;
-    }
-    rowL[row] = L;
-  }
-  __syncthreads();
-  for (int idx = threadIdx.x; idx < G * D; idx += 64 * NW) {
-    const int row = idx / D, d = idx % D;
-    const int head = kvh * G + row;
-    const float* po = p.part_o + ((size_t)tok * p.Hq + head) * D + d;
-    const size_t sstride = (size_t)p.total_q * p.Hq * D;
-    float acc = 0.f;
-#pragma unroll 8
-    for (int sp = 0; sp < nvalid; ++sp) acc += po[sp * sstride] * wm[sp * 16 + row];
-    const float L = rowL[row];
-    p.out[(size_t)tok * p.out_stride + (size_t)head * D + d] = f2bf(L > 0.f ? acc / L : 0.f);
+    store_row4(p, tok, (size_t)(kvh * G + row) * D + 4 * c, acc * (L > 0.f ? 1.f / L : 0.f));
   }
 }
 

@@ -31,7 +31,7 @@ def check(q, kc, vc, m, got):
     want = A.paged_attention_ref(q.float(), kc, vc, m, q.shape[2] ** -0.5)
     size = A.paged_attention_ref(q.float(), kc, vc.abs(), m, q.shape[2] ** -0.5)
     # the weights and the result are rounded to bf16's 8 bits: at most 2^-8 of each; 1.05 for fp32's sums and exponents
-    assert ((got.view_as(want).float() - want).abs() <= 1.05 * 2 ** -8 * (want.abs() + size)).all()
+    assert ((got.reshape(want.shape).float() - want).abs() <= 1.05 * 2 ** -8 * (want.abs() + size)).all()
 
 
 def split(m, H, D, dev, n, most):
@@ -94,3 +94,20 @@ def test_few_parts_take_the_merging_kernel(dev, seqs, takes):
     assert A.decode_mw_takes(m, G) == takes
     check(q, kc, vc, m, A.paged_attention(q, kc, vc, m, D ** -0.5))
     assert int(A.decode_counters(dev)[: seqs * G].abs().sum()) == 0
+
+
+@pytest.mark.parametrize("n", [0, 128])
+def test_rows_of_any_alignment(dev, n):
+    """The merging kernel's output rows at strides and offsets that no 8-byte store takes; 3, 9 and 17 parts."""
+    D, H, G = 64, 14, 2
+    lens, nb, rows = [300, 1100, 2100], 0, []
+    for c in lens:
+        rows.append((list(range(nb, nb + -(-c // 16))), c))
+        nb += -(-c // 16)
+    q, kc, vc, m = batch(dev, rows, nb, H, G, D, 16, n)
+    split(m, H, D, dev, n, max(lens))
+    m.extra = {"decode_nw": 24}
+    A.decode_counters(dev)
+    out = torch.zeros(3, H * D + 3, dtype=torch.bfloat16, device=dev)
+    check(q, kc, vc, m, A.paged_attention(q, kc, vc, m, D ** -0.5, out=out[:, 1:H * D + 1]))
+    assert not out[:, 0].any() and not out[:, H * D + 1:].any()
