@@ -338,9 +338,13 @@ __global__ __launch_bounds__(64 * NW, D <= 64 && NW == 4 ? 4 : 1) void attn_fwd_
 // 3 runs the staggered ping-pong schedule described at its loop (two barrier
 // intervals per tile, waves 4-7 one interval behind).  Barriers are raw
 // s_barrier: __syncthreads() would drain the younger tile with a vmcnt(0).
-template <int D, int RPW, int NS, int NW = 8>
-__global__ __launch_bounds__(64 * NW) void attn_prefill_kernel(AttnParams p) {
+//
+// TEAMS = 2 (few walks for the chip): two teams of NW waves take the tiles of the same rows in turn, each with its own
+// ring, and meet at the end.
+template <int D, int RPW, int NS, int NW = 8, int TEAMS = 1>
+__global__ __launch_bounds__(64 * NW * TEAMS) void attn_prefill_kernel(AttnParams p) {
   static_assert(NS == 2 || NW == 8, "the staggered schedule pairs waves w and w + 4 on one SIMD");
+  static_assert(TEAMS == 1 || (TEAMS == 2 && NS == 2 && RPW == 1), "two teams: 16-row waves");
   constexpr int RB = 2 * D;            // bytes per K/V row
   constexpr int CPR = D / 8;           // 16-B chunks per row
   constexpr int NC = D / 32;
@@ -354,10 +358,12 @@ __global__ __launch_bounds__(64 * NW) void attn_prefill_kernel(AttnParams p) {
   constexpr int MAXB = kPrefillMaxBlocks;  // block-table window in LDS (32 K keys)
   static_assert(PPW >= 1 && PPW * NW == NP, "piece split");
   static_assert(NS == 2 || NS == 3, "ring stages");
-  __shared__ __attribute__((aligned(16))) char smem[NS * 2 * TILE + MAXB * 4];
-  int* bt_lds = reinterpret_cast<int*>(smem + NS * 2 * TILE);
+  __shared__ __attribute__((aligned(16))) char all_lds[TEAMS * NS * 2 * TILE + MAXB * 4];
+  int* bt_lds = reinterpret_cast<int*>(all_lds + TEAMS * NS * 2 * TILE);
 
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * NW));
+  const int lane = threadIdx.x & 63, wave = TEAMS == 1 ? threadIdx.x >> 6 : (threadIdx.x >> 6) & (NW - 1);
+  char* smem = all_lds + team * NS * 2 * TILE;
   const int h4 = lane >> 4, li = lane & 15;
   // the tiles of all sequences and kv heads, longest walks first; turned by one from tile to tile, so that no XCD (the workgroups'
   // number modulo 8) is left with the sequences that have no such tile: 7 sequences of 8192 tokens, 28 / 4 heads, 153 -> 140 us
@@ -380,7 +386,7 @@ __global__ __launch_bounds__(64 * NW) void attn_prefill_kernel(AttnParams p) {
   // pieces in flight.  The launcher guarantees bt_stride <= MAXB.
   const int nb = (kv_hi + BS - 1) / BS;
   const int32_t* bt = p.block_tables + (size_t)seq * p.bt_stride;
-  for (int i = threadIdx.x; i < nb; i += 64 * NW) {
+  for (int i = threadIdx.x; i < nb; i += 64 * NW * TEAMS) {
     int b = bt[i];
     if (!index_ok(b, p.nblocks, ERR_BLOCK_PREFILL)) b = 0;  // reported; block 0 read instead of faulting
     bt_lds[i] = b;
@@ -560,15 +566,35 @@ __global__ __launch_bounds__(64 * NW) void attn_prefill_kernel(AttnParams p) {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  issue(0, 0);
+  if (team < ntiles) issue(team * KT, 0);
   if constexpr (NS == 2) {
-    for (int t = 0; t < ntiles; ++t) {
+    for (int i = 0; i * TEAMS < ntiles; ++i) {
+      const int t = i * TEAMS + team;
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       bar();
-      if (t + 1 < ntiles) issue((t + 1) * KT, (t + 1) & 1);
-      const char* k_lds = smem + (t & 1) * 2 * TILE;
+      if (t + TEAMS < ntiles) issue((t + TEAMS) * KT, (i + 1) & 1);
+      if (TEAMS > 1 && t >= ntiles) continue;  // (the last round's second team)
+      const char* k_lds = smem + (i & 1) * 2 * TILE;
       phaseA(t * KT, k_lds);
       phaseB(k_lds + TILE);
+    }
+    if constexpr (TEAMS > 1) {  // the second team's sums through the rings, lane by lane, to the first
+      static_assert(NW * (ND + 1) * 1024 <= TEAMS * NS * 2 * TILE, "exchange");
+      f32x4_t* x = reinterpret_cast<f32x4_t*>(all_lds) + wave * (ND + 1) * 64 + lane;
+      __syncthreads();
+      if (team == 1) {
+#pragma unroll
+        for (int n = 0; n < ND; ++n) x[n * 64] = o[0][n];
+        x[ND * 64] = f32x4_t{m[0], lsum[0], 0.f, 0.f};
+      }
+      __syncthreads();
+      if (team == 1) return;
+      const f32x4_t y = x[ND * 64];
+      const float top = fmaxf(m[0], y[0]), tu = top == -INFINITY ? 0.f : top;
+      const float wa = __builtin_amdgcn_exp2f(m[0] - tu), wb = __builtin_amdgcn_exp2f(y[0] - tu);
+      lsum[0] = lsum[0] * wa + y[1] * wb;
+#pragma unroll
+      for (int n = 0; n < ND; ++n) o[0][n] = o[0][n] * wa + x[n * 64] * wb;
     }
   } else {
     // Staggered ping-pong over a 3-stage ring (cdna guide "Two waves per SIMD"): waves 4-7 run one
@@ -1456,12 +1482,12 @@ int launch_decode_prefix(const AttnParams& prm, int n_items, int rg, hipStream_t
   return (int)hipGetLastError();
 }
 
-template <int D, int RPW, int NS, int NW>
+template <int D, int RPW, int NS, int NW, int TEAMS = 1>
 int launch_prefill_rows(const AttnParams& prm_in, int nseq, int max_q_len, hipStream_t stream) {
   constexpr int ROWS = 16 * RPW * NW;
   AttnParams prm = prm_in;
   prm.tiles_per_seq = (max_q_len * prm.G + ROWS - 1) / ROWS;
-  attn_prefill_kernel<D, RPW, NS, NW><<<dim3(nseq * prm.tiles_per_seq, prm.Hkv), 64 * NW, 0, stream>>>(prm);
+  attn_prefill_kernel<D, RPW, NS, NW, TEAMS><<<dim3(nseq * prm.tiles_per_seq, prm.Hkv), 64 * NW * TEAMS, 0, stream>>>(prm);
   return (int)hipGetLastError();
 }
 
@@ -1475,6 +1501,10 @@ template <int D>
 int launch_prefill(const AttnParams& prm, int nseq, int max_q_len, int nw, hipStream_t stream) {
   if (nw == 6) return launch_prefill_rows<D, 2, 3, 8>(prm, nseq, max_q_len, stream);
   const long wgs = ((long)prm.total_q * prm.G + 255) / 256 * prm.Hkv;
+  // two teams of waves on a walk where a CU gets one such workgroup at most; one / two: 1187 x 1 (56) 29.1 / 21.5, 2048 x 1 (96)
+  // 46.6 / 32.7, 2048 x 4 (96) 25.8 / 22.6, 3600 x 12 (170) 21.8 / 31.1; 28 / 4 heads 600 x 1 (68) 17.7 / 14.0, 1000 x 2 (112) 21.3 /
+  // 19.2, 1500 x 1 (168) 37.9 / 43.1
+  if (wgs <= 120) return launch_prefill_rows<D, 1, 2, 4, 2>(prm, nseq, max_q_len, stream);
   if (wgs <= 200) return launch_prefill_rows<D, 1, 2, 4>(prm, nseq, max_q_len, stream);
   if (wgs <= 280) return launch_prefill_rows<D, 1, 2, 8>(prm, nseq, max_q_len, stream);
   return launch_prefill_rows<D, 2, 2, 8>(prm, nseq, max_q_len, stream);

@@ -15,7 +15,7 @@
 // (the compiler's wait before the transposed reads), took 445 k cycles at 2.09 GHz; this takes 356 k at 1.95: matrix cores 45 %,
 // vector instructions 46 %, LDS 15 % of them.  The order of the walks, longest first over all portions and heads, is worth 5 to 9 %
 // (busy CUs 83 -> 93 % of the time).  Measured, us, before -> after: window 219 -> 200, capped 265 -> 239, blocks of 1024
-// 131 -> 121, all keys 7 x 8192 tokens 163 -> 148, 1 x 8192 710 -> 641, 3 x 2405 56 -> 50; 12 / 2 heads 1 x 1187 38 -> 35.
+// 131 -> 121, all keys 7 x 8192 tokens 163 -> 148, 1 x 8192 710 -> 641, 3 x 2405 56 -> 50; 12 / 2 heads 1 x 1187 38 -> 25.
 #include "sink.h"
 
 GRAG_ERR_UNIT(sink_prefill)
@@ -38,8 +38,9 @@ template <int D, int MR> __device__ __forceinline__ int sp_pswz(int row) {
 }
 
 // MR: rows a wave, the matrix instruction's width (16 x 16 x 32 or 32 x 32 x 16)
-template <int D, bool CAP, int MR>
-__global__ void __launch_bounds__(256, MR == 32 ? 2 : 4) sink_prefill_kernel(const SinkArgs p) {
+// TEAMS: 4 waves each, that walk the tiles of the same rows in turn
+template <int D, bool CAP, int MR, int TEAMS>
+__global__ void __launch_bounds__(256 * TEAMS, MR == 32 || TEAMS > 1 ? 2 : 4) sink_prefill_kernel(const SinkArgs p) {
   constexpr int NW = 4, KD = 512 / MR, AR = MR * MR / 64;  // waves; a product's depth, its results a lane
   constexpr int RB = 2 * D, CPR = D / 8, NC = D / KD, ND = D / MR, NT = SP_KT / MR, TILE = SP_KT * RB;
   constexpr int ROWS = MR * NW, PPW = TILE / 1024 / NW, RPP = 1024 / RB;
@@ -50,9 +51,11 @@ __global__ void __launch_bounds__(256, MR == 32 ? 2 : 4) sink_prefill_kernel(con
   };
   static_assert(PPW * RPP == SP_BS, "a wave's DMA rows sit in one cache block");
   // (one array: beside a second one the compiler waits for the DMA in flight before every tile's reads)
-  __shared__ __attribute__((aligned(16))) char smem[2 * 2 * TILE + 4 * SP_MAXB];
-  int* bt_lds = reinterpret_cast<int*>(smem + 2 * 2 * TILE);
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __shared__ __attribute__((aligned(16))) char all_lds[TEAMS * 2 * 2 * TILE + 4 * SP_MAXB];
+  int* bt_lds = reinterpret_cast<int*>(all_lds + TEAMS * 2 * 2 * TILE);
+  const int lane = threadIdx.x & 63, team = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & (NW - 1));
+  char* smem = all_lds + team * 2 * 2 * TILE;
   const int hh = lane / MR, li = lane % MR;  // this lane's row is li; its keys (and head numbers) are 8 i + 4 hh + 0..3
   // the walks of all portions and kv heads, longest first; turned by one from tile to tile, so that no XCD (the workgroups' number
   // modulo 8) is left with the portions that have no such tile
@@ -72,7 +75,7 @@ __global__ void __launch_bounds__(256, MR == 32 ? 2 : 4) sink_prefill_kernel(con
   const int kb = nkeep * (SP_KT / SP_BS), skip = kfirst / SP_BS - kb;
   const int nb = min((kv_hi + SP_BS - 1) / SP_BS - skip, SP_MAXB);
   const int* bt = p.bt + (size_t)seq * p.bt_stride;
-  for (int i = threadIdx.x; i < nb; i += 64 * NW) {
+  for (int i = threadIdx.x; i < nb; i += 64 * NW * TEAMS) {
     int b = bt[i < kb ? i : i + skip];
     if (!index_ok(b, p.nblocks, ERR_BLOCK_PREFILL)) b = 0;  // reported; block 0 read instead of faulting
     bt_lds[i] = b;
@@ -88,7 +91,9 @@ __global__ void __launch_bounds__(256, MR == 32 ? 2 : 4) sink_prefill_kernel(con
   const int lim = valid ? min(kv_hi, pos0 + pq + 1) : 0, low = sp_first(p, pos0 + pq);
   const float sc = p.scale * (p.hscale ? p.hscale[head] : 1.f);
   const bool pre = p.hscale || !(p.scale > 0.f);  // scores scaled before the mask and the maximum, else in the exponent's fma
-  float m = p.sinks[head] * LOG2E, lsum = hh == 0 ? 1.f : 0.f;  // the maximum starts at the sink, whose weight is 1 of the sum
+  // the maximum starts at the sink, whose weight is 1 of the sum (of the first team's; the others only need a number)
+  float m = p.sinks[head] * LOG2E, lsum = hh == 0 && team == 0 ? 1.f : 0.f;
+  if (team > 0) m = fmaxf(m, -1e30f);
   bf16x8_t qf[NC];
   const bf16* qp = p.q + ((size_t)tok * p.H + head) * D + 8 * hh;
 #pragma unroll
@@ -112,13 +117,13 @@ __global__ void __launch_bounds__(256, MR == 32 ? 2 : 4) sink_prefill_kernel(con
     return left < 0 ? last_slot : left;
   };
   auto base = [&](int blk) { return ((size_t)blk * p.G + kvh) * SP_BS * D; };
-  auto dma_k = [&](int i, size_t at, int most, int t) {
+  auto dma_k = [&](int i, size_t at, int most, int buf) {
     const int r = i * RPP + lrow;
-    sp_dma_s(p.k + at, min(r, most) * RB + ((lch ^ sp_kswz<D>(r)) << 4), smem + (t & 1) * 2 * TILE + (wave * PPW + i) * 1024);
+    sp_dma_s(p.k + at, min(r, most) * RB + ((lch ^ sp_kswz<D>(r)) << 4), smem + (buf & 1) * 2 * TILE + (wave * PPW + i) * 1024);
   };
-  auto dma_v = [&](int i, size_t at, int most, int t) {
+  auto dma_v = [&](int i, size_t at, int most, int buf) {
     const int r = i * RPP + lrow;
-    sp_dma_s(p.v + at, min(r, most) * RB + ((lch ^ sp_pswz<D, MR>(r)) << 4), smem + (t & 1) * 2 * TILE + TILE + (wave * PPW + i) * 1024);
+    sp_dma_s(p.v + at, min(r, most) * RB + ((lch ^ sp_pswz<D, MR>(r)) << 4), smem + (buf & 1) * 2 * TILE + TILE + (wave * PPW + i) * 1024);
   };
   acc_t o[ND];
 #pragma unroll
@@ -231,32 +236,33 @@ __global__ void __launch_bounds__(256, MR == 32 ? 2 : 4) sink_prefill_kernel(con
   // CU wait for each other's)
   size_t vat;
   {
-    const int b0 = __builtin_amdgcn_readfirstlane(table(0)), b1 = __builtin_amdgcn_readfirstlane(table(1));
+    const int t0 = team, t1 = team + TEAMS;
+    const int b0 = __builtin_amdgcn_readfirstlane(table(t0)), b1 = __builtin_amdgcn_readfirstlane(table(t1));
 #pragma unroll
-    for (int i = 0; i < PPW; ++i) dma_k(i, base(b0), slots(0), 0);
+    for (int i = 0; i < PPW; ++i) dma_k(i, base(b0), slots(t0), 0);
 #pragma unroll
-    for (int i = 0; i < PPW; ++i) dma_v(i, base(b0), slots(0), 0);
+    for (int i = 0; i < PPW; ++i) dma_v(i, base(b0), slots(t0), 0);
     vat = base(b1);
 #pragma unroll
-    for (int i = 0; i < PPW; ++i) dma_k(i, vat, slots(1), 1);
+    for (int i = 0; i < PPW; ++i) dma_k(i, vat, slots(t1), 1);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PPW) : "memory");  // K of tile 0
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   }
-  for (int t = 0; t < ntiles; ++t) {
-    const int kt0 = start(t);
-    const char* k_lds = smem + (t & 1) * 2 * TILE;
-    const bool sees = kt0 < lim_max && (kt0 + SP_KT > low_min || kt0 < p.keep);  // a row of the wave, a key of the tile
-    const int nblk = table(t + 2);
+  for (int j = 0; j * TEAMS < ntiles; ++j) {
+    const int t = j * TEAMS + team, kt0 = start(t);
+    const char* k_lds = smem + (j & 1) * 2 * TILE;
+    const bool sees = t < ntiles && kt0 < lim_max && (kt0 + SP_KT > low_min || kt0 < p.keep);  // a row of the wave, a key of the tile
+    const int nblk = table(t + 2 * TEAMS);
     if (sees) scores(kt0, k_lds);
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     const size_t kat = base(__builtin_amdgcn_readfirstlane(nblk));
-    const int kmost = slots(t + 2), vmost = slots(t + 1);
+    const int kmost = slots(t + 2 * TEAMS), vmost = slots(t + TEAMS);
     if (!sees) {
 #pragma unroll
-      for (int i = 0; i < PPW; ++i) dma_v(i, vat, vmost, t + 1), dma_k(i, kat, kmost, t);
+      for (int i = 0; i < PPW; ++i) dma_v(i, vat, vmost, j + 1), dma_k(i, kat, kmost, j);
       vat = kat;
       continue;
     }
@@ -274,7 +280,7 @@ __global__ void __launch_bounds__(256, MR == 32 ? 2 : 4) sink_prefill_kernel(con
         o[n] = mma(vf[u & 1][n], ph[u & 1], o[n]);
       }
 #pragma unroll
-      for (int i = u * PPW / NP; i < (u + 1) * PPW / NP; ++i) dma_v(i, vat, vmost, t + 1), dma_k(i, kat, kmost, t);
+      for (int i = u * PPW / NP; i < (u + 1) * PPW / NP; ++i) dma_v(i, vat, vmost, j + 1), dma_k(i, kat, kmost, j);
       if (u + 1 < NP) {
         weights(u + 1);
 #pragma unroll
@@ -290,6 +296,23 @@ __global__ void __launch_bounds__(256, MR == 32 ? 2 : 4) sink_prefill_kernel(con
     vat = kat;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if constexpr (TEAMS > 1) {  // the second team's sums through the buffers, lane by lane, to the first
+    static_assert(TEAMS == 2 && AR == 4 && NW * (ND + 1) * 1024 <= 2 * 2 * 2 * TILE, "exchange");
+    f32x4_t* x = reinterpret_cast<f32x4_t*>(all_lds) + wave * (ND + 1) * 64 + lane;
+    __syncthreads();
+    if (team == 1) {
+#pragma unroll
+      for (int n = 0; n < ND; ++n) x[n * 64] = o[n];
+      x[ND * 64] = f32x4_t{m, lsum, 0.f, 0.f};
+    }
+    __syncthreads();
+    if (team == 1) return;
+    const f32x4_t y = x[ND * 64];
+    const float top = fmaxf(m, y[0]), a = __builtin_amdgcn_exp2f(m - top), b = __builtin_amdgcn_exp2f(y[0] - top);
+    lsum = lsum * a + y[1] * b;
+#pragma unroll
+    for (int n = 0; n < ND; ++n) o[n] = o[n] * a + x[n * 64] * b;
+  }
   if constexpr (MR == 16) lsum += __shfl_xor(lsum, 16, 64);
   lsum += __shfl_xor(lsum, 32, 64);
   if (!valid) return;
@@ -333,15 +356,20 @@ hipError_t sink_prefill_launch(const void* q, const void* k, const void* v, void
   // 110 / 136; 28 / 4 heads, 1500 x 1 (329) 56.2 / 46.9, 2048 x 1 (448) 65.3 / 72.0, 2048 x 4 (448) 42.3 / 36.5, 3000 x 8 (657)
   // 35.1 / 45.6; window 1024, 12 / 2 heads, 4000 x 2 (375) 54.0 / 64.1.
   long tiles = ((long)max_q_len * a.R + 127) / 128;
-  const bool few = ((long)rows * a.R + 127) / 128 * G <= 340;
+  const long wgs = ((long)rows * a.R + 127) / 128 * G;
+  // and where those are a CU's at most, two teams of 4 waves that take the walk's tiles in turn: one / two, 600 x 1 (57) 19.5 /
+  // 15.7, 1187 x 1 (112) 35.1 / 24.6, 2048 x 1 (192) 53.2 / 38.8, 2048 x 4 (192) 31.0 / 26.0, 3600 x 1 (338) 89.7 / 97.2; 28 / 4
+  // heads 600 x 1 (132) 21.4 / 16.0, 1000 x 3 (219) 16.8 / 19.3.
+  const bool few = wgs <= 340, teams = wgs <= 200;
   if (few) tiles = ((long)max_q_len * a.R + 63) / 64;
   if (tiles * nseq * G > 0x7fffffffL - (tiles > 0 ? tiles : 0)) return hipErrorInvalidValue;
   a.tiles = (int)tiles, a.nseq = nseq;
   const dim3 grid((unsigned)(tiles * nseq * G));
-#define SINK_PREFILL(DD, CAP)                                                                                        \
-  {                                                                                                                  \
-    if (few) hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 16>), grid, dim3(256), 0, st, a);                      \
-    else hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 32>), grid, dim3(256), 0, st, a);                          \
+#define SINK_PREFILL(DD, CAP)                                                                                           \
+  {                                                                                                                     \
+    if (teams) hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 16, 2>), grid, dim3(512), 0, st, a);                    \
+    else if (few) hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 16, 1>), grid, dim3(256), 0, st, a);                 \
+    else hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 32, 1>), grid, dim3(256), 0, st, a);                          \
   }
   if (d == 64 && softcap > 0.f) SINK_PREFILL(64, true)
   else if (d == 64) SINK_PREFILL(64, false)

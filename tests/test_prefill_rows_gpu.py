@@ -1,5 +1,5 @@
-"""Paged prefill attention by rows a workgroup (csrc/kernels/attention.hip launch_prefill: 64, 128 or 256 by all rows) against
-fp32 attention: portions that end beside a workgroup's and a wave's rows, cached tokens before some, one of one token."""
+"""Paged prefill attention by rows a workgroup (csrc/kernels/attention.hip launch_prefill: 64, with one or two teams of
+waves, 128 or 256 by all rows) against fp32 attention: portions that end beside a workgroup's and a wave's rows, cached tokens before some, one of one token."""
 import pytest
 import torch
 
@@ -9,7 +9,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("D,H,G,lens,past,wgs", [
-    (128, 28, 4, [37, 1, 300, 64], [0, 61, 0, 5], (1, 200)), (64, 12, 2, [129, 16, 640], [200, 0, 63], (1, 200)),
+    (128, 28, 4, [37, 1, 300, 64], [0, 61, 0, 5], (1, 120)), (64, 12, 2, [129, 16, 640], [200, 0, 63], (1, 120)),
+    (64, 7, 1, [1, 64], [0, 64], (1, 120)), (128, 28, 4, [600, 1, 700, 64], [0, 61, 3, 5], (121, 200)),
+    (64, 32, 8, [511, 257, 1, 300], [0, 7, 900, 0], (121, 200)),
     (128, 28, 4, [1000, 33, 1, 910], [0, 31, 64, 1], (201, 280)), (64, 32, 8, [511, 257, 1, 900], [0, 7, 900, 0], (201, 280)),
     (128, 28, 4, [1500, 17, 1201], [5, 0, 63], (281, 400)), (64, 32, 8, [1025, 700, 640, 1], [0, 1, 0, 300], (281, 400))])
 def test_rows(dev, D, H, G, lens, past, wgs):

@@ -16,9 +16,13 @@ FORMS = {"causal": {}, "window": dict(window=150), "kept": dict(window=90, keep=
 @pytest.mark.parametrize("D,H,G,lens,past", [
     (64, 24, 8, [640, 33, 1, 705, 128, 321], [0, 31, 64, 0, 1, 0]), (128, 28, 4, [1100, 16, 577, 64], [5, 0, 0, 63])])
 def test_rows(dev, D, H, G, lens, past, form):
+    assert -(-sum(lens) * (H // G) // 128) * G > 340  # the 128-row workgroups
+    check(dev, D, H, G, lens, past, form)
+
+
+def check(dev, D, H, G, lens, past, form):
     g = torch.Generator(device=dev).manual_seed(D + len(form))
-    BS, ctx, T, R = 16, [n + p for n, p in zip(lens, past)], sum(lens), H // G
-    assert -(-T * R // 128) * G > 340  # the 128-row workgroups
+    BS, ctx, T = 16, [n + p for n, p in zip(lens, past)], sum(lens)
     q0 = torch.tensor([0] + lens).cumsum(0)
     width, nb = -(-max(ctx) // BS), sum(-(-c // BS) for c in ctx)
     perm, bt, at = torch.randperm(nb, generator=torch.Generator().manual_seed(1)), torch.zeros(len(ctx), width, dtype=torch.int32), 0
@@ -43,3 +47,11 @@ def test_rows(dev, D, H, G, lens, past, form):
     assert not want.isnan().any()
     # the result's own rounding to bf16 is 2^-9; the weights reach the sums with 16 bits
     assert ((got - want).abs() <= 2 ** -8 * want.abs() + 2e-4).all(), (got - want).abs().max()
+
+
+@pytest.mark.parametrize("form", sorted(FORMS))
+@pytest.mark.parametrize("D,H,G,lens,past", [(128, 12, 2, [300, 1, 65, 16], [0, 63, 1500, 700]), (64, 14, 2, [16], [0]), (64, 6, 1, [64, 65], [64, 0])])
+def test_two_teams(dev, D, H, G, lens, past, form):
+    """Few rows: two teams of waves on a walk's tiles, of which one may have none, or none that a row sees."""
+    assert -(-sum(lens) * (H // G) // 128) * G <= 200
+    check(dev, D, H, G, lens, past, form)
