@@ -158,8 +158,8 @@ class BertEncoder:
 
     def _layers_bound(self, h, seq_start, seq_len, max_len: int):
         """_layers with every kernel chosen once and its buffers allocated once for all layers: 7 calls of about 4 us a layer, where
-        the ops one by one took 140 us of Python a layer, more than the GPU up to some 5000 tokens (24 chunks of 4200
-        tokens 1730 -> 1120 us, 16 of 1136 1690 -> 760)."""
+        the ops one by one took 140 us of Python a layer, more than the GPU up to some 5000 tokens (chunks of 1752
+        tokens in all 1737 -> 1007 us, of 60 1462 -> 764)."""
         cfg, T = self.cfg, h.shape[0]
         H, I, nh, eps = cfg.hidden_size, cfg.intermediate_size, cfg.num_heads, float(cfg.layer_norm_eps)
         new = lambda n: torch.empty(T, n, dtype=h.dtype, device=h.device)  # noqa: E731
