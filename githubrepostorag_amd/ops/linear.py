@@ -448,7 +448,9 @@ def glu_linear(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: flo
     if x.is_cuda and x.dim() == 2 and x.shape[0] >= _tile.PREFILL_MIN_M and w.shape[0] % 16 == 0:
         M, N = x.shape[0], w.shape[0]
         tiles, ncu = -(-M // 256) * -(-N // 256), _tile._num_cus()
-        if (M * N >= GLU_FILL * 65536 * ncu * -(-tiles // ncu) or _tile.pair_plan(M, N, x.shape[1], True) is not None) and _tile.supported(x, w) and _plain_product(x, w):
+        fills = M * N >= GLU_FILL * 65536 * ncu * -(-tiles // ncu)
+        small = x.shape[1] >= 256 and _tile.pair_plan(M, N, x.shape[1], True) is not None  # (shorter contractions: two launches)
+        if (fills or small) and _tile.supported(x, w) and _plain_product(x, w):
             return _tile.gemm_glu(x, w, limit, alpha, shift)
     return clamped_glu(linear(x, w), limit, alpha, shift)
 
