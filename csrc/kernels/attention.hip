@@ -903,7 +903,9 @@ __global__ __launch_bounds__(64) void paged_decode_kernel(AttnParams p) {
 }
 
 // Combine split-KV partials of decode (q_len == 1 per sequence: token == seq), and the shared-prefix parts
-// of a sequence whose first keys paged_decode_prefix_kernel covered.
+// of a sequence whose first keys paged_decode_prefix_kernel covered.  Four parts and their (m, l) come in one round trip (part
+// after part, the maximum first, each took two); with the decode kernel, us: 64 sequences of 70000 keys (4 parts) 34.3 -> 33.1,
+// 8 of 60000 (29 parts) 37.5 -> 33.7, 12 / 2 heads 24 of 60000 (17 parts) 21.9 -> 18.7; eight at a time the same.
 template <int D>
 __global__ __launch_bounds__(D) void attn_combine_kernel(AttnParams p) {
   const int tok = blockIdx.x, head = blockIdx.y, d = threadIdx.x;
@@ -912,25 +914,36 @@ __global__ __launch_bounds__(D) void attn_combine_kernel(AttnParams p) {
   int nvalid = (ctx - pre + p.split_len - 1) / p.split_len;
   nvalid = max(1, min(nvalid, p.num_splits));
   const int npre = pre > 0 ? prefix_planes(p, tok, pre) : 0;
-  float M = -INFINITY;
-  for (int s = 0; s < nvalid; ++s)
-    M = fmaxf(M, p.part_ml[(((size_t)s * p.total_q + tok) * p.Hq + head) * 2]);
-  for (int s = 0; s < npre; ++s)
-    M = fmaxf(M, p.pre_ml[(((size_t)s * p.total_q + tok) * p.Hq + head) * 2]);
-  const float Mu = M == -INFINITY ? 0.f : M;
-  float L = 0.f, acc = 0.f;
-  for (int s = 0; s < nvalid; ++s) {
-    const size_t base = ((size_t)s * p.total_q + tok) * p.Hq + head;
-    const float w = exp2f(p.part_ml[base * 2] - Mu);
-    L += p.part_ml[base * 2 + 1] * w;
-    acc += p.part_o[base * D + d] * w;
-  }
-  for (int s = 0; s < npre; ++s) {
-    const size_t base = ((size_t)s * p.total_q + tok) * p.Hq + head;
-    const float w = exp2f(p.pre_ml[base * 2] - Mu);
-    L += p.pre_ml[base * 2 + 1] * w;
-    acc += p.pre_o[base * D + d] * w;
-  }
+  const size_t row = (size_t)tok * p.Hq + head, step = (size_t)p.total_q * p.Hq;
+  float M = -INFINITY, L = 0.f, acc = 0.f;
+  auto take = [&](const float* ml, const float* o, int n) {
+    constexpr int kAt = 4;
+    for (int s0 = 0; s0 < n; s0 += kAt) {
+      float2 v[kAt];
+      float x[kAt];
+#pragma unroll
+      for (int i = 0; i < kAt; ++i) {
+        const size_t r = min(s0 + i, n - 1) * step + row;
+        v[i] = *reinterpret_cast<const float2*>(ml + r * 2);
+        x[i] = o[r * D + d];
+      }
+      float top = M;
+#pragma unroll
+      for (int i = 0; i < kAt; ++i) top = fmaxf(top, v[i].x);  // (the last part's again past the end: no other maximum)
+      const float mu = top == -INFINITY ? 0.f : top, keep = exp2f(M - mu);
+      M = top;
+      L *= keep;
+      acc *= keep;
+#pragma unroll
+      for (int i = 0; i < kAt; ++i) {
+        const float w = s0 + i < n ? exp2f(v[i].x - mu) : 0.f;
+        L = fmaf(v[i].y, w, L);
+        acc = fmaf(x[i], w, acc);
+      }
+    }
+  };
+  take(p.part_ml, p.part_o, nvalid);
+  if (npre > 0) take(p.pre_ml, p.pre_o, npre);
   p.out[(size_t)tok * p.out_stride + (size_t)head * D + d] = f2bf(L > 0.f ? acc / L : 0.f);
 }
 

@@ -355,7 +355,7 @@ def paged_decode_mw_rope(qkv, bias, positions, cos_sin, k_cache, v_cache, meta: 
     """Decode attention straight from the qkv projection's deferred split-K planes (ops/gemm.py SplitKPartial):
     the kernel forms q with bias + NeoX RoPE in registers, folds the new token's key in from registers, and stores
     the new K / V to meta.slot_mapping's slots -- what ops/elementwise.qkv_rope_kvstore + paged_attention do in
-    two launches (the small-kernel floor VERDICT r5 item 4 measured: RoPE 6.5 us of a B = 1 layer).  Returns
+    two launches (RoPE alone 6.5 us of a B = 1 layer).  Returns
     out [T, Hq * D], or None when the small-batch decode kernel would not take this step (the caller then runs
     the two-launch path)."""
     from .gemm import SplitKPartial
