@@ -83,6 +83,18 @@ def decode_counters(dev: torch.device) -> torch.Tensor:
                       lambda d: torch.zeros(1 << 16, dtype=torch.int32, device=d))
 
 
+def _decode_tickets(dev: torch.device, nsplit: int) -> torch.Tensor:
+    """The tickets of one launch of several parts: the owner's, or without one the current stream's own, since two launches on two
+    streams of a thread would count on the same words, and the first to arrive of one be taken for the last.  A capture that
+    nothing owns keeps the thread's."""
+    from .gemm import WS
+
+    own = decode_counters(dev)  # (also where it is not used: a later capture finds it)
+    if nsplit == 1 or WS.owner() is not None or torch.cuda.is_current_stream_capturing():
+        return own
+    return WS.for_stream(torch.device(dev), 0)[1]
+
+
 def decode_variant(nsplit: int, split_len: int, waves: int | None = None) -> int:
     """Decode kernel per split plan, 32-key tiles.  ``waves``: the launch's (sequence x kv-head x split) count; more than
     DECODE_NS3_WAVES of several parts over 512 rows take the 3-stage ring, at least DECODE_NT_MIN_WAVES load K/V non-temporally
@@ -320,7 +332,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                  ptr(meta.block_tables), meta.block_tables.stride(0), ptr(meta.q_start), ptr(meta.ctx_len),
                  meta.num_seqs, T, Hq, Hkv, D, BS, float(scale), nsplit, meta.split_len if nsplit > 1 else 0,
                  ptr(meta.part_o) if nsplit > 1 else None, ptr(meta.part_ml) if nsplit > 1 else None,
-                 ptr(decode_counters(q.device)), DECODE_MW[nw], k_cache.shape[0])
+                 ptr(_decode_tickets(q.device, nsplit)), DECODE_MW[nw], k_cache.shape[0])
             return out
         if nw in DECODE_MW:
             nw = decode_variant(nsplit, meta.split_len, meta.num_seqs * Hkv * nsplit)
@@ -377,7 +389,7 @@ def paged_decode_mw_rope(qkv, bias, positions, cos_sin, k_cache, v_cache, meta: 
          ptr(meta.slot_mapping), ptr(k_cache), ptr(v_cache), ptr(out), out.stride(0), ptr(meta.block_tables),
          meta.block_tables.stride(0), ptr(meta.q_start), ptr(meta.ctx_len), meta.num_seqs, qkv.M, Hq, Hkv, D, BS,
          float(scale), nsplit, meta.split_len if nsplit > 1 else 0, ptr(meta.part_o) if nsplit > 1 else None,
-         ptr(meta.part_ml) if nsplit > 1 else None, ptr(decode_counters(qkv.device)), DECODE_MW[nw],
+         ptr(meta.part_ml) if nsplit > 1 else None, ptr(_decode_tickets(qkv.device, nsplit)), DECODE_MW[nw],
          k_cache.shape[0], k_cache.shape[0] * BS, cos_sin.numel() // D)
     return out
 

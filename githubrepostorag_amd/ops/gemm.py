@@ -430,9 +430,10 @@ class _Workspace:
         return self.owner() is not None and self.ready(dev, floats) and self.has_counters(dev)
 
     def for_stream(self, dev: torch.device, floats: int) -> tuple[torch.Tensor, torch.Tensor]:
-        """(slab, tickets) of a stream-K launch that callers without an owner make, on whatever streams they use: the slab is the
-        allocator's (ordered by the current stream), the tickets the current stream's own, of the TICKET_STREAMS used last by
-        this thread.  An owner runs on one stream at a time and has its own."""
+        """(slab, tickets) of a launch that callers without an owner make, on whatever streams they use (stream-K products, the
+        decode attention's parts): the slab is the allocator's (ordered by the current stream), the tickets the current
+        stream's own, of the TICKET_STREAMS used last by this thread, zero at rest.  An owner runs on one stream at a time and
+        has its own."""
         if self.owner() is not None:
             return self.get(dev, floats), self.counters(dev)
         tab = getattr(self._tls, "tickets", None)
@@ -443,7 +444,7 @@ class _Workspace:
         if c is None:
             if len(tab) >= TICKET_STREAMS:
                 tab.pop(next(iter(tab)))
-            c = torch.zeros(1 << 14, dtype=torch.int32, device=dev)
+            c = torch.zeros(1 << 16, dtype=torch.int32, device=dev)  # (a word a tile, or a decode row and kv head)
         tab[key] = c
         return torch.empty(floats, dtype=torch.float32, device=dev), c
 
