@@ -66,10 +66,13 @@ def decode_mw_takes(meta, Hkv: int) -> bool:
     """Whether a decode step without a kernel of its own choice takes the small-batch kernel: few rows, or so few parts in all
     that the launches it saves (the combine, the RoPE pass) count for more than its 4 waves' LDS.  us without / with, RoPE pass not
     counted, sequences x keys (parts): 28 / 4 heads 8 x 1000 (128) 15.3 / 14.6, 24 x 300 (192) 14.7 / 13.3, 5 x 3000 (240) 19.9 /
-    22.5; 12 / 2 heads 16 x 300 (64) 14.4 / 11.7, 12 x 2000 (192) 17.7 / 16.1."""
+    22.5; 12 / 2 heads 16 x 300 (64) 14.4 / 11.7, 12 x 2000 (192) 17.7 / 16.1.  The latter not in a capture without an owner whose
+    tickets are there: other kernels need none."""
+    from .gemm import WS
+
     rows = meta.num_seqs * Hkv
     few = meta.cascade is None and rows * meta.num_splits <= DECODE_MW_PARTS
-    return DECODE_MW_ROWS > 0 and (rows <= DECODE_MW_ROWS or few)
+    return DECODE_MW_ROWS > 0 and (rows <= DECODE_MW_ROWS or few and WS.scratch_ok("decode_tickets"))
 
 
 def decode_counters(dev: torch.device) -> torch.Tensor:

@@ -448,6 +448,12 @@ class _Workspace:
         tab[key] = c
         return torch.empty(floats, dtype=torch.float32, device=dev), c
 
+    def scratch_ok(self, name: str) -> bool:
+        """Whether a launch that could do without may take its scratch() now: in a capture only an owner's that is there."""
+        if not (torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing()):
+            return True
+        return self.owner() is not None and torch.cuda.current_device() in self.owner().get(name, {})
+
     def scratch(self, name: str, dev: torch.device, make):
         """A persistent per-owner scratch tensor (ticket arrays, small merge buffers) under ``name``: the
         owner's (an engine's, an embedder's) while one is set, else this thread's.  Every kernel that keeps
