@@ -1529,12 +1529,12 @@ int launch_prefill(const AttnParams& prm, int nseq, int max_q_len, int nw, hipSt
 
 template <int D>
 int dispatch_nw(const AttnParams& prm, int nseq, int max_q_len, int nw, bool paged, hipStream_t stream) {
-  // nw == 1 / 3 with q_len == 1: LDS-DMA pipelined decode kernel with 64- / 32-key
+  // nw == 1 / 3 with q_len == 1 and up to 16 heads a kv head: LDS-DMA pipelined decode kernel with 64- / 32-key
   // tiles (32-key tiles halve the LDS ring so more single-wave workgroups share a
-  // CU); nw == 2: the generic kernel with one wave per workgroup (A/B reference)
+  // CU); nw == 2, and more heads: the generic kernel with one wave per workgroup
   // nw == 7 / 8: 32-key tiles in a 4- / 3-stage ring; nw == 11 / 12: 3 / 8 with non-temporal K/V loads
-  if (paged && (nw == 1 || nw == 3 || nw == 7 || nw == 8 || nw == 11 || nw == 12) && prm.tiles_per_seq == 1 &&
-      prm.G <= 16 && prm.BS % 16 == 0)
+  if (paged && (nw == 1 || nw == 3 || nw == 7 || nw == 8 || nw == 11 || nw == 12) && max_q_len == 1 && prm.G <= 16 &&
+      prm.BS % 16 == 0)
     return launch_decode<D>(prm, nseq, nw == 1 ? 64 : 32, nw == 7 ? 4 : (nw == 8 || nw == 12) ? 3 : 2,
                             nw >= 11, stream);
   if (nw == 5 || nw == 6) {  // LDS-DMA prefill: 8 waves, 2-stage (5) / staggered 3-stage (6) ring
@@ -1592,7 +1592,8 @@ GRAG_API int grag_paged_attention(const void* q, int q_stride, const void* k_cac
   // 8-wave prefill needs KV blocks of 16 and a block table that fits its LDS window; otherwise
   // the 4-wave kernel (same math) takes the launch
   if (nw >= 5 && !(BS == 16 && bt_stride <= kPrefillMaxBlocks && (D == 128 || D == 64))) nw = 4;
-  const int rows_per_wg = nw >= 5 ? 256 : 16 * (nw == 2 ? 1 : nw);  // nw 5/6: 256 GQA rows per workgroup
+  // GQA rows per workgroup: nw 5/6 256, nw 4 64, the decode codes 16 (heads past 16 of a kv head: more workgroups of the one-wave kernel)
+  const int rows_per_wg = nw == 5 || nw == 6 ? 256 : nw == 4 ? 64 : 16;
   prm.tiles_per_seq = (max_q_len * prm.G + rows_per_wg - 1) / rows_per_wg;
   if (nw == 1 && max_q_len != 1) return (int)hipErrorInvalidValue;
   prm.num_splits = num_splits < 1 ? 1 : num_splits;

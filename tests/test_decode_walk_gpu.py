@@ -59,6 +59,21 @@ def test_walk(dev, D, H, G, BS, n):
         check(q, kc, vc, m, A.paged_attention(q, kc, vc, m, D ** -0.5))
 
 
+@pytest.mark.parametrize("D,H", [(64, 32), (128, 17), (64, 80), (32, 33)])
+@pytest.mark.parametrize("n", [0, 256])
+def test_more_heads_than_a_wave_has_columns(dev, D, H, n):
+    """Past 16 query heads a kv head: several workgroups of the one-wave kernel a row, by the default choice and every code."""
+    lens, nb, rows = [1, 77, 600], 0, []
+    for c in lens:
+        rows.append((list(range(nb, nb + -(-c // 16))), c))
+        nb += -(-c // 16)
+    q, kc, vc, m = batch(dev, rows, nb, H, 1, D, 16, H)
+    split(m, H, D, dev, n, max(lens))
+    for code in (None, 1, 2, 3, 7, 8, 11, 12):
+        m.extra = {} if code is None else {"decode_nw": code}
+        check(q, kc, vc, m, A.paged_attention(q, kc, vc, m, D ** -0.5, out=torch.full((3, H * D), 9.0, device=dev).bfloat16()))
+
+
 @pytest.mark.parametrize("blocks", [9, 63, 67])
 @pytest.mark.parametrize("n", [0, 512])
 def test_behind_a_prefix(dev, blocks, n):
