@@ -1590,8 +1590,8 @@ GRAG_API int grag_paged_attention(const void* q, int q_stride, const void* k_cac
   prm.BS = BS;
   prm.bt_stride = bt_stride;
   // 8-wave prefill needs KV blocks of 16 and a block table that fits its LDS window; otherwise
-  // the 4-wave kernel (same math) takes the launch
-  if (nw >= 5 && !(BS == 16 && bt_stride <= kPrefillMaxBlocks && (D == 128 || D == 64))) nw = 4;
+  // the 4-wave kernel (same math) takes the launch.  The decode codes have no such limits
+  if ((nw == 5 || nw == 6) && !(BS == 16 && bt_stride <= kPrefillMaxBlocks && (D == 128 || D == 64))) nw = 4;
   // GQA rows per workgroup: nw 5/6 256, nw 4 64, the decode codes 16 (heads past 16 of a kv head: more workgroups of the one-wave kernel)
   const int rows_per_wg = nw == 5 || nw == 6 ? 256 : nw == 4 ? 64 : 16;
   prm.tiles_per_seq = (max_q_len * prm.G + rows_per_wg - 1) / rows_per_wg;
