@@ -936,9 +936,10 @@ __global__ __launch_bounds__(D) void attn_combine_kernel(AttnParams p) {
       acc *= keep;
 #pragma unroll
       for (int i = 0; i < kAt; ++i) {
-        const float w = s0 + i < n ? exp2f(v[i].x - mu) : 0.f;
+        const bool on = s0 + i < n;  // (its value too, not its weight alone: a part may hold infinities)
+        const float w = on ? exp2f(v[i].x - mu) : 0.f;
         L = fmaf(v[i].y, w, L);
-        acc = fmaf(x[i], w, acc);
+        acc = fmaf(on ? x[i] : 0.f, w, acc);
       }
     }
   };
@@ -1426,9 +1427,10 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_mw_kernel(AttnParams p, 
       acc *= keep;
 #pragma unroll
       for (int i = 0; i < kAt; ++i) {
-        const float wt = s0 + i < nvalid ? exp2f(ml[i].x - mu) : 0.f;
+        const bool on = s0 + i < nvalid;  // (its values too, not its weight alone: a part may hold infinities)
+        const float wt = on ? exp2f(ml[i].x - mu) : 0.f;
         L = fmaf(ml[i].y, wt, L);
-        acc += x[i] * wt;
+        acc += (on ? x[i] : f32x4_t{0.f, 0.f, 0.f, 0.f}) * wt;
       }
     }
     store_row4(p, tok, (size_t)(kvh * G + row) * D + 4 * c, acc * (L > 0.f ? 1.f / L : 0.f));

@@ -148,3 +148,18 @@ def test_rows_of_any_alignment(dev, n):
     out = torch.zeros(3, H * D + 3, dtype=torch.bfloat16, device=dev)
     check(q, kc, vc, m, A.paged_attention(q, kc, vc, m, D ** -0.5, out=out[:, 1:H * D + 1]))
     assert not out[:, 0].any() and not out[:, H * D + 1:].any()
+
+
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("code", [3, 24])
+def test_infinite_values(dev, parts, code):
+    """An infinite value in the last part stays an infinity of its sign: parts that are not there add nothing."""
+    D, H, G = 64, 6, 2
+    rows = [(list(range(8 * parts)), 128 * parts)]
+    q, kc, vc, m = batch(dev, rows, 8 * parts, H, G, D, 16, parts)
+    vc[-1, :, :, 5], vc[-1, :, :, 6] = float("inf"), float("-inf")
+    split(m, H, D, dev, 128 if parts > 1 else 0, 128 * parts)
+    m.extra = {"decode_nw": code}
+    got = A.paged_attention(q, kc, vc, m, D ** -0.5).view(H, D).float()
+    assert (got[:, 5] == float("inf")).all() and (got[:, 6] == float("-inf")).all()
+    assert got[:, [d for d in range(D) if d not in (5, 6)]].isfinite().all()
