@@ -939,9 +939,10 @@ def dec_capture_ok(dev: torch.device, M: int, N: int, K: int, silu: bool = False
     return fl == 0 or not torch.cuda.is_current_stream_capturing() or WS.ready(dev, fl)
 
 
-def capture_ok(dev: torch.device, M: int, N: int, K: int, silu: bool = False, act: int = ACT_NONE) -> bool:
-    """False only inside a hipGraph capture whose split-K slab was not sized by an eager step."""
-    if pair_plan(M, N, K, silu or act != ACT_NONE) is not None:  # (no slab)
+def capture_ok(dev: torch.device, M: int, N: int, K: int, silu: bool = False, act: int = ACT_NONE, pair: bool = True) -> bool:
+    """False only inside a hipGraph capture whose split-K slab was not sized by an eager step.  ``pair``: the operands meet
+    pair_takes(), without which a small product has schedule()'s slab."""
+    if pair and pair_plan(M, N, K, silu or act != ACT_NONE) is not None:  # (no slab)
         return True
     ks, sk = schedule(M, N, K, silu)
     fl = _ws_floats(M, N, ks, sk)
@@ -956,7 +957,8 @@ def mlp_gate_up(x: torch.Tensor, w_gu: torch.Tensor, b_gu: torch.Tensor | None =
     if x.is_cuda and (M >= 33 or dec_small(M, w_gu.shape[0], K, True)) and supported(x, w_gu) and dec_plan(M, w_gu.shape[0], K, True) is not None \
             and dec_capture_ok(x.device, M, w_gu.shape[0], K, True):
         return gemm_decode(x, w_gu, b_gu, epi=EPI_SILU)
-    if not x.is_cuda or (supported(x, w_gu) and capture_ok(x.device, M, w_gu.shape[0], K, True)):
+    if not x.is_cuda or (supported(x, w_gu)
+                         and capture_ok(x.device, M, w_gu.shape[0], K, True, pair=pair_takes(x, w_gu, b_gu))):
         return gemm_silu(x, w_gu, b_gu)
     y = torch.nn.functional.linear(x, w_gu, b_gu).view(M, -1, 2, 32)
     return (torch.nn.functional.silu(y[:, :, 0].float()) * y[:, :, 1].float()).to(x.dtype).reshape(M, -1)

@@ -398,7 +398,7 @@ def bound_product(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, act:
     def ordinary(x, w, b):
         if not act:
             return linear(x, w, b)
-        if _tile.supported(x, w) and _tile.capture_ok(x.device, M, N, K, act=act):
+        if _tile.supported(x, w) and _tile.capture_ok(x.device, M, N, K, act=act, pair=_tile.pair_takes(x, w, b)):
             return _tile.gemm(x, w, b, act=act)
         return bias_act(linear(x, w), b, act, inplace=True)
 

@@ -101,3 +101,26 @@ def test_captured_without_an_eager_step(dev):
         x.normal_()
         g.replay()
         assert torch.equal(y, G.gemm(x, w, b, act=G.ACT_GELU))
+
+
+@pytest.mark.parametrize("at", [0, 4])
+def test_gate_up_captured_with_a_bias_at_any_address(monkeypatch, at):
+    """A bias that the small tiles refuse (no multiple of 8 bytes), in a capture whose slab was not sized: the library's branch
+    and no K parts.  (On a host that launches nothing.)"""
+    from types import SimpleNamespace
+
+    M, F, K = 300, 1536, 2048  # K parts without the small tiles
+    b = torch.zeros(2 * F + 8).bfloat16()[at // 2:][:2 * F]
+    w = torch.empty(2 * F, 1).bfloat16().expand(2 * F, K)
+    x = SimpleNamespace(shape=(M, K), is_cuda=True, device=torch.device("cpu"), dtype=torch.bfloat16, stride=lambda i: K if i == 0 else 1,
+                        data_ptr=lambda: 0)
+    monkeypatch.setattr(G, "_NCU", [256])
+    monkeypatch.setattr(G, "supported", lambda *a: True)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    assert G.pair_plan(M, 2 * F, K, True) is not None and G.schedule(M, 2 * F, K, True)[0] > 1
+    took = []
+    monkeypatch.setattr(torch.nn.functional, "linear", lambda *a: took.append("library") or torch.zeros(M, 2 * F).bfloat16())
+    monkeypatch.setattr(G, "gemm_silu", lambda *a: took.append("pair" if G.pair_takes(*a) else "parts"))
+    with G.WS.owned_by({}):
+        G.mlp_gate_up(x, w, b)
+    assert took == (["library"] if at else ["pair"])
