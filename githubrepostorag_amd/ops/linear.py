@@ -284,23 +284,24 @@ def gemm_splitk(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None,
     return y.to(x.dtype)
 
 
-def kernel_for(M: int, N: int, K: int, tile_ok: bool = True, dev: torch.device | None = None) -> str:
+def kernel_for(M: int, N: int, K: int, tile_ok: bool = True, dev: torch.device | None = None, pair_ok: bool = True) -> str:
     """The kernel linear() runs a bf16 [M, K] x [N, K]^T projection on: "pair" / "decode" / "tile" / "tile_prefill"
     (owned MFMA kernels of ops/gemm.py), "skinny" / "stream" (owned weight-streaming kernels here),
     "splitk" (K-sliced library bmm) or "library" (hipBLASLt).  ``tile_ok``: the operands meet
     ops/gemm.supported (alignment, K % 64).  ``dev``: check that a hipGraph capture in progress can use
-    the split-K / stream-K workspaces (None: plan as in steady state, workspaces ready)."""
+    the split-K / stream-K workspaces (None: plan as in steady state, workspaces ready).  ``pair_ok``: they meet
+    ops/gemm.pair_takes."""
     capturing = dev is not None and torch.cuda.is_current_stream_capturing()
     if tile_ok:
-        if _tile.pair_plan(M, N, K) is not None:
+        if pair_ok and _tile.pair_plan(M, N, K) is not None:
             return "pair"
         if (TILE_MIN_M <= M or _tile.dec_small(M, N, K)) and _tile.dec_plan(M, N, K) is not None and (
                 dev is None or _tile.dec_capture_ok(dev, M, N, K)):
             return "decode"
-        if use_tile(M, N, K) and (dev is None or _tile.capture_ok(dev, M, N, K)):
+        if use_tile(M, N, K) and (dev is None or _tile.capture_ok(dev, M, N, K, pair=pair_ok)):
             return "tile"
         if M >= _tile.PREFILL_MIN_M and _tile.prefill_plan(M, N, K) is not None and (
-                dev is None or _tile.capture_ok(dev, M, N, K)):
+                dev is None or _tile.capture_ok(dev, M, N, K, pair=pair_ok)):
             return "tile_prefill"
     if splitk_parts(M, N, K):
         return "splitk"
@@ -317,7 +318,7 @@ def kernel_for(M: int, N: int, K: int, tile_ok: bool = True, dev: torch.device |
     if K % 16 == 0 and N % 4 == 0 and use_stream(M, N, K) and stream_ready:
         return "stream"
     if tile_ok and (_tile.wide_plan(M, N, K) is not None or _tile.unmeasured_plan(M, N, K) is not None and (
-            dev is None or _tile.capture_ok(dev, M, N, K))):
+            dev is None or _tile.capture_ok(dev, M, N, K, pair=pair_ok))):
         return "tile_prefill"
     return "library"
 
@@ -331,17 +332,17 @@ def _differentiated(*ts) -> bool:
     return fwAD._current_level >= 0 or (torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts))
 
 
-def _plain_product(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> bool:
+def _plain_product(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None, align: int = 16) -> bool:
     """Whether the owned kernel may stand in for the library's product of x [M, K] and w: it checks no operand against
     another, and it knows no derivative, trace, dispatch or function mode, tensor subclass or autocast.  What fails here goes
-    to the library, which handles or refuses it."""
+    to the library, which handles or refuses it.  ``align``: bytes that the bias' address has to be a multiple of."""
     if has_torch_function((x, w, b)) or torch._C._len_torch_function_stack():
         return False
     at = x.get_device()
     if w.dim() != 2 or w.size(1) != x.size(1) or w.get_device() != at or w.dtype != x.dtype or w.is_meta:
         return False
     if b is not None and not (b.dim() == 1 and b.size(0) == w.size(0) and b.get_device() == at and b.dtype == x.dtype
-                              and not b.is_meta and b.is_contiguous() and b.data_ptr() % 16 == 0):
+                              and not b.is_meta and b.is_contiguous() and b.data_ptr() % align == 0):
         return False
     return not (_differentiated(x, w, b) or torch.is_autocast_enabled() or torch._C._get_tracing_state() is not None
                 or torch._C._len_torch_dispatch_stack() or at >= 0 and at != torch.cuda.current_device())
@@ -362,9 +363,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> t
         N = w.shape[0]
         kind = kernel_for(M, N, K, _tile.supported(x, w), x.device)
         if kind == "pair":
-            if _plain_product(x, w, b) and _tile.pair_takes(x, w, b):
+            if not _plain_product(x, w, b, align=2):
+                return torch.nn.functional.linear(x, w, b)
+            if _tile.pair_takes(x, w, b):
                 return _tile.gemm_pair(x, w, b, _tile.pair_plan(M, N, K))
-            return torch.nn.functional.linear(x, w, b)
+            kind = kernel_for(M, N, K, True, x.device, pair_ok=False)
         if kind == "decode":
             return _tile.gemm_decode(x, w, b)
         if kind == "tile":

@@ -124,3 +124,19 @@ def test_gate_up_captured_with_a_bias_at_any_address(monkeypatch, at):
     with G.WS.owned_by({}):
         G.mlp_gate_up(x, w, b)
     assert took == (["library"] if at else ["pair"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,other", [(100, 768, 768, "decode"), (256, 768, 1024, "decode"), (700, 768, 768, "library")])
+@pytest.mark.parametrize("at", [8, 4, 2])
+def test_linear_with_a_bias_at_any_address(dev, monkeypatch, M, N, K, other, at):
+    """What the small tiles refuse goes to the kernel that the shape has without them; a bias at 8 bytes they take."""
+    x, w, b = _mk(dev, M, N, K)
+    b = torch.cat([b[: at // 2], b])[at // 2:]
+    assert L.kernel_for(M, N, K) == "pair" and L.kernel_for(M, N, K, pair_ok=False) == other
+    took = []
+    for name in ("gemm_pair", "gemm_decode", "gemm"):
+        monkeypatch.setattr(G, name, lambda *a, _f=getattr(G, name), _n=name, **k: took.append(_n) or _f(*a, **k))
+    y = L.linear(x, w, b)
+    assert took == (["gemm_pair"] if at == 8 else ["gemm_decode"] if other == "decode" else [])
+    torch.testing.assert_close(y.double(), x.double() @ w.double().T + b.double(), **TOL)
