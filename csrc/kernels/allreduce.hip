@@ -147,9 +147,11 @@ GRAG_API int grag_ar_alloc(long bytes, void** ptr) {
 }
 // For the last moments of a process only: ordinary memory over a freed uncached region has read stale afterwards.
 GRAG_API int grag_ar_free(void* ptr) { return (int)hipFree(ptr); }
-// Zero a region that a new communicator takes over.
+// Zero a region that a new communicator takes over: behind everything in flight on the device (hipMemset waits for no
+// non-blocking stream), so that no launch of the communicator before writes its flags behind the zeros.
 GRAG_API int grag_ar_clear(void* ptr, long bytes) {
-  hipError_t e = hipMemset(ptr, 0, (size_t)bytes);
+  hipError_t e = hipDeviceSynchronize();
+  if (e == hipSuccess) e = hipMemset(ptr, 0, (size_t)bytes);
   return e != hipSuccess ? (int)e : (int)hipDeviceSynchronize();
 }
 

@@ -1,7 +1,10 @@
 """Regions of the one-shot all-reduce outlive their communicators (parallel/custom_ar.py): freed uncached memory gave
 later tensors stale values on the GPU, so a closed communicator's regions are kept and handed to the next one."""
 import ctypes
+import subprocess
+import sys
 
+from githubrepostorag_amd.ops import _lib
 from githubrepostorag_amd.parallel import custom_ar
 
 
@@ -38,3 +41,21 @@ def test_regions_are_kept_and_cleared_not_freed(monkeypatch):
     kept = {k: list(v) for k, v in custom_ar._KEPT.items()}
     exported.close()
     assert custom_ar._KEPT == kept and not freed  # a peer may still map it: kept, but not handed out again
+
+
+STUBS = """
+#include <stdio.h>
+int hipMemset(void* p, int v, unsigned long n) { printf("memset %ld %d %lu\\n", (long)p, v, n); fflush(stdout); return 0; }
+int hipDeviceSynchronize(void) { printf("wait\\n"); fflush(stdout); return 0; }
+"""
+
+
+def test_a_region_is_cleared_behind_what_is_in_flight(tmp_path):
+    """grag_ar_clear waits for the device before it writes the zeros and after: the runtime's calls, by two stubs in their place."""
+    src, so = tmp_path / "stubs.c", tmp_path / "stubs.so"
+    src.write_text(STUBS)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    run = ("import ctypes; ctypes.CDLL({!r}, mode=ctypes.RTLD_GLOBAL); f = ctypes.CDLL({!r}).grag_ar_clear; "
+           "f.argtypes = [ctypes.c_void_p, ctypes.c_long]; assert f(4096, 512) == 0").format(str(so), str(_lib.lib_path()))
+    out = subprocess.run([sys.executable, "-c", run], check=True, capture_output=True, text=True, timeout=100).stdout
+    assert out.split("\n") == ["wait", "memset 4096 0 512", "wait", ""]
