@@ -24,10 +24,11 @@ _DEC_AUTO = "GRAG_DECODE_STAGES" not in os.environ and os.environ.get("GRAG_DECO
 # 40.3 / 33.7, B16 of 16000 17.3 / 15.6, B5 ctx3000 20.5 / 19.9, B24 ctx300 14.9 / 14.7: at every size
 DECODE_NT = {3: 11, 8: 12}
 DECODE_NT_MIN_WAVES = int(os.environ.get("GRAG_DECODE_NT_MIN_WAVES", "0"))
-# multi-part plans over at least 512 (sequence x kv head) rows and of more waves than the chip holds at once with 2-stage rings (5 a
-# CU) take the 3-stage ring (3 a CU, as many bytes in flight): us of 11 / 12, 28 / 4 heads: B192 ctx3000 (1536 waves) 207 / 194,
-# B176 ctx1500 (1408) 104 / 97.5, but B128 ctx1500 (1024) 71.8 / 82.8 and B128 of 130000 keys in all (1024) 56.3 / 75.0; parts of
-# unequal sequences are often empty, so that fewer rows rarely fill it (B83 of 68807 keys, 1328 parts: a step 781 / 803) (0: off)
+# multi-part plans over at least DECODE_NS3_ROWS (sequence x kv head) rows and of more waves than the chip holds at once with
+# 2-stage rings (5 a CU) take the 3-stage ring (3 a CU, as many bytes in flight): us of 11 / 12, 28 / 4 heads: B192 ctx3000 (1536
+# waves) 207 / 194, B176 ctx1500 (1408) 104 / 97.5, but B128 ctx1500 (1024) 71.8 / 82.8 and B128 of 130000 keys in all (1024) 56.3 / 75.0; parts of
+# unequal sequences are often empty, so that fewer rows rarely fill it (B83 of 68807 keys, 1328 parts: a step 781 / 803) (either 0: off)
+DECODE_NS3_ROWS = int(os.environ.get("GRAG_DECODE_NS3_ROWS", "512"))
 DECODE_NS3_WAVES = int(os.environ.get("GRAG_DECODE_NS3_WAVES", "1280"))
 _DEC_NT = os.environ.get("GRAG_DECODE_NT", "auto")
 
@@ -100,12 +101,12 @@ def _decode_tickets(dev: torch.device, nsplit: int) -> torch.Tensor:
 
 def decode_variant(nsplit: int, split_len: int, waves: int | None = None) -> int:
     """Decode kernel per split plan, 32-key tiles.  ``waves``: the launch's (sequence x kv-head x split) count; more than
-    DECODE_NS3_WAVES of several parts over 512 rows take the 3-stage ring, at least DECODE_NT_MIN_WAVES load K/V non-temporally
-    (GRAG_DECODE_RING_AUTO=1: the 3-stage ring for parts that cover more than 2048 keys)."""
+    DECODE_NS3_WAVES of several parts over DECODE_NS3_ROWS rows take the 3-stage ring, at least DECODE_NT_MIN_WAVES load K/V
+    non-temporally (GRAG_DECODE_RING_AUTO=1: the 3-stage ring for parts that cover more than 2048 keys)."""
     auto3 = _DEC_AUTO and os.environ.get("GRAG_DECODE_RING_AUTO") == "1"
     nw = DECODE_RING_NW[3] if auto3 and nsplit > 1 and nsplit * split_len > 2048 else DECODE_NW
-    if (_DEC_AUTO and DECODE_NS3_WAVES and nsplit > 1 and waves is not None and waves > DECODE_NS3_WAVES
-            and waves // nsplit >= 512):
+    if (_DEC_AUTO and DECODE_NS3_ROWS and DECODE_NS3_WAVES and nsplit > 1 and waves is not None and waves > DECODE_NS3_WAVES
+            and waves // nsplit >= DECODE_NS3_ROWS):
         nw = DECODE_RING_NW[3]
     nt = _DEC_NT == "1" or (_DEC_NT == "auto" and waves is not None and waves >= DECODE_NT_MIN_WAVES)
     return DECODE_NT.get(nw, nw) if nt else nw
