@@ -57,5 +57,6 @@ def test_a_region_is_cleared_behind_what_is_in_flight(tmp_path):
     subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
     run = ("import ctypes; ctypes.CDLL({!r}, mode=ctypes.RTLD_GLOBAL); f = ctypes.CDLL({!r}).grag_ar_clear; "
            "f.argtypes = [ctypes.c_void_p, ctypes.c_long]; assert f(4096, 512) == 0").format(str(so), str(_lib.lib_path()))
+    _lib.lib()  # (built)
     out = subprocess.run([sys.executable, "-c", run], check=True, capture_output=True, text=True, timeout=100).stdout
     assert out.split("\n") == ["wait", "memset 4096 0 512", "wait", ""]
