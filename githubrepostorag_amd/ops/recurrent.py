@@ -32,18 +32,53 @@ LINEAR_SCAN_CHUNK = 64
 
 
 @functools.lru_cache(256)  # (a step's layers ask the same)
-def _scan_walks(max_q: int, tokens: int, nseq: int, tiles: float, split: bool) -> tuple[float, int]:
-    """(walks, chunks a part) of the matrix-core scan (csrc/kernels/linscan.hip) for a step of ``nseq`` portions with
-    ``tokens`` tokens, the longest ``max_q``, and ``tiles`` (head, 64 columns) tiles a portion: its length in walks of a
-    64-token chunk and the cut of a portion that makes it shortest.  Workgroups start longest first, so several portions
-    take the longest walk or the chip's share of all and about a third of a walk for its uneven end; a single portion whole
-    rounds of equal parts.  Where portions are cut, all parts but the last are walked for the state alone before (0.42 of a
-    walk), and a part reads the states of those before it.  ``split``: operands in three parts (one workgroup a CU, 12 us a
-    chunk), else two workgroups a CU and 5.7 us.
+def _scan_cut(max_q: int, tokens: int, nseq: int, tiles: int, split: bool, d: int) -> int:
+    """Chunks of 64 tokens a part of the matrix-core scan (csrc/kernels/linscan.hip), for a step of ``nseq`` portions with
+    ``tokens`` tokens, the longest ``max_q``, ``tiles`` (head, 64 columns) tiles a portion and ``d`` state rows: the cut that makes
+    the step shortest, in walks of a chunk.  Workgroups start longest first, so several portions take the longest walk or
+    the chip's share of all and part of a walk for its uneven end; a single portion whole rounds of equal parts.  A walk of some chunks costs some more for its start and its state.  Where portions are cut, all parts but the
+    last are walked for the state alone before (about a quarter of a walk), and a part reads the states of those before it.
+    ``split``: operands in three parts (one workgroup a CU, 12 us a chunk), else two workgroups a CU and 5.7 us.
 
-    us, cut at 2 / 4 / 8 / 16 chunks / not at all: 28 heads of 128 x 128 with SiLU 3 portions of 4096 tokens 291 / 270 / 260
-    / 269 / 340 (taken 8), 7 of 8192 567 / 498 / 465 / 443 / 410 - 448 (none); state space, 56 heads of 128 x 64, 3 of 4096
-    141 / 116 / 110 / 149 / 171 (8); 24 of 128 x 64, one of 8192 177 / 122 / 115 / 146 / 517 (8)."""
+    From 455 points of 21 sizes, 1 - 20 portions, 65 - 8192 tokens, every cut timed: the cut taken is 1.015 of the best in the
+    geometric mean and 1.31 at most (without the cost of a walk's start 1.038 and up to 1.37, where parts of one chunk were taken:
+    fp32, 8 heads of 64 x 128, 2 portions of 1500 tokens, cut at 1 / 2 / 3 chunks 89 / 65 / 84 us).  28 heads of 128 x 128 with SiLU,
+    3 portions of 4096 tokens, cut at 2 / 4 / 8 / 16 / not at all 291 / 270 / 260 / 269 / 340 (taken 8), 7 of 8192 567 / 498 / 465 /
+    443 / 410 - 448 (none); state space, 56 heads of 128 x 64, 3 of 4096 141 / 116 / 110 / 149 / 171 (8); 24 of 128 x 64, one of
+    8192 177 / 122 / 115 / 146 / 517 (8); 80 of 16 x 64, one of 4096 250 / 207 / 236 / 261 / 564, at 12 218 (12, one pass 208)."""
+    slots, read, start, ahead_start, tail, first, const, odd = (
+        (256, 0.002, 1.87, 1.59, 0.59, 0.24, 0.69, 1.12) if split else (512, 0.5, 1.79, 0.15, 0.83, 0.275, 1.1, 1.15))
+    chunks, total = -(-max_q // LINEAR_SCAN_CHUNK), tokens / LINEAR_SCAN_CHUNK + (nseq - 1) / 2
+    share = tiles / slots  # of a round, a workgroup for each tile
+
+    def walk(s, work, more):  # of parts of s chunks that are ``work`` chunks together
+        if nseq == 1:
+            return -(-int(-(-work // s) * tiles) // slots) * (s + more)
+        return max(s + more, work / s * share * (s + more) + tail * s)
+
+    best, part, s = walk(chunks, chunks, start), chunks, 1
+    if nseq > 1:
+        best = max(chunks + start, (total + nseq * start) * share + tail * total / nseq)
+    while s < chunks:
+        ahead = total - nseq * s / 2 if nseq > 1 else (-(-chunks // s) - 1) * s
+        cost = walk(s, chunks if nseq == 1 else total, start) + first * walk(s, max(ahead, s), ahead_start) + const
+        cost += read * d / 128 * chunks / s * max(1.0, total / s * share)
+        if s > 3 and s & (s - 1):  # (6, 12, ..: less often the best than they seem)
+            cost *= odd
+        if cost < best:
+            best, part = cost, s
+        s += max(1, s // 2) if s & (s - 1) == 0 else s // 3  # 1, 2, 3, 4, 6, 8, 12, 16, ..
+    return part
+
+
+@functools.lru_cache(256)  # (a step's layers ask the same)
+def _scan_walks(max_q: int, tokens: int, nseq: int, tiles: float, split: bool) -> float:
+    """Walks of a 64-token chunk that a step of the matrix-core scan takes, as _scan_taken reckons (roughly; _scan_cut for the cut):
+    ``nseq`` portions with ``tokens`` tokens, the longest ``max_q``, and ``tiles`` (head, 64 columns) tiles a portion, crowding
+    counted.  Several portions take the longest walk or the chip's share of all and about a third of a walk for its uneven
+    end; a single portion whole rounds of equal parts.  Where portions are cut, all parts but the last are walked for the state alone before (0.42 of a
+    walk), and a part reads the states of those before it.  ``split``: operands in three parts (one workgroup a CU, 12 us a
+    chunk), else two workgroups a CU and 5.7 us."""
     slots, read, crowd = (256, 0.026, 1.0) if split else (512, 0.11, 1.2)  # (whole portions often have a CU of their own)
     chunks, total = -(-max_q // LINEAR_SCAN_CHUNK), tokens / LINEAR_SCAN_CHUNK + (nseq - 1) / 2
     share = tiles / slots  # of a round, a workgroup for each tile
@@ -53,15 +88,14 @@ def _scan_walks(max_q: int, tokens: int, nseq: int, tiles: float, split: bool) -
             return -(-int(-(-work // s) * tiles) // slots) * s
         return max(s, work * share + 0.35 * s)
 
-    best, part, s = max(chunks, total * share + 0.35 * total / nseq), chunks, 1
+    best, s = max(chunks, total * share + 0.35 * total / nseq), 1
     while s < chunks:
         ahead = total - nseq * s / 2 if nseq > 1 else (-(-chunks // s) - 1) * s
         cost = walk(s, chunks if nseq == 1 else total) + 0.42 * walk(s, max(ahead, s)) + 1
         cost = crowd * (cost + read * chunks / s * max(1.0, total / s * share))
-        if cost < best:
-            best, part = cost, s
+        best = min(best, cost)
         s += max(1, s // 2) if s & (s - 1) == 0 else s // 3  # 1, 2, 3, 4, 6, 8, 12, 16, ..
-    return best, part
+    return best
 
 
 def _scan_taken(m: AttnMetadata, tokens: int, H: int, d: int, vd: int, split: bool, exact: bool) -> bool:
@@ -73,15 +107,16 @@ def _scan_taken(m: AttnMetadata, tokens: int, H: int, d: int, vd: int, split: bo
     (of portions of a chunk: as many as their rounds) of 2.9 + 0.021 d where exact with one part an operand, 0.4 + 0.10 d
     with three, 5.9 + 0.039 d and 14.6 + 0.084 d otherwise; a round of workgroups that share a CU costs 1.6 walks, of
     those that do not 1.1.  One-pass kernels: 9.5 + a chain of 0.14 + 0.0345 d a token and 3.5e-7 a token and number of
-    the state, twice that where portions are cut at 64.  The choice is within 1 % of the faster side in the geometric
-    mean, also over 144 points of other sizes; a rule on the portions' length alone was 13 % off (scan against one pass: fp32, 28 heads of 16 x 16, 64 x 64
-    tokens 153 / 54; fp32 state space, 56 heads of 8 x 16, 7 portions of 8192 728 / 158)."""
+    the state, twice that where portions are cut at 64.  Of 470 points of 21 sizes the choice is within 0.2 % of the faster
+    side in the geometric mean; the most that was lost is 1.34 (fp32, 56 heads of 16 x 64, 5 portions of 1187 tokens, scan / one pass
+    100 / 134).  A rule on the portions' length alone was 13 % off (scan against one pass: fp32, 28 heads of 16 x 16, 64 x 64 tokens
+    153 / 54; fp32 state space, 56 heads of 8 x 16, 7 portions of 8192 728 / 158)."""
     if m.max_q_len < LINEAR_SCAN_MIN or d > lib().grag_linear_scan_max_dim():
         return False
     base, span = ((0.4, 0.10) if split else (2.9, 0.021)) if exact else ((14.6, 0.084) if split else (5.9, 0.039))
     slots, crowd = (256, 1.1) if split else (512, 1.6)
     load, cut = H * -(-vd // 64) * crowd, m.max_q_len > LINEAR_SCAN_CHUNK
-    walks = _scan_walks(m.max_q_len, tokens, m.num_seqs, load, split)[0] if cut else max(1.0, m.num_seqs * load / slots)
+    walks = _scan_walks(m.max_q_len, tokens, m.num_seqs, load, split) if cut else max(1.0, m.num_seqs * load / slots)
     chain, work = min(m.max_q_len, 64) * (0.14 + 0.0345 * d), 3.5e-7 * tokens * H * d * vd
     return (base + span * d) * walks < (2 if cut else 1) * math.hypot(chain, work)
 
@@ -92,14 +127,14 @@ def _scan_exact(x: torch.Tensor, offs: tuple, d: int, vd: int, rd: int = 0) -> b
             and x.stride(0) % 4 == 0 and all(o % 4 == 0 for o in offs))
 
 
-def _scan_part(max_q: int, tokens: int, nseq: int, tiles: int, split: bool) -> int:
+def _scan_part(max_q: int, tokens: int, nseq: int, tiles: int, split: bool, d: int) -> int:
     """Tokens per part of the matrix-core scan."""
-    return _scan_walks(max_q, tokens, nseq, tiles, split)[1] * LINEAR_SCAN_CHUNK
+    return _scan_cut(max_q, tokens, nseq, tiles, split, d) * LINEAR_SCAN_CHUNK
 
 
 def _scan_ws(m: AttnMetadata, rows: int, H: int, d: int, vd: int, split: bool, device):
     """(part, ws, wa) of a matrix-core scan: the part length and its fp32 scratch (None where no portion is cut)."""
-    part = _scan_part(m.max_q_len, rows, m.num_seqs, H * -(-vd // 64), split)
+    part = _scan_part(m.max_q_len, rows, m.num_seqs, H * -(-vd // 64), split, d)
     if m.max_q_len <= part:
         return part, None, None
     n = m.num_seqs * -(-m.max_q_len // part)

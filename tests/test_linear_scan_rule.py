@@ -30,6 +30,22 @@ def test_rule(dtype, act, lens, H, d, vd, scan, passes, monkeypatch):
     assert recurrent._scan_taken(m, sum(lens), H, d, vd, act or dtype == "f32", exact) == (scan < passes)
 
 
+# longest portion, tokens, portions, heads, d, vd, operands in three parts, us by chunks a part
+CUTS = [(914, 1500, 2, 8, 64, 128, True, {1: 89, 2: 65, 3: 84, 4: 106, 8: 192, 15: 253}),
+        (551, 800, 2, 28, 16, 16, True, {1: 67, 2: 53, 3: 69, 4: 87, 9: 122}),
+        (800, 800, 1, 12, 128, 128, False, {1: 33, 2: 26, 3: 30, 4: 35, 6: 46, 8: 59, 13: 62}),
+        (8192, 8192, 1, 12, 128, 128, True, {1: 646, 2: 320, 3: 297, 4: 231, 6: 246, 8: 264, 16: 274, 32: 530, 128: 1427}),
+        (3094, 4096, 2, 28, 128, 128, False, {1: 354, 2: 155, 3: 118, 4: 114, 6: 111, 8: 98, 12: 130, 16: 113, 49: 225}),
+        (8192, 8192, 1, 80, 16, 64, False, {1: 1107, 2: 559, 4: 419, 8: 384, 12: 421, 16: 453, 24: 422, 32: 514, 128: 1125})]
+
+
+@pytest.mark.parametrize("max_q,tokens,nseq,H,d,vd,split,us", CUTS)
+def test_cut(max_q, tokens, nseq, H, d, vd, split, us):
+    """A portion's cut within 1.15 of the best that was measured."""
+    part = recurrent._scan_part(max_q, tokens, nseq, H * -(-vd // 64), split, d)
+    assert part % 64 == 0 and us[min(part // 64, max(us))] <= 1.15 * min(us.values())
+
+
 def test_exact_rows():
     x = torch.empty(4, 400, dtype=torch.bfloat16)
     ok = recurrent._scan_exact
