@@ -369,13 +369,10 @@ __global__ __launch_bounds__(64 * NW * TEAMS) void attn_prefill_kernel(AttnParam
   const int lane = threadIdx.x & 63, wave = TEAMS == 1 ? threadIdx.x >> 6 : (threadIdx.x >> 6) & (NW - 1);
   char* smem = all_lds + team * NS * 2 * TILE;
   const int h4 = lane >> 4, li = lane & 15;
-  // the tiles of all sequences and kv heads, longest walks first; turned by one from tile to tile, so that no XCD (the workgroups'
-  // number modulo 8) is left with the sequences that have no such tile: 7 sequences of 8192 tokens, 28 / 4 heads, 153 -> 140 us
-  // (sequence by sequence, the last one's long walks ran alone)
-  const int tiles = p.tiles_per_seq, streams = gridDim.x / tiles * gridDim.y;
-  const unsigned id = blockIdx.x + gridDim.x * blockIdx.y, rank = id / streams, stream = (id + rank) % streams;
-  const int seq = stream / gridDim.y, kvh = stream % gridDim.y;
-  const int tile = tiles - 1 - (int)rank;
+  // us before, sequence by sequence / turned by one from tile to tile / so: 28 / 4 heads 7 sequences of 8192 tokens 153 / 133 / 126, 8 of
+  // 8000 129 / 141 / 106; 12 / 2 heads 4 of 8000 145 / 188 / 128, 2 of 8000 173 / 199 / 170
+  const WalkOrder at = walk_order(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x / p.tiles_per_seq, gridDim.y, p.tiles_per_seq);
+  const int seq = at.seq, kvh = at.kvh, tile = at.tile;
   const int q0 = p.q_start[seq], qlen = p.q_start[seq + 1] - q0;
   const int ctx = p.ctx_len[seq];
   const int G = p.G;

@@ -47,6 +47,20 @@ __device__ __forceinline__ short f2bits(float f) {
   return __builtin_bit_cast(short, b);
 }
 
+// The (sequence, kv head) stream and the tile of a sequence that workgroup `id` of a causal prompt attention walks: longest walks first,
+// the last tile of every sequence, the last but one, and so on.  Workgroups are dealt to the shader engines in turn, 8 XCDs of 4, and
+// run where they were dealt; each tile number's streams are turned against those before it, so that every engine meets every
+// sequence, also where the streams are a divisor or a multiple of 32 in number (turned by one a tile, an engine saw two of 4
+// sequences and the longest one's engines worked on alone).  A list of 32 engines of 8 CUs each tells the measured times within a few
+// percent; over 600 random batches this order takes 1.10 of what the chip's share or the longest walk alone allow in the
+// geometric mean, turned by one 1.11, sequence by sequence 1.24.
+struct WalkOrder { int seq, kvh, tile; };
+__device__ __forceinline__ WalkOrder walk_order(unsigned id, unsigned nseq, unsigned kv_heads, unsigned tiles) {
+  const unsigned streams = nseq * kv_heads, rank = id / streams;
+  const unsigned stream = (id + (rank + rank / 4 + rank / 8) % nseq * kv_heads) % streams;
+  return {(int)(stream / kv_heads), (int)(stream % kv_heads), (int)(tiles - 1 - rank)};
+}
+
 // a += four consecutive floats of each of S fp32 split-K planes (plane stride `plane` elements), in plane order.
 // Up to 16 planes are walked in one fully unrolled, branch-free pass of 2, 4, 8, 12 or 16 (indices past S re-read
 // plane 0 and add zero: fma(1, y, x) rounds as x + y), more in passes of 16 before it, so a pass's loads are all in flight

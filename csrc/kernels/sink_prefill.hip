@@ -57,11 +57,9 @@ __global__ void __launch_bounds__(256 * TEAMS, MR == 32 || TEAMS > 1 ? 2 : 4) si
   const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & (NW - 1));
   char* smem = all_lds + team * 2 * 2 * TILE;
   const int hh = lane / MR, li = lane % MR;  // this lane's row is li; its keys (and head numbers) are 8 i + 4 hh + 0..3
-  // the walks of all portions and kv heads, longest first; turned by one from tile to tile, so that no XCD (the workgroups' number
-  // modulo 8) is left with the portions that have no such tile
-  const int streams = p.nseq * p.G, rank = blockIdx.x / streams, stream = (int)(blockIdx.x + rank) % streams;
-  const int seq = stream / p.G, kvh = stream % p.G;
-  const int row_base = (p.tiles - 1 - rank) * ROWS;
+  const WalkOrder at = walk_order(blockIdx.x, p.nseq, p.G, p.tiles);
+  const int seq = at.seq, kvh = at.kvh;
+  const int row_base = at.tile * ROWS;
   const int q0 = p.q_start[seq], qlen = p.q_start[seq + 1] - q0, ctx = p.ctx_len[seq], pos0 = ctx - qlen;
   const int R = p.R, nrows = qlen * R;
   if (row_base >= nrows) return;
