@@ -1507,23 +1507,47 @@ int launch_prefill_rows(const AttnParams& prm_in, int nseq, int max_q_len, hipSt
   return (int)hipGetLastError();
 }
 
-// Rows a workgroup by the 256-row workgroups that all rows make: a walk's time is the chain of its tiles, shorter with 16 rows a wave
-// than with 32, and few walks leave the chip idle, many are paid by the reads a row.  us of 256 rows (8 waves of 32) / 128 (8 of
-// 16) / 64 (4 of 16), tokens by sequences: 12 / 2 heads, 300 x 1 (16 workgroups) 18.3 / 12.8 / 13.7, 1187 x 1 (56) 43.3 / 29.9 /
-// 28.8, 3600 x 12 (170) 29.5 / 22.5 / 22.1, 8192 x 4 (384) 96.8 / 117 / 121; 28 / 4 heads, 600 x 1 (68) 27.6 / 18.8 / 17.6,
-// 1500 x 1 (168) 54.8 / 39.5 / 38.1, 2048 x 1 (224) 70.2 / 52.5 / 57.8, 2048 x 4 (224) 38.6 / 31.8 / 30.4, 3000 x 1 (332) 99.4 /
-// 106 / 106, 3000 x 8 (332) 37.4 / 41.4 / 39.7, 8192 x 7 (896) 129 / 159 / 162.
+// The shape of a prompt attention's workgroups: 0 two teams of 4 waves on 64 rows, 1 64 rows, 2 128 rows by 8 waves of 16, 3 256 rows
+// by 8 waves of 32.  A walk's time is the chain of its tiles, shorter with 16 rows a wave than with 32 and with two teams than
+// with one; many walks are paid by the reads a row.  So a shape's time is its time a tile (of 256 rows': 1), times the rounds of its
+// workgroups where they are more than the chip holds (kSlots a CU, a little less than fit: unequal walks).  Of uneven prompts a
+// sequence's last tile is half full.  Rounds count by a walk's mean length over the longest's, with kPast cached keys before each
+// prompt: the host does not know how many there are.
+// 947 batches of 1 - 128 prompts, 30 - 8192 tokens, no, 300 and 1000 cached keys, heads of 128 (28 / 4, 12 / 2) and 64 (16 / 4, 12 /
+// 12), all four shapes timed: 1.036 and 1.022 of the best in the geometric mean; by the rows' 256-row workgroups alone (lines at
+// 120, 200 and 280) 1.08 and 1.09.  us in 256 rows before / by those lines / now, unequal prompts: 28 / 4 heads 24 of 768 tokens in all
+// 10.8 / 14.8 / 7.4, 24 of 1536 behind 1000 cached keys each 46 / 67 / 56; 12 / 2 heads 40 of 2000 12.8 / 16.1 / 10.6.  us of the four shapes,
+// 28 / 4 heads: 1187 x 1 32.1 / 28.8 / 29.7 / 43.5, 8192 x 7 - / 164 / 150 / 133; 12 / 2 heads 2048 x 1 31.8 / 43.4 / 44.2 / 66.5, 4000 x 4
+// - / 48 / 48 / 54.
+struct PrefillShape {
+  float tau, slots;
+  int rows;
+};
+int prefill_shape(int D, int nseq, long total_q, int max_q_len, int G, int Hkv) {
+  static const PrefillShape k128[4] = {{0.47f, 0.68f, 64}, {0.66f, 1.3f, 64}, {0.87f, 1.25f, 128}, {1.f, 1.9f, 256}};
+  static const PrefillShape k64[4] = {{0.57f, 1.5f, 64}, {0.59f, 2.5f, 64}, {0.58f, 1.58f, 128}, {1.f, 1.52f, 256}};
+  constexpr double kPast = 700;
+  const PrefillShape* shapes = D == 128 ? k128 : k64;
+  const double mean = (double)total_q / nseq, part = (mean / 2 + kPast) / (max_q_len + kPast), cus = grag::device_cus();
+  int best = 0;
+  double least = 0;
+  for (int s = 0; s < 4; ++s) {
+    const int rows = shapes[s].rows;
+    const double wgs = Hkv * fmin((double)nseq * (((long)max_q_len * G + rows - 1) / rows), (double)total_q * G / rows + 0.5 * nseq);
+    const double t = shapes[s].tau * fmax(1.0, part * wgs / (shapes[s].slots * cus));
+    if (s == 0 || t < least) best = s, least = t;
+  }
+  return best;
+}
 template <int D>
 int launch_prefill(const AttnParams& prm, int nseq, int max_q_len, int nw, hipStream_t stream) {
   if (nw == 6) return launch_prefill_rows<D, 2, 3, 8>(prm, nseq, max_q_len, stream);
-  const long wgs = ((long)prm.total_q * prm.G + 255) / 256 * prm.Hkv;
-  // two teams of waves on a walk where a CU gets one such workgroup at most; one / two: 1187 x 1 (56) 29.1 / 21.5, 2048 x 1 (96)
-  // 46.6 / 32.7, 2048 x 4 (96) 25.8 / 22.6, 3600 x 12 (170) 21.8 / 31.1; 28 / 4 heads 600 x 1 (68) 17.7 / 14.0, 1000 x 2 (112) 21.3 /
-  // 19.2, 1500 x 1 (168) 37.9 / 43.1
-  if (wgs <= 120) return launch_prefill_rows<D, 1, 2, 4, 2>(prm, nseq, max_q_len, stream);
-  if (wgs <= 200) return launch_prefill_rows<D, 1, 2, 4>(prm, nseq, max_q_len, stream);
-  if (wgs <= 280) return launch_prefill_rows<D, 1, 2, 8>(prm, nseq, max_q_len, stream);
-  return launch_prefill_rows<D, 2, 2, 8>(prm, nseq, max_q_len, stream);
+  switch (prefill_shape(D, nseq, prm.total_q, max_q_len, prm.G, prm.Hkv)) {
+    case 0: return launch_prefill_rows<D, 1, 2, 4, 2>(prm, nseq, max_q_len, stream);
+    case 1: return launch_prefill_rows<D, 1, 2, 4>(prm, nseq, max_q_len, stream);
+    case 2: return launch_prefill_rows<D, 1, 2, 8>(prm, nseq, max_q_len, stream);
+    default: return launch_prefill_rows<D, 2, 2, 8>(prm, nseq, max_q_len, stream);
+  }
 }
 
 template <int D>
@@ -1552,6 +1576,10 @@ int dispatch_nw(const AttnParams& prm, int nseq, int max_q_len, int nw, bool pag
 }
 
 }  // namespace
+
+GRAG_API int grag_prefill_attn_shape(int D, int nseq, int total_q, int max_q_len, int G, int Hkv) {  // (for tests)
+  return nseq < 1 || (D != 64 && D != 128) ? -1 : prefill_shape(D, nseq, total_q, max_q_len, G, Hkv);
+}
 
 // Paged attention (prefill / decode).  q: [T, Hq, D] token-major rows of
 // stride q_stride; caches [blocks, Hkv, BS, D]; out [T, Hq*D] (stride

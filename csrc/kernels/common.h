@@ -26,6 +26,19 @@ typedef __bf16 bf16;
 
 namespace grag {
 
+// compute units of the current device (cached per device; a host query, legal during graph capture)
+inline int device_cus() {
+  static int cus[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cus[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cus[dev] = n;
+  }
+  return cus[dev];
+}
+
 // f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): register arrays that its number indexes stay in registers,
 // also in loops that the unroller would give up on (they would lie in scratch memory)
 template <int N, int I = 0, typename F>

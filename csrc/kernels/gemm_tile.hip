@@ -947,21 +947,6 @@ GRAG_API int grag_splitk_reduce(const void* ws, const void* bias, void* C, int l
 //   otherwise every tile is one workgroup.
 // Requirements (checked): K % 64 == 0, every split >= 2 K-tiles, lda/ldw % 8 == 0,
 // N % 8 == 0 (silu: N % 64 == 0), ldc % 8 == 0, 16-B aligned pointers.
-namespace {
-// compute units of the current device (cached per device; a host query, legal during graph capture)
-int device_cus() {
-  static int cus[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cus[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev] = n;
-  }
-  return cus[dev];
-}
-}  // namespace
-
 static int gemm_tile_run(const void* A, const void* W, const void* bias, void* C, int lda, int ldw, int ldc, int M, int N,
                          int K, int epi, int act, int ksplit, int sk_grid, void* ws, void* cnt, float limit, float alpha,
                          float shift, hipStream_t stream) {

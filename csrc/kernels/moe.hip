@@ -1596,19 +1596,6 @@ GRAG_API hipError_t grag_moe_table_route(const int* tok, const int* table, int n
   return hipGetLastError();
 }
 
-// compute units of the current device (cached per device; a host query, legal during graph capture)
-static int moe_cus() {
-  static int cus[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cus[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev] = n;
-  }
-  return cus[dev];
-}
-
 // rows = T * top sorted rows.  gated 1: a = h [T][lda], w = [E][2N][K], out [rows][N]; gated 0: a = [rows][lda] sorted,
 // w = [E][N][K], out [rows][ldo] in (token, choice) order; gated 3: as 1 with one branch, w = [E][N][K]; gated 2: one matrix per head (E heads, top = tokens, rows =
 // tokens * E): a = [tokens * E][lda], w = [E][N][K], out [tokens * E][ldo], offs / order unused.
@@ -1646,7 +1633,7 @@ GRAG_API hipError_t grag_moe_gemm(const void* a, int lda, const void* w, const i
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
     const long o_bytes = (long)rows * ldo * 2;
     if (K >= 320 && w_bytes * E < (1L << 31) && o_bytes < (1L << 31) && N % 8 == 0 && ldo % 8 == 0 && al16(out) && rows < (1 << 28)) {
-      const int cus = moe_cus();
+      const int cus = device_cus();
 #define MOE_CHAIN(G)                                                                                                     \
   hipLaunchKernelGGL(moe_gemm_chain_kernel<G>, dim3((unsigned)(blocks < cus ? blocks : cus)), dim3(kTileThreads), 0, st, \
                      (const bf16*)a, lda, (int)a_bytes, (const bf16*)w, (int)(w_bytes * E), offs, order, rows, E, top, N, K,     \
