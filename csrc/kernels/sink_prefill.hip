@@ -338,6 +338,52 @@ bool sink_prefill_takes(int d, int vd, int v_ld, int BS, int max_q_len, int R, i
   return keys <= (long)SP_MAXB * SP_BS;
 }
 
+// The shape of a launch's workgroups: 0 two teams of 4 waves on 64 rows, 1 64 rows by 4 waves of 16, 2 128 rows by 4 waves of 32.  A
+// walk's time is its start and the chain of its tiles (kTau each, kStart tiles' worth), shorter with 16 rows a wave than with 32,
+// and two teams take the tiles in turn; many walks are paid by the reads a row, in rounds of their workgroups where they are more
+// than the chip holds (kSlots a CU).  Of uneven prompts a portion's last tile is half full.  Rounds count by a walk's mean length
+// over the longest's, with kPast cached keys before each portion (the host does not know how many there are), at most the
+// window; a table of two tiles' blocks has no second team's work.
+// 1774 batches of 1 - 128 portions, 30 - 8192 tokens, no, 300 and 1000 cached keys, all keys and window 256, heads of 128 (28 / 4, 12 /
+// 2) and 64 (16 / 4, 12 / 12), all three shapes timed: 1.018 of the best in the geometric mean; by the rows' 128-row workgroups alone
+// (lines at 200 and 340) 1.05.  us in 128 rows before / by those lines / now, unequal portions: 28 / 4 heads 40 of 800 tokens in all 9.6 /
+// 18.8 / 8.7, 12 of 480 7.1 / 11.9 / 8.1; 12 / 2 heads 24 of 1536 8.7 / 13.7 / 9.3.  us of the three, 28 / 4 heads, all keys: 600 x 1 16.0 /
+// 21.4 / 27.6, 1187 x 1 - / 38 / 46, 2048 x 4 - / 36.5 / 42.3, 3000 x 8 - / 45.6 / 35.1; 12 / 2 heads 1187 x 1 24.6 / 35.1 / 45.7, 3600 x 12 - /
+// 25.0 / 31.4, 8192 x 4 - / 136 / 110.
+static int sink_prefill_shape(int D, int nseq, long rows, int max_q_len, int R, int G, long reach, long table) {
+  struct Shape {
+    float tau, start, slots;
+    int rows;
+  };
+  static const Shape k128[3] = {{0.35f, 2.5f, 0.38f, 64}, {1.36f, 3.6f, 1.75f, 64}, {1.37f, 4.1f, 3.5f, 128}};
+  static const Shape k64[3] = {{0.34f, 2.f, 0.42f, 64}, {1.44f, 1.5f, 2.6f, 64}, {2.18f, 1.55f, 2.2f, 128}};
+  constexpr double kPast = 1100;
+  const Shape* shapes = D == 128 ? k128 : k64;
+  const double mean = (double)rows / nseq, far = fmin(max_q_len + kPast, (double)reach + 32);
+  const double part = fmin(mean / 2 + kPast, (double)reach) / far, tiles = fmin(max_q_len, (double)reach + 32) / SP_KT;
+  const double cus = device_cus();
+  int best = -1;
+  double least = 0;
+  for (int s = table <= 2 * SP_KT ? 1 : 0; s < 3; ++s) {
+    const int r = shapes[s].rows;
+    const double wgs = G * fmin((double)nseq * (((long)max_q_len * R + r - 1) / r), (double)rows * R / r + 0.5 * nseq);
+    const double t = (shapes[s].tau * tiles + shapes[s].start) * fmax(1.0, part * wgs / (shapes[s].slots * cus));
+    if (best < 0 || t < least) best = s, least = t;
+  }
+  return best;
+}
+static long sink_reach(int chunk, int window) {  // keys that a query sees at most
+  long reach = 1L << 40;
+  if (chunk > 0) reach = chunk;
+  if (window > 0 && window < reach) reach = window;
+  return reach;
+}
+// (for tests)
+GRAG_API int grag_sink_prefill_shape(int D, int nseq, int rows, int max_q_len, int R, int G, int chunk, int window, int bt_stride) {
+  return nseq < 1 || (D != 64 && D != 128) ? -1 : sink_prefill_shape(D, nseq, rows, max_q_len, R, G, sink_reach(chunk, window),
+                                                                     (long)bt_stride * SP_BS);
+}
+
 hipError_t sink_prefill_launch(const void* q, const void* k, const void* v, void* out, int out_ld, const int* bt, int bt_stride,
                                const int* q_start, const int* ctx_len, const float* sinks, int nseq, int max_q_len, int rows, int H,
                                int G, int d, float scale, float out_scale, int nblocks, const float* hscale, const void* hgate,
@@ -348,25 +394,15 @@ hipError_t sink_prefill_launch(const void* q, const void* k, const void* v, void
   a.out_ld = out_ld, a.bt_stride = bt_stride, a.H = H, a.G = G, a.R = H / G, a.nblocks = nblocks;
   a.gate_ld = gate_ld, a.chunk = chunk, a.window = window, a.keep = keep;
   a.scale = scale, a.out_scale = out_scale, a.softcap = softcap;
-  // 128 rows a workgroup, or 64 in waves of 16 where those of all `rows` queries are few for the chip: a walk's time is the chain of
-  // its tiles, shorter with 16 rows a wave.  us of 128 / 64 rows, all keys, tokens by portions (128-row workgroups): 12 / 2 heads,
-  // 600 x 1 (57) 24.4 / 19.3, 1187 x 1 (112) 45.7 / 35.1, 2048 x 4 (192) 38.7 / 30.8, 3600 x 12 (338) 31.4 / 25.0, 8192 x 4 (768)
-  // 110 / 136; 28 / 4 heads, 1500 x 1 (329) 56.2 / 46.9, 2048 x 1 (448) 65.3 / 72.0, 2048 x 4 (448) 42.3 / 36.5, 3000 x 8 (657)
-  // 35.1 / 45.6; window 1024, 12 / 2 heads, 4000 x 2 (375) 54.0 / 64.1.
-  long tiles = ((long)max_q_len * a.R + 127) / 128;
-  const long wgs = ((long)rows * a.R + 127) / 128 * G;
-  // and where those are a CU's at most, two teams of 4 waves that take the walk's tiles in turn: one / two, 600 x 1 (57) 19.5 /
-  // 15.7, 1187 x 1 (112) 35.1 / 24.6, 2048 x 1 (192) 53.2 / 38.8, 2048 x 4 (192) 31.0 / 26.0, 3600 x 1 (338) 89.7 / 97.2; 28 / 4
-  // heads 600 x 1 (132) 21.4 / 16.0, 1000 x 3 (219) 16.8 / 19.3.
-  const bool few = wgs <= 340, teams = wgs <= 200;
-  if (few) tiles = ((long)max_q_len * a.R + 63) / 64;
+  const int shape = sink_prefill_shape(d, nseq, rows, max_q_len, a.R, G, sink_reach(chunk, window), (long)bt_stride * SP_BS);
+  const long per = shape == 2 ? 128 : 64, tiles = ((long)max_q_len * a.R + per - 1) / per;
   if (tiles * nseq * G > 0x7fffffffL - (tiles > 0 ? tiles : 0)) return hipErrorInvalidValue;
   a.tiles = (int)tiles, a.nseq = nseq;
   const dim3 grid((unsigned)(tiles * nseq * G));
 #define SINK_PREFILL(DD, CAP)                                                                                           \
   {                                                                                                                     \
-    if (teams) hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 16, 2>), grid, dim3(512), 0, st, a);                    \
-    else if (few) hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 16, 1>), grid, dim3(256), 0, st, a);                 \
+    if (shape == 0) hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 16, 2>), grid, dim3(512), 0, st, a);               \
+    else if (shape == 1) hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 16, 1>), grid, dim3(256), 0, st, a);          \
     else hipLaunchKernelGGL((sink_prefill_kernel<DD, CAP, 32, 1>), grid, dim3(256), 0, st, a);                          \
   }
   if (d == 64 && softcap > 0.f) SINK_PREFILL(64, true)

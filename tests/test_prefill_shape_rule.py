@@ -1,4 +1,4 @@
-"""Which workgroups a prompt attention takes (csrc/kernels/attention.hip prefill_shape): within a
+"""Which workgroups a prompt attention takes (csrc/kernels/attention.hip prefill_shape, sink_prefill.hip sink_prefill_shape): within a
 sixth of the best of the shapes that were timed, us by shape."""
 import pytest
 
@@ -17,12 +17,27 @@ def test_prompt_shape(D, n, tokens, most, G, heads, us):
     assert us[lib().grag_prefill_attn_shape(D, n, tokens, most, G, heads)] <= 1.17 * min(us)
 
 
+# D, portions, tokens, longest, heads a kv head, kv heads, window, blocks of the table, us of 64 rows by two teams / 64 / 128 rows
+SINK = [(128, 40, 800, 52, 7, 4, 0, 4, (18.8, 11.8, 11.1)), (128, 12, 480, 57, 7, 4, 0, 4, (12.0, 8.2, 8.3)),
+        (128, 24, 1536, 64, 6, 2, 0, 4, (13.9, 8.6, 8.6)), (128, 1, 1187, 1187, 6, 2, 0, 75, (24.3, 34.4, 45.0)),
+        (128, 4, 4000, 1549, 6, 2, 256, 97, (45.1, 32.0, 26.6)), (64, 8, 256, 55, 1, 12, 0, 4, (5.5, 4.6, 5.2)),
+        # a table of two blocks, and 1000 cached keys before each portion
+        (128, 4, 120, 30, 7, 4, 0, 2, (7.7, 6.3, 8.0)), (128, 4, 120, 30, 7, 4, 0, 65, (22.6, 32.1, 40.6))]
+
+
+@pytest.mark.parametrize("D,n,tokens,most,R,heads,window,blocks,us", SINK)
+def test_sink_shape(D, n, tokens, most, R, heads, window, blocks, us):
+    assert us[lib().grag_sink_prefill_shape(D, n, tokens, most, R, heads, 0, window, blocks)] <= 1.17 * min(us)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_any_sizes(D):
     """The smallest and largest that the launchers take have a shape."""
     for n, tokens, most, G, heads in [(1, 1, 1, 1, 1), (1, 1 << 20, 1 << 20, 16, 16), (65535, 65535, 1, 7, 4), (3, 5, 5, 48, 1)]:
         assert 0 <= lib().grag_prefill_attn_shape(D, n, tokens, most, G, heads) <= 3
-    assert lib().grag_prefill_attn_shape(96, 1, 1, 1, 1, 1) == lib().grag_prefill_attn_shape(128, 0, 0, 0, 1, 1) == -1
+        for window in (0, 1, 1024):
+            assert 0 <= lib().grag_sink_prefill_shape(D, n, tokens, most, G, heads, 0, window, 2048) <= 2
+    assert lib().grag_prefill_attn_shape(96, 1, 1, 1, 1, 1) == lib().grag_sink_prefill_shape(128, 0, 0, 0, 1, 1, 0, 0, 1) == -1
 
 
 PAST = [0, 7, 64, 1, 900, 0, 63]
@@ -41,3 +56,20 @@ def test_every_prompt_shape(dev, D, H, G, lens, past, shape):
 
     assert lib().grag_prefill_attn_shape(D, len(lens), sum(lens), max(lens), H // G, G) == shape
     rows.test_rows(dev, D, H, G, lens, past, (0, 1 << 30))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["causal", "window", "kept", "block", "cap_low", "cap_high"])
+@pytest.mark.parametrize("D,H,G,lens,past,shape", [
+    (128, 12, 2, [33, 1, 65], [0, 900, 64], 0), (128, 28, 4, [17, 65, 65, 65, 65, 65, 1, 64, 33, 17, 33], (PAST * 2)[:11], 1),
+    (128, 28, 4, [64, 1, 64, 65, 65, 1, 64, 257, 100, 100, 257, 129, 17, 257], PAST * 2, 2),
+    (64, 16, 4, [33, 1, 17], [0, 900, 64], 0), (64, 24, 8, [640, 33, 1, 705], [0, 31, 64, 0], 1),
+    (64, 24, 8, [640, 33, 1, 705, 128, 321] * 2, [0, 31, 64, 0, 1, 0] * 2, 2)])
+def test_every_sink_shape(dev, D, H, G, lens, past, shape, form):
+    """Each shape against fp32 attention, by the check of test_sink_prefill_rows_gpu.py."""
+    import test_sink_prefill_rows_gpu as rows
+
+    kw = rows.FORMS[form]
+    width = -(-max(a + b for a, b in zip(lens, past)) // 16)
+    assert lib().grag_sink_prefill_shape(D, len(lens), sum(lens), max(lens), H // G, G, kw.get("chunk", 0), kw.get("window", 0), width) == shape
+    rows.check(dev, D, H, G, lens, past, form)
