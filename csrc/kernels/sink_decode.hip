@@ -201,6 +201,17 @@ bool sink_decode_takes(int d, int vd, int v_ld, int BS, int keep, const void* q,
   return (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0 && ((uintptr_t)out & 7) == 0;
 }
 
+// Waves a part: few parts are each a chain of tiles to be shared, many fill the chip by themselves; a wave's ring is 32 KB of LDS for
+// heads of 128 and 16 for heads of 64, so the lines lie where the parts of 4 waves, of 2 no longer have a place at once (heads of 64:
+// at twice as many parts).  us of 1 / 2 / 4 waves, cold keys, parts of keys: heads of
+// 128 1024 of 512 36.5 / 40.1 / 45.4, 640 of 256 20.5 / 23.6 / 24.9, 384 of 256 20.0 / 16.9 / 19.3, 332 of 20 7.0 / 5.8 / 8.8, 32 of 128 13.8 /
+// 11.5 / 10.8; heads of 64 1328 of 512 29.4 / 30.6 / 29.9, 1024 of 900 34.6 / 33.7 / 36.5, 768 of 256 15.0 / 13.3 / 13.4.
+static int sink_decode_waves(int D, long parts) {
+  const double places = (double)device_cus() * 128 / D;
+  return parts > 2.35 * places ? 1 : parts > 1.1 * places ? 2 : 4;
+}
+GRAG_API int grag_sink_decode_waves(int D, long parts) { return D < 1 ? -1 : sink_decode_waves(D, parts); }  // (for tests)
+
 hipError_t sink_decode_launch(const void* q, const void* k, const void* v, void* out, int out_ld, const int* bt, int bt_stride,
                               const int* ctx_len, const float* sinks, int nseq, int H, int G, int d, float scale, float out_scale,
                               int nblocks, int nsplit, int split_len, float* part_o, float* part_ml, const float* hscale,
@@ -214,17 +225,14 @@ hipError_t sink_decode_launch(const void* q, const void* k, const void* v, void*
   a.scale = scale, a.out_scale = out_scale, a.softcap = softcap;
   pa.nsplit = nsplit, pa.split_len = split_len, pa.part_o = part_o, pa.part_ml = part_ml;
   const dim3 grid(nsplit, G * ((a.R + 15) / 16), nseq);
-  // Waves a part: many parts fill the chip by themselves, few are each a chain of tiles to be shared.  us of 1 / 2 / 4 waves, parts
-  // of keys: 1024 of 512 36.1 / 40.1 / 43.8, 1024 of 256 25.1 / 28.1 / 32.6, 816 of 256 24.8 / 26.2 / 27.8, 512 of 256 18.4 / 15.4 /
-  // 17.6, 384 of 256 18.8 / 15.8 / 18.2, 192 of 256 17.1 / 12.3 / 11.1, 36 of 128 13.6 / 11.1 / 10.2; 512 of 1024 46.6 / 40.3 /
-  // 42.1, 256 of 1024 43.6 / 26.1 / 21.8.
   const long parts = (long)nsplit * G * ((a.R + 15) / 16) * nseq;
+  const int waves = sink_decode_waves(d, parts);
 #define SINK_DECODE_W(DD, CAP, NW) hipLaunchKernelGGL((sink_decode_kernel<DD, NW, CAP>), grid, dim3(64 * NW), 0, st, pa)
-#define SINK_DECODE(DD, CAP)                          \
-  {                                                   \
-    if (parts >= 768) SINK_DECODE_W(DD, CAP, 1);      \
-    else if (parts >= 384) SINK_DECODE_W(DD, CAP, 2); \
-    else SINK_DECODE_W(DD, CAP, 4);                   \
+#define SINK_DECODE(DD, CAP)                        \
+  {                                                 \
+    if (waves == 1) SINK_DECODE_W(DD, CAP, 1);      \
+    else if (waves == 2) SINK_DECODE_W(DD, CAP, 2); \
+    else SINK_DECODE_W(DD, CAP, 4);                 \
   }
   if (d == 64 && softcap > 0.f) SINK_DECODE(64, true)
   else if (d == 64) SINK_DECODE(64, false)

@@ -43,7 +43,7 @@ def test_sink_decode(H, G, D, splits, opts):
 
 
 @pytest.mark.parametrize("H,G,D", [(28, 4, 128), (12, 4, 64)])
-@pytest.mark.parametrize("n,splits", [(64, (4, 512)), (129, (1, 0))])  # from 512 parts on: two waves, eight and more tiles each
+@pytest.mark.parametrize("n,splits", [(64, (4, 512)), (129, (1, 0)), (129, (3, 704))])  # one and two waves, also of eight and more tiles
 @pytest.mark.parametrize("opts", [{}, dict(window=700), dict(chunk=1100, softcap=5.0), dict(scales=True, gate=True)])
 def test_many_parts(H, G, D, n, splits, opts):
     check([(i * 397 + 61) % 2048 + 1 for i in range(n)], H, G, D, splits, opts)
