@@ -371,44 +371,51 @@ __global__ __launch_bounds__(256) void topk_lists_merge_kernel(const float* __re
   const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t base = (int64_t)(q / G) * n * G + q % G;
   const uint32_t none = 0xFFFFFFFFu;
-  float h[kMergeLists / 256];
-#pragma unroll
-  for (int u = 0; u < kMergeLists / 256; ++u) {
-    const int j = u * 256 + tid;
-    h[u] = j < n ? ps[(base + (int64_t)j * G) * k] : -INFINITY;
-  }
   if (tid == 0) count = 0;
-  for (int r = 0; r < k; ++r) {
-    float v = -INFINITY;
-    uint32_t j = none;
+  int lists;
+  bool full;  // there are k lists with something, and more
+  if (n <= k) {  // every list may hold some: nothing is picked (1000 rows, k = 30, the whole search 72 -> 54 us)
+    if (tid < n) best[tid] = tid;
+    lists = n, full = false;
+  } else {
+    float h[kMergeLists / 256];
 #pragma unroll
-    for (int u = 0; u < kMergeLists / 256; ++u)
-      if (h[u] > v) v = h[u], j = u * 256 + tid;
-    const float top = wave_top(v);
-    uint32_t first = none;  // of the lanes that have it the lowest list
-    for (unsigned long long at = __ballot(v == top && j != none); at; at &= at - 1)
-      first = min(first, (uint32_t)__builtin_amdgcn_readlane((int)j, __ffsll(at) - 1));
+    for (int u = 0; u < kMergeLists / 256; ++u) {
+      const int j = u * 256 + tid;
+      h[u] = j < n ? ps[(base + (int64_t)j * G) * k] : -INFINITY;
+    }
+    for (int r = 0; r < k; ++r) {
+      float v = -INFINITY;
+      uint32_t j = none;
 #pragma unroll
-    for (int u = 0; u < kMergeLists / 256; ++u)
-      if (first == (uint32_t)(u * 256 + tid)) h[u] = -INFINITY;
-    if (lane == 0) hv[wave * 32 + r] = top, hj[wave * 32 + r] = first;
+      for (int u = 0; u < kMergeLists / 256; ++u)
+        if (h[u] > v) v = h[u], j = u * 256 + tid;
+      const float top = wave_top(v);
+      uint32_t first = none;  // of the lanes that have it the lowest list
+      for (unsigned long long at = __ballot(v == top && j != none); at; at &= at - 1)
+        first = min(first, (uint32_t)__builtin_amdgcn_readlane((int)j, __ffsll(at) - 1));
+#pragma unroll
+      for (int u = 0; u < kMergeLists / 256; ++u)
+        if (first == (uint32_t)(u * 256 + tid)) h[u] = -INFINITY;
+      if (lane == 0) hv[wave * 32 + r] = top, hj[wave * 32 + r] = first;
+    }
+    __syncthreads();
+    // of 4 k heads the best k: as many as are ahead of one
+    if (tid < 128) {
+      const int r = tid & 31;
+      const bool on = r < k && hj[tid] != none;
+      int rank = 0;
+      if (on)
+        for (int w = 0; w < 4; ++w)
+          for (int i = 0; i < k; ++i) rank += ahead(hv[w * 32 + i], hj[w * 32 + i], hv[tid], hj[tid]) && hj[w * 32 + i] != none;
+      if (on && rank < k) best[rank] = hj[tid];
+      if (on && rank == k - 1) last_v = hv[tid], last_j = hj[tid];
+      const int got = __popcll(__ballot(on));
+      if (lane == 0) atomicAdd(&count, got);
+    }
+    __syncthreads();
+    lists = min(count, k), full = count >= k;  // (heads that are there: no list without one has anything)
   }
-  __syncthreads();
-  // of 4 k heads the best k: as many as are ahead of one
-  if (tid < 128) {
-    const int r = tid & 31;
-    const bool on = r < k && hj[tid] != none;
-    int rank = 0;
-    if (on)
-      for (int w = 0; w < 4; ++w)
-        for (int i = 0; i < k; ++i) rank += ahead(hv[w * 32 + i], hj[w * 32 + i], hv[tid], hj[tid]) && hj[w * 32 + i] != none;
-    if (on && rank < k) best[rank] = hj[tid];
-    if (on && rank == k - 1) last_v = hv[tid], last_j = hj[tid];
-    const int got = __popcll(__ballot(on));
-    if (lane == 0) atomicAdd(&count, got);
-  }
-  __syncthreads();
-  const int lists = min(count, k), full = count >= k;  // (heads that are there: no list without one has anything)
   __syncthreads();
   if (tid == 0) count = 0;
   __syncthreads();

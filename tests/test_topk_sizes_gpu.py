@@ -46,7 +46,7 @@ def test_flat_scan(dev, rows, nq, k, d, filt):
         assert len(set(row)) == len(row)
 
 
-@pytest.mark.parametrize("n,k", [(1, 4), (2, 32), (255, 10), (257, 1), (1024, 32), (1000, 17)])
+@pytest.mark.parametrize("n,k", [(1, 4), (2, 32), (17, 17), (18, 17), (32, 32), (33, 32), (255, 10), (257, 1), (1024, 32), (1000, 17)])
 def test_merge_orders_ties_by_list(dev, n, k):
     """Lists of equal and of missing values: the best k by value, then list, then place."""
     g = torch.Generator(device=dev).manual_seed(n + k)
