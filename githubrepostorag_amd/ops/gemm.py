@@ -143,6 +143,33 @@ def _prefill_table() -> dict:
     return _PREFILL["table"]
 
 
+def _prefill_row(M: int, N: int, K: int, silu: bool = False) -> list | None:
+    """The measured row whose owned kernel a product takes, or None: the shape is not measured, or the library's."""
+    t = _prefill_table().get((N, K, int(silu)))
+    if t is None:
+        return None
+    ms, rows = t
+    i = bisect.bisect_left(ms, M)
+    cand = [rows[min(i, len(rows) - 1)]]
+    if 0 < i < len(rows) and ms[i] != M:
+        cand.append(rows[i - 1])
+    # SwiGLU: owned at every bucket; plain GEMMs: owned unless the library was clearly faster (OWN_SLACK:
+    # near-ties, within box-to-box spread, go to the owned kernel).  A row of six columns is owned whatever the library takes:
+    # 210 buckets that the owned kernel had by timings with 20 us of launch in them.  One after another in a graph over cold
+    # weights, library over owned 0.97 in the geometric mean there (0.71 at worst, 1024 x 4096 at 384 rows 14.5 / 20.4 us;
+    # 1024 x 1024 at 2944 14.3 / 12.7), 0.84 and 0.41 if the 256 x 256 tile took them all (2944 rows 22.5)
+    won = [r for r in cand if r[2] is not None and (silu or r[1] is None or len(r) > 5 or r[2] < r[1] * OWN_SLACK)]
+    # a bucket with M's own row-tile count ran on the identical tile grid: its schedule transfers as is
+    same = [r for r in won if -(-r[0] // 256) == -(-M // 256)]
+    return (same or won or [None])[0]
+
+
+def stays_owned(M: int, N: int, K: int) -> bool:
+    """Whether a product is owned only for its bucket's sixth column."""
+    row = _prefill_row(M, N, K)
+    return row is not None and len(row) > 5
+
+
 def prefill_plan(M: int, N: int, K: int, silu: bool = False) -> tuple[int, int] | None:
     """(ksplit, sk) of the owned kernel for a prefill-sized GEMM, or None for the library.
 
@@ -156,26 +183,12 @@ def prefill_plan(M: int, N: int, K: int, silu: bool = False) -> tuple[int, int] 
     own row-tile grid is preferred (its schedule was measured on the identical tile count), and a tail-only
     stream-K grid is re-derived for M's own remainder (``_tail_grid``).  Unmeasured shapes: None (library)
     for plain GEMMs, ``plan`` for SwiGLU."""
-    t = _prefill_table().get((N, K, int(silu)))
-    if t is None:
+    row = _prefill_row(M, N, K, silu)
+    if row is None:
         return plan(M, N, K) if silu else None
-    ms, rows = t
-    i = bisect.bisect_left(ms, M)
-    cand = [rows[min(i, len(rows) - 1)]]
-    if 0 < i < len(rows) and ms[i] != M:
-        cand.append(rows[i - 1])
-    # SwiGLU: owned at every bucket; plain GEMMs: owned unless the library was clearly faster (OWN_SLACK:
-    # near-ties, within box-to-box spread, go to the owned kernel)
-    won = [r for r in cand if r[2] is not None and (silu or r[1] is None or r[2] < r[1] * OWN_SLACK)]
-    if not won:
-        return plan(M, N, K) if silu else None
-    # a bucket with M's own row-tile count ran on the identical tile grid: its schedule transfers as is
-    same = [r for r in won if -(-r[0] // 256) == -(-M // 256)]
-    if same:
-        won = same
-    ks, sk = won[0][3], won[0][4]
+    ks, sk = row[3], row[4]
     if ks == 1 and sk < 0:
-        sk = _tail_grid(won[0][0], M, N, sk)
+        sk = _tail_grid(row[0], M, N, sk)
     return (ks, sk) if sk_ok(M, N, K, ks, sk) else (1, 0)
 
 
@@ -266,9 +279,14 @@ def pair_plan(M: int, N: int, K: int, fused: bool = False) -> int | None:
     (20 rows 4.5 / 6.0).  Fused, K <= 2048: 64 x 64 up to 704 tiles, then 64 x 128 and 128 x 128 up to 512 each, against the
     256 x 256 tile (GELU 3072 x 768 at 300 / 1136 / 1752 / 2500 rows 24 / 31 / 42 / 45 -> 6.9 / 12.3 / 17.5 / 19.9, from 4200 on 29
     / 33; SwiGLU 4096 x 1024 260 27 -> 10, 17920 x 1536 300 35 -> 29, 400 36 / 49; 22016 x 4096 260 80 / 104)."""
-    if not _ON or M < 1 or max(M, N) * K >= 1 << 30 or K > (2048 if fused else 1024):
+    if not _ON or M < 1 or max(M, N) * K >= 1 << 30:
         return None
     ncu = _num_cus()
+    if not fused and M >= PREFILL_MIN_M and not (K <= 1024 and _pair_tiles(3, M, N) <= 2 * ncu):
+        row = _prefill_row(M, N, K)  # a measured shape of its own
+        return row[5] if row is not None and len(row) > 5 and row[5] >= 0 else None
+    if K > (2048 if fused else 1024):
+        return None
     if not fused:
         return 3 if M >= 33 and _pair_tiles(3, M, N) <= 2 * ncu else None
     if _pair_tiles(3, M, N) <= 2.75 * ncu:

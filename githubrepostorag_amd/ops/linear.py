@@ -375,6 +375,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> t
         if kind == "tile_prefill":
             p = _tile.prefill_plan(M, N, K)
             if p is not None:
+                if _tile.stays_owned(M, N, K) and not _plain_product(x, w, b, align=2):
+                    return torch.nn.functional.linear(x, w, b)
                 return _tile.gemm(x, w, b, ksplit=p[0], sk=p[1])
             if _plain_product(x, w, b):
                 p = _tile.wide_plan(M, N, K) or _tile.unmeasured_plan(M, N, K)

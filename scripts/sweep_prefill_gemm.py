@@ -237,6 +237,8 @@ def main():
         merged = dict(old["table"])
         for key, rows in table.items():  # rows below the sweep's range (decode-batch rows) are kept
             lo = min(r[0] for r in rows)
+            kept = {r[0]: r[5:] for r in merged.get(key, [])}  # (buckets that stay on the owned kernels)
+            rows = [r + kept.get(r[0], []) for r in rows]
             merged[key] = sorted([r for r in merged.get(key, []) if r[0] < lo] + rows)
         extra = {k: v for k, v in old.items() if k not in ("arch", "note", "mstep", "table")}
         extra["resweep"] = f"{sorted(table)} re-swept ({round(time.time() - t_start, 1)} s)"

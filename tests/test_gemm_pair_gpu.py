@@ -89,6 +89,22 @@ def test_linear(dev, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,shape", [(2944, 1024, 1024, 3), (640, 1024, 4096, 3), (2900, 1024, 4096, 2), (6528, 1024, 1024, 1),
+                                         (2150, 2048, 1536, 0), (10880, 1024, 4096, None)])
+def test_linear_of_a_bucket_that_stays_owned(dev, monkeypatch, M, N, K, shape):
+    """Measured products that keep the owned kernels: the tile of the bucket's row, bit for bit the 256 x 256 tile's; a gradient
+    on the library's."""
+    x, w, b = _mk(dev, M, N, K)
+    monkeypatch.setattr(G, "gemm_pair", lambda *a, _f=G.gemm_pair, **k: took.append(a[3]) or _f(*a, **k))
+    took = []
+    y = L.linear(x, w, b)
+    assert took == ([] if shape is None else [shape]) and torch.equal(y, G.gemm(x, w, b, ksplit=1, sk=0))
+    torch.testing.assert_close(y.double(), x.double() @ w.double().T + b.double(), **TOL)
+    w.requires_grad_(True)
+    assert L.linear(x, w, b).requires_grad
+
+
+@pytest.mark.gpu
 def test_captured_without_an_eager_step(dev):
     """A product that has no slab can be captured before any eager one."""
     x, w, b = _mk(dev, 100, 3072, 768)

@@ -1,7 +1,9 @@
 """Decode-GEMM dispatch rules of ops/linear.py (CPU: predicates only; the
 numerics of every path are in tests/test_kernels_gpu.py)."""
+import pytest
 import torch
 
+from githubrepostorag_amd.ops import linear as L
 from githubrepostorag_amd.ops.linear import splitk_parts, use_splitk
 from githubrepostorag_amd.ops import gemm as G
 
@@ -93,6 +95,23 @@ def test_prefill_plan_schedules_pass_launcher_rule():
                     assert G.sk_ok(M, N, K, *p), (M, N, K, p)
     finally:
         G._num_cus = G_ncu
+
+
+@pytest.mark.parametrize("N,K,Ms", [(1024, 1024, (384, 2944, 8320, 16256)), (1024, 4096, (384, 2944, 10880, 16256)),
+                                    (1536, 1536, (2944, 10624)), (2048, 1536, (640, 8064)), (3072, 1024, (896, 16256)),
+                                    (4096, 1024, (640, 12160)), (4608, 3584, (384, 2176)), (3584, 3584, (1408, 4480))])
+def test_buckets_that_stay_owned(monkeypatch, N, K, Ms):
+    """Products that ran on the owned kernels keep them where a finer timing puts the library ahead: also with operands that
+    the small tiles don't take, and between two buckets."""
+    monkeypatch.setattr(G, "_num_cus", lambda: 256)
+    G.pair_plan.cache_clear()
+    for M in Ms:
+        for m in (M, M - 100):
+            shape = G.pair_plan(m, N, K)
+            assert L.kernel_for(m, N, K) == ("tile_prefill" if shape is None else "pair")
+            assert L.kernel_for(m, N, K, pair_ok=False) == "tile_prefill"
+            assert G.sk_ok(m, N, K, *G.prefill_plan(m, N, K))
+    G.pair_plan.cache_clear()
 
 
 def test_sk_ok_mirrors_launcher():
