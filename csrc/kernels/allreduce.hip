@@ -139,14 +139,13 @@ __global__ __launch_bounds__(kThreads) void ar_oneshot_kernel(Peers peers, int r
 GRAG_API long grag_ar_data_offset() { return (long)kMaxBlocks * kMaxRanks * sizeof(unsigned) + 256; }
 GRAG_API long grag_ar_region_bytes(long slot_bytes) { return grag_ar_data_offset() + 2 * slot_bytes; }
 
-// Allocate a zeroed uncached (fine-grained) region that peers can map.
+// Allocate a zeroed uncached (fine-grained) region that peers can map.  There is no call to free one: ordinary memory over a freed
+// uncached region has read stale afterwards.
 GRAG_API int grag_ar_alloc(long bytes, void** ptr) {
   hipError_t e = hipExtMallocWithFlags(ptr, (size_t)bytes, hipDeviceMallocUncached);
   if (e != hipSuccess) return (int)e;
   return (int)hipMemset(*ptr, 0, (size_t)bytes);
 }
-// For the last moments of a process only: ordinary memory over a freed uncached region has read stale afterwards.
-GRAG_API int grag_ar_free(void* ptr) { return (int)hipFree(ptr); }
 // Zero a region that a new communicator takes over: behind everything in flight on the device (hipMemset waits for no
 // non-blocking stream), so that no launch of the communicator before writes its flags behind the zeros.
 GRAG_API int grag_ar_clear(void* ptr, long bytes) {

@@ -33,7 +33,7 @@ log = logging.getLogger(__name__)
 P, I, L = ctypes.c_void_p, ctypes.c_int, ctypes.c_long
 _SIGS = {
     "grag_ar_data_offset": ([], L), "grag_ar_region_bytes": ([L], L), "grag_ar_alloc": ([L, P], I),
-    "grag_ar_clear": ([P, L], I), "grag_ar_free": ([P], I), "grag_ar_get_handle": ([P, P], I), "grag_ar_handle_size": ([], I),
+    "grag_ar_clear": ([P, L], I), "grag_ar_get_handle": ([P, P], I), "grag_ar_handle_size": ([], I),
     "grag_ar_open_handle": ([P, P], I), "grag_ar_close_handle": ([P], I),
     "grag_ar_oneshot": ([P, I, I, P, P, L, L, P, P, I, L, P], I),
     "grag_ar_oneshot_op": ([P, I, I, I, P, P, L, L, P, P, I, L, P], I),

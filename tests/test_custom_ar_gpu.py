@@ -161,7 +161,6 @@ def _ipc_worker(rank, world, port, q):
         dist.barrier()
         _fn("grag_ar_close_handle")(p.value)
         dist.barrier()
-        _fn("grag_ar_free")(base)
         dist.destroy_process_group()
         q.put((rank, ok, ""))
     except Exception as e:  # report, never hang the parent
