@@ -25,14 +25,8 @@ typedef __attribute__((address_space(3))) bf16x4_t sp_lds4_t;
 template <int D> __device__ __forceinline__ int sp_kswz(int row) { return D == 128 ? row & 15 : (row >> 1) & 7; }
 template <int D> __device__ __forceinline__ int sp_vswz(int row) { return D == 128 ? (row & 7) << 1 : ((row >> 1) & 3) << 1; }
 
-// 16 bytes a lane from `off` bytes behind a wave-uniform base of `bytes` bytes into 1 KB of LDS, lane after lane
-__device__ __forceinline__ void sp_dma(const bf16* base, int bytes, int off, char* dst) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000), (sp_lds_t*)dst, 16,
-                                           off, 0, 0, 0);
-}
-
-// The same from a wave-uniform base, with no bound, in a form whose wait the compiler leaves to the caller: it puts one for
-// everything in flight before each transposed read behind the builtin.
+// 16 bytes a lane from `off` bytes behind a wave-uniform base, with no bound, into 1 KB of LDS, lane after lane, in a form whose
+// wait the compiler leaves to the caller: behind the builtin it puts one for everything in flight before each transposed read.
 __device__ __forceinline__ void sp_dma_s(const bf16* base, unsigned off, char* dst) {
   const unsigned lds = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(sp_lds_t*)dst);
   unsigned keep;

@@ -37,6 +37,7 @@ template <int MT, int NT, int ST>
 __device__ __forceinline__ void pair_loop(char* smem, const void* A, int a_bytes, const void* W, int w_bytes,
                                           const unsigned (&offA)[MT], const unsigned (&offB)[NT], int nk,
                                           f32x4_t (&acc)[MT][NT]) {
+  static_assert(ST == 2 || ST == 3, "the waits below");
   constexpr int STAGE = kPairStage<MT, NT>, P = MT + NT;
   const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(A), 0, a_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(W), 0, w_bytes, 0x00020000);
@@ -80,7 +81,6 @@ __device__ __forceinline__ void pair_loop(char* smem, const void* A, int a_bytes
   // step t has landed when only the ST - 1 (at the end: fewer) steps behind it are in flight
   auto landed = [&](int behind) __attribute__((always_inline)) {
     if (behind >= ST - 1) pair_wait_vm<(ST - 1) * P>();
-    else if (ST > 3 && behind == 2) pair_wait_vm<2 * P>();
     else if (ST > 2 && behind == 1) pair_wait_vm<P>();
     else pair_wait_vm<0>();
   };
@@ -96,7 +96,6 @@ __device__ __forceinline__ void pair_loop(char* smem, const void* A, int a_bytes
     if (t + 1 < nk) {
       // the own reads of this buffer and the own pieces of step t + 1 are there; behind the barrier everyone's
       if (t + ST <= nk) pair_wait_vm<(ST - 2) * P>();
-      else if (ST > 3 && t + 3 == nk) pair_wait_vm<P>();
       else pair_wait_vm<0>();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       pair_bar();
