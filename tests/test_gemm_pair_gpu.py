@@ -76,10 +76,15 @@ def test_rule(monkeypatch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(40, 768, 768), (300, 2304, 768), (700, 18944, 1536), (8000, 2304, 768)])
-def test_linear(dev, M, N, K):
+@pytest.mark.parametrize("M,N,K,kind,shape", [(40, 768, 768, "pair", 3), (300, 2304, 768, "pair", 3), (700, 18944, 1536, "tile_prefill", None),
+                                              (8000, 2304, 768, "tile_prefill", 0)])
+def test_linear(dev, monkeypatch, M, N, K, kind, shape):
     """Plain products that linear() runs here, with a gradient on the library's."""
     x, w, b = _mk(dev, M, N, K)
+    took = []
+    monkeypatch.setattr(G, "gemm_pair", lambda *a, _f=G.gemm_pair, **k: took.append(a[3]) or _f(*a, **k))
+    assert L.kernel_for(M, N, K) == kind
+    assert torch.equal(L.linear(x, w, b), G.gemm(x, w, b, ksplit=1, sk=0)) and took == ([] if shape is None else [shape])
     ref = x.double() @ w.double().T + b.double()
     torch.testing.assert_close(L.linear(x, w, b).double(), ref, **TOL)
     w.requires_grad_(True)

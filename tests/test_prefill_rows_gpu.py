@@ -1,5 +1,6 @@
-"""Paged prefill attention by rows a workgroup (csrc/kernels/attention.hip launch_prefill: 64, with one or two teams of
-waves, 128 or 256 by all rows) against fp32 attention: portions that end beside a workgroup's and a wave's rows, cached tokens before some, one of one token."""
+"""Paged prefill attention (csrc/kernels/attention.hip launch_prefill) against fp32 attention over rising numbers of rows:
+portions that end beside a workgroup's and a wave's rows, cached tokens before some, one of one token.  Which shape of workgroup
+each takes is established in test_prefill_shape_rule.py."""
 import pytest
 import torch
 

@@ -1,9 +1,10 @@
-"""The prefill attention's 128-row workgroups of 32-row waves (csrc/kernels/sink_prefill.hip) against the plain fp32 attention:
-portions that end at and beside their edges and those of the waves, cached tokens before some, walks whose last tile is one
-key, and caps met by the power series and by tanhf."""
+"""The prefill attention's workgroups (csrc/kernels/sink_prefill.hip: 128 rows, or 64 by one or two teams of waves) against the
+plain fp32 attention: portions that end at and beside their edges and those of the waves, cached tokens before some, walks whose
+last tile is one key, and caps met by the power series and by tanhf."""
 import pytest
 import torch
 
+from githubrepostorag_amd.ops._lib import lib
 from githubrepostorag_amd.ops.attention import AttnMetadata, sink_attention, sink_attention_ref
 
 pytestmark = pytest.mark.gpu
@@ -16,8 +17,13 @@ FORMS = {"causal": {}, "window": dict(window=150), "kept": dict(window=90, keep=
 @pytest.mark.parametrize("D,H,G,lens,past", [
     (64, 24, 8, [640, 33, 1, 705, 128, 321], [0, 31, 64, 0, 1, 0]), (128, 28, 4, [1100, 16, 577, 64], [5, 0, 0, 63])])
 def test_rows(dev, D, H, G, lens, past, form):
-    assert -(-sum(lens) * (H // G) // 128) * G > 340  # the 128-row workgroups
+    assert shape(D, H, G, lens, past, form) == (1 if D == 64 else 2)  # one team of 64 rows, 128 rows
     check(dev, D, H, G, lens, past, form)
+
+
+def shape(D, H, G, lens, past, form):
+    kw, width = FORMS[form], -(-max(n + p for n, p in zip(lens, past)) // 16)
+    return lib().grag_sink_prefill_shape(D, len(lens), sum(lens), max(lens), H // G, G, kw.get("chunk", 0), kw.get("window", 0), width)
 
 
 def check(dev, D, H, G, lens, past, form):
@@ -50,8 +56,11 @@ def check(dev, D, H, G, lens, past, form):
 
 
 @pytest.mark.parametrize("form", sorted(FORMS))
-@pytest.mark.parametrize("D,H,G,lens,past", [(128, 12, 2, [300, 1, 65, 16], [0, 63, 1500, 700]), (64, 14, 2, [16], [0]), (64, 6, 1, [64, 65], [64, 0])])
-def test_two_teams(dev, D, H, G, lens, past, form):
-    """Few rows: two teams of waves on a walk's tiles, of which one may have none, or none that a row sees."""
-    assert -(-sum(lens) * (H // G) // 128) * G <= 200
+@pytest.mark.parametrize("D,H,G,lens,past,teams", [
+    (128, 12, 2, [300, 1, 65, 16], [0, 63, 1500, 700], 2), (64, 6, 1, [64, 1, 65], [900, 0, 0], 2), (64, 14, 2, [16], [0], 1),
+    (64, 6, 1, [64, 65], [64, 0], 1)])
+def test_two_teams(dev, D, H, G, lens, past, teams, form):
+    """Few rows: two teams of waves on a walk's tiles, of which one may have none, or none that a row sees; one team for the
+    shortest walks."""
+    assert shape(D, H, G, lens, past, form) == 2 - teams
     check(dev, D, H, G, lens, past, form)
