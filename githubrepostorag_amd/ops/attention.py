@@ -27,7 +27,8 @@ DECODE_NT_MIN_WAVES = int(os.environ.get("GRAG_DECODE_NT_MIN_WAVES", "0"))
 # multi-part plans over at least DECODE_NS3_ROWS (sequence x kv head) rows and of more waves than the chip holds at once with
 # 2-stage rings (5 a CU) take the 3-stage ring (3 a CU, as many bytes in flight): us of 11 / 12, 28 / 4 heads: B192 ctx3000 (1536
 # waves) 207 / 194, B176 ctx1500 (1408) 104 / 97.5, but B128 ctx1500 (1024) 71.8 / 82.8 and B128 of 130000 keys in all (1024) 56.3 / 75.0; parts of
-# unequal sequences are often empty, so that fewer rows rarely fill it (B83 of 68807 keys, 1328 parts: a step 781 / 803) (either 0: off)
+# unequal sequences are often empty, so that fewer rows rarely fill it (B83 of 68807 keys, 1328 parts: a step 781 / 803) (either 0: off;
+# waves of a device of 256 CUs)
 DECODE_NS3_ROWS = int(os.environ.get("GRAG_DECODE_NS3_ROWS", "512"))
 DECODE_NS3_WAVES = int(os.environ.get("GRAG_DECODE_NS3_WAVES", "1280"))
 _DEC_NT = os.environ.get("GRAG_DECODE_NT", "auto")
@@ -39,7 +40,7 @@ _DEC_NT = os.environ.get("GRAG_DECODE_NT", "auto")
 DECODE_MW = {22: 2, 24: 4}
 DECODE_MW_CODE = int(os.environ.get("GRAG_DECODE_MW_CODE", "24"))
 DECODE_MW_ROWS = int(os.environ.get("GRAG_DECODE_MW", "16"))
-DECODE_MW_PARTS = 200  # or sequences x kv heads x parts at most this many (decode_mw_takes)
+DECODE_MW_PARTS = 200  # or sequences x kv heads x parts at most this many on 256 CUs (decode_mw_takes)
 MW_SPLITS = int(os.environ.get("GRAG_DECODE_MW_SPLITS", "20"))  # target parts per sequence at B = 1
 
 
@@ -69,10 +70,10 @@ def decode_mw_takes(meta, Hkv: int) -> bool:
     counted, sequences x keys (parts): 28 / 4 heads 8 x 1000 (128) 15.3 / 14.6, 24 x 300 (192) 14.7 / 13.3, 5 x 3000 (240) 19.9 /
     22.5; 12 / 2 heads 16 x 300 (64) 14.4 / 11.7, 12 x 2000 (192) 17.7 / 16.1.  The latter not in a capture without an owner whose
     tickets are there: other kernels need none."""
-    from .gemm import WS
+    from .gemm import WS, _num_cus
 
     rows = meta.num_seqs * Hkv
-    few = meta.cascade is None and rows * meta.num_splits <= DECODE_MW_PARTS
+    few = meta.cascade is None and rows * meta.num_splits * 256 <= DECODE_MW_PARTS * _num_cus()
     return DECODE_MW_ROWS > 0 and (rows <= DECODE_MW_ROWS or few and WS.scratch_ok("decode_tickets"))
 
 
@@ -103,10 +104,12 @@ def decode_variant(nsplit: int, split_len: int, waves: int | None = None) -> int
     """Decode kernel per split plan, 32-key tiles.  ``waves``: the launch's (sequence x kv-head x split) count; more than
     DECODE_NS3_WAVES of several parts over DECODE_NS3_ROWS rows take the 3-stage ring, at least DECODE_NT_MIN_WAVES load K/V
     non-temporally (GRAG_DECODE_RING_AUTO=1: the 3-stage ring for parts that cover more than 2048 keys)."""
+    from .gemm import _num_cus
+
     auto3 = _DEC_AUTO and os.environ.get("GRAG_DECODE_RING_AUTO") == "1"
     nw = DECODE_RING_NW[3] if auto3 and nsplit > 1 and nsplit * split_len > 2048 else DECODE_NW
-    if (_DEC_AUTO and DECODE_NS3_ROWS and DECODE_NS3_WAVES and nsplit > 1 and waves is not None and waves > DECODE_NS3_WAVES
-            and waves // nsplit >= DECODE_NS3_ROWS):
+    if (_DEC_AUTO and DECODE_NS3_ROWS and DECODE_NS3_WAVES and nsplit > 1 and waves is not None
+            and waves * 256 > DECODE_NS3_WAVES * _num_cus() and waves // nsplit >= DECODE_NS3_ROWS):
         nw = DECODE_RING_NW[3]
     nt = _DEC_NT == "1" or (_DEC_NT == "auto" and waves is not None and waves >= DECODE_NT_MIN_WAVES)
     return DECODE_NT.get(nw, nw) if nt else nw

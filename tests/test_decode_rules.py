@@ -17,6 +17,19 @@ def test_ring_by_rows_and_waves(monkeypatch):
     assert A.decode_variant(2, 2048, 1536) == 11
 
 
+def test_rules_by_the_device(monkeypatch):
+    """A quarter of the CUs: a quarter of the parts that a launch's rules count."""
+    from types import SimpleNamespace
+
+    from githubrepostorag_amd.ops import gemm as G
+
+    monkeypatch.setattr(G.WS, "scratch_ok", lambda name: True)
+    meta = lambda n: SimpleNamespace(num_seqs=n, num_splits=2, cascade=None)  # noqa: E731
+    for ncu, most in ((256, 25), (64, 6)):
+        monkeypatch.setattr(G, "_NCU", [ncu])
+        assert A.decode_mw_takes(meta(most), 4) and not A.decode_mw_takes(meta(most + 1), 4)
+
+
 # D, parts, us of 1 / 2 / 4 waves
 @pytest.mark.parametrize("D,parts,us", [(128, 1024, (36.5, 40.1, 45.4)), (128, 640, (20.5, 23.6, 24.9)), (128, 384, (20.0, 16.9, 19.3)),
                                         (128, 332, (7.0, 5.8, 8.8)), (128, 32, (13.8, 11.5, 10.8)), (64, 1024, (34.6, 33.7, 36.5)),
