@@ -36,8 +36,9 @@ def _scan_cut(max_q: int, tokens: int, nseq: int, tiles: int, split: bool, d: in
     """Chunks of 64 tokens a part of the matrix-core scan (csrc/kernels/linscan.hip), for a step of ``nseq`` portions with
     ``tokens`` tokens, the longest ``max_q``, ``tiles`` (head, 64 columns) tiles a portion and ``d`` state rows: the cut that makes
     the step shortest, in walks of a chunk.  Workgroups start longest first, so several portions take the longest walk or
-    the chip's share of all and part of a walk for its uneven end; a single portion whole rounds of equal parts.  A walk of some chunks costs some more for its start and its state.  Where portions are cut, all parts but the
-    last are walked for the state alone before (about a quarter of a walk), and a part reads the states of those before it.
+    the chip's share of all and part of a walk for its uneven end; a single portion whole rounds of equal parts.  A walk of some
+    chunks costs some more for its start and its state.  Where portions are cut, all parts but the last are walked for the
+    state alone before (about a quarter of a walk), and a part reads the states of those before it.
     ``split``: operands in three parts (one workgroup a CU, 12 us a chunk), else two workgroups a CU and 5.7 us.
 
     From 455 points of 21 sizes, 1 - 20 portions, 65 - 8192 tokens, every cut timed: the cut taken is 1.015 of the best in the
@@ -76,8 +77,9 @@ def _scan_walks(max_q: int, tokens: int, nseq: int, tiles: float, split: bool) -
     """Walks of a 64-token chunk that a step of the matrix-core scan takes, as _scan_taken reckons (roughly; _scan_cut for the cut):
     ``nseq`` portions with ``tokens`` tokens, the longest ``max_q``, and ``tiles`` (head, 64 columns) tiles a portion, crowding
     counted.  Several portions take the longest walk or the chip's share of all and about a third of a walk for its uneven
-    end; a single portion whole rounds of equal parts.  Where portions are cut, all parts but the last are walked for the state alone before (0.42 of a
-    walk), and a part reads the states of those before it.  ``split``: operands in three parts (one workgroup a CU, 12 us a
+    end; a single portion whole rounds of equal parts.  Where portions are cut, all parts but the last are walked for the
+    state alone before (0.42 of a walk), and a part reads the states of those before it.  ``split``: operands in three parts (one
+    workgroup a CU, 12 us a
     chunk), else two workgroups a CU and 5.7 us."""
     slots, read, crowd = (256, 0.026, 1.0) if split else (512, 0.11, 1.2)  # (whole portions often have a CU of their own)
     chunks, total = -(-max_q // LINEAR_SCAN_CHUNK), tokens / LINEAR_SCAN_CHUNK + (nseq - 1) / 2
