@@ -60,6 +60,12 @@ __device__ __forceinline__ short f2bits(float f) {
   return __builtin_bit_cast(short, b);
 }
 
+// LDS-DMA: 16 bytes a lane from rs + off + soff to dst + 16 * lane (no template: the host's pass knows the builtin in none)
+typedef __attribute__((address_space(3))) void lds_t;
+__device__ __forceinline__ void lds_dma16(const __amdgpu_buffer_rsrc_t& rs, char* dst, unsigned off, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_t*)dst, 16, off, soff, 0, 0);
+}
+
 // The (sequence, kv head) stream and the tile of a sequence that workgroup `id` of a causal prompt attention walks: longest walks first,
 // the last tile of every sequence, the last but one, and so on.  Workgroups are dealt to the shader engines in turn, 8 XCDs of 4, and
 // run where they were dealt; each tile number's streams are turned against those before it, so that every engine meets every

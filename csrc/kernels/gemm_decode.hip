@@ -39,7 +39,7 @@
 //     (ops/gemm.py interleave_gate_up): a wave's two n-tiles are then the 16
 //     gate rows and the 16 matching up rows, so the product forms in registers.
 
-#include "common.h"
+#include "act.h"
 
 using namespace grag;
 
@@ -49,20 +49,6 @@ GRAG_API int grag_splitk_reduce(const void* ws, const void* bias, void* C, int l
 namespace {
 
 enum { EPI_STORE = 0, EPI_SILU = 1, EPI_PARTIAL = 2 };
-
-enum { ACT_NONE = 0, ACT_GELU = 1, ACT_GELU_TANH = 3 };
-
-__device__ __forceinline__ float silu_f(float x) { return x / (1.f + __expf(-x)); }
-__device__ __forceinline__ float gelu_tanh_f(float x) {
-  const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-  return 0.5f * x * (2.f - 2.f * __builtin_amdgcn_rcpf(1.f + __expf(2.f * u)));
-}
-template <int ACT>
-__device__ __forceinline__ float act_f(float x) {
-  if constexpr (ACT == ACT_GELU) return gelu_erf(x);
-  else if constexpr (ACT == ACT_GELU_TANH) return gelu_tanh_f(x);
-  else return x;
-}
 
 // LDS-DMA piece (1 KiB per wave instruction, lane-linear at wave-uniform lds_dst); M0 saved/set/restored in
 // one statement; completion tracked only by the caller's counted vmcnt.

@@ -8,6 +8,7 @@
 // three steps in flight; 300 rows of 3072 x 768 with GELU 24 us as K parts and their sum -> 6.9).  Over many rounds 128 x 192
 // tiles reach 1.15 PF/s where 256 x 256 ones reach 1.45: per product they fetch 1.7 times the bytes, and the LDS-DMA of a CU is
 // busy (without it the same loop runs at 1.6, without the fragment reads at 1.3).  Measured: ops/gemm.py pair_plan.
+#include "act.h"
 #include "tile_pair.h"
 
 using namespace grag;
@@ -15,7 +16,6 @@ using namespace grag;
 namespace {
 
 enum { EPI_STORE = 0, EPI_SILU = 1, EPI_GLU = 3 };
-enum { ACT_NONE = 0, ACT_GELU = 1, ACT_GELU_TANH = 3 };
 
 struct PairArgs {
   const bf16* A;
@@ -30,20 +30,6 @@ struct PairArgs {
 };
 
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ float silu_f(float x) { return x / (1.f + __expf(-x)); }
-__device__ __forceinline__ float gelu_tanh_f(float x) {
-  const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-  return 0.5f * x * (2.f - 2.f * __builtin_amdgcn_rcpf(1.f + __expf(2.f * u)));
-}
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  return (uint32_t)(uint16_t)f2bits(lo) | ((uint32_t)(uint16_t)f2bits(hi) << 16);
-}
-template <int ACT> __device__ __forceinline__ float act_f(float x) {
-  if constexpr (ACT == ACT_GELU) return gelu_erf(x);
-  else if constexpr (ACT == ACT_GELU_TANH) return gelu_tanh_f(x);
-  else return x;
-}
 
 template <int MT, int NT, int ST, int EPI, int ACT>
 __global__ __launch_bounds__(kPairThreads, MT * NT >= 16 ? 2 : 3) void gemm_pair_kernel(PairArgs p) {

@@ -37,6 +37,7 @@
 // (LDS image lane-linear, rule 21) — conflict-free for the b128 lane groups.
 // The MFMA is issued with the W fragment as operand A, so each lane ends with
 // 4 consecutive output columns of one row: 8-byte bf16 / 16-byte fp32 stores.
+#include "act.h"
 #include "tile256.h"
 
 using namespace grag;
@@ -51,24 +52,6 @@ constexpr int kBuf = 4 * kSlot;   // one K-tile: A q0, A q1, B q0, B q1
 constexpr int kThreads = 512;
 
 enum { EPI_STORE = 0, EPI_SILU = 1, EPI_PARTIAL = 2, EPI_GLU = 3 };
-enum { ACT_NONE = 0, ACT_GELU = 1, ACT_SILU = 2, ACT_GELU_TANH = 3 };
-
-__device__ __forceinline__ float silu_f(float x) { return x / (1.f + __expf(-x)); }
-__device__ __forceinline__ float gelu_tanh_f(float x) {
-  const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-  return 0.5f * x * (2.f - 2.f * __builtin_amdgcn_rcpf(1.f + __expf(2.f * u)));
-}
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  return (uint32_t)(uint16_t)f2bits(lo) | ((uint32_t)(uint16_t)f2bits(hi) << 16);
-}
-template <int ACT>
-__device__ __forceinline__ float act_f(float x) {
-  if constexpr (ACT == ACT_GELU) return gelu_erf(x);
-  else if constexpr (ACT == ACT_SILU) return silu_f(x);
-  else if constexpr (ACT == ACT_GELU_TANH) return gelu_tanh_f(x);
-  else return x;
-}
-
 __device__ __forceinline__ void glds16(const void* g, char* l) {
   __builtin_amdgcn_global_load_lds((glb_void_t*)g, (lds_void_t*)l, 16, 0, 0);
 }

@@ -16,7 +16,7 @@
 //   * (s, -z*s) as float2 [rows][K/128], loaded per K-step (8 B per lane per tile, L2-resident);
 //   * rows are stored in the order the waves consume them; for the SwiGLU gate/up weight each 32-row block
 //     is [16 gate rows | the 16 matching up rows] so silu(g)*u forms in registers (EPI_SILU).
-#include "common.h"
+#include "act.h"
 
 // Diagnostic builds only (scripts/dev/w4_diag.py, never the shipped library): GRAG_W4_DIAG bit 0 drains
 // every load before each step's barrier (no loads in flight across compute), bit 1 pads the workgroup's LDS
@@ -35,22 +35,9 @@ GRAG_API int grag_splitk_reduce(const void* ws, const void* bias, void* C, int l
 namespace {
 
 enum { EPI_STORE = 0, EPI_SILU = 1, EPI_PARTIAL = 2 };
-enum { ACT_NONE = 0, ACT_GELU = 1, ACT_GELU_TANH = 3 };
 constexpr int kDepth = 4;   // K-steps issued ahead (ring of kDepth + 1 slots)
 
 constexpr int kGroup = 128; // quantisation group along K
-
-__device__ __forceinline__ float silu_f(float x) { return x / (1.f + __expf(-x)); }
-__device__ __forceinline__ float gelu_tanh_f(float x) {
-  const float u = 0.7978845608028654f * (x + 0.044715f * x * x * x);
-  return 0.5f * x * (2.f - 2.f * __builtin_amdgcn_rcpf(1.f + __expf(2.f * u)));
-}
-template <int ACT>
-__device__ __forceinline__ float act_f(float x) {
-  if constexpr (ACT == ACT_GELU) return gelu_erf(x);
-  else if constexpr (ACT == ACT_GELU_TANH) return gelu_tanh_f(x);
-  else return x;
-}
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) void glb_void_t;

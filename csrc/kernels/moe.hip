@@ -1053,7 +1053,7 @@ moe_gemm_tile_kernel(const bf16* __restrict__ a, int lda, int a_bytes, const bf1
 
 // 4 bytes a lane from rs + off to dst + 4 * lane (no template: the host's pass knows the builtin in none)
 __device__ __forceinline__ void moe_dma4(const __amdgpu_buffer_rsrc_t& rs, int* dst, unsigned off) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (tile_lds_t*)dst, 4, off, 0, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_t*)dst, 4, off, 0, 0, 0);
 }
 
 // The same as chains of tiles, one workgroup a CU (tile256_chain): the next tile's source rows come to LDS while one is

@@ -8,8 +8,6 @@
 
 namespace grag {
 
-typedef __attribute__((address_space(3))) void tile_lds_t;
-
 constexpr int kTileSlot = 128 * 128;        // bytes: 128 rows x 64 bf16
 constexpr int kTileBuf = 4 * kTileSlot;     // one K step: A q0, A q1, B q0, B q1
 constexpr int kTileThreads = 512;
@@ -50,11 +48,6 @@ __device__ __forceinline__ int tile_piece_row(int i) {
   return (2 * (threadIdx.x >> 6) + i) * 8 + ((threadIdx.x & 63) >> 3);
 }
 __device__ __forceinline__ int tile_piece_chunk(int i) { return (threadIdx.x & 7) ^ ((tile_piece_row(i) >> 1) & 7); }
-
-// 16 bytes a lane from rs + off + soff to dst + 16 * lane (no template: the host's pass knows the builtin in none)
-__device__ __forceinline__ void tile_dma(const __amdgpu_buffer_rsrc_t& rs, char* dst, unsigned off, int soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (tile_lds_t*)dst, 16, off, soff, 0, 0);
-}
 
 // Two-phase schedule: 32 MFMAs per barrier interval.  Per K step t (buffer b = t & 1):
 //   L1 reads A q0, B q0, B q1 (16 b128)  refill A q1 of step t+1 (buffer b^1; read there in L2(t-1))
@@ -97,13 +90,13 @@ __device__ __forceinline__ void tile256_loop(char* smem, const __amdgpu_buffer_r
   auto issueA = [&](int q, int kt, int buf) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, (tile_lds_t*)(smem + buf * kTileBuf + q * kTileSlot + (2 * w + i) * 1024),
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, (lds_t*)(smem + buf * kTileBuf + q * kTileSlot + (2 * w + i) * 1024),
                                                16, offA[q][i], kt * 128, 0, 0);
   };
   auto issueB = [&](int q, int kt, int buf) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, (tile_lds_t*)(smem + buf * kTileBuf + (2 + q) * kTileSlot + (2 * w + i) * 1024),
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, (lds_t*)(smem + buf * kTileBuf + (2 + q) * kTileSlot + (2 * w + i) * 1024),
                                                16, offB[q][i], kt * 128, 0, 0);
   };
   TileA a;
@@ -204,12 +197,12 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
   };
   auto issueA = [&](const TileOff& o, int q, int kt, int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) tile_dma(rsA, smem + buf * kTileBuf + q * kTileSlot + (2 * w + i) * 1024, o[2 * q + i], kt * 128);
+    for (int i = 0; i < 2; ++i) lds_dma16(rsA, smem + buf * kTileBuf + q * kTileSlot + (2 * w + i) * 1024, o[2 * q + i], kt * 128);
   };
   auto issueB = [&](const TileOff& o, int q, int kt, int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      tile_dma(rsB, smem + buf * kTileBuf + (2 + q) * kTileSlot + (2 * w + i) * 1024, o[4 + 2 * q + i], kt * 128);
+      lds_dma16(rsB, smem + buf * kTileBuf + (2 + q) * kTileSlot + (2 * w + i) * 1024, o[4 + 2 * q + i], kt * 128);
   };
   TileA a;
   TileB b0, b1;

@@ -8,8 +8,6 @@
 
 namespace grag {
 
-typedef __attribute__((address_space(3))) void pair_lds_t;
-
 constexpr int kPairThreads = 256;
 template <int MT, int NT> constexpr int kPairStage = (MT + NT) * 4096;  // bytes of a K step: 32 MT rows of A, 32 NT of B
 
@@ -23,11 +21,6 @@ __device__ __forceinline__ void pair_bar() {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-}
-
-// 16 bytes a lane from rs + off + soff to dst + 16 * lane (no template: the host's pass knows the builtin in none)
-__device__ __forceinline__ void pair_dma(const __amdgpu_buffer_rsrc_t& rs, char* dst, unsigned off, int soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (pair_lds_t*)dst, 16, off, soff, 0, 0);
 }
 
 // acc += A B^T over nk >= 1 K steps.  offA / offB: byte offsets of the thread's DMA pieces at the first step (pair_piece_row /
@@ -49,10 +42,10 @@ __device__ __forceinline__ void pair_loop(char* smem, const void* A, int a_bytes
   auto issue = [&](int kt, int buf) {
 #pragma unroll
     for (int i = 0; i < MT; ++i)
-      pair_dma(rsA, smem + buf * STAGE + (4 * i + w) * 1024, offA[i], kt * 128);
+      lds_dma16(rsA, smem + buf * STAGE + (4 * i + w) * 1024, offA[i], kt * 128);
 #pragma unroll
     for (int i = 0; i < NT; ++i)
-      pair_dma(rsB, smem + buf * STAGE + (4 * (MT + i) + w) * 1024, offB[i], kt * 128);
+      lds_dma16(rsB, smem + buf * STAGE + (4 * (MT + i) + w) * 1024, offB[i], kt * 128);
   };
 #pragma unroll
   for (int m = 0; m < MT; ++m)
