@@ -39,6 +39,7 @@ _SIGS = {
     "grag_bias_act": [P, P, P, I, I, I, P],
     "grag_pool_l2norm": [P, P, P, P, P, I, I, I, I, I, P],
     "grag_paged_attention": [P, I, P, P, P, I, P, I, P, P, I, I, I, I, I, I, I, F, I, I, I, P, P, I, I, P],
+    "grag_prefill_attn_shape": [I, I, I, I, I, I],
     "grag_splitk_add_rmsnorm_small": [P, I, P, P, P, I, I, F, P, P, P],
     "grag_paged_decode_mw": [P, I, P, P, P, I, P, I, P, P, I, I, I, I, I, I, F, I, I, P, P, P, I, I, P],
     "grag_paged_decode_mw_rope": [P, I, P, P, P, P, P, P, P, I, P, I, P, P, I, I, I, I, I, I, F, I, I, P, P, P, I, I, I,
@@ -88,6 +89,8 @@ _SIGS = {
     "grag_rope_vnorm_store": [P, I, I, I, I, P, P, I, P, P, P, P, I, I, I, I, I, I, I, ctypes.c_long, F, I, I, P, P, P, P],
     "grag_sink_attn_prefill": [P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, I, I, F, F, I, I, I, P, P, I, I, I, F, I, P],
     "grag_sink_attn_decode": [P, P, P, P, I, P, I, P, P, I, I, I, I, I, I, F, F, I, I, I, I, P, P, I, P, P, I, I, I, F, I, P],
+    "grag_sink_prefill_shape": [I, I, I, I, I, I, I, I, I],
+    "grag_sink_decode_waves": [I, L],
     "grag_relu2": [P, I64, I, P],
     "grag_decay_attn_scan": [P, I, I, I, I, P, P, P, P, P, P, I, I, I, I, I, I, P, I, I, P, P, I, I, F, P],
     "grag_decay_attn_chunk": [],
