@@ -90,7 +90,7 @@ _SIGS = {
     "grag_sink_attn_prefill": [P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, I, I, F, F, I, I, I, P, P, I, I, I, F, I, P],
     "grag_sink_attn_decode": [P, P, P, P, I, P, I, P, P, I, I, I, I, I, I, F, F, I, I, I, I, P, P, I, P, P, I, I, I, F, I, P],
     "grag_sink_prefill_shape": [I, I, I, I, I, I, I, I, I],
-    "grag_sink_decode_waves": [I, L],
+    "grag_sink_decode_waves": [I, I64],
     "grag_relu2": [P, I64, I, P],
     "grag_decay_attn_scan": [P, I, I, I, I, P, P, P, P, P, P, I, I, I, I, I, I, P, I, I, P, P, I, I, F, P],
     "grag_decay_attn_chunk": [],
