@@ -31,8 +31,11 @@
 //     the grid match the 256 CUs when U / NWV does not (Qwen2-7B gate/up at
 //     M > 128: 1184 units = 148 full 8-wave tiles, 58 % of the CUs; dealt as 4-5
 //     units to each of 256 five-wave workgroups every CU streams its share).
-//     A wave without a unit repeats its neighbour's loads (L2 hits) and stores
-//     nothing.  ksplit > 1 writes fp32 partial planes ws[split][M][N];
+//     A wave without a unit asks for one line again and again, so that every
+//     wave counts the same loads, and stores nothing (while it repeated its neighbour's
+//     rows, each of them a miss of its own, a workgroup of 2 - 3 units in 5 waves fetched
+//     twice what it used: 17920 x 1536, one row 20.1 -> 16.5 us, 18944 x 3584 in 4 waves
+//     36.5 -> 30.8, 64 rows 39.2 -> 36.2).  ksplit > 1 writes fp32 partial planes ws[split][M][N];
 //     grag_splitk_reduce (in gemm_tile.hip) sums them and applies the epilogue.
 //   * Epilogues fused in the kernel: bias + act (none / gelu-erf / gelu-tanh),
 //     SiLU(gate)*up for the gate/up weight stored interleaved in 32-row blocks
@@ -181,7 +184,7 @@ void gemm_dec_kernel(DArgs p) {
   const int u0 = (int)((long)g * p.units / p.gs);
   const int cnt = (int)((long)(g + 1) * p.units / p.gs) - u0;
   bool active = w < cnt;                          // wave-uniform
-  int q = u0 + min(w, cnt - 1);                   // this wave's unit (an idle wave repeats the last one)
+  int q = u0 + min(w, cnt - 1);                   // this wave's unit (an idle wave: the last one's number)
   if constexpr (TQ > 0) {
     if (w >= 4) {
       active = cnt > 4;
@@ -211,11 +214,14 @@ void gemm_dec_kernel(DArgs p) {
   // of one K-step are one contiguous block (row stride 64), the unit's K-steps follow each other, so a
   // wave streams one contiguous region (DRAM pages are read whole, not 128 B per row per K-step)
   const int kstride = p.packed ? 16 * NTW * 64 : 64;
+  const int kstep = active ? kstride : 0;  // a wave without a unit stays at the first line of the last one
   const bf16* wp[NTW];
 #pragma unroll
-  for (int nt = 0; nt < NTW; ++nt)
-    wp[nt] = p.packed ? p.W + (size_t)q * ks * kstride + (size_t)kb * kstride + (16 * nt + li) * 64 + 8 * h4
-                      : p.W + (size_t)min(wr[nt] + li, p.N - 1) * p.ldw + (size_t)kb * 64 + 8 * h4;
+  for (int nt = 0; nt < NTW; ++nt) {
+    const int r = active ? 16 * nt + li : 0, c = active ? 8 * h4 : 0;
+    wp[nt] = p.packed ? p.W + (size_t)q * ks * kstride + (size_t)kb * kstride + r * 64 + c
+                      : p.W + (size_t)min(active ? wr[nt] + li : wr[0], p.N - 1) * p.ldw + (size_t)kb * 64 + c;
+  }
 
   // A pieces: piece q = w*GA + i covers rows [8q, 8q+8); lane -> row 8q + L/8, physical chunk L%8
   // 32-bit element offsets (not 64-bit pointers): the MT = 16, 5-wave variant needs the registers
@@ -241,8 +247,8 @@ void gemm_dec_kernel(DArgs p) {
     for (int nt = 0; nt < NTW; ++nt) acc[mt][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   // issue K-step `step` into ring slot `slot`; a step past the range (the last D iterations) re-reads
-  // L2-resident bytes (A's own rows, one W line) so every iteration issues the same ops and the counted
-  // waits stay exact without a branch (a conditional load would make hipcc merge the ring registers through
+  // L2-resident bytes (A's own rows, one W line; that line for every step of a wave without a unit) so every
+  // iteration issues the same ops and the counted waits stay exact without a branch (a conditional load would make hipcc merge the ring registers through
   // copies that read an asm destination before its data lands)
   auto issue = [&](int step, int slot, bf16x8_t (&wreg)[GW]) {
     const bool live = step < nsteps;
@@ -250,7 +256,7 @@ void gemm_dec_kernel(DArgs p) {
 #pragma unroll
     for (int i = 0; i < GA; ++i) glds16((agw[i] ? p.nw : p.A) + (ao[i] + so), adst[i] + slot * ABYTES);
 #pragma unroll
-    for (int nt = 0; nt < NTW; ++nt) ldw2(wreg[2 * nt], wreg[2 * nt + 1], live ? wp[nt] + step * kstride : p.W);
+    for (int nt = 0; nt < NTW; ++nt) ldw2(wreg[2 * nt], wreg[2 * nt + 1], live ? wp[nt] + step * kstep : p.W);
   };
 
   // A fragment of rows 16 mt + li, logical chunk 4 s + h4 (swizzle depends on li only)
