@@ -116,6 +116,12 @@ struct DArgs {
   int lda, ldw, ldc;
   int M, N, K;
   int units, gs, ksplit, kt_split;  // wave units per K-range, workgroups per K-range
+  // quotients as products, as a workgroup's first loads wait for them (five divisions, two of them of 64 bits, cost 0.1 - 0.2 us a
+  // launch: a decode step of 17 such launches at 64 rows 709.4 -> 706.3 us): inv_k, inv_m = ceil(2^32 / ksplit, msplit), exact below 2^32 / divisor; unit run g starts at
+  // floor(g units / gs) = g unit_lo + floor(g (units mod gs) / gs), the last quotient by unit_frac = ceil(2^32 (units mod gs) / gs),
+  // exact below 65536 workgroups
+  unsigned inv_k, inv_m, unit_frac;
+  int unit_lo;
   int msplit;                       // row blocks of 16*MT (adjacent on one XCD: the W lines are shared in L2)
   int packed;                       // W in the unit-packed layout (grag_gemm_decode doc)
   unsigned long long* stamps;       // diagnostics (grag_gemm_decode_stamps): per workgroup {start, end, xcc} or null
@@ -178,11 +184,13 @@ void gemm_dec_kernel(DArgs p) {
   const int li = L & 15, h4 = L >> 4;
   const unsigned long long t_start = p.stamps ? __builtin_amdgcn_s_memrealtime() : 0ull;
   const int b = xcd_remap(blockIdx.x, gridDim.x);
-  const int split = b % p.ksplit;
-  const int mb = (b / p.ksplit) % p.msplit, g = b / (p.ksplit * p.msplit);
+  const int bk = p.ksplit == 1 ? b : (int)__umulhi(b, p.inv_k);
+  const int split = b - bk * p.ksplit;
+  const int g = p.msplit == 1 ? bk : (int)__umulhi(bk, p.inv_m);
+  const int mb = bk - g * p.msplit;
   const int m0 = mb * 16 * MT;
-  const int u0 = (int)((long)g * p.units / p.gs);
-  const int cnt = (int)((long)(g + 1) * p.units / p.gs) - u0;
+  const int u0 = p.unit_lo * g + (int)__umulhi(g, p.unit_frac);
+  const int cnt = p.unit_lo * (g + 1) + (int)__umulhi(g + 1, p.unit_frac) - u0;
   bool active = w < cnt;                          // wave-uniform
   int q = u0 + min(w, cnt - 1);                   // this wave's unit (an idle wave: the last one's number)
   if constexpr (TQ > 0) {
@@ -584,6 +592,17 @@ void gemm_dec_kernel(DArgs p) {
   }
 }
 
+// the derived quotients of units, gs, ksplit, msplit; false for a grid that they are not exact for
+bool set_deal(DArgs& a) {
+  const unsigned long long grid = (unsigned long long)a.gs * a.ksplit * a.msplit;
+  if ((a.units % a.gs != 0 && a.gs >= 65536) || (a.ksplit > a.msplit ? a.ksplit : a.msplit) * grid >= 1ull << 32) return false;
+  a.inv_k = (unsigned)(((1ull << 32) + a.ksplit - 1) / a.ksplit);
+  a.inv_m = (unsigned)(((1ull << 32) + a.msplit - 1) / a.msplit);
+  a.unit_lo = a.units / a.gs;
+  a.unit_frac = (unsigned)((((unsigned long long)(a.units % a.gs) << 32) + a.gs - 1) / a.gs);
+  return true;
+}
+
 template <int D, int NWV>
 int launch_nrm(const DArgs& a, int epi, int nwg, hipStream_t s) {
   if (epi == EPI_SILU)
@@ -695,6 +714,7 @@ GRAG_API int grag_gemm_decode_t(const void* A, const void* W, const void* bias, 
   a.stamps = g_dec_stamps;
   a.ksplit = ksplit;
   a.kt_split = kts;
+  if (!set_deal(a)) return (int)hipErrorInvalidValue;
   const int nwg = gs * ksplit * msplit;
   const int e = ksplit > 1 ? EPI_PARTIAL : epi;
   int err;
@@ -772,6 +792,7 @@ GRAG_API int grag_gemm_decode_norm(const void* planes, int S, const void* res_in
   a.nres_out = (bf16*)res_out;
   a.nw = (const bf16*)nw;
   a.neps = eps;
+  if (!set_deal(a)) return (int)hipErrorInvalidValue;
   return nwv == 4 ? launch_nrm<kDepth, 4>(a, epi, gs, stream) : launch_nrm<kDepth, 5>(a, epi, gs, stream);
 }
 
@@ -813,6 +834,7 @@ GRAG_API int grag_gemm_decode_red(const void* A, const void* W, void* residual, 
   a.rres = (bf16*)residual;
   a.rss = ss;
   a.rcnt = counters;
+  if (!set_deal(a)) return (int)hipErrorInvalidValue;
   if (groups) *groups = gs;
   const int nwg = gs * ksplit;
   if (nwv == 4)
@@ -861,6 +883,7 @@ GRAG_API int grag_gemm_decode_scaled(const void* A, const void* nw, const float*
   a.nss = ss;
   a.nG = G;
   a.neps = eps;
+  if (!set_deal(a)) return (int)hipErrorInvalidValue;
   const int nwg = gs * ksplit;
 #define SC(E, NW) gemm_dec_kernel<E, ACT_NONE, 1, kDepth, NW, 2, 0, 2, 0><<<nwg, 64 * NW, 0, stream>>>(a)
   if (epi == EPI_SILU) {
