@@ -51,7 +51,7 @@ GRAG_API int grag_splitk_reduce(const void* ws, const void* bias, void* C, int l
 
 namespace {
 
-enum { EPI_STORE = 0, EPI_SILU = 1, EPI_PARTIAL = 2 };
+enum { EPI_STORE = 0, EPI_SILU = 1, EPI_PARTIAL = 2, EPI_GLU = 3 };
 
 // LDS-DMA piece (1 KiB per wave instruction, lane-linear at wave-uniform lds_dst); M0 saved/set/restored in
 // one statement; completion tracked only by the caller's counted vmcnt.
@@ -89,7 +89,9 @@ __device__ __forceinline__ void ldw2(bf16x8_t& lo, bf16x8_t& hi, const bf16* p) 
 // nothing that consumes them can be scheduled above the wait.
 template <int N, int G>
 __device__ __forceinline__ void wait_w(bf16x8_t (&w)[G]) {
-  if constexpr (G == 4)
+  if constexpr (G == 2)
+    asm volatile("s_waitcnt vmcnt(%2)" : "+v"(w[0]), "+v"(w[1]) : "n"(N) : "memory");
+  else if constexpr (G == 4)
     asm volatile("s_waitcnt vmcnt(%4)" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]) : "n"(N) : "memory");
   else
     asm volatile("s_waitcnt vmcnt(%8)"
@@ -145,12 +147,15 @@ struct DArgs {
   bf16* rres;
   float* rss;
   unsigned* rcnt;
+  float limit, alpha, shift;  // EPI_GLU
 };
 
 constexpr int kNrmRows = 4;         // NRM: rows of the batch (the reference's --max-num-seqs 4)
 constexpr int kNrmLds = 64 * 1024;  // NRM: LDS image of the normalised rows, [M][K + 32] bf16
 
-// NTW 16-row n-tiles per wave (32 or 64 W rows): the A fragment read from LDS feeds NTW MFMAs, so NTW = 4
+// NTW 16-row n-tiles per wave (16, 32 or 64 W rows; 16 of a gated unit are 8 gate rows and the 8 up rows that belong to them).
+// Units of 16 rows deal a width closer to evenly where a workgroup gets 2 - 2.5 or 1 - 1.5 units of 32: its CU's reads bound a
+// workgroup, so its largest share does (dec_plan).  More rows per wave: the A fragment read from LDS feeds NTW MFMAs, so NTW = 4
 // halves the LDS read traffic per MFMA (at NTW = 2 it equals the LDS bandwidth at full MFMA rate).
 // TQ > 0 (tail split, NWV = 8): a workgroup owns 4 or 5 wave units; waves 0-3 compute one unit each over all
 // MT row tiles, and a 5th unit is shared by waves 4-7, TQ = MT / 4 row tiles each.  The CU's 4 SIMDs (two
@@ -173,7 +178,9 @@ void gemm_dec_kernel(DArgs p) {
   constexpr int NPC = MT * 2;                  // A pieces (1 KiB = 8 rows x 128 B) per K-step
   constexpr int GA = NRM == 1 ? 0 : (NPC + NWV - 1) / NWV;  // per wave (the last wave may repeat its final piece)
   constexpr int GW = 2 * NTW;                  // W dwordx4 per lane per K-step
-  static_assert(NTW == 2 || NTW == 4, "NTW");
+  static_assert(NTW == 1 || NTW == 2 || NTW == 4, "NTW");
+  constexpr bool GATED = EPI == EPI_SILU || EPI == EPI_GLU;
+  static_assert(!GATED || NTW <= 2 || EPI == EPI_SILU, "gated unit of 64 rows: interleaved weights only");
   static_assert(NST * ABYTES <= 160 * 1024, "LDS ring exceeds 160 KB");
   constexpr int LDSB = NRM == 1 ? kNrmLds : NST * ABYTES;
   __shared__ __attribute__((aligned(16))) char smem[LDSB];
@@ -211,9 +218,13 @@ void gemm_dec_kernel(DArgs p) {
   // matching up rows (+32); at NTW = 4 the wave owns one whole 64-row gate/up block (tiles 0,1 gate, 2,3 up).
   int wr[NTW];
   // gate/up units: the SiLU epilogue, or fp32 partials of a weight packed in gate/up units (packed == 2)
-  if (NTW == 2 && (EPI == EPI_SILU || p.packed == 2)) {
-    wr[0] = (q >> 1) * 64 + (q & 1) * 16;
-    wr[1] = wr[0] + 32;
+  // Units of 8 gate and 8 up rows (NTW = 1): lanes 8 - 15 of a tile's 16 hold the up rows, `up` behind the gate row of lane - 8.
+  int up = 0;
+  if (NTW <= 2 && (GATED || p.packed == 2)) {
+    const int o = 8 * NTW * q;  // first output column
+    wr[0] = EPI == EPI_GLU ? o : (o >> 5) * 64 + (o & 31);
+    up = EPI == EPI_GLU ? p.N >> 1 : 32;
+    if constexpr (NTW == 2) wr[NTW - 1] = wr[0] + up;
   } else {
 #pragma unroll
     for (int nt = 0; nt < NTW; ++nt) wr[nt] = 16 * NTW * q + 16 * nt;
@@ -227,8 +238,9 @@ void gemm_dec_kernel(DArgs p) {
 #pragma unroll
   for (int nt = 0; nt < NTW; ++nt) {
     const int r = active ? 16 * nt + li : 0, c = active ? 8 * h4 : 0;
+    const int row = wr[nt] + (NTW == 1 && GATED ? (li & 7) + (li >= 8 ? up : 0) : li);
     wp[nt] = p.packed ? p.W + (size_t)q * ks * kstride + (size_t)kb * kstride + r * 64 + c
-                      : p.W + (size_t)min(active ? wr[nt] + li : wr[0], p.N - 1) * p.ldw + (size_t)kb * 64 + c;
+                      : p.W + (size_t)min(active ? row : wr[0], p.N - 1) * p.ldw + (size_t)kb * 64 + c;
   }
 
   // A pieces: piece q = w*GA + i covers rows [8q, 8q+8); lane -> row 8q + L/8, physical chunk L%8
@@ -449,7 +461,7 @@ void gemm_dec_kernel(DArgs p) {
       if constexpr (NRM == 1) {
         if (t0 + u < nsteps) compute_nrm(t0 + u, wf[u]);
       } else {
-        if (t0 + u < nsteps) compute(u, wf[u]);  // uniform: a split's last round may be partial
+        if (active && t0 + u < nsteps) compute(u, wf[u]);  // uniform: a split's last round may be partial
       }
     }
   }
@@ -481,19 +493,40 @@ void gemm_dec_kernel(DArgs p) {
   if (active) {
     constexpr int NM = MT;
     const int mr0 = m0;
-    if constexpr (EPI == EPI_SILU) {
+    if constexpr (GATED && NTW == 1) {  // this lane has 4 gate sums (h4 < 2) or the up sums of the lane 32 before it
+      bf16* C = (bf16*)p.C;
+      const int oc = 8 * q + 4 * (h4 & 1), gr = wr[0] + 4 * (h4 & 1);
+      float bg[4], bu[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        bg[r] = EPI == EPI_SILU && p.bias ? (float)p.bias[gr + r] : 0.f;
+        bu[r] = EPI == EPI_SILU && p.bias ? (float)p.bias[gr + up + r] : 0.f;
+      }
+#pragma unroll
+      for (int mt = 0; mt < NM; ++mt) {
+        const int m = mr0 + mt * 16 + li;
+        bf16x4_t o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float u = __shfl_xor(acc[mt][0][r], 32);
+          o[r] = f2bits(EPI == EPI_GLU ? glu_f(acc[mt][0][r], u, p.limit, p.alpha, p.shift)
+                                       : silu_f(acc[mt][0][r] + bg[r]) * (u + bu[r]));
+        }
+        if (m < p.M && h4 < 2) *reinterpret_cast<bf16x4_t*>(C + (size_t)m * p.ldc + oc) = o;
+      }
+    } else if constexpr (GATED) {
       bf16* C = (bf16*)p.C;
       constexpr int NP = NTW / 2;  // gate/up tile pairs: (nt, nt + NP)
 #pragma unroll
       for (int j = 0; j < NP; ++j) {
         const int gr = wr[j] + 4 * h4, ur = wr[j + NP] + 4 * h4;
         if (ur >= p.N) continue;
-        const int oc = (gr >> 6) * 32 + (gr & 31);  // gate row 64 q + c  ->  output column 32 q + c
+        const int oc = EPI == EPI_GLU ? gr : (gr >> 6) * 32 + (gr & 31);  // gate row 64 q + c  ->  output column 32 q + c
         float bg[4], bu[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          bg[r] = p.bias ? (float)p.bias[gr + r] : 0.f;
-          bu[r] = p.bias ? (float)p.bias[ur + r] : 0.f;
+          bg[r] = EPI == EPI_SILU && p.bias ? (float)p.bias[gr + r] : 0.f;
+          bu[r] = EPI == EPI_SILU && p.bias ? (float)p.bias[ur + r] : 0.f;
         }
 #pragma unroll
         for (int mt = 0; mt < NM; ++mt) {
@@ -501,7 +534,9 @@ void gemm_dec_kernel(DArgs p) {
           if (m >= p.M || !mine(mt)) continue;
           bf16x4_t o;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) o[r] = f2bits(silu_f(acc[mt][j][r] + bg[r]) * (acc[mt][j + NP][r] + bu[r]));
+          for (int r = 0; r < 4; ++r)
+            o[r] = f2bits(EPI == EPI_GLU ? glu_f(acc[mt][j][r], acc[mt][j + NP][r], p.limit, p.alpha, p.shift)
+                                         : silu_f(acc[mt][j][r] + bg[r]) * (acc[mt][j + NP][r] + bu[r]));
           *reinterpret_cast<bf16x4_t*>(C + (size_t)m * p.ldc + oc) = o;
         }
       }
@@ -617,7 +652,10 @@ int launch_v(const DArgs& a, int epi, int act, int nwg, hipStream_t s) {
 #define GO(E, AC) gemm_dec_kernel<E, AC, MT, D, NWV, NTW, TQ><<<nwg, 64 * NWV, 0, s>>>(a)
   if (epi == EPI_PARTIAL) GO(EPI_PARTIAL, ACT_NONE);
   else if (epi == EPI_SILU) GO(EPI_SILU, ACT_NONE);
-  else if (act == ACT_GELU) GO(EPI_STORE, ACT_GELU);
+  else if (epi == EPI_GLU) {
+    if constexpr (TQ == 0) GO(EPI_GLU, ACT_NONE);
+    else return (int)hipErrorInvalidValue;
+  } else if (act == ACT_GELU) GO(EPI_STORE, ACT_GELU);
   else if (act == ACT_GELU_TANH) GO(EPI_STORE, ACT_GELU_TANH);
   else GO(EPI_STORE, ACT_NONE);
 #undef GO
@@ -629,7 +667,7 @@ int launch_v(const DArgs& a, int epi, int act, int nwg, hipStream_t s) {
 // Variants compiled (mt = 16-row tiles of M, nwv = waves per workgroup, ntw = 16-row W tiles per wave;
 // depth kDepth): (nwv 4, ntw 2): mt 1, 2, 4, 8, 16;  (nwv 5, ntw 2): mt 1, 2, 4, 8, 12 (mt 1 / 2 also at
 // depth 8 and 12: 1-32 rows hold 2-4 KB of A per K-step, so the W ring takes the registers; balanced grids; mt 16 needs
-// more than the 256 registers a wave gets at two waves per SIMD);  (nwv 8, ntw 2): mt 12.  ntw = 4 measured no faster than 2 at M = 192 (profiles/gemm_decode_ab_v3.jsonl) and is
+// more than the 256 registers a wave gets at two waves per SIMD);  (nwv 8, ntw 2): mt 12;  (nwv 5, ntw 1): mt 1, 2, 4, 8.  ntw = 4 measured no faster than 2 at M = 192 (profiles/gemm_decode_ab_v3.jsonl) and is
 // not instantiated.
 static unsigned long long* g_dec_stamps = nullptr;
 static int g_dec_depth = 0;  // 0: kDepth; 6 / 8: deeper rings where the LDS takes them (A/B, grag_gemm_decode_depth)
@@ -652,6 +690,7 @@ GRAG_API void grag_gemm_decode_stamps(void* buf) { g_dec_stamps = (unsigned long
 // tail = 1: the 8-wave tail split (gemm_dec_kernel TQ = mt / 4): at most 5 wave units per workgroup
 GRAG_API int grag_gemm_decode_has_t(int mt, int nwv, int ntw, int tail) {
   if (tail) return ntw == 2 && nwv == 8 && (mt == 4 || mt == 8 || mt == 12 || mt == 16);
+  if (ntw == 1) return nwv == 5 && (mt == 1 || mt == 2 || mt == 4 || mt == 8);
   if (ntw != 2) return 0;
   if (nwv == 4) return mt == 1 || mt == 2 || mt == 4 || mt == 8 || mt == 16;
   if (nwv == 5) return mt == 1 || mt == 2 || mt == 4 || mt == 8 || mt == 12;
@@ -661,13 +700,45 @@ GRAG_API int grag_gemm_decode_has_t(int mt, int nwv, int ntw, int tail) {
 
 GRAG_API int grag_gemm_decode_has(int mt, int nwv, int ntw) { return grag_gemm_decode_has_t(mt, nwv, ntw, 0); }
 
+// a variant of grag_gemm_decode_has_t on a filled DArgs
+static int launch_variant(const DArgs& a, int e, int act, int mt, int nwv, int ntw, int tail, int nwg, hipStream_t stream) {
+  int err;
+  if (ntw == 1) err = mt == 1 ? launch_v<1, kDepth, 5, 1>(a, e, act, nwg, stream)
+                    : mt == 2 ? launch_v<2, kDepth, 5, 1>(a, e, act, nwg, stream)
+                    : mt == 4 ? launch_v<4, kDepth, 5, 1>(a, e, act, nwg, stream)
+                              : launch_v<8, kDepth, 5, 1>(a, e, act, nwg, stream);
+  else if (tail) err = mt == 4 ? launch_v<4, kDepth, 8, 2, 1>(a, e, act, nwg, stream)
+                 : mt == 8 ? launch_v<8, kDepth, 8, 2, 2>(a, e, act, nwg, stream)
+                 : mt == 12 ? launch_v<12, kDepth, 8, 2, 3>(a, e, act, nwg, stream)
+                            : launch_v<16, kDepth, 8, 2, 4>(a, e, act, nwg, stream);
+  else if (mt <= 2) {  // 1-32 rows (the reference's 1-4 live sequences): a 2-4 KB A ring, so the W ring can be deep
+    const int d = g_dec_depth >= 12 ? 12 : g_dec_depth >= 8 ? 8 : kDepth;
+#define SK(MT_, D_) (nwv == 4 ? launch_v<MT_, D_, 4, 2>(a, e, act, nwg, stream) : launch_v<MT_, D_, 5, 2>(a, e, act, nwg, stream))
+    err = mt == 1 ? (d == 12 ? SK(1, 12) : d == 8 ? SK(1, 8) : SK(1, kDepth))
+                  : (d == 12 ? SK(2, 12) : d == 8 ? SK(2, 8) : SK(2, kDepth));
+#undef SK
+  } else if (g_dec_depth == 8 && mt == 4 && (nwv == 4 || nwv == 5))
+    err = nwv == 4 ? launch_v<4, 8, 4, 2>(a, e, act, nwg, stream) : launch_v<4, 8, 5, 2>(a, e, act, nwg, stream);
+  else if (g_dec_depth >= 6 && (mt == 4 || mt == 8) && (nwv == 4 || nwv == 5))
+    err = nwv == 4 ? (mt == 4 ? launch_v<4, 6, 4, 2>(a, e, act, nwg, stream) : launch_v<8, 6, 4, 2>(a, e, act, nwg, stream))
+                   : (mt == 4 ? launch_v<4, 6, 5, 2>(a, e, act, nwg, stream) : launch_v<8, 6, 5, 2>(a, e, act, nwg, stream));
+  else if (nwv == 4) err = mt == 4 ? launch_v<4, kDepth, 4, 2>(a, e, act, nwg, stream)
+                     : mt == 8 ? launch_v<8, kDepth, 4, 2>(a, e, act, nwg, stream)
+                               : launch_v<16, kDepth, 4, 2>(a, e, act, nwg, stream);
+  else if (nwv == 5) err = mt == 4 ? launch_v<4, kDepth, 5, 2>(a, e, act, nwg, stream)
+                          : mt == 8 ? launch_v<8, kDepth, 5, 2>(a, e, act, nwg, stream)
+                                    : launch_v<12, kDepth, 5, 2>(a, e, act, nwg, stream);
+  else err = launch_v<12, kDepth, 8, 2>(a, e, act, nwg, stream);
+  return err;
+}
+
 // y = epilogue(x @ w^T) for M <= 16 * mt rows.  epi 0 store (act 0/1/3), 1 silu*mul (w gate/up interleaved in
 // 32-row blocks, out [M, N/2]).  ksplit > 1: fp32 planes into ws (ksplit * M * N floats), then
 // grag_splitk_reduce applies the epilogue.  gs = workgroups per K-range over the N / (16 ntw) wave units
 // (0: N / (16 ntw nwv), the plain tiling; otherwise ceil(units / gs) <= nwv).  M > 16 mt: the rows go to
 // ceil(M / (16 mt)) workgroups per unit run (at most 4).  packed = 1: W in the unit-packed layout
 // [N / (16 ntw)][K / 64][16 ntw][64] (ops/gemm.py dec_pack), ldw ignored; packed = 2: the same for an
-// interleaved gate/up weight packed in gate/up units (16 gate rows then their 16 up rows; ntw 2).
+// interleaved gate/up weight packed in gate/up units (16 gate rows then their 16 up rows; ntw 2).  ntw 1: natural W only.
 // Requirements (checked):
 // K % 64 == 0, N % (16 * ntw) == 0 (silu: N % 64 == 0), lda/ldw % 8 == 0,
 // ldc % 4 == 0, 16-B aligned A/W.
@@ -680,7 +751,8 @@ GRAG_API int grag_gemm_decode_t(const void* A, const void* W, const void* bias, 
   if (K % 64 != 0 || K < 64 || N % (16 * ntw) != 0 || lda % 8 != 0 || ldw % 8 != 0 || ldc % 4 != 0)
     return (int)hipErrorInvalidValue;
   if (epi == EPI_SILU && N % 64 != 0) return (int)hipErrorInvalidValue;
-  if (packed < 0 || packed > 2 || (packed == 2 && (ntw != 2 || N % 64 != 0))) return (int)hipErrorInvalidValue;
+  if (packed < 0 || packed > 2 || (packed != 0 && ntw == 1) || (packed == 2 && (ntw != 2 || N % 64 != 0)))
+    return (int)hipErrorInvalidValue;
   const int units = N / (16 * ntw);
   if (gs <= 0) {
     if (units % nwv != 0) return (int)hipErrorInvalidValue;
@@ -717,29 +789,7 @@ GRAG_API int grag_gemm_decode_t(const void* A, const void* W, const void* bias, 
   if (!set_deal(a)) return (int)hipErrorInvalidValue;
   const int nwg = gs * ksplit * msplit;
   const int e = ksplit > 1 ? EPI_PARTIAL : epi;
-  int err;
-  if (tail) err = mt == 4 ? launch_v<4, kDepth, 8, 2, 1>(a, e, act, nwg, stream)
-                 : mt == 8 ? launch_v<8, kDepth, 8, 2, 2>(a, e, act, nwg, stream)
-                 : mt == 12 ? launch_v<12, kDepth, 8, 2, 3>(a, e, act, nwg, stream)
-                            : launch_v<16, kDepth, 8, 2, 4>(a, e, act, nwg, stream);
-  else if (mt <= 2) {  // 1-32 rows (the reference's 1-4 live sequences): a 2-4 KB A ring, so the W ring can be deep
-    const int d = g_dec_depth >= 12 ? 12 : g_dec_depth >= 8 ? 8 : kDepth;
-#define SK(MT_, D_) (nwv == 4 ? launch_v<MT_, D_, 4, 2>(a, e, act, nwg, stream) : launch_v<MT_, D_, 5, 2>(a, e, act, nwg, stream))
-    err = mt == 1 ? (d == 12 ? SK(1, 12) : d == 8 ? SK(1, 8) : SK(1, kDepth))
-                  : (d == 12 ? SK(2, 12) : d == 8 ? SK(2, 8) : SK(2, kDepth));
-#undef SK
-  } else if (g_dec_depth == 8 && mt == 4 && (nwv == 4 || nwv == 5))
-    err = nwv == 4 ? launch_v<4, 8, 4, 2>(a, e, act, nwg, stream) : launch_v<4, 8, 5, 2>(a, e, act, nwg, stream);
-  else if (g_dec_depth >= 6 && (mt == 4 || mt == 8) && (nwv == 4 || nwv == 5))
-    err = nwv == 4 ? (mt == 4 ? launch_v<4, 6, 4, 2>(a, e, act, nwg, stream) : launch_v<8, 6, 4, 2>(a, e, act, nwg, stream))
-                   : (mt == 4 ? launch_v<4, 6, 5, 2>(a, e, act, nwg, stream) : launch_v<8, 6, 5, 2>(a, e, act, nwg, stream));
-  else if (nwv == 4) err = mt == 4 ? launch_v<4, kDepth, 4, 2>(a, e, act, nwg, stream)
-                     : mt == 8 ? launch_v<8, kDepth, 4, 2>(a, e, act, nwg, stream)
-                               : launch_v<16, kDepth, 4, 2>(a, e, act, nwg, stream);
-  else if (nwv == 5) err = mt == 4 ? launch_v<4, kDepth, 5, 2>(a, e, act, nwg, stream)
-                          : mt == 8 ? launch_v<8, kDepth, 5, 2>(a, e, act, nwg, stream)
-                                    : launch_v<12, kDepth, 5, 2>(a, e, act, nwg, stream);
-  else err = launch_v<12, kDepth, 8, 2>(a, e, act, nwg, stream);
+  const int err = launch_variant(a, e, act, mt, nwv, ntw, tail, nwg, stream);
   if (err || ksplit == 1 || keep) return err;
   return grag_splitk_reduce(ws, bias, C, ldc, M, N, ksplit, epi, act, stream);
 }
@@ -749,6 +799,35 @@ GRAG_API int grag_gemm_decode(const void* A, const void* W, const void* bias, vo
                               int packed, void* ws, hipStream_t stream) {
   return grag_gemm_decode_t(A, W, bias, C, lda, ldw, ldc, M, N, K, epi, act, mt, nwv, ntw, ksplit, gs, packed, 0, ws,
                             stream);
+}
+
+// out[M, F] = glu(x wg^T, x wu^T), w [2F, K] = wg | wu (glu_f with limit, alpha, shift on the fp32 sums): one K-range, natural W,
+// no tail.  F % (8 ntw) == 0, otherwise the requirements of grag_gemm_decode_t.
+GRAG_API int grag_gemm_decode_glu(const void* A, const void* W, void* C, int lda, int ldw, int ldc, int M, int F, int K,
+                                  int mt, int nwv, int ntw, int gs, float limit, float alpha, float shift,
+                                  hipStream_t stream) {
+  if (M <= 0 || F <= 0) return 0;
+  const int msplit = (M + 16 * mt - 1) / (16 * mt);
+  if (!grag_gemm_decode_has_t(mt, nwv, ntw, 0) || msplit > 4 || K % 64 != 0 || K < 64 || F % (8 * ntw) != 0 || lda % 8 != 0 ||
+      ldw % 8 != 0 || ldc % 4 != 0)
+    return (int)hipErrorInvalidValue;
+  const int units = F / (8 * ntw);
+  if (gs <= 0 || gs > units || (units + gs - 1) / gs > nwv) return (int)hipErrorInvalidValue;
+  DArgs a{};
+  a.A = (const bf16*)A;
+  a.W = (const bf16*)W;
+  a.C = C;
+  a.lda = lda; a.ldw = ldw; a.ldc = ldc;
+  a.M = M; a.N = 2 * F; a.K = K;
+  a.units = units;
+  a.gs = gs;
+  a.msplit = msplit;
+  a.stamps = g_dec_stamps;
+  a.ksplit = 1;
+  a.kt_split = K / 64;
+  a.limit = limit; a.alpha = alpha; a.shift = shift;
+  if (!set_deal(a)) return (int)hipErrorInvalidValue;
+  return launch_variant(a, EPI_GLU, ACT_NONE, mt, nwv, ntw, 0, gs * msplit, stream);
 }
 
 // y = epilogue(RMSNorm(res_in + sum_s planes[s]) * nw @ w^T) for M <= 4 rows (NRM kernel): the split-K RMSNorm

@@ -78,6 +78,7 @@ _SIGS = {
     "grag_gemm_decode_has": [I, I, I],
     "grag_gemm_decode_t": [P, P, P, P, I, I, I, I, I, I, I, I, I, I, I, I, I, I, I, P, P],
     "grag_gemm_decode_has_t": [I, I, I, I],
+    "grag_gemm_decode_glu": [P, P, P, I, I, I, I, I, I, I, I, I, I, F, F, F, P],
     "grag_gemm_decode_stamps": [P],
     "grag_gemm_decode_depth": [I],
     "grag_gemm_w4": [P, P, P, P, P, I, I, I, I, I, I, I, I, I, I, P, P],

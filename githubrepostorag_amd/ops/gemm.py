@@ -577,7 +577,8 @@ def gemm_glu(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: float
 # ---------------------------------------------------------------- decode regime (csrc/kernels/gemm_decode.hip)
 DEC_DEPTH = 4  # K-steps issued ahead by the decode kernel (ring of DEC_DEPTH + 1 LDS / register slots)
 _DEC_ON = os.environ.get("GRAG_DECODE_GEMM", "1") != "0"
-# (mt, nwv, ntw) compiled: mt 16-row tiles of M, nwv waves per workgroup, ntw 16-row W tiles per wave
+# (mt, nwv, ntw) compiled: mt 16-row tiles of M, nwv waves per workgroup, ntw 16-row W tiles per wave (and (1 / 2 / 4 / 8, 5, 1), which
+# dec_fine() chooses)
 DEC_VARIANTS = [(1, 4, 2), (1, 5, 2), (2, 4, 2), (2, 5, 2), (4, 4, 2), (4, 5, 2), (8, 4, 2), (8, 5, 2), (12, 5, 2),
                 (12, 8, 2), (16, 4, 2)]
 DEC_MAX_M = int(os.environ.get("GRAG_DECODE_MAX_M", "256"))
@@ -595,6 +596,16 @@ def dec_small(M: int, N: int, K: int, silu: bool = False, deferred: bool = False
     if M >= 33 or M < 1:
         return False
     return M >= DEC_MIN_M or silu or K >= 4 * N or deferred
+
+
+def dec_fine(N: int, gs: int) -> bool:
+    """Whether units of 16 rows give the workgroup with the most rows fewer than units of 32 do, in five waves: a CU reads at
+    most about 28 GB/s, so that workgroup is the product's time.  560 units of 32 on 256 workgroups are 3 at most, 1120 of 16 are
+    5: 17920 x 1536 with a gated unit, 1 / 64 / 128 rows 16.1 / 19.6 / 25.7 -> 14.2 / 17.6 / 22.8 us; 18944 x 3584 31.6 / 37.6 / 50.8
+    -> 27.2 / 32.8 / 42.3 (in 4 waves of 32 36.2 / 45.3 at 64 / 128)."""
+    most = -(-(N // 32) // gs)
+    fine = -(-(N // 16) // gs)
+    return fine < 2 * most and fine <= 5
 
 
 def dec_variants(M: int) -> list[tuple[int, int, int]]:
@@ -641,7 +652,7 @@ def dec_plan(M: int, N: int, K: int, silu: bool = False) -> tuple | None:
         if silu or units >= 4 * ncu:  # FFN-wide: balanced 5-wave grid over every CU, no K-split
             mt = -(-M // 16) if M <= 32 else 4 if M <= 64 else 8
             gs = dec_balanced_gs(N, 2, 5, 1, ncu)
-            return None if gs is None else (mt, 5, 2, 1, gs)
+            return None if gs is None else (mt, 5, 1 if dec_fine(N, gs) else 2, 1, gs)
         vs = [v for v in dec_variants(M) if v[1] == 4 and N % (16 * v[1] * v[2]) == 0]
         if not vs:
             return None
@@ -653,7 +664,7 @@ def dec_plan(M: int, N: int, K: int, silu: bool = False) -> tuple | None:
         # one workgroup a tile / of these: N 18944 (148 tiles) 1 row 39.2 / 33.2, 32 36.6 / 34.8, 64 40.8 / 39.0, 128 51.8 / 48.6;
         # N 23552 (184) 38.1 / 35.8, 39.1 / 36.7, 44.6 / 42.5, 55.2 / 52.2; N 28672 (224) 41.3 / 42.8, 44.1 / 44.4, 47.6 / 47.5)
         if 2 * tiles > ncu and 5 * tiles <= 4 * ncu:
-            return mt, nwv, ntw, 1, ncu
+            return (mt, 5, 1, 1, ncu) if dec_fine(N, ncu) else (mt, nwv, ntw, 1, ncu)
         return mt, nwv, ntw, dec_ksplit(K, max(1, ncu // tiles))
     if M <= 192:
         if deep:
@@ -669,6 +680,31 @@ def dec_plan(M: int, N: int, K: int, silu: bool = False) -> tuple | None:
     if silu or deep or units % 4 or units // 4 >= ncu:
         return None
     return 16, 4, 2, dec_ksplit(K, max(1, ncu // (units // 4)))
+
+
+def dec_own_plan(M: int, N: int, K: int, silu: bool = False) -> tuple | None:
+    """dec_plan() of a product that nobody sums planes for: from 33 rows on, whole contractions of up to 2048 in units of 16 rows
+    on every CU instead of K-ranges and the launch that sums them (us: 4608 x 1536 64 / 128 rows 14.2 / 19.6 -> 11.3 / 15.0, 8192 x
+    1536 15.7 / 20.1 -> 11.8 / 15.6, 8192 x 2048 15.3 / 20.2 -> 14.6 / 18.8, 10752 x 2048 17.5 / 22.6 -> 16.2 / 20.9; 6144 x 2560 16.1 / 21.3
+    stays before 16.8 / 22.9; up to 32 rows the skinny kernel and the library are faster)."""
+    p = dec_plan(M, N, K, silu)
+    if p is None or silu or dec_ksplit(K, p[3]) == 1 or not 33 <= M <= 128 or K > 2048 or N < 16 * _num_cus():
+        return p
+    return p[0], 5, 1, 1, min(_num_cus(), N // 16)
+
+
+def dec_wide(M: int, N: int, K: int) -> bool:
+    """1-32 rows of a plain product whose one K-range gives every CU its units: up to 16 rows, or as far as units of 16 even them
+    out.  us, skinny kernel or library / here: 18944 x 3584 1 / 16 / 32 rows 33.3 / 39.2 / 31.8 -> 27.2 / 27.8 / 28.6, 17920 x 1536 16.3 /
+    19.3 / 15.9 -> 13.9 / 14.2 / 14.7, 17920 x 2048 49 / - / 22.7 -> 20.7 / - / 21.3; 32768 x 3584 48.7 / 49.7 / 43.2 -> 46.5 / 46.6 / 45.3, the
+    last of which stays."""
+    p = dec_plan(M, N, K) if M <= 32 else None
+    return p is not None and len(p) > 4 and p[3:] == (1, _num_cus()) and (M <= 16 or p[2] == 1)
+
+
+def dec_coarse(plan: tuple | None) -> tuple | None:
+    """A decode plan in units of 32 rows: what packed weights and the folded norms have."""
+    return plan if plan is None or plan[2] != 1 else (plan[0], 5, 2, *plan[3:])
 
 
 DEC_TAIL = os.environ.get("GRAG_DEC_TAIL", "0") == "1"
@@ -733,7 +769,9 @@ def gemm_decode(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None,
     N = w.shape[0]
     if not x.is_cuda:
         return gemm_silu(x, w, b) if epi == EPI_SILU else gemm(x, w, b, act)
-    mt, nwv, ntw, ks, *rest = plan or dec_plan(M, N, K, epi == EPI_SILU)
+    if plan is None:
+        plan = dec_own_plan(M, N, K, epi == EPI_SILU) if packed is None else dec_coarse(dec_plan(M, N, K, epi == EPI_SILU))
+    mt, nwv, ntw, ks, *rest = plan
     gs = rest[0] if rest else 0
     tail = rest[1] if len(rest) > 1 else 0
     ks = dec_ksplit(K, ks)
@@ -761,7 +799,7 @@ def norm_fuse_plan(M: int, N: int, K: int, silu: bool) -> tuple[int, int] | None
     image; else None."""
     if not NORM_FUSE or M < 1 or M > 4 or M * (K * 2 + 64) > 65536:
         return None
-    p = dec_plan(M, N, K, silu)
+    p = dec_coarse(dec_plan(M, N, K, silu))
     if p is None:
         return None
     mt, nwv, ntw, ks, *rest = p
@@ -839,7 +877,7 @@ def fold_plan(M: int, N: int, K: int, silu: bool) -> tuple[int, int, int] | None
     compile (one 16-row tile, 4- / 5-wave grid, no tail split); else None."""
     if not FOLD_NORM or M < 1 or M > 4:
         return None
-    p = dec_plan(M, N, K, silu)
+    p = dec_coarse(dec_plan(M, N, K, silu))
     if p is None:
         return None
     mt, nwv, ntw, ks, *rest = p
@@ -950,7 +988,7 @@ def dec_balanced_gs(N: int, ntw: int, nwv: int, ksplit: int, ncu: int | None = N
 
 
 def dec_capture_ok(dev: torch.device, M: int, N: int, K: int, silu: bool = False) -> bool:
-    p = dec_plan(M, N, K, silu)
+    p = dec_own_plan(M, N, K, silu)
     if p is None:
         return False
     fl = dec_ws_floats(M, N, dec_ksplit(K, p[3]))

@@ -284,18 +284,19 @@ def gemm_splitk(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None,
     return y.to(x.dtype)
 
 
-def kernel_for(M: int, N: int, K: int, tile_ok: bool = True, dev: torch.device | None = None, pair_ok: bool = True) -> str:
+def kernel_for(M: int, N: int, K: int, tile_ok: bool = True, dev: torch.device | None = None, pair_ok: bool = True,
+               wide_ok: bool = True) -> str:
     """The kernel linear() runs a bf16 [M, K] x [N, K]^T projection on: "pair" / "decode" / "tile" / "tile_prefill"
     (owned MFMA kernels of ops/gemm.py), "skinny" / "stream" (owned weight-streaming kernels here),
     "splitk" (K-sliced library bmm) or "library" (hipBLASLt).  ``tile_ok``: the operands meet
     ops/gemm.supported (alignment, K % 64).  ``dev``: check that a hipGraph capture in progress can use
     the split-K / stream-K workspaces (None: plan as in steady state, workspaces ready).  ``pair_ok``: they meet
-    ops/gemm.pair_takes."""
+    ops/gemm.pair_takes.  ``wide_ok``: the product is a plain one, which dec_wide() takes from the library."""
     capturing = dev is not None and torch.cuda.is_current_stream_capturing()
     if tile_ok:
         if pair_ok and _tile.pair_plan(M, N, K) is not None:
             return "pair"
-        if (TILE_MIN_M <= M or _tile.dec_small(M, N, K)) and _tile.dec_plan(M, N, K) is not None and (
+        if (TILE_MIN_M <= M or _tile.dec_small(M, N, K) or wide_ok and _tile.dec_wide(M, N, K)) and _tile.dec_plan(M, N, K) is not None and (
                 dev is None or _tile.dec_capture_ok(dev, M, N, K)):
             return "decode"
         if use_tile(M, N, K) and (dev is None or _tile.capture_ok(dev, M, N, K, pair=pair_ok)):
@@ -368,6 +369,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> t
             if _tile.pair_takes(x, w, b):
                 return _tile.gemm_pair(x, w, b, _tile.pair_plan(M, N, K))
             kind = kernel_for(M, N, K, True, x.device, pair_ok=False)
+        if kind == "decode" and M < TILE_MIN_M and not _tile.dec_small(M, N, K) and not _plain_product(x, w, b, align=2):
+            kind = kernel_for(M, N, K, True, x.device, wide_ok=False)
         if kind == "decode":
             return _tile.gemm_decode(x, w, b)
         if kind == "tile":

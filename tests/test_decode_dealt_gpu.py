@@ -4,11 +4,12 @@ several."""
 import pytest
 import torch
 
-from githubrepostorag_amd.ops.gemm import EPI_SILU, _num_cus, dec_plan, gemm_decode, interleave_gate_up
+from githubrepostorag_amd.ops.gemm import (EPI_SILU, _num_cus, dec_own_plan, dec_plan, dec_wide, gemm_decode, interleave_gate_up)
+from githubrepostorag_amd.ops import gemm as G
+from githubrepostorag_amd.ops import linear as L
 
-pytestmark = pytest.mark.gpu
 
-
+@pytest.mark.gpu
 @pytest.mark.parametrize("K", [256, 1280])
 @pytest.mark.parametrize("M", [1, 17, 64, 128])
 @pytest.mark.parametrize("wide", [False, True])
@@ -25,6 +26,7 @@ def test_dealt(dev, wide, M, K):
     assert ((gemm_decode(x, w, b).double() - want).abs() <= 2 ** -8 * want.abs() + 1e-5).all()
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 33, 128])
 @pytest.mark.parametrize("extra", [2, 48, 1024])
 def test_dealt_gated(dev, extra, M):
@@ -40,3 +42,44 @@ def test_dealt_gated(dev, extra, M):
     got = gemm_decode(x, interleave_gate_up(wg, wu), epi=EPI_SILU).double()
     # bf16's rounding of the result; fp32 sums and exponentials of numbers of about 1
     assert ((got - want).abs() <= 2 ** -8 * want.abs() + 2e-5 * (1 + b.abs())).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 128])
+@pytest.mark.parametrize("width", [1.0625, 2.25, 2.5])
+@pytest.mark.parametrize("kind", ["plain", "silu"])
+def test_fine_units(dev, kind, width, M):
+    """Units of 16 rows (8 gate and 8 up ones of a gated unit): 2 - 5 a workgroup, and the narrowest and widest such product."""
+    ncu, K = _num_cus(), 256
+    N = int(width * ncu) // 2 * 64
+    plan = (-(-M // 16) if M <= 32 else 4 if M <= 64 else 8, 5, 1, 1, ncu)
+    g = torch.Generator(device=dev).manual_seed(M + N)
+    x = torch.randn(M, K + 8, generator=g, device=dev).bfloat16()[:, 8:]
+    w = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).bfloat16()
+    z = x.double() @ w.double().T
+    if kind == "plain":
+        b = torch.randn(N, generator=g, device=dev).bfloat16()
+        got, want, fp32 = gemm_decode(x, w, b, plan=plan), z + b.double(), 1e-5
+    else:
+        b = torch.randn(N, generator=g, device=dev).bfloat16()
+        a, u = (z + b.double()).chunk(2, 1)
+        got = gemm_decode(x, interleave_gate_up(*w.chunk(2)), interleave_gate_up(*b[:, None].chunk(2))[:, 0].contiguous(), epi=EPI_SILU,
+                          plan=plan)
+        want, fp32 = a * torch.sigmoid(a) * u, 2e-5 * (1 + u.abs())
+    assert got.shape == want.shape
+    # bf16's rounding of the result; fp32 sums and exponentials of numbers of about 1
+    assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + fp32).all()
+
+
+def test_rules(monkeypatch):
+    monkeypatch.setattr(G, "_num_cus", lambda: 256)
+    assert dec_plan(64, 17920, 1536, True) == (4, 5, 1, 1, 256)     # 560 units of 32: 3 at most, 1120 of 16: 5
+    assert dec_plan(64, 37888, 3584, True) == (4, 5, 2, 1, 256)     # 1184: 5, 2368: 10
+    assert dec_plan(100, 18944, 3584) == (8, 5, 1, 1, 256)
+    assert dec_own_plan(64, 8192, 1536) == (4, 5, 1, 1, 256) and dec_plan(64, 8192, 1536) == (4, 4, 2, 3)
+    assert dec_own_plan(64, 4096 - 128, 1536)[3] > 1 and dec_own_plan(64, 8192, 2560)[3] > 1 and dec_own_plan(32, 8192, 1536)[3] > 1
+    assert dec_wide(1, 18944, 3584) and dec_wide(32, 18944, 3584) and dec_wide(16, 32768, 3584) and not dec_wide(17, 32768, 3584)
+    assert not dec_wide(1, 152064, 3584) and not dec_wide(33, 18944, 3584) and not dec_wide(1, 8192, 1536)
+    assert L.kernel_for(1, 18944, 3584) == "decode" and L.kernel_for(1, 18944, 3584, wide_ok=False) != "decode"
+    for p, N in ((dec_plan(64, 17920, 1536, True), 17920), (dec_own_plan(64, 8192, 1536), 8192), (dec_plan(1, 18944, 3584), 18944)):
+        assert -(-(N // 16) // p[4]) <= p[1]  # what the launcher takes
