@@ -785,6 +785,30 @@ def gemm_decode(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None,
     return out
 
 
+def dec_glu_plan(M: int, F: int, K: int) -> tuple | None:
+    """(mt, nwv, ntw, gs) of the decode kernel for the gated unit of a [2 F, K] weight, or None where two launches are faster: wide
+    products (two units of 32 rows a CU), and whole contractions of dec_own_plan's sizes.  us, product and unit / one launch:
+    37888 x 3584 1 / 32 / 128 rows 61.0 / 55.8 / 76.5 -> 53.8 / 52.4 / 69.6, 17920 x 1536 18.5 / 18.5 / 27.1 -> 14.2 / 15.0 / 23.2; 7552 x 3584
+    (not taken) 15.1 / 17.0 / 27.2 -> 19.5 / 19.7 / 31.6."""
+    if M > 128 or F % 32:
+        return None
+    p = dec_plan(M, 2 * F, K, True)
+    if p is None or len(p) != 5 or 2 * F < 64 * _num_cus() and not (M >= 33 and K <= 2048 and F >= 8 * _num_cus()):
+        return None
+    return p[0], p[1], p[2], p[4]
+
+
+def gemm_decode_glu(x: torch.Tensor, w: torch.Tensor, plan: tuple, limit: float | None, alpha: float, shift: float) -> torch.Tensor:
+    """gemm_glu() by the decode kernel, ``plan`` from dec_glu_plan."""
+    M, K = x.shape
+    F = w.shape[0] // 2
+    mt, nwv, ntw, gs = plan
+    out = torch.empty(M, F, dtype=x.dtype, device=x.device)
+    call("grag_gemm_decode_glu", ptr(x), ptr(w), ptr(out), x.stride(0), w.stride(0), F, M, F, K, mt, nwv, ntw, gs,
+         math.inf if limit is None else float(limit), float(alpha), float(shift))
+    return out
+
+
 # the split-K RMSNorm folded into the gate/up projection that consumes it at 1-4 rows (grag_gemm_decode_norm).
 # Off by default: measured slower (profiles/norm_fold_ab_r6.json, same box): every workgroup re-reduces the
 # o_proj planes in its prologue while only D = 4 K-steps of W are in flight, so the W stream -- the kernel's

@@ -445,7 +445,8 @@ GLU_FILL = 0.55
 
 
 def glu_linear(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: float = 1.702, shift: float = 1.0) -> torch.Tensor:
-    """clamped_glu(linear(x, w), limit, alpha, shift) for w [2F, K] (gate | up rows): at prefill sizes one launch, the unit in
+    """clamped_glu(linear(x, w), limit, alpha, shift) for w [2F, K] (gate | up rows): at decode sizes one launch of the decode kernel
+    where dec_glu_plan() has it (the unit on the fp32 sums), at prefill sizes one launch, the unit in
     the kernel's epilogue on the fp32 sums, where the 256 x 256 tiles that are useful fill at least GLU_FILL of their rounds, or
     where the small tiles take it (2048 x 1024 at 300 rows 12.0 -> 7.4 us, 12288 x 2048 34 -> 31).
 
@@ -453,6 +454,10 @@ def glu_linear(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: flo
     384 / 255; 8960 x 1536 8192 457 / 360, 1187 79 / 70; 1.03-1.5 above the line (median 1.19), 0.47-1.3 below it (a
     last round that is nearly empty, rows that are mostly padding, or few tiles).  Error against 64 bits 0.59 of the two
     launches', which round gate and up to bf16 between them."""
+    if x.is_cuda and x.dim() == 2 and 1 <= x.shape[0] <= 128 and w.shape[0] % 64 == 0:
+        plan = _tile.dec_glu_plan(x.shape[0], w.shape[0] // 2, x.shape[1])
+        if plan is not None and _tile.supported(x, w) and _plain_product(x, w):
+            return _tile.gemm_decode_glu(x, w, plan, limit, alpha, shift)
     if x.is_cuda and x.dim() == 2 and x.shape[0] >= _tile.PREFILL_MIN_M and w.shape[0] % 16 == 0:
         M, N = x.shape[0], w.shape[0]
         tiles, ncu = -(-M // 256) * -(-N // 256), _tile._num_cus()

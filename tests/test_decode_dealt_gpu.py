@@ -4,7 +4,8 @@ several."""
 import pytest
 import torch
 
-from githubrepostorag_amd.ops.gemm import (EPI_SILU, _num_cus, dec_own_plan, dec_plan, dec_wide, gemm_decode, interleave_gate_up)
+from githubrepostorag_amd.ops.gemm import (EPI_SILU, _num_cus, dec_glu_plan, dec_own_plan, dec_plan, dec_wide, gemm_decode, gemm_decode_glu,
+                                          interleave_gate_up)
 from githubrepostorag_amd.ops import gemm as G
 from githubrepostorag_amd.ops import linear as L
 
@@ -47,10 +48,10 @@ def test_dealt_gated(dev, extra, M):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 128])
 @pytest.mark.parametrize("width", [1.0625, 2.25, 2.5])
-@pytest.mark.parametrize("kind", ["plain", "silu"])
+@pytest.mark.parametrize("kind", ["plain", "silu", "glu"])
 def test_fine_units(dev, kind, width, M):
     """Units of 16 rows (8 gate and 8 up ones of a gated unit): 2 - 5 a workgroup, and the narrowest and widest such product."""
-    ncu, K = _num_cus(), 256
+    ncu, K = _num_cus(), 320 if kind == "glu" else 256
     N = int(width * ncu) // 2 * 64
     plan = (-(-M // 16) if M <= 32 else 4 if M <= 64 else 8, 5, 1, 1, ncu)
     g = torch.Generator(device=dev).manual_seed(M + N)
@@ -60,15 +61,44 @@ def test_fine_units(dev, kind, width, M):
     if kind == "plain":
         b = torch.randn(N, generator=g, device=dev).bfloat16()
         got, want, fp32 = gemm_decode(x, w, b, plan=plan), z + b.double(), 1e-5
-    else:
+    elif kind == "silu":
         b = torch.randn(N, generator=g, device=dev).bfloat16()
         a, u = (z + b.double()).chunk(2, 1)
         got = gemm_decode(x, interleave_gate_up(*w.chunk(2)), interleave_gate_up(*b[:, None].chunk(2))[:, 0].contiguous(), epi=EPI_SILU,
                           plan=plan)
         want, fp32 = a * torch.sigmoid(a) * u, 2e-5 * (1 + u.abs())
+    else:
+        a, u = z.chunk(2, 1)
+        got = gemm_decode_glu(x, w, (*plan[:3], ncu), 1.5, 1.702, 1.0)
+        a, u = a.clamp(max=1.5), u.clamp(-1.5, 1.5)
+        want, fp32 = a * torch.sigmoid(1.702 * a) * (u + 1), 1e-4
     assert got.shape == want.shape
     # bf16's rounding of the result; fp32 sums and exponentials of numbers of about 1
     assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + fp32).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,F,K,taken", [(1, 8960, 256, True), (33, 8192, 512, True), (128, 4096, 256, True), (32, 4096, 256, False),
+                                         (129, 8960, 256, False), (64, 8960, 320, False)])
+def test_glu_linear_decode(dev, M, F, K, taken, monkeypatch):
+    seen = []
+    orig = G.gemm_decode_glu
+    monkeypatch.setattr(G, "gemm_decode_glu", lambda *a: seen.append(1) or orig(*a))
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=dev).bfloat16()
+    w = (torch.randn(2 * F, K, generator=g, device=dev) * K ** -0.5).bfloat16()
+    y = L.glu_linear(x, w, 7.0).double()
+    assert bool(seen) == taken
+    a, u = (x.double() @ w.double().T).chunk(2, 1)
+    a, u = a.clamp(max=7.0), u.clamp(-7.0, 7.0)
+    s = torch.sigmoid(1.702 * a)
+    # two launches round gate and up as well: 2^-8 of each, times the unit's slopes
+    slope = (s + 1.702 * a * s * (1 - s)).abs() * (u + 1).abs() * a.abs() + (a * s).abs() * u.abs()
+    assert ((y - a * s * (u + 1)).abs() <= 2 ** -8 * ((a * s * (u + 1)).abs() + (0 if taken else 1.01) * slope) + 1e-4).all()
+    seen.clear()
+    with torch.enable_grad():  # where a gradient is asked for, the product goes the way it went
+        L.glu_linear(x.requires_grad_(), w, 7.0)
+    assert not seen
 
 
 def test_rules(monkeypatch):
@@ -80,6 +110,8 @@ def test_rules(monkeypatch):
     assert dec_own_plan(64, 4096 - 128, 1536)[3] > 1 and dec_own_plan(64, 8192, 2560)[3] > 1 and dec_own_plan(32, 8192, 1536)[3] > 1
     assert dec_wide(1, 18944, 3584) and dec_wide(32, 18944, 3584) and dec_wide(16, 32768, 3584) and not dec_wide(17, 32768, 3584)
     assert not dec_wide(1, 152064, 3584) and not dec_wide(33, 18944, 3584) and not dec_wide(1, 8192, 1536)
+    assert dec_glu_plan(1, 8960, 1536) == (1, 5, 1, 256) and dec_glu_plan(100, 18944, 3584) == (8, 5, 2, 256)
+    assert dec_glu_plan(1, 3776, 3584) is None and dec_glu_plan(129, 18944, 3584) is None
     assert L.kernel_for(1, 18944, 3584) == "decode" and L.kernel_for(1, 18944, 3584, wide_ok=False) != "decode"
     for p, N in ((dec_plan(64, 17920, 1536, True), 17920), (dec_own_plan(64, 8192, 1536), 8192), (dec_plan(1, 18944, 3584), 18944)):
         assert -(-(N // 16) // p[4]) <= p[1]  # what the launcher takes
