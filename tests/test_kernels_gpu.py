@@ -611,3 +611,13 @@ def test_sampler_reset_slots_batched_matches_per_slot(dev):
     for name in ("temperature", "top_p", "top_k", "penalty", "rng", "seen"):
         assert torch.equal(getattr(a, name), getattr(b, name)), name
     assert a._uses_topk == b._uses_topk and a._uses_topp == b._uses_topp
+
+
+def test_stream_ptr_follows_the_current_stream(dev):
+    from githubrepostorag_amd.ops._lib import stream_ptr
+
+    s = torch.cuda.Stream()
+    assert stream_ptr() == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(s):
+        assert stream_ptr() == s.cuda_stream != torch.cuda.default_stream().cuda_stream
+    assert stream_ptr() == torch.cuda.current_stream().cuda_stream
