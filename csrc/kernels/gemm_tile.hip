@@ -690,11 +690,12 @@ auto slab_store = [&](const Acc& acc, int q) {
 // pays 8 - 10 us a round beside the products: a start, the first loads' way, and a write-out that all CUs begin together.
 // Measured, a workgroup a tile -> chains: 24000 x 2304 x 768 97 -> 85 us, 24000 x 3072 x 768 with GELU 145 -> 135, 24000 x 768 x 768
 // 44 -> 40; gate / up with SwiGLU 8192 x 37888 x 3584 1528 -> 1490, 2405 x 17920 x 1536 113 -> 107; 8192 x 14336 x 3584 597 -> 571, one
-// round of 8192 x 3584 x 18944 758 -> 761.  Bands of 4 or 6 row tiles in place of 8: within 1 %.  Bitwise the same results.
+// round of 8192 x 3584 x 18944 758 -> 761.  Tiles of 192 or 128 rows (MT = 3, 2) where they fill the rounds better: chain_rows.  Bands of 4 or 6 row tiles in place of 8: within 1 %.  Bitwise the same results.
 constexpr int kChainBias = 14336;  // columns whose bias fits the LDS behind the two buffers (28 of 32 KB)
 
-template <int EPI, int ACT, bool BIAS>
+template <int EPI, int ACT, bool BIAS, int MT>
 __global__ __launch_bounds__(kThreads, 2) void gemm_chain_kernel(Args p) {
+  constexpr int QR = 16 * MT, TM = 4 * QR;  // rows of a wave's quadrant, of a tile
   constexpr bool GATED = EPI == EPI_SILU || EPI == EPI_GLU;
   __shared__ __attribute__((aligned(16))) char smem[2 * kBuf + (BIAS ? kChainBias * 2 : 0)];
   const int tid = threadIdx.x, L = tid & 63, g = L >> 4;
@@ -720,7 +721,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_chain_kernel(Args p) {
     // bands of 8 row tiles x every column tile, rows first
     constexpr int GM = 8;
     const int band = GM * p.tiles_n, first_m = t / band * GM, gsz = min(p.tiles_m - first_m, GM);
-    m0 = __builtin_amdgcn_readfirstlane((first_m + t % band % gsz) * 256);
+    m0 = __builtin_amdgcn_readfirstlane((first_m + t % band % gsz) * TM);
     n0 = __builtin_amdgcn_readfirstlane(t % band / gsz * 256);
     if (i == 0) em = m0, en = n0;
 #pragma unroll
@@ -728,19 +729,20 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_chain_kernel(Args p) {
       const int rs = tile_piece_row(r), koff = tile_piece_chunk(r) * 8;
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
-        const int gm = min(m0 + (rs >> 6) * 128 + q * 64 + (rs & 63), p.M - 1);
+        const int wrow = MT == 4 ? rs >> 6 : MT == 2 ? rs >> 5 : rs >= 96 ? 2 : rs >= 48;
+        const int gm = min(m0 + wrow * 2 * QR + q * QR + rs - wrow * QR, p.M - 1);
         int gn = min(n0 + (rs >> 5) * 64 + q * 32 + (rs & 31), p.N - 1);
         if constexpr (EPI == EPI_GLU)
           gn = q * (p.N / 2) + min(n0 / 2 + (rs >> 5) * 32 + (rs & 31), p.N / 2 - 1);
-        o[2 * q + r] = (unsigned)(gm * p.lda + koff) * 2u;
+        o[2 * q + r] = rs < 2 * QR ? (unsigned)(gm * p.lda + koff) * 2u : kTileNone;
         o[4 + 2 * q + r] = (unsigned)(gn * p.ldw + koff) * 2u;
       }
     }
     return true;
   };
   const int width = GATED ? p.N / 2 : p.N;
-  auto emit = [&](int q, const TileAcc& l, const TileAcc& r) __attribute__((always_inline)) {
-    const int rows = min(256, p.M - em);
+  auto emit = [&](int q, const TileAccN<MT>& l, const TileAccN<MT>& r) __attribute__((always_inline)) {
+    const int rows = min(TM, p.M - em);
     // rows and columns that are not there: past the end of the tile's rows
     const __amdgpu_buffer_rsrc_t rsC = __builtin_amdgcn_make_buffer_rsrc(
         (void*)((bf16*)p.C + (size_t)em * p.ldc), 0, ((rows - 1) * p.ldc + width) * 2, 0x00020000);
@@ -769,12 +771,12 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_chain_kernel(Args p) {
         d[0][h] = s[0];
         d[1][h] = s[1];
       }
-      const int row = wr * 128 + q * 64 + 16 * mt + (L & 15);
+      const int row = wr * 2 * QR + q * QR + 16 * mt + (L & 15);
       const unsigned off = row < rows && col + wcol < width ? (unsigned)(row * p.ldc + col + wcol) * 2u : kTileNone;
       __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{d[0][0], d[0][1], d[1][0], d[1][1]}, rsC, off, 0, 0);
     };
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
+    for (int mt = 0; mt < MT; ++mt) {
       float v[2][4];
       if constexpr (GATED) {
 #pragma unroll
@@ -789,7 +791,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_chain_kernel(Args p) {
       } else {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const TileAcc& acc = h ? r : l;
+          const TileAccN<MT>& acc = h ? r : l;
 #pragma unroll
           for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
@@ -802,7 +804,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_chain_kernel(Args p) {
   };
   const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc((void*)p.A, 0, p.a_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc((void*)p.W, 0, p.w_bytes, 0x00020000);
-  tile256_chain<GATED ? 4 : 8, false>(smem, rsA, rsB, p.K >> 6, next, emit, [](int) {}, [] { return 128; });
+  tile256_chain<GATED ? MT : 2 * MT, false, MT>(smem, rsA, rsB, p.K >> 6, next, emit, [](int) {}, [] { return 128; });
 }
 
 // Split-K combine: out = epilogue(sum_s ws[s]) — 8 output columns per thread.
@@ -863,12 +865,42 @@ bool chain_ok(const Args& a) {
   return a.a_bytes > 0 && a.w_bytes > 0 && (a.bias == nullptr || (a.N <= kChainBias && !((uintptr_t)a.bias & 15))) &&
          !((uintptr_t)a.C & 15) && a.ldc < (1 << 20);
 }
+// A chain's time for tiles of `rows` rows, us: begun rounds and useful ones, each by K steps and once (the chip's power makes a
+// round that is nearly empty a shorter one).  Least squares over 105 points of nine products (widths 768 - 37888, K 768 - 18944,
+// 300 - 24000 rows), 5 % off on average.
+double chain_us(int M, int N, int K, int rows, int ncu) {
+  const long tiles = ((long)M + rows - 1) / rows * (((long)N + 255) / 256);
+  const double begun = (double)((tiles + ncu - 1) / ncu), used = (double)tiles / ncu, steps = K / 64;
+  if (rows == 256) return (.72 * begun + .64 * used) * steps + 9.2 * begun - 2.3 * used + 3.8;
+  if (rows == 192) return (.66 * begun + .43 * used) * steps + 4.0 * begun + 1.8 * used + 5.2;
+  return (.58 * begun + .32 * used) * steps + 2.5 * begun + 1.3 * used + 5.6;
+}
+// Rows of a chain's tiles: 256, which read their operands least, unless 192 or 128 leave so much less of the last round empty that
+// their estimate is 2 % shorter.  At the points above that is the fastest of the three at every one (8.7 % less time than 256 rows
+// everywhere): 37888 x 3584 with SwiGLU 300 / 900 rows 151 / 241 us -> 114 (128 rows) / 204 (192); 17920 x 1536 900 / 1800 rows 68 /
+// 105 -> 63 / 99 (192; 1187 and 2400 rows stay: 74 / 73, 118 / 123); 8192 x 1536 3000 / 4300 rows 74 / 105 -> 67 / 95; 3072 x 768 with GELU
+// 12000 rows 82 -> 72.  Bitwise the same results.
+int chain_rows(int M, int N, int K, int ncu) {
+  int rows = 256;
+  for (int r : {192, 128})
+    if (chain_us(M, N, K, r, ncu) < 0.98 * chain_us(M, N, K, rows, ncu)) rows = r;
+  return rows;
+}
+
+template <int EPI, int ACT, int MT>
+int launch_chain_rows(Args a, int ncu, hipStream_t stream) {
+  a.tiles_m = (a.M + 64 * MT - 1) / (64 * MT);
+  const int nwg = min(a.tiles_m * a.tiles_n, ncu);
+  if (a.bias != nullptr) gemm_chain_kernel<EPI, ACT, true, MT><<<nwg, kThreads, 0, stream>>>(a);
+  else gemm_chain_kernel<EPI, ACT, false, MT><<<nwg, kThreads, 0, stream>>>(a);
+  return (int)hipGetLastError();
+}
 template <int EPI, int ACT>
 int launch_chain(const Args& a, int ncu, hipStream_t stream) {
-  const int nwg = min(a.tiles_m * a.tiles_n, ncu);
-  if (a.bias != nullptr) gemm_chain_kernel<EPI, ACT, true><<<nwg, kThreads, 0, stream>>>(a);
-  else gemm_chain_kernel<EPI, ACT, false><<<nwg, kThreads, 0, stream>>>(a);
-  return (int)hipGetLastError();
+  const int rows = chain_rows(a.M, a.N, a.K, ncu);
+  if (rows == 192) return launch_chain_rows<EPI, ACT, 3>(a, ncu, stream);
+  if (rows == 128) return launch_chain_rows<EPI, ACT, 2>(a, ncu, stream);
+  return launch_chain_rows<EPI, ACT, 4>(a, ncu, stream);
 }
 
 template <int EPI, int ACT>
@@ -882,6 +914,13 @@ int launch(const Args& a, hipStream_t stream) {
 }
 
 }  // namespace
+
+// The rows of whole tiles that grag_gemm_tile takes for a product (256, 192, 128) on a chip of ncu CUs, and its estimate for `rows`
+// in ns (ops/gemm.py asks both).
+GRAG_API int grag_gemm_chain_rows(int M, int N, int K, int ncu) { return chain_rows(M, N, K, ncu); }
+GRAG_API int grag_gemm_chain_ns(int M, int N, int K, int rows, int ncu) {
+  return (int)fmin(1000. * chain_us(M, N, K, rows, ncu), 2e9);
+}
 
 // MFMA shape of the tile kernel for later launches (16: v_mfma_f32_16x16x32_bf16, the default; 32:
 // v_mfma_f32_32x32x16_bf16); any other value only queries.  Returns the previous shape.

@@ -12,23 +12,27 @@ constexpr int kTileSlot = 128 * 128;        // bytes: 128 rows x 64 bf16
 constexpr int kTileBuf = 4 * kTileSlot;     // one K step: A q0, A q1, B q0, B q1
 constexpr int kTileThreads = 512;
 
-typedef f32x4_t TileAcc[4][2];   // a quadrant: [16 rows][16 columns]
-typedef bf16x8_t TileA[4][2];    // [16 rows][k step of 32]
+template <int MT> using TileAccN = f32x4_t[MT][2];  // a quadrant: [16 rows][16 columns]
+template <int MT> using TileAN = bf16x8_t[MT][2];   // [16 rows][k step of 32]
+typedef TileAccN<4> TileAcc;
+typedef TileAN<4> TileA;
 typedef bf16x8_t TileB[2][2];    // [16 columns][k step]
 
-__device__ __forceinline__ void tile_zero(TileAcc& c) {
+template <int MT>
+__device__ __forceinline__ void tile_zero(TileAccN<MT>& c) {
 #pragma unroll
-  for (int m = 0; m < 4; ++m)
+  for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int n = 0; n < 2; ++n) c[m][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 }
 // (the W fragment is operand A, so that a lane ends with 4 consecutive output columns of one row)
-__device__ __forceinline__ void tile_mma(TileAcc& acc, const TileA& a, const TileB& b) {
+template <int MT>
+__device__ __forceinline__ void tile_mma(TileAccN<MT>& acc, const TileAN<MT>& a, const TileB& b) {
   __builtin_amdgcn_s_setprio(1);
 #pragma unroll
   for (int s = 0; s < 2; ++s)
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int nt = 0; nt < 2; ++nt)
         acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[nt][s], a[mt][s], acc[mt][nt], 0, 0, 0);
@@ -101,10 +105,10 @@ __device__ __forceinline__ void tile256_loop(char* smem, const __amdgpu_buffer_r
   };
   TileA a;
   TileB b0, b1;
-  tile_zero(acc00);
-  tile_zero(acc01);
-  tile_zero(acc11);
-  tile_zero(acc10);
+  tile_zero<4>(acc00);
+  tile_zero<4>(acc01);
+  tile_zero<4>(acc11);
+  tile_zero<4>(acc10);
   const int klast = nk - 1;
   issueA(0, 0, 0);
   issueB(0, 0, 0);
@@ -128,8 +132,8 @@ __device__ __forceinline__ void tile256_loop(char* smem, const __amdgpu_buffer_r
     tile_bar();
     // M1
     if (!PARTIAL || live > 0) {
-      tile_mma(acc00, a, b0);
-      tile_mma(acc01, a, b1);
+      tile_mma<4>(acc00, a, b0);
+      tile_mma<4>(acc01, a, b1);
     }
     tile_bar();
     // L2
@@ -142,8 +146,8 @@ __device__ __forceinline__ void tile256_loop(char* smem, const __amdgpu_buffer_r
     tile_bar();
     // M2
     if (!PARTIAL || live > 64) {
-      tile_mma(acc10, a, b0);
-      tile_mma(acc11, a, b1);
+      tile_mma<4>(acc10, a, b0);
+      tile_mma<4>(acc11, a, b1);
     }
     tile_bar();
   };
@@ -166,11 +170,13 @@ __device__ __forceinline__ void tile256_loop(char* smem, const __amdgpu_buffer_r
 //   emit(q, l, r): stores row quadrant q (columns of acc(q)0, acc(q)1) of the tile in exactly ST2 vector-memory instructions
 //   ahead(i): (nk >= 5) called in the second step of tile i - 1; what its vector-memory instructions bring to LDS is there for
 //   next(i)
-//   live(): rows of this wave's 128 that the tile of the last next has; quadrants without any are not multiplied (PARTIAL only)
+// MT: 16-row tiles of a quadrant: 4, or 3 and 2 for tiles of 192 and 128 rows (a wave's quadrants of 48 and 32).  An A slot then has 96
+// and 64 rows; the pieces of the others (tile_piece_row) are kTileNone.
+//   live(): rows of this wave's 32 MT that the tile of the last next has; quadrants without any are not multiplied (PARTIAL only)
 typedef unsigned TileOff __attribute__((ext_vector_type(8)));  // A [quadrant][piece], B the same (a vector: kept in registers)
 constexpr unsigned kTileNone = 0x80000000u;      // past the end of any operand (< 2 GB): loads zeros without a trip to memory
 
-template <int ST2, bool PARTIAL, typename Next, typename Emit, typename Ahead, typename Live>
+template <int ST2, bool PARTIAL, int MT = 4, typename Next, typename Emit, typename Ahead, typename Live>
 __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_rsrc_t& rsA, const __amdgpu_buffer_rsrc_t& rsB,
                                               int nk, Next&& next, Emit&& emit, Ahead&& ahead, Live&& live) {
   const int L = threadIdx.x & 63;
@@ -179,10 +185,10 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
   const bool lag = w >= 4;
   const int cb = (L >> 4) ^ ((L >> 1) & 7);
   const int off0 = (L & 15) * 128 + cb * 16, off1 = (L & 15) * 128 + (cb ^ 4) * 16;
-  auto readA = [&](TileA& a, int q, int buf) __attribute__((always_inline)) {
-    const char* base = smem + buf * kTileBuf + q * kTileSlot + wr * 64 * 128;
+  auto readA = [&](TileAN<MT>& a, int q, int buf) __attribute__((always_inline)) {
+    const char* base = smem + buf * kTileBuf + q * kTileSlot + wr * 16 * MT * 128;
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
+    for (int mt = 0; mt < MT; ++mt) {
       a[mt][0] = *reinterpret_cast<const bf16x8_t*>(base + mt * 2048 + off0);
       a[mt][1] = *reinterpret_cast<const bf16x8_t*>(base + mt * 2048 + off1);
     }
@@ -204,9 +210,9 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
     for (int i = 0; i < 2; ++i)
       lds_dma16(rsB, smem + buf * kTileBuf + (2 + q) * kTileSlot + (2 * w + i) * 1024, o[4 + 2 * q + i], kt * 128);
   };
-  TileA a;
+  TileAN<MT> a;
   TileB b0, b1;
-  TileAcc acc00, acc01, acc11, acc10;
+  TileAccN<MT> acc00, acc01, acc11, acc10;
   TileOff cur;
   next(0, cur);
   issueA(cur, 0, 0, 0);
@@ -219,9 +225,9 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
   tile_wait_vm<6>();  // step 0 landed
   tile_bar();
   if (lag) tile_bar();
-  tile_zero(acc00);
-  tile_zero(acc01);
-  int buf = 0, rows = 128;
+  tile_zero<MT>(acc00);
+  tile_zero<MT>(acc01);
+  int buf = 0, rows = 32 * MT;
   bool more = true, behind = false;  // behind: a tile's stores lie between the loads
   auto step = [&](int i, int kt, auto first_c, auto last_c) __attribute__((always_inline)) {
     constexpr bool FIRST = decltype(first_c)::value, LAST = decltype(last_c)::value;
@@ -231,8 +237,8 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
       emit(1, acc10, acc11);
     }
     if (FIRST) {
-      tile_zero(acc10);
-      tile_zero(acc11);
+      tile_zero<MT>(acc10);
+      tile_zero<MT>(acc11);
     }
     readA(a, 0, buf);
     readB(b0, 0, buf);
@@ -247,8 +253,8 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
     tile_bar();
     // M1
     if (!PARTIAL || rows > 0) {
-      tile_mma(acc00, a, b0);
-      tile_mma(acc01, a, b1);
+      tile_mma<MT>(acc00, a, b0);
+      tile_mma<MT>(acc01, a, b1);
     }
     tile_bar();
     // L2
@@ -263,8 +269,8 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
       refill();
       tile_wait_vm<8>();
       emit(0, acc00, acc01);
-      tile_zero(acc00);
-      tile_zero(acc01);
+      tile_zero<MT>(acc00);
+      tile_zero<MT>(acc01);
       readA(a, 1, buf);
     } else {
       readA(a, 1, buf);
@@ -275,9 +281,9 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
     tile_wait_lds();
     tile_bar();
     // M2
-    if (!PARTIAL || rows > 64) {
-      tile_mma(acc10, a, b0);
-      tile_mma(acc11, a, b1);
+    if (!PARTIAL || rows > 16 * MT) {
+      tile_mma<MT>(acc10, a, b0);
+      tile_mma<MT>(acc11, a, b1);
     }
     tile_bar();
     buf ^= 1;

@@ -26,7 +26,7 @@ from pathlib import Path
 
 import torch
 
-from ._lib import call, ptr
+from ._lib import call, lib, ptr
 
 ACT_NONE, ACT_GELU, ACT_SILU, ACT_GELU_TANH = 0, 1, 2, 3
 EPI_STORE, EPI_SILU, EPI_PARTIAL, EPI_GLU = 0, 1, 2, 3
@@ -170,6 +170,25 @@ def stays_owned(M: int, N: int, K: int) -> bool:
     return row is not None and len(row) > 5
 
 
+@functools.lru_cache(4096)
+def _chain(M: int, N: int, K: int, ncu: int) -> tuple[int, float, float]:
+    rows = lib().grag_gemm_chain_rows(M, N, K, ncu)
+    us, whole = (lib().grag_gemm_chain_ns(M, N, K, r, ncu) / 1e3 for r in (rows, 256))
+    return rows, us, us / whole
+
+
+def chain_tiles(M: int, N: int, K: int) -> tuple[int, float, float]:
+    """(rows of the tiles that whole-tile products take, the estimate in us, over that of tiles of 256 rows): chain_rows of
+    csrc/kernels/gemm_tile.hip."""
+    return _chain(M, N, K, _num_cus())
+
+
+def chain_fill(M: int, N: int, K: int, rows: int | None = None) -> float:
+    """The share of the rounds of CUs that a product's whole tiles (of ``rows`` rows; those that it takes) fill."""
+    rows, ncu = rows or chain_tiles(M, N, K)[0], _num_cus()
+    return M * N / (256 * rows * ncu * -(-(-(-M // rows) * -(-N // 256)) // ncu))
+
+
 def prefill_plan(M: int, N: int, K: int, silu: bool = False) -> tuple[int, int] | None:
     """(ksplit, sk) of the owned kernel for a prefill-sized GEMM, or None for the library.
 
@@ -189,6 +208,10 @@ def prefill_plan(M: int, N: int, K: int, silu: bool = False) -> tuple[int, int] 
     ks, sk = row[3], row[4]
     if ks == 1 and sk < 0:
         sk = _tail_grid(row[0], M, N, sk)
+    if ks == 1 and sk and K <= 4096:  # swept when whole tiles had 256 rows: 16 such rows 0.99 - 1.27 of the streamed time, median
+        _, us, ratio = chain_tiles(M, N, K)  # 1.1 (37888 x 3584 300 rows 126 -> 112 us, 2048 x 1536 8320 64 -> 55); 0.82 - 0.94 of it at K
+        if ratio < 0.9 and us < 0.95 * row[2]:  # 9472 and 18944, where a part of a tile is longer beside its fixup
+            return 1, 0
     return (ks, sk) if sk_ok(M, N, K, ks, sk) else (1, 0)
 
 
@@ -326,15 +349,15 @@ def gemm_pair(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, shape: i
 
 @functools.lru_cache(4096)
 def wide_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
-    """(1, 0) where a plain product of K >= 1152 outside the measured table goes to the owned kernel in whole tiles: where they
-    fill 0.65 of their rounds of CUs.  228 points of 19 widths and depths (1536 - 28672 x 1536 - 13824) at 400 - 8192 rows, one
-    product after another of different weights: library over owned 1.08 in the geometric mean above the line (102 points,
-    0.95 - 1.61: 18944 x 3584 at 2405 rows 360 / 232 us, 4000 500 / 385), 0.98 at 0.6 - 0.65 in one round, 0.84 and less
-    below a half."""
-    tiles, ncu = -(-M // 256) * -(-N // 256), _num_cus()
+    """(1, 0) where a plain product of K >= 1152 outside the measured table goes to the owned kernel in whole tiles of 256 or 192
+    rows: where they fill 0.65 of their rounds of CUs.  Tiles of 256 rows, 228 points of 19 widths and depths (1536 - 28672 x 1536 -
+    13824) at 400 - 8192 rows, one product after another of different weights: library over owned 1.08 in the geometric mean above
+    the line (102 points, 0.95 - 1.61: 18944 x 3584 at 2405 rows 360 / 232 us, 4000 500 / 385), 0.98 at 0.6 - 0.65 in one round, 0.84
+    and less below a half.  Where those of 192 take their place, 208 points of nine widths: 1.06 (0.87 - 1.74: 18944 x 3584 900 rows
+    135 / 126, 8192 x 1536 2609 83 / 64; 14336 x 7168 621 114 / 132); 59 of tiles of 128 rows 0.98, which stay the library's."""
     if M < PREFILL_MIN_M or K < 1152 or K % 64 or max(M, N) * K >= 1 << 30 or (N, K, 0) in _prefill_table():
         return None
-    return (1, 0) if M * N >= 0.65 * 65536 * ncu * -(-tiles // ncu) else None
+    return (1, 0) if chain_tiles(M, N, K)[0] != 128 and chain_fill(M, N, K) >= 0.65 else None
 
 
 def set_mfma(mf: int) -> int:

@@ -441,18 +441,20 @@ def bound_product(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, act:
     return run
 
 
-GLU_FILL = 0.55
+GLU_FILL = {256: 0.55, 192: 0.45, 128: 0.65}  # by the tiles' rows
 
 
 def glu_linear(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: float = 1.702, shift: float = 1.0) -> torch.Tensor:
     """clamped_glu(linear(x, w), limit, alpha, shift) for w [2F, K] (gate | up rows): at decode sizes one launch of the decode kernel
     where dec_glu_plan() has it (the unit on the fp32 sums), at prefill sizes one launch, the unit in
-    the kernel's epilogue on the fp32 sums, where the 256 x 256 tiles that are useful fill at least GLU_FILL of their rounds, or
+    the kernel's epilogue on the fp32 sums, where the whole tiles fill at least GLU_FILL of their rounds, or
     where the small tiles take it (2048 x 1024 at 300 rows 12.0 -> 7.4 us, 12288 x 2048 34 -> 31).
 
     Back to back, library + unit / one launch, with 7 widths at 277-8192 rows: 18944 x 3584 8192 rows 1706 / 1581 us, 1187
     384 / 255; 8960 x 1536 8192 457 / 360, 1187 79 / 70; 1.03-1.5 above the line (median 1.19), 0.47-1.3 below it (a
-    last round that is nearly empty, rows that are mostly padding, or few tiles).  Error against 64 bits 0.59 of the two
+    last round that is nearly empty, rows that are mostly padding, or few tiles).  The same with tiles of fewer rows, 8 widths at K 512 -
+    3584: of 192 rows 1.05 - 2.6 at all 125 points (from 0.46 on), of 128 1.15 in the geometric mean at 36 points from 0.55 on, 0.86 - 0.97
+    at K = 3584 below 0.65 (8192 x 3584 622 rows 47.8 / 55.4; 37888 x 3584 316 rows 123 / 111).  Error against 64 bits 0.59 of the two
     launches', which round gate and up to bf16 between them."""
     if x.is_cuda and x.dim() == 2 and 1 <= x.shape[0] <= 128 and w.shape[0] % 64 == 0:
         plan = _tile.dec_glu_plan(x.shape[0], w.shape[0] // 2, x.shape[1])
@@ -460,8 +462,9 @@ def glu_linear(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: flo
             return _tile.gemm_decode_glu(x, w, plan, limit, alpha, shift)
     if x.is_cuda and x.dim() == 2 and x.shape[0] >= _tile.PREFILL_MIN_M and w.shape[0] % 16 == 0:
         M, N = x.shape[0], w.shape[0]
-        tiles, ncu = -(-M // 256) * -(-N // 256), _tile._num_cus()
-        fills = M * N >= GLU_FILL * 65536 * ncu * -(-tiles // ncu)
+        K = x.shape[1]
+        rows = _tile.chain_tiles(M, N, K)[0]
+        fills = _tile.chain_fill(M, N, K, 256) >= GLU_FILL[256] or K >= 256 and _tile.chain_fill(M, N, K) >= GLU_FILL[rows]
         small = x.shape[1] >= 256 and _tile.pair_plan(M, N, x.shape[1], True) is not None  # (shorter contractions: two launches)
         if (fills or small) and _tile.supported(x, w) and _plain_product(x, w):
             return _tile.gemm_glu(x, w, limit, alpha, shift)
