@@ -865,18 +865,14 @@ bool chain_ok(const Args& a) {
   return a.a_bytes > 0 && a.w_bytes > 0 && (a.bias == nullptr || (a.N <= kChainBias && !((uintptr_t)a.bias & 15))) &&
          !((uintptr_t)a.C & 15) && a.ldc < (1 << 20);
 }
-// A chain's time for tiles of `rows` rows, us: begun rounds and useful ones, each by K steps and once (the chip's power makes a
-// round that is nearly empty a shorter one).  Least squares over 105 points of nine products (widths 768 - 37888, K 768 - 18944,
-// 300 - 24000 rows), 5 % off on average.
 double chain_us(int M, int N, int K, int rows, int ncu) {
-  const long tiles = ((long)M + rows - 1) / rows * (((long)N + 255) / 256);
-  const double begun = (double)((tiles + ncu - 1) / ncu), used = (double)tiles / ncu, steps = K / 64;
-  if (rows == 256) return (.72 * begun + .64 * used) * steps + 9.2 * begun - 2.3 * used + 3.8;
-  if (rows == 192) return (.66 * begun + .43 * used) * steps + 4.0 * begun + 1.8 * used + 5.2;
-  return (.58 * begun + .32 * used) * steps + 2.5 * begun + 1.3 * used + 5.6;
+  const float tiles = (float)(((long)M + rows - 1) / rows * (((long)N + 255) / 256));
+  return rows == 256   ? tile_chain_us<4>(tiles, tiles, K / 64, ncu)
+         : rows == 192 ? tile_chain_us<3>(tiles, tiles, K / 64, ncu)
+                       : tile_chain_us<2>(tiles, tiles, K / 64, ncu);
 }
 // Rows of a chain's tiles: 256, which read their operands least, unless 192 or 128 leave so much less of the last round empty that
-// their estimate is 2 % shorter.  At the points above that is the fastest of the three at every one (8.7 % less time than 256 rows
+// their estimate (tile_chain_us) is 2 % shorter.  At its 105 points that is the fastest of the three at every one (8.7 % less time than 256 rows
 // everywhere): 37888 x 3584 with SwiGLU 300 / 900 rows 151 / 241 us -> 114 (128 rows) / 204 (192); 17920 x 1536 900 / 1800 rows 68 /
 // 105 -> 63 / 99 (192; 1187 and 2400 rows stay: 74 / 73, 118 / 123); 8192 x 1536 3000 / 4300 rows 74 / 105 -> 67 / 95; 3072 x 768 with GELU
 // 12000 rows 82 -> 72.  Bitwise the same results.

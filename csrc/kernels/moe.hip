@@ -1056,58 +1056,70 @@ __device__ __forceinline__ void moe_dma4(const __amdgpu_buffer_rsrc_t& rs, int* 
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_t*)dst, 4, off, 0, 0, 0);
 }
 
+// a wave's sum of ints, by moves between neighbouring lanes (a shuffle through LDS is ten times the way)
+__device__ __forceinline__ int wave_total(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // 1, 2, 4, 8 lanes down within 16
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // lane 15 of rows 0, 2 and lane 31 into those behind
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 // The same as chains of tiles, one workgroup a CU (tile256_chain): the next tile's source rows come to LDS while one is
 // multiplied, its first K steps behind this one's last, and the stores go out while the other waves multiply.  A workgroup a tile
 // waited for its expert's bounds, its rows, its first loads and, all CUs at once, for its stores: 4096 tokens x 4 of 16 experts,
 // width 3584, unit width 3776, routing and both products 1221 -> 1099 us (1.26 PFLOP/s in the products; the matrix cores and the
 // power they draw bound it).  K of at least 5 steps, all experts' weights and the result under 2 GB, 16-byte stores; other
 // products keep the workgroup a tile.
-template <int GATED>
-__global__ void __launch_bounds__(kTileThreads, 2)
-moe_gemm_chain_kernel(const bf16* __restrict__ a, int lda, int a_bytes, const bf16* __restrict__ w, int w_bytes,
-                      const int* __restrict__ offs, const int* __restrict__ order, int nrows, int E, int top, int N, int K,
-                      bf16* __restrict__ out, int ldo, int o_bytes, MoeEpi ep) {
-  constexpr int COLS = GATED == 1 ? 128 : 256;
-  // (one array: the compiler waits for every load in flight where a read of one array could meet a DMA into another)
-  __shared__ __attribute__((aligned(16))) char smem[2 * kTileBuf + 2 * 1024 + (RT_MAXR + 1) * 4];
+struct MoeChain {
+  const bf16* a;
+  const bf16* w;
+  const int* offs;
+  const int* order;
+  bf16* out;
+  int lda, a_bytes, w_bytes, nrows, E, top, N, K, ldo, o_bytes;
+  MoeEpi ep;
+};
+template <int GATED, int MT>
+__device__ __forceinline__ void moe_chain(char* smem, const MoeChain& p, int tiles) {
+  constexpr int COLS = GATED == 1 ? 128 : 256, QR = 16 * MT, TM = 4 * QR;  // rows of a wave's quadrant, of a tile
   int* srow = reinterpret_cast<int*>(smem + 2 * kTileBuf);  // [2][256] the entries of `order` of a tile's rows
-  int* so = srow + 512;
+  const int* so = srow + 512;
+  const MoeEpi& ep = p.ep;
+  const int lda = p.lda, top = p.top, N = p.N, K = p.K, ldo = p.ldo;
   const int tid = threadIdx.x, L = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wid >> 2, wc = wid & 3;
-  for (int e = tid; e <= E; e += kTileThreads) so[e] = offs[e];
-  __syncthreads();
   const int ncol = (N + COLS - 1) / COLS;
-  int nt = 0;
-  for (int e = 0; e < E; ++e) nt += (so[e + 1] - so[e] + 255) >> 8;
-  const int tiles = __builtin_amdgcn_readfirstlane(nt) * ncol;
   // an XCD (blockIdx % 8) has a contiguous range of the tiles, its workgroups every step-th of that
   const int x = blockIdx.x & 7, per = tiles >> 3, rest = tiles & 7, first = x * per + min(x, rest), last = first + per + (x < rest);
   const int step = (gridDim.x - x + 7) >> 3, mine = first + (blockIdx.x >> 3);
   if (mine >= last) return;
   // tile t's expert, first row, rows and first column; from tile to tile t only rises
   struct At { int e, base, r0, rows, n0; };
-  auto find = [&](int t, At p) __attribute__((always_inline)) {
+  auto find = [&](int t, At f) __attribute__((always_inline)) {
     int r, cnt;
     for (;;) {
-      r = __builtin_amdgcn_readfirstlane(so[p.e]);
-      cnt = __builtin_amdgcn_readfirstlane(so[p.e + 1]) - r;
-      const int n = ((cnt + 255) >> 8) * ncol;
-      if (t < p.base + n) break;
-      p.base += n;
-      ++p.e;
+      r = __builtin_amdgcn_readfirstlane(so[f.e]);
+      cnt = __builtin_amdgcn_readfirstlane(so[f.e + 1]) - r;
+      const int n = (cnt + TM - 1) / TM * ncol;
+      if (t < f.base + n) break;
+      f.base += n;
+      ++f.e;
     }
-    const int in = t - p.base, m = (cnt + 255) >> 8;
-    p.r0 = r + in % m * 256;
-    p.rows = min(256, cnt - in % m * 256);
-    p.n0 = in / m * COLS;
-    return p;
+    const int in = t - f.base, m = (cnt + TM - 1) / TM;
+    f.r0 = r + in % m * TM;
+    f.rows = min(TM, cnt - in % m * TM);
+    f.n0 = in / m * COLS;
+    return f;
   };
-  const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc((void*)a, 0, a_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, w_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsC = __builtin_amdgcn_make_buffer_rsrc((void*)out, 0, o_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsO = __builtin_amdgcn_make_buffer_rsrc((void*)order, 0, nrows * 4, 0x00020000);
-  auto rows_to_lds = [&](int i, const At& p) __attribute__((always_inline)) {  // by waves 0 - 3, 64 rows each
-    if (wid < 4) moe_dma4(rsO, srow + (i & 1) * 256 + 64 * wid, (unsigned)(p.r0 + min(64 * wid + L, p.rows - 1)) * 4u);
+  const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, p.a_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc((void*)p.w, 0, p.w_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsC = __builtin_amdgcn_make_buffer_rsrc((void*)p.out, 0, p.o_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsO = __builtin_amdgcn_make_buffer_rsrc((void*)p.order, 0, p.nrows * 4, 0x00020000);
+  auto rows_to_lds = [&](int i, const At& f) __attribute__((always_inline)) {  // by waves 0 - 3, 64 rows each
+    if (wid < 4) moe_dma4(rsO, srow + (i & 1) * 256 + 64 * wid, (unsigned)(f.r0 + min(64 * wid + L, f.rows - 1)) * 4u);
   };
   At at = find(mine, At{0, 0, 0, 0, 0}), em = at, nx = at;  // of the loads issued last, of the results, of the rows brought last
   rows_to_lds(0, at);
@@ -1130,18 +1142,19 @@ moe_gemm_chain_kernel(const bf16* __restrict__ a, int lda, int a_bytes, const bf
       const int rs = tile_piece_row(r), c = tile_piece_chunk(r) * 8;
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
-        const int lr = (rs >> 6) * 128 + q * 64 + (rs & 63);
+        const int half = MT == 4 ? rs >> 6 : MT == 2 ? rs >> 5 : rs >= 96 ? 2 : rs >= 48;
+        const int lr = min(half * 2 * QR + q * QR + rs - half * QR, TM - 1);
         const int src = GATED == 0 ? at.r0 + min(lr, at.rows - 1) : srow[(i & 1) * 256 + lr] / top;
         const int gn = GATED == 1 ? q * N + min(at.n0 + (rs >> 5) * 32 + (rs & 31), N - 1)
                                   : min(at.n0 + (rs >> 5) * 64 + q * 32 + (rs & 31), N - 1);
-        o[2 * q + r] = ((unsigned)src * (unsigned)lda + c) * 2u;
+        o[2 * q + r] = rs < 2 * QR ? ((unsigned)src * (unsigned)lda + c) * 2u : kTileNone;
         o[4 + 2 * q + r] = ((wbase + gn) * (unsigned)K + c) * 2u;
       }
     }
     return true;
   };
   int ei = 0;  // the tile that is stored
-  auto emit = [&](int qm, const TileAcc& l, const TileAcc& r) __attribute__((always_inline)) {
+  auto emit = [&](int qm, const TileAccN<MT>& l, const TileAccN<MT>& r) __attribute__((always_inline)) {
     const int wcol = ((L >> 4) & 1) * 16 + (L >> 5) * 8;
     auto put = [&](int rs, int nb, auto&& val) __attribute__((always_inline)) {
       uint32_t d[2][2];
@@ -1156,14 +1169,14 @@ moe_gemm_chain_kernel(const bf16* __restrict__ a, int lda, int a_bytes, const bf
         d[0][h] = s[0];
         d[1][h] = s[1];
       }
-      const int lr = 128 * wr + 64 * qm + 16 * rs + (L & 15);
+      const int lr = 2 * QR * wr + QR * qm + 16 * rs + (L & 15);
       const unsigned row = (unsigned)(GATED == 0 ? srow[(ei & 1) * 256 + lr] : em.r0 + lr);
       const unsigned off = lr < em.rows && nb + wcol < N ? (row * (unsigned)ldo + nb + wcol) * 2u : kTileNone;
       typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
       __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{d[0][0], d[0][1], d[1][0], d[1][1]}, rsC, off, 0, 0);
     };
 #pragma unroll
-    for (int rs = 0; rs < 4; ++rs) {
+    for (int rs = 0; rs < MT; ++rs) {
       if constexpr (GATED == 1) {
         put(rs, em.n0 + wc * 32, [&](int s, int i, int c) { return glu_unit(l[s][i][c], r[s][i][c], ep); });
       } else {
@@ -1177,9 +1190,40 @@ moe_gemm_chain_kernel(const bf16* __restrict__ a, int lda, int a_bytes, const bf
     }
     if (qm == 1) em = at, ++ei;
   };
-  tile256_chain<GATED == 1 ? 4 : 8, true>(smem, rsA, rsB, K >> 6, next, emit, ahead,
-                                          [&] { return __builtin_amdgcn_readfirstlane(at.rows - 128 * wr); });
+  tile256_chain<GATED == 1 ? MT : 2 * MT, true, MT>(smem, rsA, rsB, K >> 6, next, emit, ahead,
+                                                    [&] { return __builtin_amdgcn_readfirstlane(at.rows - 2 * QR * wr); });
 }
+
+// Tiles of 256, 192 or 128 rows, as the experts' row counts (known here alone) make the shortest rounds by the dense kernel's estimate,
+// with the rows in place of the tiles as its useful share, since an expert's last rows cost about theirs.  124 products of both bench
+// sizes, 430 - 4096 tokens x 4 of 16 experts: 0.1 % behind the best of the three on average, 7 % before tiles of 256 everywhere
+// (width 3584, unit width 3776, 1100 / 2000 tokens: first product 310 / 409 us -> 271 / 411, second 175 / 253 -> 146 / 218).
+template <int GATED>
+__global__ void __launch_bounds__(kTileThreads, 2) moe_gemm_chain_kernel(const MoeChain p) {
+  // (one array: the compiler waits for every load in flight where a read of one array could meet a DMA into another)
+  __shared__ __attribute__((aligned(16))) char smem[2 * kTileBuf + 2 * 1024 + (RT_MAXR + 1) * 4];
+  int* so = reinterpret_cast<int*>(smem + 2 * kTileBuf) + 512;
+  for (int e = threadIdx.x; e <= p.E; e += kTileThreads) so[e] = p.offs[e];
+  __syncthreads();
+  int n4 = 0, n3 = 0, n2 = 0;
+  for (int e = threadIdx.x & 63; e < p.E; e += 64) {
+    const int cnt = so[e + 1] - so[e];
+    n4 += (cnt + 255) / 256, n3 += (cnt + 191) / 192, n2 += (cnt + 127) / 128;
+  }
+  n4 = wave_total(n4), n3 = wave_total(n3), n2 = wave_total(n2);
+  const int ncol = (p.N + (GATED == 1 ? 127 : 255)) / (GATED == 1 ? 128 : 256), steps = p.K >> 6, cus = gridDim.x;
+  n4 *= ncol, n3 *= ncol, n2 *= ncol;
+  const float full = (float)so[p.E] * ncol;  // (of one row)
+  const float t4 = tile_chain_us<4>(n4, full / 256, steps, cus), t3 = tile_chain_us<3>(n3, full / 192, steps, cus),
+              t2 = tile_chain_us<2>(n2, full / 128, steps, cus);
+  int rows = t3 < 0.96f * t4 ? 192 : 256;
+  if (t2 < 0.96f * (rows == 192 ? t3 : t4)) rows = 128;
+  rows = __builtin_amdgcn_readfirstlane(rows);
+  if (rows == 256) moe_chain<GATED, 4>(smem, p, n4);
+  else if (rows == 192) moe_chain<GATED, 3>(smem, p, n3);
+  else moe_chain<GATED, 2>(smem, p, n2);
+}
+
 
 // ------------------------------------------------------------------------------------------------ residual boundary
 // x [T][H] fp32, in place: x <- keep x + mult * sigmoid(gate + gbias) * (a + bcoef_t b + sum_k ecoef_(t,k) e_(t,k)), every
@@ -1634,10 +1678,11 @@ GRAG_API hipError_t grag_moe_gemm(const void* a, int lda, const void* w, const i
     const long o_bytes = (long)rows * ldo * 2;
     if (K >= 320 && w_bytes * E < (1L << 31) && o_bytes < (1L << 31) && N % 8 == 0 && ldo % 8 == 0 && al16(out) && rows < (1 << 28)) {
       const int cus = device_cus();
-#define MOE_CHAIN(G)                                                                                                     \
-  hipLaunchKernelGGL(moe_gemm_chain_kernel<G>, dim3((unsigned)(blocks < cus ? blocks : cus)), dim3(kTileThreads), 0, st, \
-                     (const bf16*)a, lda, (int)a_bytes, (const bf16*)w, (int)(w_bytes * E), offs, order, rows, E, top, N, K,     \
-                     (bf16*)out, ldo, (int)o_bytes, ep)
+      const long most = ((long)rows / 128 + E) * tcols;
+      const MoeChain p{(const bf16*)a, (const bf16*)w, offs, order, (bf16*)out, lda, (int)a_bytes, (int)(w_bytes * E), rows, E, top, N,
+                       K, ldo, (int)o_bytes, ep};
+#define MOE_CHAIN(G) \
+  hipLaunchKernelGGL(moe_gemm_chain_kernel<G>, dim3((unsigned)(most < cus ? most : cus)), dim3(kTileThreads), 0, st, p)
       if (gated == 1) MOE_CHAIN(1);
       else if (gated == 3) MOE_CHAIN(3);
       else MOE_CHAIN(0);
