@@ -1,5 +1,4 @@
-// Fused cosine-score + metadata-filter + top-k for the GPU vector index
-// (SURVEY §2.7 N3a/N3b/N3c/N3e).
+// Fused cosine-score + metadata-filter + top-k for the GPU vector index.
 //
 // Vectors are stored L2-normalised in bf16, so cosine == dot product.
 // S^T[row][q] = X · Q^T on v_mfma_f32_16x16x32_bf16: A = 16 database rows read
@@ -16,10 +15,7 @@
 // partner list, then a half-cleaner network), so each wave emits one list per
 // query.  In a flat scan the workgroup's waves merge theirs through LDS (three
 // rounds), and topk_lists_merge_kernel picks the best of the workgroups' lists.
-// (The lists of
-// all waves through a library sort took 15 launches and 100 us behind a scan of
-// 330 us: 1M x 768, 16 queries, k = 10, 428 -> 323, 20K rows
-// 103 -> 38.)
+// (The lists of all waves through a library sort took 15 launches and 100 us.)
 // Work items leave a list per wave for grag_topk_merge.
 //
 // Filters (N3c): up to 4 predicates over dictionary-encoded int32 columns
@@ -126,6 +122,7 @@ __device__ __forceinline__ void list_merge_xor(float (&v)[K], uint32_t (&id)[K],
 // What the filters ask of rows row .. row + 3 (rows from r1 on: the last one's): a bit per row of the bitmap, a column's value per
 // filter and row
 typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 struct RowKeys {
   uint32_t alive;
   i32x4_t col[4];
@@ -188,6 +185,20 @@ __global__ __launch_bounds__(64 * NWAVES) void score_topk_kernel(TopkParams p) {
     slot_base = ((int64_t)blockIdx.y * p.nchunks + blockIdx.x) * NQ;
   }
 
+  // A tile's 32-dim steps in batches of U, two batches of registers: one in flight while the other is multiplied, the next tile's
+  // first one too, so that 8 waves a CU keep the stream up.  The filters' columns of a tile's rows are loaded ahead of its batches.
+  constexpr int U = NQT == 1 ? 6 : NQT == 2 ? 4 : 3, STEP = 16 * NWAVES;
+  const int nc = d / 32;
+  bf16x8_t a0[U], a1[U];
+  auto load = [&](bf16x8_t (&a)[U], int64_t t0, int c) __attribute__((always_inline)) {
+    const bf16* xp = p.X + min(t0 + li, r1 - 1) * d + 8 * h4 + 32 * c;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (c + u < nc) a[u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(xp + 32 * u));
+  };
+  const int64_t first = r0 + wave * 16;
+  if (first < r1) load(a0, first, 0);  // (ahead of the queries: a small table's first rows take as long to come)
+
   // stage the query tile: row qq, chunk ch -> qq*RB + ((ch ^ (qq & SWZ)) << 4)
   for (int c = threadIdx.x; c < NQ * CPR; c += 64 * NWAVES) {
     const int qq = c / CPR, ch = c % CPR;
@@ -226,19 +237,6 @@ __global__ __launch_bounds__(64 * NWAVES) void score_topk_kernel(TopkParams p) {
     }
   });
 
-  // A tile's 32-dim steps in batches of U, two batches of registers: one in flight while the other is multiplied, the next tile's
-  // first one too, so that 8 waves a CU keep the stream up.  The filters' columns of a tile's rows are loaded ahead of its batches.
-  constexpr int U = NQT == 1 ? 6 : NQT == 2 ? 4 : 3, STEP = 16 * NWAVES;
-  const int nc = d / 32;
-  bf16x8_t a0[U], a1[U];
-  auto load = [&](bf16x8_t (&a)[U], int64_t t0, int c) __attribute__((always_inline)) {
-    const bf16* xp = p.X + min(t0 + li, r1 - 1) * d + 8 * h4 + 32 * c;
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (c + u < nc) a[u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(xp + 32 * u));
-  };
-  const int64_t first = r0 + wave * 16;
-  if (first < r1) load(a0, first, 0);
 #pragma unroll 1
   for (int64_t t0 = first; t0 < r1; t0 += STEP) {
     const RowKeys keys = row_keys(p, t0 + 4 * h4, r1);
@@ -336,112 +334,104 @@ __global__ __launch_bounds__(64 * NWAVES) void score_topk_kernel(TopkParams p) {
 
 // (value, number) in falling order of value, ties by rising number
 __device__ __forceinline__ bool ahead(float v, uint32_t i, float w, uint32_t j) { return v > w || (v == w && i < j); }
-// the largest of a wave's numbers, by moves between neighbouring lanes (lane 63 ends with it)
-template <int CTRL, int ROWS> __device__ __forceinline__ float max_step(float v) {
-  const float low = -INFINITY;
-  return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(low), __float_as_int(v), CTRL, ROWS, 0xf, false)));
-}
-__device__ __forceinline__ float wave_top(float v) {
-  v = max_step<0x111, 0xf>(v);  // 1, 2, 4, 8 lanes down within 16, then lane 15 of rows 0, 2 and lane 31 into those behind
-  v = max_step<0x112, 0xf>(v);
-  v = max_step<0x114, 0xf>(v);
-  v = max_step<0x118, 0xf>(v);
-  v = max_step<0x142, 0xa>(v);
-  v = max_step<0x143, 0xc>(v);
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
-
 constexpr int kMergeLists = 1024;  // lists of a query at most
 
+// A number as one of the same order among the whole numbers, 0 for what no list holds (-inf; NaN); -0 is 0
+__device__ __forceinline__ uint32_t order_key(float v) {
+  if (!(v > -INFINITY)) return 0;
+  const uint32_t b = __float_as_uint(v + 0.f);
+  return b ^ ((b >> 31) ? 0xFFFFFFFFu : 0x80000000u);
+}
+
 // The final lists of a flat scan: query q's sorted lists of k are rows (q / G * n + j) * G + q % G, j < n <= kMergeLists, of ps /
-// pi.  grid (nq), 256 threads.  Only the k lists with the best heads can hold one of the best k, and of those only what is not
-// behind the last of these heads: every wave takes the best k of its quarter of the heads one by one, wave 0 the best k of these;
-// their elements, loaded at once with their ids, are ranked by counting.  Three ways to memory, where folding list into list took
-// one for each of a thread's lists and then 64 merges of sorted lists in registers: 1M rows, 16 queries, k = 10 26 us -> 12,
-// 64 queries, k = 30 48 -> 28 (with 256 lists in place of 1024).
-__global__ __launch_bounds__(256) void topk_lists_merge_kernel(const float* __restrict__ ps, const int64_t* __restrict__ pi,
-                                                               int n, int G, int k, float* __restrict__ out_s,
-                                                               int64_t* __restrict__ out_i) {
-  __shared__ float hv[4 * 32], cv[32 * 32];
-  __shared__ uint32_t hj[4 * 32], best[32], cnum[32 * 32];
+// pi.  grid (nq), a multiple of 64 threads, no fewer than n.  Only the k lists with the best heads can hold one of the best k, and of
+// those only what is not behind the last of these heads: each wave ranks its 64 heads by counting, the best k of each are ranked
+// once more, and the elements of the k lists, loaded at once with their ids, as well.  Bound by three ways to memory (lists folded
+// one into the next took one for each of a thread's lists and 64 merges in registers).  The whole search with
+// 20K rows, 16 queries: k = 10 32.3 us -> 27.5 and k = 30 61 -> 41, against taking the best head k times, a wave's maximum each.
+__global__ __launch_bounds__(1024) void topk_lists_merge_kernel(const float* __restrict__ ps, const int64_t* __restrict__ pi, int n,
+                                                                int G, int k, float* __restrict__ out_s, int64_t* __restrict__ out_i) {
+  __shared__ __attribute__((aligned(16))) uint32_t heads[kMergeLists];
+  __shared__ float cv[32 * 32];
+  __shared__ uint32_t hk[kMergeLists / 64 * 32], hj[kMergeLists / 64 * 32], best[32], cnum[32 * 32];
   __shared__ int64_t cid[32 * 32];
-  __shared__ float last_v;
-  __shared__ uint32_t last_j;
-  __shared__ int count;
-  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ uint32_t last_key, last_list;
+  __shared__ int count, wave_got[kMergeLists / 64];
+  const int q = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, threads = blockDim.x;
   const int64_t base = (int64_t)(q / G) * n * G + q % G;
-  const uint32_t none = 0xFFFFFFFFu;
-  if (tid == 0) count = 0;
-  int lists;
-  bool full;  // there are k lists with something, and more
+  if (tid == 0) count = 0, last_key = last_list = 0;  // (key 0: nothing is behind it)
+  int picked = n;
   if (n <= k) {  // every list may hold some: nothing is picked (1000 rows, k = 30, the whole search 72 -> 54 us)
     if (tid < n) best[tid] = tid;
-    lists = n, full = false;
   } else {
-    float h[kMergeLists / 256];
-#pragma unroll
-    for (int u = 0; u < kMergeLists / 256; ++u) {
-      const int j = u * 256 + tid;
-      h[u] = j < n ? ps[(base + (int64_t)j * G) * k] : -INFINITY;
-    }
-    for (int r = 0; r < k; ++r) {
-      float v = -INFINITY;
-      uint32_t j = none;
-#pragma unroll
-      for (int u = 0; u < kMergeLists / 256; ++u)
-        if (h[u] > v) v = h[u], j = u * 256 + tid;
-      const float top = wave_top(v);
-      uint32_t first = none;  // of the lanes that have it the lowest list
-      for (unsigned long long at = __ballot(v == top && j != none); at; at &= at - 1)
-        first = min(first, (uint32_t)__builtin_amdgcn_readlane((int)j, __ffsll(at) - 1));
-#pragma unroll
-      for (int u = 0; u < kMergeLists / 256; ++u)
-        if (first == (uint32_t)(u * 256 + tid)) h[u] = -INFINITY;
-      if (lane == 0) hv[wave * 32 + r] = top, hj[wave * 32 + r] = first;
-    }
-    __syncthreads();
-    // of 4 k heads the best k: as many as are ahead of one
-    if (tid < 128) {
-      const int r = tid & 31;
-      const bool on = r < k && hj[tid] != none;
+    const int waves = (n + 63) / 64;
+    if (wave < waves) {
+      const uint32_t key = tid < n ? order_key(ps[(base + (int64_t)tid * G) * k]) : 0;
+      heads[tid] = key;
+      __builtin_amdgcn_wave_barrier();  // (a wave's own 64: LDS takes its accesses in order)
       int rank = 0;
-      if (on)
-        for (int w = 0; w < 4; ++w)
-          for (int i = 0; i < k; ++i) rank += ahead(hv[w * 32 + i], hj[w * 32 + i], hv[tid], hj[tid]) && hj[w * 32 + i] != none;
-      if (on && rank < k) best[rank] = hj[tid];
-      if (on && rank == k - 1) last_v = hv[tid], last_j = hj[tid];
-      const int got = __popcll(__ballot(on));
-      if (lane == 0) atomicAdd(&count, got);
+      const u32x4_t* of = reinterpret_cast<const u32x4_t*>(heads + wave * 64);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const u32x4_t w = of[i];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) rank += w[u] > key;
+      }
+      unsigned long long in = __ballot(key != 0 && rank < k);
+      if (__popcll(in) > k) {  // equal heads at the end of the k: the lower lists
+        for (int i = 0; i < 64; ++i) rank += heads[wave * 64 + i] == key && i < lane;
+        in = __ballot(key != 0 && rank < k);
+      }
+      const int got = __popcll(in), place = __popcll(in & ((1ull << lane) - 1));
+      if (in >> lane & 1) hk[wave * k + place] = key, hj[wave * k + place] = tid;
+      if (lane >= got && lane < k) hk[wave * k + lane] = 0, hj[wave * k + lane] = 0;
+      if (lane == 0) wave_got[wave] = got;
     }
     __syncthreads();
-    lists = min(count, k), full = count >= k;  // (heads that are there: no list without one has anything)
+    int all = 0;
+    for (int w = 0; w < waves; ++w) all += wave_got[w];
+    picked = min(all, k);
+    for (int x = tid >> 2; x < waves * k; x += threads / 4) {
+      const uint32_t key = hk[x], j = hj[x];
+      int rank = 0;
+      for (int i = tid & 3; i < waves * k; i += 4) rank += hk[i] > key || (hk[i] == key && hj[i] < j);
+      rank += __shfl_xor(rank, 1, 64);
+      rank += __shfl_xor(rank, 2, 64);
+      if ((tid & 3) == 0 && key != 0 && rank < k) {
+        best[rank] = j;
+        if (rank == k - 1) last_key = key, last_list = j;
+      }
+    }
   }
   __syncthreads();
-  if (tid == 0) count = 0;
-  __syncthreads();
-  for (int e = tid; e < lists * k; e += 256) {
+  for (int e = tid; e < picked * k; e += threads) {
     const uint32_t j = best[e / k];
     const int t = e % k;
     const int64_t at = (base + (int64_t)j * G) * k + t;
     const float v = ps[at];
     const int64_t id = pi[at];
+    const uint32_t key = order_key(v);
     // (of lists with equal values the heads decide: behind the last head's list nothing that equals it is among the best)
-    if (v != -INFINITY && (!full || v > last_v || (v == last_v && j <= last_j))) {
+    if (key != 0 && (key > last_key || (key == last_key && j <= last_list))) {
       const int c = atomicAdd(&count, 1);
       cv[c] = v, cnum[c] = j * (uint32_t)k + t, cid[c] = id;
     }
   }
   __syncthreads();
   const int c = count;
-  for (int e = tid; e < c; e += 256) {
+  for (int x = tid >> 2; x < c; x += threads / 4) {
+    const float v = cv[x];
+    const uint32_t m = cnum[x];
     int rank = 0;
-    for (int i = 0; i < c; ++i) rank += ahead(cv[i], cnum[i], cv[e], cnum[e]);
-    if (rank < k) {
-      out_s[(int64_t)q * k + rank] = cv[e];
-      out_i[(int64_t)q * k + rank] = cid[e];
+    for (int i = tid & 3; i < c; i += 4) rank += ahead(cv[i], cnum[i], v, m);
+    rank += __shfl_xor(rank, 1, 64);
+    rank += __shfl_xor(rank, 2, 64);
+    if ((tid & 3) == 0 && rank < k) {
+      out_s[(int64_t)q * k + rank] = v;
+      out_i[(int64_t)q * k + rank] = cid[x];
     }
   }
-  for (int r = c + tid; r < k; r += 256) {
+  for (int r = c + tid; r < k; r += threads) {
     out_s[(int64_t)q * k + r] = -INFINITY;
     out_i[(int64_t)q * k + r] = -1;
   }
@@ -499,7 +489,7 @@ GRAG_API int grag_topk_lists_merge(const float* ps, const int64_t* pi, int n, in
                                    int64_t* out_i, hipStream_t stream) {
   if (nq <= 0) return 0;
   if (n < 1 || n > kMergeLists || G < 1 || k < 1 || k > 32) return (int)hipErrorInvalidValue;
-  topk_lists_merge_kernel<<<nq, 256, 0, stream>>>(ps, pi, n, G, k, out_s, out_i);
+  topk_lists_merge_kernel<<<nq, std::max(k > 16 ? 1024 : 256, (n + 63) / 64 * 64), 0, stream>>>(ps, pi, n, G, k, out_s, out_i);
   return (int)hipGetLastError();
 }
 

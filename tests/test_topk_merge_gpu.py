@@ -1,0 +1,36 @@
+"""The merge of a flat scan's lists (csrc/kernels/topk.hip, topk_lists_merge_kernel) against a sort on the CPU: list counts around a
+wave, around k and at the most it takes, equal values, empty and unfilled lists, infinities."""
+import pytest
+import torch
+
+from githubrepostorag_amd.ops._lib import call, ptr
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("values", ["distinct", "equal", "sparse"])
+@pytest.mark.parametrize("k", [1, 5, 16, 17, 32])
+@pytest.mark.parametrize("n", [1, 31, 33, 64, 65, 255, 257, 1024])
+def test_lists_merge(n, k, values):
+    nq, G = 19, 16
+    g = torch.Generator().manual_seed(n * 100 + k)
+    tiles = -(-nq // G)
+    s = torch.randn(tiles, n, G, k, generator=g)
+    if values == "equal":  # a handful of values, both zeros and both ends among them
+        s = torch.tensor([-1.5, -0.0, 0.0, 0.25, 3.0, float("inf")])[torch.randint(0, 6, s.shape, generator=g)]
+    if values == "sparse":  # a few rows in all, in lists that are full, partly full or empty
+        keep = torch.randint(0, k + 1, (tiles, n, G, 1), generator=g)
+        keep[torch.rand(tiles, n, G, 1, generator=g) > 20 / n] = 0
+        s = torch.where(torch.arange(k) < keep, s, float("-inf"))
+    s = s.sort(-1, descending=True).values
+    ids = torch.randperm(s.numel(), generator=g).view(s.shape)
+    ids = torch.where(s == float("-inf"), -1, ids)
+    out_s = torch.full((nq, k), 7.0).cuda()
+    out_i = torch.full((nq, k), -7).cuda()
+    ds, di = s.cuda(), ids.cuda()
+    call("grag_topk_lists_merge", ptr(ds), ptr(di), n, G, nq, k, ptr(out_s), ptr(out_i))
+    # a query's elements in order of list, then place: a stable sort keeps the lower list of equal values
+    flat = s.transpose(1, 2).reshape(tiles * G, n * k)[:nq]
+    ws, at = flat.sort(dim=-1, descending=True, stable=True)
+    wi = ids.transpose(1, 2).reshape(tiles * G, n * k)[:nq].gather(1, at)
+    assert torch.equal(out_s.cpu(), ws[:, :k]) and torch.equal(out_i.cpu(), wi[:, :k])
