@@ -1,9 +1,10 @@
 """The merge of a flat scan's lists (csrc/kernels/topk.hip, topk_lists_merge_kernel) against a sort on the CPU: list counts around a
-wave, around k and at the most it takes, equal values, empty and unfilled lists, infinities."""
+wave, around k and at the most it takes, equal values, empty and unfilled lists, infinities; and the scan's order of equal scores."""
 import pytest
 import torch
 
 from githubrepostorag_amd.ops._lib import call, ptr
+from githubrepostorag_amd.ops.topk import score_topk
 
 pytestmark = pytest.mark.gpu
 
@@ -34,3 +35,29 @@ def test_lists_merge(n, k, values):
     ws, at = flat.sort(dim=-1, descending=True, stable=True)
     wi = ids.transpose(1, 2).reshape(tiles * G, n * k)[:nq].gather(1, at)
     assert torch.equal(out_s.cpu(), ws[:, :k]) and torch.equal(out_i.cpu(), wi[:, :k])
+
+
+@pytest.mark.parametrize("k", [3, 16, 32])
+@pytest.mark.parametrize("N", [100, 5000])
+def test_equal_scores_and_no_scores(N, k):
+    """Rows that occur several times come by their number; rows that are no number are no hits; scores of both signs."""
+    d, nq = 64, 33
+    g = torch.Generator().manual_seed(N + k)
+    some = torch.nn.functional.normalize(torch.randn(7, d, generator=g), dim=1)
+    which = torch.randint(0, 7, (N,), generator=g)
+    X = some[which].bfloat16()
+    bad = torch.arange(N) % 11 == 5
+    X[bad] = float("nan")
+    Q = torch.nn.functional.normalize(torch.randn(nq, d, generator=g), dim=1).bfloat16()
+    Q[0], Q[1] = -some[0].bfloat16(), 0  # (a query of which every score but one kind's is above the least; one of equal scores)
+    s, i = score_topk(X.cuda(), Q.cuda(), k)
+    s, i = s.cpu(), i.cpu()
+    for q in range(nq):
+        full = Q[q].float() @ some.bfloat16().float().T  # 7 values: well apart, or equal
+        order = full.sort(dim=0, descending=True, stable=True)
+        want = torch.where(bad, -9.0, full[which])
+        ws, wi = want.sort(dim=0, descending=True, stable=True)
+        kinds = which[i[q]]
+        assert bool((want[i[q]] > -9).all()) and (s[q] - ws[:k]).abs().max() < d * 2 ** -24
+        if order.values.diff().abs().min() > d * 2 ** -23 or q == 1:
+            assert torch.equal(i[q], wi[:k]), (q, kinds)
