@@ -12,9 +12,13 @@ from .linear import num_cus
 OP_EQ, OP_BITAND = 1, 2
 MAX_FILTERS = 4
 MAX_K = 32
-# 64 queries a workgroup read the rows once for all of them but leave two waves a SIMD for the lists' upkeep: from ~half a
-# million rows the reads win (1M x 768: 64 queries 639 -> 532 us, 128 1220 -> 870), below they do not (100K: 122 against 221)
-NQT4_MIN_ROWS = 1 << 19
+# 64 queries a workgroup read the rows once for all of them, but take twice the lists' upkeep and half the loads in flight: they win
+# where the table is as large as this many rows of 768 (60 queries, k = 16 / 5 with 64 against 32 a workgroup, us: 104K rows of 768
+# 70 / 62 against 63 / 59, 130K 76 / 68 against 74 / 70, 163K 87 / 79 against 87 / 83, 260K 135 / 127 against 145 / 141, 1M 405 / 397
+# against 483 / 479; 208K rows of 384 78 / 70 against 78 / 74, 417K 138 / 130 against 147 / 143; of 1152 69K 72 / 64 against 65 / 61, 87K
+# 77 / 69 against 83 / 80), and in no table of narrower rows (780K of 256: 209 / 201 against 205 / 200)
+NQT4_MIN_ROWS = 1 << 17
+NQT4_MIN_D = 384
 _MAX_LISTS = 1024  # lists of a query that the merge takes
 NQT4_MAX_D = 1152  # widest rows of which a workgroup's LDS holds 64 queries
 
@@ -110,7 +114,7 @@ def _nqt_for(nq, d, kmax, rows):
         return 1 if nq <= 16 else 2
     if nq <= 16:
         return 1
-    if nq <= 32 or d > NQT4_MAX_D or rows < NQT4_MIN_ROWS:
+    if nq <= 32 or not NQT4_MIN_D <= d <= NQT4_MAX_D or rows * d < NQT4_MIN_ROWS * 768:
         return 2
     return 4
 
@@ -139,8 +143,8 @@ def score_topk(X: torch.Tensor, Q: torch.Tensor, k: int, preds=None, bitmap=None
     nqt = _nqt_for(nq, d, kmax, rows)
     nqtiles = (nq + nqt * 16 - 1) // (nqt * 16)
     # a workgroup per CU in all: the kernel keeps its stream up with 8 waves a CU, and every workgroup more is a list more to build and
-    # to merge (1M rows 1024 / 512 / 256 workgroups: 16 queries 334 / 304 / 298 us, 64 with k = 30 and a filter 831 / 741 / 665; 85K
-    # rows, 21 queries 104 / 79 / 61)
+    # to merge (1024 / 512 / 256 workgroups, us: 1M rows, 16 queries 284 / 271 / 265, 64 with k = 30 700 / 655 / 577; 250K, 16 queries 102
+    # / 86 / 79; 85K, 21 queries 70 / 57 / 43)
     target = max(1, min(_MAX_LISTS, num_cus()) // nqtiles)
     rows_per_wg = max(128, -(-rows // target))
     rows_per_wg = -(-rows_per_wg // 16) * 16
