@@ -311,24 +311,40 @@ delta_prep_kernel(const T* __restrict__ xc, int C, const T* __restrict__ proj, i
 }
 
 // ------------------------------------------------------------------------------------------------ scan over the chunks
-// grid nseq * H * ceil(vd / 16) (the column tiles of a head beside each other, on one XCD), 256 threads.  Wave w has token
+// The sequence with the item-th longest portion (equal ones, and more than 64 sequences, as they come).
+__device__ __forceinline__ int by_length(const int* q_start, int nseq, int item) {
+  if (nseq > 64) return item;
+  const int lane = threadIdx.x & 63, own = min(lane, nseq - 1), len = q_start[own + 1] - q_start[own];
+  int rank = 0;
+  for (int j = 0; j < nseq; ++j) {
+    const int o = __builtin_amdgcn_readlane(len, j);
+    rank += o > len || (o == len && j < lane);
+  }
+  return __ffsll((unsigned long long)__ballot(lane < nseq && rank == item)) - 1;
+}
+
+// grid 8 * ceil(nseq * H / 8) * ceil(vd / 16): the column tiles of a head beside each other on one XCD (they read the same operands),
+// the next head on the next XCD, the longest portions first (a contiguous range of sequences an XCD left those with short ones idle: 28
+// heads of 128 x 128, 12 portions of 7000 tokens together 305 us -> 174, 4 of 2500 129 -> 74; by q / k heads, 4 here, one portion is
+// slower by a tenth than by heads), 256 threads.  Wave w has token
 // block w of every chunk and rows 32 kg .. + 31 of the state's 16 columns for kg = w, w + 4.  NDM >= ND = ceil(d / 32).
 template <typename T, int NDM>
 __global__ void __launch_bounds__(256)
 delta_scan_kernel(const T* __restrict__ xc, int C, float* __restrict__ state, const int* __restrict__ slots,
-                  const int* __restrict__ q_start, const int* __restrict__ ctx_len, float* __restrict__ out, int H, int G,
-                  int d, int vd, int nslots, const T* __restrict__ wk, const float* __restrict__ wh, int nchunks) {
+                  const int* __restrict__ q_start, const int* __restrict__ ctx_len, float* __restrict__ out, int nseq,
+                  int H, int G, int d, int vd, int nslots, const T* __restrict__ wk, const float* __restrict__ wh, int nchunks) {
   constexpr int NG = (NDM + 3) / 4, RS = Right<T>::PLANES * 512;
   __shared__ __attribute__((aligned(16))) T So[NDM * RS];  // S_0 as right operands
   __shared__ __attribute__((aligned(16))) T Co[2 * RS];    // e^(L_63 - L_t) / |k_t| u_t as right operands
   __shared__ __attribute__((aligned(16))) float Rl[4][256], Ul[4][256];
   const int ntile = (vd + 15) / 16;
-  const int id = xcd_remap(blockIdx.x, gridDim.x);
-  const int tile = id % ntile, h = (id / ntile) % H, seq = id / ntile / H;
+  const int tile = (blockIdx.x >> 3) % ntile, unit = (blockIdx.x >> 3) / ntile * 8 + (blockIdx.x & 7), h = unit % H, gk = h / (H / G);
+  if (unit >= nseq * H) return;
+  const int seq = by_length(q_start, nseq, unit / H);
   const int qa = q_start[seq], qlen = q_start[seq + 1] - qa;
   if (qlen <= 0) return;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, ql = lane & 15, quad = lane >> 4;
-  const int ND = (d + 31) / 32, dp = 32 * ND, gk = h / (H / G), n = 16 * tile + ql;
+  const int ND = (d + 31) / 32, dp = 32 * ND, n = 16 * tile + ql;
   const bool n_ok = n < vd, fresh = ctx_len[seq] - qlen == 0;
   const int slot = slots[seq];
   const bool slot_ok = index_ok(slot, nslots, ERR_SAMPLER_SLOT);
@@ -634,7 +650,7 @@ GRAG_API hipError_t grag_delta_scan(const void* xc, int C, const void* proj, int
   const size_t bytes = (kq > tri ? kq : tri) + (2560 + 5 * DC) * sizeof(float);
 #define DELTA_SCAN(NDM)                                                                                              \
   hipLaunchKernelGGL((delta_scan_kernel<T, NDM>), grid, dim3(256), 0, st, (const T*)xc, C, state, slots, q_start,    \
-                     ctx_len, out, H, G, d, vd, nslots, (const T*)wk, (const float*)wh, nchunks)
+                     ctx_len, out, nseq, H, G, d, vd, nslots, (const T*)wk, (const float*)wh, nchunks)
   DT_DISPATCH(dt, {
     if (bytes > 48 * 1024) {
       const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_prep_kernel<T>),
@@ -643,7 +659,7 @@ GRAG_API hipError_t grag_delta_scan(const void* xc, int C, const void* proj, int
     }
     hipLaunchKernelGGL(delta_prep_kernel<T>, dim3(H, maxch, nseq), dim3(256), bytes, st, (const T*)xc, C, (const T*)proj,
                        ld, boff, aoff, a_log, dt_bias, q_start, H, G, d, vec, (T*)wk, (float*)wh, nchunks);
-    const dim3 grid((unsigned)nseq * H * ntile);
+    const dim3 grid(((unsigned)nseq * H + 7) / 8 * 8 * ntile);
     if (ND <= 2) {
       DELTA_SCAN(2);
     } else if (ND <= 4) {
