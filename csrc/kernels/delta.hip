@@ -326,9 +326,13 @@ __device__ __forceinline__ int by_length(const int* q_start, int nseq, int item)
 // grid 8 * ceil(nseq * H / 8) * ceil(vd / 16): the column tiles of a head beside each other on one XCD (they read the same operands),
 // the next head on the next XCD, the longest portions first (a contiguous range of sequences an XCD left those with short ones idle: 28
 // heads of 128 x 128, 12 portions of 7000 tokens together 305 us -> 174, 4 of 2500 129 -> 74; by q / k heads, 4 here, one portion is
-// slower by a tenth than by heads), 256 threads.  Wave w has token
+// slower by a tenth than by heads), 256 threads.  Bound by the latency of a chunk's steps, two workgroups a CU; a wave has up to four
+// times another's fp32 steps, so the next 256 workgroups give their tokens to the waves in the other order.  EXACT: d = 32 NDM, so that
+// nothing is tested between the products and LDS is read ahead of them; with that and loads on every path (below) the mixer of 12
+// heads over one portion of 1200 tokens 82 us -> 70, that of 28 heads over 12 portions of 7000 together 330 -> 311 (with 32 columns a
+// workgroup in place of 16 before that: 115, 398).  Wave w has token
 // block w of every chunk and rows 32 kg .. + 31 of the state's 16 columns for kg = w, w + 4.  NDM >= ND = ceil(d / 32).
-template <typename T, int NDM>
+template <typename T, int NDM, bool EXACT>
 __global__ void __launch_bounds__(256)
 delta_scan_kernel(const T* __restrict__ xc, int C, float* __restrict__ state, const int* __restrict__ slots,
                   const int* __restrict__ q_start, const int* __restrict__ ctx_len, float* __restrict__ out, int nseq,
@@ -343,8 +347,9 @@ delta_scan_kernel(const T* __restrict__ xc, int C, float* __restrict__ state, co
   const int seq = by_length(q_start, nseq, unit / H);
   const int qa = q_start[seq], qlen = q_start[seq + 1] - qa;
   if (qlen <= 0) return;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, ql = lane & 15, quad = lane >> 4;
-  const int ND = (d + 31) / 32, dp = 32 * ND, n = 16 * tile + ql;
+  const int lane = threadIdx.x & 63, ql = lane & 15, quad = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) ^ (blockIdx.x >> 8 & 1 ? 3 : 0));
+  const int ND = EXACT ? NDM : (d + 31) / 32, dp = 32 * ND, n = 16 * tile + ql;
   const bool n_ok = n < vd, fresh = ctx_len[seq] - qlen == 0;
   const int slot = slots[seq];
   const bool slot_ok = index_ok(slot, nslots, ERR_SAMPLER_SLOT);
@@ -367,91 +372,112 @@ delta_scan_kernel(const T* __restrict__ xc, int C, float* __restrict__ state, co
   const size_t kstep = (size_t)G * 3 * DC * dp, hstep = (size_t)H * HB_FLOATS;
   const T* kb = wk + ((size_t)crow * G + gk) * 3 * DC * dp;
   const float* hb = wh + ((size_t)crow * H + h) * HB_FLOATS;
-  const T* vp = xc + (size_t)(qa + 16 * w + 4 * quad) * C + 2 * G * d + h * vd + (n_ok ? n : 0);
+  const T* vp = xc + (size_t)qa * C + 2 * G * d + h * vd + (n_ok ? n : 0);
   float* op = out + (size_t)(qa + 16 * w + 4 * quad) * (size_t)(H * vd) + h * vd + n;
   // operands of the chunk at hand; each set is fetched for the next chunk as soon as this one has used it
   Frag<T> kf[NDM], qf[NDM], tf[NG][2][2];
   f32x4_t Tf[4], Mf[4], sa, sb, sq, sc;
   T vv[4];
   float end;
+  // (every load is issued on every path, past what is there again at the last of it: only then are the waits counted, and what was
+  // fetched for the next chunk stays in flight)
   auto fetch_qk = [&](const T* kc, const float* hc, int left) {
 #pragma unroll
-    for (int k = 0; k < NDM; ++k)
-      if (k < ND) {
-        kf[k].load(kc + ((w * ND + k) * 64 + lane) * 8);
-        qf[k].load(kc + DC * dp + ((w * ND + k) * 64 + lane) * 8);
-      }
+    for (int k = 0; k < NDM; ++k) {
+      const int kg = min(k, ND - 1);
+      kf[k].load(kc + ((w * ND + kg) * 64 + lane) * 8);
+      qf[k].load(kc + DC * dp + ((w * ND + kg) * 64 + lane) * 8);
+    }
     sa = *reinterpret_cast<const f32x4_t*>(hc + 5120 + 16 * w + 4 * quad);
     sb = *reinterpret_cast<const f32x4_t*>(hc + 5120 + 64 + 16 * w + 4 * quad);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) vv[i] = 16 * w + 4 * quad + i < left ? vp[(size_t)i * C] : (T)0.f;
+    for (int i = 0; i < 4; ++i) vv[i] = vp[(size_t)min(16 * w + 4 * quad + i, left - 1) * C];
   };
   auto fetch_t = [&](const float* hc) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j <= w) Tf[j] = *reinterpret_cast<const f32x4_t*>(hc + (w * (w + 1) / 2 + j) * 256 + lane * 4);
+    for (int j = 0; j < 4; ++j) Tf[j] = *reinterpret_cast<const f32x4_t*>(hc + (w * (w + 1) / 2 + min(j, w)) * 256 + lane * 4);
     sc = *reinterpret_cast<const f32x4_t*>(hc + 5120 + 192 + 16 * w + 4 * quad);
   };
   auto fetch_m = [&](const T* kc, const float* hc) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j <= w) Mf[j] = *reinterpret_cast<const f32x4_t*>(hc + 2560 + (w * (w + 1) / 2 + j) * 256 + lane * 4);
+    for (int j = 0; j < 4; ++j) Mf[j] = *reinterpret_cast<const f32x4_t*>(hc + 2560 + (w * (w + 1) / 2 + min(j, w)) * 256 + lane * 4);
     sq = *reinterpret_cast<const f32x4_t*>(hc + 5120 + 128 + 16 * w + 4 * quad);
     end = hc[5120 + 256];
 #pragma unroll
     for (int g = 0; g < NG; ++g)
-      if (w + 4 * g < ND) {
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+      for (int b = 0; b < 2; ++b)
 #pragma unroll
-          for (int ks = 0; ks < 2; ++ks)
-            tf[g][b][ks].load(kc + 2 * DC * dp + (((2 * (w + 4 * g) + b) * 2 + ks) * 64 + lane) * 8);
-      }
+        for (int ks = 0; ks < 2; ++ks)
+          tf[g][b][ks].load(kc + 2 * DC * dp + (((2 * min(w + 4 * g, ND - 1) + b) * 2 + ks) * 64 + lane) * 8);
   };
   fetch_qk(kb, hb, qlen);
   fetch_t(hb);
   fetch_m(kb, hb);
   const f32x4_t zero = f32x4_t{0.f, 0.f, 0.f, 0.f};
   for (int c = 0; c < nch; ++c) {
-    const bool more = c + 1 < nch;
     const int left = qlen - c * DC;
+    const bool more = left > DC;
+    kb += more ? kstep : 0;  // (the next chunk's, or this one's again)
+    hb += more ? hstep : 0;
+    vp += more ? (size_t)DC * C : 0;
     __syncthreads();
     // the start state seen by the chunk's keys and queries, and the right-hand side of the triangular system
     f32x4_t ks = zero, qs = zero;
+    if (EXACT) {  // (with nothing tested the reads of a block run ahead of the products of the one before)
+      Right<T> b[2];
+      b[0].load(So, lane);
 #pragma unroll
-    for (int k = 0; k < NDM; ++k)
-      if (k < ND) {
-        Right<T> b;
-        b.load(So + k * RS, lane);
-        ks = mm32(kf[k], b, ks);
-        qs = mm32(qf[k], b, qs);
+      for (int k = 0; k < NDM; ++k) {
+        if (k + 1 < NDM) b[(k + 1) & 1].load(So + (k + 1) * RS, lane);
+        ks = mm32(kf[k], b[k & 1], ks);
+        qs = mm32(qf[k], b[k & 1], qs);
       }
+    } else {
+#pragma unroll
+      for (int k = 0; k < NDM; ++k)
+        if (k < ND) {
+          Right<T> b;
+          b.load(So + k * RS, lane);
+          ks = mm32(kf[k], b, ks);
+          qs = mm32(qf[k], b, qs);
+        }
+    }
     f32x4_t r;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = fmaf(sb[i], (float)vv[i], -sa[i] * ks[i]);
+    for (int i = 0; i < 4; ++i) r[i] = fmaf(sb[i], 16 * w + 4 * quad + i < left ? (float)vv[i] : 0.f, -sa[i] * ks[i]);
     *reinterpret_cast<f32x4_t*>(&Rl[w][lane * 4]) = r;
-    vp += (size_t)DC * C;
-    if (more) fetch_qk(kb + kstep, hb + hstep, left - DC);
+    fetch_qk(kb, hb, more ? left - DC : left);
     __syncthreads();
-    f32x4_t u = zero;
+    f32x4_t u = zero, x[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = *reinterpret_cast<const f32x4_t*>(&Rl[j][lane * 4]);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (j <= w) u = mm16(Tf[j], *reinterpret_cast<const f32x4_t*>(&Rl[j][lane * 4]), u);
+      if (j <= w) u = mm16(Tf[j], x[j], u);
     *reinterpret_cast<f32x4_t*>(&Ul[w][lane * 4]) = u;
     Right<T>::store(Co + (w >> 1) * RS, lane, w & 1, sc * u);
-    if (more) fetch_t(hb + hstep);
+    fetch_t(hb);
     __syncthreads();
     f32x4_t o = sq * qs;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j <= w) o = mm16(Mf[j], *reinterpret_cast<const f32x4_t*>(&Ul[j][lane * 4]), o);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (n_ok && 16 * w + 4 * quad + i < left) op[(size_t)i * (H * vd)] = o[i];
-    op += (size_t)DC * (H * vd);
     Right<T> cu[2];
 #pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = *reinterpret_cast<const f32x4_t*>(&Ul[j][lane * 4]);
+#pragma unroll
     for (int k = 0; k < 2; ++k) cu[k].load(Co + k * RS, lane);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j <= w) o = mm16(Mf[j], x[j], o);
+    if (more) {  // (all rows are there)
+      if (n_ok)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) op[(size_t)i * (H * vd)] = o[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (n_ok && 16 * w + 4 * quad + i < left) op[(size_t)i * (H * vd)] = o[i];
+    }
+    op += (size_t)DC * (H * vd);
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
       if (w + 4 * g >= ND) continue;
@@ -461,9 +487,7 @@ delta_scan_kernel(const T* __restrict__ xc, int C, float* __restrict__ state, co
         Right<T>::store(So + (w + 4 * g) * RS, lane, b, S[g][b]);
       }
     }
-    kb += kstep;
-    hb += hstep;
-    if (more) fetch_m(kb, hb);
+    fetch_m(kb, hb);
   }
   if (!slot_ok || !n_ok) return;
 #pragma unroll
@@ -648,9 +672,10 @@ GRAG_API hipError_t grag_delta_scan(const void* xc, int C, const void* proj, int
   const size_t lk = dp + (dt == 0 ? 8 : 4);
   const size_t kq = 2 * DC * lk * (dt == 0 ? 2 : 4), tri = DC * 68 * sizeof(float);
   const size_t bytes = (kq > tri ? kq : tri) + (2560 + 5 * DC) * sizeof(float);
-#define DELTA_SCAN(NDM)                                                                                              \
-  hipLaunchKernelGGL((delta_scan_kernel<T, NDM>), grid, dim3(256), 0, st, (const T*)xc, C, state, slots, q_start,    \
-                     ctx_len, out, nseq, H, G, d, vd, nslots, (const T*)wk, (const float*)wh, nchunks)
+#define DELTA_SCAN(NDM)                                                                                               \
+  (ND == NDM ? &delta_scan_kernel<T, NDM, true> : &delta_scan_kernel<T, NDM, false>)<<<grid, 256, 0, st>>>(           \
+      (const T*)xc, C, state, slots, q_start, ctx_len, out, nseq, H, G, d, vd, nslots, (const T*)wk, (const float*)wh, \
+      nchunks)
   DT_DISPATCH(dt, {
     if (bytes > 48 * 1024) {
       const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_prep_kernel<T>),
