@@ -116,22 +116,27 @@ __device__ __forceinline__ float sum4(float v) {
 __device__ __forceinline__ int chunk_row(int qa, int seq) { return qa / DC + seq; }
 
 // ------------------------------------------------------------------------------------------------ operands of the scan
-// grid (H, max chunks, nseq), 256 threads.  wk [nchunks][G] blocks of 3 DC dp T's: K frags [4][ND][64][8], Q frags (the
+// grid (8 * ceil(max chunks / 8) * H, nseq), 256 threads: the heads of a chunk beside each other on one XCD, as they read the same rows of
+// q and k and the same lines of the projection, the next chunk on the next XCD (the mixer of 28 heads of 128 x 128, 12 portions of 7000 tokens
+// together 313 us -> 305).  NDE: ceil(d / 32) where it is compiled in (0: any), so that the reads of a triangle's block run ahead of its
+// products; a wave forms a block of both triangles at once, which share k's rows and the decays (this kernel 67 -> 52 us, 7 chunks
+// of 12 heads 14.4 -> 11).  wk [nchunks][G] blocks of 3 DC dp T's: K frags [4][ND][64][8], Q frags (the
 // same), K^T frags [2 ND][2][64][8] (dp = 32 ND: d rounded up, zeros behind d); wh [nchunks][H] blocks of HB_FLOATS.
 // Lower block (i, j <= i) of a 64 x 64 triangle has number i (i + 1) / 2 + j.
-template <typename T>
+template <typename T, int NDE>
 __global__ void __launch_bounds__(256)
 delta_prep_kernel(const T* __restrict__ xc, int C, const T* __restrict__ proj, int ld, int boff, int aoff,
                   const float* __restrict__ a_log, const float* __restrict__ dt_bias, const int* __restrict__ q_start,
                   int H, int G, int d, int vec, T* __restrict__ wk, float* __restrict__ wh, int nchunks) {
   extern __shared__ __attribute__((aligned(16))) unsigned char dsm[];
-  const int seq = blockIdx.z, c = blockIdx.y, h = blockIdx.x, R = H / G, gk = h / R;
+  const int seq = blockIdx.y, c = (blockIdx.x >> 3) / H * 8 + ((blockIdx.x + seq) & 7), h = (blockIdx.x >> 3) % H;
+  const int R = H / G, gk = h / R;
   const int qa = q_start[seq], qlen = q_start[seq + 1] - qa;
   if (c * DC >= qlen) return;
   const int crow = chunk_row(qa, seq) + c;
   if (crow >= nchunks) return;
   const int nrow = min(DC, qlen - c * DC), r0 = qa + c * DC;
-  const int ND = (d + 31) / 32, dp = 32 * ND, lk = dp + (sizeof(T) == 2 ? 8 : 4);
+  const int ND = NDE ? NDE : (d + 31) / 32, dp = 32 * ND, lk = dp + (sizeof(T) == 2 ? 8 : 4);
   T* Ks = reinterpret_cast<T*>(dsm);
   T* Qs = Ks + DC * lk;
   float* Ts = reinterpret_cast<float*>(dsm);  // [64][68], in the place of K and Q once they have been used
@@ -221,34 +226,39 @@ delta_prep_kernel(const T* __restrict__ xc, int C, const T* __restrict__ proj, i
   }
   // the triangles A (into LDS) and M (into the scratch), transposed products: rows s, column t, which is the order a left
   // operand with row t wants
-  for (int idx = w; idx < 20; idx += 4) {
-    const int p = idx % 10, i = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3, j = p - i * (i + 1) / 2;
-    const bool isq = idx >= 10;
-    const T* ap = Ks + (16 * j + ql) * lk;
-    const T* bp = (isq ? Qs : Ks) + (16 * i + ql) * lk;
-    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int p = w; p < 10; p += 4) {
+    const int i = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3, j = p - i * (i + 1) / 2;
+    const T *kj = Ks + (16 * j + ql) * lk, *ki = Ks + (16 * i + ql) * lk, *qi = Qs + (16 * i + ql) * lk;
+    f32x4_t acc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
     for (int kg = 0; kg < ND; ++kg) {
       if constexpr (sizeof(T) == 2) {
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(ap + 32 * kg + 8 * quad),
-                                                      *reinterpret_cast<const bf16x8_t*>(bp + 32 * kg + 8 * quad), acc, 0,
-                                                      0, 0);
+        const int o = 32 * kg + 8 * quad;
+        const bf16x8_t x = *reinterpret_cast<const bf16x8_t*>(kj + o);
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, *reinterpret_cast<const bf16x8_t*>(ki + o), acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, *reinterpret_cast<const bf16x8_t*>(qi + o), acc[1], 0, 0, 0);
       } else {
 #pragma unroll
-        for (int e = 0; e < 2; ++e)
-          acc = mm16(*reinterpret_cast<const f32x4_t*>(ap + 32 * kg + 16 * e + 4 * quad),
-                     *reinterpret_cast<const f32x4_t*>(bp + 32 * kg + 16 * e + 4 * quad), acc);
+        for (int e = 0; e < 2; ++e) {
+          const int o = 32 * kg + 16 * e + 4 * quad;
+          const f32x4_t x = *reinterpret_cast<const f32x4_t*>(kj + o);
+          acc[0] = mm16(x, *reinterpret_cast<const f32x4_t*>(ki + o), acc[0]);
+          acc[1] = mm16(x, *reinterpret_cast<const f32x4_t*>(qi + o), acc[1]);
+        }
       }
     }
-    const int t = 16 * i + ql;
-    const float lt = lh[t], lt2 = ll[t], ft = isq ? rq[t] : be[t] * rk[t];
+    const int t = 16 * i + ql, s0 = 16 * j + 4 * quad;
+    const float lt = lh[t], lt2 = ll[t], ft[2] = {be[t] * rk[t], rq[t]};
+    const f32x4_t ls = *reinterpret_cast<const f32x4_t*>(lh + s0), ls2 = *reinterpret_cast<const f32x4_t*>(ll + s0),
+                  rs = *reinterpret_cast<const f32x4_t*>(rk + s0);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int s = 16 * j + 4 * quad + r;
-      const float e = expf(fminf((lt - lh[s]) + (lt2 - ll[s]), 0.f)) * ft * rk[s];
-      acc[r] = (isq ? s <= t : s < t) ? acc[r] * e : 0.f;
+      const float e = expf(fminf((lt - ls[r]) + (lt2 - ls2[r]), 0.f));
+      acc[0][r] = s0 + r < t ? acc[0][r] * (e * ft[0] * rs[r]) : 0.f;
+      acc[1][r] = s0 + r <= t ? acc[1][r] * (e * ft[1] * rs[r]) : 0.f;
     }
-    float* dst = isq ? hb + 2560 + p * 256 : Af + p * 256;
-    *reinterpret_cast<f32x4_t*>(dst + lane * 4) = acc;
+    *reinterpret_cast<f32x4_t*>(Af + p * 256 + lane * 4) = acc[0];
+    *reinterpret_cast<f32x4_t*>(hb + 2560 + p * 256 + lane * 4) = acc[1];
   }
   if (w == 3) {
     const float lt = lh[lane] + ll[lane], el = expf(lt);
@@ -677,13 +687,14 @@ GRAG_API hipError_t grag_delta_scan(const void* xc, int C, const void* proj, int
       (const T*)xc, C, state, slots, q_start, ctx_len, out, nseq, H, G, d, vd, nslots, (const T*)wk, (const float*)wh, \
       nchunks)
   DT_DISPATCH(dt, {
+    auto* prep = ND == 4 ? &delta_prep_kernel<T, 4> : ND == 2 ? &delta_prep_kernel<T, 2> : &delta_prep_kernel<T, 0>;
     if (bytes > 48 * 1024) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_prep_kernel<T>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(prep), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               (int)bytes);
       if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(delta_prep_kernel<T>, dim3(H, maxch, nseq), dim3(256), bytes, st, (const T*)xc, C, (const T*)proj,
-                       ld, boff, aoff, a_log, dt_bias, q_start, H, G, d, vec, (T*)wk, (float*)wh, nchunks);
+    prep<<<dim3((maxch + 7) / 8 * 8 * H, nseq), 256, bytes, st>>>((const T*)xc, C, (const T*)proj, ld, boff, aoff, a_log, dt_bias,
+                                                                  q_start, H, G, d, vec, (T*)wk, (float*)wh, nchunks);
     const dim3 grid(((unsigned)nseq * H + 7) / 8 * 8 * ntile);
     if (ND <= 2) {
       DELTA_SCAN(2);
