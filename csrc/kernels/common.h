@@ -218,6 +218,19 @@ __device__ __forceinline__ int xcd_remap(int orig, int nwg) {
   return base + orig / 8;
 }
 
+// The sequence with the item-th longest portion (equal ones, and more than 64 sequences, as they come): for workgroups that walk whole
+// portions, so that the last ones to start are short.
+__device__ __forceinline__ int by_length(const int* q_start, int nseq, int item) {
+  if (nseq > 64) return item;
+  const int lane = threadIdx.x & 63, own = min(lane, nseq - 1), len = q_start[own + 1] - q_start[own];
+  int rank = 0;
+  for (int j = 0; j < nseq; ++j) {
+    const int o = __builtin_amdgcn_readlane(len, j);
+    rank += o > len || (o == len && j < lane);
+  }
+  return __ffsll((unsigned long long)__ballot(lane < nseq && rank == item)) - 1;
+}
+
 // ---- device-side index guard --------------------------------------------------------------------
 // Kernels whose addresses come from index INPUTS (token ids, KV slot ids, block-table entries, row ids,
 // cross-workgroup tickets) check them.  An out-of-range index skips its access and records (code, value)

@@ -321,18 +321,6 @@ delta_prep_kernel(const T* __restrict__ xc, int C, const T* __restrict__ proj, i
 }
 
 // ------------------------------------------------------------------------------------------------ scan over the chunks
-// The sequence with the item-th longest portion (equal ones, and more than 64 sequences, as they come).
-__device__ __forceinline__ int by_length(const int* q_start, int nseq, int item) {
-  if (nseq > 64) return item;
-  const int lane = threadIdx.x & 63, own = min(lane, nseq - 1), len = q_start[own + 1] - q_start[own];
-  int rank = 0;
-  for (int j = 0; j < nseq; ++j) {
-    const int o = __builtin_amdgcn_readlane(len, j);
-    rank += o > len || (o == len && j < lane);
-  }
-  return __ffsll((unsigned long long)__ballot(lane < nseq && rank == item)) - 1;
-}
-
 // grid 8 * ceil(nseq * H / 8) * ceil(vd / 16): the column tiles of a head beside each other on one XCD (they read the same operands),
 // the next head on the next XCD, the longest portions first (a contiguous range of sequences an XCD left those with short ones idle: 28
 // heads of 128 x 128, 12 portions of 7000 tokens together 305 us -> 174, 4 of 2500 129 -> 74; by q / k heads, 4 here, one portion is

@@ -373,8 +373,14 @@ __global__ void ssm_chunk_prefix_kernel(float* __restrict__ state, const int* __
 //   staging   wave w forms the step sizes of its 16 channels for the 16 tokens -- for bf16 one 16 x 16 matrix-core tile
 //             (operand lane: row lane % 16, k = 8 (lane / 16) .. + 7; result lane: tokens 4 (lane / 16) + i, channel
 //             lane % 16) -- and leaves (dt log2 e, dt x) per (token, channel) in LDS, beside the tokens' B and C rows;
-//   walk      every thread updates its numbers; the four parts of a channel add up their share of y;
+//   walk      every thread updates its numbers, four tokens at a time (up to 16 of them: the next four's are read meanwhile);
+//             the four parts of a channel add up their share of y;
 //   store     the lane that formed dt adds D x, gates and stores.
+// Bound by a token's chain where a CU has few waves (one portion: 0.145 us a token), else by vector instructions (four of 20 are
+// exponentials of a quarter's rate: 173 cycles a token and workgroup, 140 at best).  Reading a token's numbers as it was walked left
+// the latency of LDS to every token; the rows of low go through LDS, for registers that three workgroups a CU leave; and whole
+// portions start longest first, so that a CU's workgroups are not all long ones.  Channels 3584, 12 portions of 7000 tokens
+// together: 281 us with the convolution -> 206, one of 1200 77 -> 70.
 // Long portions are cut into chunks of `chunk` tokens (a multiple of SC_TB) that run side by side:
 //   MODE 0  the whole portion, from and to the slot's state;
 //   MODE 1  grid.z = chunk: the chunk's own contribution from a zero state -> ws [nseq * maxchunks][inner][N], and the sum
@@ -390,6 +396,21 @@ __device__ __forceinline__ float quad_sum(float v) {
   return v;
 }
 
+// what a lane of the walk reads for four tokens: their (dt log2 e, dt x), its four of their B and (OUT) C
+template <bool OUT> struct Walk4 {
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  f32x2_t d[4];
+  f32x4_t b[4], c[OUT ? 4 : 1];
+  __device__ __forceinline__ void read(const f32x2_t* sd, const float* bc) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      d[u] = sd[u * SC_CH];
+      b[u] = *reinterpret_cast<const f32x4_t*>(bc + u * 32);
+      if (OUT) c[u] = *reinterpret_cast<const f32x4_t*>(bc + u * 32 + 16);
+    }
+  }
+};
+
 template <typename T, int NPT, int MODE>
 __global__ void __launch_bounds__(256)
 chan_scan_kernel(const T* __restrict__ xc, const T* __restrict__ low, int low_ld, const T* __restrict__ wdt, int R, int Rp,
@@ -399,11 +420,13 @@ chan_scan_kernel(const T* __restrict__ xc, const T* __restrict__ low, int low_ld
                  int nslots, float* __restrict__ ws, float* __restrict__ wa, int chunk_len, int maxchunks) {
   constexpr float LOG2E = 1.4426950408889634f;
   constexpr int NP = 4 * NPT;
+  constexpr int NW = 8;  // matrix fragments kept in registers (R up to 256); the rest is read again per tile
   typedef float f32x2_t __attribute__((ext_vector_type(2)));
   __shared__ __attribute__((aligned(16))) float bc[SC_TB][2][NP];
   __shared__ __attribute__((aligned(16))) f32x2_t sd[SC_TB][SC_CH];
   __shared__ float sy[MODE == 1 ? 1 : SC_TB][SC_CH];
-  const int seq = blockIdx.y, c0 = blockIdx.x * SC_CH;
+  __shared__ bf16x8_t ls[sizeof(T) == 2 ? NW : 1][64];  // the tile's rows of low as fragments: all four waves multiply them
+  const int seq = MODE == 0 ? by_length(q_start, gridDim.y, blockIdx.y) : blockIdx.y, c0 = blockIdx.x * SC_CH;  // (longest first)
   int qa = q_start[seq], qlen = q_start[seq + 1] - qa;
   if (qlen <= 0) return;
   const bool fresh = ctx_len[seq] - qlen == 0;
@@ -456,9 +479,8 @@ chan_scan_kernel(const T* __restrict__ xc, const T* __restrict__ low, int low_ld
   const int scc = sc_ok ? sc : 0;  // (loads of lanes past the last channel or token go to a valid place and are not used)
   const float bias = sc_ok ? dt_bias[sc] : 0.f, dsk = sc_ok ? Dv[sc] : 0.f;
   const T* wrow = wdt + (size_t)scc * Rp;
-  constexpr int NW = 8;  // matrix fragments kept in registers (R up to 256); the rest is read again per tile
   constexpr int NB = NPT <= 8 ? SC_TB * 2 * NP / 256 : 1;  // B / C elements per thread fetched ahead
-  bf16x8_t wf[NW], lf[NW];
+  bf16x8_t wf[NW], lf[NW / 4];  // (lf: a wave's share of the tile's rows of low, every fourth fragment)
   T xn[4], zn[4], bn[NB];  // (as they are read: nothing waits for them before the walk is over)
   if (sizeof(T) == 2) {
 #pragma unroll
@@ -483,8 +505,8 @@ chan_scan_kernel(const T* __restrict__ xc, const T* __restrict__ low, int low_ld
     if (sizeof(T) == 2) {
       const T* lrow = low + (size_t)(qa + t0 + min(ql, nb - 1)) * low_ld;
 #pragma unroll
-      for (int k = 0; k < NW; ++k)
-        if (32 * k < Rp) lf[k] = lfrag(lrow, k);
+      for (int k = 0; k < NW / 4; ++k)
+        if (32 * (wid + 4 * k) < Rp) lf[k] = lfrag(lrow, wid + 4 * k);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -497,7 +519,16 @@ chan_scan_kernel(const T* __restrict__ xc, const T* __restrict__ low, int low_ld
       for (int u = 0; u < NB; ++u) bn[u] = bc_at(t0, nb, threadIdx.x + 256 * u);
     }
   };
+  auto share = [&]() {
+    if (sizeof(T) == 2) {
+#pragma unroll
+      for (int k = 0; k < NW / 4; ++k)
+        if (32 * (wid + 4 * k) < Rp) ls[wid + 4 * k][lane] = lf[k];
+    }
+  };
   fetch(0);
+  share();
+  __syncthreads();
   float dtsum = 0.f;
   for (int t0 = 0; t0 < qlen; t0 += SC_TB) {
     const int nb = min(SC_TB, qlen - t0);
@@ -507,7 +538,7 @@ chan_scan_kernel(const T* __restrict__ xc, const T* __restrict__ low, int low_ld
       f32x4_t acc = f32x4_t{bias, bias, bias, bias};
 #pragma unroll
       for (int k = 0; k < NW; ++k)
-        if (32 * k < Rp) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lf[k], wf[k], acc, 0, 0, 0);
+        if (32 * k < Rp) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ls[k][lane], wf[k], acc, 0, 0, 0);
       const T* lrow = low + (size_t)(qa + t0 + min(ql, nb - 1)) * low_ld;
       for (int k = NW; 32 * k < Rp; ++k)
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
@@ -528,7 +559,6 @@ chan_scan_kernel(const T* __restrict__ xc, const T* __restrict__ low, int low_ld
       xv[i] = (float)xn[i];
       if (MODE != 1) zv[i] = (float)zn[i];
     }
-    __syncthreads();  // the tile before is consumed
     // (a token past the portion's end leaves the state as it is: dt = 0, B = C = 0)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -543,30 +573,61 @@ chan_scan_kernel(const T* __restrict__ xc, const T* __restrict__ low, int low_ld
     }
     __syncthreads();
     if (t0 + SC_TB < qlen) fetch(t0 + SC_TB);  // in flight during the walk
-    for (int t4 = 0; t4 < nb; t4 += 4) {
+    if constexpr (NPT == 4) {  // four tokens at a time, the next four's numbers read meanwhile
+      Walk4<MODE != 1> at, next;
+      at.read(&sd[0][cl], &bc[0][0][4 * part]);
+      for (int t4 = 0; t4 < nb; t4 += 4) {
+        const int tn = min(t4 + 4, SC_TB - 4);
+        next.read(&sd[tn][cl], &bc[tn][0][4 * part]);
+        float ex[4][4], y[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int t = t4 + u;
-        const f32x2_t d = sd[t][cl];
-        float y = 0.f;
+        for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int j = 0; j < NPT / 4; ++j) {
-          const f32x4_t b4 = *reinterpret_cast<const f32x4_t*>(&bc[t][0][4 * (part + 4 * j)]);
+          for (int e = 0; e < 4; ++e) ex[u][e] = __builtin_amdgcn_exp2f(at.d[u][0] * a2[e]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            S[4 * j + e] = fmaf(__builtin_amdgcn_exp2f(d[0] * a2[4 * j + e]), S[4 * j + e], d[1] * b4[e]);
-          if (MODE != 1) {
-            const f32x4_t c4 = *reinterpret_cast<const f32x4_t*>(&bc[t][1][4 * (part + 4 * j)]);
+        for (int u = 0; u < 4; ++u) {
+          y[u] = 0.f;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) y = fmaf(S[4 * j + e], c4[e], y);
+          for (int e = 0; e < 4; ++e) {
+            S[e] = fmaf(ex[u][e], S[e], at.d[u][1] * at.b[u][e]);
+            if (MODE != 1) y[u] = fmaf(S[e], at.c[u][e], y[u]);
           }
+          if (MODE == 1) dtsum += at.d[u][0];
         }
-        if (MODE == 1) dtsum += d[0];
-        else sy[t][cl] = quad_sum(y);
+        if (MODE != 1) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) y[u] = quad_sum(y[u]);
+          sy[t4 + part][cl] = part < 2 ? (part == 0 ? y[0] : y[1]) : (part == 2 ? y[2] : y[3]);
+        }
+        at = next;
+      }
+    } else {
+      for (int t4 = 0; t4 < nb; t4 += 4) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int t = t4 + u;
+          const f32x2_t d = sd[t][cl];
+          float y = 0.f;
+#pragma unroll
+          for (int j = 0; j < NPT / 4; ++j) {
+            const f32x4_t b4 = *reinterpret_cast<const f32x4_t*>(&bc[t][0][4 * (part + 4 * j)]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              S[4 * j + e] = fmaf(__builtin_amdgcn_exp2f(d[0] * a2[4 * j + e]), S[4 * j + e], d[1] * b4[e]);
+            if (MODE != 1) {
+              const f32x4_t c4 = *reinterpret_cast<const f32x4_t*>(&bc[t][1][4 * (part + 4 * j)]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) y = fmaf(S[4 * j + e], c4[e], y);
+            }
+          }
+          if (MODE == 1) dtsum += d[0];
+          else sy[t][cl] = quad_sum(y);
+        }
       }
     }
+    if (t0 + SC_TB < qlen) share();
+    __syncthreads();
     if (MODE != 1) {
-      __syncthreads();
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int t = 4 * quad + i;

@@ -392,19 +392,27 @@ def _ssm_scan_cpu(xbc, dtraw, dt_bias, a_log, skip, state, m, H, G, N, P, out):
 
 
 # ---------------------------------------------------------------------------------------------- per-channel scan
-CHAN_SCAN_WGS = 1024  # workgroups (64 channels x one sequence x one chunk) that a portion is cut for
+CHAN_SCAN_WGS = 1024  # workgroups (64 channels x one sequence x one chunk) that fill the chip
 
 
-def _chan_chunk(nseq: int, max_q: int, inner: int) -> int:
-    """Chunk length of the per-channel scan (0: one pass).  The chunked form does the recurrence twice, so a step with
-    enough (channel tile, sequence) workgroups of its own stays whole; others get the longest chunks that fill the chip."""
-    tiles = nseq * -(-inner // 64)
-    if max_q <= 64 or 2 * tiles >= CHAN_SCAN_WGS:
+def _chan_chunk(nseq: int, max_q: int, inner: int, tokens: int | None = None) -> int:
+    """Chunk length of the per-channel scan (0: one pass) for ``nseq`` portions of ``tokens`` together (None: all of ``max_q``).
+
+    The chunked form does the recurrence twice, about 20 us and 0.59 ns a token and 64 channels in all; one pass takes the
+    longest portion's chain, 0.145 us a token, or 0.33 ns a token and 64 channels.  So several portions that fill a quarter of
+    the chip stay whole where their longest is short against the work of all (us, one pass / chunks of 64: 3584 channels, 8
+    portions of 4000 together 129 / 172, 8 of 8000 266 / 310, 4 of 2500 207 / 129; 1536, 16 of 5000 86 / 102, 10 of 5000 110 / 104).
+    Chunks of 128 save starts where there are enough of them and the portions' ends are few, 256 for one portion (chunks of 64 /
+    128 / 256: 1536 channels, one of 4000 101 / 87 / 112, of 1200 48 / 55 / 88, 8 of 4000 94 / 100 / 107; 3584, one of 1200 78 / 71 / 102,
+    of 8192 343 / 309 / 304, 2 of 5000 216 / 199 / 219)."""
+    per = -(-inner // 64)
+    tiles, tokens = nseq * per, nseq * max_q if tokens is None else tokens
+    whole = nseq > 1 and 4 * tiles >= CHAN_SCAN_WGS and 0.145 * max_q < 20 + 0.59e-3 * tokens * per
+    if max_q <= 64 or 2 * tiles >= CHAN_SCAN_WGS or whole:
         return 0
-    for c in (256, 128):
-        if max_q > 2 * c and tiles * -(-max_q // c) >= CHAN_SCAN_WGS:
-            return c
-    return 64
+    if nseq == 1 and max_q > 512 and tokens * per >= 256 * CHAN_SCAN_WGS:
+        return 256
+    return 128 if max_q > 256 and tokens >= 700 * nseq and tokens * per >= 51 * CHAN_SCAN_WGS else 64
 
 
 def pad_step_matrix(w: torch.Tensor) -> torch.Tensor:
@@ -437,7 +445,7 @@ def selective_scan(xc: torch.Tensor, low: torch.Tensor, wdt: torch.Tensor, R: in
         assert dt_bias.numel() == inner and skip.numel() == inner and zoff + inner <= proj.shape[1]
         if N > lib().grag_chan_scan_max_state():
             raise ValueError(f"the scan kernel holds {lib().grag_chan_scan_max_state()} state numbers per channel")
-        chunk, ws, wa = _chan_chunk(m.num_seqs, m.max_q_len, inner), None, None
+        chunk, ws, wa = _chan_chunk(m.num_seqs, m.max_q_len, inner, r1 - r0), None, None
         if chunk:
             nch = m.num_seqs * -(-m.max_q_len // chunk)
             ws = torch.empty(nch * inner * N, dtype=torch.float32, device=xc.device)
