@@ -124,6 +124,18 @@ __device__ __forceinline__ f32x4_t widen(f32x4_t v) { return v; }
 // ------------------------------------------------------------------------------------------------ elements
 __device__ __forceinline__ float elt(const bf16* p) { return (float)*p; }
 __device__ __forceinline__ float elt(const float* p) { return *p; }
+// an element as it is stored: nothing waits for it before it is used
+template <typename TI> struct Raw;
+template <> struct Raw<bf16> {
+  short v = 0;
+  __device__ __forceinline__ void load(const bf16* p) { v = *reinterpret_cast<const short*>(p); }
+  __device__ __forceinline__ float value() const { return bits2f(v); }
+};
+template <> struct Raw<float> {
+  float v = 0.f;
+  __device__ __forceinline__ void load(const float* p) { v = *p; }
+  __device__ __forceinline__ float value() const { return v; }
+};
 __device__ __forceinline__ float softplus_x(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 __device__ __forceinline__ float silu_acc(float x) { return x / (1.f + expf(-x)); }
 __device__ __forceinline__ float pow2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -379,7 +391,7 @@ linear_scan_kernel(const ScanArgs a) {
   constexpr int KT = 4 * ND, KR = LTHREADS / KT, KL = LC / KR > 0 ? LC / KR : 1;  // threads a row, rows a pass, passes
   const int krow = tid / KT, kc = 8 * (tid % KT), vrow = tid >> 3, vc = 8 * (tid & 7);
   TI4 kr[KL][2], vr[2], qr[OUT ? ND : 1][2];
-  float dtr = 0.f;
+  Raw<TI> dtr;
   auto fetch = [&](int c) __attribute__((always_inline)) {
     const int end = min(qlen - c * LC, LC) - 1;
     const size_t t0 = (size_t)(qa + c * LC) * a.ld;
@@ -402,8 +414,7 @@ linear_scan_kernel(const ScanArgs a) {
     }
   };
   auto fetch_dt = [&](int c) __attribute__((always_inline)) {
-    if (SSM)
-      dtr = c * LC + lane < qlen ? elt(reinterpret_cast<const TI*>(a.proj) + (size_t)(qa + c * LC + lane) * a.pld + a.dtoff + h) : 0.f;
+    if (SSM) dtr.load(reinterpret_cast<const TI*>(a.proj) + (size_t)(qa + min(c * LC + lane, qlen - 1)) * a.pld + a.dtoff + h);
   };
   auto position = [&](int t) __attribute__((always_inline)) {
     if (AP == 1 || !a.rd) return 0;
@@ -412,7 +423,7 @@ linear_scan_kernel(const ScanArgs a) {
   };
   float lsum = 0.f;  // the part's log2 decay
   // the head's constants: log2 of the decay and its sign, or the state-space rate and bias
-  const float lam = SSM ? 1.f : a.decay[h], bias = SSM ? a.dt_bias[h] : 0.f;
+  const float lam = SSM ? 1.f : a.decay[h], bias = SSM ? a.dt_bias[h] : 0.f, skip = SSM ? a.skip[h] : 0.f;
   const float rate = SSM ? -expf(a.a_log[h]) * 1.4426950408889634f : fmaxf(log2f(fabsf(lam)), -4000.f);  // (lam^n = 0 for 0)
   const bool neg = lam < 0.f;
   auto scalars = [&](int c) __attribute__((always_inline)) {  // by one wave: lane = token of chunk c
@@ -420,7 +431,7 @@ linear_scan_kernel(const ScanArgs a) {
     const float sign = neg && (lane & 1) ? -1.f : 1.f, esign = neg && (n & 1) ? -1.f : 1.f;  // of lam^lane, lam^n
     float cs = 0.f, hi, lo = 0.f, ehi, elo;
     if (SSM) {
-      if (lane < n) cs = softplus_x(dtr + bias);
+      if (lane < n) cs = softplus_x(dtr.value() + bias);
       hi = rate * cs;
       wave_scan2(hi, lo);
       ehi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hi), 63));
@@ -524,11 +535,11 @@ linear_scan_kernel(const ScanArgs a) {
                           __builtin_amdgcn_readfirstlane(__float_as_int(ends[buf][2]));
     if (by_token) break;
     if (c + 1 < nch) {
-      fetch(c + 1);
-      if (w == 4) {
+      if (w == 4) {  // (before the rows: what it waits for, spills among it, does not wait for them)
         scalars(c + 1);
         if (c + 2 < nch) fetch_dt(c + 2);
       }
+      fetch(c + 1);
     }
     if (OUT) {
       const int t = 16 * tb + ql;
@@ -587,7 +598,12 @@ linear_scan_kernel(const ScanArgs a) {
         for (int b = 0; b < 2; ++b) {
           const int c0 = 16 * (2 * vh + b) + 4 * quad;
           float* op = a.out + (size_t)(t0 + t) * ((size_t)a.H * a.vd) + h * a.vd + tile * LVT + c0;
-          if (SSM) o[b] += a.skip[h] * widen(raw4<FULL>(xv + (size_t)(t0 + t) * a.ld, c0, vn));
+          if (SSM) {  // (x as it lies in LDS where its one part is all of it: from memory it came behind the next chunk's rows, and
+                      // every wave waited for it and for them: state space, 56 heads, 3 portions of 4096 tokens 105 us -> 95)
+            if constexpr (AP == 1)
+              o[b] += skip * widen(*reinterpret_cast<const bf16x4_t*>(Vs + (2 * tb + vh) * 512 + place(quad, ql, vh) * 8 + 4 * b));
+            else o[b] += skip * widen(raw4<FULL>(xv + (size_t)(t0 + t) * a.ld, c0, vn));
+          }
           if (FULL) *reinterpret_cast<f32x4_t*>(op) = o[b];
           else
 #pragma unroll
