@@ -353,11 +353,17 @@ def wide_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
     rows: where they fill 0.65 of their rounds of CUs.  Tiles of 256 rows, 228 points of 19 widths and depths (1536 - 28672 x 1536 -
     13824) at 400 - 8192 rows, one product after another of different weights: library over owned 1.08 in the geometric mean above
     the line (102 points, 0.95 - 1.61: 18944 x 3584 at 2405 rows 360 / 232 us, 4000 500 / 385), 0.98 at 0.6 - 0.65 in one round, 0.84
-    and less below a half.  Where those of 192 take their place, 208 points of nine widths: 1.06 (0.87 - 1.74: 18944 x 3584 900 rows
-    135 / 126, 8192 x 1536 2609 83 / 64; 14336 x 7168 621 114 / 132); 59 of tiles of 128 rows 0.98, which stay the library's."""
+    and less below a half.  Those of 192 rows where only they fill that much,
+    in up to two rounds: from a depth of 2048 on 1.09 in the geometric mean of 19 points of six widths (0.99 - 1.34: 18944 x 3584 900 rows
+    134 / 124 us, 7168 x 2048 3000 91 / 77), shallower ones where they fill 0.83 (8192 x 1536 2609 rows 80 / 63; 1187, filling 0.77,
+    33.6 / 33.2, 10752 x 1536 1900 0.81 61 / 65); three rounds stay (18944 x 3584 1641 205 / 195)."""
     if M < PREFILL_MIN_M or K < 1152 or K % 64 or max(M, N) * K >= 1 << 30 or (N, K, 0) in _prefill_table():
         return None
-    return (1, 0) if chain_tiles(M, N, K)[0] != 128 and chain_fill(M, N, K) >= 0.65 else None
+    if chain_fill(M, N, K, 256) >= 0.65:
+        return (1, 0)
+    rounds = -(-(-(-M // 192) * -(-N // 256)) // _num_cus())
+    takes = chain_tiles(M, N, K)[0] == 192 and rounds <= 2 and chain_fill(M, N, K) >= (0.65 if K >= 2048 else 0.83)
+    return (1, 0) if takes else None
 
 
 def set_mfma(mf: int) -> int:
