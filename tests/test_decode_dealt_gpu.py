@@ -46,6 +46,25 @@ def test_dealt_gated(dev, extra, M):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [17, 32])
+@pytest.mark.parametrize("K", [512, 1280])
+@pytest.mark.parametrize("share", [0.01, 0.625])
+def test_dealt_one_idle(dev, share, K, M):
+    """4 - 5 units of 32 rows to 5 waves: the wave without one goes along with its neighbour, and stores nothing."""
+    ncu = _num_cus()
+    N = 64 * int((2 + share / 2) * ncu)
+    assert dec_plan(M, N, K, True) == (2, 5, 2, 1, ncu)
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    x = torch.randn(M, K, generator=g, device=dev).bfloat16()
+    wg, wu = ((torch.randn(N // 2, K, generator=g, device=dev) * K ** -0.5).bfloat16() for _ in range(2))
+    a, b = x.double() @ wg.double().T, x.double() @ wu.double().T
+    want = a * torch.sigmoid(a) * b
+    got = gemm_decode(x, interleave_gate_up(wg, wu), epi=EPI_SILU).double()
+    # bf16's rounding of the result; fp32 sums and exponentials of numbers of about 1
+    assert ((got - want).abs() <= 2 ** -8 * want.abs() + 2e-5 * (1 + b.abs())).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 128])
 @pytest.mark.parametrize("width", [1.0625, 2.25, 2.5])
 @pytest.mark.parametrize("kind", ["plain", "silu", "glu"])
