@@ -32,7 +32,7 @@
 //     M > 128: 1184 units = 148 full 8-wave tiles, 58 % of the CUs; dealt as 4-5
 //     units to each of 256 five-wave workgroups every CU streams its share).
 //     A wave without a unit asks for one line again and again, so that every
-//     wave counts the same loads, and stores nothing (while it repeated its neighbour's
+//     wave counts the same loads, and stores nothing; one case: `reads` (while it repeated its neighbour's
 //     rows, each of them a miss of its own, a workgroup of 2 - 3 units in 5 waves fetched
 //     twice what it used: 17920 x 1536, one row 20.1 -> 16.5 us, 18944 x 3584 in 4 waves
 //     36.5 -> 30.8, 64 rows 39.2 -> 36.2).  ksplit > 1 writes fp32 partial planes ws[split][M][N];
