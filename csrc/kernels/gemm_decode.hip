@@ -121,7 +121,8 @@ struct DArgs {
   // quotients as products, as a workgroup's first loads wait for them (five divisions, two of them of 64 bits, cost 0.1 - 0.2 us a
   // launch: a decode step of 17 such launches at 64 rows 709.4 -> 706.3 us): inv_k, inv_m = ceil(2^32 / ksplit, msplit), exact below 2^32 / divisor; unit run g starts at
   // floor(g units / gs) = g unit_lo + floor(g (units mod gs) / gs), the last quotient by unit_frac = ceil(2^32 (units mod gs) / gs),
-  // exact below 65536 workgroups
+  // exact below 65536 workgroups; with more a run may start one unit from there, and still none has more than ceil(units / gs) of
+  // them: from run to run that quotient rises by 0 or 1, and it ends at units mod gs
   unsigned inv_k, inv_m, unit_frac;
   int unit_lo;
   int msplit;                       // row blocks of 16*MT (adjacent on one XCD: the W lines are shared in L2)
@@ -635,7 +636,7 @@ void gemm_dec_kernel(DArgs p) {
 // the derived quotients of units, gs, ksplit, msplit; false for a grid that they are not exact for
 bool set_deal(DArgs& a) {
   const unsigned long long grid = (unsigned long long)a.gs * a.ksplit * a.msplit;
-  if ((a.units % a.gs != 0 && a.gs >= 65536) || (a.ksplit > a.msplit ? a.ksplit : a.msplit) * grid >= 1ull << 32) return false;
+  if ((a.ksplit > a.msplit ? a.ksplit : a.msplit) * grid >= 1ull << 32) return false;
   a.inv_k = (unsigned)(((1ull << 32) + a.ksplit - 1) / a.ksplit);
   a.inv_m = (unsigned)(((1ull << 32) + a.msplit - 1) / a.msplit);
   a.unit_lo = a.units / a.gs;

@@ -134,3 +134,17 @@ def test_rules(monkeypatch):
     assert L.kernel_for(1, 18944, 3584) == "decode" and L.kernel_for(1, 18944, 3584, wide_ok=False) != "decode"
     for p, N in ((dec_plan(64, 17920, 1536, True), 17920), (dec_own_plan(64, 8192, 1536), 8192), (dec_plan(1, 18944, 3584), 18944)):
         assert -(-(N // 16) // p[4]) <= p[1]  # what the launcher takes
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [32 * 327691, 32 * 262149])
+def test_dealt_many(dev, N):
+    """More than 65536 workgroups that the units do not divide into: 65539 of 4 - 5 units, 65538 of 3 - 4."""
+    K, gs = 64, 65539 if N == 32 * 327691 else 65538
+    g = torch.Generator(device=dev).manual_seed(gs)
+    x = torch.randn(2, K, generator=g, device=dev).bfloat16()
+    w = torch.randn(N, K, generator=g, device=dev, dtype=torch.bfloat16)
+    got = gemm_decode(x, w, plan=(1, 5, 2, 1, gs)).float()
+    want = x.float() @ w.float().T
+    # bf16's rounding of the result, and fp32 sums of 64 products of about 1 in another order
+    assert ((got - want).abs() <= 2 ** -8 * want.abs() + 64 * 2 ** -23 * 16).all()
