@@ -798,14 +798,15 @@ def gemm_decode(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None,
                 out: torch.Tensor | None = None, packed: "DecPacked | None" = None) -> torch.Tensor:
     """Decode-regime GEMM: y = act(x @ w.T + b) (epi EPI_STORE) or the SwiGLU product of an interleaved
     gate/up weight (epi EPI_SILU, out [M, N/2]).  ``plan`` = (mt, nwv, ntw, ksplit[, gs]) overrides dec_plan
-    (gs: workgroups per K-range over the N / (16 ntw) wave units; 0 = the plain N / (16 ntw nwv) tiling)."""
+    (gs: workgroups per K-range over the N / (16 ntw) wave units; 0 = the plain N / (16 ntw nwv) tiling).  Packed weights take
+    the plan in units of 32 rows."""
     M, K = x.shape
     N = w.shape[0]
     if not x.is_cuda:
         return gemm_silu(x, w, b) if epi == EPI_SILU else gemm(x, w, b, act)
     if plan is None:
-        plan = dec_own_plan(M, N, K, epi == EPI_SILU) if packed is None else dec_coarse(dec_plan(M, N, K, epi == EPI_SILU))
-    mt, nwv, ntw, ks, *rest = plan
+        plan = dec_own_plan(M, N, K, epi == EPI_SILU) if packed is None else dec_plan(M, N, K, epi == EPI_SILU)
+    mt, nwv, ntw, ks, *rest = plan if packed is None else dec_coarse(plan)
     gs = rest[0] if rest else 0
     tail = rest[1] if len(rest) > 1 else 0
     ks = dec_ksplit(K, ks)

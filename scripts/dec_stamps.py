@@ -28,7 +28,7 @@ dev = torch.device("cuda")
 x = torch.randn(a.M, K, device=dev, dtype=torch.bfloat16)
 ncopy = max(2, min(8, (700 << 20) // (N * K * 2) + 1))
 ws = [torch.randn(N, K, device=dev, dtype=torch.bfloat16) * 0.02 for _ in range(ncopy)]
-plan = G.dec_plan(a.M, N, K, silu) if a.plan == "auto" else tuple(int(v) for v in a.plan.split(":"))
+plan = (G.dec_plan if a.packed else G.dec_own_plan)(a.M, N, K, silu) if a.plan == "auto" else tuple(int(v) for v in a.plan.split(":"))
 pk = [G.DecPacked(w, silu) for w in ws] if a.packed else [None] * ncopy
 G.WS.reserve(dev, G.dec_ws_floats(a.M, N, G.dec_ksplit(K, plan[3])))
 epi = G.EPI_SILU if silu else G.EPI_STORE

@@ -64,7 +64,7 @@ def main():
                          "natural [N, K] layout, same plan (dec_plan, or --plan)")
     ap.add_argument("--tail", type=int, default=0, help="1: also the 8-wave tail-split decode schedules")
     ap.add_argument("--depths", default="", help="ring depths to A/B on the dispatched decode plan (e.g. 6,8)")
-    ap.add_argument("--plan", default="", help="mt,nwv,ntw,ksplit[,gs] for the packed A/B (default dec_plan)")
+    ap.add_argument("--plan", default="", help="mt,nwv,ntw,ksplit[,gs] for the packed A/B (default: the product's own)")
     ap.add_argument("--hot", type=int, default=0, help="1: also every arm on one weight copy (cache-hot)")
     ap.add_argument("--tile", default="", help="stream-K grids of the 256x256 tile kernel to A/B (e.g. 256:192; "
                                                "k2 = 2-way split-K with the reduce)")
@@ -86,9 +86,10 @@ def main():
                 else:
                     arms["linear"] = lambda w: linear(x, w)
                     arms["deferred"] = lambda w: linear_deferred(x, w)
-                plan = tuple(int(v) for v in a.plan.replace(":", ",").split(",")) if a.plan else G.dec_plan(M, N, K, silu)
+                plan = tuple(int(v) for v in a.plan.replace(":", ",").split(",")) if a.plan else G.dec_own_plan(M, N, K, silu)
                 if a.packed and plan is not None:
                     pks = [G.DecPacked(w, silu) for w in ws]
+                    plan = plan if a.plan else G.dec_coarse(G.dec_plan(M, N, K, silu))  # one plan that both layouts have
                     G.WS.reserve(dev, G.dec_ws_floats(M, N, G.dec_ksplit(K, plan[3])))
                     epi = G.EPI_SILU if silu else G.EPI_STORE
                     arms["dec_natural"] = lambda w, plan=plan, epi=epi: G.gemm_decode(x, w, epi=epi, plan=plan)
@@ -115,7 +116,7 @@ def main():
                             arms[f"dec_deferred_ks{kk}"] = lambda w, pl=pl, kk=kk: G.gemm_deferred(
                                 x, w, ("decode", kk, pl))
                 for d in [int(v) for v in a.depths.replace(":", ",").split(",") if v.strip()]:
-                    if plan is None or plan[1] not in (4, 5) or plan[0] > (2 if d == 12 else 4 if d == 8 else 8) \
+                    if plan is None or plan[1] not in (4, 5) or plan[2] != 2 or plan[0] > (2 if d == 12 else 4 if d == 8 else 8) \
                             or (plan[0] <= 2 and d == 6):
                         continue
                     epi = G.EPI_SILU if silu else G.EPI_STORE

@@ -148,3 +148,22 @@ def test_dealt_many(dev, N):
     want = x.float() @ w.float().T
     # bf16's rounding of the result, and fp32 sums of 64 products of about 1 in another order
     assert ((got - want).abs() <= 2 ** -8 * want.abs() + 64 * 2 ** -23 * 16).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 64, 128])
+@pytest.mark.parametrize("silu", [False, True])
+def test_packed_takes_the_plan(dev, silu, M):
+    """Packed weights with the product's own plan, also one in units of 16 rows, which only natural weights have."""
+    ncu, K = _num_cus(), 512
+    N = 64 * (9 * ncu // 8)  # 2.25 units of 32 a CU
+    plan = dec_plan(M, N, K, silu)
+    assert plan[2:] == (1, 1, ncu)
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=dev).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).bfloat16()
+    epi = EPI_SILU if silu else G.EPI_STORE
+    packed = G.DecPacked(w, silu)
+    want = gemm_decode(x, w, epi=epi, plan=G.dec_coarse(plan))  # the same sums in the same order
+    assert torch.equal(gemm_decode(x, w, epi=epi, plan=plan, packed=packed), want)
+    assert torch.equal(gemm_decode(x, w, epi=epi, packed=packed), want)
