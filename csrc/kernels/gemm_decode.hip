@@ -32,7 +32,7 @@
 //     M > 128: 1184 units = 148 full 8-wave tiles, 58 % of the CUs; dealt as 4-5
 //     units to each of 256 five-wave workgroups every CU streams its share).
 //     A wave without a unit asks for one line again and again, so that every
-//     wave counts the same loads, and stores nothing; one case: `reads` (while it repeated its neighbour's
+//     wave counts the same loads, and stores nothing (while it repeated its neighbour's
 //     rows, each of them a miss of its own, a workgroup of 2 - 3 units in 5 waves fetched
 //     twice what it used: 17920 x 1536, one row 20.1 -> 16.5 us, 18944 x 3584 in 4 waves
 //     36.5 -> 30.8, 64 rows 39.2 -> 36.2).  ksplit > 1 writes fp32 partial planes ws[split][M][N];
@@ -234,19 +234,17 @@ void gemm_dec_kernel(DArgs p) {
   // of one K-step are one contiguous block (row stride 64), the unit's K-steps follow each other, so a
   // wave streams one contiguous region (DRAM pages are read whole, not 128 B per row per K-step)
   const int kstride = p.packed ? 16 * NTW * 64 : 64;
-  // A wave without a unit stays at the first line of the last one.  At 17 - 32 rows of an interleaved gated unit's units of 32 the only
-  // such wave of a workgroup goes along with its neighbour instead (37888 x 3584 in 4 - 5 units; a step of
-  // 18 / 26 / 32 rows 534.0 / 585.7 / 590.1 -> 531.1 / 582.6 / 587.4 us); the line is the faster
-  // in units of 16 and for the products that are not gated (a step of 20 rows of a 1b decoder 499.4 against 501.0 us).
-  const bool reads = active || (EPI == EPI_SILU && MT == 2 && NTW == 2 && TQ == 0 && cnt == NWV - 1);
-  const int kstep = reads ? kstride : 0;
+  // A wave without a unit stays at the first line of the last one.  (A gated unit at 17 - 32 rows, where such a wave goes along with its
+  // neighbour / stays, us: 27648 x 5120 63.1 / 58.7, 26624 x 3072 38.2 / 35.8, 36864 x 4096 70.0 / 69.5, 33792 x 2048 37.0 / 37.4, 37888 x
+  // 3584 52.0 / 52.7.)
+  const int kstep = active ? kstride : 0;
   const bf16* wp[NTW];
 #pragma unroll
   for (int nt = 0; nt < NTW; ++nt) {
-    const int r = reads ? 16 * nt + li : 0, c = reads ? 8 * h4 : 0;
+    const int r = active ? 16 * nt + li : 0, c = active ? 8 * h4 : 0;
     const int row = wr[nt] + (NTW == 1 && GATED ? (li & 7) + (li >= 8 ? up : 0) : li);
     wp[nt] = p.packed ? p.W + (size_t)q * ks * kstride + (size_t)kb * kstride + r * 64 + c
-                      : p.W + (size_t)min(reads ? row : wr[0], p.N - 1) * p.ldw + (size_t)kb * 64 + c;
+                      : p.W + (size_t)min(active ? row : wr[0], p.N - 1) * p.ldw + (size_t)kb * 64 + c;
   }
 
   // A pieces: piece q = w*GA + i covers rows [8q, 8q+8); lane -> row 8q + L/8, physical chunk L%8

@@ -50,7 +50,7 @@ def test_dealt_gated(dev, extra, M):
 @pytest.mark.parametrize("K", [512, 1280])
 @pytest.mark.parametrize("share", [0.01, 0.625])
 def test_dealt_one_idle(dev, share, K, M):
-    """4 - 5 units of 32 rows to 5 waves: the wave without one goes along with its neighbour, and stores nothing."""
+    """4 - 5 units of 32 rows to 5 waves: the wave without one stores nothing."""
     ncu = _num_cus()
     N = 64 * int((2 + share / 2) * ncu)
     assert dec_plan(M, N, K, True) == (2, 5, 2, 1, ncu)
