@@ -914,6 +914,7 @@ int launch(const Args& a, hipStream_t stream) {
 // The rows of whole tiles that grag_gemm_tile takes for a product (256, 192, 128) on a chip of ncu CUs, and its estimate for `rows`
 // in ns (ops/gemm.py asks both).
 GRAG_API int grag_gemm_chain_rows(int M, int N, int K, int ncu) { return chain_rows(M, N, K, ncu); }
+GRAG_API int grag_gemm_chain_bias() { return kChainBias; }  // columns of a bias at most
 GRAG_API int grag_gemm_chain_ns(int M, int N, int K, int rows, int ncu) {
   return (int)fmin(1000. * chain_us(M, N, K, rows, ncu), 2e9);
 }

@@ -196,7 +196,8 @@ class BertEncoder:
             a = varlen_attention(qkv, seq_start, seq_len, max_len, nh, cfg.head_dim, self.scale, causal=False)
             h = layernorm(linear(a, L.o_w), L.ln1_g, L.ln1_b, eps, bias=L.o_b, residual=h)
             if _tile.supported(h, L.f1_w) and _tile.capture_ok(
-                    h.device, h.shape[0], L.f1_w.shape[0], H, act=_tile.ACT_GELU, pair=_tile.pair_takes(h, L.f1_w, L.f1_b)):
+                    h.device, h.shape[0], L.f1_w.shape[0], H, act=_tile.ACT_GELU, pair=_tile.pair_takes(h, L.f1_w, L.f1_b),
+                    chain=_tile.chain_takes(h, L.f1_w, L.f1_b)):
                 f = _tile.gemm(h, L.f1_w, L.f1_b, act=_tile.ACT_GELU)  # bias + GELU in the GEMM epilogue
             else:
                 f = bias_act(linear(h, L.f1_w), L.f1_b, ACT_GELU, inplace=True)

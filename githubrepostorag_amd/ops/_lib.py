@@ -72,6 +72,7 @@ _SIGS = {
     "grag_gemm_pair": [P, P, P, P, I, I, I, I, I, I, I, I, I, F, F, F, P],
     "grag_gemm_chain_rows": [I, I, I, I],
     "grag_gemm_chain_ns": [I, I, I, I, I],
+    "grag_gemm_chain_bias": [],
     "grag_gemm_tile": [P, P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, P],
     "grag_splitk_reduce": [P, P, P, I, I, I, I, I, I, P],
     "grag_gemm_tile_mfma": [I],

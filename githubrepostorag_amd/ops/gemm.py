@@ -189,7 +189,21 @@ def chain_fill(M: int, N: int, K: int, rows: int | None = None) -> float:
     return M * N / (256 * rows * ncu * -(-(-(-M // rows) * -(-N // 256)) // ncu))
 
 
-def prefill_plan(M: int, N: int, K: int, silu: bool = False) -> tuple[int, int] | None:
+def chain_fits(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> bool:
+    """Whether whole tiles of a product of these sizes go in chains (csrc/kernels/gemm_tile.hip chain_ok), which alone have tiles of 192
+    and 128 rows.  Asks for sizes and strides only, which any tensor has."""
+    N = w.shape[0]
+    return (x.shape[0] * x.stride(0) < 1 << 30 and N * w.stride(0) < 1 << 30 and N < 1 << 20
+            and (b is None or N <= lib().grag_gemm_chain_bias()))
+
+
+def chain_takes(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None, out: torch.Tensor | None = None) -> bool:
+    """chain_fits(), and addresses that the chain's wide accesses take."""
+    return (chain_fits(x, w, b) and (b is None or b.data_ptr() % 16 == 0)
+            and (out is None or out.data_ptr() % 16 == 0 and out.stride(0) < 1 << 20))
+
+
+def prefill_plan(M: int, N: int, K: int, silu: bool = False, chain: bool = True) -> tuple[int, int] | None:
     """(ksplit, sk) of the owned kernel for a prefill-sized GEMM, or None for the library.
 
     From the dense M sweep of scripts/sweep_prefill_gemm.py (tuning/gemm_prefill_gfx950.json; library
@@ -201,16 +215,20 @@ def prefill_plan(M: int, N: int, K: int, silu: bool = False) -> tuple[int, int] 
     SiLU*mul pass: owned won all 63 buckets on Qwen2-7B / 1.5B).  Of the two buckets around M, the one on M's
     own row-tile grid is preferred (its schedule was measured on the identical tile count), and a tail-only
     stream-K grid is re-derived for M's own remainder (``_tail_grid``).  Unmeasured shapes: None (library)
-    for plain GEMMs, ``plan`` for SwiGLU."""
+    for plain GEMMs, ``plan`` for SwiGLU.  ``chain``: the operands meet chain_takes().
+
+    The sweep's whole tiles had 256 rows.  Where those of 192 or 128 rows are clearly shorter, a streamed tail gives way to them: 16 such
+    products of K up to 4096 0.99 - 1.27 of the streamed time, median 1.1 (37888 x 3584 300 rows 126 -> 112 us, 2048 x 1536 8320 64 ->
+    55); not at K 9472 and 18944 (0.82 - 0.94), where a part of a tile is longer beside its fixup."""
     row = _prefill_row(M, N, K, silu)
     if row is None:
         return plan(M, N, K) if silu else None
     ks, sk = row[3], row[4]
     if ks == 1 and sk < 0:
         sk = _tail_grid(row[0], M, N, sk)
-    if ks == 1 and sk and K <= 4096:  # swept when whole tiles had 256 rows: 16 such rows 0.99 - 1.27 of the streamed time, median
-        _, us, ratio = chain_tiles(M, N, K)  # 1.1 (37888 x 3584 300 rows 126 -> 112 us, 2048 x 1536 8320 64 -> 55); 0.82 - 0.94 of it at K
-        if ratio < 0.9 and us < 0.95 * row[2]:  # 9472 and 18944, where a part of a tile is longer beside its fixup
+    if ks == 1 and sk and K <= 4096 and chain:
+        _, us, ratio = chain_tiles(M, N, K)
+        if ratio < 0.9 and us < 0.95 * row[2]:
             return 1, 0
     return (ks, sk) if sk_ok(M, N, K, ks, sk) else (1, 0)
 
@@ -273,10 +291,10 @@ def unmeasured_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
     return unmeasured_schedule(M, N, K)
 
 
-def schedule(M: int, N: int, K: int, silu: bool = False) -> tuple[int, int]:
-    """(ksplit, sk) the owned kernel runs a shape with when the caller does not pin one."""
+def schedule(M: int, N: int, K: int, silu: bool = False, chain: bool = True) -> tuple[int, int]:
+    """(ksplit, sk) the owned kernel runs a shape with when the caller does not pin one.  ``chain``: as prefill_plan's."""
     if M >= PREFILL_MIN_M:
-        p = prefill_plan(M, N, K, silu) or (None if silu else unmeasured_schedule(M, N, K))
+        p = prefill_plan(M, N, K, silu, chain) or (None if silu else unmeasured_schedule(M, N, K))
         if p is not None:
             return p
     return plan(M, N, K)
@@ -353,7 +371,7 @@ def gemm_pair(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, shape: i
 
 
 @functools.lru_cache(4096)
-def wide_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
+def wide_plan(M: int, N: int, K: int, chain: bool = True) -> tuple[int, int] | None:
     """(1, 0) where a plain product of K >= 1152 outside the measured table goes to the owned kernel in whole tiles of 256 or 192
     rows: where they fill 0.65 of their rounds of CUs.  Tiles of 256 rows, 228 points of 19 widths and depths (1536 - 28672 x 1536 -
     13824) at 400 - 8192 rows, one product after another of different weights: library over owned 1.08 in the geometric mean above
@@ -361,11 +379,14 @@ def wide_plan(M: int, N: int, K: int) -> tuple[int, int] | None:
     and less below a half.  Those of 192 rows where only they fill that much,
     in up to two rounds: from a depth of 2048 on 1.09 in the geometric mean of 19 points of six widths (0.99 - 1.34: 18944 x 3584 900 rows
     134 / 124 us, 7168 x 2048 3000 91 / 77), shallower ones where they fill 0.83 (8192 x 1536 2609 rows 80 / 63; 1187, filling 0.77,
-    33.6 / 33.2, 10752 x 1536 1900 0.81 61 / 65); three rounds stay (18944 x 3584 1641 205 / 195)."""
+    33.6 / 33.2, 10752 x 1536 1900 0.81 61 / 65); three rounds stay (18944 x 3584 1641 205 / 195).  ``chain``: the operands meet
+    chain_takes(), without which there are no tiles of 192 rows."""
     if M < PREFILL_MIN_M or K < 1152 or K % 64 or max(M, N) * K >= 1 << 30 or (N, K, 0) in _prefill_table():
         return None
     if chain_fill(M, N, K, 256) >= 0.65:
         return (1, 0)
+    if not chain:
+        return None
     rounds = -(-(-(-M // 192) * -(-N // 256)) // _num_cus())
     takes = chain_tiles(M, N, K)[0] == 192 and rounds <= 2 and chain_fill(M, N, K) >= (0.65 if K >= 2048 else 0.83)
     return (1, 0) if takes else None
@@ -561,7 +582,7 @@ def gemm(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None, act: i
         shape = pair_plan(M, N, K, act != ACT_NONE)
         if shape is not None and pair_takes(x, w, b, out):
             return gemm_pair(x, w, b, shape, EPI_STORE, act, out)
-        ksplit, sk = schedule(M, N, K)
+        ksplit, sk = schedule(M, N, K, chain=chain_takes(x, w, b, out))
         if (ksplit, sk) == (1, 0) and pair_fills(M, N, K) and pair_takes(x, w, b, out):
             return gemm_pair(x, w, b, 0, EPI_STORE, act, out)
     sk = sk or 0
@@ -587,7 +608,7 @@ def gemm_silu(x: torch.Tensor, w_gu: torch.Tensor, b_gu: torch.Tensor | None = N
         shape = pair_plan(M, N2, K, True)
         if shape is not None and pair_takes(x, w_gu, b_gu, out):
             return gemm_pair(x, w_gu, b_gu, shape, EPI_SILU, ACT_NONE, out)
-        ksplit, sk = schedule(M, N2, K, True)
+        ksplit, sk = schedule(M, N2, K, True, chain_takes(x, w_gu, b_gu, out))
     sk = sk or 0
     if out is None:
         out = torch.empty(M, N2 // 2, dtype=x.dtype, device=x.device)
@@ -1054,12 +1075,13 @@ def dec_capture_ok(dev: torch.device, M: int, N: int, K: int, silu: bool = False
     return fl == 0 or not torch.cuda.is_current_stream_capturing() or WS.ready(dev, fl)
 
 
-def capture_ok(dev: torch.device, M: int, N: int, K: int, silu: bool = False, act: int = ACT_NONE, pair: bool = True) -> bool:
+def capture_ok(dev: torch.device, M: int, N: int, K: int, silu: bool = False, act: int = ACT_NONE, pair: bool = True,
+               chain: bool = True) -> bool:
     """False only inside a hipGraph capture whose split-K slab was not sized by an eager step.  ``pair``: the operands meet
-    pair_takes(), without which a small product has schedule()'s slab."""
+    pair_takes(), without which a small product has schedule()'s slab; ``chain``: chain_takes(), without which a streamed tail has."""
     if pair and pair_plan(M, N, K, silu or act != ACT_NONE) is not None:  # (no slab)
         return True
-    ks, sk = schedule(M, N, K, silu)
+    ks, sk = schedule(M, N, K, silu, chain)
     fl = _ws_floats(M, N, ks, sk)
     return fl == 0 or not torch.cuda.is_current_stream_capturing() or (WS.ready(dev, fl) and (
         not sk or WS.has_counters(dev)))
@@ -1073,7 +1095,8 @@ def mlp_gate_up(x: torch.Tensor, w_gu: torch.Tensor, b_gu: torch.Tensor | None =
             and dec_capture_ok(x.device, M, w_gu.shape[0], K, True):
         return gemm_decode(x, w_gu, b_gu, epi=EPI_SILU)
     if not x.is_cuda or (supported(x, w_gu)
-                         and capture_ok(x.device, M, w_gu.shape[0], K, True, pair=pair_takes(x, w_gu, b_gu))):
+                         and capture_ok(x.device, M, w_gu.shape[0], K, True, pair=pair_takes(x, w_gu, b_gu),
+                                        chain=chain_takes(x, w_gu, b_gu))):
         return gemm_silu(x, w_gu, b_gu)
     y = torch.nn.functional.linear(x, w_gu, b_gu).view(M, -1, 2, 32)
     return (torch.nn.functional.silu(y[:, :, 0].float()) * y[:, :, 1].float()).to(x.dtype).reshape(M, -1)

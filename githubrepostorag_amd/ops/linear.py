@@ -285,13 +285,14 @@ def gemm_splitk(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None,
 
 
 def kernel_for(M: int, N: int, K: int, tile_ok: bool = True, dev: torch.device | None = None, pair_ok: bool = True,
-               wide_ok: bool = True) -> str:
+               wide_ok: bool = True, chain_ok: bool = True) -> str:
     """The kernel linear() runs a bf16 [M, K] x [N, K]^T projection on: "pair" / "decode" / "tile" / "tile_prefill"
     (owned MFMA kernels of ops/gemm.py), "skinny" / "stream" (owned weight-streaming kernels here),
     "splitk" (K-sliced library bmm) or "library" (hipBLASLt).  ``tile_ok``: the operands meet
     ops/gemm.supported (alignment, K % 64).  ``dev``: check that a hipGraph capture in progress can use
     the split-K / stream-K workspaces (None: plan as in steady state, workspaces ready).  ``pair_ok``: they meet
-    ops/gemm.pair_takes.  ``wide_ok``: the product is a plain one, which dec_wide() takes from the library."""
+    ops/gemm.pair_takes.  ``wide_ok``: the product is a plain one, which dec_wide() takes from the library.  ``chain_ok``: the operands
+    meet ops/gemm.chain_fits."""
     capturing = dev is not None and torch.cuda.is_current_stream_capturing()
     if tile_ok:
         if pair_ok and _tile.pair_plan(M, N, K) is not None:
@@ -302,7 +303,7 @@ def kernel_for(M: int, N: int, K: int, tile_ok: bool = True, dev: torch.device |
         if use_tile(M, N, K) and (dev is None or _tile.capture_ok(dev, M, N, K, pair=pair_ok)):
             return "tile"
         if M >= _tile.PREFILL_MIN_M and _tile.prefill_plan(M, N, K) is not None and (
-                dev is None or _tile.capture_ok(dev, M, N, K, pair=pair_ok)):
+                dev is None or _tile.capture_ok(dev, M, N, K, pair=pair_ok, chain=chain_ok)):
             return "tile_prefill"
     if splitk_parts(M, N, K):
         return "splitk"
@@ -318,8 +319,8 @@ def kernel_for(M: int, N: int, K: int, tile_ok: bool = True, dev: torch.device |
         return "skinny"
     if K % 16 == 0 and N % 4 == 0 and use_stream(M, N, K) and stream_ready:
         return "stream"
-    if tile_ok and (_tile.wide_plan(M, N, K) is not None or _tile.unmeasured_plan(M, N, K) is not None and (
-            dev is None or _tile.capture_ok(dev, M, N, K, pair=pair_ok))):
+    if tile_ok and (_tile.wide_plan(M, N, K, chain_ok) is not None or _tile.unmeasured_plan(M, N, K) is not None and (
+            dev is None or _tile.capture_ok(dev, M, N, K, pair=pair_ok, chain=chain_ok))):
         return "tile_prefill"
     return "library"
 
@@ -362,13 +363,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> t
             and x.stride(1) == 1 and w.stride(1) == 1):
         M, K = x.shape
         N = w.shape[0]
-        kind = kernel_for(M, N, K, _tile.supported(x, w), x.device)
+        chain = M < _tile.PREFILL_MIN_M or _tile.chain_fits(x, w, b)
+        kind = kernel_for(M, N, K, _tile.supported(x, w), x.device, chain_ok=chain)
         if kind == "pair":
             if not _plain_product(x, w, b, align=2):
                 return torch.nn.functional.linear(x, w, b)
             if _tile.pair_takes(x, w, b):
                 return _tile.gemm_pair(x, w, b, _tile.pair_plan(M, N, K))
-            kind = kernel_for(M, N, K, True, x.device, pair_ok=False)
+            kind = kernel_for(M, N, K, True, x.device, pair_ok=False, chain_ok=chain)
         if kind == "decode" and M < TILE_MIN_M and not _tile.dec_small(M, N, K) and not _plain_product(x, w, b, align=2):
             kind = kernel_for(M, N, K, True, x.device, wide_ok=False)
         if kind == "decode":
@@ -376,13 +378,17 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> t
         if kind == "tile":
             return _tile.gemm(x, w, b)
         if kind == "tile_prefill":
-            p = _tile.prefill_plan(M, N, K)
+            p = _tile.prefill_plan(M, N, K, chain=chain)
             if p is not None:
                 if _tile.stays_owned(M, N, K) and not _plain_product(x, w, b, align=2):
                     return torch.nn.functional.linear(x, w, b)
+                if chain and not _tile.chain_takes(x, w, b):  # (a bias at an odd address)
+                    p = _tile.prefill_plan(M, N, K, chain=False)
+                    if not _tile.capture_ok(x.device, M, N, K, pair=False, chain=False):
+                        return torch.nn.functional.linear(x, w, b)
                 return _tile.gemm(x, w, b, ksplit=p[0], sk=p[1])
             if _plain_product(x, w, b):
-                p = _tile.wide_plan(M, N, K) or _tile.unmeasured_plan(M, N, K)
+                p = _tile.wide_plan(M, N, K, chain) or _tile.unmeasured_plan(M, N, K)
                 if p == (1, 0) and _tile.pair_fills(M, N, K) and _tile.pair_takes(x, w, b):
                     return _tile.gemm_pair(x, w, b, 0)
                 return _tile.gemm(x, w, b, ksplit=p[0], sk=p[1])
@@ -406,17 +412,19 @@ def bound_product(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, act:
     def ordinary(x, w, b):
         if not act:
             return linear(x, w, b)
-        if _tile.supported(x, w) and _tile.capture_ok(x.device, M, N, K, act=act, pair=_tile.pair_takes(x, w, b)):
+        if _tile.supported(x, w) and _tile.capture_ok(x.device, M, N, K, act=act, pair=_tile.pair_takes(x, w, b),
+                                                       chain=_tile.chain_takes(x, w, b)):
             return _tile.gemm(x, w, b, act=act)
         return bias_act(linear(x, w), b, act, inplace=True)
 
     name, tail = None, ()
     if x.is_cuda and _tile.supported(x, w) and _plain_product(x, w, b):
         shape = _tile.pair_plan(M, N, K, act != 0)
-        kind = "tile_prefill" if act else kernel_for(M, N, K, True, x.device)
+        chain = _tile.chain_takes(x, w, b)
+        kind = "tile_prefill" if act else kernel_for(M, N, K, True, x.device, chain_ok=chain)
         if shape is None and kind == "tile_prefill":
-            plan = _tile.schedule(M, N, K) if act else _tile.prefill_plan(M, N, K) or _tile.wide_plan(M, N, K) or _tile.unmeasured_plan(
-                M, N, K)
+            plan = _tile.schedule(M, N, K, chain=chain) if act else (
+                _tile.prefill_plan(M, N, K, chain=chain) or _tile.wide_plan(M, N, K, chain) or _tile.unmeasured_plan(M, N, K))
             if plan == (1, 0):
                 measured = not act and _tile.prefill_plan(M, N, K) is not None
                 shape = 0 if not measured and _tile.pair_fills(M, N, K) else None
@@ -488,8 +496,8 @@ def glu_linear(x: torch.Tensor, w: torch.Tensor, limit: float | None, alpha: flo
     if x.is_cuda and x.dim() == 2 and x.shape[0] >= _tile.PREFILL_MIN_M and w.shape[0] % 16 == 0:
         M, N = x.shape[0], w.shape[0]
         K = x.shape[1]
-        rows = _tile.chain_tiles(M, N, K)[0]
-        fills = _tile.chain_fill(M, N, K, 256) >= GLU_FILL[256] or K >= 256 and _tile.chain_fill(M, N, K) >= GLU_FILL[rows]
+        rows = _tile.chain_tiles(M, N, K)[0] if _tile.chain_fits(x, w) else 256
+        fills = _tile.chain_fill(M, N, K, 256) >= GLU_FILL[256] or K >= 256 and _tile.chain_fill(M, N, K, rows) >= GLU_FILL[rows]
         small = x.shape[1] >= 256 and _tile.pair_plan(M, N, x.shape[1], True) is not None  # (shorter contractions: two launches)
         if (fills or small) and _tile.supported(x, w) and _plain_product(x, w):
             return _tile.gemm_glu(x, w, limit, alpha, shift)
