@@ -376,11 +376,14 @@ def wide_plan(M: int, N: int, K: int, chain: bool = True) -> tuple[int, int] | N
     rows: where they fill 0.65 of their rounds of CUs.  Tiles of 256 rows, 228 points of 19 widths and depths (1536 - 28672 x 1536 -
     13824) at 400 - 8192 rows, one product after another of different weights: library over owned 1.08 in the geometric mean above
     the line (102 points, 0.95 - 1.61: 18944 x 3584 at 2405 rows 360 / 232 us, 4000 500 / 385), 0.98 at 0.6 - 0.65 in one round, 0.84
-    and less below a half.  Those of 192 rows where only they fill that much,
-    in up to two rounds: from a depth of 2048 on 1.09 in the geometric mean of 19 points of six widths (0.99 - 1.34: 18944 x 3584 900 rows
-    134 / 124 us, 7168 x 2048 3000 91 / 77), shallower ones where they fill 0.83 (8192 x 1536 2609 rows 80 / 63; 1187, filling 0.77,
-    33.6 / 33.2, 10752 x 1536 1900 0.81 61 / 65); three rounds stay (18944 x 3584 1641 205 / 195).  ``chain``: the operands meet
-    chain_takes(), without which there are no tiles of 192 rows."""
+    and less below a half.
+
+    Those of 192 rows where only they fill that much, 33 widths and depths (3072 - 22016 x 1152 - 8192) at 300 - 8192 rows, the same
+    way.  In two rounds and more 1.09 in the geometric mean of 200 points (two rounds 1.08, 157 points, 17 more than 5 % behind; three
+    1.14, none: 18944 x 3584 900 / 1641 rows 134 / 126, 207 / 192, 8192 x 1536 2405 59.4 / 59.7, 2594 79 / 56).  In one round the two are
+    near each other: K of 2048 and more 1.015 of 76 points (0.88 - 1.22), shallower ones 1.04 of 6 where the tiles fill 0.83 of it and
+    1.00 of 56 below (8192 x 1536 1187 rows 31 / 32), which stay the library's.  ``chain``: the operands meet chain_takes(),
+    without which there are no tiles of 192 rows."""
     if M < PREFILL_MIN_M or K < 1152 or K % 64 or max(M, N) * K >= 1 << 30 or (N, K, 0) in _prefill_table():
         return None
     if chain_fill(M, N, K, 256) >= 0.65:
@@ -388,7 +391,7 @@ def wide_plan(M: int, N: int, K: int, chain: bool = True) -> tuple[int, int] | N
     if not chain:
         return None
     rounds = -(-(-(-M // 192) * -(-N // 256)) // _num_cus())
-    takes = chain_tiles(M, N, K)[0] == 192 and rounds <= 2 and chain_fill(M, N, K) >= (0.65 if K >= 2048 else 0.83)
+    takes = chain_tiles(M, N, K)[0] == 192 and chain_fill(M, N, K) >= (0.83 if rounds == 1 and K < 2048 else 0.65)
     return (1, 0) if takes else None
 
 

@@ -68,10 +68,12 @@ def test_rule(monkeypatch):
     assert [G.pair_plan(M, 3072, 768, True) for M in (1, 300, 1136, 1752, 4200)] == [3, 3, 2, 1, None]
     assert G.pair_plan(300, 3072, 1088) is None and G.pair_plan(300, 22016, 4096, True) is None  # deep
     assert G.pair_fills(24000, 768, 768) and not G.pair_fills(12000, 2304, 768) and not G.pair_fills(21504, 768, 768)
-    # rows, width, depth, library and owned us
-    for M, N, K, lib, own in [(2405, 18944, 3584, 360, 232), (4000, 18944, 3584, 500, 385), (1641, 18944, 3584, 195, 212),
-                              (1187, 8192, 1536, 32, 34), (1641, 8192, 1536, 41, 38), (2405, 8192, 1536, 60, 68)]:
-        assert (G.wide_plan(M, N, K) is not None) == (own < lib), (M, N, K)
+    # rows, width, depth, library and owned us (the latter in tiles of 192 rows at 900, 1187, 1641 x 18944 and 2405 x 8192); runs of one
+    # side differ by 2 %
+    for M, N, K, lib, own in [(2405, 18944, 3584, 365, 237), (4000, 18944, 3584, 502, 387), (1641, 18944, 3584, 207, 192),
+                              (900, 18944, 3584, 134, 126), (1187, 8192, 1536, 30.9, 32.1), (1641, 8192, 1536, 40.1, 40.4),
+                              (2405, 8192, 1536, 59.4, 59.7), (1632, 10752, 1536, 71.1, 61.2), (2594, 12288, 6144, 326, 315)]:
+        assert (G.wide_plan(M, N, K) is not None) == (own < 1.02 * lib), (M, N, K)
     assert G.wide_plan(4000, 3584, 3584) is None  # a measured shape keeps its rows
 
 
