@@ -181,7 +181,7 @@ void gemm_dec_kernel(DArgs p) {
   constexpr int GW = 2 * NTW;                  // W dwordx4 per lane per K-step
   static_assert(NTW == 1 || NTW == 2 || NTW == 4, "NTW");
   constexpr bool GATED = EPI == EPI_SILU || EPI == EPI_GLU;
-  static_assert(!GATED || NTW <= 2 || EPI == EPI_SILU, "gated unit of 64 rows: interleaved weights only");
+  static_assert(EPI != EPI_GLU || (NTW <= 2 && TQ == 0), "gate | up halves: units of 16 or 32 rows, no tail split");
   static_assert(NST * ABYTES <= 160 * 1024, "LDS ring exceeds 160 KB");
   constexpr int LDSB = NRM == 1 ? kNrmLds : NST * ABYTES;
   __shared__ __attribute__((aligned(16))) char smem[LDSB];
@@ -221,7 +221,7 @@ void gemm_dec_kernel(DArgs p) {
   // gate/up units: the SiLU epilogue, or fp32 partials of a weight packed in gate/up units (packed == 2)
   // Units of 8 gate and 8 up rows (NTW = 1): lanes 8 - 15 of a tile's 16 hold the up rows, `up` behind the gate row of lane - 8.
   int up = 0;
-  if (NTW <= 2 && (GATED || p.packed == 2)) {
+  if (NTW <= 2 && (GATED || (NTW == 2 && p.packed == 2))) {
     const int o = 8 * NTW * q;  // first output column
     wr[0] = EPI == EPI_GLU ? o : (o >> 5) * 64 + (o & 31);
     up = EPI == EPI_GLU ? p.N >> 1 : 32;
@@ -654,14 +654,24 @@ int launch_nrm(const DArgs& a, int epi, int nwg, hipStream_t s) {
 template <int MT, int D, int NWV, int NTW, int TQ = 0>
 int launch_v(const DArgs& a, int epi, int act, int nwg, hipStream_t s) {
 #define GO(E, AC) gemm_dec_kernel<E, AC, MT, D, NWV, NTW, TQ><<<nwg, 64 * NWV, 0, s>>>(a)
-  if (epi == EPI_PARTIAL) GO(EPI_PARTIAL, ACT_NONE);
-  else if (epi == EPI_SILU) GO(EPI_SILU, ACT_NONE);
-  else if (epi == EPI_GLU) {
-    if constexpr (TQ == 0) GO(EPI_GLU, ACT_NONE);
-    else return (int)hipErrorInvalidValue;
-  } else if (act == ACT_GELU) GO(EPI_STORE, ACT_GELU);
+  if (epi == EPI_PARTIAL) {  // (units of 16 rows: whole contractions only)
+    if constexpr (NTW == 1) return (int)hipErrorInvalidValue;
+    else GO(EPI_PARTIAL, ACT_NONE);
+  } else if (epi == EPI_SILU) GO(EPI_SILU, ACT_NONE);
+  else if (act == ACT_GELU) GO(EPI_STORE, ACT_GELU);
   else if (act == ACT_GELU_TANH) GO(EPI_STORE, ACT_GELU_TANH);
   else GO(EPI_STORE, ACT_NONE);
+#undef GO
+  return (int)hipGetLastError();
+}
+
+template <int NTW>
+int launch_glu(const DArgs& a, int mt, int nwg, hipStream_t s) {
+#define GO(MT) gemm_dec_kernel<EPI_GLU, ACT_NONE, MT, kDepth, 5, NTW><<<nwg, 320, 0, s>>>(a)
+  if (mt == 1) GO(1);
+  else if (mt == 2) GO(2);
+  else if (mt == 4) GO(4);
+  else GO(8);
 #undef GO
   return (int)hipGetLastError();
 }
@@ -742,7 +752,7 @@ static int launch_variant(const DArgs& a, int e, int act, int mt, int nwv, int n
 // (0: N / (16 ntw nwv), the plain tiling; otherwise ceil(units / gs) <= nwv).  M > 16 mt: the rows go to
 // ceil(M / (16 mt)) workgroups per unit run (at most 4).  packed = 1: W in the unit-packed layout
 // [N / (16 ntw)][K / 64][16 ntw][64] (ops/gemm.py dec_pack), ldw ignored; packed = 2: the same for an
-// interleaved gate/up weight packed in gate/up units (16 gate rows then their 16 up rows; ntw 2).  ntw 1: natural W only.
+// interleaved gate/up weight packed in gate/up units (16 gate rows then their 16 up rows; ntw 2).  ntw 1: natural W and one K-range.
 // Requirements (checked):
 // K % 64 == 0, N % (16 * ntw) == 0 (silu: N % 64 == 0), lda/ldw % 8 == 0,
 // ldc % 4 == 0, 16-B aligned A/W.
@@ -767,6 +777,7 @@ GRAG_API int grag_gemm_decode_t(const void* A, const void* W, const void* bias, 
   // (grag_splitk_add_rmsnorm: split-K reduce + residual add + RMSNorm in one pass)
   const bool keep = epi == EPI_PARTIAL;
   if (epi != EPI_STORE && epi != EPI_SILU && !keep) return (int)hipErrorInvalidValue;
+  if (ntw == 1 && (keep || ksplit > 1)) return (int)hipErrorInvalidValue;
   if (act != ACT_NONE && act != ACT_GELU && act != ACT_GELU_TANH) return (int)hipErrorInvalidValue;
   if ((epi == EPI_SILU || keep) && act != ACT_NONE) return (int)hipErrorInvalidValue;
   if (keep && bias != nullptr) return (int)hipErrorInvalidValue;
@@ -806,13 +817,13 @@ GRAG_API int grag_gemm_decode(const void* A, const void* W, const void* bias, vo
 }
 
 // out[M, F] = glu(x wg^T, x wu^T), w [2F, K] = wg | wu (glu_f with limit, alpha, shift on the fp32 sums): one K-range, natural W,
-// no tail.  F % (8 ntw) == 0, otherwise the requirements of grag_gemm_decode_t.
+// no tail; mt 1, 2, 4 or 8 on the five-wave grid.  F % (8 ntw) == 0, otherwise the requirements of grag_gemm_decode_t.
 GRAG_API int grag_gemm_decode_glu(const void* A, const void* W, void* C, int lda, int ldw, int ldc, int M, int F, int K,
                                   int mt, int nwv, int ntw, int gs, float limit, float alpha, float shift,
                                   hipStream_t stream) {
   if (M <= 0 || F <= 0) return 0;
   const int msplit = (M + 16 * mt - 1) / (16 * mt);
-  if (!grag_gemm_decode_has_t(mt, nwv, ntw, 0) || msplit > 4 || K % 64 != 0 || K < 64 || F % (8 * ntw) != 0 || lda % 8 != 0 ||
+  if (nwv != 5 || mt > 8 || !grag_gemm_decode_has_t(mt, nwv, ntw, 0) || msplit > 4 || K % 64 != 0 || K < 64 || F % (8 * ntw) != 0 || lda % 8 != 0 ||
       ldw % 8 != 0 || ldc % 4 != 0)
     return (int)hipErrorInvalidValue;
   const int units = F / (8 * ntw);
@@ -831,7 +842,7 @@ GRAG_API int grag_gemm_decode_glu(const void* A, const void* W, void* C, int lda
   a.kt_split = K / 64;
   a.limit = limit; a.alpha = alpha; a.shift = shift;
   if (!set_deal(a)) return (int)hipErrorInvalidValue;
-  return launch_variant(a, EPI_GLU, ACT_NONE, mt, nwv, ntw, 0, gs * msplit, stream);
+  return ntw == 1 ? launch_glu<1>(a, mt, gs * msplit, stream) : launch_glu<2>(a, mt, gs * msplit, stream);
 }
 
 // y = epilogue(RMSNorm(res_in + sum_s planes[s]) * nw @ w^T) for M <= 4 rows (NRM kernel): the split-K RMSNorm
