@@ -325,16 +325,17 @@ delta_prep_kernel(const T* __restrict__ xc, int C, const T* __restrict__ proj, i
 // the next head on the next XCD, the longest portions first (a contiguous range of sequences an XCD left those with short ones idle: 28
 // heads of 128 x 128, 12 portions of 7000 tokens together 305 us -> 174, 4 of 2500 129 -> 74; by q / k heads, 4 here, one portion is
 // slower by a tenth than by heads), 256 threads.  Bound by the latency of a chunk's steps, two workgroups a CU; a wave has up to four
-// times another's fp32 steps, so the next 256 workgroups give their tokens to the waves in the other order.  EXACT: d = 32 NDM, so that
-// nothing is tested between the products and LDS is read ahead of them; with that and loads on every path (below) the mixer of 12
-// heads over one portion of 1200 tokens 82 us -> 70, that of 28 heads over 12 portions of 7000 together 330 -> 311 (with 32 columns a
-// workgroup in place of 16 before that: 115, 398).  Wave w has token
-// block w of every chunk and rows 32 kg .. + 31 of the state's 16 columns for kg = w, w + 4.  NDM >= ND = ceil(d / 32).
+// times another's fp32 steps, so the second workgroup of a CU (every other `cus` of them, the device's CUs) gives its tokens to the
+// waves in the other order.  EXACT: d = 32 NDM, so that nothing is tested between the products and LDS is read ahead of them; with
+// that and loads on every path (below) the mixer of 12 heads over one portion of 1200 tokens 82 us -> 70, that of 28 heads over 12
+// portions of 7000 together 330 -> 311 (with 32 columns a workgroup in place of 16 before that: 115, 398).  Wave w has token block w
+// of every chunk and rows 32 kg .. + 31 of the state's 16 columns for kg = w, w + 4.  NDM >= ND = ceil(d / 32).
 template <typename T, int NDM, bool EXACT>
 __global__ void __launch_bounds__(256)
 delta_scan_kernel(const T* __restrict__ xc, int C, float* __restrict__ state, const int* __restrict__ slots,
                   const int* __restrict__ q_start, const int* __restrict__ ctx_len, float* __restrict__ out, int nseq,
-                  int H, int G, int d, int vd, int nslots, const T* __restrict__ wk, const float* __restrict__ wh, int nchunks) {
+                  int H, int G, int d, int vd, int nslots, const T* __restrict__ wk, const float* __restrict__ wh, int nchunks,
+                  unsigned cus) {
   constexpr int NG = (NDM + 3) / 4, RS = Right<T>::PLANES * 512;
   __shared__ __attribute__((aligned(16))) T So[NDM * RS];  // S_0 as right operands
   __shared__ __attribute__((aligned(16))) T Co[2 * RS];    // e^(L_63 - L_t) / |k_t| u_t as right operands
@@ -346,7 +347,7 @@ delta_scan_kernel(const T* __restrict__ xc, int C, float* __restrict__ state, co
   const int qa = q_start[seq], qlen = q_start[seq + 1] - qa;
   if (qlen <= 0) return;
   const int lane = threadIdx.x & 63, ql = lane & 15, quad = lane >> 4;
-  const int w = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) ^ (blockIdx.x >> 8 & 1 ? 3 : 0));
+  const int w = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) ^ (blockIdx.x / cus & 1 ? 3 : 0));
   const int ND = EXACT ? NDM : (d + 31) / 32, dp = 32 * ND, n = 16 * tile + ql;
   const bool n_ok = n < vd, fresh = ctx_len[seq] - qlen == 0;
   const int slot = slots[seq];
@@ -673,7 +674,7 @@ GRAG_API hipError_t grag_delta_scan(const void* xc, int C, const void* proj, int
 #define DELTA_SCAN(NDM)                                                                                               \
   (ND == NDM ? &delta_scan_kernel<T, NDM, true> : &delta_scan_kernel<T, NDM, false>)<<<grid, 256, 0, st>>>(           \
       (const T*)xc, C, state, slots, q_start, ctx_len, out, nseq, H, G, d, vd, nslots, (const T*)wk, (const float*)wh, \
-      nchunks)
+      nchunks, (unsigned)device_cus())
   DT_DISPATCH(dt, {
     auto* prep = ND == 4 ? &delta_prep_kernel<T, 4> : ND == 2 ? &delta_prep_kernel<T, 2> : &delta_prep_kernel<T, 0>;
     if (bytes > 48 * 1024) {
