@@ -218,6 +218,19 @@ __device__ __forceinline__ int xcd_remap(int orig, int nwg) {
   return base + orig / 8;
 }
 
+// an element as it is stored, widened where it is used: nothing waits for it before
+template <typename T> struct Stored;
+template <> struct Stored<bf16> {
+  short v;
+  __device__ __forceinline__ void load(const bf16* p) { v = *reinterpret_cast<const short*>(p); }
+  __device__ __forceinline__ float value() const { return bits2f(v); }
+};
+template <> struct Stored<float> {
+  float v;
+  __device__ __forceinline__ void load(const float* p) { v = *p; }
+  __device__ __forceinline__ float value() const { return v; }
+};
+
 // The sequence with the item-th longest portion (equal ones, and more than 64 sequences, as they come): for workgroups that walk whole
 // portions, so that the last ones to start are short.
 __device__ __forceinline__ int by_length(const int* q_start, int nseq, int item) {

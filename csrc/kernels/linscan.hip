@@ -124,18 +124,6 @@ __device__ __forceinline__ f32x4_t widen(f32x4_t v) { return v; }
 // ------------------------------------------------------------------------------------------------ elements
 __device__ __forceinline__ float elt(const bf16* p) { return (float)*p; }
 __device__ __forceinline__ float elt(const float* p) { return *p; }
-// an element as it is stored: nothing waits for it before it is used
-template <typename TI> struct Raw;
-template <> struct Raw<bf16> {
-  short v = 0;
-  __device__ __forceinline__ void load(const bf16* p) { v = *reinterpret_cast<const short*>(p); }
-  __device__ __forceinline__ float value() const { return bits2f(v); }
-};
-template <> struct Raw<float> {
-  float v = 0.f;
-  __device__ __forceinline__ void load(const float* p) { v = *p; }
-  __device__ __forceinline__ float value() const { return v; }
-};
 __device__ __forceinline__ float softplus_x(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 __device__ __forceinline__ float silu_acc(float x) { return x / (1.f + expf(-x)); }
 __device__ __forceinline__ float pow2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -391,7 +379,7 @@ linear_scan_kernel(const ScanArgs a) {
   constexpr int KT = 4 * ND, KR = LTHREADS / KT, KL = LC / KR > 0 ? LC / KR : 1;  // threads a row, rows a pass, passes
   const int krow = tid / KT, kc = 8 * (tid % KT), vrow = tid >> 3, vc = 8 * (tid & 7);
   TI4 kr[KL][2], vr[2], qr[OUT ? ND : 1][2];
-  Raw<TI> dtr;
+  Stored<TI> dtr;
   auto fetch = [&](int c) __attribute__((always_inline)) {
     const int end = min(qlen - c * LC, LC) - 1;
     const size_t t0 = (size_t)(qa + c * LC) * a.ld;

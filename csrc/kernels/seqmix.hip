@@ -1554,19 +1554,6 @@ __global__ void mingru_scan_kernel(const T* __restrict__ proj, int ld, int zoff,
 // time: a step's two layers of that size took 86 us, a load and a fold after the other, and take 47.
 constexpr int MINGRU_CHUNK = 32;
 
-// an element as it is stored, widened where it is used: nothing waits for it before
-template <typename T> struct Stored;
-template <> struct Stored<bf16> {
-  short v;
-  __device__ __forceinline__ void load(const bf16* p) { v = *reinterpret_cast<const short*>(p); }
-  __device__ __forceinline__ float value() const { return bits2f(v); }
-};
-template <> struct Stored<float> {
-  float v;
-  __device__ __forceinline__ void load(const float* p) { v = *p; }
-  __device__ __forceinline__ float value() const { return v; }
-};
-
 template <typename T, int PASS>
 __global__ void mingru_chunk_kernel(const T* __restrict__ proj, int ld, int zoff, int xoff, int goff,
                                     const float* __restrict__ bz, const float* __restrict__ bx,
