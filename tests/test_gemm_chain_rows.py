@@ -2,6 +2,7 @@
 results of a workgroup a tile of 256 rows, bit for bit, also with last tiles that end inside a wave's half or quadrant."""
 import pytest
 import torch
+import torch.nn.functional as F
 
 from githubrepostorag_amd.ops import gemm as G
 from githubrepostorag_amd.ops import linear as L
@@ -9,7 +10,7 @@ from githubrepostorag_amd.ops._lib import lib
 
 
 @pytest.mark.parametrize("M,N,K,rows", [(300, 37888, 3584, 128), (900, 37888, 3584, 192), (700, 37888, 3584, 256), (8192, 37888, 3584, 256),
-                                        (900, 17920, 1536, 192), (2400, 17920, 1536, 256), (12000, 3072, 768, 192), (8192, 14336, 3584, 256)])
+                                        (900, 17920, 1536, 192), (1187, 17920, 1536, 192), (2400, 17920, 1536, 256), (12000, 3072, 768, 192), (8192, 14336, 3584, 256)])
 def test_rule(M, N, K, rows):
     assert lib().grag_gemm_chain_rows(M, N, K, 256) == rows
     us = {r: lib().grag_gemm_chain_ns(M, N, K, r, 256) for r in (256, 192, 128)}
@@ -29,20 +30,32 @@ def test_plans(monkeypatch):
     G.wide_plan.cache_clear()
 
 
-# M: last tiles of 1 row, of one row past a wave's first quadrant / half, all but one; N: ragged columns
+# last tiles of 1 row, of one row past a wave's first quadrant and half, all but one; ragged columns, a bias that the chain takes
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,rows", [(1, 128), (33, 128), (65, 128), (127, 128), (577, 192), (625, 192), (673, 192), (767, 192)])
-@pytest.mark.parametrize("N,K", [(16320, 128), (16384, 320)])
-def test_rows(dev, M, rows, N, K):
-    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+@pytest.mark.parametrize("rows,last", [(r, n) for r in (256, 192, 128) for n in (1, r // 4 + 1, r // 2 + 1, r - 1)])
+@pytest.mark.parametrize("N,K", [(14272, 128), (14336, 320)])
+def test_rows(dev, monkeypatch, rows, last, N, K):
+    M = {256: 768, 192: 576, 128: 384}[rows] + last
+    if G._num_cus() == 256:
         assert lib().grag_gemm_chain_rows(M, N, K, 256) == rows
+    monkeypatch.setattr(G, "pair_plan", lambda *a: None)  # (the gated unit of these sizes is the small tiles')
     g = torch.Generator(device=dev).manual_seed(M + N + K)
     x = torch.randn(M, K + 8, generator=g, device=dev).bfloat16()[:, 8:]
     w, b = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).bfloat16(), torch.randn(N, generator=g, device=dev).bfloat16()
-    for f in (lambda: G.gemm(x, w, ksplit=1, sk=0), lambda: G.gemm(x, w[:8192], b[:8192], act=G.ACT_GELU, ksplit=1, sk=0),
-              lambda: G.gemm_silu(x, w, b, ksplit=1, sk=0), lambda: G.gemm_silu(x, w, ksplit=1, sk=0),
-              lambda: G.gemm_glu(x, w, 7.0, 1.702, 1.0)):
+    assert G.chain_takes(x, w, b)
+    z = x.double() @ w.double().T
+    zb = z + b.double()
+    unit = lambda t: (lambda a, u: F.silu(a) * u)(*(h.T for h in G.deinterleave_gate_up(t.T.contiguous())))  # noqa: E731
+    gate, up = z.chunk(2, 1)
+    gate = gate.clamp(max=1.0)
+    glu = gate * torch.sigmoid(1.702 * gate) * (up.clamp(-1, 1) + 1)
+    for f, want in ((lambda: G.gemm(x, w, ksplit=1, sk=0), z), (lambda: G.gemm(x, w, b, act=G.ACT_GELU, ksplit=1, sk=0), F.gelu(zb)),
+                    (lambda: G.gemm(x, w, b, act=G.ACT_GELU_TANH, ksplit=1, sk=0), F.gelu(zb, approximate="tanh")),
+                    (lambda: G.gemm_silu(x, w, b, ksplit=1, sk=0), unit(zb)), (lambda: G.gemm_silu(x, w, ksplit=1, sk=0), unit(z)),
+                    (lambda: G.gemm_glu(x, w, 1.0, 1.702, 1.0), glu)):
         got = f()
+        # half an ulp of bf16 of the value, the fp32 sums' rounding (K terms of order 1) and the activation's on top
+        torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=2 ** -8 * 0.05)
         prev = G.set_sched(1)  # a workgroup a tile of 256 rows
         try:
             assert torch.equal(got, f())
