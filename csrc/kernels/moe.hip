@@ -1194,10 +1194,19 @@ __device__ __forceinline__ void moe_chain(char* smem, const MoeChain& p, int til
                                                     [&] { return __builtin_amdgcn_readfirstlane(at.rows - 2 * QR * wr); });
 }
 
-// Tiles of 256, 192 or 128 rows, as the experts' row counts (known here alone) make the shortest rounds by the dense kernel's estimate,
-// with the rows in place of the tiles as its useful share, since an expert's last rows cost about theirs.  124 products of both bench
-// sizes, 430 - 4096 tokens x 4 of 16 experts: 0.1 % behind the best of the three on average, 7 % before tiles of 256 everywhere
-// (width 3584, unit width 3776, 1100 / 2000 tokens: first product 310 / 409 us -> 271 / 411, second 175 / 253 -> 146 / 218).
+// Tiles of 256, 192 or 128 rows, as the experts' row counts (known on the device alone) make the shortest rounds by the dense kernel's
+// estimate, with the rows in place of the tiles as its useful share, since an expert's last rows cost about theirs.  124 products of
+// both bench sizes, 430 - 4096 tokens x 4 of 16 experts: 0.1 % behind the best of the three on average, 7 % before tiles of 256
+// everywhere (width 3584, unit width 3776, 1100 / 2000 tokens: first product 310 / 409 us -> 271 / 411, second 175 / 253 -> 146 / 218).
+// n4, n3, n2: the tiles of 256, 192, 128 rows of one column of tiles; rows: of all experts.
+__host__ __device__ __forceinline__ int moe_chain_rows(int n4, int n3, int n2, int rows, int ncol, int steps, int cus) {
+  const float full = (float)rows * ncol;  // (of one row)
+  const float t4 = tile_chain_us<4>(n4 * ncol, full / 256, steps, cus), t3 = tile_chain_us<3>(n3 * ncol, full / 192, steps, cus),
+              t2 = tile_chain_us<2>(n2 * ncol, full / 128, steps, cus);
+  const bool fewer = t3 < 0.96f * t4;
+  return t2 < 0.96f * (fewer ? t3 : t4) ? 128 : fewer ? 192 : 256;
+}
+
 template <int GATED>
 __global__ void __launch_bounds__(kTileThreads, 2) moe_gemm_chain_kernel(const MoeChain p) {
   // (one array: the compiler waits for every load in flight where a read of one array could meet a DMA into another)
@@ -1211,19 +1220,12 @@ __global__ void __launch_bounds__(kTileThreads, 2) moe_gemm_chain_kernel(const M
     n4 += (cnt + 255) / 256, n3 += (cnt + 191) / 192, n2 += (cnt + 127) / 128;
   }
   n4 = wave_total(n4), n3 = wave_total(n3), n2 = wave_total(n2);
-  const int ncol = (p.N + (GATED == 1 ? 127 : 255)) / (GATED == 1 ? 128 : 256), steps = p.K >> 6, cus = gridDim.x;
-  n4 *= ncol, n3 *= ncol, n2 *= ncol;
-  const float full = (float)so[p.E] * ncol;  // (of one row)
-  const float t4 = tile_chain_us<4>(n4, full / 256, steps, cus), t3 = tile_chain_us<3>(n3, full / 192, steps, cus),
-              t2 = tile_chain_us<2>(n2, full / 128, steps, cus);
-  int rows = t3 < 0.96f * t4 ? 192 : 256;
-  if (t2 < 0.96f * (rows == 192 ? t3 : t4)) rows = 128;
-  rows = __builtin_amdgcn_readfirstlane(rows);
-  if (rows == 256) moe_chain<GATED, 4>(smem, p, n4);
-  else if (rows == 192) moe_chain<GATED, 3>(smem, p, n3);
-  else moe_chain<GATED, 2>(smem, p, n2);
+  const int ncol = (p.N + (GATED == 1 ? 127 : 255)) / (GATED == 1 ? 128 : 256);
+  const int rows = __builtin_amdgcn_readfirstlane(moe_chain_rows(n4, n3, n2, so[p.E], ncol, p.K >> 6, gridDim.x));
+  if (rows == 256) moe_chain<GATED, 4>(smem, p, n4 * ncol);
+  else if (rows == 192) moe_chain<GATED, 3>(smem, p, n3 * ncol);
+  else moe_chain<GATED, 2>(smem, p, n2 * ncol);
 }
-
 
 // ------------------------------------------------------------------------------------------------ residual boundary
 // x [T][H] fp32, in place: x <- keep x + mult * sigmoid(gate + gbias) * (a + bcoef_t b + sum_k ecoef_(t,k) e_(t,k)), every
@@ -1640,6 +1642,35 @@ GRAG_API hipError_t grag_moe_table_route(const int* tok, const int* table, int n
   return hipGetLastError();
 }
 
+// Columns of tiles of a product of the experts; whether its sizes are those of the 256 x 256 tile, and of its chains (moe_gemm_chain_kernel)
+static int moe_cols(int N, int gated) { return (N + (gated == 1 ? 127 : 255)) / (gated == 1 ? 128 : 256); }
+static long moe_weight_bytes(int N, int K, int gated) { return (long)(gated == 1 ? 2 * N : N) * K * 2; }
+static bool moe_tiles(int rows, int E, int N, int K, int gated) {
+  // (one branch, up to 64 tiles: the 128 x 128 tiles are four times as many workgroups, 60 tiles 66 us where these take 77, 24 24 / 25;
+  // from 96 on 52 / 42; with gate and up a tile has 128 columns, and 16 tiles take 19 for 21)
+  const bool many = gated == 1 || (long)((rows / E + 255) / 256) * E * moe_cols(N, gated) > 64;
+  return many && K % 64 == 0 && K >= 128 && rows >= MOE_TILE_MIN * E && E <= RT_MAXR && moe_weight_bytes(N, K, gated) < (1L << 31);
+}
+static bool moe_chains(int rows, int E, int N, int K, int gated) {
+  return moe_tiles(rows, E, N, K, gated) && K >= 320 && moe_weight_bytes(N, K, gated) * E < (1L << 31) && N % 8 == 0 && rows < (1 << 28);
+}
+static int moe_chain_grid(int rows, int E, int N, int gated, int cus) {
+  const long most = ((long)rows / 128 + E) * moe_cols(N, gated);
+  return (int)(most < cus ? most : cus);
+}
+
+// The rows of the tiles (256, 192, 128) that a chain over `rows` sorted rows, counts[e] of them expert e's (the others nobody's), takes on a
+// chip of `cus` CUs; 0 where grag_moe_gemm's sizes are not a chain's.
+GRAG_API int grag_moe_chain_rows(const int* counts, int E, int rows, int N, int K, int gated, int cus) {
+  if (gated == 2 || E < 1 || !moe_chains(rows, E, N, K, gated)) return 0;
+  int n4 = 0, n3 = 0, n2 = 0, all = 0;
+  for (int e = 0; e < E; ++e) {
+    n4 += (counts[e] + 255) / 256, n3 += (counts[e] + 191) / 192, n2 += (counts[e] + 127) / 128;
+    all += counts[e];
+  }
+  return moe_chain_rows(n4, n3, n2, all, moe_cols(N, gated), K >> 6, moe_chain_grid(rows, E, N, gated, cus));
+}
+
 // rows = T * top sorted rows.  gated 1: a = h [T][lda], w = [E][2N][K], out [rows][N]; gated 0: a = [rows][lda] sorted,
 // w = [E][N][K], out [rows][ldo] in (token, choice) order; gated 3: as 1 with one branch, w = [E][N][K]; gated 2: one matrix per head (E heads, top = tokens, rows =
 // tokens * E): a = [tokens * E][lda], w = [E][N][K], out [tokens * E][ldo], offs / order unused.
@@ -1666,23 +1697,17 @@ GRAG_API hipError_t grag_moe_gemm(const void* a, int lda, const void* w, const i
   }
   // K in whole steps, and operands within 32-bit byte offsets (a gathered has at most rows / top rows, every row of h one pair)
   const long a_rows = moe_gathers(gated) ? (rows + top - 1) / top : rows;
-  const long a_bytes = a_rows * lda * 2, w_bytes = (long)(gated == 1 ? 2 * N : N) * K * 2;
-  const int tcols = (N + (gated == 1 ? 127 : 255)) / (gated == 1 ? 128 : 256);
-  // (one branch, up to 64 tiles: the 128 x 128 tiles are four times as many workgroups, 60 tiles 66 us where these take 77, 24 24 / 25;
-  // from 96 on 52 / 42; with gate and up a tile has 128 columns, and 16 tiles take 19 for 21)
-  const bool many = gated == 1 || (long)((rows / E + 255) / 256) * E * tcols > 64;
-  if (dt == 0 && gated != 2 && many && K % 64 == 0 && K >= 128 && lda % 8 == 0 && al16(a) && al16(w) &&
-      rows >= MOE_TILE_MIN * E && E <= RT_MAXR && a_bytes < (1L << 31) && w_bytes < (1L << 31)) {
-    const long blocks = ((long)rows / 256 + E) * tcols;
+  const long a_bytes = a_rows * lda * 2, w_bytes = moe_weight_bytes(N, K, gated);
+  if (dt == 0 && gated != 2 && moe_tiles(rows, E, N, K, gated) && lda % 8 == 0 && al16(a) && al16(w) && a_bytes < (1L << 31)) {
+    const long blocks = ((long)rows / 256 + E) * moe_cols(N, gated);
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
     const long o_bytes = (long)rows * ldo * 2;
-    if (K >= 320 && w_bytes * E < (1L << 31) && o_bytes < (1L << 31) && N % 8 == 0 && ldo % 8 == 0 && al16(out) && rows < (1 << 28)) {
-      const int cus = device_cus();
-      const long most = ((long)rows / 128 + E) * tcols;
+    if (moe_chains(rows, E, N, K, gated) && o_bytes < (1L << 31) && ldo % 8 == 0 && al16(out)) {
+      const int nwg = moe_chain_grid(rows, E, N, gated, device_cus());
       const MoeChain p{(const bf16*)a, (const bf16*)w, offs, order, (bf16*)out, lda, (int)a_bytes, (int)(w_bytes * E), rows, E, top, N,
                        K, ldo, (int)o_bytes, ep};
 #define MOE_CHAIN(G) \
-  hipLaunchKernelGGL(moe_gemm_chain_kernel<G>, dim3((unsigned)(most < cus ? most : cus)), dim3(kTileThreads), 0, st, p)
+  hipLaunchKernelGGL(moe_gemm_chain_kernel<G>, dim3((unsigned)nwg), dim3(kTileThreads), 0, st, p)
       if (gated == 1) MOE_CHAIN(1);
       else if (gated == 3) MOE_CHAIN(3);
       else MOE_CHAIN(0);

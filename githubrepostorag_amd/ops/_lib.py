@@ -73,6 +73,7 @@ _SIGS = {
     "grag_gemm_chain_rows": [I, I, I, I],
     "grag_gemm_chain_ns": [I, I, I, I, I],
     "grag_gemm_chain_bias": [],
+    "grag_moe_chain_rows": [P, I, I, I, I, I, I],
     "grag_gemm_tile": [P, P, P, P, I, I, I, I, I, I, I, I, I, I, P, P, P],
     "grag_splitk_reduce": [P, P, P, I, I, I, I, I, I, P],
     "grag_gemm_tile_mfma": [I],
