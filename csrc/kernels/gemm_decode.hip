@@ -118,10 +118,10 @@ struct DArgs {
   int lda, ldw, ldc;
   int M, N, K;
   int units, gs, ksplit, kt_split;  // wave units per K-range, workgroups per K-range
-  // quotients as products, as a workgroup's first loads wait for them (five divisions, two of them of 64 bits, cost 0.1 - 0.2 us a
-  // launch: a decode step of 17 such launches at 64 rows 709.4 -> 706.3 us): inv_k, inv_m = ceil(2^32 / ksplit, msplit), exact below 2^32 / divisor; unit run g starts at
-  // floor(g units / gs) = g unit_lo + floor(g (units mod gs) / gs), the last quotient by unit_frac = ceil(2^32 (units mod gs) / gs),
-  // exact below 65536 workgroups; with more a run may start one unit from there, and still none has more than ceil(units / gs) of
+  // quotients as products, as a workgroup's first loads wait for them (five divisions, two of them of 64 bits: a step of 17 such
+  // launches at 64 rows 714 -> 711 us, near its noise): inv_k, inv_m = ceil(2^32 / ksplit, msplit), exact below 2^32 / divisor; unit
+  // run g starts at floor(g units / gs) = g unit_lo + floor(g (units mod gs) / gs), the last quotient by unit_frac =
+  // ceil(2^32 (units mod gs) / gs), exact below 65536 workgroups; with more a run may start one unit from there, and still none has more than ceil(units / gs) of
   // them: from run to run that quotient rises by 0 or 1, and it ends at units mod gs
   unsigned inv_k, inv_m, unit_frac;
   int unit_lo;
@@ -681,8 +681,9 @@ int launch_glu(const DArgs& a, int mt, int nwg, hipStream_t s) {
 // Variants compiled (mt = 16-row tiles of M, nwv = waves per workgroup, ntw = 16-row W tiles per wave;
 // depth kDepth): (nwv 4, ntw 2): mt 1, 2, 4, 8, 16;  (nwv 5, ntw 2): mt 1, 2, 4, 8, 12 (mt 1 / 2 also at
 // depth 8 and 12: 1-32 rows hold 2-4 KB of A per K-step, so the W ring takes the registers; balanced grids; mt 16 needs
-// more than the 256 registers a wave gets at two waves per SIMD);  (nwv 8, ntw 2): mt 12;  (nwv 5, ntw 1): mt 1, 2, 4, 8.  ntw = 4 measured no faster than 2 at M = 192 (profiles/gemm_decode_ab_v3.jsonl) and is
-// not instantiated.
+// more than the 256 registers a wave gets at two waves per SIMD);  (nwv 8, ntw 2): mt 12;  (nwv 5, ntw 1): mt 1, 2, 4, 8, one K-range;
+// gated units of separate halves: (nwv 5, ntw 1 and 2): mt 1, 2, 4, 8.  ntw = 4 measured no faster than 2 at M = 192
+// (profiles/gemm_decode_ab_v3.jsonl) and is not instantiated.
 static unsigned long long* g_dec_stamps = nullptr;
 static int g_dec_depth = 0;  // 0: kDepth; 6 / 8: deeper rings where the LDS takes them (A/B, grag_gemm_decode_depth)
 

@@ -690,7 +690,8 @@ auto slab_store = [&](const Acc& acc, int q) {
 // pays 8 - 10 us a round beside the products: a start, the first loads' way, and a write-out that all CUs begin together.
 // Measured, a workgroup a tile -> chains: 24000 x 2304 x 768 97 -> 85 us, 24000 x 3072 x 768 with GELU 145 -> 135, 24000 x 768 x 768
 // 44 -> 40; gate / up with SwiGLU 8192 x 37888 x 3584 1528 -> 1490, 2405 x 17920 x 1536 113 -> 107; 8192 x 14336 x 3584 597 -> 571, one
-// round of 8192 x 3584 x 18944 758 -> 761.  Tiles of 192 or 128 rows (MT = 3, 2) where they fill the rounds better: chain_rows.  Bands of 4 or 6 row tiles in place of 8: within 1 %.  Bitwise the same results.
+// round of 8192 x 3584 x 18944 758 -> 761.  Tiles of 192 or 128 rows (MT = 3, 2) where they fill the rounds better: chain_rows.
+// Bands of 4 or 6 row tiles in place of 8: within 1 %.  Bitwise the same results.
 constexpr int kChainBias = 14336;  // columns whose bias fits the LDS behind the two buffers (28 of 32 KB)
 
 template <int EPI, int ACT, bool BIAS, int MT>
@@ -872,10 +873,11 @@ double chain_us(int M, int N, int K, int rows, int ncu) {
                        : tile_chain_us<2>(tiles, tiles, K / 64, ncu);
 }
 // Rows of a chain's tiles: 256, which read their operands least, unless 192 or 128 leave so much less of the last round empty that
-// their estimate (tile_chain_us) is 2 % shorter.  At its 105 points that is the fastest of the three at every one (8.7 % less time than 256 rows
-// everywhere): 37888 x 3584 with SwiGLU 300 / 900 rows 151 / 241 us -> 114 (128 rows) / 204 (192); 17920 x 1536 900 / 1800 rows 68 /
-// 105 -> 63 / 99 (192; 1187 and 2400 rows stay: 74 / 73, 118 / 123); 8192 x 1536 3000 / 4300 rows 74 / 105 -> 67 / 95; 3072 x 768 with GELU
-// 12000 rows 82 -> 72.  Bitwise the same results.
+// their estimate (tile_chain_us) is 2 % shorter.  At 83 points of ten products, 300 - 24000 rows, that is within 1 % of the fastest of the
+// three, and 6 % less time than 256 rows everywhere: 37888 x 3584 with SwiGLU 300 / 900 rows 150 / 229 us -> 119 (128 rows) / 199
+// (192; 620 and 1187 rows stay: 165 / 192, 244 / 313); 17920 x 1536 900 / 1187 / 1800 rows 69 / 74 / 105 -> 62 / 64 / 92 (192; 1500 and
+// 2400 rows stay: 77 / 89, 113 / 124); 8192 x 1536 3000 / 4300 rows 73 / 101 -> 63 / 90; 3072 x 768 with GELU 12000 rows 83 -> 73.  Bitwise
+// the same results.
 int chain_rows(int M, int N, int K, int ncu) {
   int rows = 256;
   for (int r : {192, 128})

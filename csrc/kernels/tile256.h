@@ -305,8 +305,8 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
 }
 
 // A chain's time, us, for `tiles` tiles of 64 MT rows and 256 columns on ncu CUs, `full` of them if they were all full: begun rounds and
-// useful ones, each by K steps and once (the chip's power makes a round that is nearly empty a shorter one).  Least squares over 105 points of nine products (widths 768 -
-// 37888, K 768 - 18944, 300 - 24000 rows), 5 % off on average.
+// useful ones, each by K steps and once (the chip's power makes a round that is nearly empty a shorter one).  Least squares over 105
+// points of nine products (widths 768 - 37888, K 768 - 18944, 300 - 24000 rows), 5 % off on average there and 6 % at 83 others.
 template <int MT> __host__ __device__ inline float tile_chain_us(float tiles, float full, int steps, int ncu) {
   const float begun = ceilf(tiles / (float)ncu), used = full / (float)ncu;
   if (MT == 4) return (.72f * begun + .64f * used) * steps + 9.2f * begun - 2.3f * used + 3.8f;
