@@ -121,8 +121,8 @@ struct DArgs {
   // quotients as products, as a workgroup's first loads wait for them (five divisions, two of them of 64 bits: a step of 17 such
   // launches at 64 rows 714 -> 711 us, near its noise): inv_k, inv_m = ceil(2^32 / ksplit, msplit), exact below 2^32 / divisor; unit
   // run g starts at floor(g units / gs) = g unit_lo + floor(g (units mod gs) / gs), the last quotient by unit_frac =
-  // ceil(2^32 (units mod gs) / gs), exact below 65536 workgroups; with more a run may start one unit from there, and still none has more than ceil(units / gs) of
-  // them: from run to run that quotient rises by 0 or 1, and it ends at units mod gs
+  // ceil(2^32 (units mod gs) / gs), exact below 65536 workgroups; with more a run may start one unit from there, and still none has
+  // more than ceil(units / gs) of them: from run to run that quotient rises by 0 or 1, and it ends at units mod gs
   unsigned inv_k, inv_m, unit_frac;
   int unit_lo;
   int msplit;                       // row blocks of 16*MT (adjacent on one XCD: the W lines are shared in L2)
@@ -272,8 +272,8 @@ void gemm_dec_kernel(DArgs p) {
 
   // issue K-step `step` into ring slot `slot`; a step past the range (the last D iterations) re-reads
   // L2-resident bytes (A's own rows, one W line; that line for every step of a wave without a unit) so every
-  // iteration issues the same ops and the counted waits stay exact without a branch (a conditional load would make hipcc merge the ring registers through
-  // copies that read an asm destination before its data lands)
+  // iteration issues the same ops and the counted waits stay exact without a branch (a conditional load would make
+  // hipcc merge the ring registers through copies that read an asm destination before its data lands)
   auto issue = [&](int step, int slot, bf16x8_t (&wreg)[GW]) {
     const bool live = step < nsteps;
     const int so = live ? step * 64 : 0;

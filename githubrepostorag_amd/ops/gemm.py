@@ -317,11 +317,14 @@ def pair_plan(M: int, N: int, K: int, fused: bool = False) -> int | None:
     One product after another of different weights, in a graph, us.  Plain, K <= 1024: 64 x 64 tiles up to two a CU beat the
     library (768 x 768 at 300 / 1136 / 1752 rows 7.1 / 7.9 / 9.4 -> 6.1 / 6.4 / 7.7; 2304 x 768 600 9.4 -> 7.8, 1136, 648 tiles,
     10.0 / 10.5) and the decode kernel's K parts (64 / 256 rows 10.5 / 19.6 -> 6.1 / 6.3); up to 32 rows the skinny kernel stays
-    (20 rows 4.5 / 6.0); K 1152 - 1536 above 256 rows in 0.56 to 2 tiles a CU: the library or the owned tiles over these 1.14 in the
-    geometric mean of 98 points of 8 widths, 0.96 at worst, 4 of them more than 2 % behind, all next to the lower line (1536 x 1536 at 330
-    / 700 / 1300 rows 9.0 / 11.8 / 13.4 -> 9.1 / 10.8 / 12.2; 2304 x 1152 400 9.7 -> 7.8; 3072 x 1536 330 16.8 -> 12.9; with fewer tiles
-    260 rows 8.1 / 9.1, with more 1100 of 2304 18.1 / 19.6), and a launch from Python in 4 us for the library's 18.  Fused, K <= 2048: 64 x 64 up to 704 tiles, then 64 x 128 and 128 x 128 up to 512 each, against the
-    256 x 256 tile (GELU 3072 x 768 at 300 / 1136 / 1752 / 2500 rows 24 / 31 / 42 / 45 -> 6.9 / 12.3 / 17.5 / 19.9, from 4200 on 29
+    (20 rows 4.5 / 6.0).
+
+    Plain, K 1152 - 1536 above 256 rows, in 0.56 to 2 tiles a CU: the library or the owned tiles over these 1.14 in the geometric mean
+    of 98 points of 8 widths, 0.96 at worst, 4 of them, at 260 - 340 rows, more than 2 % behind (1536 x 1536 at 330 / 700 / 1300 rows 9.0 /
+    11.8 / 13.4 -> 9.1 / 10.8 / 12.2; 2304 x 1152 400 9.7 -> 7.8; 3072 x 1536 330 16.8 -> 12.9; with fewer tiles 1536 x 1536 260 8.1 /
+    9.1, with more 2304 x 1536 1100 18.1 / 19.6), and a launch from Python in 4 us for the library's 18.
+
+    Fused, K <= 2048: 64 x 64 up to 704 tiles, then 64 x 128 and 128 x 128 up to 512 each, against the 256 x 256 tile (GELU 3072 x 768 at 300 / 1136 / 1752 / 2500 rows 24 / 31 / 42 / 45 -> 6.9 / 12.3 / 17.5 / 19.9, from 4200 on 29
     / 33; SwiGLU 4096 x 1024 260 27 -> 10, 17920 x 1536 300 35 -> 29, 400 36 / 49; 22016 x 4096 260 80 / 104)."""
     if not _ON or M < 1 or max(M, N) * K >= 1 << 30:
         return None
