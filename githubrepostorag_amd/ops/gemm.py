@@ -763,9 +763,11 @@ def dec_wide(M: int, N: int, K: int) -> bool:
     return p is not None and len(p) > 4 and p[3:] == (1, _num_cus()) and (M <= 16 or p[2] == 1)
 
 
-def dec_coarse(plan: tuple | None) -> tuple | None:
-    """A decode plan in units of 32 rows: what packed weights and the folded norms have."""
-    return plan if plan is None or plan[2] != 1 else (plan[0], 5, 2, *plan[3:])
+def dec_coarse(plan: tuple | None, N: int) -> tuple | None:
+    """A decode plan of N columns in units of 32 rows: what packed weights and the folded norms have."""
+    if plan is None or plan[2] != 1:
+        return plan
+    return plan[0], 5, 2, plan[3], *(min(gs, N // 32) for gs in plan[4:5]), *plan[5:]
 
 
 DEC_TAIL = os.environ.get("GRAG_DEC_TAIL", "0") == "1"
@@ -833,7 +835,7 @@ def gemm_decode(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None,
         return gemm_silu(x, w, b) if epi == EPI_SILU else gemm(x, w, b, act)
     if plan is None:
         plan = dec_own_plan(M, N, K, epi == EPI_SILU) if packed is None else dec_plan(M, N, K, epi == EPI_SILU)
-    mt, nwv, ntw, ks, *rest = plan if packed is None else dec_coarse(plan)
+    mt, nwv, ntw, ks, *rest = plan if packed is None else dec_coarse(plan, N)
     gs = rest[0] if rest else 0
     tail = rest[1] if len(rest) > 1 else 0
     ks = dec_ksplit(K, ks)
@@ -885,7 +887,7 @@ def norm_fuse_plan(M: int, N: int, K: int, silu: bool) -> tuple[int, int] | None
     image; else None."""
     if not NORM_FUSE or M < 1 or M > 4 or M * (K * 2 + 64) > 65536:
         return None
-    p = dec_coarse(dec_plan(M, N, K, silu))
+    p = dec_coarse(dec_plan(M, N, K, silu), N)
     if p is None:
         return None
     mt, nwv, ntw, ks, *rest = p
@@ -963,7 +965,7 @@ def fold_plan(M: int, N: int, K: int, silu: bool) -> tuple[int, int, int] | None
     compile (one 16-row tile, 4- / 5-wave grid, no tail split); else None."""
     if not FOLD_NORM or M < 1 or M > 4:
         return None
-    p = dec_coarse(dec_plan(M, N, K, silu))
+    p = dec_coarse(dec_plan(M, N, K, silu), N)
     if p is None:
         return None
     mt, nwv, ntw, ks, *rest = p

@@ -89,7 +89,7 @@ def main():
                 plan = tuple(int(v) for v in a.plan.replace(":", ",").split(",")) if a.plan else G.dec_own_plan(M, N, K, silu)
                 if a.packed and plan is not None:
                     pks = [G.DecPacked(w, silu) for w in ws]
-                    plan = plan if a.plan else G.dec_coarse(G.dec_plan(M, N, K, silu))  # one plan that both layouts have
+                    plan = plan if a.plan else G.dec_coarse(G.dec_plan(M, N, K, silu), N)  # one plan that both layouts have
                     G.WS.reserve(dev, G.dec_ws_floats(M, N, G.dec_ksplit(K, plan[3])))
                     epi = G.EPI_SILU if silu else G.EPI_STORE
                     arms["dec_natural"] = lambda w, plan=plan, epi=epi: G.gemm_decode(x, w, epi=epi, plan=plan)

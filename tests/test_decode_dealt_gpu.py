@@ -164,6 +164,19 @@ def test_packed_takes_the_plan(dev, silu, M):
     w = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).bfloat16()
     epi = EPI_SILU if silu else G.EPI_STORE
     packed = G.DecPacked(w, silu)
-    want = gemm_decode(x, w, epi=epi, plan=G.dec_coarse(plan))  # the same sums in the same order
+    want = gemm_decode(x, w, epi=epi, plan=G.dec_coarse(plan, N))  # the same sums in the same order
     assert torch.equal(gemm_decode(x, w, epi=epi, plan=plan, packed=packed), want)
     assert torch.equal(gemm_decode(x, w, epi=epi, packed=packed), want)
+
+
+@pytest.mark.gpu
+def test_packed_takes_the_own_plan(dev):
+    """A plan with more workgroups than the product has units of 32 rows."""
+    ncu, K, M = _num_cus(), 512, 64
+    N = 64 * (3 * ncu // 8)  # 1.5 units of 16 a CU, 0.75 of 32
+    plan = G.dec_own_plan(M, N, K)
+    assert plan[1:] == (5, 1, 1, ncu) and G.dec_coarse(plan, N)[1:] == (5, 2, 1, N // 32)
+    g = torch.Generator(device=dev).manual_seed(3)
+    x = torch.randn(M, K, generator=g, device=dev).bfloat16()
+    w = (torch.randn(N, K, generator=g, device=dev) * K ** -0.5).bfloat16()
+    assert torch.equal(gemm_decode(x, w, plan=plan, packed=G.DecPacked(w)), gemm_decode(x, w, plan=G.dec_coarse(plan, N)))
