@@ -828,8 +828,8 @@ GRAG_API int grag_gemm_decode_glu(const void* A, const void* W, void* C, int lda
                                   hipStream_t stream) {
   if (M <= 0 || F <= 0) return 0;
   const int msplit = (M + 16 * mt - 1) / (16 * mt);
-  if (nwv != 5 || mt > 8 || !grag_gemm_decode_has_t(mt, nwv, ntw, 0) || msplit > 4 || K % 64 != 0 || K < 64 || F % (8 * ntw) != 0 || lda % 8 != 0 ||
-      ldw % 8 != 0 || ldc % 4 != 0)
+  if (nwv != 5 || mt > 8 || !grag_gemm_decode_has_t(mt, nwv, ntw, 0) || msplit > 4 || K % 64 != 0 || K < 64 ||
+      F % (8 * ntw) != 0 || lda % 8 != 0 || ldw % 8 != 0 || ldc % 4 != 0)
     return (int)hipErrorInvalidValue;
   const int units = F / (8 * ntw);
   if (gs <= 0 || gs > units || (units + gs - 1) / gs > nwv) return (int)hipErrorInvalidValue;

@@ -292,7 +292,8 @@ __device__ __forceinline__ bool scan_item(const ScanArgs& a, int item, ScanItem&
 // XCDs that had the long ones walked on while others were done: 7 portions of 8192 tokens, a CU was busy 48 % of the time.
 // ND = ceil(d / 32).  AP = 1 takes 76 KB of LDS and 128 registers: two workgroups share a CU, one's products over the other's
 // staging.  FULL: d = 32 ND, vd is a multiple of 64 and rows are aligned for 4-element accesses (rd / 2 a multiple of 4), so that
-// nothing is tested per element: of the ~4000 instructions a chunk took with the tests, half were theirs.  Rows behind a portion's end are copies of its last row with weight c_s = 0.
+// nothing is tested per element: of the ~4000 instructions a chunk took with the tests, half were theirs.  Rows behind a portion's
+// end are copies of its last row with weight c_s = 0.
 template <typename TI, int AP, bool SSM, bool FULL, int ND, int MODE>
 __global__ void __launch_bounds__(LTHREADS, AP == 1 ? 4 : 2)
 linear_scan_kernel(const ScanArgs a) {

@@ -324,8 +324,9 @@ def pair_plan(M: int, N: int, K: int, fused: bool = False) -> int | None:
     11.8 / 13.4 -> 9.1 / 10.8 / 12.2; 2304 x 1152 400 9.7 -> 7.8; 3072 x 1536 330 16.8 -> 12.9; with fewer tiles 1536 x 1536 260 8.1 /
     9.1, with more 2304 x 1536 1100 18.1 / 19.6), and a launch from Python in 4 us for the library's 18.
 
-    Fused, K <= 2048: 64 x 64 up to 704 tiles, then 64 x 128 and 128 x 128 up to 512 each, against the 256 x 256 tile (GELU 3072 x 768 at 300 / 1136 / 1752 / 2500 rows 24 / 31 / 42 / 45 -> 6.9 / 12.3 / 17.5 / 19.9, from 4200 on 29
-    / 33; SwiGLU 4096 x 1024 260 27 -> 10, 17920 x 1536 300 35 -> 29, 400 36 / 49; 22016 x 4096 260 80 / 104)."""
+    Fused, K <= 2048: 64 x 64 up to 704 tiles, then 64 x 128 and 128 x 128 up to 512 each, against the 256 x 256 tile (GELU 3072 x 768
+    at 300 / 1136 / 1752 / 2500 rows 24 / 31 / 42 / 45 -> 6.9 / 12.3 / 17.5 / 19.9, from 4200 on 29 / 33; SwiGLU 4096 x 1024 260 27 -> 10,
+    17920 x 1536 300 35 -> 29, 400 36 / 49; 22016 x 4096 260 80 / 104)."""
     if not _ON or M < 1 or max(M, N) * K >= 1 << 30:
         return None
     ncu = _num_cus()

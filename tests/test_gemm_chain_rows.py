@@ -10,7 +10,8 @@ from githubrepostorag_amd.ops._lib import lib
 
 
 @pytest.mark.parametrize("M,N,K,rows", [(300, 37888, 3584, 128), (900, 37888, 3584, 192), (700, 37888, 3584, 256), (8192, 37888, 3584, 256),
-                                        (900, 17920, 1536, 192), (1187, 17920, 1536, 192), (2400, 17920, 1536, 256), (12000, 3072, 768, 192), (8192, 14336, 3584, 256)])
+                                        (900, 17920, 1536, 192), (1187, 17920, 1536, 192), (2400, 17920, 1536, 256),
+                                        (12000, 3072, 768, 192), (8192, 14336, 3584, 256)])
 def test_rule(M, N, K, rows):
     assert lib().grag_gemm_chain_rows(M, N, K, 256) == rows
     us = {r: lib().grag_gemm_chain_ns(M, N, K, r, 256) for r in (256, 192, 128)}
