@@ -346,11 +346,12 @@ def pair_plan(M: int, N: int, K: int, fused: bool = False) -> int | None:
 
 @functools.lru_cache(4096)
 def pair_fills(M: int, N: int, K: int) -> bool:
-    """Whether short contractions whose 256 x 256 tiles would leave their last round of CUs nearly empty go in 128 x 192 ones:
-    24000 x 768 x 768 (282 tiles) 40 -> 34.5 us, 8000 x 2304 x 768 (288) 38 -> 34; fuller ones not (12000 x 2304 x 768, 0.82 of
-    the rounds, 42 / 52)."""
+    """Whether short contractions whose 256 x 256 tiles are one round of CUs and a rest of up to a fifth go in 128 x 192 ones: chains
+    of 192 rows / these, us, 22500 x 768 x 512 24.2 / 23.5, 24000 x 768 x 768 32.5 / 32.5, 9500 x 1920 x 512 (1.19 rounds) 25.0 / 23.8,
+    0.95 - 1.03 of 13 points; with longer rests 6000 x 3200 x 768 (1.22) 32.1 / 37.8, 27000 x 768 x 768 (1.24) 32.7 / 38.3, 1.06 - 1.18
+    of 7."""
     tiles, ncu = -(-M // 256) * -(-N // 256), _num_cus()
-    return K <= 1024 and tiles > ncu and M * N < 0.62 * 65536 * ncu * -(-tiles // ncu)
+    return K <= 1024 and ncu < tiles <= 1.2 * ncu
 
 
 def pair_takes(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None, out: torch.Tensor | None = None) -> bool:

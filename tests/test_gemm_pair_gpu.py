@@ -163,3 +163,14 @@ def test_linear_with_a_bias_at_any_address(dev, monkeypatch, M, N, K, other, at)
     y = L.linear(x, w, b)
     assert took == (["gemm_pair"] if at == 8 else ["gemm_decode"] if other == "decode" else [])
     torch.testing.assert_close(y.double(), x.double() @ w.double().T + b.double(), **TOL)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,takes", [(768, True), (1024, True), (1088, False)])
+def test_rounds_of_small_tiles(dev, K, takes):
+    """Short contractions of one round of CUs and up to a fifth go in small tiles: 255, 258, 306 and 309 tiles on 256 CUs."""
+    if G._num_cus() != 256:
+        pytest.skip("the row counts are those of 256 CUs")
+    assert [G.pair_fills(t * 256, 768, K) for t in (85, 86, 102, 103)] == [False, takes, takes, False]
+    x, w, b = _mk(dev, 86 * 256 - 7, 768, K)
+    assert torch.equal(G.gemm(x, w, b), G.gemm(x, w, b, ksplit=1, sk=0))
