@@ -18,8 +18,4 @@ __device__ __forceinline__ float act_f(float x) {
   else if constexpr (ACT == ACT_GELU_TANH) return gelu_tanh_f(x);
   else return x;
 }
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  return (uint32_t)(uint16_t)f2bits(lo) | ((uint32_t)(uint16_t)f2bits(hi) << 16);
-}
-
 }  // namespace grag

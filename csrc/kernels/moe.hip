@@ -1015,7 +1015,7 @@ moe_gemm_tile_kernel(const bf16* __restrict__ a, int lda, int a_bytes, const bf1
       for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-          d[i][h] = (uint32_t)(uint16_t)f2bits(val(rs, i, 2 * h)) | ((uint32_t)(uint16_t)f2bits(val(rs, i, 2 * h + 1)) << 16);
+          d[i][h] = pack_bf16x2(val(rs, i, 2 * h), val(rs, i, 2 * h + 1));
       if (wide) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -1162,7 +1162,7 @@ __device__ __forceinline__ void moe_chain(char* smem, const MoeChain& p, int til
       for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-          d[i][h] = (uint32_t)(uint16_t)f2bits(val(rs, i, 2 * h)) | ((uint32_t)(uint16_t)f2bits(val(rs, i, 2 * h + 1)) << 16);
+          d[i][h] = pack_bf16x2(val(rs, i, 2 * h), val(rs, i, 2 * h + 1));
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const auto s = __builtin_amdgcn_permlane16_swap(d[0][h], d[1][h], false, false);
