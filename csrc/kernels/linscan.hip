@@ -89,15 +89,6 @@ __device__ __forceinline__ bf16x4_t ld4t(const bf16* p, int ql, int quad, int kg
 }
 
 template <int N> struct Parts { bf16x8_t p[N]; };
-template <int N> __device__ __forceinline__ void split4(f32x4_t x, bf16x4_t (&p)[N]) {
-#pragma unroll
-  for (int j = 0; j < N; ++j)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      p[j][i] = f2bits(x[i]);
-      if (j + 1 < N) x[i] -= bits2f(p[j][i]);
-    }
-}
 template <int N> __device__ __forceinline__ Parts<N> split8(f32x4_t a, f32x4_t b) {
   bf16x4_t pa[N], pb[N];
   split4<N>(a, pa);
@@ -614,11 +605,10 @@ linear_scan_kernel(const ScanArgs a) {
       f32x4_t v[2];
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
-        v[e] = zero;
+        bf16x4_t vp[AP];
 #pragma unroll
-        for (int y = AP - 1; y >= 0; --y)
-          v[e] += widen(ld4t(Vs + y * VN + (2 * (2 * p + e) + (tb >> 1)) * 512, ql, quad, tb >> 1, tb & 1));
-        v[e] *= *reinterpret_cast<const f32x4_t*>(&sc[buf][5][32 * p + 16 * e + 4 * quad]);
+        for (int y = 0; y < AP; ++y) vp[y] = ld4t(Vs + y * VN + (2 * (2 * p + e) + (tb >> 1)) * 512, ql, quad, tb >> 1, tb & 1);
+        v[e] = join4<AP>(vp) * *reinterpret_cast<const f32x4_t*>(&sc[buf][5][32 * p + 16 * e + 4 * quad]);
       }
       const Parts<3> wv = split8<3>(v[0], v[1]);
 #pragma unroll
