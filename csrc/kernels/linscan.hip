@@ -12,7 +12,8 @@
 // seqmix.hip and ssm.hip, which still take decode rows and heads of more than 128 rows), waited on LDS broadcasts at 3 % of
 // the fp32 vector rate.  Here a chunk is bound by vector instructions (the splits, SiLU) and the latency of its dependent
 // steps.  Measured, those kernels -> this one with workgroups in order of sequence -> longest first (scan_item): decay with
-// SiLU, 28 heads of 128 x 128, 7 portions of 8192 tokens 2150 -> 748 -> 410 us, 1 x 1187 635 -> 110; without SiLU 2060 -> 214 -> 153
+// SiLU, 28 heads of 128 x 128, 7 portions of 8192 tokens 2150 -> 748 -> 410 us, 1 x 1187 635 -> 110 (with the splits and the halves of
+// q below, 390 in a model's step where it was 470 there); without SiLU 2060 -> 214 -> 153
 // and 602 -> 50; state space, 56 heads of 128 x 64, 3 portions of 4096 tokens 1450 -> 165 -> 115 us.
 //
 // Precision: nothing is rounded to 16 bits that was not before.  An operand is the sum of bf16 parts of 8 bits of mantissa
@@ -122,7 +123,7 @@ __device__ __forceinline__ float pow2(float x) { return __builtin_amdgcn_exp2f(x
 // reciprocal with one Newton step.  Below -87 the factor stays at e^-87 (times |x| < 2^20: under 2e-32).
 __device__ __forceinline__ float silu_x(float x) {
   constexpr float L2E = 1.4426950408889634f, L2E_LO = 1.9259629911266175e-8f;
-  const float m = fmaxf(x, -87.f), hi = -m * L2E, lo = fmaf(-m, L2E_LO, fmaf(-m, L2E, -hi));
+  const float m = __builtin_amdgcn_fmed3f(x, -87.f, INFINITY), hi = -m * L2E, lo = fmaf(-m, L2E_LO, fmaf(-m, L2E, -hi));
   const float e = pow2(hi), d = 1.f + fmaf(e, lo * 0.6931471805599453f, e);
   const float r = __builtin_amdgcn_rcpf(d);
   return x * fmaf(fmaf(-d, r, 1.f), r, r);
@@ -185,8 +186,7 @@ __device__ __forceinline__ void parts4(const ScanArgs& a, bf16x4_t (&p)[1], bf16
   p[0] = v;
 }
 template <bool FULL, typename TI, typename TV>
-__device__ __forceinline__ void parts4(const ScanArgs& a, bf16x4_t (&p)[3], TV raw, const TI* row, int c0, int pos,
-                                       bool rotary) {
+__device__ __forceinline__ f32x4_t value4(const ScanArgs& a, TV raw, const TI* row, int c0, int pos, bool rotary) {
   f32x4_t v = widen(raw);
   if (a.act) {
 #pragma unroll
@@ -221,7 +221,12 @@ __device__ __forceinline__ void parts4(const ScanArgs& a, bf16x4_t (&p)[3], TV r
       }
     }
   }
-  split4<3>(v, p);
+  return v;
+}
+template <bool FULL, typename TI, typename TV>
+__device__ __forceinline__ void parts4(const ScanArgs& a, bf16x4_t (&p)[3], TV raw, const TI* row, int c0, int pos,
+                                       bool rotary) {
+  split4<3>(value4<FULL>(a, raw, row, c0, pos, rotary), p);
 }
 
 // ------------------------------------------------------------------------------------------------ the scan
@@ -294,6 +299,12 @@ linear_scan_kernel(const ScanArgs a) {
   __shared__ __attribute__((aligned(16))) bf16 Ks[AP * KN];                      // [part][16 tokens][32 dims]
   __shared__ __attribute__((aligned(16))) bf16 Vs[AP * VN];                      // [part][16 tokens][32 columns]
   __shared__ __attribute__((aligned(16))) bf16 So[OUT ? 4 * ND * 3 * 512 : 8];  // [16 columns][32 dims][part]
+  // The two waves of a token block need the same q.  With three parts each makes half of its dims (SiLU is 12 instructions and two slow
+  // ones an element, of about 60 elements a thread) and both read all of it as fp32 from LDS, whose splits are the short part: 28
+  // heads of 128 x 128 with SiLU, 7 portions of 8192 tokens 450 -> 390 us.  The parts themselves would not fit the LDS (158 of 160 KB).
+  constexpr bool HALVES = OUT && AP == 3 && ND > 1;
+  constexpr int QN = HALVES ? ND / 2 : ND;  // 32-dim groups of q that a wave makes
+  __shared__ __attribute__((aligned(16))) float Qs[HALVES ? 4 * ND * 512 : 4];  // [16 tokens][32 dims]
   __shared__ __attribute__((aligned(16))) float sc[2][6][LC];  // L (two floats) | c_s | sign_t | 2^(L_t) | 2^(L_end - L_s) c_s
   __shared__ float ends[2][3];                                 // 2^(L_end) | L_end | not 0: too large for the products
   __shared__ __attribute__((aligned(16))) int odd[LTHREADS / 64];  // a wave's numbers are too large for the products
@@ -370,7 +381,8 @@ linear_scan_kernel(const ScanArgs a) {
   // krow + 512 / (4 ND), ... of k and 8 columns of a row of v; per wave its 16 rows of q as operands
   constexpr int KT = 4 * ND, KR = LTHREADS / KT, KL = LC / KR > 0 ? LC / KR : 1;  // threads a row, rows a pass, passes
   const int krow = tid / KT, kc = 8 * (tid % KT), vrow = tid >> 3, vc = 8 * (tid & 7);
-  TI4 kr[KL][2], vr[2], qr[OUT ? ND : 1][2];
+  TI4 kr[KL][2], vr[2], qr[OUT ? QN : 1][2];
+  const int qk = HALVES ? vh * QN : 0;
   Stored<TI> dtr;
   auto fetch = [&](int c) __attribute__((always_inline)) {
     const int end = min(qlen - c * LC, LC) - 1;
@@ -387,10 +399,10 @@ linear_scan_kernel(const ScanArgs a) {
     const size_t t0 = (size_t)(qa + c * LC) * a.ld;
     if (OUT) {
 #pragma unroll
-      for (int k = 0; k < ND; ++k)
+      for (int k = 0; k < QN; ++k)
 #pragma unroll
         for (int b = 0; b < 2; ++b)
-          qr[k][b] = raw4<FULL>(xq + t0 + min(16 * tb + ql, end) * a.ld, 32 * k + 16 * b + 4 * quad, a.d);
+          qr[k][b] = raw4<FULL>(xq + t0 + min(16 * tb + ql, end) * a.ld, 32 * (qk + k) + 16 * b + 4 * quad, a.d);
     }
   };
   auto fetch_dt = [&](int c) __attribute__((always_inline)) {
@@ -456,7 +468,7 @@ linear_scan_kernel(const ScanArgs a) {
       for (int x = 0; x < KL; ++x) big = squares(kr[x][e], big);
       big = squares(vr[e], big);
 #pragma unroll
-      for (int k = 0; k < (OUT ? ND : 0); ++k) big = squares(qr[k][e], big);
+      for (int k = 0; k < (OUT ? QN : 0); ++k) big = squares(qr[k][e], big);
     }
     const bool fits = __all(fmaf(big_s, SCAN_BIG / SCAN_BIG_S, big) < SCAN_BIG);  // (false for NaN)
     if (lane == 0) odd[w] = !fits;
@@ -498,14 +510,23 @@ linear_scan_kernel(const ScanArgs a) {
           *reinterpret_cast<bf16x4_t*>(So + ((tb * ND + (j >> 1)) * 3 + x) * 512 + lane * 8 + 4 * (j & 1)) = p[x];
       }
       const int rr = t0 + min(16 * tb + ql, min(n, LC) - 1), pos = position(rr);
+      if constexpr (HALVES) {
 #pragma unroll
-      for (int k = 0; k < ND; ++k) {
-        bf16x4_t p[2][AP];
+        for (int k = 0; k < QN; ++k)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
-          parts4<FULL>(a, p[b], qr[k][b], xq + (size_t)rr * a.ld, 32 * k + 16 * b + 4 * quad, pos, true);
+          for (int b = 0; b < 2; ++b)
+            *reinterpret_cast<f32x4_t*>(Qs + ((tb * ND + qk + k) * 2 + b) * 256 + lane * 4) =
+                value4<FULL>(a, qr[k][b], xq + (size_t)rr * a.ld, 32 * (qk + k) + 16 * b + 4 * quad, pos, true);
+      } else {
 #pragma unroll
-        for (int y = 0; y < AP; ++y) qf[k].p[y] = join(p[0][y], p[1][y]);
+        for (int k = 0; k < ND; ++k) {
+          bf16x4_t p[2][AP];
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+            parts4<FULL>(a, p[b], qr[k][b], xq + (size_t)rr * a.ld, 32 * k + 16 * b + 4 * quad, pos, true);
+#pragma unroll
+          for (int y = 0; y < AP; ++y) qf[k].p[y] = join(p[0][y], p[1][y]);
+        }
       }
     }
     __syncthreads();
@@ -520,6 +541,13 @@ linear_scan_kernel(const ScanArgs a) {
         if (c + 2 < nch) fetch_dt(c + 2);
       }
       fetch(c + 1);
+    }
+    if constexpr (HALVES) {
+#pragma unroll
+      for (int k = 0; k < ND; ++k) {
+        const float* q = Qs + (tb * ND + k) * 512 + lane * 4;
+        qf[k] = split8<3>(*reinterpret_cast<const f32x4_t*>(q), *reinterpret_cast<const f32x4_t*>(q + 256));
+      }
     }
     if (OUT) {
       const int t = 16 * tb + ql;
