@@ -123,7 +123,7 @@ __device__ __forceinline__ float pow2(float x) { return __builtin_amdgcn_exp2f(x
 // reciprocal with one Newton step.  Below -87 the factor stays at e^-87 (times |x| < 2^20: under 2e-32).
 __device__ __forceinline__ float silu_x(float x) {
   constexpr float L2E = 1.4426950408889634f, L2E_LO = 1.9259629911266175e-8f;
-  const float m = __builtin_amdgcn_fmed3f(x, -87.f, INFINITY), hi = -m * L2E, lo = fmaf(-m, L2E_LO, fmaf(-m, L2E, -hi));
+  const float m = __builtin_amdgcn_fmed3f(x, -87.f, 0x1p100f), hi = -m * L2E, lo = fmaf(-m, L2E_LO, fmaf(-m, L2E, -hi));
   const float e = pow2(hi), d = 1.f + fmaf(e, lo * 0.6931471805599453f, e);
   const float r = __builtin_amdgcn_rcpf(d);
   return x * fmaf(fmaf(-d, r, 1.f), r, r);
@@ -180,53 +180,45 @@ template <bool FULL> __device__ __forceinline__ f32x4_t raw4(const float* row, i
   for (int e = 0; e < 4; ++e) v[e] = c0 + e < n ? row[c0 + e] : 0.f;
   return v;
 }
-// the parts of 4 raw elements: as they are, or SiLU and (q and k) rotary of the first rd dims
-template <bool FULL, typename TI>
-__device__ __forceinline__ void parts4(const ScanArgs& a, bf16x4_t (&p)[1], bf16x4_t v, const TI*, int, int, bool) {
-  p[0] = v;
+// SiLU of numbers that are multiplied next to each other (one branch: a branch for every four left a wave waiting for its exponentials
+// and reciprocals)
+template <int N> __device__ __forceinline__ void silu_all(const ScanArgs& a, f32x4_t (&v)[N]) {
+  if (!a.act) return;
+#pragma unroll
+  for (int n = 0; n < N; ++n)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[n][e] = silu_x(v[n][e]);
 }
-template <bool FULL, typename TI, typename TV>
-__device__ __forceinline__ f32x4_t value4(const ScanArgs& a, TV raw, const TI* row, int c0, int pos, bool rotary) {
-  f32x4_t v = widen(raw);
-  if (a.act) {
+// rotary of elements c0 .. c0 + 3 (SiLU behind them) of q or k, where c0 < rd; their partners are read again
+template <bool FULL, typename TI>
+__device__ __forceinline__ void rotary4(const ScanArgs& a, f32x4_t& v, const TI* row, int c0, int pos) {
+  const int half = a.rd >> 1;
+  if (FULL) {  // (half is a multiple of 4: the four turn with four in a row)
+    if (c0 < a.rd) {
+      const bool lo = c0 < half;
+      const int fi = lo ? c0 : c0 - half;
+      f32x4_t u = widen(raw4<true>(row, lo ? c0 + half : fi, 0));
+      if (a.act) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = silu_x(v[e]);
-  }
-  if (rotary && a.rd) {
-    const int half = a.rd >> 1;
-    if (FULL) {  // (half is a multiple of 4: the four turn with four in a row)
-      if (c0 < a.rd) {
-        const bool lo = c0 < half;
-        const int fi = lo ? c0 : c0 - half;
-        f32x4_t u = widen(raw4<true>(row, lo ? c0 + half : fi, 0));
-        if (a.act) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) u[e] = silu_x(u[e]);
-        }
-        const float* tab = a.rope + (size_t)pos * a.rd + fi;
-        const f32x4_t c = *reinterpret_cast<const f32x4_t*>(tab), s = *reinterpret_cast<const f32x4_t*>(tab + half);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = lo ? v[e] * c[e] - u[e] * s[e] : v[e] * c[e] + u[e] * s[e];
+        for (int e = 0; e < 4; ++e) u[e] = silu_x(u[e]);
       }
-    } else {
+      const float* tab = a.rope + (size_t)pos * a.rd + fi;
+      const f32x4_t c = *reinterpret_cast<const f32x4_t*>(tab), s = *reinterpret_cast<const f32x4_t*>(tab + half);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = c0 + e;
-        if (i >= a.rd) continue;
-        const int fi = i < half ? i : i - half;
-        float other = elt(row + (i < half ? i + half : i - half));
-        if (a.act) other = silu_x(other);
-        const float c = a.rope[(size_t)pos * a.rd + fi], s = a.rope[(size_t)pos * a.rd + half + fi];
-        v[e] = i < half ? v[e] * c - other * s : v[e] * c + other * s;
-      }
+      for (int e = 0; e < 4; ++e) v[e] = lo ? v[e] * c[e] - u[e] * s[e] : v[e] * c[e] + u[e] * s[e];
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = c0 + e;
+      if (i >= a.rd) continue;
+      const int fi = i < half ? i : i - half;
+      float other = elt(row + (i < half ? i + half : i - half));
+      if (a.act) other = silu_x(other);
+      const float c = a.rope[(size_t)pos * a.rd + fi], s = a.rope[(size_t)pos * a.rd + half + fi];
+      v[e] = i < half ? v[e] * c - other * s : v[e] * c + other * s;
     }
   }
-  return v;
-}
-template <bool FULL, typename TI, typename TV>
-__device__ __forceinline__ void parts4(const ScanArgs& a, bf16x4_t (&p)[3], TV raw, const TI* row, int c0, int pos,
-                                       bool rotary) {
-  split4<3>(value4<FULL>(a, raw, row, c0, pos, rotary), p);
 }
 
 // ------------------------------------------------------------------------------------------------ the scan
@@ -306,6 +298,7 @@ linear_scan_kernel(const ScanArgs a) {
   constexpr int QN = HALVES ? ND / 2 : ND;  // 32-dim groups of q that a wave makes
   __shared__ __attribute__((aligned(16))) float Qs[HALVES ? 4 * ND * 512 : 4];  // [16 tokens][32 dims]
   __shared__ __attribute__((aligned(16))) float sc[2][6][LC];  // L (two floats) | c_s | sign_t | 2^(L_t) | 2^(L_end - L_s) c_s
+  __shared__ float pw[OUT && !SSM ? 80 : 1];
   __shared__ float ends[2][3];                                 // 2^(L_end) | L_end | not 0: too large for the products
   __shared__ __attribute__((aligned(16))) int odd[LTHREADS / 64];  // a wave's numbers are too large for the products
   const int ntile = (a.vd + LVT - 1) / LVT;
@@ -448,6 +441,14 @@ linear_scan_kernel(const ScanArgs a) {
     }
   };
   const f32x4_t zero = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // A decay's weights of a triangle are the walk's: lam^n c for n = 63 .. 0 tokens between, then zeros for the keys behind a query: a
+  // product and an LDS read a pair where 2^(L_t - L_s) and its mask were nine instructions and a branch.  (The state space's are the
+  // tokens'.  Without the branch, the mask on the exponent, they took more registers than there are: 142 us for 3 portions of 4096
+  // tokens -> 144.)  With SiLU in one block for all of a thread's elements, 28 heads of 128 x 128, 7 portions of 8192 tokens 390 -> 360 us.
+  if (OUT && !SSM && tid < 80) {
+    const int n = 63 - tid;
+    pw[tid] = n < 0 ? 0.f : a.kscale * pow2(rate * (float)n) * (neg && (n & 1) ? -1.f : 1.f);
+  }
   if (w == 4) {
     fetch_dt(0);
     scalars(0);
@@ -472,31 +473,55 @@ linear_scan_kernel(const ScanArgs a) {
     }
     const bool fits = __all(fmaf(big_s, SCAN_BIG / SCAN_BIG_S, big) < SCAN_BIG);  // (false for NaN)
     if (lane == 0) odd[w] = !fits;
+    auto put_k = [&](int r, int dim, const bf16x4_t (&p)[AP]) __attribute__((always_inline)) {
+      const int kg = dim >> 5;
 #pragma unroll
-    for (int x = 0; x < KL; ++x) {
-      const int r = krow + x * KR;
-      if (KR > LC && r >= LC) continue;
-      const int rr = t0 + min(r, min(n, LC) - 1), pos = position(rr);
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const int dim = kc + 4 * e, kg = dim >> 5;
-        bf16x4_t p[AP];
-        parts4<FULL>(a, p, kr[x][e], xk + (size_t)rr * a.ld, dim, pos, true);
-#pragma unroll
-        for (int y = 0; y < AP; ++y)
-          *reinterpret_cast<bf16x4_t*>(Ks + y * KN + ((r >> 4) * ND + kg) * 512 + place((dim >> 2) & 3, r & 15, kg) * 8 +
-                                       4 * ((dim >> 4) & 1)) = p[y];
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const int dim = vc + 4 * e, kg = dim >> 5;
-      bf16x4_t p[AP];
-      parts4<FULL>(a, p, vr[e], xv, 0, 0, false);  // (SiLU of the zeros behind the last column is 0)
+      for (int y = 0; y < AP; ++y)
+        *reinterpret_cast<bf16x4_t*>(Ks + y * KN + ((r >> 4) * ND + kg) * 512 + place((dim >> 2) & 3, r & 15, kg) * 8 +
+                                     4 * ((dim >> 4) & 1)) = p[y];
+    };
+    auto put_v = [&](int dim, const bf16x4_t (&p)[AP]) __attribute__((always_inline)) {
+      const int kg = dim >> 5;
 #pragma unroll
       for (int y = 0; y < AP; ++y)
         *reinterpret_cast<bf16x4_t*>(Vs + y * VN + ((vrow >> 4) * 2 + kg) * 512 + place((dim >> 2) & 3, vrow & 15, kg) * 8 +
                                      4 * ((dim >> 4) & 1)) = p[y];
+    };
+    const bool krows = KR <= LC || krow < LC;  // (more threads than k has rows: one pass)
+    if constexpr (AP == 1) {
+#pragma unroll
+      for (int x = 0; x < KL; ++x)
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          if (krows) put_k(krow + x * KR, kc + 4 * e, {kr[x][e]});
+#pragma unroll
+      for (int e = 0; e < 2; ++e) put_v(vc + 4 * e, {vr[e]});
+    } else {
+      if (krows) {
+        f32x4_t val[2 * KL];
+#pragma unroll
+        for (int x = 0; x < 2 * KL; ++x) val[x] = widen(kr[x >> 1][x & 1]);
+        silu_all(a, val);
+#pragma unroll
+        for (int x = 0; x < 2 * KL; ++x) {
+          const int r = krow + (x >> 1) * KR, dim = kc + 4 * (x & 1);
+          if (a.rd) {
+            const int rr = t0 + min(r, min(n, LC) - 1);
+            rotary4<FULL>(a, val[x], xk + (size_t)rr * a.ld, dim, position(rr));
+          }
+          bf16x4_t p[AP];
+          split4<AP>(val[x], p);
+          put_k(r, dim, p);
+        }
+      }
+      f32x4_t val[2] = {widen(vr[0]), widen(vr[1])};  // (SiLU of the zeros behind the last column is 0)
+      silu_all(a, val);
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        bf16x4_t p[AP];
+        split4<AP>(val[e], p);
+        put_v(vc + 4 * e, p);
+      }
     }
     Parts<AP> qf[OUT ? ND : 1];
     if (OUT) {
@@ -509,23 +534,27 @@ linear_scan_kernel(const ScanArgs a) {
         for (int x = 0; x < 3; ++x)
           *reinterpret_cast<bf16x4_t*>(So + ((tb * ND + (j >> 1)) * 3 + x) * 512 + lane * 8 + 4 * (j & 1)) = p[x];
       }
-      const int rr = t0 + min(16 * tb + ql, min(n, LC) - 1), pos = position(rr);
-      if constexpr (HALVES) {
+      if constexpr (AP == 1) {
 #pragma unroll
-        for (int k = 0; k < QN; ++k)
-#pragma unroll
-          for (int b = 0; b < 2; ++b)
-            *reinterpret_cast<f32x4_t*>(Qs + ((tb * ND + qk + k) * 2 + b) * 256 + lane * 4) =
-                value4<FULL>(a, qr[k][b], xq + (size_t)rr * a.ld, 32 * (qk + k) + 16 * b + 4 * quad, pos, true);
+        for (int k = 0; k < ND; ++k) qf[k].p[0] = join(qr[k][0], qr[k][1]);
       } else {
+        f32x4_t val[2 * QN];
 #pragma unroll
-        for (int k = 0; k < ND; ++k) {
-          bf16x4_t p[2][AP];
+        for (int x = 0; x < 2 * QN; ++x) val[x] = widen(qr[x >> 1][x & 1]);
+        silu_all(a, val);
+        if (a.rd) {
+          const int rr = t0 + min(16 * tb + ql, min(n, LC) - 1), pos = position(rr);
 #pragma unroll
-          for (int b = 0; b < 2; ++b)
-            parts4<FULL>(a, p[b], qr[k][b], xq + (size_t)rr * a.ld, 32 * k + 16 * b + 4 * quad, pos, true);
+          for (int x = 0; x < 2 * QN; ++x)
+            rotary4<FULL>(a, val[x], xq + (size_t)rr * a.ld, 32 * (qk + (x >> 1)) + 16 * (x & 1) + 4 * quad, pos);
+        }
+        if constexpr (HALVES) {
 #pragma unroll
-          for (int y = 0; y < AP; ++y) qf[k].p[y] = join(p[0][y], p[1][y]);
+          for (int x = 0; x < 2 * QN; ++x)
+            *reinterpret_cast<f32x4_t*>(Qs + ((tb * ND + qk) * 2 + x) * 256 + lane * 4) = val[x];
+        } else {
+#pragma unroll
+          for (int k = 0; k < ND; ++k) qf[k] = split8<AP>(val[2 * k], val[2 * k + 1]);
         }
       }
     }
@@ -583,12 +612,18 @@ linear_scan_kernel(const ScanArgs a) {
             m[e] = mul(kf, qf[k], m[e]);
           }
           __builtin_amdgcn_sched_barrier(0);
-          const f32x4_t ls = *reinterpret_cast<const f32x4_t*>(&sc[buf][0][16 * j + 4 * quad]);
-          const f32x4_t ls2 = *reinterpret_cast<const f32x4_t*>(&sc[buf][1][16 * j + 4 * quad]);
-          const f32x4_t cs = *reinterpret_cast<const f32x4_t*>(&sc[buf][2][16 * j + 4 * quad]);
+          if constexpr (SSM) {
+            const f32x4_t ls = *reinterpret_cast<const f32x4_t*>(&sc[buf][0][16 * j + 4 * quad]);
+            const f32x4_t ls2 = *reinterpret_cast<const f32x4_t*>(&sc[buf][1][16 * j + 4 * quad]);
+            const f32x4_t cs = *reinterpret_cast<const f32x4_t*>(&sc[buf][2][16 * j + 4 * quad]);
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            m[e][i] = 16 * j + 4 * quad + i <= t ? m[e][i] * (pow2((lt - ls[i]) + (lt2 - ls2[i])) * (cs[i] * ft)) : 0.f;
+            for (int i = 0; i < 4; ++i)
+              m[e][i] = 16 * j + 4 * quad + i <= t ? m[e][i] * (pow2((lt - ls[i]) + (lt2 - ls2[i])) * (cs[i] * ft)) : 0.f;
+          } else {
+            const float* at = pw + 63 - t + 16 * j + 4 * quad;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) m[e][i] *= at[i];
+          }
         }
         const Parts<3> ms = split8<3>(m[0], m[1]);
 #pragma unroll
