@@ -71,10 +71,17 @@ template <> struct Right<bf16> {
     for (int j = 0; j < 3; ++j) p[j] = *reinterpret_cast<const bf16x8_t*>(s + (j * 64 + lane) * 8);
   }
   static __device__ __forceinline__ void store(bf16* s, int lane, int half, f32x4_t x) {
-    bf16x4_t p[3];
-    split4<3>(x, p);
+    bf16x4_t h, m, l;
 #pragma unroll
-    for (int j = 0; j < 3; ++j) *reinterpret_cast<bf16x4_t*>(s + (j * 64 + lane) * 8 + 4 * half) = p[j];
+    for (int i = 0; i < 4; ++i) {
+      h[i] = f2bits(x[i]);
+      const float r = x[i] - bits2f(h[i]);
+      m[i] = f2bits(r);
+      l[i] = f2bits(r - bits2f(m[i]));
+    }
+    *reinterpret_cast<bf16x4_t*>(s + (0 * 64 + lane) * 8 + 4 * half) = h;
+    *reinterpret_cast<bf16x4_t*>(s + (1 * 64 + lane) * 8 + 4 * half) = m;
+    *reinterpret_cast<bf16x4_t*>(s + (2 * 64 + lane) * 8 + 4 * half) = l;
   }
 };
 template <> struct Right<float> {
