@@ -73,7 +73,7 @@ __device__ __forceinline__ bf16x4_t pack4(f32x4_t v) { return __builtin_bit_cast
 // What the bf16 numbers of a pair (pack_bf16x2) leave of the two floats: x -= its half, one v_dot2_f32_bf16 each (p . (-1, 0) + x) where
 // the number's way back to fp32 and the difference are two.  Exact for finite pairs, 4 M of all exponents compared bit for bit; a pair
 // with an infinity or a NaN leaves NaN in both.  The factors are registers: as a literal -1 is encoded as the inline constant of an
-// fp32 operand and multiplies the other half.  In the scans' splits (linscan.hip, delta.hip), with the pairs' conversions: state space, 3
+// fp32 operand and multiplies the other half.  In the splits of linscan.hip, with the pairs' conversions: state space, 3
 // portions of 4096 tokens, 148 -> 142 us; a decay scan of a hybrid prompt step of 8192 tokens 470 -> 450.
 template <bool ADD>
 __device__ __forceinline__ void dot_bf16x2(uint32_t p, float& lo, float& hi) {
