@@ -30,7 +30,7 @@ __device__ __forceinline__ float silu_acc(float x) { return x / (1.f + expf(-x))
 __device__ __forceinline__ float tanh_acc(float x) {
   const float a = fabsf(x);
   const float x2 = x * x;
-  const float small = x * (1.f + x2 * (-0.33333334f + x2 * 0.13333334f));
+  float small = x * (1.f + x2 * (-0.33333334f + x2 * 0.13333334f));
   const float h = -2.885390043258667f * a;                             // -2 / ln 2, its first 24 bits
   const float l = fmaf(-2.885390043258667f, a, -h) - 3.8519259e-8f * a;  // the product's rounding and the rest of it
   float t = __builtin_amdgcn_exp2f(h);
@@ -38,6 +38,7 @@ __device__ __forceinline__ float tanh_acc(float x) {
   const float n = 1.f - t, d = 1.f + t, rc = __builtin_amdgcn_rcpf(d);
   float q = n * rc;
   q = fmaf(fmaf(-d, q, n), rc, q);
+  asm("" : "+v"(small), "+v"(q));  // (both, and a select: as a branch an element they waited for their exponentials one by one)
   return a < 0.02f ? small : copysignf(q, x);
 }
 
