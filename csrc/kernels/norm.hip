@@ -355,7 +355,74 @@ __global__ __launch_bounds__(kThreads) void layernorm_kernel(
   }
 }
 
-// BERT embeddings: LN(word[id] + pos[p] + type[tt]) — one block per token.
+// BERT embeddings: LN(word[id] + pos[p] + type[tt]).  Up to 1024 columns a wave a token, as layernorm_wave_kernel: 24000 tokens of 768
+// 37.8 us in workgroups of 256 threads a token, here 22.7.
+template <int VPT>
+__global__ __launch_bounds__(kThreads) void bert_embed_ln_wave_kernel(
+    const int32_t* __restrict__ ids, const int32_t* __restrict__ pos_ids,
+    const int32_t* __restrict__ type_ids, const bf16* __restrict__ word,
+    const bf16* __restrict__ pos, const bf16* __restrict__ type, const bf16* __restrict__ gamma,
+    const bf16* __restrict__ beta, bf16* __restrict__ out, int T, int H, int V, int P, float eps) {
+  const int lane = threadIdx.x & 63, t = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6), nvec = H >> 3;
+  if (t >= T) return;
+  int tid = ids[t], pid = pos_ids[t];
+  if (!index_ok(tid, V, ERR_BERT_TOKEN)) tid = 0;  // reported; row 0 read instead
+  if (!index_ok(pid, P, ERR_BERT_TOKEN)) pid = 0;
+  const bf16x8_t* wr = reinterpret_cast<const bf16x8_t*>(word + (size_t)tid * H);
+  const bf16x8_t* pr = reinterpret_cast<const bf16x8_t*>(pos + (size_t)pid * H);
+  const bf16x8_t* tr = reinterpret_cast<const bf16x8_t*>(type + (size_t)(type_ids ? type_ids[t] : 0) * H);
+  const bf16x8_t zero = bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+  bf16x8_t wv[VPT], pv[VPT], tv[VPT], gv[VPT], ev[VPT];
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int idx = lane + i * 64;
+    wv[i] = pv[i] = tv[i] = gv[i] = ev[i] = zero;
+    if (idx < nvec) {
+      wv[i] = wr[idx];
+      pv[i] = pr[idx];
+      tv[i] = tr[idx];
+      gv[i] = reinterpret_cast<const bf16x8_t*>(gamma)[idx];
+      ev[i] = reinterpret_cast<const bf16x8_t*>(beta)[idx];
+    }
+  }
+  float v[VPT][8], s = 0.f, s2 = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    float a[8], b[8], c[8];
+    unpack8(wv[i], a);
+    unpack8(pv[i], b);
+    unpack8(tv[i], c);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      v[i][j] = a[j] + b[j] + c[j];
+      s += v[i][j];
+    }
+  }
+  const float mean = wave_sum(s) / (float)H;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i)
+    if (lane + i * 64 < nvec) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float d = v[i][j] - mean;
+        s2 += d * d;
+      }
+    }
+  const float inv = rsqrtf(wave_sum(s2) / (float)H + eps);
+  bf16x8_t* orow = reinterpret_cast<bf16x8_t*>(out + (size_t)t * H);
+#pragma unroll
+  for (int i = 0; i < VPT; ++i)
+    if (lane + i * 64 < nvec) {
+      float g[8], b[8], o[8];
+      unpack8(gv[i], g);
+      unpack8(ev[i], b);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = (v[i][j] - mean) * inv * g[j] + b[j];
+      orow[lane + i * 64] = pack8(o);
+    }
+}
+
+// Wider rows: a workgroup a token.
 template <int VPT>
 __global__ __launch_bounds__(kThreads) void bert_embed_ln_kernel(
     const int32_t* __restrict__ ids, const int32_t* __restrict__ pos_ids,
@@ -622,6 +689,14 @@ GRAG_API int grag_bert_embed_ln(const int32_t* ids, const int32_t* pos_ids,
                                 int T, int H, int V, int P, float eps, hipStream_t stream) {
   if (T <= 0) return 0;
   if (H % 8 != 0 || H > 8 * 8 * kThreads) return (int)hipErrorInvalidValue;
+  constexpr int rows = kThreads / 64;
+  auto wave = [&](auto kern) {
+    kern<<<(T + rows - 1) / rows, kThreads, 0, stream>>>(ids, pos_ids, type_ids, (const bf16*)word, (const bf16*)pos, (const bf16*)type,
+                                                         (const bf16*)gamma, (const bf16*)beta, (bf16*)out, T, H, V, P, eps);
+    return (int)hipGetLastError();
+  };
+  if (H <= 512) return wave(bert_embed_ln_wave_kernel<1>);
+  if (H <= 1024) return wave(bert_embed_ln_wave_kernel<2>);
   auto args = [&](auto kern) {
     kern<<<T, kThreads, 0, stream>>>(ids, pos_ids, type_ids, (const bf16*)word, (const bf16*)pos,
                                      (const bf16*)type, (const bf16*)gamma, (const bf16*)beta,

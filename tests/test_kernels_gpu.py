@@ -64,6 +64,22 @@ def test_embeddings(dev):
     close(N.embed_gather(ids, word), word.cpu()[ids.cpu().long()], 0)
 
 
+@pytest.mark.parametrize("T,H", [(1, 8), (5, 512), (7, 520), (3, 1024), (6, 1032), (2, 2056)])
+def test_bert_embed_ln_widths(T, H):
+    """A wave a token up to 1024 columns, a workgroup from there on; token counts that are no multiple of a workgroup's four."""
+    from githubrepostorag_amd.ops import norm as N
+
+    g = torch.Generator().manual_seed(T * 3000 + H)
+    word, pos, typ = (torch.randn(n, H, generator=g).to(torch.bfloat16) for n in (50, 20, 2))
+    gamma, beta = (torch.randn(H, generator=g).to(torch.bfloat16) for _ in range(2))
+    ids, pids, tids = (torch.randint(0, n, (T,), generator=g, dtype=torch.int32) for n in (50, 20, 2))
+    for t in (None, tids):
+        want = N.bert_embed_ln_ref(ids, pids, t, word, pos, typ, gamma, beta, 1e-12)
+        got = N.bert_embed_ln(*(None if x is None else x.cuda() for x in (ids, pids, t, word, pos, typ, gamma, beta)), 1e-12).cpu()
+        # both round an fp32 result once: one bf16 step (2^-8) apart where it lies between two
+        torch.testing.assert_close(got.float(), want.float(), rtol=2 ** -7, atol=2e-6)
+
+
 def test_qkv_rope_kvstore(dev):
     T, Hq, Hkv, D, BS, NB = 29, 28, 4, 128, 16, 8
     qkv = rnd(T, (Hq + 2 * Hkv) * D, dev=dev)
