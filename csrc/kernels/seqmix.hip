@@ -161,6 +161,18 @@ dyt_residual_vec_kernel(const T* __restrict__ y, const float* __restrict__ plane
   }
 }
 
+// embed_f32_kernel, H a multiple of 4 and aligned pointers: four elements a thread in one trip behind the token's (element by element, 14
+// trips one after another: 64 tokens of 3584 8.1 us, 8192 55, here 4.7 and 33).  grid (T, ceil(H / 1024))
+template <typename T>
+__global__ void __launch_bounds__(256)
+embed_f32_vec_kernel(const int* __restrict__ ids, const T* __restrict__ table, float* __restrict__ out, int H, int vocab, float scale) {
+  const int t = blockIdx.x, i = blockIdx.y * 1024 + threadIdx.x * 4, id = ids[t];
+  if (i >= H) return;
+  const bool ok = index_ok(id, vocab, ERR_EMBED_TOKEN);
+  const f32x4_t v = ok ? ld4(table + (size_t)id * H + i) * scale : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  *reinterpret_cast<f32x4_t*>(out + (size_t)t * H + i) = v;
+}
+
 // ------------------------------------------------------------------------------------------------ rotary + K/V store
 // proj [T, ld]: q heads at column qoff (H x d), k heads at koff (G x d), v heads at voff (G x vd).
 // q_out [T, H*d] = rotated q; k_cache [nblk, G, BS, d] <- rotated k; v_cache [nblk, G, BS, vd] <- v / rms(v).
@@ -1701,6 +1713,11 @@ using namespace grag;
 GRAG_API hipError_t grag_embed_f32(const int* ids, const void* table, float* out, int T_, int H, int vocab, int dt,
                                    float scale, hipStream_t st) {
   if (T_ <= 0) return hipSuccess;
+  if (H % 4 == 0 && !((uintptr_t)out & 15) && !((uintptr_t)table & (dt == 0 ? 7 : 15))) {
+    DT_DISPATCH(dt, hipLaunchKernelGGL(embed_f32_vec_kernel<T>, dim3(T_, (H + 1023) / 1024), dim3(256), 0, st, ids, (const T*)table,
+                                       out, H, vocab, scale);)
+    return hipGetLastError();
+  }
   DT_DISPATCH(dt, hipLaunchKernelGGL(embed_f32_kernel<T>, dim3(T_), dim3(256), 0, st, ids, (const T*)table, out, H,
                                      vocab, scale);)
   return hipGetLastError();
