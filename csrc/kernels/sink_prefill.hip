@@ -142,8 +142,10 @@ __global__ void __launch_bounds__(256 * TEAMS, MR == 32 || TEAMS > 1 ? 2 : 4) si
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) {
       s[tt] = acc_t{};
+      if (tt == 0) __builtin_amdgcn_s_setprio(1);  // (before the CU's other workgroup, whose values' products have instructions between)
 #pragma unroll
       for (int c = 0; c < NC; ++c) s[tt] = mma(kf[tt][c], qf[c], s[tt]);
+      if (tt == NT - 1) __builtin_amdgcn_s_setprio(0);
     }
     if constexpr (CAP) {  // cap in the natural domain, then to log2
       // Below 1/4 by tanh's power series to x^9, whose next term is 1/10 of fp32's rounding there; a tile with a larger score by
@@ -265,9 +267,11 @@ __global__ void __launch_bounds__(256 * TEAMS, MR == 32 || TEAMS > 1 ? 2 : 4) si
       continue;
     }
     const char* v_lds = k_lds + TILE;
+    __builtin_amdgcn_s_setprio(1);
     load_v(v_lds, 0);
     maximum();
     weights(0);
+    __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < NP; ++u) {
