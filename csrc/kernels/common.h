@@ -74,7 +74,7 @@ __device__ __forceinline__ bf16x4_t pack4(f32x4_t v) { return __builtin_bit_cast
 // the number's way back to fp32 and the difference are two.  Exact for finite pairs, 4 M of all exponents compared bit for bit; a pair
 // with an infinity or a NaN leaves NaN in both.  The factors are registers: as a literal -1 is encoded as the inline constant of an
 // fp32 operand and multiplies the other half.  In the splits of linscan.hip, with the pairs' conversions: state space, 3
-// portions of 4096 tokens, 148 -> 142 us; a decay scan of a hybrid prompt step of 8192 tokens 470 -> 450.
+// portions of 4096 tokens, 149 -> 144 us; a decay scan of a hybrid prompt step of 8192 tokens, 20 us of 470.
 template <bool ADD>
 __device__ __forceinline__ void dot_bf16x2(uint32_t p, float& lo, float& hi) {
   uint32_t kl = ADD ? 0x00003f80u : 0x0000bf80u, kh = kl << 16;

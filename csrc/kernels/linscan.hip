@@ -12,8 +12,8 @@
 // seqmix.hip and ssm.hip, which still take decode rows and heads of more than 128 rows), waited on LDS broadcasts at 3 % of
 // the fp32 vector rate.  Here a chunk is bound by vector instructions (the splits, SiLU) and the latency of its dependent
 // steps.  Measured, those kernels -> this one with workgroups in order of sequence -> longest first (scan_item): decay with
-// SiLU, 28 heads of 128 x 128, 7 portions of 8192 tokens 2150 -> 748 -> 410 us, 1 x 1187 635 -> 110 (with the splits and the halves of
-// q below, 390 in a model's step where it was 470 there); without SiLU 2060 -> 214 -> 153
+// SiLU, 28 heads of 128 x 128, 7 portions of 8192 tokens 2150 -> 748 -> 410 us, 1 x 1187 635 -> 110 (with the splits, the halves of
+// q and the table below, 380 - 390 in a model's step where it was 474 there); without SiLU 2060 -> 214 -> 153
 // and 602 -> 50; state space, 56 heads of 128 x 64, 3 portions of 4096 tokens 1450 -> 165 -> 115 us.
 //
 // Precision: nothing is rounded to 16 bits that was not before.  An operand is the sum of bf16 parts of 8 bits of mantissa
@@ -100,7 +100,8 @@ template <int N> __device__ __forceinline__ Parts<N> split8(f32x4_t a, f32x4_t b
   return s;
 }
 // The parts of the products a * b, whose rounding the second part takes along: without it the states' error against 64 bits is 1 - 2 %
-// larger (8 heads of 128 x 128, 500 + 333 tokens 1.16e-7 -> 1.19e-7), with it state space of 3 portions of 4096 tokens takes 144 us for 142.
+// larger (8 heads of 128 x 128, 500 + 333 tokens 1.16e-7 -> 1.19e-7), with it state space of 3 portions of 4096 tokens takes 144 us
+// for 142.
 __device__ __forceinline__ Parts<3> split8(f32x4_t a0, f32x4_t b0, f32x4_t a1, f32x4_t b1) {
   Parts<3> s;
   bf16x4_t lo[2][2], hi[2];
@@ -312,7 +313,7 @@ linear_scan_kernel(const ScanArgs a) {
   __shared__ __attribute__((aligned(16))) bf16 So[OUT ? 4 * ND * 3 * 512 : 8];  // [16 columns][32 dims][part]
   // The two waves of a token block need the same q.  With three parts each makes half of its dims (SiLU is 12 instructions and two slow
   // ones an element, of about 60 elements a thread) and both read all of it as fp32 from LDS, whose splits are the short part: 28
-  // heads of 128 x 128 with SiLU, 7 portions of 8192 tokens 450 -> 390 us.  The parts themselves would not fit the LDS (158 of 160 KB).
+  // heads of 128 x 128 with SiLU, 7 portions of 8192 tokens, 60 us of 450.  The parts themselves would not fit the LDS (158 of 160 KB).
   constexpr bool HALVES = OUT && AP == 3 && ND > 1;
   constexpr int QN = HALVES ? ND / 2 : ND;  // 32-dim groups of q that a wave makes
   __shared__ __attribute__((aligned(16))) float Qs[HALVES ? 4 * ND * 512 : 4];  // [16 tokens][32 dims]
@@ -463,7 +464,8 @@ linear_scan_kernel(const ScanArgs a) {
   // A decay's weights of a triangle are the walk's: lam^n c for n = 63 .. 0 tokens between, then zeros for the keys behind a query: a
   // product and an LDS read a pair where 2^(L_t - L_s) and its mask were nine instructions and a branch.  (The state space's are the
   // tokens'.  Without the branch, the mask on the exponent, they took more registers than there are: 142 us for 3 portions of 4096
-  // tokens, 2.5 more.)  With SiLU in one block for all of a thread's elements, 28 heads of 128 x 128, 7 portions of 8192 tokens 390 -> 360 us.
+  // tokens, 2.5 more.)  With SiLU in one block for all of a thread's elements, 28 heads of 128 x 128, 7 portions of 8192 tokens, 30 us
+  // of 390.
   if (OUT && !SSM && tid < 80) {
     const int n = 63 - tid;
     pw[tid] = n < 0 ? 0.f : a.kscale * pow2(rate * (float)n) * (neg && (n & 1) ? -1.f : 1.f);

@@ -271,7 +271,8 @@ __device__ __forceinline__ void tile256_chain(char* smem, const __amdgpu_buffer_
       tile_zero<MT>(acc00);
       tile_zero<MT>(acc01);
       readA(a, 1, buf);
-      tile_wait_vm<8 + ST2>();  // (behind the stores: what it waits for comes in while they are made; experts of 4096 tokens 1128 -> 1124 us)
+      // (behind the stores: what it waits for comes in while they are made; experts of 4096 tokens 1128 -> 1124 us)
+      tile_wait_vm<8 + ST2>();
     } else {
       readA(a, 1, buf);
       refill();

@@ -52,6 +52,29 @@ def test_layernorm(dev, H):
     close(y, N.layernorm_ref(x.cpu(), g.cpu(), be.cpu(), 1e-12, b.cpu(), r.cpu()), 5e-2)
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("scale", [0.125, -0.3, 0.0])
+def test_varlen_attention_scales(dev, D, scale):
+    """A scale in the exponent's factor, and those of 0 and less, which turn the order; keys that grow along a text, so that its maximum
+    moves by more than 2^8 from tile to tile, and some that shrink."""
+    from githubrepostorag_amd.ops import attention as A
+
+    g = torch.Generator().manual_seed(D)
+    H, lens = 3, [1, 64, 65, 200, 257]
+    T = sum(lens)
+    qkv = torch.randn(T, 3, H, D, generator=g)
+    at = torch.cat([torch.arange(n) for n in lens]).float()
+    qkv[:, 1, 0] *= (1 + at / 16)[:, None]
+    qkv[:, 1, 1] /= (1 + at / 16)[:, None]
+    qkv = qkv.reshape(T, -1).to(torch.bfloat16)
+    start = torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], dtype=torch.int32)
+    want = A.varlen_attention_ref(qkv.double(), start, H, D, scale).float()
+    got = A.varlen_attention(qkv.to(dev), start.to(dev), torch.tensor(lens, dtype=torch.int32, device=dev), max(lens), H, D, scale).cpu()
+    # a mean of values of at most 5, whose weights (2^-9 each, their sum is not rounded) and result (2^-9) are rounded to bf16
+    assert qkv.abs()[:, 2 * H * D:].max() < 5.5
+    assert float((got.float() - want).abs().max()) < 5.5 * 2 ** -8
+
+
 def test_embeddings(dev):
     V, H, P = 1000, 384, 512
     word, pos, typ = rnd(V, H, dev=dev), rnd(P, H, dev=dev, seed=1), rnd(2, H, dev=dev, seed=2)
