@@ -147,7 +147,16 @@ __global__ __launch_bounds__(64 * NW, D <= 64 && NW == 4 ? 4 : 1) void attn_fwd_
   const int wrow0 = min(row_base + __builtin_amdgcn_readfirstlane(wave) * 16, nrows - 1);
   const int wave_lim_min = min(kv_hi, p.causal ? ctx - qlen + wrow0 / G + 1 : ctx);
 
-  const float f = p.scale_log2 > 0.f ? p.scale_log2 : 1.f;
+  // the scale is the exponent's factor and more than 0: the queries take the sign of one that is less, and all of one that is 0 or none
+  float f = p.scale_log2;
+  if (!(f > 0.f)) {
+    const float by = f < 0.f ? -1.f : f;
+    f = f < 0.f ? -f : 1.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qf[c][e] = f2bits(bits2f(qf[c][e]) * by);
+  }
   float m = -INFINITY, lsum = 0.f;
   f32x4_t o[ND];
 #pragma unroll
@@ -222,13 +231,7 @@ __global__ __launch_bounds__(64 * NW, D <= 64 && NW == 4 ? 4 : 1) void attn_fwd_
       }
     }
     // this lane holds keys kt0 + 16t + 4*h4 + r of query row li.  The mask runs only on tiles that reach the wave's first row's
-    // limit (a real wave-uniform branch, see attn_prefill_kernel); the scale is the exponent's factor, but for one of 0 or less,
-    // which turns the order
-    if (!(p.scale_log2 > 0.f)) {
-      asm volatile("");
-#pragma unroll
-      for (int t = 0; t < 4; ++t) s[t] *= p.scale_log2;
-    }
+    // limit (a real wave-uniform branch, see attn_prefill_kernel)
     if (kt0 + KT > wave_lim_min) {
       asm volatile("");
 #pragma unroll
@@ -246,18 +249,18 @@ __global__ __launch_bounds__(64 * NW, D <= 64 && NW == 4 ? 4 : 1) void attn_fwd_
       for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, s[t][r]);
     tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    // the maximum moves, and with it the sums' scale, only where a row's passes it by 2^kRescaleLog2 (as in attn_prefill_kernel): with the
-    // scale in the exponent's fma 36 vector instructions a tile fewer; an encoder batch of 24000 tokens 5622 -> 5600 us.  (Two LDS
-    // buffers and one barrier a tile gained nothing; five waves a SIMD in place of four spill, 3 % more time.)
-    const float m_new = fmaxf(m, tmax * f);
-    if (__any(m_new > m + kRescaleLog2)) {
-      const float alpha = __builtin_amdgcn_exp2f(m - (m_new == -INFINITY ? 0.f : m_new));
-      m = m_new;
-      lsum *= alpha;
+    // Every tile's maximum counts, so that a row's largest weight is 1 and rounds to itself: with one that moves by 2^kRescaleLog2 at a time
+    // (attn_prefill_kernel) the outputs were 4 - 19 % further from 64 bits, texts of 120 and 256 tokens, for 2 % less time.  The scale
+    // in the exponent's fma: 64 texts of 500-512 tokens, 12 heads, D = 64 99.1 -> 96.8 us, D = 32 69.8 -> 66.9; 128 of 60-320 alike, D = 64
+    // 53.5 and 52.6, D = 32 41.7 and 40.2; one of 50 3.77 and 3.78, 3.40 and 3.40.  (D = 32 at seven waves a SIMD in place of six:
+    // these within 1 %, 8 texts of 256 6.37 -> 6.57.  Two LDS buffers and one barrier a tile gained nothing; D = 64 at five waves in
+    // place of four spills, 3 % more time.)
+    const float m_new = fmaxf(m, tmax * f), nm = m_new == -INFINITY ? 0.f : -m_new;
+    const float alpha = __builtin_amdgcn_exp2f(m + nm);
+    m = m_new;
+    lsum *= alpha;
 #pragma unroll
-      for (int n = 0; n < ND; ++n) o[n] *= alpha;
-    }
-    const float nm = m == -INFINITY ? 0.f : -m;
+    for (int n = 0; n < ND; ++n) o[n] *= alpha;
     float pr[4][4], sum[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {

@@ -75,6 +75,28 @@ def test_varlen_attention_scales(dev, D, scale):
     assert float((got.float() - want).abs().max()) < 5.5 * 2 ** -8
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_varlen_attention_leading_key(dev, D):
+    """Texts whose values are all 0 but that of one late key, which each row sees more than any other: its weight, the largest, is 1 and
+    has no rounding in bf16, and the sum of the weights is fp32, so that the result is off by its own rounding alone.  (With weights
+    relative to a maximum of an earlier tile it is off by up to two.)"""
+    from githubrepostorag_amd.ops import attention as A
+
+    g = torch.Generator().manual_seed(D)
+    n, H, S = 130, 4, 8
+    qkv = torch.zeros(S, n, 3, H, D)
+    qkv[:, :, 0, :, 0] = 1 + torch.rand(S, n, H, generator=g)
+    qkv[:, :, 1, :, 0] = torch.rand(S, n, H, generator=g)
+    qkv[:, 100, 1, :, 0] = 2 + torch.rand(S, H, generator=g)
+    qkv[:, 100, 2] = 1
+    qkv = qkv.reshape(S * n, -1).to(torch.bfloat16)
+    start = torch.arange(0, S * n + 1, n, dtype=torch.int32)
+    want = A.varlen_attention_ref(qkv.double(), start, H, D, 1.0)
+    got = A.varlen_attention(qkv.to(dev), start.to(dev), torch.full((S,), n, dtype=torch.int32, device=dev), n, H, D, 1.0).cpu()
+    half = 2.0 ** (torch.floor(torch.log2(want)) - 8)  # half an ulp of a bf16 result, and 2^-6 of that for the fp32 sums
+    assert bool(((got.double() - want).abs() <= (1 + 2.0 ** -6) * half).all())
+
+
 def test_embeddings(dev):
     V, H, P = 1000, 384, 512
     word, pos, typ = rnd(V, H, dev=dev), rnd(P, H, dev=dev, seed=1), rnd(2, H, dev=dev, seed=2)
