@@ -24,17 +24,18 @@ template <> __device__ __forceinline__ void stf<float>(float* p, float v) { *p =
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + __expf(-x)); }
 __device__ __forceinline__ float sigmoid_acc(float x) { return 1.f / (1.f + expf(-x)); }
 __device__ __forceinline__ float silu_acc(float x) { return x / (1.f + expf(-x)); }
-// The same as sigmoid_acc without its scaled division and expf (32 instructions, 19 here) or a branch: 2^(hi + lo) by the bare instruction,
-// 1 + e as two floats, a reciprocal with one correction step.  4 M random numbers of [-1, 1] / [-8, 8] / [-20, 20], error of the value, rms
-// and largest in 1e-8: sigmoid_acc 4.0, 12.8 / 3.8, 13.0 / 3.7, 15.4, here 3.0, 9.9 / 2.8, 10.8 / 2.8, 10.8.  Infinities and NaN as there;
-// below -87.3, where the value is less than 1.2e-38, 0.  minGRU, two layers of 1187 tokens in a step, 2024 -> 2013 us of it.
+// The same as sigmoid_acc without its scaled division and expf (32 instructions, 21 here) or a branch: 2^(hi + lo) by the bare instruction,
+// 1 + e as two floats, a reciprocal with one correction step, all of a quarter of 1 + e, whose reciprocal is a normal number up to
+// e = 2^128.  Infinities, NaN and values below 2^-126 (x below -87.3; 0 from -88.72 on) as there.  4 M random numbers of [-1, 1] / [-8, 8]
+// / [-20, 20] / [-88, 88], relative error, rms and largest in 1e-8: sigmoid_acc 4.1, 12.8 / 9.3, 43 / 20, 80 / 81, 276, here 2.9, 10.0 /
+// 2.8, 11.0 / 2.8, 10.8 / 2.6, 20.3.  minGRU, 1187 tokens of 1536 channels, 22.9 -> 19.5 us.
 __device__ __forceinline__ float sigmoid_x(float x) {
   constexpr float L2E = 1.4426950408889634f, L2E_LO = 1.9259629911266175e-8f;
   const float hi = -x * L2E, lo = fminf(fmaf(-x, L2E_LO, fmaf(-x, L2E, -hi)), 1.f);  // (no number for an infinite x: 1 then)
-  const float t = __builtin_amdgcn_exp2f(hi), d = 1.f + t, b = d - 1.f, r = __builtin_amdgcn_rcpf(d);
-  const float rest = fmaf(t, 0.6931471805599453f * lo, (1.f - (d - b)) + (t - b));
+  const float t = 0.25f * __builtin_amdgcn_exp2f(hi), d = 0.25f + t, b = d - 0.25f, r = __builtin_amdgcn_rcpf(d);
+  const float rest = fmaf(t, 0.6931471805599453f * lo, (0.25f - (d - b)) + (t - b));
   const float q = fmaf(fmaf(-rest, r, fmaf(-d, r, 1.f)), r, r);
-  return hi > 126.f ? 0.f : q;
+  return hi >= 128.f ? 0.f : 0.25f * q;
 }
 // tanh in fp32 to a few ulp: (1 - e^-2|x|) / (1 + e^-2|x|), a short odd series below 0.02 where that form cancels.
 // The exponential is the bare instruction with its argument's rounding put back; the quotient (divisor in [1, 2]) is a

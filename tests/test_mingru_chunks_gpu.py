@@ -41,3 +41,34 @@ def test_chunks(lens, W, dtype):
         tol = (64 * 2 ** -24 + (2 ** -8 if dtype == torch.bfloat16 else 0)) * big * float(gate.abs().max())
         assert (y[at - l:at].cpu().double() - want).abs().max() < tol
     assert torch.equal(state[0].cpu(), st[0])
+
+
+def test_ends_of_the_range():
+    """Single numbers in each of the three gates, out to infinities, NaN and gates below 2^-126: z, the candidate and the output's SiLU
+    alone, in portions of 70 tokens whose every second token makes the state 0 again (z = 1, candidate 0)."""
+    inf = float("inf")
+    v = torch.tensor([0.0, 1e-30, -1e-30, 0.5, -0.5, 17.0, -17.0, 80.0, -80.0, -86.9, -87.2, -87.4, -88.0, -88.5, -88.7, 88.0, 88.7, 89.0, -100.0,
+                      100.0, -1e4, 1e4, -3e38, 3e38, inf, -inf, float("nan")])
+    W, n = v.numel(), 70
+    x = torch.empty(3, n, 3, W)  # (which gate, token, z | candidate | gate, number)
+    x[:, ::2, 0], x[:, ::2, 1], x[:, ::2, 2] = inf, -inf, 64.0
+    for i, row in enumerate(((v, 0.5, 64.0), (inf, v, 64.0), (inf, 0.5, v))):
+        for j in range(3):
+            x[i, 1::2, j] = row[j]
+    st = torch.zeros(3, W)
+    state, zero = st.cuda(), torch.zeros(W).cuda()
+    y = mingru_scan(x.reshape(3 * n, 3 * W).cuda(), 0, W, 2 * W, zero, zero, state, _meta("cuda", [n] * 3, [n] * 3, [2, 0, 1]), W)
+    x = x.double()
+    sig = lambda a: torch.where(a < -88.72284, 0.0, torch.sigmoid(a))  # (1 + e^-a is infinite in 32 bits there)
+    z, gate = sig(x[:, :, 0]), x[:, :, 2] * sig(x[:, :, 2])
+    cand = torch.where(x[:, :, 1] >= 0, x[:, :, 1] + 0.5, sig(x[:, :, 1]))
+    S, want = torch.zeros(3, W, dtype=torch.float64), []
+    for t in range(n):
+        S = (1 - z[:, t]) * S + z[:, t] * cand[:, t]
+        want.append((S * gate[:, t]).float())  # (3e38 and more times 64: infinite in 32 bits)
+    want, got = torch.stack(want, 1), y.cpu().view(3, n, W)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isinf(), want.isinf()) and torch.equal(got[got.isinf()], want[want.isinf()])
+    f = want.isfinite()
+    # 2 ulp of a gate and one of each product; a gate of less than 2^-126 is off by up to 2^-149, 89 times that in the result
+    assert bool(((got.double() - want.double()).abs()[f] <= 2.0 ** -21 * want[f].abs().double() + 89 * 2.0 ** -149).all())
