@@ -345,13 +345,26 @@ def pair_plan(M: int, N: int, K: int, fused: bool = False) -> int | None:
 
 
 @functools.lru_cache(4096)
-def pair_fills(M: int, N: int, K: int) -> bool:
-    """Whether short contractions whose 256 x 256 tiles are one round of CUs and a rest of up to a fifth go in 128 x 192 ones: chains
-    of 192 rows / these, us, 22500 x 768 x 512 24.2 / 23.5, 24000 x 768 x 768 32.5 / 32.5, 9500 x 1920 x 512 (1.19 rounds) 25.0 / 23.8,
-    0.95 - 1.03 of 13 points; with longer rests 6000 x 3200 x 768 (1.22) 32.1 / 37.8, 27000 x 768 x 768 (1.24) 32.7 / 38.3, 1.06 - 1.18
-    of 7."""
+def pair_fills(M: int, N: int, K: int, act: bool = False, chain: bool = True) -> bool:
+    """Whether short contractions of more 256 x 256 tiles than CUs go in 128 x 192 ones.  ``act``: with an activation, beside which
+    a chain of tiles has no products; ``chain``: the operands meet chain_takes().
+
+    434 products of 64 - 72000 columns, K 128 - 1024, one after another of different weights, us, chains / these.  Plain, as many small
+    tiles as three a CU: 0.88 - 1.17, and 1.02 in the geometric mean where no line below takes them off (22500 x 768 x 512 24.2 / 23.5,
+    42419 x 384 x 384 22.7 / 22.0, 9651 x 1920 x 384 22.8 / 22.3); a fourth a CU costs as much as three (26035 x 768 x 768 33.6 / 39.6).
+    Not at less than 1536 rows, which chains have tiles of 128 rows for or are alike at (300 x 36864 x 768 26.6 / 30.8), nor where a column
+    or less of them is deep (94899 x 128 x 768 38.6 / 44.0).  With GELU 1.21 (37555 x 384 x 384 31.6 / 26.1), and 1.17 up to four a CU
+    where K is 384 or less (28339 x 640 x 256 30.3 / 27.5; 768 deep 43.1 / 43.9).  The choice is 1.001 (GELU 1.002) of the better in the
+    geometric mean, 1.04 (1.10) at most.  Without chains a workgroup a tile has 1.29 (1.42) of these' time up to 0.62 of the rounds."""
     tiles, ncu = -(-M // 256) * -(-N // 256), _num_cus()
-    return K <= 1024 and ncu < tiles <= 1.2 * ncu
+    if K > 1024 or tiles <= ncu:
+        return False
+    if not chain:
+        return M * N < 0.62 * 65536 * ncu * -(-tiles // ncu)
+    small = _pair_tiles(0, M, N)
+    if act:
+        return small <= (4 if K <= 384 else 3) * ncu
+    return small <= 3 * ncu and M >= 1536 and (N > 192 or N * K <= 1 << 15)
 
 
 def pair_takes(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None, out: torch.Tensor | None = None) -> bool:
@@ -590,8 +603,9 @@ def gemm(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None, act: i
         shape = pair_plan(M, N, K, act != ACT_NONE)
         if shape is not None and pair_takes(x, w, b, out):
             return gemm_pair(x, w, b, shape, EPI_STORE, act, out)
-        ksplit, sk = schedule(M, N, K, chain=chain_takes(x, w, b, out))
-        if (ksplit, sk) == (1, 0) and pair_fills(M, N, K) and pair_takes(x, w, b, out):
+        chain = chain_takes(x, w, b, out)
+        ksplit, sk = schedule(M, N, K, chain=chain)
+        if (ksplit, sk) == (1, 0) and pair_fills(M, N, K, act != ACT_NONE, chain) and pair_takes(x, w, b, out):
             return gemm_pair(x, w, b, 0, EPI_STORE, act, out)
     sk = sk or 0
     if out is None:

@@ -389,7 +389,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None = None) -> t
                 return _tile.gemm(x, w, b, ksplit=p[0], sk=p[1])
             if _plain_product(x, w, b):
                 p = _tile.wide_plan(M, N, K, chain) or _tile.unmeasured_plan(M, N, K)
-                if p == (1, 0) and _tile.pair_fills(M, N, K) and _tile.pair_takes(x, w, b):
+                if p == (1, 0) and _tile.pair_fills(M, N, K, chain=chain) and _tile.pair_takes(x, w, b):
                     return _tile.gemm_pair(x, w, b, 0)
                 return _tile.gemm(x, w, b, ksplit=p[0], sk=p[1])
             return torch.nn.functional.linear(x, w, b)
@@ -427,7 +427,7 @@ def bound_product(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, act:
                 _tile.prefill_plan(M, N, K, chain=chain) or _tile.wide_plan(M, N, K, chain) or _tile.unmeasured_plan(M, N, K))
             if plan == (1, 0):
                 measured = not act and _tile.prefill_plan(M, N, K) is not None
-                shape = 0 if not measured and _tile.pair_fills(M, N, K) else None
+                shape = 0 if not measured and _tile.pair_fills(M, N, K, act != 0, chain) else None
                 if shape is None:
                     name, tail = "grag_gemm_tile", (_tile.EPI_STORE, act, 1, 0, None, None)
         if shape is not None and (act or kind == "pair" or kind == "tile_prefill"):

@@ -168,9 +168,36 @@ def test_linear_with_a_bias_at_any_address(dev, monkeypatch, M, N, K, other, at)
 @pytest.mark.gpu
 @pytest.mark.parametrize("K,takes", [(768, True), (1024, True), (1088, False)])
 def test_rounds_of_small_tiles(dev, K, takes):
-    """Short contractions of one round of CUs and up to a fifth go in small tiles: 255, 258, 306 and 309 tiles on 256 CUs."""
+    """Short contractions of more tiles than CUs go in small tiles up to three of them a CU: 255, 258, 288 and 291 tiles on 256 CUs, the
+    last two of 768 and 776 small ones."""
     if G._num_cus() != 256:
         pytest.skip("the row counts are those of 256 CUs")
-    assert [G.pair_fills(t * 256, 768, K) for t in (85, 86, 102, 103)] == [False, takes, takes, False]
+    assert [G.pair_fills(t * 256, 768, K) for t in (85, 86, 96, 97)] == [False, takes, takes, False]
     x, w, b = _mk(dev, 86 * 256 - 7, 768, K)
     assert torch.equal(G.gemm(x, w, b), G.gemm(x, w, b, ksplit=1, sk=0))
+
+
+@pytest.mark.parametrize("M,N,K,act,chain,takes", [
+    (42419, 384, 384, False, True, True), (32768, 384, 384, False, True, False), (50611, 384, 384, False, True, False),  # (three a CU)
+    (50611, 384, 384, True, True, True), (50611, 384, 448, True, True, False), (66000, 384, 384, True, True, False),  # (four with GELU)
+    (300, 36864, 768, False, True, False), (300, 36864, 768, True, True, True), (1600, 10752, 512, False, True, True),  # (few rows)
+    (68787, 128, 256, False, True, True), (68787, 128, 320, False, True, False),  # (a deep column)
+    (27000, 768, 768, False, True, False), (27000, 768, 768, False, False, True), (28000, 768, 768, False, False, False)])  # (no chains)
+def test_lines_of_small_tiles(monkeypatch, M, N, K, act, chain, takes):
+    monkeypatch.setattr(G, "_NCU", [256])
+    assert G.pair_fills(M, N, K, act, chain) == takes
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("at,took", [(0, 0), (4, 1)])
+def test_small_tiles_without_chains(dev, monkeypatch, at, took):
+    """A bias at an address that chains do not take: small tiles up to 0.62 of the rounds, and the same results."""
+    if G._num_cus() != 256:
+        pytest.skip("the row counts are those of 256 CUs")
+    x, w, b = _mk(dev, 97 * 256, 768, 192)
+    b = torch.cat([b, b[:at]])[at:] if at else b
+    calls, pair = [], G.gemm_pair
+    monkeypatch.setattr(G, "gemm_pair", lambda *a, **k: calls.append(1) or pair(*a, **k))
+    y = G.gemm(x, w, b)
+    assert len(calls) == took
+    torch.testing.assert_close(y.double(), x.double() @ w.double().T + b.double(), **TOL)
