@@ -11,10 +11,10 @@
 // What bounds it: one thread per state column, three vector instructions per state element and token (the kernels of
 // seqmix.hip and ssm.hip, which still take decode rows and heads of more than 128 rows), waited on LDS broadcasts at 3 % of
 // the fp32 vector rate.  Here a chunk is bound by vector instructions (the splits, SiLU) and the latency of its dependent
-// steps.  Measured, those kernels -> this one with workgroups in order of sequence -> longest first (scan_item): decay with
-// SiLU, 28 heads of 128 x 128, 7 portions of 8192 tokens 2150 -> 748 -> 410 us, 1 x 1187 635 -> 110 (with the splits, the halves of
-// q and the table below, 380 - 390 in a model's step where it was 474 there); without SiLU 2060 -> 214 -> 153
-// and 602 -> 50; state space, 56 heads of 128 x 64, 3 portions of 4096 tokens 1450 -> 165 -> 115 us.
+// steps.  Measured, those kernels -> this one with workgroups in order of sequence -> longest first (scan_item) -> with pairs split
+// together, the halves of q and the table below: decay with SiLU, 28 heads of 128 x 128, 7 portions of 8192 tokens in all 2150 -> 748
+// -> 386 -> 311 us, 1 x 1187 635 -> 108 -> 92; without SiLU 2060 -> 214 -> 153 -> 152 and 602 -> 47 -> 45; state space, 56 heads of
+// 128 x 64, 3 portions of 4096 tokens 1450 -> 165 -> 100 -> 94.
 //
 // Precision: nothing is rounded to 16 bits that was not before.  An operand is the sum of bf16 parts of 8 bits of mantissa
 // each, and a product of operands is the matrix-core products of their parts (exact, fp32 sums).  What is fp32 (S, the
@@ -301,7 +301,7 @@ __device__ __forceinline__ bool scan_item(const ScanArgs& a, int item, ScanItem&
 // ND = ceil(d / 32).  AP = 1 takes 76 KB of LDS and 128 registers: two workgroups share a CU, one's products over the other's
 // staging.  FULL: d = 32 ND, vd is a multiple of 64 and rows are aligned for 4-element accesses (rd / 2 a multiple of 4), so that
 // nothing is tested per element: of the ~4000 instructions a chunk took with the tests, half were theirs.  Rows behind a portion's
-// end are copies of its last row with weight c_s = 0.
+// end are copies of its last row: their weight into the state is 0 (row 5 of sc), and of the queries only they themselves see them.
 template <typename TI, int AP, bool SSM, bool FULL, int ND, int MODE>
 __global__ void __launch_bounds__(LTHREADS, AP == 1 ? 4 : 2)
 linear_scan_kernel(const ScanArgs a) {
@@ -447,6 +447,8 @@ linear_scan_kernel(const ScanArgs a) {
       hi = rate * m, lo = fmaf(rate, m, -hi);
       ehi = rate * n, elo = fmaf(rate, (float)n, -ehi);
     }
+    // (The first four are read for a state space's outputs alone.  Stored for those alone, decays took 0.4 % less time on average of 84
+    // sizes, but 6 portions of 700 tokens, 32 heads of 32 x 64 with SiLU, 54.0 us for 52.5.)
     sc[buf][0][lane] = hi;
     sc[buf][1][lane] = lo;
     sc[buf][2][lane] = cs * sign;
@@ -658,10 +660,15 @@ linear_scan_kernel(const ScanArgs a) {
         }
       }
       if (t < n) {
+        // (The address of a decay of 128 registers is made here: carried through the loop it was spilled, and its way back waits as below.
+        // 28 heads of 128 x 128 without SiLU, 7 portions of 8192 tokens 165 -> 152 us.  Others spill no less so or lose a little:
+        // state space, 3 x 4096 247 -> 261; 32 heads of 32 x 64 with SiLU, 7 x 1000 73.5 -> 76.1.)
+        int own = t;
+        if constexpr (!SSM && AP == 1) asm volatile("" : "+v"(own));
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
           const int c0 = 16 * (2 * vh + b) + 4 * quad;
-          float* op = a.out + (size_t)(t0 + t) * ((size_t)a.H * a.vd) + h * a.vd + tile * LVT + c0;
+          float* op = a.out + (size_t)(t0 + own) * ((size_t)a.H * a.vd) + h * a.vd + tile * LVT + c0;
           if (SSM) {  // (x as it lies in LDS where its one part is all of it: from memory it came behind the next chunk's rows, and
                       // every wave waited for it and for them: state space, 56 heads, 3 portions of 4096 tokens 105 us -> 95)
             if constexpr (AP == 1)
