@@ -39,14 +39,16 @@ def _scan_cut(max_q: int, tokens: int, nseq: int, tiles: int, split: bool, d: in
     the chip's share of all and part of a walk for its uneven end; a single portion whole rounds of equal parts.  A walk of some
     chunks costs some more for its start and its state.  Where portions are cut, all parts but the last are walked for the
     state alone before (about a quarter of a walk), and a part reads the states of those before it.
-    ``split``: operands in three parts (one workgroup a CU, 12 us a chunk), else two workgroups a CU and 5.7 us.
+    ``split``: operands in three parts (one workgroup a CU, 9 us a chunk), else two workgroups a CU and 4.5 us.
 
-    From 455 points of 21 sizes, 1 - 20 portions, 65 - 8192 tokens, every cut timed: the cut taken is 1.015 of the best in the
-    geometric mean and 1.31 at most (without the cost of a walk's start 1.038 and up to 1.37, where parts of one chunk were taken:
-    fp32, 8 heads of 64 x 128, 2 portions of 1500 tokens, cut at 1 / 2 / 3 chunks 89 / 65 / 84 us).  28 heads of 128 x 128 with SiLU,
-    3 portions of 4096 tokens, cut at 2 / 4 / 8 / 16 / not at all 291 / 270 / 260 / 269 / 340 (taken 8), 7 of 8192 567 / 498 / 465 /
-    443 / 410 - 448 (none); state space, 56 heads of 128 x 64, 3 of 4096 141 / 116 / 110 / 149 / 171 (8); 24 of 128 x 64, one of
-    8192 177 / 122 / 115 / 146 / 517 (8); 80 of 16 x 64, one of 4096 250 / 207 / 236 / 261 / 564, at 12 218 (12, one pass 208)."""
+    From 455 points of 21 sizes, 1 - 20 portions, 65 - 8192 tokens, every cut timed: the cut taken was 1.015 of the best in the
+    geometric mean and 1.31 at most (without the cost of a walk's start 1.038 and up to 1.37, where parts of one chunk were taken).
+    Since then a chunk in three parts takes a fifth less and one in one part 3 % less; of 140 sizes measured again, 32 - 57344 tokens, the cut
+    taken is 1.026 and 1.038 of the best in the geometric mean, 1.19 and 1.26 at most.  Us now: fp32, 8 heads of 64 x 128, 2 portions of
+    1500 tokens, cut at 1 / 2 / 3 chunks 72 / 51 / 65 (taken 2); 28 heads of 128 x 128 with SiLU, 3 portions of 4096 tokens, cut at 2 / 4
+    / 8 / 16 / not at all 247 / 220 / 212 / 243 / 202 (taken 8), 7 of 8192 469 / 408 / 374 / 368 / 311 (none); state space, 56 heads of
+    128 x 64, 3 of 4096 129 / 102 / 94 / 118 / 97 (8); 24 of 128 x 64, one of 8192 175 / 113 / 101 / 116 / 517 (8); 80 of 16 x 64, one
+    of 4096 247 / 205 / 232 / 253 / 517, at 12 213 (12, one pass 210)."""
     slots, read, start, ahead_start, tail, first, const, odd = (
         (256, 0.002, 1.87, 1.59, 0.59, 0.24, 0.69, 1.12) if split else (512, 0.5, 1.79, 0.15, 0.83, 0.275, 1.1, 1.15))
     chunks, total = -(-max_q // LINEAR_SCAN_CHUNK), tokens / LINEAR_SCAN_CHUNK + (nseq - 1) / 2
@@ -79,8 +81,7 @@ def _scan_walks(max_q: int, tokens: int, nseq: int, tiles: float, split: bool) -
     counted.  Several portions take the longest walk or the chip's share of all and about a third of a walk for its uneven
     end; a single portion whole rounds of equal parts.  Where portions are cut, all parts but the last are walked for the
     state alone before (0.42 of a walk), and a part reads the states of those before it.  ``split``: operands in three parts (one
-    workgroup a CU, 12 us a
-    chunk), else two workgroups a CU and 5.7 us."""
+    workgroup a CU), else two workgroups a CU."""
     slots, read, crowd = (256, 0.026, 1.0) if split else (512, 0.11, 1.2)  # (whole portions often have a CU of their own)
     chunks, total = -(-max_q // LINEAR_SCAN_CHUNK), tokens / LINEAR_SCAN_CHUNK + (nseq - 1) / 2
     share = tiles / slots  # of a round, a workgroup for each tile
@@ -109,10 +110,11 @@ def _scan_taken(m: AttnMetadata, tokens: int, H: int, d: int, vd: int, split: bo
     (of portions of a chunk: as many as their rounds) of 2.9 + 0.021 d where exact with one part an operand, 0.4 + 0.10 d
     with three, 5.9 + 0.039 d and 14.6 + 0.084 d otherwise; a round of workgroups that share a CU costs 1.6 walks, of
     those that do not 1.1.  One-pass kernels: 9.5 + a chain of 0.14 + 0.0345 d a token and 3.5e-7 a token and number of
-    the state, twice that where portions are cut at 64.  Of 470 points of 21 sizes the choice is within 0.2 % of the faster
-    side in the geometric mean; the most that was lost is 1.34 (fp32, 56 heads of 16 x 64, 5 portions of 1187 tokens, scan / one pass
-    100 / 134).  A rule on the portions' length alone was 13 % off (scan against one pass: fp32, 28 heads of 16 x 16, 64 x 64 tokens
-    153 / 54; fp32 state space, 56 heads of 8 x 16, 7 portions of 8192 728 / 158)."""
+    the state, twice that where portions are cut at 64.  Of 470 points of 21 sizes the choice was within 0.2 % of the faster
+    side in the geometric mean, and of 140 sizes measured again since the scan became faster within 0.1 %, 1.07 at most.  Small fp32 heads that
+    fill the chip are still reckoned as before, and lose the most: 56 heads of 16 x 64, 5 portions of 1187 tokens, scan / one pass 80 / 132,
+    not taken.  A rule on the portions' length alone was 13 % off (scan against one pass: fp32, 28 heads of 16 x 16, 64 x 64 tokens
+    95 / 52; fp32 state space, 56 heads of 8 x 16, 7 portions of 8192 431 / 155)."""
     if m.max_q_len < LINEAR_SCAN_MIN or d > lib().grag_linear_scan_max_dim():
         return False
     base, span = ((0.4, 0.10) if split else (2.9, 0.021)) if exact else ((14.6, 0.084) if split else (5.9, 0.039))
