@@ -45,6 +45,16 @@ __global__ void __launch_bounds__(256 * TEAMS, MR == 32 || TEAMS > 1 ? 2 : 4) si
   constexpr int RB = 2 * D, CPR = D / 8, NC = D / KD, ND = D / MR, NT = SP_KT / MR, TILE = SP_KT * RB;
   constexpr int ROWS = MR * NW, PPW = TILE / 1024 / NW, RPP = 1024 / RB;
   typedef float acc_t __attribute__((ext_vector_type(AR)));
+  // With two teams the scores and the first weights go before the SIMD's other waves, whose values' products have instructions between: of
+  // 101 launches 2 % less time, of 54 capped ones 6 % (12 / 2 heads of 64, 512 rows on 7000 keys 109 -> 91 us), one longer (45.9 -> 47.9).
+  // One team lost as often as it gained, 433 launches 0.94 - 1.10 of the time (8192 rows, 12 / 2 heads of 64 207 -> 222; of 128, 4 x 2048
+  // 96 -> 90).
+  auto before_others = [](bool on) __attribute__((always_inline)) {
+    if constexpr (TEAMS > 1) {
+      if (on) __builtin_amdgcn_s_setprio(1);
+      else __builtin_amdgcn_s_setprio(0);
+    }
+  };
   auto mma = [](bf16x8_t a, bf16x8_t b, acc_t c) {
     if constexpr (MR == 16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
     else return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -142,10 +152,10 @@ __global__ void __launch_bounds__(256 * TEAMS, MR == 32 || TEAMS > 1 ? 2 : 4) si
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) {
       s[tt] = acc_t{};
-      if (tt == 0) __builtin_amdgcn_s_setprio(1);  // (before the CU's other workgroup, whose values' products have instructions between)
+      if (tt == 0) before_others(true);
 #pragma unroll
       for (int c = 0; c < NC; ++c) s[tt] = mma(kf[tt][c], qf[c], s[tt]);
-      if (tt == NT - 1) __builtin_amdgcn_s_setprio(0);
+      if (tt == NT - 1) before_others(false);
     }
     if constexpr (CAP) {  // cap in the natural domain, then to log2
       // Below 1/4 by tanh's power series to x^9, whose next term is 1/10 of fp32's rounding there; a tile with a larger score by
@@ -267,11 +277,11 @@ __global__ void __launch_bounds__(256 * TEAMS, MR == 32 || TEAMS > 1 ? 2 : 4) si
       continue;
     }
     const char* v_lds = k_lds + TILE;
-    __builtin_amdgcn_s_setprio(1);
+    before_others(true);
     load_v(v_lds, 0);
     maximum();
     weights(0);
-    __builtin_amdgcn_s_setprio(0);
+    before_others(false);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < NP; ++u) {
