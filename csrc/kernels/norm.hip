@@ -356,7 +356,10 @@ __global__ __launch_bounds__(kThreads) void layernorm_kernel(
 }
 
 // BERT embeddings: LN(word[id] + pos[p] + type[tt]).  Up to 1024 columns a wave a token, as layernorm_wave_kernel: 24000 tokens of 768
-// 37.8 us in workgroups of 256 threads a token, here 22.7.
+// 34.3 us in workgroups of 256 threads a token, here 18.0; from 513 columns on at 800 tokens and more, as with fewer a token's chain of two
+// loads a lane is longer than the workgroup's (us, workgroups / here: 768 columns 50 / 500 / 800 / 2000 tokens 2.84 / 3.07 / 3.27 /
+// 4.24 and 3.00 / 3.12 / 3.24 / 3.75, 1024 2.75 / 3.05 / 3.50 / 4.38 and 3.00 / 3.14 / 3.24 / 3.86; 384 2.82 / 2.95 / 3.16 / 3.93
+// and 2.60 / 2.67 / 2.73 / 2.91).
 template <int VPT>
 __global__ __launch_bounds__(kThreads) void bert_embed_ln_wave_kernel(
     const int32_t* __restrict__ ids, const int32_t* __restrict__ pos_ids,
@@ -422,7 +425,7 @@ __global__ __launch_bounds__(kThreads) void bert_embed_ln_wave_kernel(
     }
 }
 
-// Wider rows: a workgroup a token.
+// Wider rows, and few tokens of more than 512 columns: a workgroup a token.
 template <int VPT>
 __global__ __launch_bounds__(kThreads) void bert_embed_ln_kernel(
     const int32_t* __restrict__ ids, const int32_t* __restrict__ pos_ids,
@@ -696,7 +699,7 @@ GRAG_API int grag_bert_embed_ln(const int32_t* ids, const int32_t* pos_ids,
     return (int)hipGetLastError();
   };
   if (H <= 512) return wave(bert_embed_ln_wave_kernel<1>);
-  if (H <= 1024) return wave(bert_embed_ln_wave_kernel<2>);
+  if (H <= 1024 && T >= 800) return wave(bert_embed_ln_wave_kernel<2>);
   auto args = [&](auto kern) {
     kern<<<T, kThreads, 0, stream>>>(ids, pos_ids, type_ids, (const bf16*)word, (const bf16*)pos,
                                      (const bf16*)type, (const bf16*)gamma, (const bf16*)beta,

@@ -111,7 +111,7 @@ def test_embeddings(dev):
 
 @pytest.mark.parametrize("T,H", [(1, 8), (5, 512), (7, 520), (3, 1024), (6, 1032), (2, 2056)])
 def test_bert_embed_ln_widths(T, H):
-    """A wave a token up to 1024 columns, a workgroup from there on; token counts that are no multiple of a workgroup's four."""
+    """A wave a token up to 512 columns, a workgroup from there on; token counts that are no multiple of a workgroup's four."""
     from githubrepostorag_amd.ops import norm as N
 
     g = torch.Generator().manual_seed(T * 3000 + H)
@@ -123,6 +123,23 @@ def test_bert_embed_ln_widths(T, H):
         got = N.bert_embed_ln(*(None if x is None else x.cuda() for x in (ids, pids, t, word, pos, typ, gamma, beta)), 1e-12).cpu()
         # both round an fp32 result once: one bf16 step (2^-8) apart where it lies between two
         torch.testing.assert_close(got.float(), want.float(), rtol=2 ** -7, atol=2e-6)
+
+
+@pytest.mark.parametrize("H", [512, 520, 768, 1024, 1032])
+@pytest.mark.parametrize("T", [799, 801])
+def test_bert_embed_ln_many_tokens(T, H):
+    """From 800 tokens on a wave a token up to 1024 columns: against 64 bits, one bf16 rounding (2^-8) and 64 fp32 ones of the two terms."""
+    from githubrepostorag_amd.ops import norm as N
+
+    g = torch.Generator().manual_seed(T * 3000 + H)
+    word, pos, typ = (torch.randn(n, H, generator=g).to(torch.bfloat16) for n in (50, 20, 2))
+    gamma, beta = (torch.randn(H, generator=g).to(torch.bfloat16) for _ in range(2))
+    ids, pids, tids = (torch.randint(0, n, (T,), generator=g, dtype=torch.int32) for n in (50, 20, 2))
+    got = N.bert_embed_ln(*(x.cuda() for x in (ids, pids, tids, word, pos, typ, gamma, beta)), 1e-12).cpu().double()
+    v = word.double()[ids.long()] + pos.double()[pids.long()] + typ.double()[tids.long()]
+    scaled = torch.nn.functional.layer_norm(v, (H,), eps=1e-12) * gamma.double()
+    want = scaled + beta.double()
+    assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + 64 * 2.0 ** -24 * (scaled.abs() + beta.double().abs())).all())
 
 
 def test_qkv_rope_kvstore(dev):
