@@ -254,3 +254,29 @@ def test_all_parts_of_an_operand(d, vd, dtype):
     q, k, v = x[:, :H * d].view(n, H, d)[..., 0], x[:, H * d:2 * H * d].view(n, H, d)[..., 0], x[:, 2 * H * d:].view(n, H, vd)
     want = torch.stack([(q * k)[:, 0, None] * v[:, 0], q[:, 1, None] * state[0, 1, 0].double()], 1)
     assert ((got - want).abs() / want).max() < (9 + (6 if act else 0)) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("e", [-108, -90, -60, -30, -8, 0, 9, 17])
+@pytest.mark.parametrize("which", ["q", "k", "v", "state"])
+def test_parts_at_all_exponents(which, e):
+    """test_all_parts_of_an_operand with one operand of 2^e to 2^(e + 1), from the least that has all its parts (the third of 2^-108 is
+    2^-124, of lesser numbers it goes below 2^-126 and is 0) to the largest that the products take (the state: 2^58)."""
+    dev = torch.device("cuda")
+    g = torch.Generator().manual_seed(e + 200)
+    n, H, d, vd = 70, 2, 128, 64
+    m, _ = _meta([n], [6], dev)
+    e = 58 if which == "state" and e == 17 else e
+    up = 15 if e < -60 else 0  # (the others, so that the result is a normal number)
+    x = {c: (1 + torch.rand(n, H, w, generator=g)) * 2.0 ** (e if c == which else up) for c, w in (("q", 1), ("k", 1), ("v", vd))}
+    q, k = torch.zeros(n, H, d), torch.zeros(n, H, d)
+    q[..., :1], k[..., :1] = x["q"], x["k"]
+    k[:, 1] = 0
+    state = torch.zeros(1, H, d, vd)
+    state[:, 1, 0] = (1 + torch.rand(vd, generator=g)) * 2.0 ** (e if which == "state" else up)
+    st = state.to(dev)
+    proj = torch.cat([t.reshape(n, -1) for t in (q, k, x["v"])], 1).to(dev)
+    got = recurrent.decay_attention(proj, 0, H * d, 2 * H * d, torch.tensor([0.0, 1.0], device=dev), st, m, H, d, vd, act=False)
+    got = got.double().cpu().view(n, H, vd)
+    q, k, v = (x[c].double() for c in "qkv")
+    want = torch.stack([q[:, 0] * k[:, 0] * v[:, 0], q[:, 1] * state[0, 1, 0].double()], 1)
+    assert ((got - want).abs() / want).max() < 9 * 2.0 ** -24
